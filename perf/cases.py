@@ -138,13 +138,15 @@ def _weights(model, device):
     kept = torch.rand(vocab, grp["count"], generator=g).argsort(1)[:, :grp["keep"]]
     open_ = torch.zeros(vocab, grp["count"]).scatter_(1, kept, 1.0).repeat_interleave(size, 1)
     pick = (torch.rand(vocab, e, generator=g) + open_).topk(top, 1).indices
-    code = torch.zeros(vocab, e).scatter_(1, pick, 16.0)
+    code = torch.zeros(vocab, e).scatter_(1, pick, 28.0)
     ten["embed"][:, :e] += code.to(device, ten["embed"].dtype)
     for i, _ in moe:
         # each layer reads the columns shifted by whole groups, so layers differ in their choice
         w = ten[f"l{i}.mlp.router"]
-        w *= 0.1
-        w[torch.arange(e), (torch.arange(e) + i * size) % e] += 1.0
+        w *= 0.05
+        w[torch.arange(e), (torch.arange(e) + i * size) % e] += 0.5
+        if f"l{i}.mlp.correction" in ten:       # balanced experts need little correction
+            ten[f"l{i}.mlp.correction"] *= 0.01
     return ten
 
 
