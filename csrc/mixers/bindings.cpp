@@ -164,6 +164,13 @@ int mx_moe_pairs(float* out, void* y, const void* h, int bf16, long h_stride, co
                  float limit, int act, hipStream_t s);
 int mx_moe_topk(int* idx, float* wts, const float* z, const float* corr, long rows, int experts, int top,
                 int groups, int keep, hipStream_t s);
+int mx_few_rows_max();
+int mx_few_rows_gemm(void* Y, int y_f32, long y_stride, const void* X, long x_stride, int rows, const void* W,
+                     const void* bias, int N, int K, int act, float limit, hipStream_t s);
+int mx_experts_few(float* out, void* y, float* d, const void* h, long h_stride, const int* idx, const float* wts,
+                   const void* wgu, const void* wdown, int rows, int top, int experts, int ff, int width, float limit,
+                   int act, void* ys, float* ds, float* sg, const void* shared_w, const void* shared_down,
+                   int shared_ff, float shared_limit, hipStream_t s);
 }
 
 namespace {
@@ -794,6 +801,62 @@ void moe_route_top_logits(Tensor idx, Tensor wts, Tensor h, Tensor router, OptT 
 
 // act 0: clamped GLU, 1: relu^2 (the experts' first matrix is [ff, width], up alone, instead of
 // [2 ff, width], gate | up), 2: silu GLU
+void few_rows_gemm(Tensor y, Tensor x, Tensor w, OptT bias, int64_t act, double limit) {
+  check_rows(x, "x");
+  check_rows(y, "y");
+  const bool glu = act >= 1 && act <= 4;
+  TORCH_CHECK(x.scalar_type() == at::kBFloat16 && w.is_cuda() && w.scalar_type() == at::kBFloat16 && w.dim() == 2 &&
+              w.is_contiguous() && x.size(1) == w.size(1) && act >= 0 && act <= 5, "few_rows_gemm: bf16 rows and weights");
+  TORCH_CHECK(y.size(0) == x.size(0) && y.size(1) * (glu ? 2 : 1) == w.size(0) && x.size(0) <= mx_few_rows_max(),
+              "few_rows_gemm: shapes");
+  if (bias)
+    TORCH_CHECK(bias->is_cuda() && bias->scalar_type() == at::kBFloat16 && bias->is_contiguous() &&
+                bias->numel() == w.size(0), "few_rows_gemm: bias");
+  chk(mx_few_rows_gemm(y.data_ptr(), y.scalar_type() == at::kFloat, y.stride(0), x.data_ptr(), x.stride(0),
+                       (int)x.size(0), w.data_ptr(), bias ? bias->data_ptr() : nullptr, (int)y.size(1),
+                       (int)x.size(1), (int)act, (float)limit, stream()), "few_rows_gemm");
+}
+
+void experts_few(Tensor out, Tensor h, Tensor idx, Tensor wts, Tensor wgu, Tensor wdown, double limit, int64_t act,
+                 OptT shared_w, OptT shared_down, double shared_limit, bool shared_gate) {
+  check_f32(out, "out");
+  check_rows(h, "h");
+  check_i32(idx, "idx");
+  check_f32(wts, "wts");
+  TORCH_CHECK(act >= 1 && act <= 5, "experts_few: activation");
+  const int64_t t = h.size(0), width = h.size(1), top = idx.dim() == 2 ? idx.size(1) : 0;
+  const int64_t mult = act == 5 ? 1 : 2;
+  auto bf16 = [](const Tensor& w) { return w.is_cuda() && w.scalar_type() == at::kBFloat16 && w.is_contiguous(); };
+  TORCH_CHECK(h.scalar_type() == at::kBFloat16 && bf16(wgu) && bf16(wdown) && wgu.dim() == 3 && wdown.dim() == 3 &&
+              wgu.size(0) == wdown.size(0) && wgu.size(2) == width && wdown.size(1) == width &&
+              wgu.size(1) == mult * wdown.size(2), "experts_few: expert weights");
+  TORCH_CHECK(idx.dim() == 2 && idx.size(0) == t && wts.numel() == t * top && out.numel() == t * width &&
+              t <= mx_few_rows_max() && top >= 1, "experts_few: shapes");
+  const int64_t ff = wdown.size(2);
+  int64_t fs = 0;
+  if (shared_w) {
+    TORCH_CHECK(shared_down && bf16(*shared_w) && bf16(*shared_down) && shared_w->dim() == 2 &&
+                shared_down->dim() == 2 && shared_w->size(1) == width && shared_down->size(0) == width,
+                "experts_few: shared expert");
+    fs = shared_down->size(1);
+    TORCH_CHECK(shared_w->size(0) == mult * fs + (shared_gate ? 1 : 0), "experts_few: shared expert's rows");
+  }
+  Tensor y = at::empty({t * top, ff}, h.options()), d = at::empty({t * top, width}, out.options());
+  Tensor ys, ds, sg;
+  if (shared_w) {
+    ys = at::empty({t, fs}, h.options());
+    ds = at::empty({t, width}, out.options());
+    if (shared_gate) sg = at::empty({t}, out.options());
+  }
+  chk(mx_experts_few(out.data_ptr<float>(), y.data_ptr(), d.data_ptr<float>(), h.data_ptr(), h.stride(0),
+                     idx.data_ptr<int>(), wts.data_ptr<float>(), wgu.data_ptr(), wdown.data_ptr(), (int)t, (int)top,
+                     (int)wgu.size(0), (int)ff, (int)width, (float)limit, (int)act,
+                     shared_w ? ys.data_ptr() : nullptr, shared_w ? ds.data_ptr<float>() : nullptr,
+                     shared_w && shared_gate ? sg.data_ptr<float>() : nullptr,
+                     shared_w ? shared_w->data_ptr() : nullptr, shared_w ? shared_down->data_ptr() : nullptr, (int)fs,
+                     (float)shared_limit, stream()), "experts_few");
+}
+
 void moe_pairs(Tensor out, Tensor h, Tensor idx, Tensor wts, Tensor wgu, Tensor wdown, double limit, int64_t act) {
   const bool relu_sq = act == 1;
   TORCH_CHECK(act >= 0 && act <= 2, "moe_pairs: activation");
@@ -1208,6 +1271,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("causal_softmax", &causal_softmax);
   m.def("moe_topk", &moe_topk);
   m.def("moe_pairs", &moe_pairs);
+  m.def("few_rows_gemm", &few_rows_gemm);
+  m.def("experts_few", &experts_few);
+  m.def("few_rows_max", []() { return (int64_t)mx_few_rows_max(); });
   m.def("act_glu", &act_glu);
   m.def("add_norm_shift", &add_norm_shift);
   m.def("rot_norm_prep", &rot_norm_prep);

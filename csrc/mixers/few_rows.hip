@@ -1,0 +1,369 @@
+// Products with few rows (decode steps) on the matrix units, weights read in place:
+//   few_rows_gemm   Y[r, n] = sum_k X[r, k] W[n, k] (+ bias[n]), bf16 or fp32 out; or, gated,
+//                   Y[r, c] = act(X W_gate^T, X W_up^T), W = [gate | up]; or relu(X W^T)^2
+//   experts_first   the chosen experts' first matrices (and the shared expert's) with the
+//                   activation, one read of an expert's matrix for all rows that chose it
+//   experts_down    their second matrices, one fp32 row per (row, chosen expert)
+//   experts_combine out[r] = sum_k w[r, k] d[r, k] + shared part
+// The core and its layout: few_rows.h.
+#include "few_rows.h"
+
+namespace mx {
+
+constexpr int kFewRows = 64;       // most rows of X
+
+// partial sums of the waves -> one sum per (tile, block, lane), in wave order.  red: [WV][NT * NB][64] float4
+template <int NT, int NB, int WV>
+__device__ __forceinline__ void few_rows_park(float4* red, const fr_f32x4 (&acc)[NT][NB], int wave, int lane) {
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+      red[(wave * NT * NB + t * NB + b) * 64 + lane] = make_float4(acc[t][b][0], acc[t][b][1], acc[t][b][2], acc[t][b][3]);
+}
+template <int NT, int NB, int WV>
+__device__ __forceinline__ void few_rows_sum(const float4* red, int t, int b, int lane, float (&v)[4]) {
+  v[0] = v[1] = v[2] = v[3] = 0.f;
+#pragma unroll
+  for (int w = 0; w < WV; ++w) {
+    const float4 p = red[(w * NT * NB + t * NB + b) * 64 + lane];
+    v[0] += p.x;
+    v[1] += p.y;
+    v[2] += p.z;
+    v[3] += p.w;
+  }
+}
+
+// ---------------------------------------------------------------------------------
+// one workgroup of WV waves per P tiles of 16 output columns (GLU: P tiles of the gate and the
+// same of the up matrix).
+// ---------------------------------------------------------------------------------
+template <int P, bool GLU, int NB, int WV, int U, typename TO>
+__global__ void __launch_bounds__(64 * WV)
+few_rows_gemm_kernel(TO* __restrict__ Y, long y_stride, const bf16_t* __restrict__ X, long x_stride, int rows,
+                     const bf16_t* __restrict__ W, const bf16_t* __restrict__ bias, int N, int K, int act, float limit,
+                     int vec) {
+  constexpr int NT = GLU ? 2 * P : P;
+  extern __shared__ float4 red[];                // few_rows_lds bytes: X stages, then partial sums
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n0 = blockIdx.x * 16 * P;
+  const bf16_t* wp[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) wp[t] = W + ((long)min(n0 + 16 * (t % P) + (lane & 15), N - 1) + (t / P) * (long)N) * K;
+  fr_f32x4 acc[NT][NB];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int b = 0; b < NB; ++b) acc[t][b] = fr_f32x4{0.f, 0.f, 0.f, 0.f};
+  few_rows_core<NT, NB, WV, U>(acc, wp, [&](int r) { return X + r * x_stride; }, rows, K,
+                               reinterpret_cast<char*>(red) + wave * kFrStage<NB, U>, wave, lane);
+  __syncthreads();
+  few_rows_park<NT, NB, WV>(red, acc, wave, lane);
+  __syncthreads();
+  // entry (tile, block, lane'): lane' = 16 q' + row, columns 4 q' .. 4 q' + 3
+  for (int e = tid; e < P * NB * 64; e += 64 * WV) {
+    const int el = e & 63, b = (e >> 6) % NB, t = (e >> 6) / NB;
+    const int r = 16 * b + (el & 15), c = n0 + 16 * t + 4 * (el >> 4);
+    if (r >= rows || c >= N) continue;
+    float v[4];
+    few_rows_sum<NT, NB, WV>(red, t, b, el, v);
+    if constexpr (GLU) {
+      float u[4];
+      few_rows_sum<NT, NB, WV>(red, t + P, b, el, u);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = fr_act(act, limit, v[i], u[i]);
+    } else {
+      if (bias != nullptr) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] += c + i < N ? ft::bf16_to_f32(bias[c + i]) : 0.f;
+      }
+      if (act == kFrReluSq) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = fr_act(act, limit, v[i], 0.f);
+      }
+    }
+    fr_store4(Y + r * y_stride, c, N, vec != 0, v);
+  }
+}
+
+// ---------------------------------------------------------------------------------
+// Experts of few rows.  A workgroup owns one tile of 16 (two) columns of one expert's matrix and
+// serves every row that chose the expert: the matrix is read once however many rows share it.
+// blockIdx.y: expert; == experts: the shared expert, which serves all rows.
+// Bound by the stream of the chosen experts' matrices.  32 rows, top 4 of 32 experts of 1536 (relu^2)
+// and a shared one: 44 + 50 us for 214 MB each, 4.9 and 4.3 TB/s, where one read per (row, choice)
+// took 105 + 101 us; 16 rows, top 6 of 32 gated experts of 1024: 54 + 30 us, before 112 + 54.
+// ---------------------------------------------------------------------------------
+struct ExpertSet {
+  const bf16_t* w;        // [experts][rows_w][K]
+  const bf16_t* shared;   // [shared rows][K_shared], or null
+  int experts, K, N;      // N: output columns (GLU: of gate and of up each)
+  int shared_K, shared_N;
+};
+
+// the (row, choice) pairs that chose expert e -> list, ascending; returns their number.  At most
+// one pair per row.  All threads of the workgroup call it.
+template <int WV>
+__device__ __forceinline__ int pairs_of(const int* __restrict__ idx, int pairs, int top, int experts, int e, int* list,
+                                        int* counts) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  int total = 0;
+  for (int p0 = 0; p0 < pairs; p0 += 64 * WV) {
+    const int p = p0 + tid;
+    int v = -1;
+    if (p < pairs) {
+      v = idx[p];
+      if (v < 0 || v >= experts) v = 0;
+    }
+    const uint64_t m = __ballot(v == e);
+    if (lane == 0) counts[wave] = __popcll(m);
+    __syncthreads();
+    int before = total;
+    for (int w = 0; w < WV; ++w) {
+      if (w < wave) before += counts[w];
+      total += counts[w];
+    }
+    if (v == e) {
+      const int at = before + __popcll(m & ((1ull << lane) - 1));
+      if (at < kFewRows) list[at] = p;
+    }
+    __syncthreads();
+  }
+  return min(total, kFewRows);
+}
+
+// the tile's sums for the listed rows: f(entry row in the list, column, sums, up sums)
+template <int P, bool GLU, int NB, int WV, int U, typename F>
+__device__ __forceinline__ void expert_tile(float4* red, const bf16_t* W, int N, int K, int n0, const bf16_t* X,
+                                            long x_stride, const int* list, int count, int div, int wave, int lane,
+                                            F out) {
+  constexpr int NT = GLU ? 2 * P : P;
+  const bf16_t* wp[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) wp[t] = W + ((long)min(n0 + 16 * (t % P) + (lane & 15), N - 1) + (t / P) * (long)N) * K;
+  fr_f32x4 acc[NT][NB];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int b = 0; b < NB; ++b) acc[t][b] = fr_f32x4{0.f, 0.f, 0.f, 0.f};
+  few_rows_core<NT, NB, WV, U>(acc, wp, [&](int r) { return X + (long)(list[r] / div) * x_stride; }, count, K,
+                               reinterpret_cast<char*>(red) + wave * kFrStage<NB, U>, wave, lane);
+  __syncthreads();
+  few_rows_park<NT, NB, WV>(red, acc, wave, lane);
+  __syncthreads();
+  for (int e = threadIdx.x; e < P * NB * 64; e += 64 * WV) {
+    const int el = e & 63, b = (e >> 6) % NB, t = (e >> 6) / NB;
+    const int r = 16 * b + (el & 15), c = n0 + 16 * t + 4 * (el >> 4);
+    if (r >= count || c >= N) continue;
+    float v[4], u[4] = {0.f, 0.f, 0.f, 0.f};
+    few_rows_sum<NT, NB, WV>(red, t, b, el, v);
+    if constexpr (GLU) few_rows_sum<NT, NB, WV>(red, t + P, b, el, u);
+    out(r, c, v, u);
+  }
+}
+
+// blocks of 16 rows that the listed rows fill, at most MB
+template <int P, bool GLU, int WV, int MB, typename F>
+__device__ __forceinline__ void expert_tile_any(float4* red, const bf16_t* W, int N, int K, int n0, const bf16_t* X,
+                                                long x_stride, const int* list, int count, int div, int wave, int lane,
+                                                F out) {
+  if (MB == 1 || count <= 16) expert_tile<P, GLU, 1, WV, 1>(red, W, N, K, n0, X, x_stride, list, count, div, wave, lane, out);
+  else if (MB == 2 || count <= 32) expert_tile<P, GLU, 2, WV, 1>(red, W, N, K, n0, X, x_stride, list, count, div, wave, lane, out);
+  else expert_tile<P, GLU, MB, WV, 1>(red, W, N, K, n0, X, x_stride, list, count, div, wave, lane, out);
+}
+
+// y[pair] = act(first matrices of the pair's expert times its row of h); ys[row] the same of the
+// shared expert; with a shared gate (one more row of its matrix) sg[row] = that row's product, by
+// the workgroup past the shared expert's last tile.
+constexpr int kExpWaves = 4;
+// X stages and partial sums (two tiles) of a tile with MB blocks of rows
+template <int MB>
+constexpr int kExpLds = kExpWaves * (kFrStage<MB, 1> > 2048 * MB ? kFrStage<MB, 1> : 2048 * MB);
+
+template <bool GLU, int MB>
+__global__ void __launch_bounds__(64 * kExpWaves)
+experts_first_kernel(bf16_t* __restrict__ y, bf16_t* __restrict__ ys, float* __restrict__ sg,
+                     const bf16_t* __restrict__ h, long h_stride, int rows, const int* __restrict__ idx, int top,
+                     ExpertSet E, int act, float limit, float shared_limit, int vec) {
+  constexpr int P = GLU ? 1 : 2;
+  __shared__ float4 red[kExpLds<MB> / 16];
+  __shared__ int list[kFewRows], counts[kExpWaves];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int e = blockIdx.y, n0 = blockIdx.x * 16 * P;
+  if (e < E.experts) {
+    if (n0 >= E.N) return;
+    const int count = pairs_of<kExpWaves>(idx, rows * top, top, E.experts, e, list, counts);
+    if (count == 0) return;
+    const bf16_t* W = E.w + (long)e * E.N * (GLU ? 2 : 1) * E.K;
+    expert_tile_any<P, GLU, kExpWaves, MB>(red, W, E.N, E.K, n0, h, h_stride, list, count, top, wave, lane,
+                                       [&](int r, int c, float (&v)[4], float (&u)[4]) {
+#pragma unroll
+                                         for (int i = 0; i < 4; ++i) v[i] = fr_act(act, limit, v[i], u[i]);
+                                         fr_store4(y + (long)list[r] * E.N, c, E.N, vec != 0, v);
+                                       });
+    return;
+  }
+  const int tiles = (E.shared_N + 16 * P - 1) / (16 * P);
+  if ((int)blockIdx.x > tiles || ((int)blockIdx.x == tiles && sg == nullptr)) return;
+  if (tid < rows) list[tid] = tid;
+  __syncthreads();
+  if ((int)blockIdx.x == tiles) {
+    const bf16_t* W = E.shared + (long)E.shared_N * (GLU ? 2 : 1) * E.K;
+    expert_tile_any<1, false, kExpWaves, MB>(red, W, 1, E.K, 0, h, h_stride, list, rows, 1, wave, lane,
+                                         [&](int r, int c, float (&v)[4], float (&)[4]) { if (c == 0) sg[r] = v[0]; });
+    return;
+  }
+  expert_tile_any<P, GLU, kExpWaves, MB>(red, E.shared, E.shared_N, E.K, n0, h, h_stride, list, rows, 1, wave, lane,
+                                     [&](int r, int c, float (&v)[4], float (&u)[4]) {
+#pragma unroll
+                                       for (int i = 0; i < 4; ++i) v[i] = fr_act(act, shared_limit, v[i], u[i]);
+                                       fr_store4(ys + (long)r * E.shared_N, c, E.shared_N, vec != 0, v);
+                                     });
+}
+
+// d[pair] = W_down of the pair's expert times y[pair], ds[row] the shared expert's, fp32
+template <int MB>
+__global__ void __launch_bounds__(64 * kExpWaves)
+experts_down_kernel(float* __restrict__ d, float* __restrict__ ds, const bf16_t* __restrict__ y,
+                    const bf16_t* __restrict__ ys, int rows, const int* __restrict__ idx, int top, ExpertSet E, int vec) {
+  constexpr int P = 2;
+  __shared__ float4 red[kExpLds<MB> / 16];
+  __shared__ int list[kFewRows], counts[kExpWaves];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int e = blockIdx.y, n0 = blockIdx.x * 16 * P;
+  float* dst = d;
+  const bf16_t *W = E.w + (long)e * E.N * E.K, *X = y;
+  int K = E.K, count = rows;
+  if (e < E.experts) {
+    count = pairs_of<kExpWaves>(idx, rows * top, top, E.experts, e, list, counts);
+    if (count == 0) return;
+  } else {
+    if (tid < rows) list[tid] = tid;
+    __syncthreads();
+    dst = ds;
+    W = E.shared;
+    X = ys;
+    K = E.shared_K;
+  }
+  expert_tile_any<P, false, kExpWaves, MB>(red, W, E.N, K, n0, X, K, list, count, 1, wave, lane,
+                                       [&](int r, int c, float (&v)[4], float (&)[4]) {
+                                         fr_store4(dst + (long)list[r] * E.N, c, E.N, vec != 0, v);
+                                       });
+}
+
+// out[row] = sum_k wts[row, k] d[row, k] + shared[row] * (sigmoid(sg[row]) or 1)
+__global__ void __launch_bounds__(256)
+experts_combine_kernel(float* __restrict__ out, const float* __restrict__ d, const float* __restrict__ wts,
+                       const float* __restrict__ ds, const float* __restrict__ sg, int top, int width) {
+  const long row = blockIdx.y;
+  const int c = blockIdx.x * 256 + threadIdx.x;
+  if (c >= width) return;
+  float v = 0.f;
+#pragma unroll 4
+  for (int k = 0; k < top; ++k) v += wts[row * top + k] * d[(row * top + k) * width + c];
+  if (ds != nullptr) v += ds[row * width + c] * (sg != nullptr ? sigmoidf_(sg[row]) : 1.f);
+  out[row * width + c] = v;
+}
+
+template <int P, bool GLU, int NB, int WV, int U, typename TO>
+int few_rows_launch(void* Y, long y_stride, const void* X, long x_stride, int rows, const void* W, const void* bias,
+                    int N, int K, int act, float limit, int vec, hipStream_t s) {
+  constexpr int NT = GLU ? 2 * P : P;
+  constexpr int kRed = WV * NT * NB * 1024, kX = WV * kFrStage<NB, U>, lds = kRed > kX ? kRed : kX;
+  auto kernel = few_rows_gemm_kernel<P, GLU, NB, WV, U, TO>;
+  if constexpr (lds > 64 * 1024) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (e != hipSuccess) return (int)e;
+  }
+  hipLaunchKernelGGL(kernel, dim3((unsigned)((N + 16 * P - 1) / (16 * P))), dim3(64 * WV), lds, s, (TO*)Y, y_stride,
+                     (const bf16_t*)X, x_stride, rows, (const bf16_t*)W, (const bf16_t*)bias, N, K, act, limit, vec);
+  return (int)hipGetLastError();
+}
+
+// Tiles per workgroup, waves and steps in flight, measured with weights that come from HBM (K = 2048
+// unless said; us at 1 / 16 / 32 / 64 rows, the vendor's product beside it):
+//   N = 2048 and 3072: 8 waves, two steps       5.3 5.9 7.0 8.6      (vendor 11.0 11.0 11.1 11.6)
+//   N = 2048, K = 8192                          11.6 13.8 18.0 24.6  (13.1 13.2 16.0 22.6)
+//   N = 10272: 4 waves, one step, more groups   11.8 11.7 14.8 22.1  (16.4 14.3 14.3 15.7)
+//   N = 32768: four tiles share an X fragment   26.9 27.7 29.0 34.2  (35.1 33.5 35.2 36.2; 24.0 at 5.6 TB/s)
+//   gated, 2 x 8192: 4 waves                    15.7 15.7 17.5 21.8  (18 + 5 for the activation)
+// Below 1024 columns of X a wave has one step or none: four waves.
+template <bool GLU, int NB, typename TO>
+int few_rows_pick(void* Y, long y_stride, const void* X, long x_stride, int rows, const void* W, const void* bias,
+                  int N, int K, int act, float limit, int vec, hipStream_t s) {
+#define FR_RUN(P, WV, U) \
+  few_rows_launch<P, GLU, NB, WV, U, TO>(Y, y_stride, X, x_stride, rows, W, bias, N, K, act, limit, vec, s)
+  if constexpr (GLU) {
+    return FR_RUN(1, 4, NB == 4 ? 2 : 1);
+  } else {
+    if (N >= 16384 || (NB == 4 && N > 4096)) return FR_RUN(4, 4, 1);
+    return N > 4096 || K < 1024 ? FR_RUN(1, 4, 1) : FR_RUN(1, 8, 2);
+  }
+#undef FR_RUN
+}
+
+}  // namespace mx
+
+using namespace mx;
+
+extern "C" int mx_few_rows_max() { return kFewRows; }
+
+extern "C" int mx_few_rows_gemm(void* Y, int y_f32, long y_stride, const void* X, long x_stride, int rows,
+                                const void* W, const void* bias, int N, int K, int act, float limit, hipStream_t s) {
+  if (rows <= 0 || N <= 0) return 0;
+  if (rows > kFewRows || K < 8 || K % 8 || x_stride % 8 || act < kFrStore || act > kFrReluSq) return -1;
+  if (((uintptr_t)X) % 16 || ((uintptr_t)W) % 16) return -2;
+  const bool glu = act >= kFrGelu && act <= kFrClamp;
+  if (glu && (bias != nullptr || y_f32)) return -3;
+  const int es = y_f32 ? 4 : 2;
+  const int vec = y_stride % 4 == 0 && ((uintptr_t)Y) % (4 * es) == 0;
+  const int nb = rows <= 16 ? 1 : rows <= 32 ? 2 : 4;
+#define FR_GO(GLU, TO)                                                                                               \
+  (nb == 1   ? few_rows_pick<GLU, 1, TO>(Y, y_stride, X, x_stride, rows, W, bias, N, K, act, limit, vec, s)          \
+   : nb == 2 ? few_rows_pick<GLU, 2, TO>(Y, y_stride, X, x_stride, rows, W, bias, N, K, act, limit, vec, s)          \
+             : few_rows_pick<GLU, 4, TO>(Y, y_stride, X, x_stride, rows, W, bias, N, K, act, limit, vec, s))
+  if (glu) return FR_GO(true, bf16_t);
+  return y_f32 ? FR_GO(false, float) : FR_GO(false, bf16_t);
+#undef FR_GO
+}
+
+extern "C" int mx_experts_few(float* out, void* y, float* d, const void* h, long h_stride, const int* idx,
+                              const float* wts, const void* wgu, const void* wdown, int rows, int top, int experts,
+                              int ff, int width, float limit, int act, void* ys, float* ds, float* sg,
+                              const void* shared_w, const void* shared_down, int shared_ff, float shared_limit,
+                              hipStream_t s) {
+  if (rows <= 0) return 0;
+  if (rows > kFewRows || experts < 1 || experts > 65534 || top < 1 || top > experts || ff % 8 || width % 8 ||
+      ff < 8 || width < 8 || h_stride % 8 || shared_ff % 8 || act < kFrGelu || act > kFrReluSq) return -1;
+  if (((uintptr_t)h) % 16 || ((uintptr_t)wgu) % 16 || ((uintptr_t)wdown) % 16 || ((uintptr_t)shared_w) % 16 ||
+      ((uintptr_t)shared_down) % 16) return -2;
+  const bool glu = act != kFrReluSq;
+  const int cols = glu ? 16 : 32;
+  const bool sh = shared_w != nullptr;
+  const int tiles = (ff + cols - 1) / cols, tiles_s = sh ? (shared_ff + cols - 1) / cols + (sg != nullptr) : 0;
+  ExpertSet first{(const bf16_t*)wgu, (const bf16_t*)shared_w, experts, width, ff, width, shared_ff};
+  const dim3 g1((unsigned)(tiles > tiles_s ? tiles : tiles_s), (unsigned)(experts + (sh ? 1 : 0))), block(64 * kExpWaves);
+  ExpertSet down{(const bf16_t*)wdown, (const bf16_t*)shared_down, experts, ff, width, shared_ff, width};
+  const dim3 g2((unsigned)((width + 31) / 32), g1.y);
+#define EX_FIRST(GLU, MB)                                                                                              \
+  hipLaunchKernelGGL((experts_first_kernel<GLU, MB>), g1, block, 0, s, (bf16_t*)y, (bf16_t*)ys, sg, (const bf16_t*)h, \
+                     h_stride, rows, idx, top, first, act, limit, shared_limit, 1)
+#define EX_GO(MB)                                                                                                   \
+  do {                                                                                                              \
+    if (glu) EX_FIRST(true, MB); else EX_FIRST(false, MB);                                                          \
+    hipLaunchKernelGGL((experts_down_kernel<MB>), g2, block, 0, s, d, ds, (const bf16_t*)y, (const bf16_t*)ys, rows, \
+                       idx, top, down, 1);                                                                          \
+  } while (0)
+  if (rows <= 16) EX_GO(1);
+  else if (rows <= 32) EX_GO(2);
+  else EX_GO(4);
+#undef EX_GO
+#undef EX_FIRST
+  hipLaunchKernelGGL(experts_combine_kernel, dim3((unsigned)((width + 255) / 256), (unsigned)rows), dim3(256), 0, s,
+                     out, d, wts, sh ? ds : nullptr, sg, top, width);
+  return (int)hipGetLastError();
+}

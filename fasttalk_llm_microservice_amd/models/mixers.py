@@ -13,9 +13,10 @@ what a token costs in pages.
 
 Each class takes its sizes and constants as constructor arguments and a ``get(name)``
 callable that returns a weight tensor ([out, in] for projections), so a model file only
-describes which sublayers it stacks.  Matrix products are vendor GEMMs (``F.linear`` /
-``torch.bmm``) in the compute dtype with fp32 accumulation; everything around them runs
-in the HIP kernels (GPU) or their PyTorch twins (CPU backend).
+describes which sublayers it stacks.  Matrix products of many rows are vendor GEMMs
+(``F.linear`` / ``torch.bmm``) in the compute dtype with fp32 accumulation, those of decode steps
+the few-rows kernels (``ops.mixers.linear``); everything around them runs in the HIP kernels
+(GPU) or their PyTorch twins (CPU backend).
 """
 from __future__ import annotations
 
@@ -118,12 +119,12 @@ class LatentAttention:
 
     def __call__(self, h, ctx: StepContext, cache) -> torch.Tensor:
         t = h.shape[0]
-        qd = F.linear(h, self.wqd)
+        qd = M.linear(h, self.wqd)
         q, dkv = qd[:, :self.n_first], qd[:, self.n_first:self.n_down]
         if self.wuq is not None:
             cq = M.latent_down_prep(q, self.dq_norm, dkv, self.dkv_norm, self.eps, self.table, self.rot_dims,
                                     ctx.positions, ctx.slot_mapping, cache, self.rank, self.interleaved)
-            q = F.linear(cq, self.wuq)
+            q = M.linear(cq, self.wuq)
         else:
             M.latent_kv_write(dkv, self.dkv_norm, self.eps, self.table, self.rot_dims, ctx.positions,
                               ctx.slot_mapping, cache, self.rank, self.interleaved)
@@ -143,9 +144,9 @@ class LatentAttention:
             ol = M.latent_attention(qa, qr, cache, seg, self.scale, self.rank, sink=self.sink)
         o = torch.bmm(ol, self.wuvT)                                  # [heads, T, vdim]
         if self.gated:
-            return F.linear(M.head_gate(o, qd[:, self.n_down:], self.dtype), self.wo)
+            return M.linear(M.head_gate(o, qd[:, self.n_down:], self.dtype), self.wo)
         o = o.transpose(0, 1).reshape(t, self.heads * self.dv).to(self.dtype)
-        return F.linear(o, self.wo)
+        return M.linear(o, self.wo)
 
 
 class ChannelDelta:
@@ -186,16 +187,16 @@ class ChannelDelta:
 
     def __call__(self, h, ctx: StepContext, state) -> torch.Tensor:
         s_rec, s_conv = state
-        qkv = F.linear(h, self.wqkv)
-        lo = F.linear(h, self.wlo)
-        a = F.linear(lo[:, :self.ra], self.wa2)
-        gp = F.linear(lo[:, self.ra:self.ra + self.rg], self.wg2)
+        qkv = M.linear(h, self.wqkv)
+        lo = M.linear(h, self.wlo)
+        a = M.linear(lo[:, :self.ra], self.wa2)
+        gp = M.linear(lo[:, self.ra:self.ra + self.rg], self.wg2)
         b = lo[:, self.ra + self.rg:].contiguous()
         qkv = M.short_conv_silu(qkv, self.conv_w, s_conv, ctx.seg)
         o = M.gated_delta_rule(qkv, a, b, self.a_log, self.dt_bias, s_rec, ctx.seg, self.heads,
                                self.kvh, self.dk, self.dv)
         y = M.head_rms_gate(o, self.norm, gp, self.eps, self.heads, self.dv, self.dtype)
-        return F.linear(y, self.wo)
+        return M.linear(y, self.wo)
 
 
 class HeadDelta:
@@ -235,14 +236,14 @@ class HeadDelta:
 
     def __call__(self, h, ctx: StepContext, state) -> torch.Tensor:
         s_rec, s_conv = state
-        p = F.linear(h, self.win)
+        p = M.linear(h, self.win)
         c, ng, nh = self.channels, self.heads * self.dv, self.heads
         q, k, v, lg, beta = M.conv_delta_prep(p[:, :c], p[:, c + ng:c + ng + nh], p[:, c + ng + nh:c + ng + 2 * nh],
                                               self.conv_w, s_conv, self.a_log, self.dt_bias, ctx.seg, nh, self.kvh,
                                               self.dk, self.dv)
         o = M.head_delta_rule(q, k, v, lg, beta, s_rec, ctx.seg)
         y = M.head_rms_gate(o, self.norm, p[:, c:c + ng], self.eps, nh, self.dv, self.dtype, silu=True)
-        return F.linear(y, self.wo)
+        return M.linear(y, self.wo)
 
 
 class WindowedAttention:
@@ -315,11 +316,11 @@ class SigmoidAttention(WindowedAttention):
             raise ValueError("attention norm / bias tensors do not fit the head sizes")
 
     def __call__(self, h, ctx: StepContext, cache) -> torch.Tensor:
-        qkv = F.linear(h, self.wqkv, self.bias)
+        qkv = M.linear(h, self.wqkv, self.bias)
         q = M.attn_prep(qkv, self.nq, self.nk, self.q_norm, self.k_norm, self.eps, None, 0, self.spec.dk,
                         ctx.positions, ctx.slot_mapping, cache[0], cache[1])
         o = self.attend(q, ctx, cache)
-        return F.linear(o.view(h.shape[0], -1).to(self.dtype), self.wo)
+        return M.linear(o.view(h.shape[0], -1).to(self.dtype), self.wo)
 
 
 class DifferentialAttention(WindowedAttention):
@@ -350,14 +351,14 @@ class DifferentialAttention(WindowedAttention):
             if rot_dims else None
 
     def __call__(self, h, ctx: StepContext, cache) -> torch.Tensor:
-        qkvg = F.linear(h, self.wqkv)
+        qkvg = M.linear(h, self.wqkv)
         n = self.nq + self.nk + self.nv
         q = M.attn_prep(qkvg[:, :n], self.nq, self.nk, None, None, self.eps, self.table, self.rot_dims,
                         self.spec.dk, ctx.positions, ctx.slot_mapping, cache[0], cache[1])
         a = self.attend(q, ctx, cache)
         o = M.diff_combine(a, qkvg[:, n:], self.lam, 1.0 - self.diff, self.eps, self.spec.heads,
                            self.spec.dv, self.dtype)
-        return F.linear(o, self.wo)
+        return M.linear(o, self.wo)
 
 
 class ConvSinkAttention(WindowedAttention):
@@ -411,7 +412,7 @@ class ConvSinkAttention(WindowedAttention):
         return self.attend(q, ctx, (kc, vc)).view(qkv.shape[0], -1)
 
     def __call__(self, h, ctx: StepContext, cache) -> torch.Tensor:
-        return F.linear(self.rows(F.linear(h, self.wqkv), ctx, cache).to(self.dtype), self.wo)
+        return M.linear(self.rows(M.linear(h, self.wqkv), ctx, cache).to(self.dtype), self.wo)
 
 
 class BiasedWindowAttention(WindowedAttention):
@@ -448,7 +449,7 @@ class BiasedWindowAttention(WindowedAttention):
         self.n_in = self.nq + own
 
     def __call__(self, h, ctx: StepContext, cache) -> torch.Tensor:
-        p = F.linear(h, self.wqkv)
+        p = M.linear(h, self.wqkv)
         if self.cache_of is not None:
             q = M.attn_prep(p[:, :self.nq], self.nq, 0, self.q_norm, None, self.eps, None, 0, self.spec.dk,
                             ctx.positions, ctx.slot_mapping, None, None)
@@ -456,7 +457,7 @@ class BiasedWindowAttention(WindowedAttention):
             q = M.attn_prep(p[:, :self.n_in], self.nq, self.nk, self.q_norm, self.k_norm, self.eps, None, 0,
                             self.spec.dk, ctx.positions, ctx.slot_mapping, cache[0], cache[1])
         o = self.attend(q, ctx, cache)
-        return F.linear(M.sigmoid_gate(o.view(h.shape[0], -1), p[:, self.n_in:], self.dtype), self.wo)
+        return M.linear(M.sigmoid_gate(o.view(h.shape[0], -1), p[:, self.n_in:], self.dtype), self.wo)
 
 
 class RotaryBlockAttention(WindowedAttention):
@@ -478,11 +479,11 @@ class RotaryBlockAttention(WindowedAttention):
         self.table = M.rope_table(max_pos, rot_dims, rot_base, device=device, ramp=rot_ramp) if rot_dims else None
 
     def __call__(self, h, ctx: StepContext, cache) -> torch.Tensor:
-        qkv = F.linear(h, self.wqkv)
+        qkv = M.linear(h, self.wqkv)
         q = M.attn_prep(qkv, self.nq, self.nk, None, None, self.eps, self.table, self.rot_dims, self.spec.dk,
                         ctx.positions, ctx.slot_mapping, cache[0], cache[1])
         o = self.attend(q, ctx, cache)
-        return F.linear(o.view(h.shape[0], -1).to(self.dtype), self.wo)
+        return M.linear(o.view(h.shape[0], -1).to(self.dtype), self.wo)
 
 
 class TalkingHeadsAttention:
@@ -533,7 +534,7 @@ class TalkingHeadsAttention:
     def __call__(self, h, ctx: StepContext, cache) -> torch.Tensor:
         kc, vc = cache
         seg = ctx.seg
-        p = F.linear(h, self.wqkg, self.bias)
+        p = M.linear(h, self.wqkg, self.bias)
         q = M.rot_norm_prep(p, self.nq, self.nk, self.spec.dk, self.table, self.rot_dims, self.eps, self.q_scale,
                             ctx.positions, ctx.slot_mapping, kc, vc)
         gate = p[:, self.nq + self.nk:]
@@ -545,7 +546,7 @@ class TalkingHeadsAttention:
         else:
             o = torch.empty(h.shape[0], self.nq, dtype=self.dtype, device=h.device)
             M.talk_attention(o, q, gate, kc, vc, seg, self.spec)
-        return F.linear(o, self.wo, self.bo)
+        return M.linear(o, self.wo, self.bo)
 
 
 class GatedLinearAttention:
@@ -579,12 +580,12 @@ class GatedLinearAttention:
         return _state_slots(((self.heads, self.dk, self.dv),), num_slots, device)[0]
 
     def __call__(self, h, ctx: StepContext, state) -> torch.Tensor:
-        p = F.linear(h, self.win)
-        a = F.linear(p[:, self.nqkv + self.ng:], self.wa2)
+        p = M.linear(h, self.win)
+        a = M.linear(p[:, self.nqkv + self.ng:], self.wa2)
         o = M.gated_linear_attention(p, a, self.a_bias, self.tau, state, ctx.seg, self.heads, self.dk, self.dv)
         y = M.head_rms_gate(o, self.norm, p[:, self.nqkv:self.nqkv + self.ng], self.eps, self.heads, self.dv,
                             self.dtype, silu=True)
-        return F.linear(y, self.wo)
+        return M.linear(y, self.wo)
 
 
 class Retention:
@@ -624,10 +625,10 @@ class Retention:
         return M.retention(p, self.table, self.rot_dims, self.log_decay, state, ctx.seg, self.heads, self.dk, self.dv)
 
     def __call__(self, h, ctx: StepContext, state) -> torch.Tensor:
-        p = F.linear(h, self.win)
+        p = M.linear(h, self.win)
         y = M.head_rms_gate(self.rows(p, ctx, state), self.unit, p[:, self.nqkv:], self.eps, self.heads, self.dv,
                             self.dtype, silu=True)
-        return F.linear(y, self.wo)
+        return M.linear(y, self.wo)
 
 
 class SideBySideSum:
@@ -652,13 +653,13 @@ class SideBySideSum:
                 self.right.alloc_cache(num_blocks, block_size, dtype, num_slots, device))
 
     def __call__(self, h, ctx: StepContext, cache) -> torch.Tensor:
-        p = F.linear(h, self.win)
+        p = M.linear(h, self.win)
         r = self.right
         pr = p[:, self.n_left:self.n_left + r.nqkv + r.ng]
         a = self.left.rows(p[:, :self.n_left], ctx, cache[0])
         o = r.rows(pr, ctx, cache[1])
         y = M.scaled_pair_rows(a, self.left_scale, o, pr[:, r.nqkv:], self.right_scale, r.eps, r.heads, r.dv, self.dtype)
-        return F.linear(y, self.wo)
+        return M.linear(y, self.wo)
 
 
 class SideBySide:
@@ -722,14 +723,14 @@ class StateSpaceMixer:
 
     def __call__(self, h, ctx: StepContext, state) -> torch.Tensor:
         s_rec, s_conv = state
-        p = F.linear(h, self.win)
+        p = M.linear(h, self.win)
         z = p[:, :self.inner]
         xbc = M.short_conv_silu(p[:, self.inner:self.inner + self.channels], self.conv_w, s_conv, ctx.seg,
                                 bias=self.conv_b)
         y = M.ssd_scan(xbc, p[:, self.inner + self.channels:], self.a_log, self.dt_bias, self.d_skip, s_rec,
                        ctx.seg, self.heads, self.groups, self.n, self.dv)
         y = M.gate_group_norm(y, z, self.norm, self.eps, self.norm_groups, self.dtype)
-        return F.linear(y, self.wo)
+        return M.linear(y, self.wo)
 
 
 class GatedFF:
@@ -737,15 +738,13 @@ class GatedFF:
     g = min(gate h, limit), u = clamp(up h, +-limit), down(g sigmoid(1.702 g) (u + 1))."""
 
     def __init__(self, get: Get, dtype, device, act: str = "gelu_tanh", limit: float = 0.0):
-        glu = {"gelu_tanh": M.gelu_glu, "relu": M.relu_glu, "silu": M.silu_glu,
-               "clamp_glu": lambda gu: M.clamp_swiglu(gu, float(limit))}
-        if act not in glu:
+        if act not in ("gelu_tanh", "relu", "silu", "clamp_glu"):
             raise ValueError("unknown feed-forward activation")
         self.wgu, self.down = _glu_weights(get, "", dtype, device)
-        self.glu = glu[act]
+        self.act, self.limit = act, float(limit)
 
     def __call__(self, h, ctx=None) -> torch.Tensor:
-        return F.linear(self.glu(F.linear(h, self.wgu)), self.down)
+        return M.linear(M.linear_act(h, self.wgu, self.act, self.limit), self.down)
 
 
 class DenseFF:
@@ -756,7 +755,7 @@ class DenseFF:
         self.down = get("down").to(device, dtype).contiguous()
 
     def __call__(self, h, ctx=None) -> torch.Tensor:
-        return F.linear(M.relu_sq(F.linear(h, self.up)), self.down)
+        return M.linear(M.linear_act(h, self.up, "relu_sq"), self.down)
 
 
 def _glu_weights(get: Get, prefix: str, dtype, device, extra: Optional[torch.Tensor] = None):
@@ -850,14 +849,19 @@ class MoEFF:
 
     def __call__(self, h, ctx=None) -> torch.Tensor:
         t, width = h.shape
+        if t <= self.PAIR_ROWS and M.experts_few_ok(h, self.wgu, self.wdown, self.shared):
+            # decode-size steps: a matrix is read once for all rows, nothing read back on the host
+            idx, wts = self.route(h)
+            return M.experts_few(h, idx, wts, self.wgu, self.wdown, self.act, self.limit, self.shared,
+                                 self.shared_limit if self.shared is not None else 0.0, self.shared_gate)
         if self.shared is not None and not self.shared_gate:
             # an ungated shared expert's output is what the chosen experts' are added to
-            out = F.linear(self._act(F.linear(h, self.shared[0]), self.shared_limit), self.shared[1]).float()
+            out = M.linear(self._act(M.linear(h, self.shared[0]), self.shared_limit), self.shared[1]).float()
         else:
             out = torch.zeros(t, width, dtype=torch.float32, device=h.device)
         idx, wts = self.route(h)
         if t <= self.PAIR_ROWS:
-            # decode-size steps: per-pair weight streaming, nothing read back on the host
+            # fp32 (or rows that are not whole 16-byte pieces): per-pair weight streaming
             M.moe_pairs(out, h, idx, wts, self.wgu, self.wdown, self.limit, self.act)
             return self._shared(out, h)
         # rows sorted by expert: each expert's rows are one group of two grouped products
@@ -875,19 +879,19 @@ class MoEFF:
         M.gather_add_rows(out, d, inv.view(t, self.top).int(), wts)
         return self._shared(out, h)
 
-    # rows up to which every (row, expert) pair streams its expert's weights (decode);
-    # above, rows are sorted by expert and run as grouped products
+    # rows up to which a step's experts stream their weights with nothing sorted (decode); above,
+    # rows are sorted by expert and run as grouped products
     PAIR_ROWS = 64
 
     def _shared(self, out, h):
         if self.shared is not None and self.shared_gate:
             w1, wdown = self.shared
-            u = F.linear(h, w1)
+            u = M.linear(h, w1)
             if self.act == "clamp_glu":
                 y = M.clamp_swiglu(u, self.shared_limit)
             else:
                 y = M.relu_sq_rows(u, u.shape[1] - 1)
-            M.scale_add_rows(out, F.linear(y, wdown), None, u[:, -1].contiguous(), sigmoid=True)
+            M.scale_add_rows(out, M.linear(y, wdown), None, u[:, -1].contiguous(), sigmoid=True)
         return out
 
 
@@ -902,5 +906,5 @@ class TokenSide:
         self.norm = get("norm").to(device, torch.float32)
 
     def __call__(self, xc, ctx: StepContext) -> torch.Tensor:
-        g = M.side_gate(F.linear(xc, self.gate), self.table, ctx.ids, self.col0, self.dim)
-        return F.linear(g, self.proj)
+        g = M.side_gate(M.linear(xc, self.gate), self.table, ctx.ids, self.col0, self.dim)
+        return M.linear(g, self.proj)

@@ -72,6 +72,70 @@ class Segments:
 
 
 # ---------------------------------------------------------------------------------
+# products with weights [out, in]
+# ---------------------------------------------------------------------------------
+
+# most rows of a product that streams its weights once through the few-rows kernel (a decode
+# step's; the vendor's tiles fill up beyond)
+FEW_ROWS = 64
+# activations of the few-rows kernels
+FEW_ACTS = {None: 0, "gelu_tanh": 1, "relu": 2, "silu": 3, "clamp_glu": 4, "relu_sq": 5, "silu_glu": 3}
+
+
+def _few_rows(x, w) -> bool:
+    """bf16 rows and weights of whole 16-byte pieces, at most FEW_ROWS rows, on a GPU."""
+    return bool(x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2
+                and 1 <= x.shape[0] <= FEW_ROWS and x.shape[1] % 8 == 0 and x.shape[1] >= 8 and x.stride(1) == 1
+                and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and w.is_contiguous())
+
+
+def _few_rows_pays(rows: int, n: int, k: int) -> bool:
+    """Where the few-rows kernel is at least level with the vendor's product (timings beside its
+    configurations in few_rows.hip): always up to 16 rows; above, long sums into few columns have
+    too few workgroups to hide reading X, and many rows against a middling number of columns
+    fill the vendor's tiles."""
+    if rows <= 16:
+        return True
+    if rows <= 32:
+        return k < 8192 or n > 4096
+    return n >= 16384 or (n <= 4096 and k <= 4096)
+
+
+def linear(x, w, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """x w^T (+ bias) in x's dtype, fp32 accumulation."""
+    if _few_rows(x, w) and _few_rows_pays(x.shape[0], w.shape[0], x.shape[1]):
+        y = torch.empty(x.shape[0], w.shape[0], dtype=x.dtype, device=x.device)
+        native_mixers().few_rows_gemm(y, x, w, bias, 0, 0.0)
+        return y
+    return torch.nn.functional.linear(x, w, bias)
+
+
+def linear_f32(x, w) -> torch.Tensor:
+    """x w^T with fp32 accumulation and fp32 output."""
+    if _few_rows(x, w) and _few_rows_pays(x.shape[0], w.shape[0], x.shape[1]):
+        y = torch.empty(x.shape[0], w.shape[0], dtype=torch.float32, device=x.device)
+        native_mixers().few_rows_gemm(y, x, w, None, 0, 0.0)
+        return y
+    return mm_f32(x, w.t())
+
+
+def linear_act(x, w, act: str, limit: float = 0.0) -> torch.Tensor:
+    """act of x w^T: w = [gate | up] rows for the gated forms ("gelu_tanh", "relu", "silu",
+    "clamp_glu" with ``limit``), one matrix for "relu_sq".  Few rows: one kernel, the products
+    stay fp32 up to the activation's result."""
+    if _few_rows(x, w):
+        n = w.shape[0] if act == "relu_sq" else w.shape[0] // 2
+        y = torch.empty(x.shape[0], n, dtype=x.dtype, device=x.device)
+        native_mixers().few_rows_gemm(y, x, w, None, FEW_ACTS[act], float(limit))
+        return y
+    u = torch.nn.functional.linear(x, w)
+    if act == "relu_sq":
+        return relu_sq(u)
+    return clamp_swiglu(u, limit) if act == "clamp_glu" else {"gelu_tanh": gelu_glu, "relu": relu_glu,
+                                                              "silu": silu_glu}[act](u)
+
+
+# ---------------------------------------------------------------------------------
 # residual stream (fp32) and norms
 # ---------------------------------------------------------------------------------
 
@@ -967,6 +1031,26 @@ def moe_pairs(out, h, idx, wts, wgu, wdown, limit: float = 0.0, act: str = "clam
         native_mixers().moe_pairs(out, h, idx, wts, wgu, wdown, float(limit), EXPERT_ACTS[act])
     else:
         ref.moe_pairs(out, h, idx, wts, wgu, wdown, limit, act)
+
+
+def experts_few_ok(h, wgu, wdown, shared) -> bool:
+    """Whether :func:`experts_few` takes these rows and weights (``shared``: the shared expert's two
+    matrices, or None)."""
+    ws = [wgu, wdown] + (list(shared) if shared is not None else [])
+    return bool(_few_rows(h, wgu) and all(w.dtype == torch.bfloat16 and w.shape[-1] % 8 == 0 and w.data_ptr() % 16 == 0
+                                          and w.is_contiguous() for w in ws))
+
+
+def experts_few(h, idx, wts, wgu, wdown, act: str, limit: float = 0.0, shared=None, shared_limit: float = 0.0,
+                shared_gate: bool = False) -> torch.Tensor:
+    """fp32 sum_k wts[:, k] * expert_{idx[:, k]}(h) (+ the shared expert, times the sigmoid of its
+    last row's product if ``shared_gate``), for few rows: every chosen expert's matrices are read
+    once for all rows that chose it.  No host round trip."""
+    out = torch.empty(h.shape, dtype=torch.float32, device=h.device)
+    native_mixers().experts_few(out, h, idx, wts, wgu, wdown, float(limit), FEW_ACTS[act],
+                                shared[0] if shared is not None else None,
+                                shared[1] if shared is not None else None, float(shared_limit), bool(shared_gate))
+    return out
 
 
 def clamp_swiglu(gu, limit: float):
