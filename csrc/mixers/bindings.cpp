@@ -165,6 +165,13 @@ int mx_moe_pairs(float* out, void* y, const void* h, int bf16, long h_stride, co
 int mx_moe_topk(int* idx, float* wts, const float* z, const float* corr, long rows, int experts, int top,
                 int groups, int keep, hipStream_t s);
 int mx_few_rows_max();
+int mx_band_attn_fits(int dk, int dv, int block_size);
+int mx_band_attn(float* out, const float* q, const void* k_cache, const void* v_cache, const int* start,
+                 const int* pos0, const int* kv_len, const int* bt, int bt_stride, int num_segs, int long_segs,
+                 long long_rows, int heads, int maps, int kv_heads, int dk, int dv, int window, float scale, int sigmoid,
+                 const float* r1, const float* r2, const float* pb, int block_size, int num_blocks, int min_rows,
+                 float softcap, int has_sink, float sink, const float* sinks, int blocks, int keep_first,
+                 const float* dist_bias, int nd, hipStream_t s);
 int mx_few_rows_gemm(void* Y, int y_f32, long y_stride, const void* X, long x_stride, int rows, const void* W,
                      const void* bias, int N, int K, int act, float limit, hipStream_t s);
 int mx_experts_few(float* out, void* y, float* d, const void* h, long h_stride, const int* idx, const float* wts,
@@ -1019,6 +1026,42 @@ void window_attention(Tensor out, Tensor q, Tensor k_cache, Tensor v_cache, Tens
       "window_attention");
 }
 
+void band_attention(Tensor out, Tensor q, Tensor k_cache, Tensor v_cache, Tensor start, Tensor pos0, Tensor kv_len,
+                    Tensor bt, int64_t num_segs, int64_t long_segs, int64_t long_rows, int64_t heads, int64_t maps,
+                    int64_t kv_heads, int64_t dk, int64_t dv, int64_t window, double scale, bool sigmoid, OptT r1,
+                    OptT r2, OptT pb, int64_t min_rows, double softcap, c10::optional<double> sink, OptT sinks,
+                    bool blocks, int64_t keep_first, OptT dist_bias) {
+  check_f32(out, "out");
+  check_f32(q, "q");
+  TORCH_CHECK(keep_first >= 0 && (!blocks || window >= 1) && min_rows >= 1, "band attention mask");
+  if (dist_bias) {
+    check_f32(*dist_bias, "distance bias");
+    TORCH_CHECK(dist_bias->dim() == 2 && dist_bias->size(0) >= 1 && dist_bias->size(1) == heads * maps,
+                "distance bias [distances, heads]");
+  }
+  TORCH_CHECK(heads >= 1 && maps >= 1 && kv_heads >= 1 && heads % kv_heads == 0, "band attention sizes");
+  const int64_t hq = heads * maps, t = q.size(0);
+  TORCH_CHECK(q.dim() == 2 && q.size(1) == hq * dk && out.numel() == t * hq * dv && long_rows <= t &&
+              long_segs <= num_segs, "q / out");
+  check_cache(k_cache, kv_heads * maps * dk, "k_cache");
+  check_cache(v_cache, kv_heads * dv, "v_cache");
+  TORCH_CHECK(k_cache.scalar_type() == at::kBFloat16 && v_cache.scalar_type() == at::kBFloat16 &&
+              k_cache.size(0) == v_cache.size(0) && k_cache.size(1) == v_cache.size(1), "k / v caches: bf16, alike");
+  check_segs(start, pos0, kv_len, num_segs);
+  check_i32(bt, "block tables");
+  TORCH_CHECK(bt.dim() == 2 && bt.size(0) >= num_segs, "block tables");
+  TORCH_CHECK((bool)r1 == (bool)r2, "r1 and r2 go together");
+  chk(mx_band_attn(out.data_ptr<float>(), q.data_ptr<float>(), k_cache.data_ptr(), v_cache.data_ptr(),
+                   start.data_ptr<int>(), pos0.data_ptr<int>(), kv_len.data_ptr<int>(), bt.data_ptr<int>(),
+                   (int)bt.size(1), (int)num_segs, (int)long_segs, long_rows, (int)heads, (int)maps, (int)kv_heads,
+                   (int)dk, (int)dv, (int)window, (float)scale, sigmoid ? 1 : 0, opt_f32(r1, hq, "r1"),
+                   opt_f32(r2, hq, "r2"), opt_f32(pb, hq, "pb"), (int)k_cache.size(1), (int)k_cache.size(0),
+                   (int)min_rows, (float)softcap, sink || sinks ? 1 : 0, sink ? (float)*sink : 0.f,
+                   opt_f32(sinks, hq, "sinks"), blocks ? 1 : 0, (int)keep_first,
+                   dist_bias ? dist_bias->data_ptr<float>() : nullptr, dist_bias ? (int)dist_bias->size(0) : 0,
+                   stream()), "band_attention");
+}
+
 void band_weights(Tensor S, int64_t rows, int64_t first_pos, int64_t key0, int64_t heads, int64_t maps,
                   int64_t kv_heads, int64_t window, double scale, bool sigmoid, OptT r1, OptT r2, OptT pb,
                   double softcap, c10::optional<double> sink, OptT sinks, bool blocks, int64_t keep_first,
@@ -1285,6 +1328,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("attn_prep", &attn_prep);
   m.def("window_attention", &window_attention);
   m.def("band_weights", &band_weights);
+  m.def("band_attention", &band_attention);
+  m.def("band_attention_fits", [](int64_t dk, int64_t dv, int64_t bs) {
+    return mx_band_attn_fits((int)dk, (int)dv, (int)bs) != 0;
+  });
   m.def("diff_combine", &diff_combine);
   m.def("ssd_scan", &ssd_scan);
   m.def("gate_group_norm", &gate_group_norm);

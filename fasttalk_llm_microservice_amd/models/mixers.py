@@ -288,7 +288,8 @@ class WindowedAttention:
         kc, vc = cache
         seg = ctx.seg
         if seg.host is not None and seg.max_rows >= self.PRODUCT_ROWS:
-            out = torch.zeros(q.shape[0], self.spec.heads * self.spec.maps, self.spec.dv,
+            # (every row belongs to a segment, short or long)
+            out = torch.empty(q.shape[0], self.spec.heads * self.spec.maps, self.spec.dv,
                               dtype=torch.float32, device=q.device)
             if min(b - a for a, b in zip(seg.host[0][:-1], seg.host[0][1:])) < self.PRODUCT_ROWS:
                 M.window_attention(q, kc, vc, seg, self.spec, skip_from=self.PRODUCT_ROWS, out=out)

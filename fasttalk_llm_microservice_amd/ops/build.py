@@ -151,6 +151,8 @@ def build_kernels(force: bool = False, jobs: int = 8, verbose: bool = True,
 
 
 MIXER_FLAGS = NO_PK_F32
+# per kernel file, as KERNEL_FLAGS: accumulators that the vector units rescale between products
+MIXER_KERNEL_FLAGS = {"band_attn": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
 
 
 def build_mixers(force: bool = False, jobs: int = 8, verbose: bool = True) -> Path:
@@ -165,7 +167,8 @@ def build_mixers(force: bool = False, jobs: int = 8, verbose: bool = True) -> Pa
         ["-DTORCH_EXTENSION_NAME=_C_mixers"]
     bflags = [HIPCC, f"--offload-arch={ARCH}"] + tflags + [f"-I{CSRC / 'include'}", f"-I{src}"] \
         + MIXER_FLAGS
-    jobs_list = [(k, bdir / (k.stem + ".o"), kflags, headers) for k in sorted(src.glob("*.hip"))]
+    jobs_list = [(k, bdir / (k.stem + ".o"), kflags + MIXER_KERNEL_FLAGS.get(k.stem, []), headers)
+                 for k in sorted(src.glob("*.hip"))]
     jobs_list.append((src / "bindings.cpp", bdir / "bindings.o", bflags + ["-x", "hip"], headers))
     changed = False
     with cf.ThreadPoolExecutor(max_workers=max(1, jobs)) as ex:

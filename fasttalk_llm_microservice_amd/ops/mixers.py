@@ -764,10 +764,21 @@ def window_attention_products(out, q, k_cache, v_cache, seg: Segments, spec: Win
     scores are one product with M = (query heads of the group) x rows, the weights come
     from :func:`band_weights` (fp32) and the sums are a second product with the value
     head.  Operands are fp32 (cached rows are widened), so scores, weights and sums are
-    true fp32.  Needs the segments' host copies; writes its rows of ``out``."""
+    true fp32.  bf16 caches whose heads fit its tiles run in one kernel for all segments instead
+    (csrc/mixers/band_attn.hip), to the same exactness.  Needs the segments' host copies; writes
+    its rows of ``out``."""
     sp = spec
     start, pos0, kv_len = seg.host
     bs = k_cache.shape[1]
+    if q.is_cuda and k_cache.dtype == torch.bfloat16 and native_mixers().band_attention_fits(sp.dk, sp.dv, bs):
+        # one kernel for all segments, scores never in memory
+        ns = [n for n in (b - a for a, b in zip(start[:-1], start[1:])) if n >= min_rows]
+        native_mixers().band_attention(out, q, k_cache, v_cache, seg.start, seg.pos0, seg.kv_len, seg.block_tables,
+                                       seg.num, len(ns), sum(ns), sp.heads, sp.maps, sp.kv_heads, sp.dk, sp.dv,
+                                       sp.window, float(sp.scale), bool(sp.sigmoid), sp.r1, sp.r2, sp.pb, min_rows,
+                                       float(sp.softcap), *_sink_args(sp.sink), bool(sp.blocks), int(sp.keep_first),
+                                       sp.dist_bias)
+        return out
     rep = sp.heads // sp.kv_heads
     gk = sp.kv_heads * sp.maps
     for s in range(seg.num):

@@ -1,0 +1,121 @@
+"""The one-pass attention of long segments (csrc/mixers/band_attn.hip) against the same attention in
+64 bits: every mask and score term, at the edges of its tiles (64 keys, 16 pairs a wave, 64 and 128 a
+workgroup), several segments with short ones among them.  Its error may not exceed that of the
+banded fp32 products it stands for."""
+import math
+
+import pytest
+import torch
+
+from fasttalk_llm_microservice_amd.ops import mixers as M
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def segments(lens, pos0, bs, g):
+    start = [0]
+    for n in lens:
+        start.append(start[-1] + n)
+    kv = [p + n for p, n in zip(pos0, lens)]
+    nb = [-(-k // bs) for k in kv]
+    perm = torch.randperm(sum(nb), generator=g).int()
+    bt = torch.zeros(len(lens), max(nb), dtype=torch.int32)
+    at = 0
+    for i, k in enumerate(nb):
+        bt[i, :k] = perm[at:at + k]
+        at += k
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)   # noqa: E731
+    return M.Segments(i32(start), i32(pos0), i32([0] * len(lens)), i32(kv), bt.to(DEV), len(lens), max(lens), max(kv),
+                      host=(start, list(pos0), kv)), sum(nb)
+
+
+def reference(q, kc, vc, seg, sp, min_rows):
+    out = torch.zeros(q.shape[0], sp.heads * sp.maps, sp.dv, dtype=torch.float64, device=DEV)
+    bs, rep, d64 = kc.shape[1], sp.heads // sp.kv_heads, torch.float64
+    par = lambda t: None if t is None else t.to(d64)   # noqa: E731
+    for s in range(seg.num):
+        a, b = seg.host[0][s], seg.host[0][s + 1]
+        if b - a < min_rows:
+            continue
+        p0, kv = seg.host[1][s], seg.host[2][s]
+        pages = seg.block_tables[s, :-(-kv // bs)].long()
+        k = kc[pages].reshape(-1, sp.kv_heads * sp.maps, sp.dk)[:kv].to(d64)
+        v = vc[pages].reshape(-1, sp.kv_heads, sp.dv)[:kv].to(d64)
+        i = torch.arange(p0, p0 + b - a, device=DEV)[:, None]
+        j = torch.arange(kv, device=DEV)[None]
+        seen = j <= i
+        if sp.window > 0:
+            near = (i // sp.window == j // sp.window) if sp.blocks else (i - j < sp.window)
+            seen = seen & (near | (j < sp.keep_first))
+        d = (i - j).clamp_min(0)
+        for h in range(sp.heads):
+            for m in range(sp.maps):
+                x = h * sp.maps + m
+                z = q[a:b].view(b - a, -1, sp.dk)[:, x].to(d64) @ k[:, h // rep * sp.maps + m].T * sp.scale
+                if sp.softcap:
+                    z = sp.softcap * torch.tanh(z / sp.softcap)
+                if sp.r1 is not None:
+                    z = z - par(sp.r1)[x] * torch.log1p(par(sp.r2)[x] * d)
+                if sp.dist_bias is not None:
+                    z = z + par(sp.dist_bias)[d.clamp_max(sp.dist_bias.shape[0] - 1), x]
+                if sp.sigmoid:
+                    w = torch.sigmoid(z + (par(sp.pb)[x] if sp.pb is not None else 0.0)) * seen
+                else:
+                    z = z.masked_fill(~seen, -math.inf)
+                    if sp.sink is not None:
+                        sk = par(sp.sink)[x] if isinstance(sp.sink, torch.Tensor) else torch.tensor(sp.sink, dtype=d64, device=DEV)
+                        z = torch.cat([z, sk.expand(b - a, 1)], 1)
+                    w = torch.softmax(z, -1)[:, :kv]
+                out[a:b, x] = w @ v[:, h // rep]
+    return out
+
+
+def cases():
+    f = lambda *s: dict(zip(("heads", "kv_heads", "dk", "dv", "window"), s))   # noqa: E731
+    yield "causal", f(4, 1, 128, 128, 0), {}, [64], [0]
+    yield "causal, cap, sink 0", f(4, 2, 128, 128, 0), dict(softcap=30.0, sink=0.0), [200, 5, 33], [0, 7, 100]
+    yield "window", f(3, 1, 64, 128, 100), {}, [65, 130], [0, 301]
+    yield "window, kept, table", f(4, 2, 128, 128, 70), dict(keep_first=9, table=90), [300, 32], [0, 511]
+    yield "window, kept beyond a tile", f(2, 2, 64, 64, 40), dict(keep_first=130), [257], [64]
+    yield "blocks", f(4, 1, 128, 64, 96), dict(blocks=True), [191, 97], [95, 0]
+    yield "two maps", f(4, 2, 64, 128, 128), dict(maps=2), [129, 63], [0, 1000]
+    yield "sigmoid, distance", f(2, 1, 128, 128, 150), dict(sigmoid=True, terms=True), [260], [31]
+    yield "sink per head, one key head each", f(2, 2, 128, 128, 33), dict(sinks=True), [32, 70], [0, 640]
+    yield "many pairs (eight waves)", f(16, 4, 128, 128, 0), dict(softcap=20.0), [1024], [0]
+    yield "three heads a group, many pairs", f(48, 16, 64, 64, 256), {}, [700, 400], [0, 90]
+
+
+@pytest.mark.parametrize("name,sizes,opt,lens,pos0", list(cases()), ids=[c[0] for c in cases()])
+@pytest.mark.parametrize("bs", [4, 16])
+def test_against_64_bits(name, sizes, opt, lens, pos0, bs, monkeypatch):
+    g = torch.Generator().manual_seed(len(name) * 10 + bs)
+    rnd = lambda *s: torch.randn(*s, generator=g)   # noqa: E731
+    opt = dict(opt)
+    hq = sizes["heads"] * opt.get("maps", 1)
+    table, terms, sinks = opt.pop("table", 0), opt.pop("terms", False), opt.pop("sinks", False)
+    extra = {}
+    if table:
+        extra["dist_bias"] = (0.5 * rnd(table, hq)).to(DEV)
+    if terms:
+        extra.update({k: torch.rand(hq, generator=g).to(DEV) for k in ("r1", "r2", "pb")})
+    if sinks:
+        extra["sink"] = rnd(hq).to(DEV)
+    sp = M.WindowSpec(scale=sizes["dk"] ** -0.5, **sizes, **opt, **extra)
+    seg, blocks = segments(lens, pos0, bs, g)
+    kc = rnd(blocks, bs, sp.kv_heads * sp.maps * sp.dk).to(DEV, torch.bfloat16)
+    vc = rnd(blocks, bs, sp.kv_heads * sp.dv).to(DEV, torch.bfloat16)
+    q = (2.0 * rnd(sum(lens), hq * sp.dk)).to(DEV)
+    want = reference(q, kc, vc, seg, sp, 32)
+    out = torch.full((q.shape[0], hq, sp.dv), 7.0, device=DEV)
+    got = M.window_attention_products(out, q, kc, vc, seg, sp, 32)
+    rows = torch.cat([torch.full((n,), n >= 32) for n in lens]).to(DEV)
+    assert bool((got[~rows] == 7.0).all())                     # short segments are not this path's
+    # the same attention as fp32 products on widened caches (another path of the same function)
+    old = M.window_attention_products(torch.zeros_like(out), q, kc.float(), vc.float(), seg, sp, 32)
+    norm = float(want[rows].norm())
+    e_new, e_old = (float((x.double() - want)[rows].norm()) / norm for x in (got, old))
+    # fp32 sums of a few hundred terms: about 2^-22; no further from 64 bits than the products
+    assert e_new < 1e-6 and e_new < 1.5 * e_old + 1e-7, (e_new, e_old)
+    again = M.window_attention_products(torch.zeros_like(out), q, kc, vc, seg, sp, 32)
+    assert torch.equal(again[rows], got[rows])
