@@ -112,7 +112,11 @@ int mx_ssd_max_state();
 int mx_ssd_scan(float* y, const void* xbc, int bf16, long x_stride, const void* dt, long dt_stride,
                 const float* a_log, const float* dt_bias, const float* d_skip, float* state, const int* start,
                 const int* pos0, const int* slot, int num_segs, int heads, int groups, int n, int dv, int num_slots,
-                hipStream_t s);
+                int skip_from, hipStream_t s);
+int mx_ssd_chunks(float* y, const void* xbc, int bf16, long stride, const void* dt, long dt_stride, const float* a_log,
+                  const float* dt_bias, const float* d_skip, float* state, float* ws_s, float* ws_g, float* ws_h,
+                  long rows, const int* start, const int* pos0, const int* slot, int num_segs, int max_rows, int heads,
+                  int groups, int n, int dv, int num_slots, int min_rows, hipStream_t s);
 int mx_gate_group_norm(void* out, int out_bf16, const float* y, const void* z, int z_bf16, long z_stride,
                        const float* w, long rows, int groups, int gs, float eps, hipStream_t s);
 int mx_add_rms_norm(float* x, const void* y, int y_bf16, long y_stride, const float* wb, const float* add_vec,
@@ -1100,8 +1104,8 @@ void diff_combine(Tensor out, Tensor a, Tensor gate, double lam, double post, do
 }
 
 void ssd_scan(Tensor y, Tensor xbc, Tensor dt, Tensor a_log, Tensor dt_bias, Tensor d_skip, Tensor state,
-              Tensor start, Tensor pos0, Tensor slot, int64_t num_segs, int64_t heads, int64_t groups, int64_t n,
-              int64_t dv) {
+              Tensor start, Tensor pos0, Tensor slot, int64_t num_segs, int64_t max_rows, int64_t heads, int64_t groups,
+              int64_t n, int64_t dv, bool walk, int64_t chunk_from) {
   check_f32(y, "y");
   check_rows(xbc, "xbc");
   check_rows(dt, "dt");
@@ -1117,10 +1121,24 @@ void ssd_scan(Tensor y, Tensor xbc, Tensor dt, Tensor a_log, Tensor dt_bias, Ten
               d_skip.numel() == heads && y.numel() == t * heads * dv, "state-space shapes");
   TORCH_CHECK(state.dim() == 4 && state.size(1) == heads && state.size(2) == n && state.size(3) == dv, "state");
   check_segs(start, pos0, slot, num_segs);
-  chk(mx_ssd_scan(y.data_ptr<float>(), xbc.data_ptr(), bf(xbc), xbc.stride(0), dt.data_ptr(), dt.stride(0),
-                  a_log.data_ptr<float>(), dt_bias.data_ptr<float>(), d_skip.data_ptr<float>(),
-                  state.data_ptr<float>(), start.data_ptr<int>(), pos0.data_ptr<int>(), slot.data_ptr<int>(),
-                  (int)num_segs, (int)heads, (int)groups, (int)n, (int)dv, (int)state.size(0), stream()), "ssd_scan");
+  TORCH_CHECK(max_rows <= t && chunk_from >= 1, "state-space rows");
+  const bool chunks = max_rows >= chunk_from && n <= mx_chunk_max_dk();
+  if (walk || !chunks)
+    chk(mx_ssd_scan(y.data_ptr<float>(), xbc.data_ptr(), bf(xbc), xbc.stride(0), dt.data_ptr(), dt.stride(0),
+                    a_log.data_ptr<float>(), dt_bias.data_ptr<float>(), d_skip.data_ptr<float>(),
+                    state.data_ptr<float>(), start.data_ptr<int>(), pos0.data_ptr<int>(), slot.data_ptr<int>(),
+                    (int)num_segs, (int)heads, (int)groups, (int)n, (int)dv, (int)state.size(0),
+                    chunks ? (int)chunk_from : 0, stream()), "ssd_scan");
+  if (!chunks) return;
+  const int64_t nc = chunk_bound(t, num_segs);
+  Tensor ws_s = at::empty({nc, heads, n, dv}, y.options()), ws_g = at::empty({nc, heads}, y.options());
+  Tensor ws_h = at::empty({2, t, heads}, y.options());
+  chk(mx_ssd_chunks(y.data_ptr<float>(), xbc.data_ptr(), bf(xbc), xbc.stride(0), dt.data_ptr(), dt.stride(0),
+                    a_log.data_ptr<float>(), dt_bias.data_ptr<float>(), d_skip.data_ptr<float>(),
+                    state.data_ptr<float>(), ws_s.data_ptr<float>(), ws_g.data_ptr<float>(), ws_h.data_ptr<float>(), t,
+                    start.data_ptr<int>(), pos0.data_ptr<int>(), slot.data_ptr<int>(), (int)num_segs, (int)max_rows,
+                    (int)heads, (int)groups, (int)n, (int)dv, (int)state.size(0), (int)chunk_from, stream()),
+      "state-space chunks");
 }
 
 void gate_group_norm(Tensor out, Tensor y, Tensor z, Tensor w, double eps, int64_t groups) {

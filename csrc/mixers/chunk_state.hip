@@ -1,5 +1,5 @@
-// Recurrences with one decay per head, long segments: the gated delta rule and retention in
-// chunk form, as fp32 matrix products (v_mfma_f32_16x16x4_f32) over chunks of 64 rows, so
+// Recurrences with one decay per head, long segments: the gated delta rule, retention and the selective
+// state-space scan (a retention whose decay changes by row) in chunk form, as fp32 matrix products (v_mfma_f32_16x16x4_f32) over chunks of 64 rows, so
 // that only one small step per chunk is sequential.
 //
 // With the rows of a chunk t = 0 .. 63, their log decays l_t, G_t = l_0 + .. + l_t and the
@@ -19,8 +19,8 @@
 //   delta_carry   per (head, 16 columns of the state), chunk after chunk: the state stays in the
 //                 accumulators of four waves (16-row tiles dealt out), whose register layout is
 //                 that of a right-hand operand; leaves w and every chunk's incoming state
-//   state_add     retention, per (chunk, head), parallel: a chunk's own contribution to the state
-//   state_carry   retention: elementwise scan over the chunks
+//   state_add     retention, state space, per (chunk, head), parallel: a chunk's own contribution to the state
+//   state_carry   retention, state space: elementwise scan over the chunks
 //   chunk_out     both, per (chunk, head, 64 columns), parallel: o from the incoming state
 // Sums of log decays are formed in double precision and only their differences are rounded, so
 // a chunk's decay ratios are as exact as a row-by-row walk's.
@@ -73,6 +73,8 @@ struct ChunkIn {
   int table_rows, rot_dims, interleaved;
   float k_scale;
   int v_frags;                         // v: fragments by workspace chunk (below) instead of rows
+  const float* v_scale;                // factor of each row of v in the state [T, heads], null: 1
+  const float* skip;                   // o += skip[h] v, null: none
 };
 
 // four consecutive entries as fp32 (16- or 8-byte load)
@@ -162,6 +164,12 @@ __device__ __forceinline__ void stage_log_decay(double* G, const ChunkIn& in, lo
   G[t] = l;
 }
 
+// rs[t] = the factor of row t of v (0 past cnt: v counts as zeros there)
+__device__ __forceinline__ void stage_row_scale(float* rs, const ChunkIn& in, long row0, int cnt, int heads, int h) {
+  const int t = threadIdx.x;
+  if (t < kC) rs[t] = t >= cnt ? 0.f : in.v_scale != nullptr ? in.v_scale[(row0 + t) * heads + h] : 1.f;
+}
+
 // the chunk of this workgroup: false if the segment has no such chunk (or is left to the walk)
 struct Chunk {
   int cnt, num, pos, slot;
@@ -183,33 +191,38 @@ __device__ __forceinline__ bool find_chunk(Chunk& c, int idx, int s, const int* 
 
 // ---------------------------------------------------------------------------------
 // grid (chunks, heads * ceil(dv / 64), segments): L = sum_j e^{G_last - G_j} k_j v_j^T into the
-// chunk's workspace [dk, dv].  Wave w: columns 16 w .. 16 w + 15 of the 64, all rows.
+// chunk's workspace [dk, dv] (v times its row factor); totals[chunk, head] = e^{G_last} if wanted.
+// Wave w: columns 16 w .. 16 w + 15 of the 64, all rows.
 // ---------------------------------------------------------------------------------
 template <typename T, int DKT>
 __global__ void __launch_bounds__(256)
-state_add_kernel(float* __restrict__ ws_s, ChunkIn in, const int* __restrict__ start, const int* __restrict__ pos0,
-                 const int* __restrict__ slot, int heads, int dk, int dv, int num_slots, int min_rows, int vec) {
+state_add_kernel(float* __restrict__ ws_s, float* __restrict__ totals, ChunkIn in, const int* __restrict__ start,
+                 const int* __restrict__ pos0, const int* __restrict__ slot, int heads, int dk, int dv, int num_slots,
+                 int min_rows, int vec) {
   constexpr int DKP = 16 * DKT, LDK = DKP + 16;
   __shared__ __attribute__((aligned(16))) float kb[kC * LDK], vb[kC * kVLD];
   __shared__ double G[kC];
+  __shared__ float rs[kC];
   Chunk c;
   if (!find_chunk(c, blockIdx.x, blockIdx.z, start, pos0, slot, min_rows, num_slots)) return;
   const int vt = (dv + 63) / 64;
   const int h = blockIdx.y / vt, col0 = blockIdx.y % vt * 64;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, lo = lane & 15, hi = lane >> 4;
   stage_log_decay(G, in, c.row0, c.cnt, heads, h);
+  stage_row_scale(rs, in, c.row0, c.cnt, heads, h);
   stage_head<T, DKP>(kb, LDK, (const T*)in.k + c.row0 * in.k_stride + (long)(h / in.rep) * dk, in.k_stride, c.cnt, dk,
                      in.table, in.table_rows, in.rot_dims, in.interleaved, c.pos, in.k_scale, vec);
   stage_cols<T>(vb, (const T*)in.v + c.row0 * in.v_stride + (long)h * dv, in.v_stride, c.cnt, col0, dv, vec);
   __syncthreads();
   const double gl = G[kC - 1];
+  if (totals != nullptr && col0 == 0 && tid == 0) totals[c.ws * heads + h] = expf((float)gl);
   f32x4 acc[DKT];
 #pragma unroll
   for (int i = 0; i < DKT; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 4
   for (int s = 0; s < kC / 4; ++s) {
     const int j = 4 * s + hi;
-    const float b = vb[j * kVLD + 16 * wave + lo] * expf((float)(gl - G[j]));
+    const float b = vb[j * kVLD + 16 * wave + lo] * (expf((float)(gl - G[j])) * rs[j]);
 #pragma unroll
     for (int i = 0; i < DKT; ++i) acc[i] = mma(kb[j * LDK + 16 * i + lo], b, acc[i]);
   }
@@ -226,11 +239,12 @@ state_add_kernel(float* __restrict__ ws_s, ChunkIn in, const int* __restrict__ s
 }
 
 // grid (ceil(dk dv / 256), heads, segments): workspaces hold every chunk's own contribution L_c
-// and become its incoming state; the last one goes to the slot
+// and become its incoming state; the last one goes to the slot.  A chunk's decay: totals[chunk, head],
+// or the head's fixed one per row.
 __global__ void __launch_bounds__(256)
-state_carry_kernel(float* __restrict__ ws_s, const double* __restrict__ log_decay, float* __restrict__ state,
-                   const int* __restrict__ start, const int* __restrict__ pos0, const int* __restrict__ slot, int heads,
-                   int size, int num_slots, int min_rows) {
+state_carry_kernel(float* __restrict__ ws_s, const double* __restrict__ log_decay, const float* __restrict__ totals,
+                   float* __restrict__ state, const int* __restrict__ start, const int* __restrict__ pos0,
+                   const int* __restrict__ slot, int heads, int size, int num_slots, int min_rows) {
   Chunk c;
   if (!find_chunk(c, 0, blockIdx.z, start, pos0, slot, min_rows, num_slots)) return;
   const int h = blockIdx.y, e = blockIdx.x * 256 + threadIdx.x;
@@ -238,19 +252,26 @@ state_carry_kernel(float* __restrict__ ws_s, const double* __restrict__ log_deca
   const int n = start[blockIdx.z + 1] - start[blockIdx.z];
   float* sp = state + ((long)c.slot * heads + h) * size + e;
   float S = c.pos > 0 ? *sp : 0.f;
-  const float full = (float)exp(log_decay[h] * kC), last = (float)exp(log_decay[h] * (n - (c.num - 1) * kC));
+  float full = 0.f, last = 0.f;
+  if (totals == nullptr) {
+    full = (float)exp(log_decay[h] * kC);
+    last = (float)exp(log_decay[h] * (n - (c.num - 1) * kC));
+  }
   float* w = ws_s + (c.ws * heads + h) * (long)size + e;
   const long step = (long)heads * size;
   constexpr int AHEAD = 8;            // contributions in flight
   for (int i0 = 0; i0 < c.num; i0 += AHEAD) {
-    float l[AHEAD];
+    float l[AHEAD], g[AHEAD];
 #pragma unroll
-    for (int u = 0; u < AHEAD; ++u) l[u] = i0 + u < c.num ? w[(i0 + u) * step] : 0.f;
+    for (int u = 0; u < AHEAD; ++u) {
+      l[u] = i0 + u < c.num ? w[(i0 + u) * step] : 0.f;
+      g[u] = totals == nullptr ? (i0 + u + 1 < c.num ? full : last) : totals[(c.ws + min(i0 + u, c.num - 1)) * heads + h];
+    }
 #pragma unroll
     for (int u = 0; u < AHEAD; ++u) {
       if (i0 + u < c.num) {
         w[(i0 + u) * step] = S;
-        S = (i0 + u + 1 < c.num ? full : last) * S + l[u];
+        S = g[u] * S + l[u];
       }
     }
   }
@@ -270,6 +291,7 @@ chunk_out_kernel(float* __restrict__ o, ChunkIn in, const float* __restrict__ ws
   constexpr int KB = kC * LDK > 64 * kPLD ? kC * LDK : 64 * kPLD;
   __shared__ __attribute__((aligned(16))) float kb[KB], vb[kC * kVLD];
   __shared__ double G[kC];
+  __shared__ float rs[kC];
   const int vt = (dv + 63) / 64;
   const int h = blockIdx.y / vt, col0 = blockIdx.y % vt * 64;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, lo = lane & 15, hi = lane >> 4;
@@ -287,6 +309,7 @@ chunk_out_kernel(float* __restrict__ o, ChunkIn in, const float* __restrict__ ws
   const long hoff = (long)(h / in.rep) * dk;
   const float* S = ws_s + ((c.ws * heads + h) * dk) * (long)dv;
   stage_log_decay(G, in, c.row0, c.cnt, heads, h);
+  stage_row_scale(rs, in, c.row0, c.cnt, heads, h);
   stage_head<T, DKP>(kb, LDK, (const T*)in.q + c.row0 * in.q_stride + hoff, in.q_stride, c.cnt, dk, in.table,
                      in.table_rows, in.rot_dims, in.interleaved, c.pos, 1.f, vec);
   const int svec = dv % 4 == 0;
@@ -346,9 +369,10 @@ chunk_out_kernel(float* __restrict__ o, ChunkIn in, const float* __restrict__ ws
     const float* kr = kb + (16 * jt + lo) * LDK + hi;
     f32x4 a = dot_steps<4 * DKT>([&](int s) { return qf[s]; }, [&](int s) { return kr[4 * s]; });
     const double gj = G[16 * jt + lo];
+    const float rj = rs[16 * jt + lo];
 #pragma unroll
     for (int r = 0; r < 4; ++r)
-      a[r] = 16 * jt + lo <= 16 * wave + 4 * hi + r ? a[r] * expf((float)(gr[r] - gj)) : 0.f;
+      a[r] = 16 * jt + lo <= 16 * wave + 4 * hi + r ? a[r] * expf((float)(gr[r] - gj)) * rj : 0.f;
     P[jt] = a;
   }
   __syncthreads();                                           // kb becomes four [16][64] strips
@@ -375,9 +399,11 @@ chunk_out_kernel(float* __restrict__ o, ChunkIn in, const float* __restrict__ ws
     const int t = 16 * wave + 4 * hi + r;
     if (t >= c.cnt) continue;
     float* op = o + ((c.row0 + t) * heads + h) * dv;
+    const float sk = in.skip != nullptr ? in.skip[h] : 0.f;
 #pragma unroll
     for (int ct = 0; ct < 4; ++ct)
-      if (col0 + 16 * ct + lo < dv) op[col0 + 16 * ct + lo] = O[ct][r];
+      if (col0 + 16 * ct + lo < dv)
+        op[col0 + 16 * ct + lo] = in.skip != nullptr ? O[ct][r] + sk * vb[t * kVLD + 16 * ct + lo] : O[ct][r];
   }
 }
 
@@ -707,12 +733,62 @@ extern "C" int mx_retention_chunks(float* o, const void* p, int bf16, long strid
   const dim3 grid((max_rows + kC - 1) / kC, heads * ((dv + 63) / 64), num_segs);
   if (grid.y > 65535 || grid.z > 65535) return -2;
   MX_DISPATCH_T(bf16, key_tiles(dk, [&](auto t) {
-    hipLaunchKernelGGL((state_add_kernel<T, decltype(t)::value>), grid, dim3(256), 0, s, ws_s, in, start, pos0, slot,
-                       heads, dk, dv, num_slots, min_rows, vec);
+    hipLaunchKernelGGL((state_add_kernel<T, decltype(t)::value>), grid, dim3(256), 0, s, ws_s, nullptr, in, start, pos0,
+                       slot, heads, dk, dv, num_slots, min_rows, vec);
   }));
   hipLaunchKernelGGL(state_carry_kernel, dim3((dk * dv + 255) / 256, heads, num_segs), dim3(256), 0, s, ws_s, log_decay,
-                     state, start, pos0, slot, heads, dk * dv, num_slots, min_rows);
+                     nullptr, state, start, pos0, slot, heads, dk * dv, num_slots, min_rows);
   MX_DISPATCH_T(bf16, (launch_out<T>(o, in, ws_s, start, pos0, slot, grid, heads, dk, dv, num_slots, min_rows, vec, s)));
+  return (int)hipGetLastError();
+}
+
+// step = softplus(dt + dt_bias) and the log decay -exp(a_log) step of every row and head
+template <typename T>
+__global__ void ssd_steps_kernel(float* __restrict__ step, float* __restrict__ lg, const T* __restrict__ dt,
+                                 long dt_stride, const float* __restrict__ a_log, const float* __restrict__ dt_bias,
+                                 long rows, int heads) {
+  const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= rows * heads) return;
+  const long row = e / heads;
+  const int h = (int)(e % heads);
+  const float v = softplusf_(ld(dt, row * dt_stride + h) + dt_bias[h]);
+  step[e] = v;
+  lg[e] = -expf(a_log[h]) * v;
+}
+
+// The selective state-space scan's long segments: q = C and k = B (one per group of heads), v = x times
+// its step, a decay per row and head, o += D x.  ws_h: 2 rows * heads floats (steps, log decays).
+extern "C" int mx_ssd_chunks(float* y, const void* xbc, int bf16, long stride, const void* dt, long dt_stride,
+                             const float* a_log, const float* dt_bias, const float* d_skip, float* state, float* ws_s,
+                             float* ws_g, float* ws_h, long rows, const int* start, const int* pos0, const int* slot,
+                             int num_segs, int max_rows, int heads, int groups, int n, int dv, int num_slots,
+                             int min_rows, hipStream_t s) {
+  if (num_segs <= 0 || max_rows < min_rows || rows <= 0) return 0;
+  if (n < 1 || n > mx_chunk_max_dk() || dv < 1 || groups < 1 || heads % groups || min_rows < 1) return -1;
+  const long es = bf16 ? 2 : 4;
+  ChunkIn in{};
+  in.v = xbc;
+  in.k = (const char*)xbc + es * heads * dv;
+  in.q = (const char*)xbc + es * ((long)heads * dv + (long)groups * n);
+  in.q_stride = in.k_stride = in.v_stride = stride;
+  in.rep = heads / groups;
+  in.v_scale = ws_h;
+  in.lg = ws_h + rows * heads;
+  in.skip = d_skip;
+  in.k_scale = 1.f;
+  const int vec = n % 4 == 0 && dv % 4 == 0 && stride % 4 == 0 && ((uintptr_t)xbc) % (4 * es) == 0;
+  const dim3 grid((max_rows + kC - 1) / kC, heads * ((dv + 63) / 64), num_segs);
+  if (grid.y > 65535 || grid.z > 65535) return -2;
+  MX_DISPATCH_T(bf16, hipLaunchKernelGGL((ssd_steps_kernel<T>), dim3((unsigned)((rows * heads + 255) / 256)), dim3(256),
+                                         0, s, ws_h, ws_h + rows * heads, (const T*)dt, dt_stride, a_log, dt_bias, rows,
+                                         heads));
+  MX_DISPATCH_T(bf16, key_tiles(n, [&](auto t) {
+    hipLaunchKernelGGL((state_add_kernel<T, decltype(t)::value>), grid, dim3(256), 0, s, ws_s, ws_g, in, start, pos0,
+                       slot, heads, n, dv, num_slots, min_rows, vec);
+  }));
+  hipLaunchKernelGGL(state_carry_kernel, dim3((n * dv + 255) / 256, heads, num_segs), dim3(256), 0, s, ws_s, nullptr,
+                     ws_g, state, start, pos0, slot, heads, n * dv, num_slots, min_rows);
+  MX_DISPATCH_T(bf16, (launch_out<T>(y, in, ws_s, start, pos0, slot, grid, heads, n, dv, num_slots, min_rows, vec, s)));
   return (int)hipGetLastError();
 }
 

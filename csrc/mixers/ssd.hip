@@ -62,13 +62,14 @@ ssd_scan_kernel(float* __restrict__ y, const T* __restrict__ xbc, long x_stride,
                 long dt_stride, const float* __restrict__ a_log, const float* __restrict__ dt_bias,
                 const float* __restrict__ d_skip, float* __restrict__ state, const int* __restrict__ start,
                 const int* __restrict__ pos0, const int* __restrict__ slot, int heads, int groups, int n,
-                int dv, int num_slots) {
+                int dv, int num_slots, int skip_from) {
   using P = SsdTile<R>;
   __shared__ __attribute__((aligned(16))) float stage[2][P::TT * P::ROWF];
   __shared__ float out_s[2][P::TT * kSCols];     // a chunk's outputs, written out after the walk
   const int s = blockIdx.z, h = blockIdx.y;
   const int sl = slot[s];
   const int r0 = start[s], rows = start[s + 1] - r0;
+  if (skip_from > 0 && rows >= skip_from) return;            // chunk form (chunk_state.hip)
   const int tid = threadIdx.x;
   const int kl = tid & (kSL - 1);
   const int cl = tid / kSL;
@@ -224,15 +225,15 @@ template <typename T, int R>
 static void launch_ssd(dim3 grid, hipStream_t s, float* y, const void* xbc, long x_stride, const void* dt,
                        long dt_stride, const float* a_log, const float* dt_bias, const float* d_skip, float* state,
                        const int* start, const int* pos0, const int* slot, int heads, int groups, int n, int dv,
-                       int num_slots) {
+                       int num_slots, int skip_from) {
   hipLaunchKernelGGL((ssd_scan_kernel<T, R>), grid, dim3(256), 0, s, y, (const T*)xbc, x_stride, (const T*)dt,
-                     dt_stride, a_log, dt_bias, d_skip, state, start, pos0, slot, heads, groups, n, dv, num_slots);
+                     dt_stride, a_log, dt_bias, d_skip, state, start, pos0, slot, heads, groups, n, dv, num_slots, skip_from);
 }
 
 extern "C" int mx_ssd_scan(float* y, const void* xbc, int bf16, long x_stride, const void* dt, long dt_stride,
                            const float* a_log, const float* dt_bias, const float* d_skip, float* state,
                            const int* start, const int* pos0, const int* slot, int num_segs, int heads, int groups,
-                           int n, int dv, int num_slots, hipStream_t s) {
+                           int n, int dv, int num_slots, int skip_from, hipStream_t s) {
   if (num_segs <= 0) return 0;
   if (n < 1 || n > mx_ssd_max_state() || dv < 1 || groups < 1 || heads % groups) return -1;
   const dim3 grid((dv + kSCols - 1) / kSCols, heads, num_segs);
@@ -240,7 +241,7 @@ extern "C" int mx_ssd_scan(float* y, const void* xbc, int bf16, long x_stride, c
   const int need = (n + kSL - 1) / kSL;
 #define MX_SSD(R)                                                                                         \
   MX_DISPATCH_T(bf16, launch_ssd<T, R>(grid, s, y, xbc, x_stride, dt, dt_stride, a_log, dt_bias, d_skip, state, \
-                                       start, pos0, slot, heads, groups, n, dv, num_slots))
+                                       start, pos0, slot, heads, groups, n, dv, num_slots, skip_from))
   if (need <= 2) MX_SSD(2);
   else if (need <= 4) MX_SSD(4);
   else if (need <= 8) MX_SSD(8);

@@ -598,7 +598,7 @@ def ssd_scan(xbc, dt, a_log, dt_bias, d_skip, state, seg: Segments, heads: int, 
     if xbc.is_cuda:
         y = torch.empty(xbc.shape[0], heads * dv, dtype=torch.float32, device=xbc.device)
         native_mixers().ssd_scan(y, xbc, dt, a_log, dt_bias, d_skip, state, seg.start, seg.pos0, seg.slot,
-                                 seg.num, heads, groups, n, dv)
+                                 seg.num, seg.max_rows, heads, groups, n, dv, _walk_below(seg), CHUNK_ROWS)
         return y
     return ref.ssd_scan(xbc, dt, a_log, dt_bias, d_skip, state, seg, heads, groups, n, dv)
 
