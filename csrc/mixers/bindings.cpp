@@ -80,7 +80,7 @@ int mx_heads_to_rows(void* out, int out_bf16, const float* o, const float* inv, 
 int mx_gla_max_dk();
 int mx_gla_scan(float* o, const void* qkv, int bf16, long qkv_stride, const void* a, long a_stride,
                 const float* a_bias, float tau, float* state, const int* start, const int* pos0, const int* slot,
-                int num_segs, int max_rows, int heads, int dk, int dv, int num_slots, hipStream_t s);
+                int num_segs, int max_rows, int heads, int dk, int dv, int num_slots, int skip_from, hipStream_t s);
 int mx_pair_embed_add(float* x, const int* ids, const void* table, int bf16, int rows, int width, long mul_prev,
                       long mul_cur, int buckets, const int* start, const int* pos0, const int* slot, int num_segs,
                       int* last_tok, int num_slots, const void* embed, int vocab, float scale, hipStream_t s);
@@ -141,7 +141,17 @@ int mx_delta_max_dk();
 int mx_delta_rule(float* o, const float* qn, const float* kn, const float* g, const float* beta,
                   const void* qkv, int bf16, long qkv_stride, float* state, const int* start, const int* pos0,
                   const int* slot, int num_segs, int heads, int kv_heads, int dk, int dv, int num_slots,
-                  hipStream_t s);
+                  int skip_from, hipStream_t s);
+int mx_channel_delta_chunks(float* o, const float* qn, const float* kn, const float* g, const float* beta,
+                            const void* v, int v_bf16, long v_stride, float* state, float* ws_s, float* ws_p,
+                            float* ws_q, float* ws_k, float* ws_g, float* ws_w, float* ws_u, const int* start,
+                            const int* pos0, const int* slot, int num_segs, int max_rows, int heads, int kv_heads,
+                            int dk, int dv, int num_slots, int min_rows, hipStream_t s);
+int mx_channel_linear_chunks(float* o, const void* qkv, int bf16, long stride, const void* a, long a_stride,
+                             const float* a_bias, float tau, float* state, float* ws_s, float* ws_p, float* ws_q,
+                             float* ws_k, float* ws_g, const int* start, const int* pos0, const int* slot,
+                             int num_segs, int max_rows, int heads, int dk, int dv, int num_slots, int min_rows,
+                             hipStream_t s);
 int mx_latent_kv_write(const void* dkv, int bf16, long stride, const float* w, float eps, const float* table,
                        int table_rows, int dims, const int* positions, const int* slots, void* cache,
                        int cache_bf16, long num_slots, long rows, int rank, int dr, int interleaved,
@@ -435,9 +445,29 @@ void short_conv_silu(Tensor out, Tensor x, Tensor w, OptT bias, Tensor hist, Ten
                          (int)max_rows, (int)c, (int)taps, (int)hist.size(0), stream()), "short_conv_silu");
 }
 
+// chunks of mx_chunk_rows() rows that the segments of a step of t rows are cut into, at most
+int64_t chunk_bound(int64_t t, int64_t num_segs) { return t / mx_chunk_rows() + num_segs; }
+
+// workspaces of the chunk forms with a decay per channel (channel_chunks.hip)
+struct ChannelSpace {
+  Tensor s, p, q, k, g, w, u;
+  ChannelSpace(int64_t nc, int64_t heads, int64_t dk, int64_t dv, bool delta, const at::TensorOptions& o) {
+    const int64_t c = mx_chunk_rows(), dkp = mx_chunk_key_pad((int)dk);
+    s = at::empty({nc, heads, dk, dv}, o);
+    p = at::empty({nc, heads, c, c}, o);
+    q = at::empty({nc, heads, c, dkp}, o);
+    k = at::empty({nc, heads, dkp, c}, o);
+    g = at::empty({nc, heads, dkp}, o);
+    if (delta) {
+      w = at::empty({nc, heads, c, dkp}, o);
+      u = at::empty({nc, heads, c, (dv + 15) / 16 * 16}, o);
+    }
+  }
+};
+
 void gated_delta_rule(Tensor o, Tensor qkv, Tensor a, Tensor b, Tensor a_log, Tensor dt_bias, Tensor state,
-                      Tensor start, Tensor pos0, Tensor slot, int64_t num_segs, int64_t heads, int64_t kv_heads,
-                      int64_t dk, int64_t dv) {
+                      Tensor start, Tensor pos0, Tensor slot, int64_t num_segs, int64_t max_rows, int64_t heads,
+                      int64_t kv_heads, int64_t dk, int64_t dv, bool walk, int64_t chunk_from) {
   check_f32(o, "o");
   check_rows(qkv, "qkv");
   check_rows(a, "a");
@@ -461,10 +491,24 @@ void gated_delta_rule(Tensor o, Tensor qkv, Tensor a, Tensor b, Tensor a_log, Te
                     qkv.data_ptr(), bf(qkv), qkv.stride(0), a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0),
                     a_log.data_ptr<float>(), dt_bias.data_ptr<float>(), t, (int)heads, (int)kv_heads, (int)dk,
                     stream()), "delta_prep");
-  chk(mx_delta_rule(o.data_ptr<float>(), qn.data_ptr<float>(), kn.data_ptr<float>(), g.data_ptr<float>(),
-                    beta.data_ptr<float>(), qkv.data_ptr(), bf(qkv), qkv.stride(0), state.data_ptr<float>(),
-                    start.data_ptr<int>(), pos0.data_ptr<int>(), slot.data_ptr<int>(), (int)num_segs, (int)heads,
-                    (int)kv_heads, (int)dk, (int)dv, (int)state.size(0), stream()), "delta_rule");
+  TORCH_CHECK(max_rows <= t && chunk_from >= 1, "delta rule rows");
+  const bool chunks = max_rows >= chunk_from && dk <= mx_chunk_max_dk();
+  if (walk || !chunks)
+    chk(mx_delta_rule(o.data_ptr<float>(), qn.data_ptr<float>(), kn.data_ptr<float>(), g.data_ptr<float>(),
+                      beta.data_ptr<float>(), qkv.data_ptr(), bf(qkv), qkv.stride(0), state.data_ptr<float>(),
+                      start.data_ptr<int>(), pos0.data_ptr<int>(), slot.data_ptr<int>(), (int)num_segs, (int)heads,
+                      (int)kv_heads, (int)dk, (int)dv, (int)state.size(0), chunks ? (int)chunk_from : 0, stream()),
+        "delta_rule");
+  if (!chunks) return;
+  const ChannelSpace ws(chunk_bound(t, num_segs), heads, dk, dv, true, f32);
+  const char* v = (const char*)qkv.data_ptr() + 2 * kv_heads * dk * qkv.element_size();
+  chk(mx_channel_delta_chunks(o.data_ptr<float>(), qn.data_ptr<float>(), kn.data_ptr<float>(), g.data_ptr<float>(),
+                              beta.data_ptr<float>(), v, bf(qkv), qkv.stride(0), state.data_ptr<float>(),
+                              ws.s.data_ptr<float>(), ws.p.data_ptr<float>(), ws.q.data_ptr<float>(),
+                              ws.k.data_ptr<float>(), ws.g.data_ptr<float>(), ws.w.data_ptr<float>(),
+                              ws.u.data_ptr<float>(), start.data_ptr<int>(), pos0.data_ptr<int>(),
+                              slot.data_ptr<int>(), (int)num_segs, (int)max_rows, (int)heads, (int)kv_heads, (int)dk,
+                              (int)dv, (int)state.size(0), (int)chunk_from, stream()), "delta rule chunks");
 }
 
 void conv_delta_prep(Tensor qn, Tensor kn, Tensor vo, Tensor lg, Tensor beta, Tensor x, Tensor a, Tensor b,
@@ -493,9 +537,6 @@ void conv_delta_prep(Tensor qn, Tensor kn, Tensor vo, Tensor lg, Tensor beta, Te
                          (int)max_rows, t, (int)hist.size(0), (int)heads, (int)kvh, (int)dk, (int)dv, stream()),
       "conv_delta_prep");
 }
-
-// chunks of mx_chunk_rows() rows that the segments of a step of t rows are cut into, at most
-int64_t chunk_bound(int64_t t, int64_t num_segs) { return t / mx_chunk_rows() + num_segs; }
 
 void head_delta_rule(Tensor o, Tensor q, Tensor k, Tensor v, Tensor lg, Tensor beta, Tensor state, Tensor start,
                      Tensor pos0, Tensor slot, int64_t num_segs, int64_t max_rows, bool walk, int64_t chunk_from) {
@@ -572,7 +613,7 @@ void scaled_pair_rows(Tensor out, Tensor a, double a_scale, Tensor o, Tensor gat
 
 void gated_linear_attention(Tensor o, Tensor qkv, Tensor a, Tensor a_bias, double tau, Tensor state, Tensor start,
                             Tensor pos0, Tensor slot, int64_t num_segs, int64_t max_rows, int64_t heads, int64_t dk,
-                            int64_t dv) {
+                            int64_t dv, bool walk, int64_t chunk_from) {
   check_f32(o, "o");
   check_rows(qkv, "qkv");
   check_rows(a, "a");
@@ -586,10 +627,22 @@ void gated_linear_attention(Tensor o, Tensor qkv, Tensor a, Tensor a_bias, doubl
   TORCH_CHECK(state.dim() == 4 && state.size(1) == heads && state.size(2) == dk && state.size(3) == dv, "state");
   check_segs(start, pos0, slot, num_segs);
   TORCH_CHECK(start.numel() >= num_segs + 1, "segments");
-  chk(mx_gla_scan(o.data_ptr<float>(), qkv.data_ptr(), bf(qkv), qkv.stride(0), a.data_ptr(), a.stride(0),
-                  a_bias.data_ptr<float>(), (float)tau, state.data_ptr<float>(), start.data_ptr<int>(),
-                  pos0.data_ptr<int>(), slot.data_ptr<int>(), (int)num_segs, (int)std::max<int64_t>(max_rows, 0),
-                  (int)heads, (int)dk, (int)dv, (int)state.size(0), stream()), "linear attention");
+  TORCH_CHECK(max_rows <= t && chunk_from >= 1, "linear attention rows");
+  const bool chunks = max_rows >= chunk_from && dk <= mx_chunk_max_dk();
+  if (walk || !chunks)
+    chk(mx_gla_scan(o.data_ptr<float>(), qkv.data_ptr(), bf(qkv), qkv.stride(0), a.data_ptr(), a.stride(0),
+                    a_bias.data_ptr<float>(), (float)tau, state.data_ptr<float>(), start.data_ptr<int>(),
+                    pos0.data_ptr<int>(), slot.data_ptr<int>(), (int)num_segs, (int)std::max<int64_t>(max_rows, 0),
+                    (int)heads, (int)dk, (int)dv, (int)state.size(0), chunks ? (int)chunk_from : 0, stream()),
+        "linear attention");
+  if (!chunks) return;
+  const ChannelSpace ws(chunk_bound(t, num_segs), heads, dk, dv, false, o.options());
+  chk(mx_channel_linear_chunks(o.data_ptr<float>(), qkv.data_ptr(), bf(qkv), qkv.stride(0), a.data_ptr(), a.stride(0),
+                               a_bias.data_ptr<float>(), (float)tau, state.data_ptr<float>(), ws.s.data_ptr<float>(),
+                               ws.p.data_ptr<float>(), ws.q.data_ptr<float>(), ws.k.data_ptr<float>(),
+                               ws.g.data_ptr<float>(), start.data_ptr<int>(), pos0.data_ptr<int>(),
+                               slot.data_ptr<int>(), (int)num_segs, (int)max_rows, (int)heads, (int)dk, (int)dv,
+                               (int)state.size(0), (int)chunk_from, stream()), "linear attention chunks");
 }
 
 void pair_embed_add(Tensor x, Tensor ids, Tensor table, int64_t mul_prev, int64_t mul_cur, int64_t buckets,

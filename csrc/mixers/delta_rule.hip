@@ -157,12 +157,13 @@ delta_rule_kernel(float* __restrict__ o, const float* __restrict__ qn, const flo
                   const float* __restrict__ g, const float* __restrict__ beta, const T* __restrict__ qkv,
                   long qkv_stride, float* __restrict__ state, const int* __restrict__ start,
                   const int* __restrict__ pos0, const int* __restrict__ slot, int heads, int kv_heads,
-                  int dk, int dv, int num_slots) {
+                  int dk, int dv, int num_slots, int skip_from) {
   using P = DeltaTile<R>;
   __shared__ float stage[2][P::TT * P::ROWF];
   const int s = blockIdx.z, h = blockIdx.y;
   const int sl = slot[s];
   const int r0 = start[s], n = start[s + 1] - r0;
+  if (skip_from > 0 && n >= skip_from) return;               // chunk form (channel_chunks.hip)
   const int tid = threadIdx.x;
   const int kl = tid & (kKL - 1);
   const int cl = tid >> 3;                // column within the tile
@@ -319,9 +320,9 @@ template <typename T, int R>
 static void launch_delta(dim3 grid, hipStream_t s, float* o, const float* qn, const float* kn,
                          const float* g, const float* beta, const void* qkv, long qkv_stride, float* state,
                          const int* start, const int* pos0, const int* slot, int heads, int kv_heads, int dk,
-                         int dv, int num_slots) {
+                         int dv, int num_slots, int skip_from) {
   hipLaunchKernelGGL((delta_rule_kernel<T, R>), grid, dim3(256), 0, s, o, qn, kn, g, beta, (const T*)qkv,
-                     qkv_stride, state, start, pos0, slot, heads, kv_heads, dk, dv, num_slots);
+                     qkv_stride, state, start, pos0, slot, heads, kv_heads, dk, dv, num_slots, skip_from);
 }
 
 extern "C" int mx_delta_max_dk() { return kKL * 32; }
@@ -329,7 +330,7 @@ extern "C" int mx_delta_max_dk() { return kKL * 32; }
 extern "C" int mx_delta_rule(float* o, const float* qn, const float* kn, const float* g, const float* beta,
                              const void* qkv, int bf16, long qkv_stride, float* state, const int* start,
                              const int* pos0, const int* slot, int num_segs, int heads, int kv_heads, int dk,
-                             int dv, int num_slots, hipStream_t s) {
+                             int dv, int num_slots, int skip_from, hipStream_t s) {
   if (num_segs <= 0) return 0;
   if (dk < 1 || dk > mx_delta_max_dk() || dv < 1 || heads % kv_heads) return -1;
   const dim3 grid((dv + kCols - 1) / kCols, heads, num_segs);
@@ -337,7 +338,7 @@ extern "C" int mx_delta_rule(float* o, const float* qn, const float* kn, const f
   const int need = (dk + kKL - 1) / kKL;
 #define MX_DELTA(R)                                                                                  \
   MX_DISPATCH_T(bf16, launch_delta<T, R>(grid, s, o, qn, kn, g, beta, qkv, qkv_stride, state, start, \
-                                         pos0, slot, heads, kv_heads, dk, dv, num_slots))
+                                         pos0, slot, heads, kv_heads, dk, dv, num_slots, skip_from))
   if (need <= 2) MX_DELTA(2);
   else if (need <= 4) MX_DELTA(4);
   else if (need <= 8) MX_DELTA(8);

@@ -77,16 +77,6 @@ __device__ __forceinline__ void gla_run(const float* p, float* v) {
   }
 }
 
-// sigmoid(z)^(1/tau) = exp(-softplus(-z) / tau) in fp32 on the hardware's exp2 / log2:
-// softplus(-z) = log(1 + e) with e = exp(-z); for small e the series e - e^2/2 keeps the
-// digits that 1 + e would drop.  The absolute error of the decay's logarithm stays near
-// 1e-7, the spacing of fp32 numbers below 1.
-__device__ __forceinline__ float gla_decay(float z, float inv_tau) {
-  const float e = __expf(-z);
-  const float sp = e < 1e-3f ? e * (1.0f - 0.5f * e) : __logf(1.0f + e);
-  return __expf(-sp * inv_tau);
-}
-
 // 16 bytes of a row, widened to floats
 template <typename T> struct GlaVec;
 template <> struct GlaVec<float> {
@@ -125,7 +115,7 @@ __global__ void __launch_bounds__(256)
 gla_scan_kernel(float* __restrict__ o, const T* __restrict__ qkv, long qkv_stride, const T* __restrict__ a,
                 long a_stride, const float* __restrict__ a_bias, float inv_tau, float* __restrict__ state,
                 const int* __restrict__ start, const int* __restrict__ pos0, const int* __restrict__ slot,
-                int heads, int dk, int dv, int num_slots) {
+                int heads, int dk, int dv, int num_slots, int skip_from) {
   using P = GlaTile<R, SHORT, C>;
   using Regs = GlaRegs<T, R, SHORT, C>;
   constexpr int kGC = C, kGCols = P::COLS;
@@ -135,6 +125,7 @@ gla_scan_kernel(float* __restrict__ o, const T* __restrict__ qkv, long qkv_strid
   const int s = blockIdx.z, h = blockIdx.y;
   const int sl = slot[s];
   const int r0 = start[s], rows = start[s + 1] - r0;
+  if (skip_from > 0 && rows >= skip_from) return;            // chunk form (channel_chunks.hip)
   const int tid = threadIdx.x;
   const int kl = tid & (kGL - 1);
   const int cl = tid / kGL;                       // column group within the workgroup
@@ -334,19 +325,19 @@ extern "C" int mx_gla_max_dk() { return kGL * 8; }
 template <typename T, int R, bool VEC, int C>
 static void launch_gla(dim3 grid, hipStream_t s, bool few, float* o, const void* qkv, long qkv_stride, const void* a,
                        long a_stride, const float* a_bias, float inv_tau, float* state, const int* start,
-                       const int* pos0, const int* slot, int heads, int dk, int dv, int num_slots) {
+                       const int* pos0, const int* slot, int heads, int dk, int dv, int num_slots, int skip_from) {
   if (few)
     hipLaunchKernelGGL((gla_scan_kernel<T, R, true, VEC, C>), grid, dim3(256), 0, s, o, (const T*)qkv, qkv_stride,
-                       (const T*)a, a_stride, a_bias, inv_tau, state, start, pos0, slot, heads, dk, dv, num_slots);
+                       (const T*)a, a_stride, a_bias, inv_tau, state, start, pos0, slot, heads, dk, dv, num_slots, skip_from);
   else
     hipLaunchKernelGGL((gla_scan_kernel<T, R, false, VEC, C>), grid, dim3(256), 0, s, o, (const T*)qkv, qkv_stride,
-                       (const T*)a, a_stride, a_bias, inv_tau, state, start, pos0, slot, heads, dk, dv, num_slots);
+                       (const T*)a, a_stride, a_bias, inv_tau, state, start, pos0, slot, heads, dk, dv, num_slots, skip_from);
 }
 
 extern "C" int mx_gla_scan(float* o, const void* qkv, int bf16, long qkv_stride, const void* a, long a_stride,
                            const float* a_bias, float tau, float* state, const int* start, const int* pos0,
                            const int* slot, int num_segs, int max_rows, int heads, int dk, int dv, int num_slots,
-                           hipStream_t s) {
+                           int skip_from, hipStream_t s) {
   if (num_segs <= 0) return 0;
   const bool few = max_rows > 0 && max_rows <= kGlaShortRows;   // the longest segment of the step (0: unknown)
   if (dk < 1 || dk > mx_gla_max_dk() || dv < 1 || heads < 1 || !(tau > 0.f)) return -1;
@@ -362,7 +353,7 @@ extern "C" int mx_gla_scan(float* o, const void* qkv, int bf16, long qkv_stride,
                    ((uintptr_t)qkv) % 16 == 0 && ((uintptr_t)a) % 16 == 0;
 #define MX_GLA_C(R, V, C)                                                                                        \
   MX_DISPATCH_T(bf16, launch_gla<T, R, V, C>(grid, s, few, o, qkv, qkv_stride, a, a_stride, a_bias, 1.0f / tau, state, \
-                                             start, pos0, slot, heads, dk, dv, num_slots))
+                                             start, pos0, slot, heads, dk, dv, num_slots, skip_from))
 #define MX_GLA(R)                                   \
   do {                                              \
     if (vec && cpl == 2) MX_GLA_C(R, true, 2);      \

@@ -64,6 +64,16 @@ __device__ __forceinline__ float add_halves(float v) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+// sigmoid(z)^(1/tau) = exp(-softplus(-z) / tau) in fp32 on the hardware's exp2 / log2:
+// softplus(-z) = log(1 + e) with e = exp(-z); for small e the series e - e^2/2 keeps the
+// digits that 1 + e would drop.  The absolute error of the decay's logarithm stays near
+// 1e-7, the spacing of fp32 numbers below 1.
+__device__ __forceinline__ float gla_decay(float z, float inv_tau) {
+  const float e = __expf(-z);
+  const float sp = e < 1e-3f ? e * (1.0f - 0.5f * e) : __logf(1.0f + e);
+  return __expf(-sp * inv_tau);
+}
+
 // tanh without branches: the Taylor polynomial up to |x| = 1/4, (1 - e^-2|x|) / (1 + e^-2|x|) beyond
 __device__ __forceinline__ float tanh_(float x) {
   const float a = fabsf(x), q = a * a;

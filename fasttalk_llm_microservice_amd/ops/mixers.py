@@ -343,8 +343,9 @@ def gated_delta_rule(qkv, a, b, a_log, dt_bias, state, seg: Segments, heads: int
     and left at the segment's last row.  Returns o fp32 [T, heads*dv]."""
     if qkv.is_cuda:
         o = torch.empty(qkv.shape[0], heads * dv, dtype=torch.float32, device=qkv.device)
-        native_mixers().gated_delta_rule(o, qkv, a, b, a_log, dt_bias, state, seg.start, seg.pos0,
-                                         seg.slot, seg.num, heads, kv_heads, dk, dv)
+        native_mixers().gated_delta_rule(o, qkv, a, b, a_log, dt_bias, state, seg.start, seg.pos0, seg.slot, seg.num,
+                                         seg.max_rows, heads, kv_heads, dk, dv, _walk_below(seg, CHANNEL_CHUNK_ROWS),
+                                         CHANNEL_CHUNK_ROWS)
         return o
     return ref.gated_delta_rule(qkv, a, b, a_log, dt_bias, state, seg, heads, kv_heads, dk, dv)
 
@@ -370,9 +371,15 @@ def conv_delta_prep(qkv, a, b, conv_w, conv_state, a_log, dt_bias, seg: Segments
     return ref.conv_delta_prep(qkv, a, b, conv_w, conv_state, a_log, dt_bias, seg, heads, kv_heads, dk, dv)
 
 
-# rows from which a segment's recurrence runs chunk by chunk as matrix products (per-head
-# decays); shorter segments and decode rows are walked row by row
+# rows from which a segment's recurrence runs chunk by chunk as matrix products; shorter segments
+# and decode rows are walked row by row
 CHUNK_ROWS = 32
+# the same with a decay per channel, and for the state-space scan, whose walks are cheaper and whose
+# chunk form has four launches.  One segment of 64 / 100 / 200 / 777 rows, 16 (state space: 32) heads of
+# 128 x 128, us: delta rule 58 61 70 99 (walk 43 62 114 423), linear attention 38 39 43 66 (25 39 70
+# 245), state space 40 41 46 98 (19 28 49 169; four segments of 200: 108, walk 97)
+CHANNEL_CHUNK_ROWS = 96
+SSD_CHUNK_ROWS = 256
 
 
 def head_delta_rule(q, k, v, log_decay, beta, state, seg: Segments) -> torch.Tensor:
@@ -384,7 +391,7 @@ def head_delta_rule(q, k, v, log_decay, beta, state, seg: Segments) -> torch.Ten
         t, heads, dv = v.shape
         o = torch.empty(t, heads * dv, dtype=torch.float32, device=v.device)
         native_mixers().head_delta_rule(o, q, k, v, log_decay, beta, state, seg.start, seg.pos0, seg.slot, seg.num,
-                                        seg.max_rows, _walk_below(seg), CHUNK_ROWS)
+                                        seg.max_rows, _walk_below(seg, CHUNK_ROWS), CHUNK_ROWS)
         return o
     return ref.head_delta_rule(q, k, v, log_decay, beta, state, seg)
 
@@ -401,17 +408,17 @@ def retention(qkv, table, rot_dims: int, log_decay, state, seg: Segments, heads:
     if qkv.is_cuda:
         o = torch.empty(qkv.shape[0], heads * dv, dtype=torch.float32, device=qkv.device)
         native_mixers().retention(o, qkv, table, rot_dims, bool(interleaved), log_decay, state, seg.start, seg.pos0,
-                                  seg.slot, seg.num, seg.max_rows, heads, dk, dv, _walk_below(seg), CHUNK_ROWS)
+                                  seg.slot, seg.num, seg.max_rows, heads, dk, dv, _walk_below(seg, CHUNK_ROWS), CHUNK_ROWS)
         return o
     return ref.retention(qkv, table, rot_dims, interleaved, log_decay, state, seg, heads, dk, dv)
 
 
-def _walk_below(seg: Segments) -> bool:
+def _walk_below(seg: Segments, chunk_rows: int) -> bool:
     """Whether a step may hold segments short enough to be walked row by row."""
-    if seg.max_rows < CHUNK_ROWS or seg.host is None:
+    if seg.max_rows < chunk_rows or seg.host is None:
         return True
     start = seg.host[0]
-    return min(b - a for a, b in zip(start[:-1], start[1:])) < CHUNK_ROWS
+    return min(b - a for a, b in zip(start[:-1], start[1:])) < chunk_rows
 
 
 def gated_linear_attention(qkv, a, a_bias, tau: float, state, seg: Segments, heads: int, dk: int,
@@ -426,7 +433,8 @@ def gated_linear_attention(qkv, a, a_bias, tau: float, state, seg: Segments, hea
     if qkv.is_cuda:
         o = torch.empty(qkv.shape[0], heads * dv, dtype=torch.float32, device=qkv.device)
         native_mixers().gated_linear_attention(o, qkv, a, a_bias, float(tau), state, seg.start, seg.pos0,
-                                               seg.slot, seg.num, seg.max_rows, heads, dk, dv)
+                                               seg.slot, seg.num, seg.max_rows, heads, dk, dv,
+                                               _walk_below(seg, CHANNEL_CHUNK_ROWS), CHANNEL_CHUNK_ROWS)
         return o
     return ref.gated_linear_attention(qkv, a, a_bias, tau, state, seg, heads, dk, dv)
 
@@ -598,7 +606,7 @@ def ssd_scan(xbc, dt, a_log, dt_bias, d_skip, state, seg: Segments, heads: int, 
     if xbc.is_cuda:
         y = torch.empty(xbc.shape[0], heads * dv, dtype=torch.float32, device=xbc.device)
         native_mixers().ssd_scan(y, xbc, dt, a_log, dt_bias, d_skip, state, seg.start, seg.pos0, seg.slot,
-                                 seg.num, seg.max_rows, heads, groups, n, dv, _walk_below(seg), CHUNK_ROWS)
+                                 seg.num, seg.max_rows, heads, groups, n, dv, _walk_below(seg, SSD_CHUNK_ROWS), SSD_CHUNK_ROWS)
         return y
     return ref.ssd_scan(xbc, dt, a_log, dt_bias, d_skip, state, seg, heads, groups, n, dv)
 

@@ -37,9 +37,12 @@ def walk(seg, state, step):
 
 def check(run, want_state, want, dv, monkeypatch):
     """run() -> (outputs, states), once in chunk form and once row by row."""
-    got = run()
-    monkeypatch.setattr(M, "CHUNK_ROWS", 1 << 30)
-    base = run()
+    both = []
+    for rows in (32, 1 << 30):
+        monkeypatch.setattr(M, "CHANNEL_CHUNK_ROWS", rows)
+        monkeypatch.setattr(M, "SSD_CHUNK_ROWS", rows)
+        both.append(run())
+    got, base = both
     rows = sorted(want)
     w = torch.stack([want[r] for r in rows])
     for i, (x, y) in enumerate(((w, lambda t: t[rows].to(D)), (want_state, lambda t: t.to(D)))):
@@ -88,3 +91,78 @@ def test_state_space(dt_, lens, pos0, heads, groups, n, dv, monkeypatch):
     if -1 in slots:
         i = slots.index(-1)
         assert bool((y[seg.host[0][i]:seg.host[0][i + 1]] == 0).all())
+
+
+@pytest.mark.parametrize("dt_", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("lens,pos0", SHAPES)
+@pytest.mark.parametrize("heads,kvh,dk,dv", [(4, 2, 128, 128), (3, 3, 20, 24), (2, 1, 64, 72), (2, 2, 12, 16)])
+@pytest.mark.parametrize("fast", [False, True], ids=["slow", "fast"])
+def test_channel_delta(dt_, lens, pos0, heads, kvh, dk, dv, fast, monkeypatch):
+    """``fast``: channels that forget within a few rows (decays down to e^-30), beside slow ones."""
+    g = torch.Generator().manual_seed(sum(lens) + dk)
+    T, slots = sum(lens), list(range(len(lens)))
+    if len(lens) > 3:
+        slots[1] = -1
+    seg = segments(lens, pos0, slots)
+    rnd = lambda *s: torch.randn(*s, generator=g).to(DEV, dt_)   # noqa: E731
+    qkv, a, b = rnd(T, 2 * kvh * dk + heads * dv), rnd(T, heads * dk), rnd(T, heads)
+    a_log = (torch.rand(heads, generator=g) + (1.5 if fast else -1.0)).to(DEV)
+    bias = ((torch.rand(heads * dk, generator=g) - 0.5) * (12.0 if fast else 2.0) - 1.0).to(DEV)
+    s0 = torch.randn(len(lens), heads, dk, dv, generator=g).to(DEV)
+    x = qkv.to(D)
+    unit = lambda v: v / torch.sqrt((v * v).sum(-1, keepdim=True) + 1e-6)   # noqa: E731
+    q = unit(x[:, :kvh * dk].view(T, kvh, dk)).repeat_interleave(heads // kvh, 1) * dk ** -0.5
+    k = unit(x[:, kvh * dk:2 * kvh * dk].view(T, kvh, dk)).repeat_interleave(heads // kvh, 1)
+    v, beta = x[:, 2 * kvh * dk:].view(T, heads, dv), torch.sigmoid(b.to(D))
+    sp = torch.nn.functional.softplus(a.to(D) + bias.to(D)).view(T, heads, dk)
+    dec = torch.exp(-torch.exp(a_log.to(D))[None, :, None] * sp)
+
+    def step(r, S):
+        S = dec[r][:, :, None] * S
+        u = beta[r][:, None] * (v[r] - (S * k[r][:, :, None]).sum(1))
+        S = S + k[r][:, :, None] * u[:, None]
+        return S, (S * q[r][:, :, None]).sum(1).flatten()
+
+    ws, wo = walk(seg, s0, step)
+
+    def run():
+        st = s0.clone()
+        return M.gated_delta_rule(qkv, a, b, a_log, bias, st, seg, heads, kvh, dk, dv), st
+
+    y, _ = check(run, ws, wo, dv, monkeypatch)
+    if -1 in slots:
+        i = slots.index(-1)
+        assert bool((y[seg.host[0][i]:seg.host[0][i + 1]] == 0).all())
+
+
+@pytest.mark.parametrize("dt_", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("lens,pos0", SHAPES)
+@pytest.mark.parametrize("heads,dk,dv", [(4, 128, 128), (3, 20, 24), (2, 64, 72), (2, 12, 16)])
+@pytest.mark.parametrize("fast", [False, True], ids=["slow", "fast"])
+def test_channel_linear(dt_, lens, pos0, heads, dk, dv, fast, monkeypatch):
+    g = torch.Generator().manual_seed(sum(lens) + dk)
+    T, slots = sum(lens), list(range(len(lens)))
+    if len(lens) > 3:
+        slots[1] = -1
+    seg = segments(lens, pos0, slots)
+    tau = 0.5 if fast else 8.0
+    p = torch.randn(T, heads * (2 * dk + dv) + 8, generator=g).to(DEV, dt_)
+    a = torch.randn(T, heads * dk, generator=g).to(DEV, dt_)
+    bias = (torch.rand(heads * dk, generator=g) * (16.0 if fast else 3.0) - (8.0 if fast else 0.0)).to(DEV)
+    s0 = torch.randn(len(lens), heads, dk, dv, generator=g).to(DEV)
+    x = p.to(D)
+    n = heads * dk
+    q, k, v = x[:, :n].view(T, heads, dk) * dk ** -0.5, x[:, n:2 * n].view(T, heads, dk), x[:, 2 * n:2 * n + heads * dv].view(T, heads, dv)
+    dec = torch.exp(torch.nn.functional.logsigmoid(a.to(D) + bias.to(D)) / tau).view(T, heads, dk)
+
+    def step(r, S):
+        S = dec[r][:, :, None] * S + k[r][:, :, None] * v[r][:, None]
+        return S, (S * q[r][:, :, None]).sum(1).flatten()
+
+    ws, wo = walk(seg, s0, step)
+
+    def run():
+        st = s0.clone()
+        return M.gated_linear_attention(p, a, bias, tau, st, seg, heads, dk, dv), st
+
+    check(run, ws, wo, dv, monkeypatch)
