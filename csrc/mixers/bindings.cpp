@@ -15,8 +15,11 @@ int mx_embed_rows(float* out, const int* ids, const void* table, int bf16, int r
 int mx_layer_norm(float* x, const void* y, int y_bf16, long y_stride, const float* w, const float* b, void* out,
                   void* cast, int out_bf16, int rows, int width, float eps, hipStream_t s);
 int mx_tanh_cap(float* x, long n, float cap, hipStream_t s);
-int mx_grouped_gemm(void* C, const void* A, const void* W, const int* offs, int groups, long M, int N, int K,
-                    hipStream_t s);
+int mx_grouped_gemm(void* C, const void* A, const int* rows, const void* W, const int* offs, int groups, long M, int N,
+                    int K, int act, float limit, hipStream_t s);
+int mx_pair_sort(int* offs, int* sorted_row, int* place, const int* idx, long rows, int top, int experts, hipStream_t s);
+int mx_experts_merge(float* out, const void* d, const int* place, const float* wts, const void* shared, const void* h,
+                     long h_stride, const void* gate_w, long rows, int top, int width, hipStream_t s);
 int mx_relu_sq_rows(void* out, const void* u, int bf16, long u_stride, long rows, int ff, hipStream_t s);
 int mx_gather_add_rows(float* out, const void* y, int y_bf16, const int* idx, const float* w, long rows, int top,
                        int width, long y_rows, hipStream_t s);
@@ -387,8 +390,8 @@ void grouped_gemm(Tensor out, Tensor a, Tensor w, Tensor offs) {
   TORCH_CHECK(out.is_cuda() && out.is_contiguous() && out.scalar_type() == at::kBFloat16 && out.dim() == 2 &&
               out.size(0) == a.size(0) && out.size(1) == w.size(1), "out: bf16 [M, N]");
   TORCH_CHECK(a.size(1) % 8 == 0 && a.size(1) >= 8, "K must be a multiple of 8");
-  chk(mx_grouped_gemm(out.data_ptr(), a.data_ptr(), w.data_ptr(), offs.data_ptr<int>(), (int)w.size(0), a.size(0),
-                      (int)w.size(1), (int)a.size(1), stream()), "grouped_gemm");
+  chk(mx_grouped_gemm(out.data_ptr(), a.data_ptr(), nullptr, w.data_ptr(), offs.data_ptr<int>(), (int)w.size(0),
+                      a.size(0), (int)w.size(1), (int)a.size(1), 0, 0.f, stream()), "grouped_gemm");
 }
 
 void clamp_swiglu(Tensor out, Tensor gu, double limit) {
@@ -921,6 +924,37 @@ void experts_few(Tensor out, Tensor h, Tensor idx, Tensor wts, Tensor wgu, Tenso
                      (float)shared_limit, stream()), "experts_few");
 }
 
+void experts_many(Tensor out, Tensor h, Tensor idx, Tensor wts, Tensor wgu, Tensor wdown, double limit, int64_t act,
+                  OptT shared, OptT gate_w) {
+  check_f32(out, "out");
+  check_i32(idx, "idx");
+  check_f32(wts, "wts");
+  TORCH_CHECK(act >= 1 && act <= 5, "experts_many: activation");
+  auto bf16 = [](const Tensor& w) { return w.is_cuda() && w.scalar_type() == at::kBFloat16 && w.is_contiguous(); };
+  const int64_t t = h.size(0), width = h.size(1), top = idx.dim() == 2 ? idx.size(1) : 0, mult = act == 5 ? 1 : 2;
+  TORCH_CHECK(bf16(h) && h.dim() == 2 && bf16(wgu) && bf16(wdown) && wgu.dim() == 3 && wdown.dim() == 3 &&
+              wgu.size(0) == wdown.size(0) && wgu.size(2) == width && wdown.size(1) == width &&
+              wgu.size(1) == mult * wdown.size(2) && width % 8 == 0 && wdown.size(2) % 8 == 0,
+              "experts_many: rows and expert weights");
+  TORCH_CHECK(idx.dim() == 2 && idx.size(0) == t && top >= 1 && wts.numel() == t * top && out.numel() == t * width,
+              "experts_many: shapes");
+  TORCH_CHECK(!shared || (bf16(*shared) && shared->numel() == t * width), "experts_many: shared expert's rows");
+  TORCH_CHECK(!gate_w || (shared && bf16(*gate_w) && gate_w->numel() == width), "experts_many: shared expert's gate");
+  const int64_t pairs = t * top, ff = wdown.size(2);
+  const int experts = (int)wgu.size(0);
+  Tensor sorted = at::empty({2 * pairs + experts}, idx.options());
+  int *row = sorted.data_ptr<int>(), *place = row + pairs, *offs = place + pairs;
+  Tensor y = at::empty({pairs, ff}, h.options()), d = at::empty({pairs, width}, h.options());
+  chk(mx_pair_sort(offs, row, place, idx.data_ptr<int>(), t, (int)top, experts, stream()), "pair_sort");
+  chk(mx_grouped_gemm(y.data_ptr(), h.data_ptr(), row, wgu.data_ptr(), offs, experts, pairs, (int)ff, (int)width,
+                      (int)act, (float)limit, stream()), "grouped_gemm");
+  chk(mx_grouped_gemm(d.data_ptr(), y.data_ptr(), nullptr, wdown.data_ptr(), offs, experts, pairs, (int)width, (int)ff,
+                      0, 0.f, stream()), "grouped_gemm");
+  chk(mx_experts_merge(out.data_ptr<float>(), d.data_ptr(), place, wts.data_ptr<float>(),
+                       shared ? shared->data_ptr() : nullptr, h.data_ptr(), h.stride(0),
+                       gate_w ? gate_w->data_ptr() : nullptr, t, (int)top, (int)width, stream()), "experts_merge");
+}
+
 void moe_pairs(Tensor out, Tensor h, Tensor idx, Tensor wts, Tensor wgu, Tensor wdown, double limit, int64_t act) {
   const bool relu_sq = act == 1;
   TORCH_CHECK(act >= 0 && act <= 2, "moe_pairs: activation");
@@ -1386,6 +1420,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("moe_topk", &moe_topk);
   m.def("moe_pairs", &moe_pairs);
   m.def("few_rows_gemm", &few_rows_gemm);
+  m.def("experts_many", &experts_many);
   m.def("experts_few", &experts_few);
   m.def("few_rows_max", []() { return (int64_t)mx_few_rows_max(); });
   m.def("act_glu", &act_glu);

@@ -855,6 +855,15 @@ class MoEFF:
             idx, wts = self.route(h)
             return M.experts_few(h, idx, wts, self.wgu, self.wdown, self.act, self.limit, self.shared,
                                  self.shared_limit if self.shared is not None else 0.0, self.shared_gate)
+        if t > self.PAIR_ROWS and M.experts_many_ok(h, self.wgu, self.wdown):
+            idx, wts = self.route(h)
+            shared = gate_w = None
+            if self.shared is not None:
+                w1, wdown = self.shared
+                if self.shared_gate:
+                    w1, gate_w = w1[:-1], w1[-1]
+                shared = M.linear(self._act(M.linear(h, w1), self.shared_limit), wdown)
+            return M.experts_many(h, idx, wts, self.wgu, self.wdown, self.act, self.limit, shared, gate_w)
         if self.shared is not None and not self.shared_gate:
             # an ungated shared expert's output is what the chosen experts' are added to
             out = M.linear(self._act(M.linear(h, self.shared[0]), self.shared_limit), self.shared[1]).float()

@@ -1072,6 +1072,21 @@ def experts_few(h, idx, wts, wgu, wdown, act: str, limit: float = 0.0, shared=No
     return out
 
 
+def experts_many_ok(h, wgu, wdown) -> bool:
+    """Whether :func:`experts_many` takes these rows and expert weights."""
+    return bool(h.is_cuda and all(x.dtype == torch.bfloat16 and x.is_contiguous() and x.shape[-1] % 8 == 0
+                                  and x.data_ptr() % 16 == 0 for x in (h, wgu, wdown)))
+
+
+def experts_many(h, idx, wts, wgu, wdown, act: str, limit: float = 0.0, shared=None, gate_w=None) -> torch.Tensor:
+    """fp32 sum_k wts[:, k] * expert_{idx[:, k]}(h) (+ ``shared``, bf16 rows, times sigmoid(h . gate_w) if
+    there is a ``gate_w``), for many rows: (row, choice) pairs sorted by expert, every expert's pairs one
+    group of two grouped products.  No host round trip."""
+    out = torch.empty(h.shape, dtype=torch.float32, device=h.device)
+    native_mixers().experts_many(out, h, idx, wts, wgu, wdown, float(limit), FEW_ACTS[act], shared, gate_w)
+    return out
+
+
 def clamp_swiglu(gu, limit: float):
     """[gate | up (| extra)] rows -> min(gate, limit) * sigmoid(1.702 gate') * (clamp(up) + 1)."""
     if gu.is_cuda:
