@@ -6,84 +6,122 @@
 //                    several experts chose is read in place), the activation in the epilogue
 //   experts_merge    out[r] = sum_k w[r, k] d[place of pair (r, k)] + shared part
 //
-// grouped_gemm: a workgroup of four waves owns BM rows x BN columns of one group (blockIdx.y walks the
-// groups' row tiles; slots past the last tile exit at once), k in steps of 64 through two LDS copies
-// with the next step's 16-byte loads in flight during the products (v_mfma_f32_16x16x32_bf16).  The weight
-// is the left operand, so a lane ends with four neighbouring columns of a row.  Gated: the staged columns
-// alternate 16 of the gate and the same 16 of the up matrix, so a lane has both sums.  Rows past a
-// group's end, columns past N and k past K are zero-filled on load and not stored.
+// grouped_gemm: a workgroup of four waves owns BM rows x 128 columns of one group, k in steps of 64 through
+// two LDS copies (v_mfma_f32_16x16x32_bf16; a wave owns BM / 2 x 64).  Two steps of 16-byte loads are in
+// flight in registers; the LDS reads of one half step run under the products of the other, one barrier a step.
+// The weight is the left operand, so a lane ends with four neighbouring columns of a row.  Gated: the staged
+// columns alternate 16 of the gate and the same 16 of the up matrix, so a lane has both sums.  Rows past a
+// group's end and columns past N repeat the last one and are not stored; k past K counts as zero.
+// LDS rows are 128 bytes with 16-byte pieces swapped by row (no bank conflicts; rows padded to 144 bytes:
+// a third of the LDS cycles were conflicts).
 // Tiles of 128 rows once the groups hold 96 on average, below that 64 (an expert's few rows leave most of a
-// taller tile empty).  16384 pairs of 32 experts, 2048 -> 2 x 1024 gated: 242 us (570 TFLOP/s), 64 x 64 tiles
-// with the gathered rows, the activation and its round trip in kernels of their own 270 + 60 + 50; whole
-// layers of 2000 rows, 32 experts: 0.95 -> 0.50 ms and 24 -> 8 launches.
-// The column tiles come first in the grid: with eight XCDs taking workgroups in turn, an expert's
-// column tile stays in one XCD's L2 for all of the expert's row tiles.
+// taller tile empty).  The tiles run group by group, bands of eight row tiles with their columns after each
+// other, and each XCD (workgroup id mod 8) takes one contiguous eighth of that order, so the tiles in flight on
+// an XCD share an expert's rows and columns in its L2.
+// Bound by the L2's rate on tall groups (128 x 128 tiles with all operands resident in L2 still take 200 of the
+// 254 us below; 128 x 256 tiles with one workgroup a CU, 264), by the read of the matrices on short ones.
+// 16384 pairs of 32 experts, 2048 -> 2 x 1024 gated, 137 GFLOP: 195 us (700 TFLOP/s) in a running model, 254
+// with cold operands; one step of loads in flight, a barrier between reads and products and tiles in grid
+// order: 242 in the model.  1800 pairs, same matrices (268 MB): 78 us in the model, was 98.
 #include "few_rows.h"
+
+#include <type_traits>
 
 namespace mx {
 
 constexpr int kGK = 64;
-constexpr int kGLd = kGK + 8;        // LDS row stride (bf16): 144 bytes, keeps 16-byte alignment
 
-template <int BM, int BN, bool GLU>
+// 2 x 2 waves, each MT x 4 tiles of 16 x 16: BM = 32 MT rows, 128 staged columns
+template <int MT, bool GLU>
 __global__ void __launch_bounds__(256, 2)
 grouped_gemm_kernel(bf16_t* __restrict__ C, const bf16_t* __restrict__ A, const int* __restrict__ rows,
-                    const bf16_t* __restrict__ W, const int* __restrict__ offs, int groups, int M, int N, int K, int act,
-                    float limit, int vec) {
-  constexpr int MT = BM / 32, NT = BN / 32;          // 16-wide tiles of a wave (2 x 2 waves)
-  constexpr int PA = BM * 8 / 256, PW = BN * 8 / 256;
-  constexpr int kStep = (BM + BN) * kGLd;
+                    const bf16_t* __restrict__ W, const int* __restrict__ offs, int groups, int M, int N, int K,
+                    int col_tiles, int act, float limit, int vec) {
+  constexpr int NT = 4, BM = 32 * MT, BN = 32 * NT;
+  constexpr int PA = BM / 32, PW = BN / 32;
+  constexpr int kStep = (BM + BN) * kGK;
   __shared__ __attribute__((aligned(16))) bf16_t stage[2 * kStep];
-  // this workgroup's group and row tile
-  int g = 0, row0 = 0, end = 0;
-  {
-    int t = blockIdx.y, prev = 0;
-    bool found = false;
-    for (g = 0; g < groups; ++g) {
-      end = min(max(offs[g], prev), M);
-      const int tiles = (end - prev + BM - 1) / BM;
-      if (t < tiles) {
-        row0 = prev + t * BM;
-        found = true;
-        break;
-      }
-      t -= tiles;
-      prev = end;
-    }
-    if (!found) return;
-  }
-  const int n0 = blockIdx.x * (GLU ? BN / 2 : BN);
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1, l15 = lane & 15, g4 = lane >> 4;
+
+  // this workgroup's group, row tile and column tile: every wave sums the groups' row tiles, a lane a group
+  int g, row0, end, ct;
+  {
+    auto span = [&](int i, int& lo, int& hi) {
+      lo = i > 0 && i < groups ? min(max(offs[i - 1], 0), M) : 0;
+      hi = i < groups ? min(max(offs[i], lo), M) : lo;
+      return (hi - lo + BM - 1) / BM;
+    };
+    int total = 0, lo = 0, hi = 0, n = 0, upto = 0;
+    for (int g0 = 0; g0 < groups; g0 += 64) {
+      n = span(g0 + lane, lo, hi);
+      upto = n;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int x = __shfl_up(upto, o, 64);
+        upto += lane >= o ? x : 0;
+      }
+      total += __shfl(upto, 63, 64);
+    }
+    const long all = (long)total * col_tiles, per = (all + 7) / 8;
+    const long t = (long)(blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if ((blockIdx.x >> 3) >= per || t >= all) return;
+    const int tile = (int)(t / col_tiles);
+    int base = 0;
+    uint64_t past = 0;
+    for (g = 0;; g += 64) {                     // (ends: tile < total)
+      if (groups > 64) {
+        n = span(g + lane, lo, hi);
+        upto = n;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+          const int x = __shfl_up(upto, o, 64);
+          upto += lane >= o ? x : 0;
+        }
+      }
+      past = __ballot(base + upto > tile);
+      if (past != 0 || g + 64 >= groups) break;
+      base += __shfl(upto, 63, 64);
+    }
+    const int at = past != 0 ? __builtin_ctzll(past) : 63;
+    g += at;
+    lo = __builtin_amdgcn_readlane(lo, at);
+    hi = __builtin_amdgcn_readlane(hi, at);
+    n = __builtin_amdgcn_readlane(n, at);
+    const int first = base + __builtin_amdgcn_readlane(upto, at) - n;
+    // inside the group: bands of eight row tiles, column tiles after each other, rows fastest
+    const int r = (int)(t - (long)first * col_tiles), band = r / (8 * col_tiles);
+    const int in = r - band * 8 * col_tiles, tall = min(8, n - 8 * band);
+    ct = in / tall;
+    row0 = lo + (8 * band + in % tall) * BM;
+    end = hi;
+  }
+  const int n0 = ct * (GLU ? BN / 2 : BN);
   const bf16_t* Wg = W + (long)g * N * (GLU ? 2 : 1) * K;
 
-  // a thread's pieces: row tid / 8 + 32 p of the tile, 8 elements at 8 (tid % 8)
+  // a thread's pieces: row tid / 8 + 32 p of the tile, 8 elements at 8 (tid % 8); rows past the group's end
+  // and columns past N repeat the last one (not stored)
   const int kp = (tid & 7) * 8;
   const bf16_t *ap[PA], *wp[PW];
 #pragma unroll
   for (int p = 0; p < PA; ++p) {
-    const int r = row0 + (tid >> 3) + 32 * p;
-    ap[p] = r < end ? A + (long)(rows != nullptr ? rows[r] : r) * K + kp : nullptr;
+    const int r = min(row0 + (tid >> 3) + 32 * p, end - 1);
+    ap[p] = A + (long)(rows != nullptr ? rows[r] : r) * K;
   }
 #pragma unroll
   for (int p = 0; p < PW; ++p) {
     const int r = (tid >> 3) + 32 * p;
-    const int col = n0 + (GLU ? (r >> 5) * 16 + (r & 15) : r);
-    wp[p] = col < N ? Wg + ((long)(GLU && (r & 16) ? N : 0) + col) * K + kp : nullptr;
+    const int col = min(n0 + (GLU ? (r >> 5) * 16 + (r & 15) : r), N - 1);
+    wp[p] = Wg + ((long)(GLU && (r & 16) ? N : 0) + col) * K;
   }
-  uint4 ra[PA], rw[PW];
-  auto fetch = [&](int k0) {
-    const bool in = k0 + kp < K;
+  uint4 ra[2][PA], rw[2][PW];
+  auto fetch = [&](auto set, int k0) {
+    constexpr int S = decltype(set)::value;
+    const int k = min(k0 + kp, K - 8);        // (past K: loaded again, zeroed when staged)
 #pragma unroll
-    for (int p = 0; p < PA; ++p) {
-      ra[p] = uint4{0, 0, 0, 0};
-      if (in && ap[p] != nullptr) ra[p] = *reinterpret_cast<const uint4*>(ap[p] + k0);
-    }
+    for (int p = 0; p < PA; ++p) ra[S][p] = *reinterpret_cast<const uint4*>(ap[p] + k);
 #pragma unroll
-    for (int p = 0; p < PW; ++p) {
-      rw[p] = uint4{0, 0, 0, 0};
-      if (in && wp[p] != nullptr) rw[p] = *reinterpret_cast<const uint4*>(wp[p] + k0);
-    }
+    for (int p = 0; p < PW; ++p) rw[S][p] = *reinterpret_cast<const uint4*>(wp[p] + k);
   };
   fr_f32x4 acc[NT][MT];
 #pragma unroll
@@ -91,40 +129,89 @@ grouped_gemm_kernel(bf16_t* __restrict__ C, const bf16_t* __restrict__ A, const 
 #pragma unroll
     for (int j = 0; j < MT; ++j) acc[i][j] = fr_f32x4{0.f, 0.f, 0.f, 0.f};
 
-  fetch(0);
-  int buf = 0;
-  for (int k0 = 0; k0 < K; k0 += kGK, buf ^= 1) {
-    bf16_t *As = stage + buf * kStep, *Ws = As + BM * kGLd;
-    const int off = (tid >> 3) * kGLd + kp;
+  // LDS: rows of 128 bytes, 16-byte piece c of row r at slot c ^ swz(r); a lane's fragment of half h of a
+  // step is piece 2 g4 + h of its row, for both operands
+  const auto swz = [](int r) { return (r >> 1) & 5; };
+  const int put = (tid >> 3) * kGK + ((tid & 7) ^ swz(tid >> 3)) * 8;
+  const int get[2] = {l15 * kGK + ((2 * g4) ^ swz(l15)) * 8, l15 * kGK + ((2 * g4 + 1) ^ swz(l15)) * 8};
+  uint4 a[2][MT], b[2][NT];
+  auto stage_in = [&](auto set, int k0) {       // registers of step k0 -> LDS copy `set`
+    constexpr int S = decltype(set)::value;
+    if (k0 + kGK > K && k0 + kp >= K) {
 #pragma unroll
-    for (int p = 0; p < PA; ++p) *reinterpret_cast<uint4*>(As + off + 32 * p * kGLd) = ra[p];
+      for (int p = 0; p < PA; ++p) ra[S][p] = uint4{0, 0, 0, 0};
 #pragma unroll
-    for (int p = 0; p < PW; ++p) *reinterpret_cast<uint4*>(Ws + off + 32 * p * kGLd) = rw[p];
-    __syncthreads();          // (the other copy's readers have passed the barrier before this one's writes)
-    if (k0 + kGK < K) fetch(k0 + kGK);
-#pragma unroll
-    for (int ks = 0; ks < kGK / 32; ++ks) {
-      uint4 a[MT], b[NT];
-#pragma unroll
-      for (int j = 0; j < MT; ++j)
-        a[j] = *reinterpret_cast<const uint4*>(As + (wm * (BM / 2) + j * 16 + l15) * kGLd + ks * 32 + g4 * 8);
-#pragma unroll
-      for (int i = 0; i < NT; ++i)
-        b[i] = *reinterpret_cast<const uint4*>(Ws + (wn * (BN / 2) + i * 16 + l15) * kGLd + ks * 32 + g4 * 8);
-#pragma unroll
-      for (int i = 0; i < NT; ++i)
-#pragma unroll
-        for (int j = 0; j < MT; ++j) acc[i][j] = fr_mfma(b[i], a[j], acc[i][j]);
+      for (int p = 0; p < PW; ++p) rw[S][p] = uint4{0, 0, 0, 0};
     }
+#pragma unroll
+    for (int p = 0; p < PA; ++p) *reinterpret_cast<uint4*>(stage + S * kStep + put + 32 * p * kGK) = ra[S][p];
+#pragma unroll
+    for (int p = 0; p < PW; ++p) *reinterpret_cast<uint4*>(stage + S * kStep + BM * kGK + put + 32 * p * kGK) = rw[S][p];
+  };
+  auto read = [&](auto set, auto half) {
+    constexpr int S = decltype(set)::value, H = decltype(half)::value;
+#pragma unroll
+    for (int j = 0; j < MT; ++j)
+      a[H][j] = *reinterpret_cast<const uint4*>(stage + S * kStep + (wm * MT + j) * 16 * kGK + get[H]);
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+      b[H][i] = *reinterpret_cast<const uint4*>(stage + S * kStep + (BM + (wn * NT + i) * 16) * kGK + get[H]);
+  };
+  auto product = [&](auto half) {
+    constexpr int H = decltype(half)::value;
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+      for (int j = 0; j < MT; ++j) acc[i][j] = fr_mfma(b[H][i], a[H][j], acc[i][j]);
+  };
+  const std::integral_constant<int, 0> even, lo_half;
+  const std::integral_constant<int, 1> odd, hi_half;
+  // Step k0 (copy `set` staged, its low half in registers): the high half's reads under the low half's
+  // products, the next step's staging, one barrier, the next low half's reads under the high half's products.
+  // The barrier also ends every wave's reads of a copy before its next writes, a step later.
+  auto step = [&](auto set, auto next, auto last, int k0) {
+    read(set, hi_half);
+    __builtin_amdgcn_sched_barrier(0);
+    product(lo_half);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (!decltype(last)::value) {
+      stage_in(next, k0 + kGK);
+      fetch(next, k0 + 3 * kGK);
+      __syncthreads();
+      read(next, lo_half);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    product(hi_half);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  fetch(even, 0);
+  __builtin_amdgcn_sched_barrier(0);        // (loads in the order they are waited for)
+  fetch(odd, kGK);
+  __builtin_amdgcn_sched_barrier(0);
+  stage_in(even, 0);
+  fetch(even, 2 * kGK);
+  __builtin_amdgcn_sched_barrier(0);
+  __syncthreads();
+  read(even, lo_half);
+  int k0 = 0;
+  for (; k0 + 2 * kGK < K; k0 += 2 * kGK) {
+    step(even, odd, std::false_type{}, k0);
+    step(odd, even, std::false_type{}, k0 + kGK);
+  }
+  if (k0 + kGK < K) {
+    step(even, odd, std::false_type{}, k0);
+    step(odd, even, std::true_type{}, k0 + kGK);
+  } else {
+    step(even, odd, std::true_type{}, k0);
   }
   // lane (g4, l15) holds columns 4 g4 .. 4 g4 + 3 of row l15 of each 16 x 16 tile
 #pragma unroll
   for (int j = 0; j < MT; ++j) {
-    const int row = row0 + wm * (BM / 2) + j * 16 + l15;
+    const int row = row0 + (wm * MT + j) * 16 + l15;
     if (row >= end) continue;
 #pragma unroll
     for (int i = 0; i < NT; i += GLU ? 2 : 1) {
-      const int col = n0 + (GLU ? wn * (BN / 4) + i * 8 : wn * (BN / 2) + i * 16) + 4 * g4;
+      const int col = n0 + (GLU ? (wn * NT + i) * 8 : (wn * NT + i) * 16) + 4 * g4;
       if (col >= N) continue;
       float v[4];
 #pragma unroll
@@ -266,20 +353,20 @@ extern "C" int mx_grouped_gemm(void* C, const void* A, const int* rows, const vo
   if (((uintptr_t)A) % 16 || ((uintptr_t)W) % 16) return -2;
   const bool glu = act >= kFrGelu && act <= kFrClamp;
   const int vec = N % 4 == 0 && ((uintptr_t)C) % 8 == 0;
+  if ((M + 63) / 64 + groups > 65535) return -3;
   // 128-row tiles once the groups fill them on average
   const bool tall = M >= 96L * groups;
-  const int bm = tall ? 128 : 64, bn = 128;
-  const long tiles = (M + bm - 1) / bm + groups;
-  if (tiles > 65535) return -3;
-  const int cols = glu ? bn / 2 : bn;
-  const dim3 grid((unsigned)((N + cols - 1) / cols), (unsigned)tiles), block(256);
-#define GG_GO(BM, GLU)                                                                                               \
-  hipLaunchKernelGGL((grouped_gemm_kernel<BM, 128, GLU>), grid, block, 0, s, (bf16_t*)C, (const bf16_t*)A, rows,      \
-                     (const bf16_t*)W, offs, groups, (int)M, N, K, act, limit, vec)
+  const int cols = 128 / (glu ? 2 : 1), col_tiles = (N + cols - 1) / cols;
+  const long tiles = ((M + (tall ? 127 : 63)) / (tall ? 128 : 64) + groups) * col_tiles;
+  if (tiles > 0x7ffffff0L) return -3;
+  const dim3 grid((unsigned)((tiles + 7) / 8 * 8));
+#define GG_GO(MT, GLU)                                                                                       \
+  hipLaunchKernelGGL((grouped_gemm_kernel<MT, GLU>), grid, dim3(256), 0, s, (bf16_t*)C, (const bf16_t*)A, rows, \
+                     (const bf16_t*)W, offs, groups, (int)M, N, K, col_tiles, act, limit, vec)
   if (tall) {
-    if (glu) GG_GO(128, true); else GG_GO(128, false);
+    if (glu) GG_GO(4, true); else GG_GO(4, false);
   } else {
-    if (glu) GG_GO(64, true); else GG_GO(64, false);
+    if (glu) GG_GO(2, true); else GG_GO(2, false);
   }
 #undef GG_GO
   return (int)hipGetLastError();
