@@ -53,8 +53,105 @@ __global__ void short_conv_kernel(T* __restrict__ out, const T* __restrict__ x, 
   st(out, row * channels + c, acc * sigmoidf_(acc));
 }
 
-// history <- the segment's last taps-1 inputs (older ones shift out); runs after
-// short_conv_kernel, one thread per (segment, channel); segments of fewer than min_rows rows
+// The same for TAPS taps and rows of whole 16-byte pieces: a thread owns the V channels of a piece over
+// kConvRows rows, all their loads in flight at once and each input read once per thread instead of once
+// per tap.  Bound by the read and write of the rows: 4096 rows of 6144 channels, bf16, 34 us
+// (one thread per value, 143).  A segment that fits one tile leaves its history here, longer ones to
+// conv_hist_kernel (another workgroup may still read the old history).
+constexpr int kConvRows = 8;
+
+template <typename T, int V>
+__device__ __forceinline__ void ld_piece(const T* p, float (&v)[V]) {
+  const uint4 u = *reinterpret_cast<const uint4*>(p);
+  if constexpr (sizeof(T) == 2) {
+    ft::unpack2(u.x, v[0], v[1]);
+    ft::unpack2(u.y, v[2], v[3]);
+    ft::unpack2(u.z, v[4], v[5]);
+    ft::unpack2(u.w, v[6], v[7]);
+  } else {
+    v[0] = __uint_as_float(u.x), v[1] = __uint_as_float(u.y);
+    v[2] = __uint_as_float(u.z), v[3] = __uint_as_float(u.w);
+  }
+}
+template <typename T, int V>
+__device__ __forceinline__ void st_piece(T* p, const float (&v)[V]) {
+  uint4 u;
+  if constexpr (sizeof(T) == 2)
+    u = make_uint4(ft::pack2(v[0], v[1]), ft::pack2(v[2], v[3]), ft::pack2(v[4], v[5]), ft::pack2(v[6], v[7]));
+  else
+    u = make_uint4(__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3]));
+  *reinterpret_cast<uint4*>(p) = u;
+}
+
+template <typename T, int TAPS>
+__global__ void __launch_bounds__(128)
+short_conv_pieces_kernel(T* __restrict__ out, const T* __restrict__ x, long x_stride, const float* __restrict__ w,
+                         const float* __restrict__ bias, float* __restrict__ hist, const int* __restrict__ start,
+                         const int* __restrict__ pos0, const int* __restrict__ slot, int channels, int num_slots) {
+  constexpr int V = 16 / sizeof(T), kOld = TAPS - 1;
+  const int s = blockIdx.z;
+  const int r0 = start[s], n = start[s + 1] - r0;
+  const int rel0 = blockIdx.y * kConvRows;
+  if (rel0 >= n) return;
+  const int c = (blockIdx.x * 128 + threadIdx.x) * V;
+  if (c >= channels) return;
+  const int sl = slot[s], rows = min(kConvRows, n - rel0);
+  T* o = out + (long)(r0 + rel0) * channels + c;
+  if (sl < 0 || sl >= num_slots) {
+    const float zero[V] = {};
+    for (int r = 0; r < rows; ++r) st_piece<T, V>(o + (long)r * channels, zero);
+    return;
+  }
+  const bool fresh = pos0[s] <= 0;
+  float* h = hist + (long)sl * kOld * channels + c;
+  const T* xp = x + (long)(r0 + rel0) * x_stride + c;
+  float in[kOld + kConvRows][V];
+#pragma unroll
+  for (int r = 0; r < kConvRows; ++r) ld_piece<T, V>(xp + (long)min(r, rows - 1) * x_stride, in[kOld + r]);
+#pragma unroll
+  for (int m = 0; m < kOld; ++m) {
+    const int src = rel0 - kOld + m;
+    if (src >= 0) {
+      ld_piece<T, V>(xp + (long)(m - kOld) * x_stride, in[m]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < V; ++i) in[m][i] = fresh ? 0.f : h[(long)(kOld + src) * channels + i];
+    }
+  }
+  float wc[V][TAPS], b[V];
+#pragma unroll
+  for (int i = 0; i < V; ++i) {
+    b[i] = bias != nullptr ? bias[c + i] : 0.f;
+#pragma unroll
+    for (int j = 0; j < TAPS; ++j) wc[i][j] = w[(long)(c + i) * TAPS + j];
+  }
+#pragma unroll
+  for (int r = 0; r < kConvRows; ++r) {
+    if (r >= rows) break;
+    float y[V];
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+      float acc = b[i];
+#pragma unroll
+      for (int j = 0; j < TAPS; ++j) acc += in[r + j][i] * wc[i][j];
+      y[i] = acc * sigmoidf_(acc);
+    }
+    st_piece<T, V>(o + (long)r * channels, y);
+  }
+  if (n <= kConvRows) {
+#pragma unroll
+    for (int r = 1; r <= kConvRows; ++r) {
+      if (r != n) continue;           // the last TAPS - 1 of the old inputs and the n new ones
+#pragma unroll
+      for (int m = 0; m < kOld; ++m)
+#pragma unroll
+        for (int i = 0; i < V; ++i) h[(long)m * channels + i] = in[r + m][i];
+    }
+  }
+}
+
+// history <- the segment's last taps-1 inputs (older ones shift out); runs after the
+// convolution, one thread per (segment, channel); segments of fewer than min_rows rows
 // are left alone
 template <typename T>
 __global__ void conv_hist_kernel(const T* __restrict__ x, long x_stride, float* __restrict__ hist,
@@ -119,6 +216,88 @@ __global__ void delta_prep_kernel(float* __restrict__ qn, float* __restrict__ kn
       g[(row * heads + h) * dk + i] = expf(-rate * softplusf_(z));
     }
     if (lane == 0) beta[row * heads + h] = sigmoidf_(ld(b, row * b_stride + h));
+  }
+}
+
+// The same for even dk of at most 128 NU: a wave owns an item of kPrepRows rows, a lane two neighbouring
+// channels at a time, all loads in flight at once and kept in registers.  Bound by the writes and the
+// decays' exponentials: 4096 rows of 16 heads of 128, 56 us (a wave per row, values read twice, 73).
+constexpr int kPrepRows = 4;
+
+__device__ __forceinline__ float2 ld_pair(const bf16_t* p) {
+  float2 v;
+  ft::unpack2(*reinterpret_cast<const uint32_t*>(p), v.x, v.y);
+  return v;
+}
+__device__ __forceinline__ float2 ld_pair(const float* p) { return *reinterpret_cast<const float2*>(p); }
+
+template <typename T, int NU>
+__global__ void __launch_bounds__(256)
+delta_prep_pairs_kernel(float* __restrict__ qn, float* __restrict__ kn, float* __restrict__ g, float* __restrict__ beta,
+                        const T* __restrict__ qkv, long qkv_stride, const T* __restrict__ a, long a_stride,
+                        const T* __restrict__ b, long b_stride, const float* __restrict__ a_log,
+                        const float* __restrict__ dt_bias, long rows, int heads, int kv_heads, int dk) {
+  const int items = kv_heads + heads;
+  const long w = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const long row0 = w / items * kPrepRows;
+  if (row0 >= rows) return;
+  const int lane = threadIdx.x & 63, it = (int)(w % items), n = (int)min((long)kPrepRows, rows - row0);
+  if (it < kv_heads) {
+    float2 q[kPrepRows][NU], k[kPrepRows][NU];
+#pragma unroll
+    for (int r = 0; r < kPrepRows; ++r) {
+      const T* p = qkv + (row0 + min(r, n - 1)) * qkv_stride + (long)it * dk;
+#pragma unroll
+      for (int u = 0; u < NU; ++u) {
+        const int i = 128 * u + 2 * lane;
+        q[r][u] = i < dk ? ld_pair(p + i) : make_float2(0.f, 0.f);
+        k[r][u] = i < dk ? ld_pair(p + (long)kv_heads * dk + i) : make_float2(0.f, 0.f);
+      }
+    }
+    const float scale = 1.0f / sqrtf((float)dk);
+#pragma unroll
+    for (int r = 0; r < kPrepRows; ++r) {
+      if (r >= n) break;
+      float sq = 0.f, sk = 0.f;
+#pragma unroll
+      for (int u = 0; u < NU; ++u) {
+        sq += q[r][u].x * q[r][u].x + q[r][u].y * q[r][u].y;
+        sk += k[r][u].x * k[r][u].x + k[r][u].y * k[r][u].y;
+      }
+      const float rq = 1.0f / sqrtf(ft::wave_sum(sq) + 1e-6f) * scale, rk = 1.0f / sqrtf(ft::wave_sum(sk) + 1e-6f);
+      const long at = ((row0 + r) * kv_heads + it) * dk;
+#pragma unroll
+      for (int u = 0; u < NU; ++u) {
+        const int i = 128 * u + 2 * lane;
+        if (i >= dk) continue;
+        *reinterpret_cast<float2*>(qn + at + i) = make_float2(q[r][u].x * rq, q[r][u].y * rq);
+        *reinterpret_cast<float2*>(kn + at + i) = make_float2(k[r][u].x * rk, k[r][u].y * rk);
+      }
+    }
+  } else {
+    const int h = it - kv_heads;
+    const float rate = expf(a_log[h]);
+    float2 z[kPrepRows][NU], bias[NU];
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+      const int i = 128 * u + 2 * lane;
+      bias[u] = i < dk ? make_float2(dt_bias[(long)h * dk + i], dt_bias[(long)h * dk + i + 1]) : make_float2(0.f, 0.f);
+#pragma unroll
+      for (int r = 0; r < kPrepRows; ++r)
+        z[r][u] = i < dk ? ld_pair(a + (row0 + min(r, n - 1)) * a_stride + (long)h * dk + i) : make_float2(0.f, 0.f);
+    }
+#pragma unroll
+    for (int r = 0; r < kPrepRows; ++r) {
+      if (r >= n) break;
+#pragma unroll
+      for (int u = 0; u < NU; ++u) {
+        const int i = 128 * u + 2 * lane;
+        if (i >= dk) continue;
+        *reinterpret_cast<float2*>(g + ((row0 + r) * heads + h) * dk + i) =
+            make_float2(expf(-rate * softplusf_(z[r][u].x + bias[u].x)), expf(-rate * softplusf_(z[r][u].y + bias[u].y)));
+      }
+    }
+    if (lane < n) beta[(row0 + lane) * heads + h] = sigmoidf_(ld(b, (row0 + lane) * b_stride + h));
   }
 }
 
@@ -280,14 +459,28 @@ extern "C" int mx_short_conv_silu(void* out, const void* x, int bf16, long x_str
   if (num_segs <= 0 || max_rows <= 0 || channels <= 0) return 0;
   if (taps < 1 || taps > kMaxTaps) return -1;
   const dim3 block(256);
-  const dim3 grid((channels + 255) / 256, max_rows, num_segs);
-  if (grid.y > 65535 || grid.z > 65535) return -2;
-  MX_DISPATCH_T(bf16, hipLaunchKernelGGL((short_conv_kernel<T>), grid, block, 0, s, (T*)out, (const T*)x, x_stride,
-                                         w, bias, hist, start, pos0, slot, channels, taps, num_slots));
-  if (taps > 1)
+  int hist_from = 1;
+  const int v = bf16 ? 8 : 4;
+  if (taps >= 2 && taps <= 4 && channels % v == 0 && x_stride % v == 0 && ((uintptr_t)x) % 16 == 0 &&
+      ((uintptr_t)out) % 16 == 0) {
+    const dim3 grid((channels / v + 127) / 128, (max_rows + kConvRows - 1) / kConvRows, num_segs);
+    if (max_rows > 65535 || grid.z > 65535) return -2;
+#define MX_CONV(TAPS)                                                                                            \
+  MX_DISPATCH_T(bf16, hipLaunchKernelGGL((short_conv_pieces_kernel<T, TAPS>), grid, dim3(128), 0, s, (T*)out,    \
+                                         (const T*)x, x_stride, w, bias, hist, start, pos0, slot, channels, num_slots))
+    if (taps == 4) { MX_CONV(4); } else if (taps == 3) { MX_CONV(3); } else { MX_CONV(2); }
+#undef MX_CONV
+    hist_from = kConvRows + 1;
+  } else {
+    const dim3 grid((channels + 255) / 256, max_rows, num_segs);
+    if (grid.y > 65535 || grid.z > 65535) return -2;
+    MX_DISPATCH_T(bf16, hipLaunchKernelGGL((short_conv_kernel<T>), grid, block, 0, s, (T*)out, (const T*)x, x_stride,
+                                           w, bias, hist, start, pos0, slot, channels, taps, num_slots));
+  }
+  if (taps > 1 && max_rows >= hist_from)
     MX_DISPATCH_T(bf16, hipLaunchKernelGGL((conv_hist_kernel<T>), dim3((channels + 255) / 256, num_segs),
                                            block, 0, s, (const T*)x, x_stride, hist, start, pos0, slot,
-                                           channels, taps, num_slots, 1));
+                                           channels, taps, num_slots, hist_from));
   return (int)hipGetLastError();
 }
 
@@ -309,7 +502,21 @@ extern "C" int mx_delta_prep(float* qn, float* kn, float* g, float* beta, const 
                              int dk, hipStream_t s) {
   const long waves = rows * (heads + kv_heads);
   if (waves <= 0) return 0;
-  const dim3 grid((unsigned)((waves + 3) / 4)), block(256);
+  const dim3 block(256);
+  const size_t pair = bf16 ? 4 : 8;
+  if (dk % 2 == 0 && dk <= 256 && qkv_stride % 2 == 0 && a_stride % 2 == 0 && ((uintptr_t)qkv) % pair == 0 &&
+      ((uintptr_t)a) % pair == 0 && (((uintptr_t)qn) | ((uintptr_t)kn) | ((uintptr_t)g)) % 8 == 0) {
+    const long quads = (rows + kPrepRows - 1) / kPrepRows * (heads + kv_heads);
+    const dim3 grid((unsigned)((quads + 3) / 4));
+#define MX_PREP(NU)                                                                                               \
+  MX_DISPATCH_T(bf16, hipLaunchKernelGGL((delta_prep_pairs_kernel<T, NU>), grid, block, 0, s, qn, kn, g, beta,    \
+                                         (const T*)qkv, qkv_stride, (const T*)a, a_stride, (const T*)b, b_stride, \
+                                         a_log, dt_bias, rows, heads, kv_heads, dk))
+    if (dk <= 128) { MX_PREP(1); } else { MX_PREP(2); }
+#undef MX_PREP
+    return (int)hipGetLastError();
+  }
+  const dim3 grid((unsigned)((waves + 3) / 4));
   MX_DISPATCH_T(bf16, hipLaunchKernelGGL((delta_prep_kernel<T>), grid, block, 0, s, qn, kn, g, beta,
                                          (const T*)qkv, qkv_stride, (const T*)a, a_stride, (const T*)b,
                                          b_stride, a_log, dt_bias, rows, heads, kv_heads, dk));
