@@ -69,34 +69,6 @@ __device__ __forceinline__ float ba_exp(float x) {
   return fmaf(e, r * 0.693147181f, e);
 }
 
-// the work item: segment and block of pairs within it (false: none).  Later blocks, which see more
-// keys, come first.
-__device__ __forceinline__ bool band_item(const BandArgs& A, int rep, int per, int item, int& seg, int& block) {
-  const int lane = threadIdx.x & 63;
-  for (int s0 = 0; s0 < A.num_segs; s0 += 64) {
-    const int s = s0 + lane;
-    int n = 0;
-    if (s < A.num_segs) n = A.start[s + 1] - A.start[s];
-    const int cnt = n >= A.min_rows ? (n * rep + per - 1) / per : 0;
-    int sum = cnt;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int v = __shfl_up(sum, o);
-      if (lane >= o) sum += v;
-    }
-    const uint64_t m = __ballot(sum > item);
-    if (m) {
-      const int l = __builtin_ctzll(m);
-      seg = s0 + l;
-      const int c = __shfl(cnt, l);
-      block = c - 1 - (item - (__shfl(sum, l) - c));
-      return true;
-    }
-    item -= __shfl(sum, 63);
-  }
-  return false;
-}
-
 // the score terms a kernel is built for (run-time tests per score cost as much as the products: a
 // block-masked 777-row layer took 70 us with them)
 enum { kBandPlain = 0, kBandCap = 1, kBandDist = 2, kBandSigmoid = 3, kBandAny = 4 };
@@ -119,7 +91,7 @@ band_attn_kernel(BandArgs A) {
   const int n = lane & 15, g4 = lane >> 4;
   const int rep = A.heads / A.kv_heads, gk = blockIdx.y, kvh = gk / A.maps, map = gk % A.maps;
   int seg, block;
-  if (!band_item(A, rep, 16 * WV, blockIdx.x, seg, block)) return;
+  if (!segment_block(A.start, A.num_segs, A.min_rows, rep, 16 * WV, blockIdx.x, seg, block)) return;
   seg = __builtin_amdgcn_readfirstlane(seg);
   block = __builtin_amdgcn_readfirstlane(block);
   const int r0 = A.start[seg], rows = A.start[seg + 1] - r0, p0 = A.pos0[seg];

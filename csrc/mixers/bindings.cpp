@@ -182,6 +182,11 @@ int mx_moe_pairs(float* out, void* y, const void* h, int bf16, long h_stride, co
 int mx_moe_topk(int* idx, float* wts, const float* z, const float* corr, long rows, int experts, int top,
                 int groups, int keep, hipStream_t s);
 int mx_few_rows_max();
+int mx_latent_prefill_fits(int rank, int dr, int block_size);
+int mx_latent_prefill(float* out, const float* qa, const float* qr, const void* cache, const int* start, const int* pos0,
+                      const int* kv_len, const int* bt, int bt_stride, int num_segs, int long_segs, long long_rows,
+                      int heads, long total_rows, int rank, int dr, int block_size, int num_blocks, float scale,
+                      int min_rows, const float* sink, hipStream_t s);
 int mx_band_attn_fits(int dk, int dv, int block_size);
 int mx_band_attn(float* out, const float* q, const void* k_cache, const void* v_cache, const int* start,
                  const int* pos0, const int* kv_len, const int* bt, int bt_stride, int num_segs, int long_segs,
@@ -1117,6 +1122,27 @@ void window_attention(Tensor out, Tensor q, Tensor k_cache, Tensor v_cache, Tens
       "window_attention");
 }
 
+void latent_prefill(Tensor out, Tensor qa, Tensor qr, Tensor cache, Tensor start, Tensor pos0, Tensor kv_len, Tensor bt,
+                    int64_t num_segs, int64_t long_segs, int64_t long_rows, double scale, int64_t rank, int64_t min_rows,
+                    OptT sink) {
+  check_f32(out, "out");
+  check_f32(qa, "qa");
+  check_f32(qr, "qr");
+  TORCH_CHECK(qa.dim() == 3 && qr.dim() == 3 && qa.size(2) == rank && out.sizes() == qa.sizes() &&
+              qr.size(0) == qa.size(1) && qr.size(1) == qa.size(0) && min_rows >= 1, "latent prefill queries");
+  const int64_t heads = qa.size(0), t = qa.size(1), dr = qr.size(2);
+  TORCH_CHECK(cache.is_cuda() && cache.is_contiguous() && cache.scalar_type() == at::kBFloat16 && cache.dim() == 3 &&
+              cache.size(2) == rank + dr, "latent cache");
+  check_segs(start, pos0, kv_len, num_segs);
+  check_i32(bt, "block tables");
+  TORCH_CHECK(bt.dim() == 2 && bt.size(0) >= num_segs && long_rows <= t && long_segs <= num_segs, "block tables / rows");
+  chk(mx_latent_prefill(out.data_ptr<float>(), qa.data_ptr<float>(), qr.data_ptr<float>(), cache.data_ptr(),
+                        start.data_ptr<int>(), pos0.data_ptr<int>(), kv_len.data_ptr<int>(), bt.data_ptr<int>(),
+                        (int)bt.size(1), (int)num_segs, (int)long_segs, long_rows, (int)heads, t, (int)rank, (int)dr,
+                        (int)cache.size(1), (int)cache.size(0), (float)scale, (int)min_rows,
+                        opt_f32(sink, heads, "sink"), stream()), "latent_prefill");
+}
+
 void band_attention(Tensor out, Tensor q, Tensor k_cache, Tensor v_cache, Tensor start, Tensor pos0, Tensor kv_len,
                     Tensor bt, int64_t num_segs, int64_t long_segs, int64_t long_rows, int64_t heads, int64_t maps,
                     int64_t kv_heads, int64_t dk, int64_t dv, int64_t window, double scale, bool sigmoid, OptT r1,
@@ -1434,6 +1460,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("attn_prep", &attn_prep);
   m.def("window_attention", &window_attention);
   m.def("band_weights", &band_weights);
+  m.def("latent_prefill", &latent_prefill);
+  m.def("latent_prefill_fits", [](int64_t rank, int64_t dr, int64_t bs) {
+    return mx_latent_prefill_fits((int)rank, (int)dr, (int)bs) != 0;
+  });
   m.def("band_attention", &band_attention);
   m.def("band_attention_fits", [](int64_t dk, int64_t dv, int64_t bs) {
     return mx_band_attn_fits((int)dk, (int)dv, (int)bs) != 0;

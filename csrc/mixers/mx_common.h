@@ -232,6 +232,35 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
   return s;
 }
 
+// the work item: segment and block of `per` pairs within it, `rep` pairs a row (false: none), of the segments
+// of at least min_rows rows.  Later blocks, which see more keys, come first.
+__device__ __forceinline__ bool segment_block(const int* start, int num_segs, int min_rows, int rep, int per, int item,
+                                              int& seg, int& block) {
+  const int lane = threadIdx.x & 63;
+  for (int s0 = 0; s0 < num_segs; s0 += 64) {
+    const int s = s0 + lane;
+    int n = 0;
+    if (s < num_segs) n = start[s + 1] - start[s];
+    const int cnt = n >= min_rows ? (n * rep + per - 1) / per : 0;
+    int sum = cnt;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(sum, o);
+      if (lane >= o) sum += v;
+    }
+    const uint64_t m = __ballot(sum > item);
+    if (m) {
+      const int l = __builtin_ctzll(m);
+      seg = s0 + l;
+      const int c = __shfl(cnt, l);
+      block = c - 1 - (item - (__shfl(sum, l) - c));
+      return true;
+    }
+    item -= __shfl(sum, 63);
+  }
+  return false;
+}
+
 }  // namespace mx
 
 #define MX_DISPATCH_T(bf16, ...)            \

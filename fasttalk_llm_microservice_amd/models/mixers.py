@@ -133,11 +133,12 @@ class LatentAttention:
         qa = torch.bmm(qn.transpose(0, 1), self.wuk)                 # [heads, T, rank]
         seg = ctx.seg
         if seg.host is not None and seg.max_rows >= self.PRODUCT_ROWS:
-            # prefill chunks: two tiled products per segment; short segments and decode
-            # rows (if any) keep the per-row kernel
-            ol = torch.zeros_like(qa)
-            M.latent_attention(qa, qr, cache, seg, self.scale, self.rank, skip_from=self.PRODUCT_ROWS,
-                               out=ol, sink=self.sink)
+            # prefill chunks in tiles; short segments and decode rows (if any) keep the per-row
+            # kernel (every row belongs to a segment, short or long)
+            ol = torch.empty_like(qa)
+            if min(b - a for a, b in zip(seg.host[0][:-1], seg.host[0][1:])) < self.PRODUCT_ROWS:
+                M.latent_attention(qa, qr, cache, seg, self.scale, self.rank, skip_from=self.PRODUCT_ROWS,
+                                   out=ol, sink=self.sink)
             M.latent_attention_products(ol, qa, qr, cache, seg, self.scale, self.rank,
                                         self.PRODUCT_ROWS, self.dtype, self.sink)
         else:

@@ -560,6 +560,27 @@ def mm_f32(a, b):
 PRODUCT_SCORE_BYTES = 1 << 30
 
 
+def latent_prefill_ok(qa, cache, rank: int, dtype) -> bool:
+    """Whether long segments run in one kernel (csrc/mixers/latent_prefill.hip) instead of two products."""
+    return bool(qa.is_cuda and dtype == torch.bfloat16 and cache.dtype == torch.bfloat16
+                and native_mixers().latent_prefill_fits(rank, cache.shape[2] - rank, cache.shape[1]))
+
+
+def _latent_prefill_pays(seg: Segments, heads: int, min_rows: int) -> bool:
+    """A workgroup of the one kernel owns 128 (row, head) pairs and walks their keys, 32 in 1.9 us, so few
+    pairs with many earlier keys leave the chip idle: 64 rows of 16 heads at position 4000 take 245 us, the two
+    products 105; 512 rows at 3500 238 and 250; 300 rows from 0 41 and 93.  The products cost about 80 us of
+    launches a segment and 4.8 us per million pairs times keys."""
+    start, _, kv_len = seg.host
+    blocks = keys = products = 0
+    for a, b, kv in zip(start[:-1], start[1:], kv_len):
+        if b - a >= min_rows:
+            blocks += ((b - a) * heads + 127) // 128
+            keys = max(keys, kv)
+            products += 80 + 4.8e-6 * (b - a) * heads * kv
+    return 20 + 0.06 * keys * ((blocks + 255) // 256) <= products
+
+
 def latent_attention_products(out, qa, qr, cache, seg: Segments, scale: float, rank: int,
                               min_rows: int, dtype, sink: Optional[torch.Tensor] = None):
     """Segments of ``min_rows`` rows or more as two matrix products: all heads share
@@ -570,6 +591,11 @@ def latent_attention_products(out, qa, qr, cache, seg: Segments, scale: float, r
     heads = qa.shape[0]
     bs = cache.shape[1]
     width = cache.shape[2]
+    if latent_prefill_ok(qa, cache, rank, dtype) and _latent_prefill_pays(seg, heads, min_rows):
+        ns = [n for n in (b - a for a, b in zip(start[:-1], start[1:])) if n >= min_rows]
+        native_mixers().latent_prefill(out, qa, qr, cache, seg.start, seg.pos0, seg.kv_len, seg.block_tables, seg.num,
+                                       len(ns), sum(ns), float(scale), rank, min_rows, sink)
+        return out
     for s in range(seg.num):
         a, b = start[s], start[s + 1]
         n = b - a

@@ -1,0 +1,77 @@
+"""Latent attention of long segments in one kernel (csrc/mixers/latent_prefill.hip) against 64 bits."""
+import pytest
+import torch
+
+from fasttalk_llm_microservice_amd.ops import mixers as M
+from test_mixer_kernels_gpu import DEV, make_seg, to_dev
+
+pytestmark = pytest.mark.gpu
+RANK, DR = 512, 64
+
+
+def reference(qa, qr, cache, seg, lens, pos0, scale, sink):
+    """fp64 on the kernel's operands (queries rounded to bf16); also sum_j p_j |c_j|."""
+    heads, t, _ = qa.shape
+    qa, qr = qa.bfloat16().double(), qr.bfloat16().double()
+    out, size, a = torch.zeros(heads, t, RANK, dtype=torch.float64, device=DEV), None, 0
+    size = torch.zeros_like(out)
+    for s, n in enumerate(lens):
+        b, kv = a + n, pos0[s] + n
+        bs = cache.shape[1]
+        k = cache[seg.block_tables[s, :(kv + bs - 1) // bs].long()].reshape(-1, RANK + DR)[:kv].double()
+        sc = (qa[:, a:b] @ k[:, :RANK].t() + (qr[a:b] @ k[:, RANK:].t()).transpose(0, 1)) * scale
+        see = torch.arange(kv, device=DEV)[None] <= (pos0[s] + torch.arange(n, device=DEV))[:, None]
+        sc = sc.masked_fill(~see, float("-inf"))
+        top = sc.max(-1, keepdim=True).values
+        if sink is not None:
+            top = torch.maximum(top, sink.double()[:, None, None])
+        p = (sc - top).exp()
+        den = p.sum(-1, keepdim=True)
+        if sink is not None:
+            den = den + (sink.double()[:, None, None] - top).exp()
+        out[:, a:b] = p / den @ k[:, :RANK]
+        size[:, a:b] = p / den @ k[:, :RANK].abs()
+        a = b
+    return out, size
+
+
+@pytest.mark.parametrize("sink", [False, True])
+@pytest.mark.parametrize("lens,pos0,heads,page", [
+    ([32], [0], 1, 8),                              # one tile of keys, a quarter of a workgroup's pairs
+    ([128, 40, 3, 64], [31, 0, 5, 2], 1, 16),       # whole workgroups; a short segment, left alone
+    ([33, 100, 65], [7, 0, 130], 3, 8),             # heads that do not divide 128
+    ([43], [1], 16, 64),
+    ([70], [900], 5, 8),                           # more than 64 pages
+])
+@pytest.mark.parametrize("rise", [0.0, 0.05])       # scores that grow with the key: the reference moves often
+def test_latent_prefill(lens, pos0, heads, page, sink, rise):
+    g = torch.Generator(device=DEV).manual_seed(sum(lens) + heads)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=DEV)      # noqa: E731
+    seg, _ = make_seg(lens, pos0, list(range(len(lens))), block_size=page)
+    seg = to_dev(seg)
+    seg.host = (seg.start.tolist(), seg.pos0.tolist(), seg.kv_len.tolist())
+    t = sum(lens)
+    cache = rnd(int(seg.block_tables.max()) + 1, page, RANK + DR)
+    qa, qr, scale = rnd(heads, t, RANK), rnd(t, heads, DR), 0.07
+    if rise:
+        for s in range(len(lens)):
+            kv = pos0[s] + lens[s]
+            rows = cache[seg.block_tables[s, :(kv + page - 1) // page].long()]
+            rows.view(-1, RANK + DR)[:, -1] = rise * torch.arange(rows.shape[0] * page, device=DEV)
+            cache[seg.block_tables[s, :rows.shape[0]].long()] = rows
+        qr[:, :, -1] = 20.0
+    cache = cache.bfloat16()
+    sinks = rnd(heads) * 3 if sink else None
+    assert M.latent_prefill_ok(qa, cache, RANK, torch.bfloat16) and M._latent_prefill_pays(seg, heads, 32)
+    out = torch.full((heads, t, RANK), 7.0, device=DEV)
+    M.latent_attention_products(out, qa, qr, cache, seg, scale, RANK, 32, torch.bfloat16, sinks)
+    want, size = reference(qa, qr, cache, seg, lens, pos0, scale, sinks)
+    a = 0
+    for n in lens:
+        got, w, z = out[:, a:a + n].double(), want[:, a:a + n], size[:, a:a + n]
+        if n < 32:
+            assert bool((got == 7.0).all())
+        else:
+            # weights rounded to bf16 (half a unit: 2^-8); scores of up to 2^8 and their sums in fp32 (2^-12)
+            assert bool(((got - w).abs() <= (2 ** -8 + 2 ** -12) * z + 1e-6).all())
+        a += n
