@@ -182,6 +182,7 @@ int mx_moe_pairs(float* out, void* y, const void* h, int bf16, long h_stride, co
 int mx_moe_topk(int* idx, float* wts, const float* z, const float* corr, long rows, int experts, int top,
                 int groups, int keep, hipStream_t s);
 int mx_few_rows_max();
+int mx_latent_decode_fits(int rank, int dr, int cache_bf16);
 int mx_latent_prefill_fits(int rank, int dr, int block_size);
 int mx_latent_prefill(float* out, const float* qa, const float* qr, const void* cache, const int* start, const int* pos0,
                       const int* kv_len, const int* bt, int bt_stride, int num_segs, int long_segs, long long_rows,
@@ -791,10 +792,12 @@ void latent_attention(Tensor out, Tensor qa, Tensor qr, Tensor cache, Tensor sta
   check_i32(bt, "block tables");
   TORCH_CHECK(bt.dim() == 2 && bt.size(0) >= num_segs && max_rows <= t, "block tables / max_rows");
   if (mx_latent_split_ws((int)heads, (int)rank, (int)dr)) {
-    // key slices: enough workgroups to fill the chip (at most 16), at least ~64 keys per slice when
+    // key slices: enough workgroups to fill the chip (at most 16; 32 of the matrix-unit form, whose workgroups
+    // are a slice's chain of a few microseconds), at least ~64 keys per slice when
     // the longest context is known (max_kv; 0 inside captured graphs), scratch <= 256 MiB
     int64_t rows = std::max<int64_t>(1, std::min<int64_t>(t, num_segs * std::max<int64_t>(1, std::min(max_rows, skip_from > 0 ? skip_from - 1 : max_rows))));
-    int64_t splits = std::max<int64_t>(1, std::min<int64_t>(16, 256 / rows));
+    const bool units = mx_latent_decode_fits((int)rank, (int)dr, bf(cache)) != 0;
+    int64_t splits = std::max<int64_t>(1, std::min<int64_t>(units ? 32 : 16, (units ? 512 : 256) / rows));
     if (max_kv > 0) splits = std::max<int64_t>(1, std::min(splits, (max_kv + 63) / 64));
     while (splits > 1 && t * splits * heads * rank * 4 > (256LL << 20)) splits /= 2;
     auto f32 = qa.options();

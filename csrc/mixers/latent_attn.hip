@@ -523,6 +523,12 @@ static void launch_split(dim3 grid, size_t lds, hipStream_t s, float* ws_acc, fl
                      block_size, num_blocks, scale, skip_from, splits, hg, tk);
 }
 
+extern "C" int mx_latent_decode_fits(int rank, int dr, int cache_bf16);
+extern "C" int mx_latent_decode(float* ws_acc, float* ws_ml, const float* qa, const float* qr, const void* cache,
+                                const int* start, const int* pos0, const int* kv_len, const int* bt, int bt_stride,
+                                int num_segs, int max_rows, int heads, long total_rows, int block_size, int num_blocks,
+                                float scale, int skip_from, int splits, hipStream_t s);
+
 extern "C" int mx_latent_attention_split(float* out, float* ws_acc, float* ws_ml, const float* qa,
                                          const float* qr, const void* cache, int cache_bf16, const int* start,
                                          const int* pos0, const int* kv_len, const int* bt, int bt_stride,
@@ -538,6 +544,13 @@ extern "C" int mx_latent_attention_split(float* out, float* ws_acc, float* ws_ml
   if (!acc || splits < 1 || splits > 64 || max_rows > 65535 || num_segs > 65535 || heads > 65535) return -1;
   const int groups = (heads + hg - 1) / hg;
   const dim3 grid(splits * groups, max_rows, num_segs);
+  if (mx_latent_decode_fits(rank, dr, cache_bf16) &&
+      ((((uintptr_t)qa) | ((uintptr_t)qr) | ((uintptr_t)cache) | ((uintptr_t)ws_acc)) % 16 == 0)) {
+    // same slices on the matrix units
+    const int rc = mx_latent_decode(ws_acc, ws_ml, qa, qr, cache, start, pos0, kv_len, bt, bt_stride, num_segs, max_rows,
+                                    heads, total_rows, block_size, num_blocks, scale, skip_from, splits, s);
+    if (rc != 0) return rc;
+  } else {
 #define MX_SPLIT(A)                                                                                      \
   do {                                                                                                   \
     if (cache_bf16)                                                                                      \
@@ -555,6 +568,7 @@ extern "C" int mx_latent_attention_split(float* out, float* ws_acc, float* ws_ml
   else if (acc <= 32) MX_SPLIT(32);
   else MX_SPLIT(64);
 #undef MX_SPLIT
+  }
   const dim3 g2(max_rows, num_segs, (heads * ((rank + 255) / 256) + 3) / 4);
   if (rank % 4 == 0 && ((uintptr_t)ws_acc) % 16 == 0)
     hipLaunchKernelGGL((latent_combine_kernel<true>), g2, dim3(256), 0, s, out, ws_acc, ws_ml, start, heads,

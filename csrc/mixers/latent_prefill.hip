@@ -12,10 +12,6 @@
 // one's operand with no exchange between lanes.  Tiles of 32 keys go to LDS by global_load_lds_dwordx4 into
 // a ring of four, two in flight; both products read the same rows, the second one through
 // ds_read_b64_tr_b16.
-// LDS image of a tile: 16-byte piece p of key k at ((p / 8 * 4 + k / 8) * 8 + k % 8) * 8 + (p % 8 ^ lp_swap(k)):
-// eight neighbouring lanes of a load read 128 neighbouring bytes of a cache row (with a key per lane the load
-// unit, one line at a time, took 5% more), and neither way of reading has bank conflicts within 16 lanes (those
-// counted are a tenth of the cycles).
 // The running maximum is a reference: it moves (and the sums are rescaled) only when a score exceeds it by a
 // factor of 2^8, so the weights stay within fp32 and bf16 range and their relative rounding is the same.
 //
@@ -27,21 +23,13 @@
 // 16 heads, from position 0: 4096 rows 305 us (0.95 PFLOP/s, of 1.46 for a large product; what is left is the
 // wait at each tile's barrier), 2048 rows 141, 777 rows 70, 300 rows 41.  Two products through memory with a
 // softmax kernel between them: 1360, 428, 126, 93 us and 9 launches per segment.
-#include "mx_common.h"
-#include "../kernels/ft_lds.h"
+#include "latent_tile.h"
 
 namespace mx {
 
-typedef __bf16 lp_bf16x8 __attribute__((ext_vector_type(8)));
-typedef float lp_f32x4 __attribute__((ext_vector_type(4)));
-typedef short lp_i16x4 __attribute__((ext_vector_type(4)));
-
-constexpr int kLpRank = 512, kLpRot = 64, kLpWidth = kLpRank + kLpRot;
-constexpr int kLpKeys = 32, kLpPairs = 128, kLpSlots = 4;
-constexpr int kLpTile = kLpKeys * kLpWidth * 2;       // bytes
+constexpr int kLpPairs = 128, kLpSlots = 4;
 constexpr int kLpInReg = 16;                          // query steps of 32 in registers, the rest in LDS
 constexpr int kLpAhead = 3;
-constexpr int kLpDma = kLpTile / 4096;                // 1 KiB loads per wave and tile
 
 struct LatPreArgs {
   float* out;
@@ -54,13 +42,6 @@ struct LatPreArgs {
   float scale;
   const float* sink;
 };
-
-__device__ __forceinline__ int lp_swap(int key) { return ((key >> 1) & 3) * 2 + ((key >> 3) & 1); }
-
-__device__ __forceinline__ lp_f32x4 lp_mfma(const uint4& a, const uint4& b, lp_f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(lp_bf16x8, a), __builtin_bit_cast(lp_bf16x8, b), c,
-                                                 0, 0, 0);
-}
 
 // d += a b with d in the accumulation registers (the compiler's own choice is one kind of register for every
 // product of a kernel, and a wave's sums alone take 256).  The wait states cover operands that a vector
@@ -149,23 +130,12 @@ latent_prefill_kernel(LatPreArgs A) {
     if (page - page0 >= 64) ids = pages(page);
     const int key = min(k0 + (lane >> 3), keys - 1);
     const long at = ((long)__builtin_amdgcn_readlane(ids, page - page0) << A.page_shift) + (key & ((1 << A.page_shift) - 1));
-    const bf16_t* src = A.cache + at * kLpWidth + ((lane & 7) ^ lp_swap(8 * wave + (lane >> 3))) * 8;
-    const uint32_t dst = lds0 + (t % kLpSlots) * kLpTile + wave * 1024;
-#pragma unroll
-    for (int i = 0; i < kLpDma; ++i) ft::glds16(src + i * 64, dst + i * 4096);
+    lp_issue(A.cache + at * kLpWidth, wave, lane, lds0 + (t % kLpSlots) * kLpTile);
   };
   for (int t = 0; t < 2 && t < tiles; ++t) issue(t);
 
-  // byte offsets in a tile.  First product: piece 4 s + g4 of key n (odd s: 4 pieces on; key tile 1: 2048 on).
-  // Second: key n / 4 of this group's four, columns 4 (n % 4) .. of a 16-column tile
-  int k_off[2];
-#pragma unroll
-  for (int h = 0; h < 2; ++h) k_off[h] = n * 128 + ((4 * h + g4) ^ lp_swap(n)) * 16;
-  const int vkey = 4 * g4 + (n >> 2);
-  int v_off[4];                           // column tile mod 4: pieces 2 j, 2 j + 1
-#pragma unroll
-  for (int j = 0; j < 4; ++j)
-    v_off[j] = vkey * 128 + ((2 * j + ((n >> 1) & 1)) ^ lp_swap(vkey)) * 16 + (n & 1) * 8;
+  int k_off[2], v_off[4];
+  lp_offsets(n, g4, k_off, v_off);
 
   lp_f32x4 s[2][2];                       // a tile's scores, [key tile][pair tile]
   float x[2][8], top;                     // exponents (base 2) relative to the reference, then weights
@@ -210,16 +180,9 @@ latent_prefill_kernel(LatPreArgs A) {
   };
   // O^T += C^T P^T of a tile, `with` likewise
   auto sums = [&](const uint8_t* tile, auto with) {
-    typedef __attribute__((address_space(3))) lp_i16x4 lds_i16x4;
     auto v_read = [&](int step) {         // column tiles 2 step, 2 step + 1
 #pragma unroll
-      for (int d = 0; d < 2; ++d) {
-        const int u = 2 * step + d;
-        const uint8_t* at = tile + (u >> 2) * 4096 + v_off[u & 3];
-        const uint2 lo = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)at));
-        const uint2 hi = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(at + 2048)));
-        ops[step % (kLpAhead + 1)][d] = make_uint4(lo.x, lo.y, hi.x, hi.y);
-      }
+      for (int d = 0; d < 2; ++d) ops[step % (kLpAhead + 1)][d] = lp_values(tile, 2 * step + d, v_off);
     };
 #pragma unroll
     for (int step = 0; step < kLpAhead; ++step) v_read(step);
