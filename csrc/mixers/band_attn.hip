@@ -52,14 +52,6 @@ __device__ __forceinline__ ba_f32x4 ba_mfma(const uint4& a, const uint4& b, ba_f
                                                  0, 0, 0);
 }
 
-// two fp32 values -> their hi, mid and lo bf16 parts
-__device__ __forceinline__ void ba_split(float a, float b, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
-  hi = ft::pack2(a, b);
-  const float a1 = a - __uint_as_float(hi << 16), b1 = b - __uint_as_float(hi & 0xffff0000u);
-  mid = ft::pack2(a1, b1);
-  lo = ft::pack2(a1 - __uint_as_float(mid << 16), b1 - __uint_as_float(mid & 0xffff0000u));
-}
-
 // e^x for x <= 0, the argument's rounding in base 2 made good; 0 far below; NaN stays NaN
 __device__ __forceinline__ float ba_exp(float x) {
   x = x < -150.f ? -150.f : x;
@@ -123,10 +115,10 @@ band_attn_kernel(BandArgs A) {
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
       const float4 u = *reinterpret_cast<const float4*>(src + 32 * s), v = *reinterpret_cast<const float4*>(src + 32 * s + 4);
-      ba_split(u.x, u.y, qp[0][s].x, qp[1][s].x, qp[2][s].x);
-      ba_split(u.z, u.w, qp[0][s].y, qp[1][s].y, qp[2][s].y);
-      ba_split(v.x, v.y, qp[0][s].z, qp[1][s].z, qp[2][s].z);
-      ba_split(v.z, v.w, qp[0][s].w, qp[1][s].w, qp[2][s].w);
+      split_bf16x3(u.x, u.y, qp[0][s].x, qp[1][s].x, qp[2][s].x);
+      split_bf16x3(u.z, u.w, qp[0][s].y, qp[1][s].y, qp[2][s].y);
+      split_bf16x3(v.x, v.y, qp[0][s].z, qp[1][s].z, qp[2][s].z);
+      split_bf16x3(v.z, v.w, qp[0][s].w, qp[1][s].w, qp[2][s].w);
     }
   }
   const float c1 = use_terms ? A.r1[a] : 0.f, c2 = use_terms ? A.r2[a] : 0.f;
@@ -266,10 +258,10 @@ band_attn_kernel(BandArgs A) {
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb) {
       uint4 pp[3];
-      ba_split(sc[2 * kb][0], sc[2 * kb][1], pp[0].x, pp[1].x, pp[2].x);
-      ba_split(sc[2 * kb][2], sc[2 * kb][3], pp[0].y, pp[1].y, pp[2].y);
-      ba_split(sc[2 * kb + 1][0], sc[2 * kb + 1][1], pp[0].z, pp[1].z, pp[2].z);
-      ba_split(sc[2 * kb + 1][2], sc[2 * kb + 1][3], pp[0].w, pp[1].w, pp[2].w);
+      split_bf16x3(sc[2 * kb][0], sc[2 * kb][1], pp[0].x, pp[1].x, pp[2].x);
+      split_bf16x3(sc[2 * kb][2], sc[2 * kb][3], pp[0].y, pp[1].y, pp[2].y);
+      split_bf16x3(sc[2 * kb + 1][0], sc[2 * kb + 1][1], pp[0].z, pp[1].z, pp[2].z);
+      split_bf16x3(sc[2 * kb + 1][2], sc[2 * kb + 1][3], pp[0].w, pp[1].w, pp[2].w);
       uint4 vf[DT];
 #pragma unroll
       for (int t = 0; t < DT; ++t)

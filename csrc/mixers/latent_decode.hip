@@ -17,14 +17,6 @@ namespace mx {
 
 constexpr int kLdKeys = 64;
 
-// two fp32 values -> their hi, mid and lo bf16 parts
-__device__ __forceinline__ void ld_split(float a, float b, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
-  hi = ft::pack2(a, b);
-  const float a1 = a - __uint_as_float(hi << 16), b1 = b - __uint_as_float(hi & 0xffff0000u);
-  mid = ft::pack2(a1, b1);
-  lo = ft::pack2(a1 - __uint_as_float(mid << 16), b1 - __uint_as_float(mid & 0xffff0000u));
-}
-
 __global__ void __launch_bounds__(512, 1)
 latent_decode_kernel(float* __restrict__ ws_acc, float* __restrict__ ws_ml, const float* __restrict__ qa,
                      const float* __restrict__ qr, const bf16_t* __restrict__ cache, const int* __restrict__ start,
@@ -81,10 +73,10 @@ latent_decode_kernel(float* __restrict__ ws_acc, float* __restrict__ ws_ml, cons
 #pragma unroll
   for (int i = 0; i < QS; ++i) {
     const float4 x = qf[i][0], y = qf[i][1];
-    ld_split(x.x, x.y, q[i][0].x, q[i][1].x, q[i][2].x);
-    ld_split(x.z, x.w, q[i][0].y, q[i][1].y, q[i][2].y);
-    ld_split(y.x, y.y, q[i][0].z, q[i][1].z, q[i][2].z);
-    ld_split(y.z, y.w, q[i][0].w, q[i][1].w, q[i][2].w);
+    split_bf16x3(x.x, x.y, q[i][0].x, q[i][1].x, q[i][2].x);
+    split_bf16x3(x.z, x.w, q[i][0].y, q[i][1].y, q[i][2].y);
+    split_bf16x3(y.x, y.y, q[i][0].z, q[i][1].z, q[i][2].z);
+    split_bf16x3(y.z, y.w, q[i][0].w, q[i][1].w, q[i][2].w);
   }
   int k_off[2], v_off[4];
   lp_offsets(n, g4, k_off, v_off);
@@ -149,8 +141,8 @@ latent_decode_kernel(float* __restrict__ ws_acc, float* __restrict__ ws_ml, cons
         sum += x[e];
       }
       uint2 hi, mid, lo;
-      ld_split(x[0], x[1], hi.x, mid.x, lo.x);
-      ld_split(x[2], x[3], hi.y, mid.y, lo.y);
+      split_bf16x3(x[0], x[1], hi.x, mid.x, lo.x);
+      split_bf16x3(x[2], x[3], hi.y, mid.y, lo.y);
       *reinterpret_cast<uint2*>(&wts[wave >> 1][0][lane][2 * (wave & 1)]) = hi;
       *reinterpret_cast<uint2*>(&wts[wave >> 1][1][lane][2 * (wave & 1)]) = mid;
       *reinterpret_cast<uint2*>(&wts[wave >> 1][2][lane][2 * (wave & 1)]) = lo;

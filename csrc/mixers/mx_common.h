@@ -83,6 +83,14 @@ __device__ __forceinline__ float tanh_(float x) {
   return copysignf(a < 0.25f ? p : r, x);
 }
 
+// two fp32 values -> their hi, mid and lo bf16 parts (24 bits: the sum is the value)
+__device__ __forceinline__ void split_bf16x3(float a, float b, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
+  hi = ft::pack2(a, b);
+  const float a1 = a - __uint_as_float(hi << 16), b1 = b - __uint_as_float(hi & 0xffff0000u);
+  mid = ft::pack2(a1, b1);
+  lo = ft::pack2(a1 - __uint_as_float(mid << 16), b1 - __uint_as_float(mid & 0xffff0000u));
+}
+
 // a wave's own LDS writes, to be read by its other lanes
 __device__ __forceinline__ void wave_lds_fence() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");

@@ -1,0 +1,277 @@
+// Windowed attention of decode rows and short segments over paged bf16 keys and values (window_attn.hip's masks,
+// score terms and weights) on the matrix units.
+//
+// fp32 queries and weights stay fp32: each is the exact sum of three bf16 parts, keys and values are bf16 already,
+// so three v_mfma_f32_16x16x32_bf16 per operand pair form the products of an fp32 multiply, summed in fp32.
+//
+// A workgroup owns one row and one key head (and score map) with the up to 16 query heads that share it; its eight
+// waves take 32 keys in turn, so a key is read once for all its heads.  S^T = K Q^T and O^T = V^T P^T, a column
+// per head: keys go straight from memory to operands, values through a wave's own LDS strip (ds_read_b64_tr_b16),
+// and weights need no exchange.  The next 32 keys load under the softmax and the sums.  The waves' (maximum, sum,
+// sums) meet in LDS at the end: one launch, whatever the length.
+// Bound by a wave's chain for few rows, by the read of the keys for many.  In running models, 16 heads of 128 on 4
+// key heads: one row, 900 keys in a block of 1024 or with a table 25 us (general kernel, a workgroup per head: 50),
+// 540 keys with sigmoid weights 18 (33), two maps of 64 16 (33); 32 rows of 540 24 (56).
+#include "mx_common.h"
+
+namespace mx {
+
+typedef __bf16 wd_bf16x8 __attribute__((ext_vector_type(8)));
+typedef float wd_f32x4 __attribute__((ext_vector_type(4)));
+typedef short wd_i16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) wd_i16x4 wd_lds_i16x4;
+
+struct WindowArgs {
+  float* out;
+  const float* q;
+  const bf16_t *kc, *vc;
+  const int *start, *pos0, *kv_len, *bt;
+  int bt_stride, num_segs, heads, maps, kv_heads, window;
+  float scale;
+  int sigmoid;
+  const float *r1, *r2, *pb;
+  int block_size, num_blocks, skip_from;
+  float softcap;
+  int has_sink;
+  float sink_all;
+  const float* sinks;
+  int blocks, keep_first;
+  const float* dist_bias;
+  int nd;
+};
+
+__device__ __forceinline__ wd_f32x4 wd_mfma(const uint4& a, const uint4& b, wd_f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(wd_bf16x8, a), __builtin_bit_cast(wd_bf16x8, b), c,
+                                                 0, 0, 0);
+}
+
+constexpr int kWdWaves = 8, kWdKeys = 32, kWdMaxRep = 16;
+
+template <int DK, int DV>
+__global__ void __launch_bounds__(64 * kWdWaves, 2)
+window_decode_kernel(WindowArgs A) {
+  constexpr int KS = DK / 32, DT = DV / 16, PV = DV / 8, VL = kWdKeys * PV / 64;
+  constexpr int kStrip = kWdKeys * DV * 2, kMerge = kWdMaxRep * DV * 4;      // bytes per wave
+  __shared__ __attribute__((aligned(16))) uint8_t lds[kWdWaves * (kStrip > kMerge ? kStrip : kMerge)];
+  __shared__ float ml[kWdWaves][2][kWdMaxRep];
+  const int row = blockIdx.x, gk = blockIdx.y;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 15, g4 = lane >> 4;
+  const int s = segment_of(A.start, A.num_segs, row);
+  const int r0 = A.start[s], rows = A.start[s + 1] - r0;
+  if (row >= A.start[A.num_segs] || (A.skip_from > 0 && rows >= A.skip_from)) return;
+  const int rep = A.heads / A.kv_heads, kvh = gk / A.maps, map = gk % A.maps, hq = A.heads * A.maps;
+  const int a = (kvh * rep + min(n, rep - 1)) * A.maps + map;
+  const long nk = (long)A.kv_heads * A.maps * DK, nv = (long)A.kv_heads * DV;
+  const int i = A.pos0[s] + (row - r0), last = min(i, A.kv_len[s] - 1);
+  const int first = A.window > 0 ? (A.blocks ? i / A.window * A.window : max(0, i - A.window + 1)) : 0;
+  // kept first positions that lie before the window go in front of it
+  const int ext = A.window > 0 ? max(0, min(min(A.keep_first, first), last + 1)) : 0;
+  const int nkeys = ext + max(0, last - first + 1);
+  const int* table = A.bt + (long)s * A.bt_stride;
+
+  auto slot_of = [&](int c) {                  // of the c-th key the row sees (none: -1)
+    if (c >= nkeys) return -1;
+    const int j = c < ext ? c : first + c - ext, blk = table[j / A.block_size];
+    return blk >= 0 && blk < A.num_blocks ? blk * A.block_size + j % A.block_size : -1;
+  };
+  uint4 k[2][KS], v[VL];
+  constexpr int kStep = kWdWaves * kWdKeys;
+  auto look = [&](int c0, int (&slot)[2]) {    // lane n of each group: keys n and 16 + n
+#pragma unroll
+    for (int t = 0; t < 2; ++t) slot[t] = slot_of(c0 + 16 * t + n);
+  };
+  auto fetch = [&](const int (&slot)[2]) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int x = 0; x < KS; ++x) {
+        k[t][x] = uint4{0, 0, 0, 0};
+        if (slot[t] >= 0) k[t][x] = *reinterpret_cast<const uint4*>(A.kc + slot[t] * nk + (long)gk * DK + 32 * x + 8 * g4);
+      }
+#pragma unroll
+    for (int x = 0; x < VL; ++x) {
+      const int key = (64 * x + lane) / PV, s0 = __shfl(slot[0], key & 15), s1 = __shfl(slot[1], key & 15);
+      const int sl = key < 16 ? s0 : s1;
+      v[x] = uint4{0, 0, 0, 0};
+      if (sl >= 0) v[x] = *reinterpret_cast<const uint4*>(A.vc + sl * nv + (long)kvh * DV + (lane % PV) * 8);
+    }
+  };
+  // slots are looked up two steps ahead of their use, so that no load waits for a table entry
+  int slot[2], next[2];
+  look(wave * kWdKeys, slot);
+  look(wave * kWdKeys + kStep, next);
+  fetch(slot);
+
+  // the queries' parts, as right operands: head n, elements 32 x + 8 g4 .. + 7
+  uint4 qp[3][KS];
+  {
+    const float* src = A.q + ((long)row * hq + a) * DK + 8 * g4;
+#pragma unroll
+    for (int x = 0; x < KS; ++x) {
+      const float4 u = *reinterpret_cast<const float4*>(src + 32 * x), w = *reinterpret_cast<const float4*>(src + 32 * x + 4);
+      split_bf16x3(u.x, u.y, qp[0][x].x, qp[1][x].x, qp[2][x].x);
+      split_bf16x3(u.z, u.w, qp[0][x].y, qp[1][x].y, qp[2][x].y);
+      split_bf16x3(w.x, w.y, qp[0][x].z, qp[1][x].z, qp[2][x].z);
+      split_bf16x3(w.z, w.w, qp[0][x].w, qp[1][x].w, qp[2][x].w);
+    }
+  }
+  const float c1 = A.r1 != nullptr ? A.r1[a] : 0.f, c2 = A.r1 != nullptr ? A.r2[a] : 0.f;
+  const float bias = A.sigmoid && A.pb != nullptr ? A.pb[a] : 0.f;
+  const bool sinks = A.has_sink && !A.sigmoid && wave == 0;
+  float mx_ = sinks ? (A.sinks != nullptr ? A.sinks[a] : A.sink_all) : -INFINITY, l_ = sinks && g4 == 0 ? 1.f : 0.f;
+  wd_f32x4 o[DT];                              // columns 16 t + 4 g4 .. of head n
+#pragma unroll
+  for (int t = 0; t < DT; ++t) o[t] = wd_f32x4{0.f, 0.f, 0.f, 0.f};
+  // values in LDS: rows of PV pieces, piece p of key j at p ^ swap(j) (no bank conflicts in the transposed read)
+  uint8_t* strip = lds + wave * kStrip;
+  const auto swap = [](int j) { return DV == 128 ? 2 * (j & 7) : 2 * ((j >> 1) & 3); };
+  const int vkey = 4 * g4 + (n >> 2);
+
+  for (int c0 = wave * kWdKeys; c0 < nkeys; c0 += kStep) {
+    wave_lds_fence();                          // (the last strip has been read)
+#pragma unroll
+    for (int x = 0; x < VL; ++x) {
+      const int key = (64 * x + lane) / PV;
+      *reinterpret_cast<uint4*>(strip + key * DV * 2 + ((lane % PV) ^ swap(key)) * 16) = v[x];
+    }
+    // (loads come back in order: the bias of this step is asked for before the next step's keys)
+    float db[2][4];
+    if (A.dist_bias != nullptr) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int c = c0 + 16 * t + 4 * g4 + e, d = i - (c < ext ? c : first + c - ext);
+          db[t][e] = A.dist_bias[(long)min(max(d, 0), A.nd - 1) * hq + a];
+        }
+    }
+    wd_f32x4 sp[3][2], sc[2];                  // (a chain per part)
+#pragma unroll
+    for (int p = 0; p < 3; ++p)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) sp[p][t] = wd_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int x = 0; x < KS; ++x)
+#pragma unroll
+      for (int p = 2; p >= 0; --p)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) sp[p][t] = wd_mfma(k[t][x], qp[p][x], sp[p][t]);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) sc[t] = sp[2][t] + sp[1][t] + sp[0][t];
+    // which of keys 16 t + 4 g4 + e there are
+    bool has[2][4];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) has[t][e] = __shfl(slot[t], 4 * g4 + e) >= 0;
+    fetch(next);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) slot[t] = next[t];
+    look(c0 + 2 * kStep, next);
+    float top = -INFINITY;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int c = c0 + 16 * t + 4 * g4 + e, d = i - (c < ext ? c : first + c - ext);
+        float z = sc[t][e] * A.scale;
+        if (A.softcap > 0.f) z = A.softcap * tanhf(z / A.softcap);
+        if (A.r1 != nullptr) z -= c1 * logf(1.0f + c2 * (float)max(d, 0));
+        if (A.dist_bias != nullptr) z += db[t][e];
+        if (A.sigmoid) z = sigmoidf_(z + bias);
+        if (!has[t][e]) z = A.sigmoid ? 0.f : -INFINITY;
+        sc[t][e] = z;
+        top = fmaxf(top, z);
+      }
+    if (!A.sigmoid) {
+      const float mn = fmaxf(mx_, ft::kgroups_max(top)), mu = mn == -INFINITY ? 0.f : mn;
+      const float f = mx_ == -INFINITY ? 0.f : expf(mx_ - mu);
+      l_ *= f;
+#pragma unroll
+      for (int t = 0; t < DT; ++t) o[t] *= f;
+      mx_ = mn;
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          sc[t][e] = expf(sc[t][e] - mu);
+          l_ += sc[t][e];
+        }
+    }
+    uint4 pp[3];
+    split_bf16x3(sc[0][0], sc[0][1], pp[0].x, pp[1].x, pp[2].x);
+    split_bf16x3(sc[0][2], sc[0][3], pp[0].y, pp[1].y, pp[2].y);
+    split_bf16x3(sc[1][0], sc[1][1], pp[0].z, pp[1].z, pp[2].z);
+    split_bf16x3(sc[1][2], sc[1][3], pp[0].w, pp[1].w, pp[2].w);
+    wave_lds_fence();
+    uint4 vt[DT];
+#pragma unroll
+    for (int t = 0; t < DT; ++t) {
+      const uint8_t* at = strip + vkey * DV * 2 + ((2 * t + ((n >> 1) & 1)) ^ swap(vkey)) * 16 + (n & 1) * 8;
+      const uint2 lo = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((wd_lds_i16x4*)at));
+      const uint2 hi = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((wd_lds_i16x4*)(at + 16 * DV * 2)));
+      vt[t] = make_uint4(lo.x, lo.y, hi.x, hi.y);
+    }
+#pragma unroll
+    for (int p = 2; p >= 0; --p)
+#pragma unroll
+      for (int t = 0; t < DT; ++t) o[t] = wd_mfma(vt[t], pp[p], o[t]);
+  }
+  // the waves' parts
+  __syncthreads();
+  l_ = ft::kgroups_sum(l_);
+  float* mine = reinterpret_cast<float*>(lds) + (long)wave * rep * DV;
+  if (n < rep) {
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+      *reinterpret_cast<float4*>(mine + n * DV + 16 * t + 4 * g4) = make_float4(o[t][0], o[t][1], o[t][2], o[t][3]);
+    if (g4 == 0) ml[wave][0][n] = mx_, ml[wave][1][n] = l_;
+  }
+  __syncthreads();
+  for (int e = tid; e < rep * DV; e += 64 * kWdWaves) {
+    const int h = e / DV;
+    float top = -INFINITY, l = 0.f, y = 0.f;
+#pragma unroll
+    for (int w = 0; w < kWdWaves; ++w) top = fmaxf(top, ml[w][0][h]);
+#pragma unroll
+    for (int w = 0; w < kWdWaves; ++w) {
+      const float f = A.sigmoid ? 1.f : ml[w][0][h] == -INFINITY ? 0.f : expf(ml[w][0][h] - top);
+      l += f * ml[w][1][h];
+      y += f * reinterpret_cast<const float*>(lds)[(long)w * rep * DV + e];
+    }
+        A.out[((long)row * hq + (kvh * rep + h) * A.maps + map) * DV + e % DV] = A.sigmoid ? y : l > 0.f ? y / l : 0.f;
+  }
+}
+
+}  // namespace mx
+
+using namespace mx;
+
+// whether the sizes and addresses fit the kernel's tiles
+extern "C" int mx_window_decode_fits(const void* out, const void* q, const void* k_cache, const void* v_cache,
+                                     int cache_bf16, int heads, int maps, int kv_heads, int dk, int dv, int block_size,
+                                     int num_blocks) {
+  return cache_bf16 && (dk == 64 || dk == 128) && (dv == 64 || dv == 128) && heads / kv_heads <= kWdMaxRep &&
+         (long)kv_heads * maps <= 65535 && (long)block_size * num_blocks <= 0x7fffffffL &&
+         ((((uintptr_t)out) | ((uintptr_t)q) | ((uintptr_t)k_cache) | ((uintptr_t)v_cache)) % 16) == 0;
+}
+
+// arguments as mx_window_attention (checked there)
+extern "C" int mx_window_decode(float* out, const float* q, const void* k_cache, const void* v_cache, const int* start,
+                                const int* pos0, const int* kv_len, const int* bt, int bt_stride, int num_segs,
+                                long total_rows, int heads, int maps, int kv_heads, int dk, int dv, int window, float scale,
+                                int sigmoid, const float* r1, const float* r2, const float* pb, int block_size,
+                                int num_blocks, int skip_from, float softcap, int has_sink, float sink,
+                                const float* sinks, int blocks, int keep_first, const float* dist_bias, int nd,
+                                hipStream_t s) {
+  const WindowArgs A{out, q, (const bf16_t*)k_cache, (const bf16_t*)v_cache, start, pos0, kv_len, bt, bt_stride, num_segs,
+                     heads, maps, kv_heads, window, scale, sigmoid, r1, r2, pb, block_size, num_blocks, skip_from, softcap,
+                     has_sink, sink, sinks, blocks, keep_first, dist_bias, nd};
+  const dim3 grid((unsigned)total_rows, (unsigned)(kv_heads * maps)), block(64 * kWdWaves);
+  if (dk == 128 && dv == 128) hipLaunchKernelGGL((window_decode_kernel<128, 128>), grid, block, 0, s, A);
+  else if (dk == 64 && dv == 128) hipLaunchKernelGGL((window_decode_kernel<64, 128>), grid, block, 0, s, A);
+  else if (dk == 128) hipLaunchKernelGGL((window_decode_kernel<128, 64>), grid, block, 0, s, A);
+  else hipLaunchKernelGGL((window_decode_kernel<64, 64>), grid, block, 0, s, A);
+  return (int)hipGetLastError();
+}
