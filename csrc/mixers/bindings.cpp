@@ -182,6 +182,11 @@ int mx_moe_pairs(float* out, void* y, const void* h, int bf16, long h_stride, co
 int mx_moe_topk(int* idx, float* wts, const float* z, const float* corr, long rows, int experts, int top,
                 int groups, int keep, hipStream_t s);
 int mx_few_rows_max();
+int mx_state_step_fits(const float* o, const float* state, int dk, int dv);
+int mx_state_step(int kind, float* o, const void* x, int bf16, long x_stride, const void* a, long a_stride, const void* b,
+                  long b_stride, const float* a_log, const float* dt_bias, const float* skip, float inv_tau, float* state,
+                  const int* start, const int* pos0, const int* slot, int num_segs, int heads, int kv_heads, int dk, int dv,
+                  int num_slots, hipStream_t s);
 int mx_latent_decode_fits(int rank, int dr, int cache_bf16);
 int mx_latent_prefill_fits(int rank, int dr, int block_size);
 int mx_latent_prefill(float* out, const float* qa, const float* qr, const void* cache, const int* start, const int* pos0,
@@ -493,6 +498,14 @@ void gated_delta_rule(Tensor o, Tensor qkv, Tensor a, Tensor b, Tensor a_log, Te
               b.scalar_type() == qkv.scalar_type(), "delta rule shapes");
   TORCH_CHECK(state.dim() == 4 && state.size(1) == heads && state.size(2) == dk && state.size(3) == dv, "state");
   check_segs(start, pos0, slot, num_segs);
+  if (max_rows == 1 && mx_state_step_fits(o.data_ptr<float>(), state.data_ptr<float>(), (int)dk, (int)dv)) {
+    chk(mx_state_step(0, o.data_ptr<float>(), qkv.data_ptr(), bf(qkv), qkv.stride(0), a.data_ptr(), a.stride(0),
+                      b.data_ptr(), b.stride(0), a_log.data_ptr<float>(), dt_bias.data_ptr<float>(), nullptr, 0.f,
+                      state.data_ptr<float>(), start.data_ptr<int>(), pos0.data_ptr<int>(), slot.data_ptr<int>(),
+                      (int)num_segs, (int)heads, (int)kv_heads, (int)dk, (int)dv, (int)state.size(0), stream()),
+        "delta rule step");
+    return;
+  }
   auto f32 = qkv.options().dtype(at::kFloat);
   Tensor qn = at::empty({t, kv_heads, dk}, f32), kn = at::empty({t, kv_heads, dk}, f32);
   Tensor g = at::empty({t, heads, dk}, f32), beta = at::empty({t, heads}, f32);
@@ -637,6 +650,13 @@ void gated_linear_attention(Tensor o, Tensor qkv, Tensor a, Tensor a_bias, doubl
   check_segs(start, pos0, slot, num_segs);
   TORCH_CHECK(start.numel() >= num_segs + 1, "segments");
   TORCH_CHECK(max_rows <= t && chunk_from >= 1, "linear attention rows");
+  if (max_rows == 1 && mx_state_step_fits(o.data_ptr<float>(), state.data_ptr<float>(), (int)dk, (int)dv)) {
+    chk(mx_state_step(1, o.data_ptr<float>(), qkv.data_ptr(), bf(qkv), qkv.stride(0), a.data_ptr(), a.stride(0), nullptr,
+                      0, nullptr, a_bias.data_ptr<float>(), nullptr, 1.0f / (float)tau, state.data_ptr<float>(),
+                      start.data_ptr<int>(), pos0.data_ptr<int>(), slot.data_ptr<int>(), (int)num_segs, (int)heads,
+                      (int)heads, (int)dk, (int)dv, (int)state.size(0), stream()), "linear attention step");
+    return;
+  }
   const bool chunks = max_rows >= chunk_from && dk <= mx_chunk_max_dk();
   if (walk || !chunks)
     chk(mx_gla_scan(o.data_ptr<float>(), qkv.data_ptr(), bf(qkv), qkv.stride(0), a.data_ptr(), a.stride(0),
@@ -1238,6 +1258,14 @@ void ssd_scan(Tensor y, Tensor xbc, Tensor dt, Tensor a_log, Tensor dt_bias, Ten
   TORCH_CHECK(state.dim() == 4 && state.size(1) == heads && state.size(2) == n && state.size(3) == dv, "state");
   check_segs(start, pos0, slot, num_segs);
   TORCH_CHECK(max_rows <= t && chunk_from >= 1, "state-space rows");
+  if (max_rows == 1 && mx_state_step_fits(y.data_ptr<float>(), state.data_ptr<float>(), (int)n, (int)dv)) {
+    chk(mx_state_step(2, y.data_ptr<float>(), xbc.data_ptr(), bf(xbc), xbc.stride(0), dt.data_ptr(), dt.stride(0), nullptr,
+                      0, a_log.data_ptr<float>(), dt_bias.data_ptr<float>(), d_skip.data_ptr<float>(), 0.f,
+                      state.data_ptr<float>(), start.data_ptr<int>(), pos0.data_ptr<int>(), slot.data_ptr<int>(),
+                      (int)num_segs, (int)heads, (int)groups, (int)n, (int)dv, (int)state.size(0), stream()),
+        "state-space step");
+    return;
+  }
   const bool chunks = max_rows >= chunk_from && n <= mx_chunk_max_dk();
   if (walk || !chunks)
     chk(mx_ssd_scan(y.data_ptr<float>(), xbc.data_ptr(), bf(xbc), xbc.stride(0), dt.data_ptr(), dt.stride(0),
