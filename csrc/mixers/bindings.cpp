@@ -30,7 +30,7 @@ int mx_conv_attn_prep(float* q_out, const void* qkv, int bf16, long stride, int 
                       const float* table, int table_rows, int rot_dims, int interleaved, long rows, hipStream_t s);
 int mx_moe_top_logits(int* idx, float* wts, const float* z, long rows, int experts, int top, int sigmoid,
                       float scale, int groups, int keep, hipStream_t s);
-int mx_moe_route_top_logits(int* idx, float* wts, const void* h, int bf16, long h_stride, const float* router,
+int mx_moe_route_few(int* idx, float* wts, const void* h, int bf16, long h_stride, const float* router,
                             const float* bias, long rows, int experts, int width, int top, int sigmoid, float scale,
                             int groups, int keep, hipStream_t s);
 int mx_scaled_pair_rows(void* out, int bf16, const float* a, int n, float a_scale, const float* o, const void* gate,
@@ -182,6 +182,9 @@ int mx_moe_pairs(float* out, void* y, const void* h, int bf16, long h_stride, co
 int mx_moe_topk(int* idx, float* wts, const float* z, const float* corr, long rows, int experts, int top,
                 int groups, int keep, hipStream_t s);
 int mx_few_rows_max();
+int mx_moe_route_fits(const void* h, long h_stride, const void* parts, int experts, int width);
+int mx_moe_route(int* idx, float* wts, const void* h, long h_stride, const void* parts, const float* bias, long rows,
+                 int experts, int width, int top, int mode, float scale, int groups, int keep, hipStream_t s);
 int mx_state_step_fits(const float* o, const float* state, int dk, int dv);
 int mx_state_step(int kind, float* o, const void* x, int bf16, long x_stride, const void* a, long a_stride, const void* b,
                   long b_stride, const float* a_log, const float* dt_bias, const float* skip, float inv_tau, float* state,
@@ -888,10 +891,52 @@ void moe_route_top_logits(Tensor idx, Tensor wts, Tensor h, Tensor router, OptT 
     check_f32(*bias, "router bias");
     TORCH_CHECK(bias->numel() == router.size(0), "router bias size");
   }
-  chk(mx_moe_route_top_logits(idx.data_ptr<int>(), wts.data_ptr<float>(), h.data_ptr(), bf(h), h.stride(0),
-                              router.data_ptr<float>(), bias ? bias->data_ptr<float>() : nullptr, h.size(0),
-                              (int)router.size(0), (int)router.size(1), (int)top, sigmoid ? 1 : 0, (float)scale,
-                              (int)groups, (int)keep, stream()), "moe_route_top_logits");
+  chk(mx_moe_route_few(idx.data_ptr<int>(), wts.data_ptr<float>(), h.data_ptr(), bf(h), h.stride(0),
+                       router.data_ptr<float>(), bias ? bias->data_ptr<float>() : nullptr, h.size(0),
+                       (int)router.size(0), (int)router.size(1), (int)top, sigmoid ? 1 : 0, (float)scale,
+                       (int)groups, (int)keep, stream()), "moe_route_top_logits");
+}
+
+void moe_route_softmax(Tensor idx, Tensor wts, Tensor h, Tensor router, Tensor corr, int64_t top, int64_t groups,
+                       int64_t keep) {
+  check_i32(idx, "idx");
+  check_f32(wts, "wts");
+  check_rows(h, "h");
+  check_f32(router, "router");
+  check_f32(corr, "correction");
+  TORCH_CHECK(router.dim() == 2 && router.size(1) == h.size(1) && top >= 1 && top <= router.size(0) &&
+              idx.numel() == h.size(0) * top && wts.numel() == h.size(0) * top && corr.numel() == router.size(0),
+              "moe_route_softmax shapes");
+  check_groups(router.size(0), top, true, groups, keep);
+  chk(mx_moe_route_few(idx.data_ptr<int>(), wts.data_ptr<float>(), h.data_ptr(), bf(h), h.stride(0),
+                       router.data_ptr<float>(), corr.data_ptr<float>(), h.size(0), (int)router.size(0),
+                       (int)router.size(1), (int)top, 2, 1.f, (int)groups, (int)keep, stream()), "moe_route_softmax");
+}
+
+// parts: [width / 32, tiles of 16 experts, 3, 64, 8]
+bool moe_route_fits(Tensor h, Tensor parts, int64_t experts) {
+  return h.is_cuda() && h.scalar_type() == at::kBFloat16 && h.dim() == 2 && h.stride(1) == 1 && parts.is_cuda() &&
+         parts.scalar_type() == at::kBFloat16 && parts.is_contiguous() && parts.dim() == 5 && parts.size(2) == 3 &&
+         parts.size(3) == 64 && parts.size(4) == 8 && parts.size(0) * 32 == h.size(1) &&
+         parts.size(1) == (experts + 15) / 16 &&
+         mx_moe_route_fits(h.data_ptr(), h.stride(0), parts.data_ptr(), (int)experts, (int)h.size(1));
+}
+
+void moe_route(Tensor idx, Tensor wts, Tensor h, Tensor parts, OptT bias, int64_t experts, int64_t top, int64_t mode, double scale,
+               int64_t groups, int64_t keep) {
+  check_i32(idx, "idx");
+  check_f32(wts, "wts");
+  TORCH_CHECK(moe_route_fits(h, parts, experts), "moe_route rows and router");
+  TORCH_CHECK(top >= 1 && top <= experts && idx.numel() == h.size(0) * top && wts.numel() == h.size(0) * top,
+              "moe_route shapes");
+  check_groups(experts, top, mode != 0, groups, keep);
+  if (bias) {
+    check_f32(*bias, "router bias");
+    TORCH_CHECK(bias->numel() == experts, "router bias size");
+  }
+  chk(mx_moe_route(idx.data_ptr<int>(), wts.data_ptr<float>(), h.data_ptr(), h.stride(0), parts.data_ptr(),
+                   bias ? bias->data_ptr<float>() : nullptr, h.size(0), (int)experts, (int)h.size(1), (int)top,
+                   (int)mode, (float)scale, (int)groups, (int)keep, stream()), "moe_route");
 }
 
 // act 0: clamped GLU, 1: relu^2 (the experts' first matrix is [ff, width], up alone, instead of
@@ -1477,6 +1522,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("moe_topk", &moe_topk);
   m.def("moe_pairs", &moe_pairs);
   m.def("few_rows_gemm", &few_rows_gemm);
+  m.def("moe_route_softmax", &moe_route_softmax);
+  m.def("moe_route", &moe_route);
+  m.def("moe_route_fits", &moe_route_fits);
   m.def("experts_many", &experts_many);
   m.def("experts_few", &experts_few);
   m.def("few_rows_max", []() { return (int64_t)mx_few_rows_max(); });

@@ -32,32 +32,26 @@ __device__ __forceinline__ Best wave_best(Best x) {
   return x;
 }
 
-__global__ void __launch_bounds__(64)
-moe_topk_kernel(int* __restrict__ idx, float* __restrict__ wts, const float* __restrict__ z,
-                const float* __restrict__ corr, int experts, int top, int groups, int keep) {
-  extern __shared__ float sm[];
-  float* s = sm;                    // softmax scores
-  float* ch = sm + experts;         // biased scores, -inf once excluded or taken
-  float* gs = sm + 2 * experts;     // group scores
-  const long row = blockIdx.x;
-  const int lane = threadIdx.x;
-  const float* zr = z + row * experts;
+// One wave: s [experts] holds a row's logits; its choice (see above).  ch [experts] and gs [groups] are scratch.
+__device__ __forceinline__ void choose_softmax_all(int* idx, float* wts, float* s, float* ch, float* gs,
+                                                   const float* corr, int experts, int top, int groups, int keep,
+                                                   int lane) {
   float mx_ = -INFINITY;
-  for (int e = lane; e < experts; e += 64) mx_ = fmaxf(mx_, zr[e]);
+  for (int e = lane; e < experts; e += 64) mx_ = fmaxf(mx_, s[e]);
   mx_ = ft::wave_max(mx_);
   float sum = 0.f;
   for (int e = lane; e < experts; e += 64) {
-    const float p = expf(zr[e] - mx_);
+    const float p = expf(s[e] - mx_);
     s[e] = p;
     sum += p;
   }
   sum = ft::wave_sum(sum);
   for (int e = lane; e < experts; e += 64) {
     const float p = s[e] / sum;
-    s[e] = p;
-    ch[e] = p + corr[e];
+    s[e] = p;                       // softmax scores
+    ch[e] = p + corr[e];            // biased scores, -inf once excluded or taken
   }
-  __syncthreads();
+  wave_lds_fence();
   if (groups > 1 && keep < groups) {
     const int gsz = experts / groups;
     for (int g = lane; g < groups; g += 64) {
@@ -65,7 +59,7 @@ moe_topk_kernel(int* __restrict__ idx, float* __restrict__ wts, const float* __r
       for (int e = g * gsz; e < (g + 1) * gsz; ++e) b = fmaxf(b, ch[e]);
       gs[g] = b;
     }
-    __syncthreads();
+    wave_lds_fence();
     // the keep best groups get +inf as a mark; the others' experts are excluded
     for (int k = 0; k < keep; ++k) {
       Best b{-INFINITY, 1 << 30};
@@ -73,11 +67,11 @@ moe_topk_kernel(int* __restrict__ idx, float* __restrict__ wts, const float* __r
         if (gs[g] != INFINITY) b = better(b, Best{gs[g], g});
       b = wave_best(b);
       if (lane == 0 && b.i < groups) gs[b.i] = INFINITY;
-      __syncthreads();
+      wave_lds_fence();
     }
     for (int e = lane; e < experts; e += 64)
       if (gs[e / gsz] != INFINITY) ch[e] = -INFINITY;
-    __syncthreads();
+    wave_lds_fence();
   }
   for (int k = 0; k < top; ++k) {
     Best b{-INFINITY, 1 << 30};
@@ -85,12 +79,24 @@ moe_topk_kernel(int* __restrict__ idx, float* __restrict__ wts, const float* __r
     b = wave_best(b);
     const int e = b.i < experts ? b.i : 0;
     if (lane == 0) {
-      idx[row * top + k] = e;
-      wts[row * top + k] = s[e];
+      idx[k] = e;
+      wts[k] = s[e];
       ch[e] = -INFINITY;
     }
-    __syncthreads();
+    wave_lds_fence();
   }
+}
+
+__global__ void __launch_bounds__(64)
+moe_topk_kernel(int* __restrict__ idx, float* __restrict__ wts, const float* __restrict__ z,
+                const float* __restrict__ corr, int experts, int top, int groups, int keep) {
+  extern __shared__ float sm[];
+  const long row = blockIdx.x;
+  const int lane = threadIdx.x;
+  for (int e = lane; e < experts; e += 64) sm[e] = z[row * experts + e];
+  wave_lds_fence();
+  choose_softmax_all(idx + row * top, wts + row * top, sm, sm + experts, sm + 2 * experts, corr, experts, top, groups,
+                     keep, lane);
 }
 
 // One wave: the logits ch of every expert outside the `keep` best of `groups` equal groups
@@ -173,17 +179,18 @@ __device__ __forceinline__ void load4(const bf16_t* p, float* v) {
   v[3] = __uint_as_float(u.y & 0xffff0000u);
 }
 
-// The same router with its logits computed here, for few rows (decode steps): z = W h + b
+// The routers with their logits computed here, for few rows (decode steps): z = W h + b
 // in fp32 (W, b fp32; h fp32 or bf16), one workgroup of sixteen waves per token, a wave
 // per expert in turn with the lanes along the width (four elements per lane and pass when
 // the rows allow 16-byte loads, several passes in flight); then wave 0 chooses as above.
 constexpr int kRouteWaves = 16;
+enum { kRouteSoftmaxTop = 0, kRouteSigmoid = 1, kRouteSoftmaxAll = 2 };     // bias: the selection bias in the last
 
 template <typename T>
 __global__ void __launch_bounds__(64 * kRouteWaves)
 moe_route_top_logits_kernel(int* __restrict__ idx, float* __restrict__ wts, const T* __restrict__ h, long h_stride,
                             const float* __restrict__ router, const float* __restrict__ bias, int experts,
-                            int width, int top, int vec, int sigmoid, float scale, int groups, int keep) {
+                            int width, int top, int vec, int mode, float scale, int groups, int keep) {
   extern __shared__ float sm[];
   float* ch = sm;
   float* val = sm + experts;
@@ -205,10 +212,14 @@ moe_route_top_logits_kernel(int* __restrict__ idx, float* __restrict__ wts, cons
       for (int i = lane; i < width; i += 64) acc += ld(hr, i) * wr[i];
     }
     acc = ft::wave_sum(acc);
-    if (lane == 0) ch[e] = acc + (bias != nullptr ? bias[e] : 0.f);
+    if (lane == 0) ch[e] = acc + (bias != nullptr && mode != kRouteSoftmaxAll ? bias[e] : 0.f);
   }
   __syncthreads();
   if (wave != 0) return;
+  if (mode == kRouteSoftmaxAll) {
+    choose_softmax_all(idx + row * top, wts + row * top, ch, val, val + experts, bias, experts, top, groups, keep, lane);
+    return;
+  }
   // one wave from here on: lane 0's LDS writes are made visible to the wave's other lanes
   // by a wave-level fence instead of a workgroup barrier
   if (keep < groups) limit_to_best_groups(ch, val + top, experts, groups, keep, lane);
@@ -226,25 +237,179 @@ moe_route_top_logits_kernel(int* __restrict__ idx, float* __restrict__ wts, cons
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   }
-  chosen_weights(wts + row * top, val, top, lane, sigmoid, scale);
+  chosen_weights(wts + row * top, val, top, lane, mode == kRouteSigmoid, scale);
+}
+
+// All routers with their logits computed here, for any number of bf16 rows: one workgroup of sixteen waves per 16
+// rows.  Logits z = W h (+ bias) with the fp32 router given as three bf16 parts (hi + mid + lo: exactly it), three
+// v_mfma_f32_16x16x32_bf16 per operand pair (the fp32 ones take five times as long), a wave a sixteenth of the
+// width, partial sums through LDS; then a wave a row, a lane an expert, every lane its expert's place in the order
+// (ties to the lower index) by comparing with all others, so no choice waits for the one before.
+// The parts lie in operand order, [width / 32][tile of 16 experts][part][lane][8], and the rows pass through LDS,
+// so that neighbouring lanes load neighbouring bytes: with a row or expert per lane the load unit took a line per
+// lane and 8 rows 17 us.
+// Bound by a CU's read of the router (12 KB an expert) behind a chain of load, product and choice: 2000 rows of
+// 2048, 32 experts 13 us; 4096 16 (rows widened, a library product and a choice kernel: 25 and 34 us in three
+// launches).  Up to 64 rows the kernel above, a workgroup per row, is faster: 8 us and 13 for 8 rows.
+constexpr int kTileRows = 16, kRouteStep = 128;      // width of a wave's turn
+
+template <int NE>
+__global__ void __launch_bounds__(64 * kRouteWaves)
+moe_route_tile_kernel(int* __restrict__ idx, float* __restrict__ wts, const bf16_t* __restrict__ h, long h_stride,
+                      const bf16_t* __restrict__ router, const float* __restrict__ bias, long rows, int experts, int width,
+                      int top, int mode, float scale, int groups, int keep) {
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+  __shared__ __attribute__((aligned(16))) uint4 strip[kRouteWaves][kTileRows][kRouteStep / 8];
+  __shared__ float part[kRouteWaves][kTileRows][16 * NE + 1];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = lane & 15, g4 = lane >> 4;
+  const long row0 = (long)blockIdx.x * kTileRows;
+  {
+    f32x4 acc[NE][3];
+#pragma unroll
+    for (int t = 0; t < NE; ++t)
+#pragma unroll
+      for (int p = 0; p < 3; ++p) acc[t][p] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int k0 = wave * kRouteStep; k0 < width; k0 += kRouteWaves * kRouteStep) {
+      uint4 x[4];
+      constexpr int kAhead = NE <= 2 ? 2 : 1;         // steps of 32 whose experts are loaded ahead (registers)
+      bf16x8 w[kAhead][NE][3];
+      auto fetch = [&](int j) {
+#pragma unroll
+        for (int t = 0; t < NE; ++t)
+#pragma unroll
+          for (int p = 0; p < 3; ++p)
+            w[j % kAhead][t][p] = *reinterpret_cast<const bf16x8*>(router + (((long)(k0 / 32 + j) * NE + t) * 3 + p) * 512 + lane * 8);
+      };
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const long r = row0 + 4 * i + g4;
+        x[i] = *reinterpret_cast<const uint4*>(h + (r < rows ? r : rows - 1) * h_stride + k0 + 8 * n);
+      }
+#pragma unroll
+      for (int j = 0; j < kAhead; ++j) fetch(j);
+      wave_lds_fence();
+#pragma unroll
+      for (int i = 0; i < 4; ++i) strip[wave][4 * i + g4][n ^ (4 * i + g4)] = x[i];
+      wave_lds_fence();
+#pragma unroll
+      for (int j = 0; j < kRouteStep / 32; ++j) {
+        const bf16x8 a = __builtin_bit_cast(bf16x8, strip[wave][n][(4 * j + g4) ^ n]);
+#pragma unroll
+        for (int t = 0; t < NE; ++t)
+#pragma unroll
+          for (int p = 0; p < 3; ++p) acc[t][p] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, w[j % kAhead][t][p], acc[t][p], 0, 0, 0);
+        if (j + kAhead < kRouteStep / 32) fetch(j + kAhead);
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < NE; ++t) {
+      const f32x4 z = acc[t][2] + acc[t][1] + acc[t][0];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) part[wave][4 * g4 + v][16 * t + n] = z[v];
+    }
+  }
+  __syncthreads();
+  const long row = row0 + wave;
+  if (row >= rows) return;
+  const bool on = lane < experts;
+  float z = 0.f;
+#pragma unroll
+  for (int w = 0; w < kRouteWaves; ++w) z += part[w][wave][min(lane, 16 * NE - 1)];
+  if (mode != kRouteSoftmaxAll && bias != nullptr && on) z += bias[lane];
+  if (!on) z = -INFINITY;
+  // ch: what the choice goes by; p: the softmax over all
+  float p = 0.f, ch = z;
+  if (mode == kRouteSoftmaxAll) {
+    const float top_z = ft::wave_max(z);
+    p = on ? expf(z - top_z) : 0.f;
+    p = p / ft::wave_sum(p);
+    ch = on ? p + bias[lane] : -INFINITY;
+  }
+  if (!(ch == ch)) ch = -INFINITY;          // (the order must hold every expert once)
+  auto at = [&](float v, int e) { return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), e)); };
+  if (keep < groups) {
+    const int gsz = experts / groups, g = lane / gsz;
+    float score = -INFINITY;
+    for (int o = 0, e = 0; o < groups; ++o) {
+      float a = -INFINITY, b = -INFINITY;    // the two largest of group o
+      for (int j = 0; j < gsz; ++j, ++e) {
+        const float v = at(ch, e);
+        b = v > a ? a : fmaxf(b, v);
+        a = fmaxf(a, v);
+      }
+      if (mode != kRouteSoftmaxAll) a = sigmoidf_(a) + (gsz > 1 ? sigmoidf_(b) : 0.f);
+      score = o == g ? a : score;
+    }
+    int better_groups = 0;
+    for (int o = 0; o < groups; ++o) {
+      const float v = at(score, o * gsz);
+      better_groups += v > score || (v == score && o < g);
+    }
+    if (better_groups >= keep) ch = -INFINITY;
+  }
+  int place = 0;
+  for (int e = 0; e < experts; ++e) {
+    const float v = at(ch, e);
+    place += v > ch || (v == ch && e < lane);
+  }
+  const bool chosen = on && place < top;
+  float w = p;
+  if (mode != kRouteSoftmaxAll) {
+    const float first = ft::wave_max(chosen ? ch : -INFINITY);
+    w = !chosen ? 0.f : mode == kRouteSigmoid ? sigmoidf_(ch) : expf(ch - first);
+    w = w / (ft::wave_sum(w) + (mode == kRouteSigmoid ? 1e-20f : 0.f)) * scale;
+  }
+  if (chosen) {
+    idx[row * top + place] = lane;
+    wts[row * top + place] = w;
+  }
 }
 
 }  // namespace mx
 
-extern "C" int mx_moe_route_top_logits(int* idx, float* wts, const void* h, int bf16, long h_stride,
-                                       const float* router, const float* bias, long rows, int experts, int width,
-                                       int top, int sigmoid, float scale, int groups, int keep, hipStream_t s) {
+// mode 0: moe_top_logits by softmax, 1: by sigmoids, 2: moe_topk (bias: the selection bias)
+extern "C" int mx_moe_route_few(int* idx, float* wts, const void* h, int bf16, long h_stride,
+                                const float* router, const float* bias, long rows, int experts, int width,
+                                int top, int mode, float scale, int groups, int keep, hipStream_t s) {
   if (rows <= 0) return 0;
-  if (experts < 1 || top < 1 || top > experts || width < 1) return -1;
+  if (experts < 1 || top < 1 || top > experts || width < 1 || mode < 0 || mode > 2 || (mode == 2 && bias == nullptr)) return -1;
   if (groups < 1 || experts % groups || keep < 1 || keep > groups || top > experts / groups * keep) return -1;
-  const size_t lds = (size_t)(experts + top + groups) * sizeof(float);
+  const size_t lds = (size_t)(experts + (mode == 2 ? experts : top) + groups) * sizeof(float);
   if (lds > 60 * 1024) return -2;
   const long es = bf16 ? 2 : 4;
   const int vec = width % 4 == 0 && h_stride % 4 == 0 && ((uintptr_t)h) % (4 * es) == 0 &&
                   ((uintptr_t)router) % 16 == 0;
   MX_DISPATCH_T(bf16, hipLaunchKernelGGL((mx::moe_route_top_logits_kernel<T>), dim3((unsigned)rows),
                                          dim3(64 * mx::kRouteWaves), lds, s, idx, wts, (const T*)h, h_stride, router,
-                                         bias, experts, width, top, vec, sigmoid, scale, groups, keep));
+                                         bias, experts, width, top, vec, mode, scale, groups, keep));
+  return (int)hipGetLastError();
+}
+
+extern "C" int mx_moe_route_fits(const void* h, long h_stride, const void* parts, int experts, int width) {
+  return experts >= 1 && experts <= 64 && width >= 1 && width % (mx::kRouteStep * mx::kRouteWaves) == 0 && h_stride % 8 == 0 &&
+         (((uintptr_t)h) | ((uintptr_t)parts)) % 16 == 0;
+}
+
+// parts: the router's three bf16 parts in operand order, whole tiles of experts; modes as mx_moe_route_few
+extern "C" int mx_moe_route(int* idx, float* wts, const void* h, long h_stride, const void* parts, const float* bias,
+                            long rows, int experts, int width, int top, int mode, float scale, int groups, int keep,
+                            hipStream_t s) {
+  if (rows <= 0) return 0;
+  if (!mx_moe_route_fits(h, h_stride, parts, experts, width) || top < 1 || mode < 0 || mode > 2 ||
+      (mode == 2 && bias == nullptr)) return -1;
+  if (groups < 1 || experts % groups || keep < 1 || keep > groups || top > experts / groups * keep) return -1;
+  const long tiles = (rows + mx::kTileRows - 1) / mx::kTileRows;
+  if (tiles > 0x7fffffffL) return -2;
+#define MX_ROUTE(NE)                                                                                         \
+  hipLaunchKernelGGL((mx::moe_route_tile_kernel<NE>), dim3((unsigned)tiles), dim3(64 * mx::kRouteWaves), 0, s, \
+                     idx, wts, (const mx::bf16_t*)h, h_stride, (const mx::bf16_t*)parts, bias, rows, experts, width, top, \
+                     mode, scale, groups, keep)
+  if (experts <= 16) MX_ROUTE(1);
+  else if (experts <= 32) MX_ROUTE(2);
+  else if (experts <= 48) MX_ROUTE(3);
+  else MX_ROUTE(4);
+#undef MX_ROUTE
   return (int)hipGetLastError();
 }
 

@@ -802,6 +802,7 @@ class MoEFF:
         self.dtype, self.routing, self.act, self.route_scale = dtype, routing, act, float(route_scale)
         self.glu = act != "relu_sq"
         self.router = get("router").to(device, torch.float32).contiguous()
+        self.router_parts = M.route_parts(self.router)
         if routing == "grouped_softmax":
             self.correction = get("correction").to(device, torch.float32).contiguous()
             self.router_bias = None
@@ -834,11 +835,19 @@ class MoEFF:
             self.shared_limit = float(shared_limit or 0.0)
 
     def route(self, h):
-        if self.routing == "grouped_softmax":
+        grouped, few = self.routing == "grouped_softmax", h.shape[0] <= self.PAIR_ROWS
+        if not few and M.moe_route_fits(h, self.router_parts, self.e):
+            limited = self.routing != "top_logits"
+            return M.moe_route(h, self.router_parts, self.correction if grouped else self.router_bias, self.e, self.top,
+                               self.routing, 1.0 if grouped else self.route_scale,
+                               self.groups if limited else 1, self.keep if limited else 1)
+        if grouped and few:
+            return M.moe_route_softmax(h, self.router, self.correction, self.top, self.groups, self.keep)
+        if grouped:
             z = F.linear(h.float(), self.router)
             return M.moe_topk(z, self.correction, self.top, self.groups, self.keep)
         sg = self.routing == "top_sigmoid"
-        if h.shape[0] <= self.PAIR_ROWS:
+        if few:
             return M.moe_route_top_logits(h, self.router, self.router_bias, self.top, sg, self.route_scale,
                                           self.groups if sg else 1, self.keep if sg else 1)
         z = F.linear(h.float(), self.router, self.router_bias)

@@ -1062,6 +1062,51 @@ def moe_route_top_logits(h, router, bias, top: int, sigmoid: bool = False, scale
     return ref.moe_top_sigmoid(z, top, scale, groups, keep) if sigmoid else ref.moe_top_logits(z, top)
 
 
+def moe_route_softmax(h, router, correction, top: int, groups: int, keep: int):
+    """:func:`moe_topk` of z = router h (fp32 router [E, width], h fp32 or bf16, fp32 accumulation) in one launch: the
+    router of few rows (decode steps)."""
+    if h.is_cuda:
+        idx = torch.empty(h.shape[0], top, dtype=torch.int32, device=h.device)
+        wts = torch.empty(h.shape[0], top, dtype=torch.float32, device=h.device)
+        native_mixers().moe_route_softmax(idx, wts, h, router, correction, top, groups, keep)
+        return idx, wts
+    return ref.moe_topk(torch.nn.functional.linear(h.float(), router), correction, top, groups, keep)
+
+
+ROUTE_MODES = {"top_logits": 0, "top_sigmoid": 1, "grouped_softmax": 2}
+
+
+def route_parts(router) -> Optional[torch.Tensor]:
+    """fp32 router [E, width] as three bf16 parts whose sum is it (hi, mid and lo: 24 bits), in the operand order of
+    :func:`moe_route`: [width / 32, tiles of 16 experts, 3, 64, 8].  None where the width does not fit."""
+    e, width = router.shape
+    if width % 32:
+        return None
+    tiles = (e + 15) // 16
+    w = torch.nn.functional.pad(router, (0, 0, 0, 16 * tiles - e))
+    hi = w.to(torch.bfloat16)
+    mid = (w - hi.float()).to(torch.bfloat16)
+    parts = torch.stack([hi, mid, (w - hi.float() - mid.float()).to(torch.bfloat16)])
+    # [part, tile, expert n, step, group g, 8] -> a lane (g, n) of a step's tile reads its 8
+    return parts.view(3, tiles, 16, width // 32, 4, 8).permute(3, 1, 0, 4, 2, 5).reshape(width // 32, tiles, 3, 64, 8) \
+        .contiguous()
+
+
+def moe_route_fits(h, parts, experts: int) -> bool:
+    """Whether :func:`moe_route` takes these rows: bf16 on a GPU, at most 64 experts, widths of whole 2048."""
+    return bool(h.is_cuda and parts is not None and native_mixers().moe_route_fits(h, parts, experts))
+
+
+def moe_route(h, parts, bias, experts: int, top: int, routing: str, scale: float = 1.0, groups: int = 1, keep: int = 1):
+    """The routers :func:`moe_topk` (``bias``: its correction), :func:`moe_top_logits` and :func:`moe_top_sigmoid`
+    (``bias``: added to the logits, or None) of z = router h in one launch, fp32 throughout; ``parts``: the fp32
+    router's :func:`route_parts`."""
+    idx = torch.empty(h.shape[0], top, dtype=torch.int32, device=h.device)
+    wts = torch.empty(h.shape[0], top, dtype=torch.float32, device=h.device)
+    native_mixers().moe_route(idx, wts, h, parts, bias, experts, top, ROUTE_MODES[routing], float(scale), groups, keep)
+    return idx, wts
+
+
 # first matrix and activation of an expert: the code the kernels take
 EXPERT_ACTS = {"clamp_glu": 0, "relu_sq": 1, "silu_glu": 2}
 
