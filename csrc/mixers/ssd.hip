@@ -215,6 +215,58 @@ __global__ void gate_group_norm_kernel(TO* __restrict__ out, const float* __rest
   }
 }
 
+// The same for groups of whole fours, at most 256 C entries: a wave's group in registers.  One row of 8 groups of
+// 512 5 us (entry by entry, read twice: 8.6).
+template <typename TZ, typename TO, int C>
+__global__ void __launch_bounds__(256)
+gate_group_norm_fours_kernel(TO* __restrict__ out, const float* __restrict__ y, const TZ* __restrict__ z, long z_stride,
+                             const float* __restrict__ w, long pairs, int groups, int gs, float eps) {
+  const long pair = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (pair >= pairs) return;
+  const int lane = threadIdx.x & 63, g = (int)(pair % groups);
+  const long row = pair / groups, at = row * groups * gs + (long)g * gs;
+  const TZ* zp = z + row * z_stride + (long)g * gs;
+  float v[C][4], wv[C][4], ss = 0.f;
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    const int i = (c * 64 + lane) * 4;
+    const bool in = i < gs;
+    float zv[4] = {0.f, 0.f, 0.f, 0.f};
+    float4 yv = make_float4(0.f, 0.f, 0.f, 0.f), u = yv;
+    if (in) {
+      yv = *reinterpret_cast<const float4*>(y + at + i);
+      u = *reinterpret_cast<const float4*>(w + (long)g * gs + i);
+      if constexpr (sizeof(TZ) == 2) {
+        const uint2 t = *reinterpret_cast<const uint2*>(zp + i);
+        ft::unpack2(t.x, zv[0], zv[1]);
+        ft::unpack2(t.y, zv[2], zv[3]);
+      } else {
+        const float4 t = *reinterpret_cast<const float4*>(zp + i);
+        zv[0] = t.x, zv[1] = t.y, zv[2] = t.z, zv[3] = t.w;
+      }
+    }
+    v[c][0] = yv.x, v[c][1] = yv.y, v[c][2] = yv.z, v[c][3] = yv.w;
+    wv[c][0] = u.x, wv[c][1] = u.y, wv[c][2] = u.z, wv[c][3] = u.w;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      v[c][k] *= zv[k] * sigmoidf_(zv[k]);
+      ss += v[c][k] * v[c][k];
+    }
+  }
+  const float r = 1.0f / sqrtf(ft::wave_sum(ss) / (float)gs + eps);
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    const int i = (c * 64 + lane) * 4;
+    if (i >= gs) continue;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[c][k] *= r * wv[c][k];
+    if constexpr (sizeof(TO) == 2)
+      *reinterpret_cast<uint2*>(out + at + i) = make_uint2(ft::pack2(v[c][0], v[c][1]), ft::pack2(v[c][2], v[c][3]));
+    else
+      *reinterpret_cast<float4*>(out + at + i) = make_float4(v[c][0], v[c][1], v[c][2], v[c][3]);
+  }
+}
+
 }  // namespace mx
 
 using namespace mx;
@@ -255,6 +307,15 @@ extern "C" int mx_gate_group_norm(void* out, int out_bf16, const float* y, const
   const long pairs = rows * groups;
   if (pairs <= 0) return 0;
   const dim3 grid((unsigned)((pairs + 3) / 4)), block(256);
+  if (z_bf16 == out_bf16 && gs % 4 == 0 && gs <= 2048 && z_stride % 4 == 0 && ((uintptr_t)y | (uintptr_t)w) % 16 == 0 &&
+      ((uintptr_t)z | (uintptr_t)out) % (z_bf16 ? 8 : 16) == 0) {
+#define MX_GGN(C)                                                                                                 \
+  MX_DISPATCH_T(z_bf16, hipLaunchKernelGGL((gate_group_norm_fours_kernel<T, T, C>), grid, block, 0, s, (T*)out, y, \
+                                           (const T*)z, z_stride, w, pairs, groups, gs, eps))
+    if (gs <= 256) { MX_GGN(1); } else if (gs <= 512) { MX_GGN(2); } else if (gs <= 1024) { MX_GGN(4); } else { MX_GGN(8); }
+#undef MX_GGN
+    return (int)hipGetLastError();
+  }
   if (z_bf16 && out_bf16)
     hipLaunchKernelGGL((gate_group_norm_kernel<bf16_t, bf16_t>), grid, block, 0, s, (bf16_t*)out, y,
                        (const bf16_t*)z, z_stride, w, pairs, groups, gs, eps);
