@@ -29,7 +29,8 @@ typedef float ba_f32x4 __attribute__((ext_vector_type(4)));
 constexpr int kBandTile = 64;
 
 struct BandArgs {
-  float* out;
+  void* out;                                  // fp32, or bf16 (rounded once, here)
+  int out_bf16;
   const float* q;
   const bf16_t *kc, *vc;
   const int *start, *pos0, *kv_len, *bt;
@@ -278,10 +279,13 @@ band_attn_kernel(BandArgs A) {
     f = l_ > 0.f ? 1.0f / l_ : (l_ == 0.f ? 0.f : l_);     // (NaN stays)
   }
   if (m < pairs) {
-    float* dst = A.out + ((long)(r0 + row) * hq + a) * DV + 4 * g4;
+    const long at = ((long)(r0 + row) * hq + a) * DV + 4 * g4;
 #pragma unroll
-    for (int t = 0; t < DT; ++t)
-      *reinterpret_cast<float4*>(dst + 16 * t) = make_float4(o[t][0] * f, o[t][1] * f, o[t][2] * f, o[t][3] * f);
+    for (int t = 0; t < DT; ++t) {
+      const float4 y = make_float4(o[t][0] * f, o[t][1] * f, o[t][2] * f, o[t][3] * f);
+      if (A.out_bf16) *reinterpret_cast<uint2*>((bf16_t*)A.out + at + 16 * t) = make_uint2(ft::pack2(y.x, y.y), ft::pack2(y.z, y.w));
+      else *reinterpret_cast<float4*>((float*)A.out + at + 16 * t) = y;
+    }
   }
 }
 
@@ -297,7 +301,7 @@ extern "C" int mx_band_attn_fits(int dk, int dv, int block_size) {
 
 // pairs: (row, query head of a group) pairs over all segments of at least min_rows rows; segments of
 // fewer rows are left alone
-extern "C" int mx_band_attn(float* out, const float* q, const void* k_cache, const void* v_cache, const int* start,
+extern "C" int mx_band_attn(void* out, int out_bf16, const float* q, const void* k_cache, const void* v_cache, const int* start,
                             const int* pos0, const int* kv_len, const int* bt, int bt_stride, int num_segs,
                             int long_segs, long long_rows, int heads, int maps, int kv_heads, int dk, int dv, int window,
                             float scale, int sigmoid, const float* r1, const float* r2, const float* pb, int block_size,
@@ -309,7 +313,7 @@ extern "C" int mx_band_attn(float* out, const float* q, const void* k_cache, con
   if (((uintptr_t)q) % 16 || ((uintptr_t)out) % 16 || ((uintptr_t)k_cache) % 16 || ((uintptr_t)v_cache) % 16) return -2;
   const long rep = heads / kv_heads, gk = (long)kv_heads * maps;
   if (long_rows * rep > 0x3fffffffL || (long)nd * heads * maps > 0x7fffffffL) return -3;
-  const BandArgs A{out, q, (const bf16_t*)k_cache, (const bf16_t*)v_cache, start, pos0, kv_len, bt, bt_stride, num_segs,
+  const BandArgs A{out, out_bf16, q, (const bf16_t*)k_cache, (const bf16_t*)v_cache, start, pos0, kv_len, bt, bt_stride, num_segs,
                    heads, maps, kv_heads, window, scale, sigmoid, r1, r2, pb, __builtin_ctz((unsigned)block_size), num_blocks, min_rows, softcap,
                    has_sink, sink, sinks, blocks, keep_first, dist_bias, nd};
   // eight waves share a staged tile once that leaves two workgroups per CU; fewer pairs: four

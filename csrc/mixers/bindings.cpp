@@ -99,7 +99,7 @@ int mx_attn_prep(float* q_out, const void* qkv, int bf16, long stride, int nq, i
                  const int* positions, const int* slots, void* k_cache, void* v_cache, int cache_bf16,
                  long num_slots, long rows, hipStream_t s);
 int mx_window_max_dv();
-int mx_window_attention(float* out, const float* q, const void* k_cache, const void* v_cache, int cache_bf16,
+int mx_window_attention(void* out, int out_bf16, const float* q, const void* k_cache, const void* v_cache, int cache_bf16,
                         const int* start, const int* pos0, const int* kv_len, const int* bt, int bt_stride,
                         int num_segs, long total_rows, int heads, int maps, int kv_heads, int dk, int dv, int window,
                         float scale, int sigmoid, const float* r1, const float* r2, const float* pb, int block_size,
@@ -196,8 +196,10 @@ int mx_latent_prefill(float* out, const float* qa, const float* qr, const void* 
                       const int* kv_len, const int* bt, int bt_stride, int num_segs, int long_segs, long long_rows,
                       int heads, long total_rows, int rank, int dr, int block_size, int num_blocks, float scale,
                       int min_rows, const float* sink, hipStream_t s);
+int mx_window_decode_fits(const void* out, const void* q, const void* k_cache, const void* v_cache, int cache_bf16,
+                          int heads, int maps, int kv_heads, int dk, int dv, int block_size, int num_blocks);
 int mx_band_attn_fits(int dk, int dv, int block_size);
-int mx_band_attn(float* out, const float* q, const void* k_cache, const void* v_cache, const int* start,
+int mx_band_attn(void* out, int out_bf16, const float* q, const void* k_cache, const void* v_cache, const int* start,
                  const int* pos0, const int* kv_len, const int* bt, int bt_stride, int num_segs, int long_segs,
                  long long_rows, int heads, int maps, int kv_heads, int dk, int dv, int window, float scale, int sigmoid,
                  const float* r1, const float* r2, const float* pb, int block_size, int num_blocks, int min_rows,
@@ -1153,12 +1155,20 @@ void conv_attn_prep(Tensor q, Tensor qkv, int64_t nq, int64_t nk, Tensor conv_w,
                         stream()), "conv_attn_prep");
 }
 
+// whether window_attention writes bf16 rows itself for these sizes
+bool window_decode_fits(Tensor q, Tensor k_cache, Tensor v_cache, int64_t heads, int64_t maps, int64_t kv_heads, int64_t dk,
+                        int64_t dv) {
+  return q.is_cuda() && k_cache.dim() >= 2 &&
+         mx_window_decode_fits(nullptr, q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), bf(k_cache), (int)heads,
+                               (int)maps, (int)kv_heads, (int)dk, (int)dv, (int)k_cache.size(1), (int)k_cache.size(0)) != 0;
+}
+
 void window_attention(Tensor out, Tensor q, Tensor k_cache, Tensor v_cache, Tensor start, Tensor pos0, Tensor kv_len,
                       Tensor bt, int64_t num_segs, int64_t max_rows, int64_t heads, int64_t maps, int64_t kv_heads,
                       int64_t dk, int64_t dv, int64_t window, double scale, bool sigmoid, OptT r1, OptT r2, OptT pb,
                       int64_t skip_from, double softcap, c10::optional<double> sink, OptT sinks, bool blocks,
                       int64_t keep_first, OptT dist_bias) {
-  check_f32(out, "out");
+  TORCH_CHECK(out.is_cuda() && is_act(out) && out.is_contiguous(), "out: fp32 / bf16 rows");
   check_f32(q, "q");
   TORCH_CHECK(keep_first >= 0 && (!blocks || window >= 1), "window attention mask");
   if (dist_bias) {
@@ -1178,7 +1188,7 @@ void window_attention(Tensor out, Tensor q, Tensor k_cache, Tensor v_cache, Tens
   check_i32(bt, "block tables");
   TORCH_CHECK(bt.dim() == 2 && bt.size(0) >= num_segs && max_rows <= t, "block tables / max_rows");
   TORCH_CHECK((bool)r1 == (bool)r2, "r1 and r2 go together");
-  chk(mx_window_attention(out.data_ptr<float>(), q.data_ptr<float>(), k_cache.data_ptr(), v_cache.data_ptr(),
+  chk(mx_window_attention(out.data_ptr(), bf(out), q.data_ptr<float>(), k_cache.data_ptr(), v_cache.data_ptr(),
                           bf(k_cache), start.data_ptr<int>(), pos0.data_ptr<int>(), kv_len.data_ptr<int>(),
                           bt.data_ptr<int>(), (int)bt.size(1), (int)num_segs, t, (int)heads, (int)maps, (int)kv_heads,
                           (int)dk, (int)dv, (int)window, (float)scale, sigmoid ? 1 : 0, opt_f32(r1, hq, "r1"),
@@ -1216,7 +1226,7 @@ void band_attention(Tensor out, Tensor q, Tensor k_cache, Tensor v_cache, Tensor
                     int64_t kv_heads, int64_t dk, int64_t dv, int64_t window, double scale, bool sigmoid, OptT r1,
                     OptT r2, OptT pb, int64_t min_rows, double softcap, c10::optional<double> sink, OptT sinks,
                     bool blocks, int64_t keep_first, OptT dist_bias) {
-  check_f32(out, "out");
+  TORCH_CHECK(out.is_cuda() && is_act(out) && out.is_contiguous(), "out: fp32 / bf16 rows");
   check_f32(q, "q");
   TORCH_CHECK(keep_first >= 0 && (!blocks || window >= 1) && min_rows >= 1, "band attention mask");
   if (dist_bias) {
@@ -1236,7 +1246,7 @@ void band_attention(Tensor out, Tensor q, Tensor k_cache, Tensor v_cache, Tensor
   check_i32(bt, "block tables");
   TORCH_CHECK(bt.dim() == 2 && bt.size(0) >= num_segs, "block tables");
   TORCH_CHECK((bool)r1 == (bool)r2, "r1 and r2 go together");
-  chk(mx_band_attn(out.data_ptr<float>(), q.data_ptr<float>(), k_cache.data_ptr(), v_cache.data_ptr(),
+  chk(mx_band_attn(out.data_ptr(), bf(out), q.data_ptr<float>(), k_cache.data_ptr(), v_cache.data_ptr(),
                    start.data_ptr<int>(), pos0.data_ptr<int>(), kv_len.data_ptr<int>(), bt.data_ptr<int>(),
                    (int)bt.size(1), (int)num_segs, (int)long_segs, long_rows, (int)heads, (int)maps, (int)kv_heads,
                    (int)dk, (int)dv, (int)window, (float)scale, sigmoid ? 1 : 0, opt_f32(r1, hq, "r1"),
@@ -1539,6 +1549,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("attn_prep", &attn_prep);
   m.def("window_attention", &window_attention);
   m.def("band_weights", &band_weights);
+  m.def("window_decode_fits", &window_decode_fits);
   m.def("latent_prefill", &latent_prefill);
   m.def("latent_prefill_fits", [](int64_t rank, int64_t dr, int64_t bs) {
     return mx_latent_prefill_fits((int)rank, (int)dr, (int)bs) != 0;

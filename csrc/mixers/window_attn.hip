@@ -714,7 +714,7 @@ extern "C" int mx_window_max_dv() { return 64 * kMaxVCols; }
 extern "C" int mx_window_decode_fits(const void* out, const void* q, const void* k_cache, const void* v_cache,
                                      int cache_bf16, int heads, int maps, int kv_heads, int dk, int dv, int block_size,
                                      int num_blocks);
-extern "C" int mx_window_decode(float* out, const float* q, const void* k_cache, const void* v_cache, const int* start,
+extern "C" int mx_window_decode(void* out, int out_bf16, const float* q, const void* k_cache, const void* v_cache, const int* start,
                                 const int* pos0, const int* kv_len, const int* bt, int bt_stride, int num_segs,
                                 long total_rows, int heads, int maps, int kv_heads, int dk, int dv, int window, float scale,
                                 int sigmoid, const float* r1, const float* r2, const float* pb, int block_size,
@@ -722,7 +722,8 @@ extern "C" int mx_window_decode(float* out, const float* q, const void* k_cache,
                                 const float* sinks, int blocks, int keep_first, const float* dist_bias, int nd,
                                 hipStream_t s);
 
-extern "C" int mx_window_attention(float* out, const float* q, const void* k_cache, const void* v_cache,
+// out_bf16: out is bf16 (only where mx_window_decode_fits)
+extern "C" int mx_window_attention(void* out_, int out_bf16, const float* q, const void* k_cache, const void* v_cache,
                                    int cache_bf16, const int* start, const int* pos0, const int* kv_len,
                                    const int* bt, int bt_stride, int num_segs, long total_rows, int heads, int maps,
                                    int kv_heads, int dk, int dv, int window, float scale, int sigmoid,
@@ -735,10 +736,12 @@ extern "C" int mx_window_attention(float* out, const float* q, const void* k_cac
   if (keep_first < 0 || (dist_bias != nullptr && nd < 1) || (blocks && window < 1)) return -1;
   const int hq = heads * maps;
   if (total_rows > 0x7fffffffL || hq > 65535) return -2;
-  if (mx_window_decode_fits(out, q, k_cache, v_cache, cache_bf16, heads, maps, kv_heads, dk, dv, block_size, num_blocks))
-    return mx_window_decode(out, q, k_cache, v_cache, start, pos0, kv_len, bt, bt_stride, num_segs, total_rows, heads,
+  if (mx_window_decode_fits(out_, q, k_cache, v_cache, cache_bf16, heads, maps, kv_heads, dk, dv, block_size, num_blocks))
+    return mx_window_decode(out_, out_bf16, q, k_cache, v_cache, start, pos0, kv_len, bt, bt_stride, num_segs, total_rows, heads,
                             maps, kv_heads, dk, dv, window, scale, sigmoid, r1, r2, pb, block_size, num_blocks, skip_from,
                             softcap, has_sink, sink, sinks, blocks, keep_first, dist_bias, nd, s);
+  if (out_bf16) return -4;
+  float* out = (float*)out_;
   const long es = cache_bf16 ? 2 : 4;
   const long nk = (long)kv_heads * maps * dk;
   const int vec = (dk * es) % 16 == 0 && (nk * es) % 16 == 0 && ((uintptr_t)k_cache) % 16 == 0;

@@ -22,7 +22,8 @@ typedef short wd_i16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) wd_i16x4 wd_lds_i16x4;
 
 struct WindowArgs {
-  float* out;
+  void* out;                                  // fp32, or bf16 (rounded once, here)
+  int out_bf16;
   const float* q;
   const bf16_t *kc, *vc;
   const int *start, *pos0, *kv_len, *bt;
@@ -240,7 +241,10 @@ window_decode_kernel(WindowArgs A) {
       l += f * ml[w][1][h];
       y += f * reinterpret_cast<const float*>(lds)[(long)w * rep * DV + e];
     }
-        A.out[((long)row * hq + (kvh * rep + h) * A.maps + map) * DV + e % DV] = A.sigmoid ? y : l > 0.f ? y / l : 0.f;
+        y = A.sigmoid ? y : l > 0.f ? y / l : 0.f;
+    const long at = ((long)row * hq + (kvh * rep + h) * A.maps + map) * DV + e % DV;
+    if (A.out_bf16) st((bf16_t*)A.out, at, y);
+    else ((float*)A.out)[at] = y;
   }
 }
 
@@ -258,14 +262,14 @@ extern "C" int mx_window_decode_fits(const void* out, const void* q, const void*
 }
 
 // arguments as mx_window_attention (checked there)
-extern "C" int mx_window_decode(float* out, const float* q, const void* k_cache, const void* v_cache, const int* start,
+extern "C" int mx_window_decode(void* out, int out_bf16, const float* q, const void* k_cache, const void* v_cache, const int* start,
                                 const int* pos0, const int* kv_len, const int* bt, int bt_stride, int num_segs,
                                 long total_rows, int heads, int maps, int kv_heads, int dk, int dv, int window, float scale,
                                 int sigmoid, const float* r1, const float* r2, const float* pb, int block_size,
                                 int num_blocks, int skip_from, float softcap, int has_sink, float sink,
                                 const float* sinks, int blocks, int keep_first, const float* dist_bias, int nd,
                                 hipStream_t s) {
-  const WindowArgs A{out, q, (const bf16_t*)k_cache, (const bf16_t*)v_cache, start, pos0, kv_len, bt, bt_stride, num_segs,
+  const WindowArgs A{out, out_bf16, q, (const bf16_t*)k_cache, (const bf16_t*)v_cache, start, pos0, kv_len, bt, bt_stride, num_segs,
                      heads, maps, kv_heads, window, scale, sigmoid, r1, r2, pb, block_size, num_blocks, skip_from, softcap,
                      has_sink, sink, sinks, blocks, keep_first, dist_bias, nd};
   const dim3 grid((unsigned)total_rows, (unsigned)(kv_heads * maps)), block(64 * kWdWaves);

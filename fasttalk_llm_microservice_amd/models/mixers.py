@@ -192,7 +192,7 @@ class ChannelDelta:
         lo = M.linear(h, self.wlo)
         a = M.linear(lo[:, :self.ra], self.wa2)
         gp = M.linear(lo[:, self.ra:self.ra + self.rg], self.wg2)
-        b = lo[:, self.ra + self.rg:].contiguous()
+        b = lo[:, self.ra + self.rg:]
         qkv = M.short_conv_silu(qkv, self.conv_w, s_conv, ctx.seg)
         o = M.gated_delta_rule(qkv, a, b, self.a_log, self.dt_bias, s_rec, ctx.seg, self.heads,
                                self.kvh, self.dk, self.dv)
@@ -284,18 +284,21 @@ class WindowedAttention:
         return (torch.zeros(num_blocks, block_size, self.nk, dtype=dtype, device=device),
                 torch.zeros(num_blocks, block_size, self.nv, dtype=dtype, device=device))
 
-    def attend(self, q, ctx: StepContext, cache) -> torch.Tensor:
-        """fp32 [T, heads*maps, dv] for fp32 queries [T, heads*maps*dk]."""
+    def attend(self, q, ctx: StepContext, cache, dtype=torch.float32) -> torch.Tensor:
+        """[T, heads*maps, dv] in ``dtype`` for fp32 queries [T, heads*maps*dk]."""
         kc, vc = cache
         seg = ctx.seg
-        if seg.host is not None and seg.max_rows >= self.PRODUCT_ROWS:
+        long = seg.host is not None and seg.max_rows >= self.PRODUCT_ROWS
+        out = None
+        if q.is_cuda or long:
             # (every row belongs to a segment, short or long)
-            out = torch.empty(q.shape[0], self.spec.heads * self.spec.maps, self.spec.dv,
-                              dtype=torch.float32, device=q.device)
+            out = torch.empty(q.shape[0], self.spec.heads * self.spec.maps, self.spec.dv, device=q.device,
+                              dtype=M.window_out_dtype(q, kc, vc, self.spec, dtype, long))
+        if long:
             if min(b - a for a, b in zip(seg.host[0][:-1], seg.host[0][1:])) < self.PRODUCT_ROWS:
                 M.window_attention(q, kc, vc, seg, self.spec, skip_from=self.PRODUCT_ROWS, out=out)
-            return M.window_attention_products(out, q, kc, vc, seg, self.spec, self.PRODUCT_ROWS)
-        return M.window_attention(q, kc, vc, seg, self.spec)
+            return M.window_attention_products(out, q, kc, vc, seg, self.spec, self.PRODUCT_ROWS).to(dtype)
+        return M.window_attention(q, kc, vc, seg, self.spec, out=out).to(dtype)
 
 
 class SigmoidAttention(WindowedAttention):
@@ -321,8 +324,8 @@ class SigmoidAttention(WindowedAttention):
         qkv = M.linear(h, self.wqkv, self.bias)
         q = M.attn_prep(qkv, self.nq, self.nk, self.q_norm, self.k_norm, self.eps, None, 0, self.spec.dk,
                         ctx.positions, ctx.slot_mapping, cache[0], cache[1])
-        o = self.attend(q, ctx, cache)
-        return M.linear(o.view(h.shape[0], -1).to(self.dtype), self.wo)
+        o = self.attend(q, ctx, cache, self.dtype)
+        return M.linear(o.view(h.shape[0], -1), self.wo)
 
 
 class DifferentialAttention(WindowedAttention):
@@ -405,16 +408,16 @@ class ConvSinkAttention(WindowedAttention):
         return super().alloc_cache(num_blocks, block_size, dtype, num_slots, device) + \
             _state_slots(((max(self.taps - 1, 0), self.channels),), num_slots, device)
 
-    def rows(self, qkv, ctx: StepContext, cache) -> torch.Tensor:
-        """fp32 [T, heads*vdim] (before the output projection) of projected rows [q | k | v]."""
+    def rows(self, qkv, ctx: StepContext, cache, dtype=torch.float32) -> torch.Tensor:
+        """[T, heads*vdim] (before the output projection) of projected rows [q | k | v], in ``dtype``."""
         kc, vc, hist = cache
         q = M.conv_attn_prep(qkv, self.nq, self.nk, self.conv_w, hist, ctx.seg, self.q_norm, self.k_norm,
                              self.eps, self.spec.dk, ctx.slot_mapping, kc, vc, self.table, self.rot_dims,
                              self.interleaved)
-        return self.attend(q, ctx, (kc, vc)).view(qkv.shape[0], -1)
+        return self.attend(q, ctx, (kc, vc), dtype).view(qkv.shape[0], -1)
 
     def __call__(self, h, ctx: StepContext, cache) -> torch.Tensor:
-        return M.linear(self.rows(M.linear(h, self.wqkv), ctx, cache).to(self.dtype), self.wo)
+        return M.linear(self.rows(M.linear(h, self.wqkv), ctx, cache, self.dtype), self.wo)
 
 
 class BiasedWindowAttention(WindowedAttention):
@@ -484,8 +487,8 @@ class RotaryBlockAttention(WindowedAttention):
         qkv = M.linear(h, self.wqkv)
         q = M.attn_prep(qkv, self.nq, self.nk, None, None, self.eps, self.table, self.rot_dims, self.spec.dk,
                         ctx.positions, ctx.slot_mapping, cache[0], cache[1])
-        o = self.attend(q, ctx, cache)
-        return M.linear(o.view(h.shape[0], -1).to(self.dtype), self.wo)
+        o = self.attend(q, ctx, cache, self.dtype)
+        return M.linear(o.view(h.shape[0], -1), self.wo)
 
 
 class TalkingHeadsAttention:

@@ -737,9 +737,21 @@ def _plain_tiles(sp: WindowSpec, k_cache) -> bool:
                 and sp.heads <= 64 and sp.heads * sp.dk <= 4096)
 
 
+def window_out_dtype(q, k_cache, v_cache, spec: WindowSpec, dtype, long: bool):
+    """The type :func:`window_attention` (and, ``long``, :func:`window_attention_products`) can leave rows in that are
+    wanted in ``dtype``: itself where the kernels of these sizes round on their way out, else fp32."""
+    sp = spec
+    if dtype != torch.bfloat16 or not q.is_cuda or k_cache.dtype != dtype:
+        return torch.float32
+    n = native_mixers()
+    rows = _plain_tiles(sp, k_cache) or n.window_decode_fits(q, k_cache, v_cache, sp.heads, sp.maps, sp.kv_heads, sp.dk, sp.dv)
+    return dtype if rows and (not long or n.band_attention_fits(sp.dk, sp.dv, k_cache.shape[1])) else torch.float32
+
+
 def window_attention(q, k_cache, v_cache, seg: Segments, spec: WindowSpec, skip_from: int = 0,
                      out: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """q fp32 [T, heads*maps*dk] against the paged caches; fp32 [T, heads*maps, dv].
+    """q fp32 [T, heads*maps*dk] against the paged caches; [T, heads*maps, dv], fp32 or as ``out``
+    (:func:`window_out_dtype`).
     ``skip_from`` > 0: segments of that many rows or more are left to the caller
     (:func:`window_attention_products`)."""
     sp = spec

@@ -119,3 +119,5 @@ def test_against_64_bits(name, sizes, opt, lens, pos0, bs, monkeypatch):
     assert e_new < 1e-6 and e_new < 1.5 * e_old + 1e-7, (e_new, e_old)
     again = M.window_attention_products(torch.zeros_like(out), q, kc, vc, seg, sp, 32)
     assert torch.equal(again[rows], got[rows])
+    half = M.window_attention_products(torch.zeros_like(out, dtype=torch.bfloat16), q, kc, vc, seg, sp, 32)
+    assert torch.equal(half[rows], got[rows].bfloat16())       # rounded once, on the way out

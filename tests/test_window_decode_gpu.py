@@ -46,7 +46,7 @@ def test_against_64_bits(name, sizes, opt, lens, pos0, bs):
     q = (2.0 * rnd(sum(lens), hq * sp.dk)).to(DEV)
     want = reference(q, kc, vc, seg, sp, 1)
     out = torch.full((q.shape[0], hq, sp.dv), 7.0, device=DEV)
-    got = M.window_attention(q, kc, vc, seg, sp, skip_from=32, out=out)
+    got = M.window_attention(q, kc, vc, seg, sp, skip_from=32, out=out.clone())
     rows = torch.cat([torch.full((n,), n < 32) for n in lens]).to(DEV)
     assert bool((got[~rows] == 7.0).all())                     # long segments are not this call's
     old = M.window_attention(q, kc.float(), vc.float(), seg, sp)      # the general kernel, on widened caches
@@ -54,3 +54,9 @@ def test_against_64_bits(name, sizes, opt, lens, pos0, bs):
     e_new, e_old = (float((x.double() - want)[rows].norm()) / norm for x in (got, old))
     # fp32 sums of a few hundred terms: about 2^-22; no further from 64 bits than the general kernel
     assert e_new < 1e-6 and e_new < 1.5 * e_old + 1e-7, (e_new, e_old)
+    # rows in bf16 are the fp32 ones, rounded once
+    if M.window_out_dtype(q, kc, vc, sp, torch.bfloat16, False) == torch.bfloat16:
+        got16 = M.window_attention(q, kc, vc, seg, sp, skip_from=32, out=out.bfloat16())
+        assert torch.equal(got16[rows], got[rows].bfloat16())
+    else:
+        assert sp.heads // sp.kv_heads > 16 and not M._plain_tiles(sp, kc)
