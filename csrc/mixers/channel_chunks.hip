@@ -9,7 +9,7 @@
 //   * block below the diagonal (I, J): prod = c_t . B_{J+1} .. B_{I-1} . u_j with c_t the product of the
 //     decays of block I up to t, u_j that of block J after j, B a block's whole product.  All three are at
 //     most one: the rows k_t c_t (times B's) against k_j u_j, on the matrix units.
-//   * diagonal block: the product walked row by row in registers, a lane per (j, quarter of the channels).
+//   * diagonal block: the product walked row by row in registers, a lane per (two j, sixteenth of the channels).
 // Nothing is divided and no logarithms are taken; what underflows is zero.
 //
 // Kernels:
@@ -18,9 +18,11 @@
 //                 inverse and U, -W
 //   chunk_carry   chunk_common.h, decays by row of the state
 //   channel_out   per (chunk, head, 64 columns), parallel: o = (q e^G) S + P w
-// channel_prep is bound by the vector units (the diagonal blocks) and one workgroup a CU (139 KB of LDS);
-// the carry by its chain.  4096 rows, 16 heads of 128 x 128, delta rule: 173 + 156 + 46 us, the walk 2080;
-// 777 rows, linear attention: 30 + 19 + 16 us, the walk 245.
+// channel_prep is bound by its phases' latencies (loads, LDS, the inverse's substitution), which follow one
+// another in the one workgroup a CU that 139 KB of LDS leave room for: hence eight waves and all of a row's
+// loads in flight (four waves, loads of one entry, a key per lane on the diagonal: 174 us where this takes
+// 101, and 30 where it takes 17); the carry by its chain.  4096 rows, 16 heads of 128 x 128, delta rule:
+// 101 + 159 + 46 us, the walk 2080; 777 rows, linear attention: 17 + 19 + 16 us, the walk 245.
 #include "chunk_common.h"
 
 namespace mx {
@@ -43,13 +45,33 @@ constexpr int kPrepFloats = 3 * kC * (16 * DKT + 4) + 2 * kC * kPLD + 4 * 16 * D
 // fragments of P: piece (row block m, key block b), lane: rows 16 m + lo, keys 16 b + 4 e + hi, e = 0 .. 3;
 // of q e^G: piece (m, 16 channels i), lane: rows 16 m + lo, channels 16 i + 4 e + hi
 
+// Eight waves, two a SIMD (the LDS leaves room for one workgroup a CU): row blocks are dealt out so that
+// both waves of a SIMD together have the same work whichever SIMD it is.  vec: 16-byte loads of q, k, g.
+constexpr int kPrepThreads = 512;
+
+// the value of the lane `ctrl` names (a permutation within 16 lanes)
+template <int ctrl>
+__device__ __forceinline__ float dpp(float x) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), ctrl, 0xf, 0xf, true));
+}
+constexpr int kSwap1 = 0xB1, kSwap2 = 0x4E, kRor4 = 0x124, kRor8 = 0x128;
+
+// sums over 16 lanes: a, b, c, d land in lanes 0, 1, 2, 3 (mod 4) of the sixteen
+__device__ __forceinline__ float sum16(float a, float b, float c, float d, int lane) {
+  const bool odd = lane & 1, two = lane & 2;
+  const float ab = (odd ? b : a) + dpp<kSwap1>(odd ? a : b), cd = (odd ? d : c) + dpp<kSwap1>(odd ? c : d);
+  float x = (two ? cd : ab) + dpp<kSwap2>(two ? ab : cd);
+  x += dpp<kRor4>(x);
+  return x + dpp<kRor8>(x);
+}
+
 template <int DKT, bool DELTA, typename TQ, typename TV>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(kPrepThreads)
 channel_prep_kernel(float* __restrict__ ws_p, float* __restrict__ ws_q, float* __restrict__ ws_k,
                     float* __restrict__ ws_g, float* __restrict__ ws_w, float* __restrict__ ws_u, ChannelIn in,
                     const int* __restrict__ start, const int* __restrict__ pos0, const int* __restrict__ slot, int heads,
-                    int dk, int dv, int num_slots, int min_rows) {
-  constexpr int DKP = 16 * DKT, LDK = DKP + 4, CH = DKP / 4;
+                    int dk, int dv, int num_slots, int min_rows, int vec) {
+  constexpr int DKP = 16 * DKT, LDK = DKP + 4;
   extern __shared__ __attribute__((aligned(16))) float lds[];
   float *kb = lds, *qb = kb + kC * LDK, *gb = qb + kC * LDK;       // rows of k, q, decays; later k u, q c, k c
   float *ab = gb + kC * LDK, *pb = ab + kC * kPLD;                 // pair weights of k (times beta) and of q
@@ -58,74 +80,103 @@ channel_prep_kernel(float* __restrict__ ws_p, float* __restrict__ ws_q, float* _
   if (!find_chunk(c, blockIdx.x, blockIdx.z, start, pos0, slot, min_rows, num_slots)) return;
   const int h = blockIdx.y;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int lo = lane & 15, hi = lane >> 4;
+  const int lo = lane & 15, hi = lane >> 4, half = wave >> 2;
   {
     const long kh = (long)(h / in.rep) * dk;
     const TQ *qp = (const TQ*)in.q + c.row0 * in.q_stride + kh, *kp = (const TQ*)in.k + c.row0 * in.k_stride + kh;
     const TQ* gp = (const TQ*)in.g + c.row0 * in.g_stride + (long)h * dk;
-#pragma unroll 4
-    for (int e = tid; e < kC * DKP; e += 256) {
-      const int t = e / DKP, i = e % DKP;
-      float k = 0.f, q = 0.f, g = 1.f;
-      if (t < c.cnt && i < dk) {
-        k = ld(kp, t * in.k_stride + i);
-        q = ld(qp, t * in.q_stride + i) * in.q_scale;
-        g = ld(gp, t * in.g_stride + i);
-        if constexpr (!DELTA) g = gla_decay(g + in.a_bias[(long)h * dk + i], in.inv_tau);
+    if (vec) {                                                     // dk a multiple of 4; addresses stay inside the rows
+      constexpr int QUADS = kC * DKP / 4, N = (QUADS + kPrepThreads - 1) / kPrepThreads;
+      float k[N][4], q[N][4], g[N][4];
+#pragma unroll
+      for (int n = 0; n < N; ++n) {
+        const int e = tid + n * kPrepThreads;
+        const int t = min(e / (DKP / 4), c.cnt - 1), i = min(e % (DKP / 4) * 4, dk - 4);
+        load4(kp + t * in.k_stride + i, k[n]);
+        load4(qp + t * in.q_stride + i, q[n]);
+        load4(gp + t * in.g_stride + i, g[n]);
       }
-      kb[t * LDK + i] = k;
-      qb[t * LDK + i] = q;
-      gb[t * LDK + i] = g;
+#pragma unroll
+      for (int n = 0; n < N; ++n) {
+        const int e = tid + n * kPrepThreads, t = e / (DKP / 4), i = e % (DKP / 4) * 4;
+        if (QUADS % kPrepThreads != 0 && e >= QUADS) continue;
+        const bool live = t < c.cnt && i < dk;
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+          if constexpr (!DELTA) g[n][x] = gla_decay(g[n][x] + in.a_bias[(long)h * dk + min(i, dk - 4) + x], in.inv_tau);
+          k[n][x] = live ? k[n][x] : 0.f;
+          q[n][x] = live ? q[n][x] * in.q_scale : 0.f;
+          g[n][x] = live ? g[n][x] : 1.f;
+        }
+        *reinterpret_cast<float4*>(kb + t * LDK + i) = make_float4(k[n][0], k[n][1], k[n][2], k[n][3]);
+        *reinterpret_cast<float4*>(qb + t * LDK + i) = make_float4(q[n][0], q[n][1], q[n][2], q[n][3]);
+        *reinterpret_cast<float4*>(gb + t * LDK + i) = make_float4(g[n][0], g[n][1], g[n][2], g[n][3]);
+      }
+    } else {
+#pragma unroll 4
+      for (int e = tid; e < kC * DKP; e += kPrepThreads) {
+        const int t = e / DKP, i = e % DKP;
+        float k = 0.f, q = 0.f, g = 1.f;
+        if (t < c.cnt && i < dk) {
+          k = ld(kp, t * in.k_stride + i);
+          q = ld(qp, t * in.q_stride + i) * in.q_scale;
+          g = ld(gp, t * in.g_stride + i);
+          if constexpr (!DELTA) g = gla_decay(g + in.a_bias[(long)h * dk + i], in.inv_tau);
+        }
+        kb[t * LDK + i] = k;
+        qb[t * LDK + i] = q;
+        gb[t * LDK + i] = g;
+      }
     }
     if (DELTA && tid < kC) bs[tid] = tid < c.cnt ? in.beta[(c.row0 + tid) * heads + h] : 0.f;
   }
   __syncthreads();
-  // diagonal blocks: lane (j = lo, channels 16 i + 4 hi + e) walks the rows after j
+  // diagonal blocks: wave (block, half) has the keys 8 half .. 8 half + 7 of a block and walks the rows from
+  // there; a lane two keys and DKT channels, so that a row read from LDS serves two keys and sixteen lanes add up
   {
-    const int r0 = 16 * wave;
-    float m[CH];
+    constexpr int VW = DKT < 4 ? DKT : 4, NV = DKT / VW;
+    typedef float vec_t __attribute__((ext_vector_type(VW)));
+    const int r0 = 16 * (wave & 3), j0 = 8 * half + 2 * hi;        // lane's channels: VW lo + 16 VW i + e
+    float m[2][DKT];
 #pragma unroll
-    for (int i = 0; i < CH / 4; ++i) {
-      const float4 u = *reinterpret_cast<const float4*>(kb + (r0 + lo) * LDK + 16 * i + 4 * hi);
-      m[4 * i] = u.x; m[4 * i + 1] = u.y; m[4 * i + 2] = u.z; m[4 * i + 3] = u.w;
-    }
-    for (int t = 0; t < 16; ++t) {
-      float sk = 0.f, sq = 0.f;
-      if (t >= lo) {
-        const float *kr = kb + (r0 + t) * LDK + 4 * hi, *qr = qb + (r0 + t) * LDK + 4 * hi, *gr = gb + (r0 + t) * LDK + 4 * hi;
-        float s0[4] = {0.f, 0.f, 0.f, 0.f}, s1[4] = {0.f, 0.f, 0.f, 0.f};
-        const bool first = t == lo;
+    for (int y = 0; y < 2; ++y)
 #pragma unroll
-        for (int i = 0; i < CH / 4; ++i) {
-          const float4 q4 = *reinterpret_cast<const float4*>(qr + 16 * i), g4 = *reinterpret_cast<const float4*>(gr + 16 * i);
-          const float qv[4] = {q4.x, q4.y, q4.z, q4.w}, gv[4] = {g4.x, g4.y, g4.z, g4.w};
-          float kv[4];
-          if constexpr (DELTA) {
-            const float4 k4 = *reinterpret_cast<const float4*>(kr + 16 * i);
-            kv[0] = k4.x; kv[1] = k4.y; kv[2] = k4.z; kv[3] = k4.w;
-          }
+      for (int i = 0; i < NV; ++i) {
+        const vec_t u = *reinterpret_cast<const vec_t*>(kb + (r0 + j0 + y) * LDK + 16 * VW * i + VW * lo);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            float& x = m[4 * i + e];
-            x *= first ? 1.f : gv[e];
-            s1[e] += qv[e] * x;
-            if constexpr (DELTA) s0[e] += kv[e] * x;
-          }
-        }
-        sq = (s1[0] + s1[1]) + (s1[2] + s1[3]);
-        sk = (s0[0] + s0[1]) + (s0[2] + s0[3]);
+        for (int e = 0; e < VW; ++e) m[y][VW * i + e] = u[e];
       }
-      sq = add_halves(add_row_pair(sq));
-      if constexpr (DELTA) sk = add_halves(add_row_pair(sk));
-      if (hi == 0) {
-        pb[(r0 + t) * kPLD + r0 + lo] = sq;                       // (0 where j > t)
-        if constexpr (DELTA) ab[(r0 + t) * kPLD + r0 + lo] = t > lo ? bs[r0 + t] * sk : 0.f;
+    if (half == 1) pb[(r0 + (lane >> 3)) * kPLD + r0 + 8 + (lane & 7)] = 0.f;     // keys behind the rows
+#pragma unroll 2
+    for (int t = 8 * half; t < 16; ++t) {
+      const float *kr = kb + (r0 + t) * LDK + VW * lo, *qr = qb + (r0 + t) * LDK + VW * lo, *gr = gb + (r0 + t) * LDK + VW * lo;
+      float sq[2][2] = {{0.f, 0.f}, {0.f, 0.f}}, sk[2][2] = {{0.f, 0.f}, {0.f, 0.f}};
+#pragma unroll
+      for (int i = 0; i < NV; ++i) {
+        const vec_t qv = *reinterpret_cast<const vec_t*>(qr + 16 * VW * i), gv = *reinterpret_cast<const vec_t*>(gr + 16 * VW * i);
+        vec_t kv = qv;
+        if constexpr (DELTA) kv = *reinterpret_cast<const vec_t*>(kr + 16 * VW * i);
+#pragma unroll
+        for (int y = 0; y < 2; ++y)
+#pragma unroll
+          for (int e = 0; e < VW; ++e) {
+            float& x = m[y][VW * i + e];
+            x *= t > j0 + y ? gv[e] : 1.f;
+            sq[y][e & 1] += qv[e] * x;
+            if constexpr (DELTA) sk[y][e & 1] += kv[e] * x;
+          }
+      }
+      const float s = sum16(sq[0][0] + sq[0][1], sk[0][0] + sk[0][1], sq[1][0] + sq[1][1], sk[1][0] + sk[1][1], lane);
+      const int j = j0 + (lo >> 1);
+      if (lo < 4) {
+        if ((lo & 1) == 0) pb[(r0 + t) * kPLD + r0 + j] = t >= j ? s : 0.f;
+        else if constexpr (DELTA) ab[(r0 + t) * kPLD + r0 + j] = t > j ? bs[r0 + t] * s : 0.f;
       }
     }
   }
   __syncthreads();
   // per channel: products within the blocks
-  for (int e = tid; e < 4 * DKP; e += 256) {
+  for (int e = tid; e < 4 * DKP; e += kPrepThreads) {
     const int d = e % DKP, r0 = 16 * (e / DKP);
     float g[16];
 #pragma unroll
@@ -148,53 +199,48 @@ channel_prep_kernel(float* __restrict__ ws_p, float* __restrict__ ws_q, float* _
   }
   __syncthreads();
   const long cs = c.ws * heads + h;
-  {
-    float kf[4 * DKT], qf[4 * DKT];
+  // below the diagonal blocks: the first four waves the rows of q, the others (delta rule) those of k, blocks
+  // in opposite order
+  if (half == 0 || DELTA) {
+    const int blk = half == 0 ? wave : 7 - wave;
+    const float* rows = half == 0 ? qb : gb;
+    float* dst = half == 0 ? pb : ab;
+    float f[4 * DKT];
 #pragma unroll
-    for (int s = 0; s < 4 * DKT; ++s) {
-      qf[s] = qb[(16 * wave + lo) * LDK + 4 * s + hi];
-      if constexpr (DELTA) kf[s] = gb[(16 * wave + lo) * LDK + 4 * s + hi];
-    }
-    for (int jt = wave - 1; jt >= 0; --jt) {
+    for (int s = 0; s < 4 * DKT; ++s) f[s] = rows[(16 * blk + lo) * LDK + 4 * s + hi];
+    for (int jt = blk - 1; jt >= 0; --jt) {
       const float* kr = kb + (16 * jt + lo) * LDK + hi;
-      const f32x4 p = dot_steps<4 * DKT>([&](int s) { return qf[s]; }, [&](int s) { return kr[4 * s]; });
+      const f32x4 p = dot_steps<4 * DKT>([&](int s) { return f[s]; }, [&](int s) { return kr[4 * s]; });
 #pragma unroll
-      for (int r = 0; r < 4; ++r) pb[(16 * wave + 4 * hi + r) * kPLD + 16 * jt + lo] = p[r];
-      if constexpr (DELTA) {
-        const f32x4 a = dot_steps<4 * DKT>([&](int s) { return kf[s]; }, [&](int s) { return kr[4 * s]; });
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int i = 16 * wave + 4 * hi + r;
-          ab[i * kPLD + 16 * jt + lo] = bs[i] * a[r];
-        }
+      for (int r = 0; r < 4; ++r) {
+        const int i = 16 * blk + 4 * hi + r;
+        dst[i * kPLD + 16 * jt + lo] = half == 0 ? p[r] : bs[i] * p[r];
       }
 #pragma unroll
-      for (int s = 0; s < 4 * DKT; ++s) {
-        const float b = bt[jt * DKP + 4 * s + hi];
-        qf[s] *= b;
-        if constexpr (DELTA) kf[s] *= b;
-      }
+      for (int s = 0; s < 4 * DKT; ++s) f[s] *= bt[jt * DKP + 4 * s + hi];
     }
-    f32x4* wq = (f32x4*)ws_q + cs * (4 * DKT * 64) + wave * DKT * 64 + lane;
+    if (half == 0) {
+      f32x4* wq = (f32x4*)ws_q + cs * (4 * DKT * 64) + blk * DKT * 64 + lane;
 #pragma unroll
-    for (int i = 0; i < DKT; ++i) wq[i * 64] = f32x4{qf[4 * i], qf[4 * i + 1], qf[4 * i + 2], qf[4 * i + 3]};
-    if constexpr (DELTA) {
+      for (int i = 0; i < DKT; ++i) wq[i * 64] = f32x4{f[4 * i], f[4 * i + 1], f[4 * i + 2], f[4 * i + 3]};
+      wave_lds_fence();
+      f32x4* wp = (f32x4*)ws_p + cs * (4 * 4 * 64) + blk * 4 * 64 + lane;
+      for (int b = 0; b <= blk; ++b) {
+        f32x4 x;
 #pragma unroll
-      for (int s = 0; s < 4 * DKT; ++s) gb[(16 * wave + lo) * LDK + 4 * s + hi] = kf[s];   // k e^G
+        for (int e = 0; e < 4; ++e) x[e] = pb[(16 * blk + lo) * kPLD + 16 * b + 4 * e + hi];
+        wp[b * 64] = x;
+      }
+    } else {
+#pragma unroll
+      for (int s = 0; s < 4 * DKT; ++s) gb[(16 * blk + lo) * LDK + 4 * s + hi] = f[s];     // k e^G
     }
   }
-  wave_lds_fence();
-  {
-    f32x4* wp = (f32x4*)ws_p + cs * (4 * 4 * 64) + wave * 4 * 64 + lane;
-    for (int b = 0; b <= wave; ++b) {
-      f32x4 x;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) x[e] = pb[(16 * wave + lo) * kPLD + 16 * b + 4 * e + hi];
-      wp[b * 64] = x;
-    }
-    // k e^{G_63 - G}: tile (i, m) columns 16 i + lo, rows 16 m + 4 hi + r
+  // k e^{G_63 - G}: tile (i, m) columns 16 i + lo, rows 16 m + 4 hi + r (delta rule: by the waves that have no
+  // part in the inverse)
+  if (half == 1 || !DELTA) {
     f32x4* wk = (f32x4*)ws_k + cs * (4 * DKT * 64) + lane;
-    for (int e = wave; e < 4 * DKT; e += 4) {
+    for (int e = DELTA ? wave - 4 : wave; e < 4 * DKT; e += DELTA ? 4 : 8) {
       const int i = e / 4, m = e % 4;
       float f = 1.f;
       for (int b = m + 1; b < 4; ++b) f *= bt[b * DKP + 16 * i + lo];
@@ -203,10 +249,19 @@ channel_prep_kernel(float* __restrict__ ws_p, float* __restrict__ ws_q, float* _
       for (int r = 0; r < 4; ++r) x[r] = kb[(16 * m + 4 * hi + r) * LDK + 16 * i + lo] * f;
       wk[e * 64] = x;
     }
-    if (tid < DKP) ws_g[cs * DKP + tid] = (bt[tid] * bt[DKP + tid]) * (bt[2 * DKP + tid] * bt[3 * DKP + tid]);
+    const int d = tid - 256;
+    if (d >= 0 && d < DKP) ws_g[cs * DKP + d] = (bt[d] * bt[DKP + d]) * (bt[2 * DKP + d] * bt[3 * DKP + d]);
   }
   if constexpr (DELTA) {
-    invert_unit_lower(ab, wave, lo, hi);
+    const int vtiles = (dv + 15) / 16;
+    float vr[16];
+    auto fetch_v = [&](int ct) {                                   // rows past cnt: beta is 0; columns past dv are not used
+      const TV* vp = (const TV*)in.v + c.row0 * in.v_stride + (long)h * dv + min(16 * ct + lo, dv - 1);
+#pragma unroll
+      for (int s = 0; s < 16; ++s) vr[s] = ld(vp, min(4 * s + hi, c.cnt - 1) * in.v_stride);
+    };
+    fetch_v(wave);                                                 // on their way during the inverse
+    invert_unit_lower<8>(ab, wave, lo, hi);
     // [W | U] = T [beta e^G k | beta v], column tiles dealt out to the waves (the inverse's barriers have
     // made every wave's rows of k e^G visible)
     float tf[4][16], fu[16];
@@ -214,7 +269,7 @@ channel_prep_kernel(float* __restrict__ ws_p, float* __restrict__ ws_q, float* _
 #pragma unroll
     for (int s = 0; s < 16; ++s) fu[s] = bs[4 * s + hi];
     f32x4* ww = (f32x4*)ws_w + cs * (4 * DKT * 64);
-    for (int ct = wave; ct < DKT; ct += 4) {
+    for (int ct = wave; ct < DKT; ct += 8) {
       float b[16];
       f32x4 x[4];
 #pragma unroll
@@ -223,14 +278,13 @@ channel_prep_kernel(float* __restrict__ ws_p, float* __restrict__ ws_q, float* _
 #pragma unroll
       for (int m = 0; m < 4; ++m) ww[(m * DKT + ct) * 64 + lane] = x[m];
     }
-    const int vtiles = (dv + 15) / 16;
     f32x4* wu = (f32x4*)ws_u + cs * (long)vtiles * 256;
-    for (int ct = wave; ct < vtiles; ct += 4) {
+    for (int ct = wave; ct < vtiles; ct += 8) {
       float b[16];
       f32x4 x[4];
-      const TV* vp = (const TV*)in.v + c.row0 * in.v_stride + (long)h * dv + min(16 * ct + lo, dv - 1);
 #pragma unroll
-      for (int s = 0; s < 16; ++s) b[s] = fu[s] * ld(vp, min(4 * s + hi, c.cnt - 1) * in.v_stride);   // beta is 0 past cnt
+      for (int s = 0; s < 16; ++s) b[s] = fu[s] * vr[s];
+      if (ct + 8 < vtiles) fetch_v(ct + 8);
       inverse_column<false>(tf, b, x);
 #pragma unroll
       for (int m = 0; m < 4; ++m) wu[(ct * 4 + m) * 64 + lane] = x[m];
@@ -332,6 +386,9 @@ int channel_run(float* o, const ChannelIn& in, const ChannelWs& ws, float* state
   const int chunks = (max_rows + kC - 1) / kC;
   const long outs = (long)heads * ((dv + 63) / 64);
   if (heads > 65535 || outs > 65535 || num_segs > 65535) return -2;
+  // whole quads of q, k and g at aligned addresses
+  const int quads = dk % 4 == 0 && in.q_stride % 4 == 0 && in.k_stride % 4 == 0 && in.g_stride % 4 == 0 &&
+                    ((uintptr_t)in.q | (uintptr_t)in.k | (uintptr_t)in.g) % (4 * sizeof(TQ)) == 0;
   int rc = 0;
   key_tiles(dk, [&](auto t) {
     constexpr int DKT = decltype(t)::value, lds = kPrepFloats<DKT> * 4;
@@ -340,8 +397,8 @@ int channel_run(float* o, const ChannelIn& in, const ChannelWs& ws, float* state
       rc = (int)hipFuncSetAttribute(reinterpret_cast<const void*>(prep), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
       if (rc != 0) return;
     }
-    hipLaunchKernelGGL(prep, dim3(chunks, heads, num_segs), dim3(256), lds, s, ws.p, ws.q, ws.k, ws.g, ws.w, ws.u, in,
-                       start, pos0, slot, heads, dk, dv, num_slots, min_rows);
+    hipLaunchKernelGGL(prep, dim3(chunks, heads, num_segs), dim3(kPrepThreads), lds, s, ws.p, ws.q, ws.k, ws.g, ws.w,
+                       ws.u, in, start, pos0, slot, heads, dk, dv, num_slots, min_rows, quads);
     const dim3 cgrid(heads, (dv + 15) / 16, num_segs);
     if (dk == 16 * DKT && dv % 16 == 0)
       hipLaunchKernelGGL((chunk_carry_kernel<DKT, true, true, DELTA, TV>), cgrid, dim3(256), 0, s, ws.s, ws.w, ws.k, ws.u,

@@ -80,10 +80,12 @@ __device__ __forceinline__ bool find_chunk(Chunk& c, int idx, int s, const int* 
 }
 
 // ab [kC][kPLD]: A below the diagonal (nothing else is read) -> T = (I + A)^-1, the blocks above the
-// diagonal blocks left as they are.  Four waves; a wave's own rows of A have been written by it.
+// diagonal blocks left as they are.  The first four of WAVES waves work; what they read of the diagonal
+// blocks of A has been written by the wave itself or before a barrier.
+template <int WAVES = 4>
 __device__ __forceinline__ void invert_unit_lower(float* ab, int wave, int lo, int hi) {
   wave_lds_fence();
-  {
+  if (WAVES == 4 || wave < 4) {
     // the wave's own diagonal block: lane lo holds column lo of its inverse (the four quarters
     // of the wave do the same work)
     float* d = ab + 16 * wave * kPLD + 16 * wave;

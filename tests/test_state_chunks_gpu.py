@@ -166,3 +166,11 @@ def test_channel_linear(dt_, lens, pos0, heads, dk, dv, fast, monkeypatch):
         return M.gated_linear_attention(p, a, bias, tau, st, seg, heads, dk, dv), st
 
     check(run, ws, wo, dv, monkeypatch)
+
+
+@pytest.mark.parametrize("dt_", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("dk,dv", [(18, 24), (7, 136), (101, 9)])
+def test_channel_sizes_off_quads(dt_, dk, dv, monkeypatch):
+    """Key sizes that are no multiple of the loads' four entries, more value tiles than waves."""
+    test_channel_delta(dt_, [65, 130], [0, 7], 2, 1, dk, dv, False, monkeypatch)
+    test_channel_linear(dt_, [65, 130], [0, 7], 2, dk, dv, True, monkeypatch)
