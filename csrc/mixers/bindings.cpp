@@ -146,10 +146,11 @@ int mx_delta_rule(float* o, const float* qn, const float* kn, const float* g, co
                   const int* slot, int num_segs, int heads, int kv_heads, int dk, int dv, int num_slots,
                   int skip_from, hipStream_t s);
 int mx_channel_delta_chunks(float* o, const float* qn, const float* kn, const float* g, const float* beta,
-                            const void* v, int v_bf16, long v_stride, float* state, float* ws_s, float* ws_p,
-                            float* ws_q, float* ws_k, float* ws_g, float* ws_w, float* ws_u, const int* start,
-                            const int* pos0, const int* slot, int num_segs, int max_rows, int heads, int kv_heads,
-                            int dk, int dv, int num_slots, int min_rows, hipStream_t s);
+                            const void* qkv, int bf16, long stride, const void* a, long a_stride,
+                            const void* b, long b_stride, const float* a_log, const float* dt_bias, float* state,
+                            float* ws_s, float* ws_p, float* ws_q, float* ws_k, float* ws_g, float* ws_w, float* ws_u,
+                            const int* start, const int* pos0, const int* slot, int num_segs, int max_rows, int heads,
+                            int kv_heads, int dk, int dv, int num_slots, int min_rows, hipStream_t s);
 int mx_channel_linear_chunks(float* o, const void* qkv, int bf16, long stride, const void* a, long a_stride,
                              const float* a_bias, float tau, float* state, float* ws_s, float* ws_p, float* ws_q,
                              float* ws_k, float* ws_g, const int* start, const int* pos0, const int* slot,
@@ -512,30 +513,35 @@ void gated_delta_rule(Tensor o, Tensor qkv, Tensor a, Tensor b, Tensor a_log, Te
     return;
   }
   auto f32 = qkv.options().dtype(at::kFloat);
-  Tensor qn = at::empty({t, kv_heads, dk}, f32), kn = at::empty({t, kv_heads, dk}, f32);
-  Tensor g = at::empty({t, heads, dk}, f32), beta = at::empty({t, heads}, f32);
-  chk(mx_delta_prep(qn.data_ptr<float>(), kn.data_ptr<float>(), g.data_ptr<float>(), beta.data_ptr<float>(),
-                    qkv.data_ptr(), bf(qkv), qkv.stride(0), a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0),
-                    a_log.data_ptr<float>(), dt_bias.data_ptr<float>(), t, (int)heads, (int)kv_heads, (int)dk,
-                    stream()), "delta_prep");
   TORCH_CHECK(max_rows <= t && chunk_from >= 1, "delta rule rows");
   const bool chunks = max_rows >= chunk_from && dk <= mx_chunk_max_dk();
-  if (walk || !chunks)
+  Tensor qn, kn, g, beta;
+  const bool ready = walk || !chunks;
+  if (ready) {
+    qn = at::empty({t, kv_heads, dk}, f32), kn = at::empty({t, kv_heads, dk}, f32);
+    g = at::empty({t, heads, dk}, f32), beta = at::empty({t, heads}, f32);
+    chk(mx_delta_prep(qn.data_ptr<float>(), kn.data_ptr<float>(), g.data_ptr<float>(), beta.data_ptr<float>(),
+                      qkv.data_ptr(), bf(qkv), qkv.stride(0), a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0),
+                      a_log.data_ptr<float>(), dt_bias.data_ptr<float>(), t, (int)heads, (int)kv_heads, (int)dk,
+                      stream()), "delta_prep");
     chk(mx_delta_rule(o.data_ptr<float>(), qn.data_ptr<float>(), kn.data_ptr<float>(), g.data_ptr<float>(),
                       beta.data_ptr<float>(), qkv.data_ptr(), bf(qkv), qkv.stride(0), state.data_ptr<float>(),
                       start.data_ptr<int>(), pos0.data_ptr<int>(), slot.data_ptr<int>(), (int)num_segs, (int)heads,
                       (int)kv_heads, (int)dk, (int)dv, (int)state.size(0), chunks ? (int)chunk_from : 0, stream()),
         "delta_rule");
+  }
   if (!chunks) return;
   const ChannelSpace ws(chunk_bound(t, num_segs), heads, dk, dv, true, f32);
-  const char* v = (const char*)qkv.data_ptr() + 2 * kv_heads * dk * qkv.element_size();
-  chk(mx_channel_delta_chunks(o.data_ptr<float>(), qn.data_ptr<float>(), kn.data_ptr<float>(), g.data_ptr<float>(),
-                              beta.data_ptr<float>(), v, bf(qkv), qkv.stride(0), state.data_ptr<float>(),
-                              ws.s.data_ptr<float>(), ws.p.data_ptr<float>(), ws.q.data_ptr<float>(),
-                              ws.k.data_ptr<float>(), ws.g.data_ptr<float>(), ws.w.data_ptr<float>(),
-                              ws.u.data_ptr<float>(), start.data_ptr<int>(), pos0.data_ptr<int>(),
-                              slot.data_ptr<int>(), (int)num_segs, (int)max_rows, (int)heads, (int)kv_heads, (int)dk,
-                              (int)dv, (int)state.size(0), (int)chunk_from, stream()), "delta rule chunks");
+  const auto made = [&](const Tensor& x) { return ready ? x.data_ptr<float>() : nullptr; };
+  chk(mx_channel_delta_chunks(o.data_ptr<float>(), made(qn), made(kn), made(g), made(beta), qkv.data_ptr(),
+                              bf(qkv), qkv.stride(0), a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0),
+                              a_log.data_ptr<float>(), dt_bias.data_ptr<float>(),
+                              state.data_ptr<float>(), ws.s.data_ptr<float>(), ws.p.data_ptr<float>(),
+                              ws.q.data_ptr<float>(), ws.k.data_ptr<float>(), ws.g.data_ptr<float>(),
+                              ws.w.data_ptr<float>(), ws.u.data_ptr<float>(), start.data_ptr<int>(),
+                              pos0.data_ptr<int>(), slot.data_ptr<int>(), (int)num_segs, (int)max_rows, (int)heads,
+                              (int)kv_heads, (int)dk, (int)dv, (int)state.size(0), (int)chunk_from, stream()),
+      "delta rule chunks");
 }
 
 void conv_delta_prep(Tensor qn, Tensor kn, Tensor vo, Tensor lg, Tensor beta, Tensor x, Tensor a, Tensor b,

@@ -23,6 +23,8 @@
 // loads in flight (four waves, loads of one entry, a key per lane on the diagonal: 174 us where this takes
 // 101, and 30 where it takes 17); the carry by its chain.  4096 rows, 16 heads of 128 x 128, delta rule:
 // 101 + 159 + 46 us, the walk 2080; 777 rows, linear attention: 17 + 19 + 16 us, the walk 245.
+// Where no segment of a step is walked, the delta rule's rows come as the projections left them and are normed
+// and their decays formed here (129 us; 101 + 56 for a kernel of its own that writes and reads them again).
 #include "chunk_common.h"
 
 namespace mx {
@@ -31,12 +33,19 @@ struct ChannelIn {
   const void *q, *k, *v;
   long q_stride, k_stride, v_stride;       // elements between rows
   int rep;                                 // heads per q / k head
-  const void* g;                           // DELTA: decays fp32 [T, heads * dk]; else their pre-activation
+  const void* g;                           // pre-activations of the decays, heads * dk columns
   long g_stride;
-  const float* a_bias;                     // [heads * dk] (pre-activation form)
+  const float* a_bias;                     // [heads * dk]
   float inv_tau, q_scale;
-  const float* beta;                       // DELTA: [T, heads]
+  // delta rule: q and k become unit vectors (q times q_scale), decays e^{-e^{a_log} softplus}, beta a sigmoid;
+  // or (a_log null) q, k, decays and beta as they stand, in fp32: where a step's short segments are walked, they
+  // have been prepared for all of its rows
+  const float* a_log;                      // [heads]
+  const void* b;                           // (pre-activations of) beta, heads columns
+  long b_stride;
 };
+
+enum ChannelRows { kLinear, kDelta, kReady };      // what channel_prep does to its rows
 
 // floats of dynamic LDS of channel_prep
 template <int DKT>
@@ -54,7 +63,7 @@ template <int ctrl>
 __device__ __forceinline__ float dpp(float x) {
   return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), ctrl, 0xf, 0xf, true));
 }
-constexpr int kSwap1 = 0xB1, kSwap2 = 0x4E, kRor4 = 0x124, kRor8 = 0x128;
+constexpr int kSwap1 = 0xB1, kSwap2 = 0x4E, kHalfMirror = 0x141, kMirror = 0x140, kRor4 = 0x124, kRor8 = 0x128;
 
 // sums over 16 lanes: a, b, c, d land in lanes 0, 1, 2, 3 (mod 4) of the sixteen
 __device__ __forceinline__ float sum16(float a, float b, float c, float d, int lane) {
@@ -65,7 +74,18 @@ __device__ __forceinline__ float sum16(float a, float b, float c, float d, int l
   return x + dpp<kRor8>(x);
 }
 
-template <int DKT, bool DELTA, typename TQ, typename TV>
+// sum over LPR lanes in a row (4 to 32, a power of two)
+template <int LPR>
+__device__ __forceinline__ float sum_lanes(float x) {
+  x += dpp<kSwap1>(x);
+  x += dpp<kSwap2>(x);
+  if constexpr (LPR > 4) x += dpp<kHalfMirror>(x);
+  if constexpr (LPR > 8) x += dpp<kMirror>(x);
+  if constexpr (LPR > 16) x = add_row_pair(x);
+  return x;
+}
+
+template <int DKT, bool DELTA, typename T>
 __global__ void __launch_bounds__(kPrepThreads)
 channel_prep_kernel(float* __restrict__ ws_p, float* __restrict__ ws_q, float* __restrict__ ws_k,
                     float* __restrict__ ws_g, float* __restrict__ ws_w, float* __restrict__ ws_u, ChannelIn in,
@@ -81,32 +101,48 @@ channel_prep_kernel(float* __restrict__ ws_p, float* __restrict__ ws_q, float* _
   const int h = blockIdx.y;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lo = lane & 15, hi = lane >> 4, half = wave >> 2;
-  {
+  auto stage = [&](auto type, auto rows) {
+    using TQ = decltype(type);
+    constexpr ChannelRows R = decltype(rows)::value;
     const long kh = (long)(h / in.rep) * dk;
     const TQ *qp = (const TQ*)in.q + c.row0 * in.q_stride + kh, *kp = (const TQ*)in.k + c.row0 * in.k_stride + kh;
     const TQ* gp = (const TQ*)in.g + c.row0 * in.g_stride + (long)h * dk;
+    const float* bias = in.a_bias + (long)h * dk;
+    const float rate = R == kDelta ? expf(in.a_log[h]) : 0.f;
+    auto decay = [&](float z, int i) {
+      if constexpr (R == kReady) return z;
+      else if constexpr (R == kDelta) return expf(-rate * softplusf_(z + bias[i]));
+      else return gla_decay(z + bias[i], in.inv_tau);
+    };
+    auto unit = [](float square) { return 1.0f / sqrtf(square + 1e-6f); };
     if (vec) {                                                     // dk a multiple of 4; addresses stay inside the rows
-      constexpr int QUADS = kC * DKP / 4, N = (QUADS + kPrepThreads - 1) / kPrepThreads;
+      constexpr int LPR = DKP / 4, QUADS = kC * LPR, N = (QUADS + kPrepThreads - 1) / kPrepThreads;
       float k[N][4], q[N][4], g[N][4];
+      const int i = tid % LPR * 4, ic = min(i, dk - 4);            // the same columns every time
 #pragma unroll
       for (int n = 0; n < N; ++n) {
-        const int e = tid + n * kPrepThreads;
-        const int t = min(e / (DKP / 4), c.cnt - 1), i = min(e % (DKP / 4) * 4, dk - 4);
-        load4(kp + t * in.k_stride + i, k[n]);
-        load4(qp + t * in.q_stride + i, q[n]);
-        load4(gp + t * in.g_stride + i, g[n]);
+        const int t = min((tid + n * kPrepThreads) / LPR, c.cnt - 1);
+        load4(kp + t * in.k_stride + ic, k[n]);
+        load4(qp + t * in.q_stride + ic, q[n]);
+        load4(gp + t * in.g_stride + ic, g[n]);
       }
 #pragma unroll
       for (int n = 0; n < N; ++n) {
-        const int e = tid + n * kPrepThreads, t = e / (DKP / 4), i = e % (DKP / 4) * 4;
-        if (QUADS % kPrepThreads != 0 && e >= QUADS) continue;
+        const int e = tid + n * kPrepThreads, t = e / LPR;
+        if (QUADS % kPrepThreads != 0 && e >= QUADS) continue;     // (whole waves)
         const bool live = t < c.cnt && i < dk;
+        float rk = 1.f, rq = in.q_scale;
+        if constexpr (R == kDelta) {
+          const float sk = (k[n][0] * k[n][0] + k[n][1] * k[n][1]) + (k[n][2] * k[n][2] + k[n][3] * k[n][3]);
+          const float sq = (q[n][0] * q[n][0] + q[n][1] * q[n][1]) + (q[n][2] * q[n][2] + q[n][3] * q[n][3]);
+          rk = unit(sum_lanes<LPR>(i < dk ? sk : 0.f));
+          rq *= unit(sum_lanes<LPR>(i < dk ? sq : 0.f));
+        }
 #pragma unroll
         for (int x = 0; x < 4; ++x) {
-          if constexpr (!DELTA) g[n][x] = gla_decay(g[n][x] + in.a_bias[(long)h * dk + min(i, dk - 4) + x], in.inv_tau);
-          k[n][x] = live ? k[n][x] : 0.f;
-          q[n][x] = live ? q[n][x] * in.q_scale : 0.f;
-          g[n][x] = live ? g[n][x] : 1.f;
+          k[n][x] = live ? k[n][x] * rk : 0.f;
+          q[n][x] = live ? q[n][x] * rq : 0.f;
+          g[n][x] = live ? decay(g[n][x], ic + x) : 1.f;
         }
         *reinterpret_cast<float4*>(kb + t * LDK + i) = make_float4(k[n][0], k[n][1], k[n][2], k[n][3]);
         *reinterpret_cast<float4*>(qb + t * LDK + i) = make_float4(q[n][0], q[n][1], q[n][2], q[n][3]);
@@ -119,17 +155,40 @@ channel_prep_kernel(float* __restrict__ ws_p, float* __restrict__ ws_q, float* _
         float k = 0.f, q = 0.f, g = 1.f;
         if (t < c.cnt && i < dk) {
           k = ld(kp, t * in.k_stride + i);
-          q = ld(qp, t * in.q_stride + i) * in.q_scale;
-          g = ld(gp, t * in.g_stride + i);
-          if constexpr (!DELTA) g = gla_decay(g + in.a_bias[(long)h * dk + i], in.inv_tau);
+          q = ld(qp, t * in.q_stride + i);
+          g = decay(ld(gp, t * in.g_stride + i), i);
+          if constexpr (R != kDelta) q *= in.q_scale;
         }
         kb[t * LDK + i] = k;
         qb[t * LDK + i] = q;
         gb[t * LDK + i] = g;
       }
+      if constexpr (R == kDelta) {                                       // eight threads a row
+        __syncthreads();
+        float *kr = kb + (tid >> 3) * LDK, *qr = qb + (tid >> 3) * LDK, sk = 0.f, sq = 0.f;
+        for (int i = tid & 7; i < DKP; i += 8) {
+          sk += kr[i] * kr[i];
+          sq += qr[i] * qr[i];
+        }
+        const float rk = unit(sum_lanes<8>(sk)), rq = unit(sum_lanes<8>(sq)) * in.q_scale;
+        for (int i = tid & 7; i < DKP; i += 8) {
+          kr[i] *= rk;
+          qr[i] *= rq;
+        }
+      }
     }
-    if (DELTA && tid < kC) bs[tid] = tid < c.cnt ? in.beta[(c.row0 + tid) * heads + h] : 0.f;
-  }
+    if (R != kLinear && tid < kC) {
+      float x = 0.f;
+      if (tid < c.cnt) {
+        x = ld((const TQ*)in.b, (c.row0 + tid) * in.b_stride + h);
+        if constexpr (R == kDelta) x = sigmoidf_(x);
+      }
+      bs[tid] = x;
+    }
+  };
+  if constexpr (!DELTA) stage(T{}, std::integral_constant<ChannelRows, kLinear>{});
+  else if (in.a_log != nullptr) stage(T{}, std::integral_constant<ChannelRows, kDelta>{});
+  else stage(float{}, std::integral_constant<ChannelRows, kReady>{});
   __syncthreads();
   // diagonal blocks: wave (block, half) has the keys 8 half .. 8 half + 7 of a block and walks the rows from
   // there; a lane two keys and DKT channels, so that a row read from LDS serves two keys and sixteen lanes add up
@@ -256,7 +315,7 @@ channel_prep_kernel(float* __restrict__ ws_p, float* __restrict__ ws_q, float* _
     const int vtiles = (dv + 15) / 16;
     float vr[16];
     auto fetch_v = [&](int ct) {                                   // rows past cnt: beta is 0; columns past dv are not used
-      const TV* vp = (const TV*)in.v + c.row0 * in.v_stride + (long)h * dv + min(16 * ct + lo, dv - 1);
+      const T* vp = (const T*)in.v + c.row0 * in.v_stride + (long)h * dv + min(16 * ct + lo, dv - 1);
 #pragma unroll
       for (int s = 0; s < 16; ++s) vr[s] = ld(vp, min(4 * s + hi, c.cnt - 1) * in.v_stride);
     };
@@ -379,7 +438,7 @@ struct ChannelWs {
   float *s, *p, *q, *k, *g, *w, *u;
 };
 
-template <bool DELTA, typename TQ, typename TV>
+template <bool DELTA, typename T>
 int channel_run(float* o, const ChannelIn& in, const ChannelWs& ws, float* state, const int* start, const int* pos0,
                 const int* slot, int num_segs, int max_rows, int heads, int dk, int dv, int num_slots, int min_rows,
                 int vec, hipStream_t s) {
@@ -388,11 +447,11 @@ int channel_run(float* o, const ChannelIn& in, const ChannelWs& ws, float* state
   if (heads > 65535 || outs > 65535 || num_segs > 65535) return -2;
   // whole quads of q, k and g at aligned addresses
   const int quads = dk % 4 == 0 && in.q_stride % 4 == 0 && in.k_stride % 4 == 0 && in.g_stride % 4 == 0 &&
-                    ((uintptr_t)in.q | (uintptr_t)in.k | (uintptr_t)in.g) % (4 * sizeof(TQ)) == 0;
+                    ((uintptr_t)in.q | (uintptr_t)in.k | (uintptr_t)in.g) % (4 * (DELTA && in.a_log == nullptr ? sizeof(float) : sizeof(T))) == 0;
   int rc = 0;
-  key_tiles(dk, [&](auto t) {
-    constexpr int DKT = decltype(t)::value, lds = kPrepFloats<DKT> * 4;
-    auto prep = channel_prep_kernel<DKT, DELTA, TQ, TV>;
+  key_tiles(dk, [&](auto tiles) {
+    constexpr int DKT = decltype(tiles)::value, lds = kPrepFloats<DKT> * 4;
+    auto prep = channel_prep_kernel<DKT, DELTA, T>;
     if constexpr (lds > 64 * 1024) {
       rc = (int)hipFuncSetAttribute(reinterpret_cast<const void*>(prep), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
       if (rc != 0) return;
@@ -401,12 +460,12 @@ int channel_run(float* o, const ChannelIn& in, const ChannelWs& ws, float* state
                        ws.u, in, start, pos0, slot, heads, dk, dv, num_slots, min_rows, quads);
     const dim3 cgrid(heads, (dv + 15) / 16, num_segs);
     if (dk == 16 * DKT && dv % 16 == 0)
-      hipLaunchKernelGGL((chunk_carry_kernel<DKT, true, true, DELTA, TV>), cgrid, dim3(256), 0, s, ws.s, ws.w, ws.k, ws.u,
-                         ws.g, (const TV*)in.v, in.v_stride, state, start, pos0, slot, heads, dk, dv, num_slots, min_rows);
+      hipLaunchKernelGGL((chunk_carry_kernel<DKT, true, true, DELTA, T>), cgrid, dim3(256), 0, s, ws.s, ws.w, ws.k, ws.u,
+                         ws.g, (const T*)in.v, in.v_stride, state, start, pos0, slot, heads, dk, dv, num_slots, min_rows);
     else
-      hipLaunchKernelGGL((chunk_carry_kernel<DKT, false, true, DELTA, TV>), cgrid, dim3(256), 0, s, ws.s, ws.w, ws.k, ws.u,
-                         ws.g, (const TV*)in.v, in.v_stride, state, start, pos0, slot, heads, dk, dv, num_slots, min_rows);
-    hipLaunchKernelGGL((channel_out_kernel<DKT, DELTA, TV>), dim3(chunks, (unsigned)outs, num_segs), dim3(256), 0, s, o, in,
+      hipLaunchKernelGGL((chunk_carry_kernel<DKT, false, true, DELTA, T>), cgrid, dim3(256), 0, s, ws.s, ws.w, ws.k, ws.u,
+                         ws.g, (const T*)in.v, in.v_stride, state, start, pos0, slot, heads, dk, dv, num_slots, min_rows);
+    hipLaunchKernelGGL((channel_out_kernel<DKT, DELTA, T>), dim3(chunks, (unsigned)outs, num_segs), dim3(256), 0, s, o, in,
                        ws.s, ws.p, ws.q, ws.u, start, pos0, slot, heads, dk, dv, num_slots, min_rows, vec);
   });
   return rc != 0 ? rc : (int)hipGetLastError();
@@ -418,28 +477,42 @@ using namespace mx;
 
 // Workspaces, floats per (chunk, head): s dk dv, p 4096, q and k 64 times the padded key size, g the padded
 // key size; delta rule: w as k, u 64 times dv up to a multiple of 16.
+// qn, kn, g, beta: the rows prepared (mx_delta_prep), or null.
 extern "C" int mx_channel_delta_chunks(float* o, const float* qn, const float* kn, const float* g, const float* beta,
-                                       const void* v, int v_bf16, long v_stride, float* state, float* ws_s, float* ws_p,
-                                       float* ws_q, float* ws_k, float* ws_g, float* ws_w, float* ws_u, const int* start,
-                                       const int* pos0, const int* slot, int num_segs, int max_rows, int heads,
-                                       int kv_heads, int dk, int dv, int num_slots, int min_rows, hipStream_t s) {
+                                       const void* qkv, int bf16, long stride, const void* a, long a_stride,
+                                       const void* b, long b_stride, const float* a_log, const float* dt_bias,
+                                       float* state, float* ws_s, float* ws_p, float* ws_q, float* ws_k, float* ws_g,
+                                       float* ws_w, float* ws_u, const int* start, const int* pos0, const int* slot,
+                                       int num_segs, int max_rows, int heads, int kv_heads, int dk, int dv,
+                                       int num_slots, int min_rows, hipStream_t s) {
   if (num_segs <= 0 || max_rows < min_rows) return 0;
   if (dk < 1 || dk > 128 || dv < 1 || kv_heads < 1 || heads % kv_heads || min_rows < 1) return -1;
   if (((uintptr_t)ws_p | (uintptr_t)ws_q | (uintptr_t)ws_k | (uintptr_t)ws_g | (uintptr_t)ws_w | (uintptr_t)ws_u) % 16) return -3;
+  const long es = bf16 ? 2 : 4;
   ChannelIn in{};
-  in.q = qn; in.k = kn; in.v = v; in.g = g;
-  in.q_stride = in.k_stride = (long)kv_heads * dk;
-  in.g_stride = (long)heads * dk;
-  in.v_stride = v_stride;
+  in.q = qkv;
+  in.k = (const char*)qkv + es * kv_heads * dk;
+  in.v = (const char*)qkv + es * 2 * kv_heads * dk;
+  in.g = a;
+  in.q_stride = in.k_stride = in.v_stride = stride;
+  in.g_stride = a_stride;
   in.rep = heads / kv_heads;
-  in.q_scale = 1.f;
-  in.beta = beta;
+  in.a_bias = dt_bias;
+  in.q_scale = 1.0f / sqrtf((float)dk);
+  in.a_log = a_log;
+  in.b = b;
+  in.b_stride = b_stride;
+  if (qn != nullptr) {
+    in.q = qn; in.k = kn; in.g = g; in.b = beta;
+    in.q_stride = in.k_stride = (long)kv_heads * dk;
+    in.g_stride = (long)heads * dk;
+    in.b_stride = heads;
+    in.a_log = nullptr;
+    in.q_scale = 1.f;
+  }
   const ChannelWs ws{ws_s, ws_p, ws_q, ws_k, ws_g, ws_w, ws_u};
-  if (v_bf16)
-    return channel_run<true, float, bf16_t>(o, in, ws, state, start, pos0, slot, num_segs, max_rows, heads, dk, dv,
-                                            num_slots, min_rows, 0, s);
-  return channel_run<true, float, float>(o, in, ws, state, start, pos0, slot, num_segs, max_rows, heads, dk, dv, num_slots,
-                                         min_rows, 0, s);
+  MX_DISPATCH_T(bf16, return (channel_run<true, T>(o, in, ws, state, start, pos0, slot, num_segs, max_rows, heads, dk, dv,
+                                                   num_slots, min_rows, 0, s)));
 }
 
 extern "C" int mx_channel_linear_chunks(float* o, const void* qkv, int bf16, long stride, const void* a, long a_stride,
@@ -464,6 +537,6 @@ extern "C" int mx_channel_linear_chunks(float* o, const void* qkv, int bf16, lon
   in.q_scale = 1.0f / sqrtf((float)dk);
   const int vec = dk % 4 == 0 && dv % 4 == 0 && stride % 4 == 0 && ((uintptr_t)qkv) % (4 * es) == 0;
   const ChannelWs ws{ws_s, ws_p, ws_q, ws_k, ws_g, nullptr, nullptr};
-  MX_DISPATCH_T(bf16, return (channel_run<false, T, T>(o, in, ws, state, start, pos0, slot, num_segs, max_rows, heads, dk,
+  MX_DISPATCH_T(bf16, return (channel_run<false, T>(o, in, ws, state, start, pos0, slot, num_segs, max_rows, heads, dk,
                                                        dv, num_slots, min_rows, vec, s)));
 }
