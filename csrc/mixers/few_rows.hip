@@ -102,11 +102,13 @@ struct ExpertSet {
   int shared_K, shared_N;
 };
 
-// the (row, choice) pairs that chose expert e -> list, ascending; returns their number.  At most
-// one pair per row.  All threads of the workgroup call it.
+// the (row, choice) pairs that chose expert e, in ascending order: those numbered from .. from + room - 1 -> list;
+// returns how many there are in all.  A router names an expert once per row, except for a row of NaN, whose choices
+// are all the same; and an index outside the experts counts as the first's.  So there may be more pairs than rows.
+// All threads of the workgroup call it; its barriers end their reads of the list before.
 template <int WV>
-__device__ __forceinline__ int pairs_of(const int* __restrict__ idx, int pairs, int top, int experts, int e, int* list,
-                                        int* counts) {
+__device__ __forceinline__ int pairs_of(const int* __restrict__ idx, int pairs, int experts, int e, int from, int room,
+                                        int* list, int* counts) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   int total = 0;
   for (int p0 = 0; p0 < pairs; p0 += 64 * WV) {
@@ -125,12 +127,12 @@ __device__ __forceinline__ int pairs_of(const int* __restrict__ idx, int pairs, 
       total += counts[w];
     }
     if (v == e) {
-      const int at = before + __popcll(m & ((1ull << lane) - 1));
-      if (at < kFewRows) list[at] = p;
+      const int at = before + __popcll(m & ((1ull << lane) - 1)) - from;
+      if (at >= 0 && at < room) list[at] = p;
     }
     __syncthreads();
   }
-  return min(total, kFewRows);
+  return total;
 }
 
 // the tile's sums for the listed rows: f(entry row in the list, column, sums, up sums)
@@ -194,15 +196,17 @@ experts_first_kernel(bf16_t* __restrict__ y, bf16_t* __restrict__ ys, float* __r
   const int e = blockIdx.y, n0 = blockIdx.x * 16 * P;
   if (e < E.experts) {
     if (n0 >= E.N) return;
-    const int count = pairs_of<kExpWaves>(idx, rows * top, top, E.experts, e, list, counts);
-    if (count == 0) return;
     const bf16_t* W = E.w + (long)e * E.N * (GLU ? 2 : 1) * E.K;
-    expert_tile_any<P, GLU, kExpWaves, MB>(red, W, E.N, E.K, n0, h, h_stride, list, count, top, wave, lane,
-                                       [&](int r, int c, float (&v)[4], float (&u)[4]) {
+    for (int from = 0, total = 1; from < total; from += 16 * MB) {       // (one turn, but for repeated choices)
+      total = pairs_of<kExpWaves>(idx, rows * top, E.experts, e, from, 16 * MB, list, counts);
+      if (total == 0) return;
+      expert_tile_any<P, GLU, kExpWaves, MB>(red, W, E.N, E.K, n0, h, h_stride, list, min(total - from, 16 * MB), top, wave, lane,
+                                         [&](int r, int c, float (&v)[4], float (&u)[4]) {
 #pragma unroll
-                                         for (int i = 0; i < 4; ++i) v[i] = fr_act(act, limit, v[i], u[i]);
-                                         fr_store4(y + (long)list[r] * E.N, c, E.N, vec != 0, v);
-                                       });
+                                           for (int i = 0; i < 4; ++i) v[i] = fr_act(act, limit, v[i], u[i]);
+                                           fr_store4(y + (long)list[r] * E.N, c, E.N, vec != 0, v);
+                                         });
+    }
     return;
   }
   const int tiles = (E.shared_N + 16 * P - 1) / (16 * P);
@@ -234,24 +238,22 @@ experts_down_kernel(float* __restrict__ d, float* __restrict__ ds, const bf16_t*
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int e = blockIdx.y, n0 = blockIdx.x * 16 * P;
-  float* dst = d;
-  const bf16_t *W = E.w + (long)e * E.N * E.K, *X = y;
-  int K = E.K, count = rows;
-  if (e < E.experts) {
-    count = pairs_of<kExpWaves>(idx, rows * top, top, E.experts, e, list, counts);
-    if (count == 0) return;
-  } else {
+  const bool own = e < E.experts;
+  float* dst = own ? d : ds;
+  const bf16_t *W = own ? E.w + (long)e * E.N * E.K : E.shared, *X = own ? y : ys;
+  const int K = own ? E.K : E.shared_K;
+  if (!own) {
     if (tid < rows) list[tid] = tid;
     __syncthreads();
-    dst = ds;
-    W = E.shared;
-    X = ys;
-    K = E.shared_K;
   }
-  expert_tile_any<P, false, kExpWaves, MB>(red, W, E.N, K, n0, X, K, list, count, 1, wave, lane,
-                                       [&](int r, int c, float (&v)[4], float (&)[4]) {
-                                         fr_store4(dst + (long)list[r] * E.N, c, E.N, vec != 0, v);
-                                       });
+  for (int from = 0, total = rows; from < total; from += 16 * MB) {
+    if (own) total = pairs_of<kExpWaves>(idx, rows * top, E.experts, e, from, 16 * MB, list, counts);
+    if (total == 0) return;
+    expert_tile_any<P, false, kExpWaves, MB>(red, W, E.N, K, n0, X, K, list, min(total - from, 16 * MB), 1, wave, lane,
+                                         [&](int r, int c, float (&v)[4], float (&)[4]) {
+                                           fr_store4(dst + (long)list[r] * E.N, c, E.N, vec != 0, v);
+                                         });
+  }
 }
 
 // out[row] = sum_k wts[row, k] d[row, k] + shared[row] * (sigmoid(sg[row]) or 1)
@@ -337,7 +339,7 @@ extern "C" int mx_experts_few(float* out, void* y, float* d, const void* h, long
                               const void* shared_w, const void* shared_down, int shared_ff, float shared_limit,
                               hipStream_t s) {
   if (rows <= 0) return 0;
-  if (rows > kFewRows || experts < 1 || experts > 65534 || top < 1 || top > experts || ff % 8 || width % 8 ||
+  if (rows > kFewRows || experts < 1 || experts > 65534 || top < 1 || ff % 8 || width % 8 ||
       ff < 8 || width < 8 || h_stride % 8 || shared_ff % 8 || act < kFrGelu || act > kFrReluSq) return -1;
   if (((uintptr_t)h) % 16 || ((uintptr_t)wgu) % 16 || ((uintptr_t)wdown) % 16 || ((uintptr_t)shared_w) % 16 ||
       ((uintptr_t)shared_down) % 16) return -2;

@@ -99,3 +99,28 @@ def test_experts(act, name, rows, experts, top, ff, width, shared):
     err = (got.double() - want).abs()
     assert bool((err <= mag * 2.0 ** -8 + 1e-5).all()), float(err.max())
     torch.testing.assert_close(got, M.experts_few(h, idx, wts, w1, w2, act, 1.5, sh, 0.75, gate), rtol=0, atol=0)
+
+
+@pytest.mark.parametrize("rows,experts,top", [(16, 8, 6), (17, 4, 6), (32, 8, 2), (64, 6, 3), (64, 32, 6)])
+@pytest.mark.parametrize("act", ["clamp_glu", "relu_sq"])
+def test_repeated_choices_keep_to_their_rows(act, rows, experts, top):
+    """More pairs than rows for one expert (rows of NaN choose it again and again, indices outside the experts count as
+    it): every row's result is that of the row alone."""
+    g = torch.Generator().manual_seed(rows + top)
+    width, ff, few = 64, 40, min(top, experts)
+    w1 = rnd(g, experts, (1 if act == "relu_sq" else 2) * ff, width, scale=width ** -0.5)
+    w2 = rnd(g, experts, width, ff, scale=ff ** -0.5)
+    h, router = rnd(g, rows, width), torch.randn(experts, width, generator=g).to(DEV)
+    h[:5] = float("nan")
+    idx, wts = M.moe_route_top_logits(h, router, None, few)
+    idx, wts = torch.cat([idx, idx[:, :top - few]], 1).contiguous(), torch.cat([wts, wts[:, :top - few]], 1).contiguous()
+    idx[6, 0], idx[7, top - 1] = -1, experts
+    idx[8:12] = 0
+    idx[rows // 2:, 1] = 0
+    spoiled = torch.full((rows * top * width,), float("nan"), device=DEV)     # what a row left out would read
+    del spoiled
+    got = M.experts_few(h, idx, wts, w1, w2, act, 1.5)
+    alone = torch.cat([M.experts_few(h[r:r + 1], idx[r:r + 1].contiguous(), wts[r:r + 1], w1, w2, act, 1.5)
+                       for r in range(rows)])
+    assert bool(alone[5:].isfinite().all()) and bool(alone[:5].isnan().all())
+    assert torch.equal(got[5:], alone[5:]) and bool(got[:5].isnan().all())
