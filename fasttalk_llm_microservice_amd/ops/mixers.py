@@ -71,6 +71,17 @@ class Segments:
     host: Optional[tuple] = None
 
 
+def _plain16(*tensors) -> bool:
+    """Dense tensors at 16-byte addresses, as kernels take them that read and write whole pieces."""
+    return all(t.is_contiguous() and t.data_ptr() % 16 == 0 for t in tensors)
+
+
+def _device_segments(seg: Segments) -> bool:
+    """Whether a kernel can read the segments itself (the product forms go by the host's copies)."""
+    return all(t.is_cuda and t.dtype == torch.int32 and t.is_contiguous()
+               for t in (seg.start, seg.pos0, seg.kv_len, seg.block_tables))
+
+
 # ---------------------------------------------------------------------------------
 # products with weights [out, in]
 # ---------------------------------------------------------------------------------
@@ -803,6 +814,15 @@ def band_weights(s, first_pos: int, key0: int, spec: WindowSpec, rep_rows: int, 
     return s
 
 
+def band_attention_ok(out, q, k_cache, v_cache, seg: Segments, spec: WindowSpec) -> bool:
+    """Whether long segments run in one kernel (csrc/mixers/band_attn.hip) instead of banded products: bf16 caches of
+    heads that fit its tiles, all operands dense and aligned."""
+    return bool(q.is_cuda and k_cache.dtype == v_cache.dtype == torch.bfloat16 and q.dtype == torch.float32 and q.dim() == 2
+                and out.dtype in (torch.float32, torch.bfloat16) and _plain16(out, q, k_cache, v_cache)
+                and _device_segments(seg)
+                and native_mixers().band_attention_fits(spec.dk, spec.dv, k_cache.shape[1]))
+
+
 def window_attention_products(out, q, k_cache, v_cache, seg: Segments, spec: WindowSpec, min_rows: int):
     """Segments of ``min_rows`` rows or more as banded matrix products: a chunk of rows
     [c0, c1) only sees the keys c0 - window + 1 .. c1 - 1 (or from the start of c0's block;
@@ -816,7 +836,7 @@ def window_attention_products(out, q, k_cache, v_cache, seg: Segments, spec: Win
     sp = spec
     start, pos0, kv_len = seg.host
     bs = k_cache.shape[1]
-    if q.is_cuda and k_cache.dtype == torch.bfloat16 and native_mixers().band_attention_fits(sp.dk, sp.dv, bs):
+    if band_attention_ok(out, q, k_cache, v_cache, seg, sp):
         # one kernel for all segments, scores never in memory
         ns = [n for n in (b - a for a, b in zip(start[:-1], start[1:])) if n >= min_rows]
         native_mixers().band_attention(out, q, k_cache, v_cache, seg.start, seg.pos0, seg.kv_len, seg.block_tables,

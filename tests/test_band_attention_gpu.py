@@ -121,3 +121,47 @@ def test_against_64_bits(name, sizes, opt, lens, pos0, bs, monkeypatch):
     assert torch.equal(again[rows], got[rows])
     half = M.window_attention_products(torch.zeros_like(out, dtype=torch.bfloat16), q, kc, vc, seg, sp, 32)
     assert torch.equal(half[rows], got[rows].bfloat16())       # rounded once, on the way out
+
+
+def off_by_one(x):
+    """x at an address two or four bytes past a 16-byte boundary"""
+    flat = torch.empty(x.numel() + 1, dtype=x.dtype, device=x.device)[1:]
+    return flat.copy_(x.flatten()).view(x.shape)
+
+
+@pytest.mark.parametrize("form", ["q columns", "q off", "q heads apart", "k off", "v off", "k pages apart", "out rows apart",
+                                  "out off", "wide tables", "table columns", "start apart"])
+def test_operands_of_other_layouts(form):
+    """Operands that are not dense or not aligned: the banded products take them."""
+    g = torch.Generator().manual_seed(3)
+    sp = M.WindowSpec(heads=4, kv_heads=2, dk=64, dv=64, window=0, scale=0.125)
+    seg, blocks = segments([40, 3, 65], [9, 0, 30], 4, g)
+    kc, vc = (torch.randn(blocks, 4, 128, generator=g).to(DEV, torch.bfloat16) for _ in range(2))
+    q = torch.randn(108, 256, generator=g).to(DEV)
+    out = torch.full((108, 4, 64), 7.0, device=DEV)
+    want = M.window_attention_products(out.clone(), q, kc, vc, seg, sp, 32)
+    if form == "q columns":
+        q = torch.cat([q, q], 1)[:, 256:]
+    elif form == "q off":
+        q = off_by_one(q)
+    elif form == "q heads apart":
+        q = q.view(108, 4, 64)
+    elif form == "k off":
+        kc = off_by_one(kc)
+    elif form == "v off":
+        vc = off_by_one(vc)
+    elif form == "k pages apart":
+        kc = torch.cat([kc, kc], 1)[:, 4:]
+    elif form == "out rows apart":
+        out = torch.full((108, 8, 64), 7.0, device=DEV)[:, 4:]
+    elif form == "out off":
+        out = off_by_one(out)
+    elif form == "wide tables":
+        seg.block_tables = seg.block_tables.long()
+    elif form == "table columns":
+        seg.block_tables = torch.cat([seg.block_tables, seg.block_tables], 1)[:, :seg.block_tables.shape[1]]
+    else:
+        seg.start = torch.stack([seg.start, seg.start], 1)[:, 0]
+    got = M.window_attention_products(out, q, kc, vc, seg, sp, 32)
+    # both forms are within 1e-6 of the sums in 64 bits (test_against_64_bits)
+    torch.testing.assert_close(got, want, rtol=0, atol=2e-6 * float(want.abs().max()))
