@@ -75,3 +75,42 @@ def test_latent_prefill(lens, pos0, heads, page, sink, rise):
             # weights rounded to bf16 (half a unit: 2^-8); scores of up to 2^8 and their sums in fp32 (2^-12)
             assert bool(((got - w).abs() <= (2 ** -8 + 2 ** -12) * z + 1e-6).all())
         a += n
+
+
+@pytest.mark.parametrize("form", ["queries across", "queries off", "rotated across", "cache off", "pages apart", "out across",
+                                  "wide tables", "bf16 queries"])
+def test_operands_of_other_layouts(form):
+    """Operands that are not dense, aligned or fp32: the two products take them."""
+    g = torch.Generator(device=DEV).manual_seed(5)
+    heads, lens, pos0 = 2, [70, 5, 33], [3, 0, 20]
+    t = sum(lens)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=DEV)      # noqa: E731
+    off = lambda x: torch.empty(x.numel() + 1, dtype=x.dtype, device=DEV)[1:].copy_(x.flatten()).view(x.shape)   # noqa: E731
+    seg, blocks = make_seg(lens, pos0, [0, 1, 2], block_size=8)
+    seg = to_dev(seg)
+    seg.host = (seg.start.tolist(), seg.pos0.tolist(), seg.kv_len.tolist())
+    cache = rnd(blocks, 8, RANK + DR).bfloat16()
+    qa, qr = rnd(heads, t, RANK).bfloat16().float(), rnd(t, heads, DR).bfloat16().float()
+    out = torch.zeros(heads, t, RANK, device=DEV)
+    want, size = reference(qa, qr, cache, seg, lens, pos0, 0.05, None)
+    if form == "queries across":
+        qa = qa.transpose(0, 1).contiguous().transpose(0, 1)
+    elif form == "queries off":
+        qa = off(qa)
+    elif form == "rotated across":
+        qr = torch.cat([qr, qr], 2)[..., DR:]
+    elif form == "cache off":
+        cache = off(cache)
+    elif form == "pages apart":
+        cache = torch.cat([cache, cache], 1)[:, 8:]
+    elif form == "out across":
+        out = out.transpose(0, 1).contiguous().transpose(0, 1)
+    elif form == "wide tables":
+        seg.block_tables = seg.block_tables.long()
+    else:
+        qa, qr = qa.bfloat16(), qr.bfloat16()
+    M.latent_attention_products(out, qa, qr, cache, seg, 0.05, RANK, 32, torch.bfloat16)
+    rows = torch.cat([torch.full((n,), n >= 32) for n in lens]).to(DEV)
+    # weights rounded to bf16 twice at most: 2^-8 (a sum and its quotient)
+    assert bool(((out.double() - want)[:, rows].abs() <= (2 ** -8 + 2 ** -12) * size[:, rows] + 1e-6).all())
+    assert bool((out[:, ~rows] == 0).all())
