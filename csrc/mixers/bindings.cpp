@@ -513,7 +513,8 @@ void gated_delta_rule(Tensor o, Tensor qkv, Tensor a, Tensor b, Tensor a_log, Te
     return;
   }
   auto f32 = qkv.options().dtype(at::kFloat);
-  TORCH_CHECK(max_rows <= t && chunk_from >= 1, "delta rule rows");
+  TORCH_CHECK(chunk_from >= 1, "delta rule rows");
+  max_rows = std::min(max_rows, t);     // (a bound may be given)
   const bool chunks = max_rows >= chunk_from && dk <= mx_chunk_max_dk();
   Tensor qn, kn, g, beta;
   const bool ready = walk || !chunks;
@@ -660,7 +661,8 @@ void gated_linear_attention(Tensor o, Tensor qkv, Tensor a, Tensor a_bias, doubl
   TORCH_CHECK(state.dim() == 4 && state.size(1) == heads && state.size(2) == dk && state.size(3) == dv, "state");
   check_segs(start, pos0, slot, num_segs);
   TORCH_CHECK(start.numel() >= num_segs + 1, "segments");
-  TORCH_CHECK(max_rows <= t && chunk_from >= 1, "linear attention rows");
+  TORCH_CHECK(chunk_from >= 1, "linear attention rows");
+  max_rows = std::min(max_rows, t);     // (a bound may be given)
   if (max_rows == 1 && mx_state_step_fits(o.data_ptr<float>(), state.data_ptr<float>(), (int)dk, (int)dv)) {
     chk(mx_state_step(1, o.data_ptr<float>(), qkv.data_ptr(), bf(qkv), qkv.stride(0), a.data_ptr(), a.stride(0), nullptr,
                       0, nullptr, a_bias.data_ptr<float>(), nullptr, 1.0f / (float)tau, state.data_ptr<float>(),
@@ -1318,7 +1320,8 @@ void ssd_scan(Tensor y, Tensor xbc, Tensor dt, Tensor a_log, Tensor dt_bias, Ten
               d_skip.numel() == heads && y.numel() == t * heads * dv, "state-space shapes");
   TORCH_CHECK(state.dim() == 4 && state.size(1) == heads && state.size(2) == n && state.size(3) == dv, "state");
   check_segs(start, pos0, slot, num_segs);
-  TORCH_CHECK(max_rows <= t && chunk_from >= 1, "state-space rows");
+  TORCH_CHECK(chunk_from >= 1, "state-space rows");
+  max_rows = std::min(max_rows, t);     // (a bound may be given)
   if (max_rows == 1 && mx_state_step_fits(y.data_ptr<float>(), state.data_ptr<float>(), (int)n, (int)dv)) {
     chk(mx_state_step(2, y.data_ptr<float>(), xbc.data_ptr(), bf(xbc), xbc.stride(0), dt.data_ptr(), dt.stride(0), nullptr,
                       0, a_log.data_ptr<float>(), dt_bias.data_ptr<float>(), d_skip.data_ptr<float>(), 0.f,

@@ -174,3 +174,23 @@ def test_channel_sizes_off_quads(dt_, dk, dv, monkeypatch):
     """Key sizes that are no multiple of the loads' four entries, more value tiles than waves."""
     test_channel_delta(dt_, [65, 130], [0, 7], 2, 1, dk, dv, False, monkeypatch)
     test_channel_linear(dt_, [65, 130], [0, 7], 2, dk, dv, True, monkeypatch)
+
+
+@pytest.mark.parametrize("lens", [[1, 1], [5, 2], [300, 4]])
+def test_longest_segment_as_a_bound(lens):
+    """``max_rows`` beyond the step's rows: the same results as with the longest segment itself."""
+    g = torch.Generator().manual_seed(11)
+    heads, dk, dv, T = 2, 32, 32, sum(lens)
+    rnd = lambda *s: (0.3 * torch.randn(*s, generator=g)).to(DEV)      # noqa: E731
+    qkv, a, b, al, bias = rnd(T, 6 * 32), rnd(T, 64), rnd(T, 2), rnd(2), rnd(64)
+    s0, out = rnd(2, heads, dk, dv), []
+    for bound in (max(lens), 4096):
+        seg = segments(lens, [3, 0], [0, 1])
+        seg.max_rows = bound
+        st = [s0.clone() for _ in range(3)]
+        out.append([M.gated_delta_rule(qkv, a, b, al, bias, st[0], seg, heads, heads, dk, dv),
+                    M.gated_linear_attention(qkv, a, bias, 4.0, st[1], seg, heads, dk, dv),
+                    M.ssd_scan(qkv, b, al, al, al, st[2], seg, heads, heads, dk, dv)] + st)
+    for x, y in zip(*out):
+        # walk and chunk form, or step and walk: fp32 sums of a few hundred terms of order 1
+        torch.testing.assert_close(x, y, rtol=1e-5, atol=1e-5)
