@@ -482,8 +482,9 @@ __global__ void ssd_steps_kernel(float* __restrict__ step, float* __restrict__ l
   const long row = e / heads;
   const int h = (int)(e % heads);
   const float v = softplusf_(ld(dt, row * dt_stride + h) + dt_bias[h]);
+  const float l = -expf(a_log[h]) * v;
   step[e] = v;
-  lg[e] = -expf(a_log[h]) * v;
+  lg[e] = l < -3e38f ? -3e38f : l;         // (sums of these are subtracted: -inf would become NaN; the decay is 0)
 }
 
 // The selective state-space scan's long segments: q = C and k = B (one per group of heads), v = x times

@@ -194,3 +194,22 @@ def test_longest_segment_as_a_bound(lens):
     for x, y in zip(*out):
         # walk and chunk form, or step and walk: fp32 sums of a few hundred terms of order 1
         torch.testing.assert_close(x, y, rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("first", [95.0, 60.0])
+def test_state_space_forgets_at_once(first, monkeypatch):
+    """Rates e^a_log up to infinity (e^95 in fp32): decays are 0, a row sees itself alone."""
+    g = torch.Generator().manual_seed(12)
+    heads, n, dv, T = 2, 16, 16, 130
+    seg = segments([T], [5], [0])
+    xbc = torch.randn(T, heads * dv + 2 * n, generator=g).to(DEV)
+    dt, bias, skip = torch.randn(T, heads, generator=g).to(DEV), torch.zeros(heads, device=DEV), torch.ones(heads, device=DEV)
+    a_log, s0 = torch.tensor([first, 0.0], device=DEV), torch.randn(1, heads, n, dv, generator=g).to(DEV)
+    out = []
+    for rows in (64, 1 << 30):
+        monkeypatch.setattr(M, "SSD_CHUNK_ROWS", rows)
+        st = s0.clone()
+        out.append((M.ssd_scan(xbc, dt, a_log, bias, skip, st, seg, heads, 1, n, dv), st))
+    for x, y in zip(*out):
+        assert bool(y.isfinite().all())
+        torch.testing.assert_close(x, y, rtol=1e-5, atol=1e-5)       # fp32 sums of a few hundred terms of order 1
