@@ -110,7 +110,8 @@ latent_prefill_kernel(LatPreArgs A) {
   for (int p = 0; p < 2; ++p)
 #pragma unroll
     for (int t = 0; t < CT; ++t) o[p][t] = lp_f32x4{0.f, 0.f, 0.f, 0.f};
-  float ref[2] = {-INFINITY, -INFINITY}, sum[2] = {0.f, 0.f};
+  // (the reference starts below every score, but finite: scores of -inf, sums that overflow, have weight 0)
+  float ref[2] = {-1e38f, -1e38f}, sum[2] = {0.f, 0.f};
   const float c = A.scale * 1.44269504f;
 
   // page ids, a lane each, of 64 pages from page0 on

@@ -114,3 +114,35 @@ def test_operands_of_other_layouts(form):
     # weights rounded to bf16 twice at most: 2^-8 (a sum and its quotient)
     assert bool(((out.double() - want)[:, rows].abs() <= (2 ** -8 + 2 ** -12) * size[:, rows] + 1e-6).all())
     assert bool((out[:, ~rows] == 0).all())
+
+
+@pytest.mark.parametrize("sink", [False, True])
+def test_scores_that_overflow(sink):
+    """Scores of -inf (products of 1e20 and -1e20) in the first tiles of keys: weight 0, as exp(-inf)."""
+    lens, pos0, t = [130], [0], 130
+    seg, blocks = make_seg(lens, pos0, [0], block_size=8)
+    seg = to_dev(seg)
+    seg.host = (seg.start.tolist(), seg.pos0.tolist(), seg.kv_len.tolist())
+    g = torch.Generator(device=DEV).manual_seed(6)
+    keys = torch.randn(blocks * 8, RANK + DR, generator=g, device=DEV)
+    keys[:70, -1] = -1e20
+    keys[70:, -1] = 0
+    cache = torch.empty_like(keys)
+    cache.view(blocks, 8, -1)[seg.block_tables[0].long()] = keys.view(blocks, 8, -1)
+    cache = cache.view(blocks, 8, -1).bfloat16()
+    qa, qr = torch.randn(1, t, RANK, generator=g, device=DEV), torch.randn(t, 1, DR, generator=g, device=DEV)
+    qr[:, :, -1] = 1e20
+    sinks = torch.ones(1, device=DEV) if sink else None
+    out = torch.full((1, t, RANK), 7.0, device=DEV)
+    M.latent_attention_products(out, qa, qr, cache, seg, 0.05, RANK, 32, torch.bfloat16, sinks)
+    qr[:, :, -1], keys[:70, -1] = 0, 0
+    see = torch.arange(130, device=DEV)
+    q = torch.cat([qa[0], qr[:, 0]], 1).bfloat16().double()
+    k = keys[:130].bfloat16().double()
+    sc = (q @ k.T * 0.05).masked_fill((see[None] > see[:, None]) | (see < 70)[None], float("-inf"))[70:]
+    if sink:
+        sc = torch.cat([sc, torch.ones(60, 1, dtype=sc.dtype, device=DEV)], 1)
+    p = torch.softmax(sc, 1)[:, :130]
+    want, size = p @ k[:, :RANK], p @ k[:, :RANK].abs()
+    # weights rounded to bf16 (half a unit: 2^-8), the rest fp32; rows that see no other score are undefined
+    assert bool(((out[0, 70:].double() - want).abs() <= (2 ** -8 + 2 ** -12) * size + 1e-6).all())
