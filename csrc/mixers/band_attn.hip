@@ -111,17 +111,7 @@ band_attn_kernel(BandArgs A) {
 
   // the queries' parts, as right operands: pair n, elements 32 s + 8 g4 .. + 7
   uint4 qp[3][KS];
-  {
-    const float* src = A.q + ((long)(r0 + row) * hq + a) * DK + 8 * g4;
-#pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      const float4 u = *reinterpret_cast<const float4*>(src + 32 * s), v = *reinterpret_cast<const float4*>(src + 32 * s + 4);
-      split_bf16x3(u.x, u.y, qp[0][s].x, qp[1][s].x, qp[2][s].x);
-      split_bf16x3(u.z, u.w, qp[0][s].y, qp[1][s].y, qp[2][s].y);
-      split_bf16x3(v.x, v.y, qp[0][s].z, qp[1][s].z, qp[2][s].z);
-      split_bf16x3(v.z, v.w, qp[0][s].w, qp[1][s].w, qp[2][s].w);
-    }
-  }
+  split_queries<KS>(A.q + ((long)(r0 + row) * hq + a) * DK + 8 * g4, qp);
   const float c1 = use_terms ? A.r1[a] : 0.f, c2 = use_terms ? A.r2[a] : 0.f;
   const float pbias = A.pb != nullptr ? A.pb[a] : 0.f;
   const float cap = A.softcap, icap = cap > 0.f ? 1.f / cap : 0.f;

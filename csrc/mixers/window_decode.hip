@@ -106,17 +106,7 @@ window_decode_kernel(WindowArgs A) {
 
   // the queries' parts, as right operands: head n, elements 32 x + 8 g4 .. + 7
   uint4 qp[3][KS];
-  {
-    const float* src = A.q + ((long)row * hq + a) * DK + 8 * g4;
-#pragma unroll
-    for (int x = 0; x < KS; ++x) {
-      const float4 u = *reinterpret_cast<const float4*>(src + 32 * x), w = *reinterpret_cast<const float4*>(src + 32 * x + 4);
-      split_bf16x3(u.x, u.y, qp[0][x].x, qp[1][x].x, qp[2][x].x);
-      split_bf16x3(u.z, u.w, qp[0][x].y, qp[1][x].y, qp[2][x].y);
-      split_bf16x3(w.x, w.y, qp[0][x].z, qp[1][x].z, qp[2][x].z);
-      split_bf16x3(w.z, w.w, qp[0][x].w, qp[1][x].w, qp[2][x].w);
-    }
-  }
+  split_queries<KS>(A.q + ((long)row * hq + a) * DK + 8 * g4, qp);
   const float c1 = A.r1 != nullptr ? A.r1[a] : 0.f, c2 = A.r1 != nullptr ? A.r2[a] : 0.f;
   const float bias = A.sigmoid && A.pb != nullptr ? A.pb[a] : 0.f;
   const bool sinks = A.has_sink && !A.sigmoid && wave == 0;

@@ -165,3 +165,23 @@ def test_operands_of_other_layouts(form):
     got = M.window_attention_products(out, q, kc, vc, seg, sp, 32)
     # both forms are within 1e-6 of the sums in 64 bits (test_against_64_bits)
     torch.testing.assert_close(got, want, rtol=0, atol=2e-6 * float(want.abs().max()))
+
+
+@pytest.mark.parametrize("kind", ["cap", "sigmoid", "two maps, cap"])
+@pytest.mark.parametrize("n", [40, 3], ids=["long", "decode"])
+def test_infinite_queries(kind, n):
+    """Queries of +-inf, or that only bf16 rounds to it: scores of +-inf, which a cap and a sigmoid map to finite ones."""
+    g = torch.Generator().manual_seed(8)
+    opt = {"cap": dict(softcap=5.0, blocks=True), "sigmoid": dict(sigmoid=True), "two maps, cap": dict(softcap=5.0, maps=2)}[kind]
+    sp = M.WindowSpec(heads=4, kv_heads=2, dk=64, dv=64, window=100, scale=0.125, **opt)
+    seg, blocks = segments([n, n], [9, 130], 8, g)
+    kc = torch.randn(blocks, 8, 128 * sp.maps, generator=g).to(DEV, torch.bfloat16)
+    vc = torch.randn(blocks, 8, 128, generator=g).to(DEV, torch.bfloat16)
+    q = torch.randn(2 * n, 4 * sp.maps * 64, generator=g).to(DEV)
+    q[0, 5], q[1, 70], q[n + 1, 64 * 4 * sp.maps - 1] = float("inf"), -float("inf"), 3.4e38
+    assert bool((kc != 0).all())
+    out = torch.full((2 * n, 4 * sp.maps, 64), 7.0, device=DEV)
+    want = reference(q, kc, vc, seg, sp, 1)
+    got = M.window_attention_products(out, q, kc, vc, seg, sp, 32) if n >= 32 else M.window_attention(q, kc, vc, seg, sp, out=out)
+    assert bool(want.isfinite().all())
+    assert float((got.double() - want).norm() / want.norm()) < 1e-6       # fp32 sums, as test_against_64_bits
