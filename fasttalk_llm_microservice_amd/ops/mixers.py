@@ -825,6 +825,29 @@ def band_attention_ok(out, q, k_cache, v_cache, seg: Segments, spec: WindowSpec)
                 and native_mixers().band_attention_fits(spec.dk, spec.dv, k_cache.shape[1]))
 
 
+def _band_pays(seg: Segments, sp: WindowSpec, min_rows: int) -> bool:
+    """A workgroup of the one kernel owns 64 (row, query head) pairs and walks their keys, so a few rows behind a long
+    context leave the chip idle, where the products' widened copies and library kernels fill it: 64 rows of 16 heads of
+    128 on 4 key heads at position 8000 take 297 us and the products 138, at 30000 1075 and 562; 32 at 2000 82 and 101, 300
+    at 4000 165 and 235, 2000 from 0 112 and 518.  A key costs the walk 36 ns (plain; 50 to 58 with a cap, a table or
+    sigmoids), 340 walks at a time; the products, whose 25 launches take 100 us to issue, the reads of the cache and the
+    pairs' sums."""
+    start, _, kv_len = seg.host
+    wide, rep = (sp.dk + sp.dv) / 256, sp.heads // sp.kv_heads
+    kind = 33 if sp.sigmoid else 30 if sp.dist_bias is not None else 28 if sp.softcap > 0 else 14
+    a = 4 + 4 * sp.kv_heads * (sp.maps * sp.dk + sp.dv) / 1024
+    b = sp.heads * sp.maps * (0.0053 + 0.0049 * wide)
+    longest = total = products = 0.0
+    for n, kv in zip((y - x for x, y in zip(start[:-1], start[1:])), kv_len):
+        if n < min_rows:
+            continue
+        keys = kv if sp.window <= 0 else min(kv, sp.window + (0 if sp.blocks else n))
+        longest = max(longest, keys)
+        total += keys * sp.kv_heads * sp.maps * (-(-n * rep // 64))
+        products += max(100.0, 20 + 1e-3 * keys * (a + b * n) * (0.8 if sp.sigmoid else 1.0))
+    return 10 + 1e-3 * (kind + 22 * wide) * max(longest, total / 340) <= products
+
+
 def window_attention_products(out, q, k_cache, v_cache, seg: Segments, spec: WindowSpec, min_rows: int):
     """Segments of ``min_rows`` rows or more as banded matrix products: a chunk of rows
     [c0, c1) only sees the keys c0 - window + 1 .. c1 - 1 (or from the start of c0's block;
@@ -833,12 +856,12 @@ def window_attention_products(out, q, k_cache, v_cache, seg: Segments, spec: Win
     from :func:`band_weights` (fp32) and the sums are a second product with the value
     head.  Operands are fp32 (cached rows are widened), so scores, weights and sums are
     true fp32.  bf16 caches whose heads fit its tiles run in one kernel for all segments instead
-    (csrc/mixers/band_attn.hip), to the same exactness.  Needs the segments' host copies; writes
-    its rows of ``out``."""
+    (:func:`band_attention_ok`), to the same exactness, unless a few rows see a long context
+    (:func:`_band_pays`).  Needs the segments' host copies; writes its rows of ``out``."""
     sp = spec
     start, pos0, kv_len = seg.host
     bs = k_cache.shape[1]
-    if band_attention_ok(out, q, k_cache, v_cache, seg, sp):
+    if band_attention_ok(out, q, k_cache, v_cache, seg, sp) and _band_pays(seg, sp, min_rows):
         # one kernel for all segments, scores never in memory
         ns = [n for n in (b - a for a, b in zip(start[:-1], start[1:])) if n >= min_rows]
         native_mixers().band_attention(out, q, k_cache, v_cache, seg.start, seg.pos0, seg.kv_len, seg.block_tables,

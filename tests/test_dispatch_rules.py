@@ -1,0 +1,38 @@
+"""Rules that choose between two forms of an operation, at sizes where both were timed (us on one MI355X, issued one
+after the other from Python): the form chosen takes at most 1.15 times the other's time."""
+import pytest
+
+from fasttalk_llm_microservice_amd.ops import mixers as M
+
+
+def segments(rows, count, pos):
+    start = [i * rows for i in range(count + 1)]
+    return M.Segments(None, None, None, None, None, count, rows, pos + rows, host=(start, [pos] * count, [pos + rows] * count))
+
+
+CAUSAL = dict(heads=16, kv_heads=4, dk=128, dv=128, window=0)
+SPECS = {
+    "plain": CAUSAL, "cap": dict(CAUSAL, softcap=30.0), "table": dict(CAUSAL, dist_bias=True),
+    "sigmoid": dict(CAUSAL, sigmoid=True), "narrow": dict(heads=8, kv_heads=8, dk=64, dv=64, window=0),
+    "window": dict(CAUSAL, window=1024), "two maps": dict(CAUSAL, dk=64, window=1024, maps=2),
+    "wide blocks": dict(heads=16, kv_heads=16, dk=128, dv=128, window=4096, blocks=True),
+}
+
+
+@pytest.mark.parametrize("spec,rows,count,pos,one,products", [
+    ("plain", 32, 1, 0, 11, 99), ("plain", 32, 1, 2000, 82, 101), ("plain", 64, 1, 8000, 297, 138),
+    ("plain", 64, 1, 30000, 1074, 562), ("plain", 300, 1, 4000, 165, 235), ("plain", 300, 1, 30000, 1090, 1930),
+    ("plain", 1000, 1, 30000, 1121, 5143), ("plain", 2000, 1, 0, 112, 518), ("plain", 40, 8, 700, 37, 768),
+    ("plain", 32, 4, 15000, 545, 776), ("plain", 33, 1, 120000, 4219, 1580),
+    ("cap", 64, 1, 8000, 409, 138), ("cap", 300, 1, 4000, 227, 240), ("cap", 32, 4, 15000, 759, 790),
+    ("table", 32, 1, 2000, 120, 104), ("table", 64, 1, 30000, 1555, 589), ("table", 1000, 1, 30000, 1592, 5763),
+    ("sigmoid", 32, 1, 2000, 117, 103), ("sigmoid", 64, 1, 30000, 1619, 477), ("sigmoid", 32, 4, 15000, 817, 648),
+    ("sigmoid", 1000, 1, 30000, 1682, 3701), ("sigmoid", 300, 1, 0, 25, 103),
+    ("narrow", 64, 1, 8000, 208, 124), ("narrow", 300, 1, 4000, 117, 165), ("narrow", 64, 1, 30000, 749, 340),
+    ("narrow", 1000, 1, 30000, 776, 2111), ("window", 64, 1, 8000, 48, 100), ("window", 300, 1, 4000, 49, 136),
+    ("two maps", 64, 1, 8000, 42, 107), ("wide blocks", 64, 1, 8000, 152, 99), ("wide blocks", 300, 1, 4000, 158, 255),
+    ("wide blocks", 2000, 1, 0, 117, 436)])
+def test_long_windowed_segments(spec, rows, count, pos, one, products):
+    sp = M.WindowSpec(scale=1.0, **SPECS[spec])
+    taken = one if M._band_pays(segments(rows, count, pos), sp, 32) else products
+    assert taken <= 1.15 * min(one, products)
