@@ -100,16 +100,41 @@ def _few_rows(x, w) -> bool:
                 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and w.is_contiguous())
 
 
-def _few_rows_pays(rows: int, n: int, k: int) -> bool:
-    """Where the few-rows kernel is at least level with the vendor's product (timings beside its
-    configurations in few_rows.hip): always up to 16 rows; above, long sums into few columns have
-    too few workgroups to hide reading X, and many rows against a middling number of columns
-    fill the vendor's tiles."""
-    if rows <= 16:
-        return True
-    if rows <= 32:
-        return k < 8192 or n > 4096
-    return n >= 16384 or (n <= 4096 and k <= 4096)
+def _few_rows_pays(rows: int, n: int, k: int, act: Optional[str] = None) -> bool:
+    """Where the few-rows kernel is at least level with the vendor's product and, with ``act``, the activation's kernel
+    (``n`` rows of w: a gated form's two matrices).  Its waves take long sums in a chain and share one read of X per
+    workgroup, so it loses with k, the sooner the more rows there are; most columns below 16384 go to workgroups of four
+    waves, whose chains are twice as long.  us at 1 / 16 / 32 / 64 rows, the vendor's beside it (weights from HBM):
+      n = 2048, k = 4096      8 9 11 14 (15 15 12 14)        k = 12288   19 21 28 39 (19 19 24 34)
+      n = 5120, k = 2048      10 10 11 18 (12 12 12 13)      k = 13824   48 47 57 88 (30 32 37 48)
+      n = 14336, k = 4096     24 28 38 33 (29 29 26 27)      n = 32768, k = 2048   28 28 28 33 (34 34 34 35)
+      gated, 2 x 1024, k = 2048   8 8 9 12 (11 12 12 13)     2 x 2048, k = 8192   32 32 36 38 (20 20 22 28)"""
+    if act == "relu_sq":
+        if n >= 16384:
+            longest = 6144
+        elif n > 4096:
+            longest = 4096 if rows <= 16 else 2048 if rows <= 32 else 1024
+        else:
+            longest = 8192 if rows <= 16 else 6144 if rows <= 32 else 4096
+    elif act is not None:
+        if rows <= 16:
+            longest = 6144 if n >= 8192 else 4096
+        elif n < 512 or (rows <= 32 and n >= 16384):
+            longest = 4096
+        else:
+            longest = 3072 if (8192 if rows <= 32 else 5120) <= n < 16384 else 2048
+    elif n >= 32768:
+        longest = 8192 if rows <= 32 else 6144 if rows <= 48 else 2048
+    elif n > 4096:
+        if rows <= 16:
+            longest = 6144 if n >= 16384 else 4096 if n >= 10240 else 3072 if n >= 8192 else 2048
+        else:
+            longest = 2048 if rows <= 32 and not 12288 < n < 16384 else 0
+    elif rows <= 16:
+        longest = max(4096, min(8192, 2 * n))
+    else:
+        longest = 4096 if rows <= 32 or n >= 512 else 1024
+    return k <= longest
 
 
 def linear(x, w, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -132,9 +157,9 @@ def linear_f32(x, w) -> torch.Tensor:
 
 def linear_act(x, w, act: str, limit: float = 0.0) -> torch.Tensor:
     """act of x w^T: w = [gate | up] rows for the gated forms ("gelu_tanh", "relu", "silu",
-    "clamp_glu" with ``limit``), one matrix for "relu_sq".  Few rows: one kernel, the products
-    stay fp32 up to the activation's result."""
-    if _few_rows(x, w):
+    "clamp_glu" with ``limit``), one matrix for "relu_sq".  Where the few-rows kernel pays, one
+    kernel, the products stay fp32 up to the activation's result."""
+    if _few_rows(x, w) and _few_rows_pays(x.shape[0], w.shape[0], x.shape[1], act):
         n = w.shape[0] if act == "relu_sq" else w.shape[0] // 2
         y = torch.empty(x.shape[0], n, dtype=x.dtype, device=x.device)
         native_mixers().few_rows_gemm(y, x, w, None, FEW_ACTS[act], float(limit))

@@ -36,3 +36,19 @@ def test_long_windowed_segments(spec, rows, count, pos, one, products):
     sp = M.WindowSpec(scale=1.0, **SPECS[spec])
     taken = one if M._band_pays(segments(rows, count, pos), sp, 32) else products
     assert taken <= 1.15 * min(one, products)
+
+
+@pytest.mark.parametrize("act,n,k,rows,few,vendor", [
+    (None, 2048, 2048, 1, 5.4, 11.1), (None, 2048, 2048, 64, 8.8, 11.7), (None, 2048, 8192, 48, 21.8, 15.1),
+    (None, 5120, 13824, 1, 47.7, 29.7), (None, 5120, 13824, 32, 56.8, 36.8), (None, 13824, 5120, 16, 42.9, 27.7),
+    (None, 14336, 4096, 1, 24.0, 29.0), (None, 14336, 4096, 32, 37.6, 26.2), (None, 8192, 2048, 16, 10.3, 13.3),
+    (None, 6144, 2048, 64, 18.6, 13.1), (None, 32768, 2048, 32, 27.7, 34.1), (None, 256, 2048, 64, 6.7, 5.3),
+    (None, 512, 16384, 64, 45.4, 19.1), (None, 20480, 5120, 17, 58.7, 42.1), ("silu", 16384, 2048, 16, 14.9, 21.1),
+    ("silu", 4096, 8192, 1, 31.7, 19.6), ("silu", 4096, 8192, 64, 37.7, 28.2), ("silu", 28672, 4096, 64, 68.3, 54.2),
+    ("silu", 28672, 4096, 16, 49.4, 63.0), ("clamp_glu", 2048, 2048, 64, 13.0, 14.6),
+    ("relu_sq", 8192, 2048, 64, 19.1, 16.2), ("relu_sq", 8192, 2048, 32, 11.8, 15.4),
+    ("relu_sq", 14336, 4096, 32, 38.1, 27.7), ("relu_sq", 2048, 8192, 48, 21.7, 17.5),
+    ("relu_sq", 2048, 8192, 1, 11.7, 15.1)])
+def test_products_of_few_rows(act, n, k, rows, few, vendor):
+    taken = few if M._few_rows_pays(rows, n, k, act) else vendor
+    assert taken <= 1.15 * min(few, vendor)
