@@ -863,7 +863,8 @@ class MoEFF:
 
     def __call__(self, h, ctx=None) -> torch.Tensor:
         t, width = h.shape
-        if t <= self.PAIR_ROWS and M.experts_few_ok(h, self.wgu, self.wdown, self.shared):
+        if t <= self.PAIR_ROWS and M.experts_few_ok(h, self.wgu, self.wdown, self.shared) and \
+                M.experts_few_pays(t * self.top, self.e, self.wdown[0].numel(), self.shared is not None):
             # decode-size steps: a matrix is read once for all rows, nothing read back on the host
             idx, wts = self.route(h)
             return M.experts_few(h, idx, wts, self.wgu, self.wdown, self.act, self.limit, self.shared,
@@ -884,7 +885,7 @@ class MoEFF:
             out = torch.zeros(t, width, dtype=torch.float32, device=h.device)
         idx, wts = self.route(h)
         if t <= self.PAIR_ROWS:
-            # fp32 (or rows that are not whole 16-byte pieces): per-pair weight streaming
+            # few pairs, fp32, or rows that are not whole 16-byte pieces: per-pair weight streaming
             M.moe_pairs(out, h, idx, wts, self.wgu, self.wdown, self.limit, self.act)
             return self._shared(out, h)
         # rows sorted by expert: each expert's rows are one group of two grouped products

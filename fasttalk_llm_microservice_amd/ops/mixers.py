@@ -1213,6 +1213,17 @@ def experts_few_ok(h, wgu, wdown, shared) -> bool:
                                           and w.is_contiguous() for w in ws))
 
 
+def experts_few_pays(pairs: int, experts: int, size: int, shared: bool) -> bool:
+    """Where :func:`experts_few` beats a read of the matrices per (row, choice) pair (:func:`moe_pairs`): once enough pairs
+    share an expert to make up for a launch over all experts.  us of the layer, matrices from HBM (per pair in brackets):
+    32 experts, top 4, relu^2 of 1536 x 2048: 32 40 57 63 71 at 1 2 4 6 8 rows (25 31 46 61 71), 93 at 32 (214); 8 of
+    4096 x 4096, top 2: 50 84 93 127 at 1 2 3 4 (40 77 97 137); 64 of 1408 x 4096, top 8: 110 151 169 185 (84 127 164 197);
+    128 of 768 x 2048, top 8: 56 87 124 at 1 4 8 (45 74 124); matrices (``size`` entries) of a few hundred KB are all
+    launches: 4 of 512 x 512, 14 at 1 to 24 rows (11 to 15).  A shared expert rides in the same launches: level at one
+    row, 0.9 of the time from 4."""
+    return shared or pairs >= max(min(0.75 * experts, 16 + 0.375 * experts), 24 if size < 1 << 20 else 0)
+
+
 def experts_few(h, idx, wts, wgu, wdown, act: str, limit: float = 0.0, shared=None, shared_limit: float = 0.0,
                 shared_gate: bool = False) -> torch.Tensor:
     """fp32 sum_k wts[:, k] * expert_{idx[:, k]}(h) (+ the shared expert, times the sigmoid of its

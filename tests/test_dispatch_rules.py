@@ -52,3 +52,16 @@ def test_long_windowed_segments(spec, rows, count, pos, one, products):
 def test_products_of_few_rows(act, n, k, rows, few, vendor):
     taken = few if M._few_rows_pays(rows, n, k, act) else vendor
     assert taken <= 1.15 * min(few, vendor)
+
+
+@pytest.mark.parametrize("experts,top,ff,width,shared,rows,few,pairs", [
+    (32, 4, 1536, 2048, False, 1, 32.0, 24.9), (32, 4, 1536, 2048, False, 4, 56.8, 46.2), (32, 4, 1536, 2048, False, 8, 70.8, 70.6),
+    (32, 4, 1536, 2048, False, 32, 92.8, 214.0), (32, 4, 1536, 2048, True, 1, 43.7, 41.7), (32, 6, 1024, 2048, True, 2, 62.0, 67.5),
+    (128, 8, 768, 2048, False, 4, 86.5, 74.4), (128, 8, 768, 2048, False, 16, 163.4, 204.5), (8, 2, 4096, 4096, False, 1, 50.0, 40.2),
+    (8, 2, 4096, 4096, False, 6, 136.7, 183.8), (8, 2, 14336, 4096, False, 1, 158.0, 138.2), (8, 2, 14336, 4096, False, 4, 436.5, 462.7),
+    (256, 8, 256, 1024, False, 8, 52.4, 46.5), (256, 8, 256, 1024, False, 48, 112.7, 137.3), (16, 2, 2048, 6144, False, 4, 126.5, 111.6),
+    (16, 2, 2048, 6144, False, 16, 214.4, 356.3), (64, 8, 1408, 4096, False, 1, 110.2, 83.9), (64, 8, 1408, 4096, False, 8, 271.9, 344.8),
+    (4, 1, 512, 512, False, 8, 14.1, 11.4), (4, 1, 512, 512, False, 64, 15.6, 22.5)])
+def test_experts_of_few_rows(experts, top, ff, width, shared, rows, few, pairs):
+    taken = few if M.experts_few_pays(rows * top, experts, ff * width, shared) else pairs
+    assert taken <= 1.15 * min(few, pairs)
