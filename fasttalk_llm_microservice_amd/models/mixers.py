@@ -844,7 +844,7 @@ class MoEFF:
             return M.moe_route(h, self.router_parts, self.correction if grouped else self.router_bias, self.e, self.top,
                                self.routing, 1.0 if grouped else self.route_scale,
                                self.groups if limited else 1, self.keep if limited else 1)
-        if grouped and few:
+        if grouped and few and M.moe_route_softmax_pays(self.e):
             return M.moe_route_softmax(h, self.router, self.correction, self.top, self.groups, self.keep)
         if grouped:
             z = F.linear(h.float(), self.router)

@@ -1155,6 +1155,12 @@ def moe_route_softmax(h, router, correction, top: int, groups: int, keep: int):
     return ref.moe_topk(torch.nn.functional.linear(h.float(), router), correction, top, groups, keep)
 
 
+def moe_route_softmax_pays(experts: int) -> bool:
+    """Where :func:`moe_route_softmax`, a workgroup per row that takes the experts sixteen at a time, beats a library
+    product and :func:`moe_topk`: 32 experts 10 us (17 for 64 rows of 2048), 64 15 (18), 128 25 (20)."""
+    return experts <= 64
+
+
 ROUTE_MODES = {"top_logits": 0, "top_sigmoid": 1, "grouped_softmax": 2}
 
 

@@ -65,3 +65,8 @@ def test_products_of_few_rows(act, n, k, rows, few, vendor):
 def test_experts_of_few_rows(experts, top, ff, width, shared, rows, few, pairs):
     taken = few if M.experts_few_pays(rows * top, experts, ff * width, shared) else pairs
     assert taken <= 1.15 * min(few, pairs)
+
+
+@pytest.mark.parametrize("experts,one,two", [(16, 6.3, 14.7), (32, 10.3, 16.7), (64, 15.4, 17.5), (128, 25.2, 20.4)])
+def test_grouped_softmax_router(experts, one, two):
+    assert (one if M.moe_route_softmax_pays(experts) else two) == min(one, two)

@@ -46,3 +46,17 @@ def test_ties_go_to_the_lower_index():
     router[7] = 1.0
     idx, wts = M.moe_route(h, M.route_parts(router), None, 40, 5, "top_logits")
     assert idx.tolist() == [[7, 0, 1, 2, 3]] * 3 and bool((wts[:, 0] > 0.99).all())
+
+
+def test_layer_of_many_experts_in_a_decode_step():
+    """More experts than one workgroup's rows pay for: the library product and the choice kernel, with the same choice."""
+    from fasttalk_llm_microservice_amd.models.mixers import MoEFF
+    g = torch.Generator().manual_seed(2)
+    sizes = {"router": (96, 128), "correction": (96,)}
+    size = lambda n: sizes.get(n, (128, 32) if n.endswith("down") else (32, 128))      # noqa: E731
+    moe = MoEFF(lambda n: rnd(*size(n), g=g, scale=0.1), 96, 4, 7.0, 8, 4, None, torch.bfloat16, DEV)
+    h = rnd(5, 128, dt=torch.bfloat16, g=g).to(DEV)
+    idx, wts = moe.route(h)
+    i2, w2 = M.moe_route_softmax(h, moe.router, moe.correction, 4, 8, 4)
+    assert torch.equal(idx, i2)
+    torch.testing.assert_close(wts, w2, rtol=1e-5, atol=1e-7)     # fp32 logits of 128 terms in another order
