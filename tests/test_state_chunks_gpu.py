@@ -213,3 +213,25 @@ def test_state_space_forgets_at_once(first, monkeypatch):
     for x, y in zip(*out):
         assert bool(y.isfinite().all())
         torch.testing.assert_close(x, y, rtol=1e-5, atol=1e-5)       # fp32 sums of a few hundred terms of order 1
+
+
+@pytest.mark.parametrize("dt_", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("heads,kvh,dk", [(16, 16, 66), (18, 6, 128), (4, 2, 256), (8, 8, 64)])
+def test_delta_preparation_of_many_rows(dt_, heads, kvh, dk):
+    """Enough rows for the preparation that takes four rows a wave (but for channels of 64), a part-filled item at the
+    end: the results of the segments alone, whose rows are prepared one by one."""
+    g = torch.Generator().manual_seed(dk)
+    count = 12288 // (heads + kvh) // 81 + 1
+    T, dv = 81 * count, 16
+    rnd = lambda *s: torch.randn(*s, generator=g).to(DEV, dt_)      # noqa: E731
+    qkv, a, b = rnd(T, 2 * kvh * dk + heads * dv), rnd(T, heads * dk + 2)[:, 2:], rnd(T, heads)
+    al, bias = torch.rand(heads, generator=g).to(DEV), torch.randn(heads * dk, generator=g).to(DEV)
+    s0 = torch.randn(count, heads, dk, dv, generator=g).to(DEV)
+    st = s0.clone()
+    o = M.gated_delta_rule(qkv, a, b, al, bias, st, segments([81] * count, [3] * count, list(range(count))), heads, kvh, dk, dv)
+    for i in range(count):
+        r, si = slice(81 * i, 81 * i + 81), s0[i:i + 1].clone()
+        alone = M.gated_delta_rule(qkv[r], a[r], b[r], al, bias, si, segments([81], [3], [0]), heads, kvh, dk, dv)
+        # sums of dk squares in another order: a few units of 2^-23 of numbers of order 1 to 10, carried over 81 rows
+        torch.testing.assert_close(o[r], alone, rtol=1e-4, atol=1e-4)
+        torch.testing.assert_close(st[i:i + 1], si, rtol=1e-4, atol=1e-4)
