@@ -379,9 +379,9 @@ def gated_delta_rule(qkv, a, b, a_log, dt_bias, state, seg: Segments, heads: int
     and left at the segment's last row.  Returns o fp32 [T, heads*dv]."""
     if qkv.is_cuda:
         o = torch.empty(qkv.shape[0], heads * dv, dtype=torch.float32, device=qkv.device)
+        chunk = CHANNEL_CHUNK_ROWS if _delta_chunks_pay(seg, heads, dk, dv) else NO_CHUNKS
         native_mixers().gated_delta_rule(o, qkv, a, b, a_log, dt_bias, state, seg.start, seg.pos0, seg.slot, seg.num,
-                                         seg.max_rows, heads, kv_heads, dk, dv, _walk_below(seg, CHANNEL_CHUNK_ROWS),
-                                         CHANNEL_CHUNK_ROWS)
+                                         seg.max_rows, heads, kv_heads, dk, dv, _walk_below(seg, chunk), chunk)
         return o
     return ref.gated_delta_rule(qkv, a, b, a_log, dt_bias, state, seg, heads, kv_heads, dk, dv)
 
@@ -416,6 +416,38 @@ CHUNK_ROWS = 32
 # 245), state space 40 41 46 98 (19 28 49 169; four segments of 200: 108, walk 97)
 CHANNEL_CHUNK_ROWS = 96
 SSD_CHUNK_ROWS = 256
+NO_CHUNKS = 1 << 30
+
+
+def _chunk_counts(seg: Segments, rows: int):
+    """(chunks of 64 rows, rows) of the segments of at least ``rows`` rows."""
+    lens = [b - a for a, b in zip(seg.host[0][:-1], seg.host[0][1:]) if b - a >= rows]
+    return sum((n + 63) // 64 for n in lens), sum(lens)
+
+
+def _delta_chunks_pay(seg: Segments, heads: int, dk: int, dv: int) -> bool:
+    """Many segments of narrow heads fill the chip with walks, whose work per row is the smaller one then.  us, chunks
+    (walks): 32 heads of 64 x 64, 16 and 64 segments of 100 rows 124 489 (113 403), 32 of 256 472 (497); of 16 x 32 79 264
+    (51 130), 266 (168); 16 heads of 128 x 128 135 554 (261 1057).  A row costs a walk r us, `slots` walks of 32 columns at
+    a time; a head's chunk c us of the chip."""
+    if seg.host is None or seg.max_rows < CHANNEL_CHUNK_ROWS:
+        return True
+    chunks, rows = _chunk_counts(seg, CHANNEL_CHUNK_ROWS)
+    r, slots, c = 0.2 + 0.0026 * dk, 480 - 1.75 * dk, 0.05 + 0.0005 * dk + 8.5e-6 * dk * dk
+    walked = rows * heads * ((dv + 31) // 32) / slots
+    return walked <= seg.max_rows or r * walked >= c * chunks * heads
+
+
+def _ssd_chunks_pay(seg: Segments, heads: int, n: int, dv: int) -> bool:
+    """The same of the state-space scan, with walks of 16 columns and both forms' whole times, the chunk form's a tenth
+    up: 16 heads of 128 x 128, 32 segments of 256 rows 420 (388), four of 2000 370 (459), of 128 x 256, 4 heads, eight of
+    300 95 (78); 32 of 64 x 64 82 (74), 32 of 256 193 (201); of 16 x 32 99 (87)."""
+    if seg.host is None or seg.max_rows < SSD_CHUNK_ROWS:
+        return True
+    chunks, rows = _chunk_counts(seg, SSD_CHUNK_ROWS)
+    walked = rows * heads * ((dv + 15) // 16) / (900 - 2.6 * n)
+    chunked = (0.012 + 0.0006 * n) * ((dv + 63) // 64) * chunks * heads
+    return 1.1 * (12 + chunked) <= 12 + (0.127 + 0.00065 * n) * max(seg.max_rows, walked)
 
 
 def head_delta_rule(q, k, v, log_decay, beta, state, seg: Segments) -> torch.Tensor:
@@ -669,8 +701,9 @@ def ssd_scan(xbc, dt, a_log, dt_bias, d_skip, state, seg: Segments, heads: int, 
     position 0) and left at the segment's last row.  Returns y fp32 [T, heads*dv]."""
     if xbc.is_cuda:
         y = torch.empty(xbc.shape[0], heads * dv, dtype=torch.float32, device=xbc.device)
+        chunk = SSD_CHUNK_ROWS if _ssd_chunks_pay(seg, heads, n, dv) else NO_CHUNKS
         native_mixers().ssd_scan(y, xbc, dt, a_log, dt_bias, d_skip, state, seg.start, seg.pos0, seg.slot,
-                                 seg.num, seg.max_rows, heads, groups, n, dv, _walk_below(seg, SSD_CHUNK_ROWS), SSD_CHUNK_ROWS)
+                                 seg.num, seg.max_rows, heads, groups, n, dv, _walk_below(seg, chunk), chunk)
         return y
     return ref.ssd_scan(xbc, dt, a_log, dt_bias, d_skip, state, seg, heads, groups, n, dv)
 

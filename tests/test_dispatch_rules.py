@@ -70,3 +70,30 @@ def test_experts_of_few_rows(experts, top, ff, width, shared, rows, few, pairs):
 @pytest.mark.parametrize("experts,one,two", [(16, 6.3, 14.7), (32, 10.3, 16.7), (64, 15.4, 17.5), (128, 25.2, 20.4)])
 def test_grouped_softmax_router(experts, one, two):
     assert (one if M.moe_route_softmax_pays(experts) else two) == min(one, two)
+
+
+def unlike(lens):
+    start = [0]
+    for n in lens:
+        start.append(start[-1] + n)
+    return M.Segments(None, None, None, None, None, len(lens), max(lens), host=(start, [5] * len(lens), [n + 5 for n in lens]))
+
+
+@pytest.mark.parametrize("heads,dk,dv,lens,chunks,walks", [
+    (16, 128, 128, [100] * 64, 554, 1057), (16, 128, 128, [96], 51, 61), (32, 64, 64, [100] * 16, 124, 113),
+    (32, 64, 64, [100] * 64, 489, 403), (32, 64, 64, [256] * 32, 472, 497), (32, 64, 64, [2000] * 4, 471, 793),
+    (4, 128, 256, [100] * 64, 212, 487), (32, 16, 32, [100] * 64, 264, 130), (32, 16, 32, [256] * 32, 266, 168),
+    (32, 16, 32, [777], 55, 181), (32, 16, 32, [2000] * 4, 277, 542), (32, 64, 64, [1] * 64 + [4000], 475, 1455)])
+def test_delta_rule_of_long_segments(heads, dk, dv, lens, chunks, walks):
+    taken = chunks if M._delta_chunks_pay(unlike(lens), heads, dk, dv) else walks
+    assert taken <= 1.1 * min(chunks, walks)
+
+
+@pytest.mark.parametrize("heads,n,dv,lens,chunks,walks", [
+    (16, 128, 128, [256] * 32, 420, 388), (16, 128, 128, [777], 59, 170), (16, 128, 128, [2000] * 4, 371, 459),
+    (16, 128, 128, [256] * 4, 64, 67), (32, 64, 64, [300] * 8, 82, 74), (32, 64, 64, [256] * 32, 193, 201),
+    (4, 128, 256, [300] * 8, 95, 78), (4, 128, 256, [2000] * 4, 183, 425), (32, 16, 32, [256] * 32, 99, 87),
+    (32, 16, 32, [300] * 8, 44, 49), (16, 128, 128, [1] * 32 + [400], 103, 125), (32, 16, 32, [4096], 77, 564)])
+def test_state_space_scan_of_long_segments(heads, n, dv, lens, chunks, walks):
+    taken = chunks if M._ssd_chunks_pay(unlike(lens), heads, n, dv) else walks
+    assert taken <= 1.1 * min(chunks, walks)
