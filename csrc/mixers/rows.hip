@@ -263,7 +263,7 @@ __device__ __forceinline__ float sum_sq(const float (&v)[C][4]) {
   return s;
 }
 
-// layer_norm_kernel, add_scaled_rms_norm_kernel and dual_rms_mean_kernel for rows of up to kRowMaxWidth: the row in
+// layer_norm_kernel, add_scaled_rms_norm_kernel and dual_rms_mean_kernel for rows that row_in_registers() takes: the row in
 // registers, all its loads in flight at once and no value read twice.  Bound by that one latency and the
 // reductions for few rows, by the rows' bytes for many.  Width 2048: layer norm of 32 rows 4.7 us, of 2000 12
 // (values read entry by entry, again for each pass: 10 and 16); scaled add and norm of 777 rows 6 (10); mean of two norms
@@ -722,13 +722,22 @@ static void row_chunks(int width, F f) {
   else f(std::integral_constant<int, 8>{});
 }
 
+// whether these rows go to the kernels that hold a row in registers (layer norm, scaled add, mean of two norms), 512 threads a
+// row.  Below 1024 entries most of those have nothing to do, which many rows feel: layer norm of 2000 rows of 256, 1024 and
+// 2048 6.6 6.9 7.4 us (entry by entry 4.1 5.4 7.6), of 64 rows 3.1 3.1 3.1 (2.8 3.7 4.8).  Rows that are no whole fours are
+// loaded entry by entry here, too, four neighbours a thread: 2050 entries, 64 rows 4.3 (5.1), 300 5.9 (5.5), 2000 15.6 (7.9).
+static bool row_in_registers(int rows, int width, int vec) {
+  if (width > kRowMaxWidth) return false;
+  return vec ? width > 1024 || (width > 512 && rows <= 512) : width > 1024 && rows <= 64;
+}
+
 template <typename TY, typename TO>
 static void launch_layer_norm(float* x, const void* y, long ys, const float* w, const float* b, void* out,
                               void* cast, int rows, int width, float eps, hipStream_t s) {
-  if (width <= kRowMaxWidth) {
-    const int vec = width % 4 == 0 && (y == nullptr || (ys % 4 == 0 && ((uintptr_t)y) % (4 * sizeof(TY)) == 0)) &&
-                    ((uintptr_t)x | (uintptr_t)w | (uintptr_t)b) % 16 == 0 &&
-                    ((uintptr_t)out | (uintptr_t)cast) % (4 * sizeof(TO)) == 0;
+  const int vec = width % 4 == 0 && (y == nullptr || (ys % 4 == 0 && ((uintptr_t)y) % (4 * sizeof(TY)) == 0)) &&
+                  ((uintptr_t)x | (uintptr_t)w | (uintptr_t)b) % 16 == 0 &&
+                  ((uintptr_t)out | (uintptr_t)cast) % (4 * sizeof(TO)) == 0;
+  if (row_in_registers(rows, width, vec)) {
     row_chunks(width, [&](auto c) {
       hipLaunchKernelGGL((layer_norm_row_kernel<TY, TO, kRowThreads, decltype(c)::value>), dim3(rows), dim3(kRowThreads),
                          0, s, x, (const TY*)y, ys, w, b, (TO*)out, (TO*)cast, width, eps, vec);
@@ -916,12 +925,12 @@ extern "C" int mx_add_scaled_rms_norm(float* x, const void* y1, int y1_bf16, lon
                                       int out_bf16, int rows, int width, float eps, hipStream_t s) {
   if (rows <= 0) return 0;
   if (y1 == nullptr && (y2 != nullptr || out == nullptr)) return -1;
-  if (width <= kRowMaxWidth) {
-    auto fits = [](const void* y, int bf16, long stride) {
-      return y == nullptr || (stride % 4 == 0 && ((uintptr_t)y) % (bf16 ? 8 : 16) == 0);
-    };
-    const int vec = width % 4 == 0 && fits(y1, y1_bf16, y1_stride) && fits(y2, y2_bf16, y2_stride) &&
-                    ((uintptr_t)x | (uintptr_t)next_w) % 16 == 0 && ((uintptr_t)out) % (out_bf16 ? 8 : 16) == 0;
+  auto fits = [](const void* y, int bf16, long stride) {
+    return y == nullptr || (stride % 4 == 0 && ((uintptr_t)y) % (bf16 ? 8 : 16) == 0);
+  };
+  const int vec = width % 4 == 0 && fits(y1, y1_bf16, y1_stride) && fits(y2, y2_bf16, y2_stride) &&
+                  ((uintptr_t)x | (uintptr_t)next_w) % 16 == 0 && ((uintptr_t)out) % (out_bf16 ? 8 : 16) == 0;
+  if (row_in_registers(rows, width, vec)) {
     row_chunks(width, [&](auto c) {
       if (out_bf16)
         hipLaunchKernelGGL((add_scaled_rms_norm_row_kernel<bf16_t, kRowThreads, decltype(c)::value>), dim3(rows),
@@ -947,10 +956,10 @@ extern "C" int mx_dual_rms_mean(float* out, const void* a, long a_stride, const 
                                 const float* wa, const float* wb, int rows, int width, float eps, float scale,
                                 hipStream_t s) {
   if (rows <= 0) return 0;
-  if (width <= kRowMaxWidth) {
-    const int vec = width % 4 == 0 && a_stride % 4 == 0 && b_stride % 4 == 0 &&
-                    ((uintptr_t)a | (uintptr_t)b) % (bf16 ? 8 : 16) == 0 &&
-                    ((uintptr_t)out | (uintptr_t)wa | (uintptr_t)wb) % 16 == 0;
+  const int vec = width % 4 == 0 && a_stride % 4 == 0 && b_stride % 4 == 0 &&
+                  ((uintptr_t)a | (uintptr_t)b) % (bf16 ? 8 : 16) == 0 &&
+                  ((uintptr_t)out | (uintptr_t)wa | (uintptr_t)wb) % 16 == 0;
+  if (row_in_registers(rows, width, vec)) {
     row_chunks(width, [&](auto c) {
       MX_DISPATCH_T(bf16, hipLaunchKernelGGL((dual_rms_mean_row_kernel<T, kRowThreads, decltype(c)::value>), dim3(rows),
                                              dim3(kRowThreads), 0, s, out, (const T*)a, a_stride, (const T*)b, b_stride,

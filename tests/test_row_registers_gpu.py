@@ -65,3 +65,26 @@ def test_attn_prep(dt, norm, rot, hd, nqh, nkh):
     torch.testing.assert_close(q2.cpu(), q1, rtol=2e-5, atol=2e-5)
     torch.testing.assert_close(kc2.cpu().float(), kc1.float(), **tol(dt))
     torch.testing.assert_close(vc2.cpu().float(), vc1.float(), **tol(dt))
+
+
+@pytest.mark.parametrize("rows,width,left", [(600, 512, 4), (600, 516, 4), (512, 516, 4), (513, 1024, 4), (600, 1028, 4), (64, 2050, 4),
+                                             (65, 2050, 4), (64, 1023, 4), (600, 2052, 3)])
+def test_norms_by_rows(rows, width, left):
+    """Both sides of the rule on rows, widths and addresses."""
+    g = torch.Generator().manual_seed(rows + width)
+    dt = torch.bfloat16
+    wide = lambda: rnd(rows, width + left, dt=dt, g=g)[:, left:]            # noqa: E731
+    w, b, x = 1 + rnd(width, g=g, scale=0.2), rnd(width, g=g), rnd(rows, width, g=g)
+    close = lambda a, e: torch.testing.assert_close(a.cpu().float(), e.float(), **tol(a.dtype))   # noqa: E731
+    y, c = wide(), wide()
+    for f, args in (("add_layer_norm_rows", lambda d: (x.clone().to(d), y.to(d), w.to(d), b.to(d), 1e-5, dt)),
+                    ("add_scaled_rms_norm_rows", lambda d: (x.clone().to(d), y.to(d), c.to(d), 0.4, w.to(d), 1e-5, dt)),
+                    ("dual_rms_mean", lambda d: (y.to(d), c.to(d), w.to(d), b.to(d), 1e-5, 0.5)),
+                    ("layer_norm_rows", lambda d: (x.to(d), w.to(d), b.to(d), 1e-5, dt))):
+        got, want = args(DEV), args("cpu")
+        if f != "layer_norm_rows" and left == 3:                     # (.to makes rows dense: offset them on the GPU again)
+            got = tuple(torch.cat([t[:, :3], t], 1)[:, 3:] if t is not None and hasattr(t, "dim") and t.dim() == 2 and t.dtype == dt
+                        else t for t in got)
+        close(getattr(M, f)(*got), getattr(R, f)(*want))
+        if "add" in f:
+            close(got[0], want[0])
