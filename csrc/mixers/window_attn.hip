@@ -89,7 +89,8 @@ __global__ void attn_prep_kernel(float* __restrict__ q_out, const T* __restrict_
 
 // The same for rows in whole groups of four entries (q and k at most 4 C NT together): four neighbours, their
 // rotation partners and weights in registers, one reduction for both norms.  Bound by one latency for few rows.
-// Rows of 16 and 4 heads of 128: one row 4.5 us, 777 rows 6 (entry by entry, read three times: 9 and 11).
+// Rows of 16 and 4 heads of 128: one row 4.5 us, 777 rows 6 (entry by entry, read three times: 9 and 11); of 4 and 1
+// heads of 64 with norms, 64 rows 3.2 (4.1), 8192 21 (17): most of a workgroup has nothing to do then.
 template <typename T>
 __device__ __forceinline__ float4 ld_four(const T* p) {
   if constexpr (sizeof(T) == 2) {
@@ -624,7 +625,7 @@ extern "C" int mx_attn_prep(float* q_out, const void* qkv, int bf16, long stride
   constexpr int kThreads = 512, kChunks = 4;
   const size_t ts = bf16 ? 8 : 16, tc = cache_bf16 ? 8 : 16;
   if (nq % 4 == 0 && nk % 4 == 0 && nv % 4 == 0 && head_dim % 4 == 0 && rot_dims % 8 == 0 && stride % 4 == 0 &&
-      nq + nk <= 4 * kThreads * kChunks && ((uintptr_t)qkv) % ts == 0 &&
+      nq + nk <= 4 * kThreads * kChunks && (nq + nk >= 512 || rows <= 512) && ((uintptr_t)qkv) % ts == 0 &&
       ((uintptr_t)q_out | (uintptr_t)wq | (uintptr_t)wk | (uintptr_t)table) % 16 == 0 &&
       ((uintptr_t)k_cache | (uintptr_t)v_cache) % tc == 0) {
 #define MX_FOURS(T, TC, C)                                                                                        \

@@ -88,3 +88,21 @@ def test_norms_by_rows(rows, width, left):
         close(getattr(M, f)(*got), getattr(R, f)(*want))
         if "add" in f:
             close(got[0], want[0])
+
+
+@pytest.mark.parametrize("rows,nqh", [(512, 3), (513, 3), (513, 7)])
+def test_attn_prep_by_rows(rows, nqh):
+    """Both sides of the rule on rows and sizes (512 entries, 512 rows)."""
+    g, dt, hd, rot = torch.Generator().manual_seed(rows), torch.bfloat16, 64, 16
+    nq, nk, nv = nqh * hd, hd, 20
+    qkv = rnd(rows, nq + nk + nv + 4, dt=dt, g=g)[:, 4:]
+    wq, wk, table = 1 + rnd(nq, g=g, scale=0.2), 1 + rnd(nk, g=g, scale=0.2), M.rope_table(40, rot, 50.0)
+    pos, slots = torch.arange(rows).int() % 40, torch.arange(rows).int() - 1
+    kc, vc = torch.zeros(-(-rows // 4), 4, nk, dtype=dt), torch.zeros(-(-rows // 4), 4, nv, dtype=dt)
+    kd, vd = kc.to(DEV), vc.to(DEV)
+    want = R.attn_prep(qkv, nq, nk, wq, wk, 1e-5, table, rot, hd, pos, slots, kc, vc)
+    wide = torch.cat([qkv[:, :4], qkv], 1).to(DEV)[:, 4:]
+    got = M.attn_prep(wide, nq, nk, wq.to(DEV), wk.to(DEV), 1e-5, table.to(DEV), rot, hd, pos.to(DEV), slots.to(DEV), kd, vd)
+    torch.testing.assert_close(got.cpu(), want, rtol=2e-5, atol=2e-5)
+    torch.testing.assert_close(kd.cpu().float(), kc.float(), **tol(dt))
+    torch.testing.assert_close(vd.cpu().float(), vc.float(), **tol(dt))
