@@ -461,7 +461,12 @@ extern "C" int mx_short_conv_silu(void* out, const void* x, int bf16, long x_str
   const dim3 block(256);
   int hist_from = 1;
   const int v = bf16 ? 8 : 4;
-  if (taps >= 2 && taps <= 4 && channels % v == 0 && x_stride % v == 0 && ((uintptr_t)x) % 16 == 0 &&
+  // pieces: decode rows, whose history then needs no launch, and enough work to hide their eight rows a thread.  us for 2 / 4
+  // taps, pieces (one thread per value): 300 rows of 256 channels 9 10 (4 5), of 2304 8.5 9.8 (6.2 8.1), of 6144 9.0 10.2
+  // (9.7 13.0); eight segments of 5, 6144 channels 5.3 6.3 (4.9 5.7), of 9 and 12288 8.9 10.5 (6.8 9.0); eight of 300, 1000
+  // channels 11.9 13.3 (11.7 16.0); one row 3.3 4.3 (4.4 4.8)
+  const bool pieces = max_rows == 1 || (long)channels * max_rows * num_segs >= 1250000;
+  if (pieces && taps >= 2 && taps <= 4 && channels % v == 0 && x_stride % v == 0 && ((uintptr_t)x) % 16 == 0 &&
       ((uintptr_t)out) % 16 == 0) {
     const dim3 grid((channels / v + 127) / 128, (max_rows + kConvRows - 1) / kConvRows, num_segs);
     if (max_rows > 65535 || grid.z > 65535) return -2;

@@ -25,3 +25,11 @@ def test_conv_pieces(dt, taps, lens, c, left):
                                None if bias is None else bias.to(DEV))
         torch.testing.assert_close(y2.cpu().float(), y1.float(), **tol(dt))
         torch.testing.assert_close(h2.cpu(), h1, rtol=0, atol=0)
+
+
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("taps", [2, 3, 4])
+@pytest.mark.parametrize("lens,c", [([400, 9, 8, 1], 1032), ([8, 2, 3, 7], 39088), ([41, 16, 17, 33], 7688)])
+def test_conv_pieces_of_many_rows(dt, taps, lens, c):
+    """Work enough for the pieces kernel: part-filled row tiles, histories left by both kernels, padding."""
+    test_conv_pieces(dt, taps, lens, c, 8)
