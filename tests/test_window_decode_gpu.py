@@ -21,12 +21,17 @@ def cases():
     yield "two maps", f(4, 2, 64, 128, 128), dict(maps=2), [1, 9], [1000, 0]
     yield "sigmoid, distance", f(2, 1, 128, 128, 150), dict(sigmoid=True, terms=True), [1, 1], [31, 400]
     yield "sink per head, one key head each", f(2, 2, 128, 128, 33), dict(sinks=True), [1, 7], [640, 0]
+    yield "sixteen heads, cap, sink per head", f(32, 2, 128, 128, 200), dict(softcap=8.0, sinks=True, keep_first=3), [1, 2], [450, 31]
     yield "seventeen heads a group (general kernel)", f(17, 1, 64, 64, 0), {}, [1], [300]
 
 
 @pytest.mark.parametrize("name,sizes,opt,lens,pos0", list(cases()), ids=[c[0] for c in cases()])
 @pytest.mark.parametrize("bs", [3, 16])
-def test_against_64_bits(name, sizes, opt, lens, pos0, bs):
+@pytest.mark.parametrize("tiles", [False, True], ids=["", "tiles"])
+def test_against_64_bits(name, sizes, opt, lens, pos0, bs, tiles, monkeypatch):
+    # attention without score terms goes to the tile kernel of the head-mixing attention, unless it is told not to
+    if not tiles:
+        monkeypatch.setattr(M, "_plain_tiles", lambda *a: False)
     g = torch.Generator().manual_seed(len(name) * 10 + bs)
     rnd = lambda *s: torch.randn(*s, generator=g)   # noqa: E731
     opt = dict(opt)
@@ -44,6 +49,10 @@ def test_against_64_bits(name, sizes, opt, lens, pos0, bs):
     kc = rnd(blocks, bs, sp.kv_heads * sp.maps * sp.dk).to(DEV, torch.bfloat16)
     vc = rnd(blocks, bs, sp.kv_heads * sp.dv).to(DEV, torch.bfloat16)
     q = (2.0 * rnd(sum(lens), hq * sp.dk)).to(DEV)
+    if tiles and not M._plain_tiles(sp, kc):
+        pytest.skip("the same kernels as without")
+    fits = tiles or M.native_mixers().window_decode_fits(q, kc, vc, sp.heads, sp.maps, sp.kv_heads, sp.dk, sp.dv)
+    assert tiles or fits == ("general kernel" not in name)
     want = reference(q, kc, vc, seg, sp, 1)
     out = torch.full((q.shape[0], hq, sp.dv), 7.0, device=DEV)
     got = M.window_attention(q, kc, vc, seg, sp, skip_from=32, out=out.clone())
@@ -55,8 +64,7 @@ def test_against_64_bits(name, sizes, opt, lens, pos0, bs):
     # fp32 sums of a few hundred terms: about 2^-22; no further from 64 bits than the general kernel
     assert e_new < 1e-6 and e_new < 1.5 * e_old + 1e-7, (e_new, e_old)
     # rows in bf16 are the fp32 ones, rounded once
-    if M.window_out_dtype(q, kc, vc, sp, torch.bfloat16, False) == torch.bfloat16:
+    assert (M.window_out_dtype(q, kc, vc, sp, torch.bfloat16, False) == torch.bfloat16) == fits
+    if fits:
         got16 = M.window_attention(q, kc, vc, seg, sp, skip_from=32, out=out.bfloat16())
         assert torch.equal(got16[rows], got[rows].bfloat16())
-    else:
-        assert sp.heads // sp.kv_heads > 16 and not M._plain_tiles(sp, kc)
