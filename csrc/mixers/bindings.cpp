@@ -949,8 +949,8 @@ void moe_route(Tensor idx, Tensor wts, Tensor h, Tensor parts, OptT bias, int64_
                    (int)mode, (float)scale, (int)groups, (int)keep, stream()), "moe_route");
 }
 
-// act 0: clamped GLU, 1: relu^2 (the experts' first matrix is [ff, width], up alone, instead of
-// [2 ff, width], gate | up), 2: silu GLU
+// activations of few_rows_gemm, experts_few and experts_many (few_rows.h): 0 none, 1 gelu GLU, 2 relu GLU, 3 silu GLU,
+// 4 clamped GLU, 5 relu^2 (one first matrix instead of gate | up)
 void few_rows_gemm(Tensor y, Tensor x, Tensor w, OptT bias, int64_t act, double limit) {
   check_rows(x, "x");
   check_rows(y, "y");
@@ -1038,6 +1038,8 @@ void experts_many(Tensor out, Tensor h, Tensor idx, Tensor wts, Tensor wgu, Tens
                        gate_w ? gate_w->data_ptr() : nullptr, t, (int)top, (int)width, stream()), "experts_merge");
 }
 
+// act 0: clamped GLU, 1: relu^2 (the experts' first matrix is [ff, width], up alone, instead of
+// [2 ff, width], gate | up), 2: silu GLU
 void moe_pairs(Tensor out, Tensor h, Tensor idx, Tensor wts, Tensor wgu, Tensor wdown, double limit, int64_t act) {
   const bool relu_sq = act == 1;
   TORCH_CHECK(act >= 0 && act <= 2, "moe_pairs: activation");
@@ -1546,7 +1548,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("moe_route_fits", &moe_route_fits);
   m.def("experts_many", &experts_many);
   m.def("experts_few", &experts_few);
-  m.def("few_rows_max", []() { return (int64_t)mx_few_rows_max(); });
   m.def("act_glu", &act_glu);
   m.def("add_norm_shift", &add_norm_shift);
   m.def("rot_norm_prep", &rot_norm_prep);

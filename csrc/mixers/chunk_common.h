@@ -238,24 +238,24 @@ chunk_carry_kernel(float* __restrict__ ws_s, const float* __restrict__ ws_w, con
     }
     f32x4 v = f.u;
     if constexpr (SOLVED) {
-    f32x4 a[4];
+      f32x4 a[4];
 #pragma unroll
-    for (int m = 0; m < 4; ++m) a[m] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (mine) {
+      for (int m = 0; m < 4; ++m) a[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (mine) {
 #pragma unroll
-      for (int ii = 0; ii < IT; ++ii)
+        for (int ii = 0; ii < IT; ++ii)
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
+          for (int r = 0; r < 4; ++r)
 #pragma unroll
-          for (int m = 0; m < 4; ++m) a[m] = mma(f.w[m][ii][r], S[ii][r], a[m]);
-    }
+            for (int m = 0; m < 4; ++m) a[m] = mma(f.w[m][ii][r], S[ii][r], a[m]);
+      }
 #pragma unroll
-    for (int m = 0; m < 4; ++m) part[m][wave][lane] = a[m];
-    __syncthreads();
-    {
-      const f32x4 v0 = part[wave][0][lane], v1 = part[wave][1][lane], v2 = part[wave][2][lane], v3 = part[wave][3][lane];
-      v = (f.u + v0) + (v1 + (v2 + v3));
-    }
+      for (int m = 0; m < 4; ++m) part[m][wave][lane] = a[m];
+      __syncthreads();
+      {
+        const f32x4 v0 = part[wave][0][lane], v1 = part[wave][1][lane], v2 = part[wave][2][lane], v3 = part[wave][3][lane];
+        v = (f.u + v0) + (v1 + (v2 + v3));
+      }
     }
     whole[idx & 1][wave][lane] = v;          // (two copies: a wave may still read the last chunk's)
     if constexpr (SOLVED) ((f32x4*)ws_u)[((((c.ws + idx) * heads + h) * gridDim.y + blockIdx.y) * 4 + wave) * 64 + lane] = v;

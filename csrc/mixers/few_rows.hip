@@ -187,7 +187,7 @@ template <bool GLU, int MB>
 __global__ void __launch_bounds__(64 * kExpWaves)
 experts_first_kernel(bf16_t* __restrict__ y, bf16_t* __restrict__ ys, float* __restrict__ sg,
                      const bf16_t* __restrict__ h, long h_stride, int rows, const int* __restrict__ idx, int top,
-                     ExpertSet E, int act, float limit, float shared_limit, int vec) {
+                     ExpertSet E, int act, float limit, float shared_limit) {
   constexpr int P = GLU ? 1 : 2;
   __shared__ float4 red[kExpLds<MB> / 16];
   __shared__ int list[kFewRows], counts[kExpWaves];
@@ -204,7 +204,7 @@ experts_first_kernel(bf16_t* __restrict__ y, bf16_t* __restrict__ ys, float* __r
                                          [&](int r, int c, float (&v)[4], float (&u)[4]) {
 #pragma unroll
                                            for (int i = 0; i < 4; ++i) v[i] = fr_act(act, limit, v[i], u[i]);
-                                           fr_store4(y + (long)list[r] * E.N, c, E.N, vec != 0, v);
+                                           fr_store4(y + (long)list[r] * E.N, c, E.N, true, v);
                                          });
     }
     return;
@@ -223,7 +223,7 @@ experts_first_kernel(bf16_t* __restrict__ y, bf16_t* __restrict__ ys, float* __r
                                      [&](int r, int c, float (&v)[4], float (&u)[4]) {
 #pragma unroll
                                        for (int i = 0; i < 4; ++i) v[i] = fr_act(act, shared_limit, v[i], u[i]);
-                                       fr_store4(ys + (long)r * E.shared_N, c, E.shared_N, vec != 0, v);
+                                       fr_store4(ys + (long)r * E.shared_N, c, E.shared_N, true, v);
                                      });
 }
 
@@ -231,7 +231,7 @@ experts_first_kernel(bf16_t* __restrict__ y, bf16_t* __restrict__ ys, float* __r
 template <int MB>
 __global__ void __launch_bounds__(64 * kExpWaves)
 experts_down_kernel(float* __restrict__ d, float* __restrict__ ds, const bf16_t* __restrict__ y,
-                    const bf16_t* __restrict__ ys, int rows, const int* __restrict__ idx, int top, ExpertSet E, int vec) {
+                    const bf16_t* __restrict__ ys, int rows, const int* __restrict__ idx, int top, ExpertSet E) {
   constexpr int P = 2;
   __shared__ float4 red[kExpLds<MB> / 16];
   __shared__ int list[kFewRows], counts[kExpWaves];
@@ -251,7 +251,7 @@ experts_down_kernel(float* __restrict__ d, float* __restrict__ ds, const bf16_t*
     if (total == 0) return;
     expert_tile_any<P, false, kExpWaves, MB>(red, W, E.N, K, n0, X, K, list, min(total - from, 16 * MB), 1, wave, lane,
                                          [&](int r, int c, float (&v)[4], float (&)[4]) {
-                                           fr_store4(dst + (long)list[r] * E.N, c, E.N, vec != 0, v);
+                                           fr_store4(dst + (long)list[r] * E.N, c, E.N, true, v);
                                          });
   }
 }
@@ -353,12 +353,12 @@ extern "C" int mx_experts_few(float* out, void* y, float* d, const void* h, long
   const dim3 g2((unsigned)((width + 31) / 32), g1.y);
 #define EX_FIRST(GLU, MB)                                                                                              \
   hipLaunchKernelGGL((experts_first_kernel<GLU, MB>), g1, block, 0, s, (bf16_t*)y, (bf16_t*)ys, sg, (const bf16_t*)h, \
-                     h_stride, rows, idx, top, first, act, limit, shared_limit, 1)
+                     h_stride, rows, idx, top, first, act, limit, shared_limit)
 #define EX_GO(MB)                                                                                                   \
   do {                                                                                                              \
     if (glu) EX_FIRST(true, MB); else EX_FIRST(false, MB);                                                          \
     hipLaunchKernelGGL((experts_down_kernel<MB>), g2, block, 0, s, d, ds, (const bf16_t*)y, (const bf16_t*)ys, rows, \
-                       idx, top, down, 1);                                                                          \
+                       idx, top, down);                                                                          \
   } while (0)
   if (rows <= 16) EX_GO(1);
   else if (rows <= 32) EX_GO(2);

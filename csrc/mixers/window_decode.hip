@@ -11,7 +11,10 @@
 // sums) meet in LDS at the end: one launch, whatever the length.
 // Bound by a wave's chain for few rows, by the read of the keys for many.  In running models, 16 heads of 128 on 4
 // key heads: one row, 900 keys in a block of 1024 or with a table 25 us (general kernel, a workgroup per head: 50),
-// 540 keys with sigmoid weights 18 (33), two maps of 64 16 (33); 32 rows of 540 24 (56).
+// 540 keys with sigmoid weights 18 (33), two maps of 64 16 (33); 32 rows of 540 24 (56).  A row takes 7.8 us however few its
+// keys (general kernel: 5.8 with one, 6.3 with ten, 9.4 with a hundred), and one query head a key head wastes fifteen
+// columns of sixteen: 64 rows of 16 such heads 32 us at 100 keys (19), 139 at 1000 (158), 385 at 8000 (545).  Lengths are not
+// known on the host where a step is replayed, so sizes alone choose.
 #include "mx_common.h"
 
 namespace mx {
@@ -231,7 +234,7 @@ window_decode_kernel(WindowArgs A) {
       l += f * ml[w][1][h];
       y += f * reinterpret_cast<const float*>(lds)[(long)w * rep * DV + e];
     }
-        y = A.sigmoid ? y : l > 0.f ? y / l : 0.f;
+    y = A.sigmoid ? y : l > 0.f ? y / l : 0.f;
     const long at = ((long)row * hq + (kvh * rep + h) * A.maps + map) * DV + e % DV;
     if (A.out_bf16) st((bf16_t*)A.out, at, y);
     else ((float*)A.out)[at] = y;
@@ -246,7 +249,7 @@ using namespace mx;
 extern "C" int mx_window_decode_fits(const void* out, const void* q, const void* k_cache, const void* v_cache,
                                      int cache_bf16, int heads, int maps, int kv_heads, int dk, int dv, int block_size,
                                      int num_blocks) {
-  return cache_bf16 && (dk == 64 || dk == 128) && (dv == 64 || dv == 128) && heads / kv_heads <= kWdMaxRep &&
+  return cache_bf16 && maps >= 1 && kv_heads >= 1 && (dk == 64 || dk == 128) && (dv == 64 || dv == 128) && heads / kv_heads <= kWdMaxRep &&
          (long)kv_heads * maps <= 65535 && (long)block_size * num_blocks <= 0x7fffffffL &&
          ((((uintptr_t)out) | ((uintptr_t)q) | ((uintptr_t)k_cache) | ((uintptr_t)v_cache)) % 16) == 0;
 }

@@ -725,7 +725,8 @@ class ModelRunner:
         thread that streams to the WebSockets).  ``Event.synchronize`` waits with the GIL
         released (another thread counts at full speed meanwhile) and returns within
         microseconds of the step's end; polling with sleeps of 0.1 ms, whose wake-ups come 0.06 ms
-        late, added 50 to 130 us to every step."""
+        late, added 50 to 130 us to every step.  The price is a core: the runtime spins while it
+        waits (1.0 core where polling takes 0.02; events made with ``blocking=True`` spin as well)."""
         if ev is None:
             if self._gaps and self._gaps[-1][1] is None:
                 self._gap_mark(False)

@@ -89,7 +89,7 @@ def _device_segments(seg: Segments) -> bool:
 # most rows of a product that streams its weights once through the few-rows kernel (a decode
 # step's; the vendor's tiles fill up beyond)
 FEW_ROWS = 64
-# activations of the few-rows kernels
+# activations of the few-rows kernels and the sorted experts (csrc/mixers/few_rows.h)
 FEW_ACTS = {None: 0, "gelu_tanh": 1, "relu": 2, "silu": 3, "clamp_glu": 4, "relu_sq": 5, "silu_glu": 3}
 
 
@@ -651,7 +651,8 @@ def _latent_prefill_pays(seg: Segments, heads: int, min_rows: int) -> bool:
 
 def latent_attention_products(out, qa, qr, cache, seg: Segments, scale: float, rank: int,
                               min_rows: int, dtype, sink: Optional[torch.Tensor] = None):
-    """Segments of ``min_rows`` rows or more as two matrix products: all heads share
+    """Segments of ``min_rows`` rows or more, in one kernel (csrc/mixers/latent_prefill.hip: bf16, ranks of 512 + 64, dense
+    operands, where :func:`_latent_prefill_pays`) or as two matrix products: all heads share
     the cached rows, so with M = heads x rows the scores are Q [M, rank+dr] C^T and the
     sums P [M, keys] C[:, :rank], with a causal softmax (fp32 statistics) in between.
     Needs the segments' host copies; writes its rows of ``out`` [heads, T, rank]."""
@@ -1199,9 +1200,10 @@ ROUTE_MODES = {"top_logits": 0, "top_sigmoid": 1, "grouped_softmax": 2}
 
 def route_parts(router) -> Optional[torch.Tensor]:
     """fp32 router [E, width] as three bf16 parts whose sum is it (hi, mid and lo: 24 bits), in the operand order of
-    :func:`moe_route`: [width / 32, tiles of 16 experts, 3, 64, 8].  None where the width does not fit."""
+    :func:`moe_route`: [width / 32, tiles of 16 experts, 3, 64, 8].  None where it takes no such router
+    (:func:`moe_route_fits`).  A copy: a router that is written to needs new parts."""
     e, width = router.shape
-    if width % 32:
+    if width % 2048 or e > 64:
         return None
     tiles = (e + 15) // 16
     w = torch.nn.functional.pad(router, (0, 0, 0, 16 * tiles - e))
@@ -1214,7 +1216,8 @@ def route_parts(router) -> Optional[torch.Tensor]:
 
 
 def moe_route_fits(h, parts, experts: int) -> bool:
-    """Whether :func:`moe_route` takes these rows: bf16 on a GPU, at most 64 experts, widths of whole 2048."""
+    """Whether :func:`moe_route` takes these rows: bf16 on a GPU, at most 64 experts (a lane each), widths of whole 2048
+    (128 for each of a workgroup's sixteen waves; other widths have not been timed)."""
     return bool(h.is_cuda and parts is not None and native_mixers().moe_route_fits(h, parts, experts))
 
 
@@ -1228,7 +1231,7 @@ def moe_route(h, parts, bias, experts: int, top: int, routing: str, scale: float
     return idx, wts
 
 
-# first matrix and activation of an expert: the code the kernels take
+# first matrix and activation of an expert: the code that the per-pair kernels take (moe_pairs.hip; FEW_ACTS of the others)
 EXPERT_ACTS = {"clamp_glu": 0, "relu_sq": 1, "silu_glu": 2}
 
 

@@ -108,6 +108,7 @@ def test_against_64_bits(name, sizes, opt, lens, pos0, bs, monkeypatch):
     q = (2.0 * rnd(sum(lens), hq * sp.dk)).to(DEV)
     want = reference(q, kc, vc, seg, sp, 32)
     out = torch.full((q.shape[0], hq, sp.dv), 7.0, device=DEV)
+    assert M.band_attention_ok(out, q, kc, vc, seg, sp) and M._band_pays(seg, sp, 32)
     got = M.window_attention_products(out, q, kc, vc, seg, sp, 32)
     rows = torch.cat([torch.full((n,), n >= 32) for n in lens]).to(DEV)
     assert bool((got[~rows] == 7.0).all())                     # short segments are not this path's
