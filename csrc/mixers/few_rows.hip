@@ -102,23 +102,21 @@ struct ExpertSet {
   int shared_K, shared_N;
 };
 
-// the (row, choice) pairs that chose expert e, in ascending order: those numbered from .. from + room - 1 -> list;
-// returns how many there are in all.  A router names an expert once per row, except for a row of NaN, whose choices
-// are all the same; and an index outside the experts counts as the first's.  So there may be more pairs than rows.
-// All threads of the workgroup call it; its barriers end their reads of the list before.
+__device__ __forceinline__ int expert_of(int v, int experts) { return v < 0 || v >= experts ? 0 : v; }
+
+// the (row, choice) pairs that chose expert e -> list, ascending, the first `room` of them; returns how many there are.
+// `once`: a row's first pair only.  All threads of the workgroup call it.
 template <int WV>
-__device__ __forceinline__ int pairs_of(const int* __restrict__ idx, int pairs, int experts, int e, int from, int room,
-                                        int* list, int* counts) {
+__device__ __forceinline__ int pairs_of(const int* __restrict__ idx, int pairs, int top, int experts, int e, bool once,
+                                        int room, int* list, int* counts) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   int total = 0;
   for (int p0 = 0; p0 < pairs; p0 += 64 * WV) {
     const int p = p0 + tid;
-    int v = -1;
-    if (p < pairs) {
-      v = idx[p];
-      if (v < 0 || v >= experts) v = 0;
-    }
-    const uint64_t m = __ballot(v == e);
+    bool mine = p < pairs && expert_of(idx[p], experts) == e;
+    if (once && mine)
+      for (int q = p / top * top; q < p; ++q) mine = mine && expert_of(idx[q], experts) != e;
+    const uint64_t m = __ballot(mine);
     if (lane == 0) counts[wave] = __popcll(m);
     __syncthreads();
     int before = total;
@@ -126,13 +124,24 @@ __device__ __forceinline__ int pairs_of(const int* __restrict__ idx, int pairs, 
       if (w < wave) before += counts[w];
       total += counts[w];
     }
-    if (v == e) {
-      const int at = before + __popcll(m & ((1ull << lane) - 1)) - from;
-      if (at >= 0 && at < room) list[at] = p;
-    }
+    const int at = before + __popcll(m & ((1ull << lane) - 1));
+    if (mine && at < room) list[at] = p;
     __syncthreads();
   }
   return total;
+}
+
+// The same for a tile with room for all rows.  A router names an expert once per row, except for a row of NaN, whose choices
+// are all the same, and an index outside the experts counts as the first's.  Where that makes more pairs than there
+// is room, the list has a row's first pair and the others take its results (`shared`).  (Walking a longer list in turns
+// cost the products 2 to 15%, in registers; looking for repeated choices always, 1 to 5 us.)
+template <int WV>
+__device__ __forceinline__ int rows_of(const int* __restrict__ idx, int pairs, int top, int experts, int e, int room, int* list,
+                                       int* counts, bool& shared) {
+  int count = pairs_of<WV>(idx, pairs, top, experts, e, false, room, list, counts);
+  shared = count > room;
+  if (shared) count = pairs_of<WV>(idx, pairs, top, experts, e, true, room, list, counts);
+  return count;
 }
 
 // the tile's sums for the listed rows: f(entry row in the list, column, sums, up sums)
@@ -196,17 +205,16 @@ experts_first_kernel(bf16_t* __restrict__ y, bf16_t* __restrict__ ys, float* __r
   const int e = blockIdx.y, n0 = blockIdx.x * 16 * P;
   if (e < E.experts) {
     if (n0 >= E.N) return;
+    bool shared;
+    const int count = rows_of<kExpWaves>(idx, rows * top, top, E.experts, e, 16 * MB, list, counts, shared);
+    if (count == 0) return;
     const bf16_t* W = E.w + (long)e * E.N * (GLU ? 2 : 1) * E.K;
-    for (int from = 0, total = 1; from < total; from += 16 * MB) {       // (one turn, but for repeated choices)
-      total = pairs_of<kExpWaves>(idx, rows * top, E.experts, e, from, 16 * MB, list, counts);
-      if (total == 0) return;
-      expert_tile_any<P, GLU, kExpWaves, MB>(red, W, E.N, E.K, n0, h, h_stride, list, min(total - from, 16 * MB), top, wave, lane,
-                                         [&](int r, int c, float (&v)[4], float (&u)[4]) {
+    expert_tile_any<P, GLU, kExpWaves, MB>(red, W, E.N, E.K, n0, h, h_stride, list, count, top, wave, lane,
+                                       [&](int r, int c, float (&v)[4], float (&u)[4]) {
 #pragma unroll
-                                           for (int i = 0; i < 4; ++i) v[i] = fr_act(act, limit, v[i], u[i]);
-                                           fr_store4(y + (long)list[r] * E.N, c, E.N, true, v);
-                                         });
-    }
+                                         for (int i = 0; i < 4; ++i) v[i] = fr_act(act, limit, v[i], u[i]);
+                                         fr_store4(y + (long)list[r] * E.N, c, E.N, true, v);
+                                       });
     return;
   }
   const int tiles = (E.shared_N + 16 * P - 1) / (16 * P);
@@ -238,22 +246,29 @@ experts_down_kernel(float* __restrict__ d, float* __restrict__ ds, const bf16_t*
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int e = blockIdx.y, n0 = blockIdx.x * 16 * P;
-  const bool own = e < E.experts;
-  float* dst = own ? d : ds;
-  const bf16_t *W = own ? E.w + (long)e * E.N * E.K : E.shared, *X = own ? y : ys;
-  const int K = own ? E.K : E.shared_K;
-  if (!own) {
+  float* dst = d;
+  const bf16_t *W = E.w + (long)e * E.N * E.K, *X = y;
+  int K = E.K, count = rows;
+  bool shared = false;
+  if (e < E.experts) {
+    count = rows_of<kExpWaves>(idx, rows * top, top, E.experts, e, 16 * MB, list, counts, shared);
+    if (count == 0) return;
+  } else {
     if (tid < rows) list[tid] = tid;
     __syncthreads();
+    dst = ds;
+    W = E.shared;
+    X = ys;
+    K = E.shared_K;
   }
-  for (int from = 0, total = rows; from < total; from += 16 * MB) {
-    if (own) total = pairs_of<kExpWaves>(idx, rows * top, E.experts, e, from, 16 * MB, list, counts);
-    if (total == 0) return;
-    expert_tile_any<P, false, kExpWaves, MB>(red, W, E.N, K, n0, X, K, list, min(total - from, 16 * MB), 1, wave, lane,
-                                         [&](int r, int c, float (&v)[4], float (&)[4]) {
-                                           fr_store4(dst + (long)list[r] * E.N, c, E.N, true, v);
-                                         });
-  }
+  expert_tile_any<P, false, kExpWaves, MB>(red, W, E.N, K, n0, X, K, list, count, 1, wave, lane,
+                                       [&](int r, int c, float (&v)[4], float (&)[4]) {
+                                         const int p = list[r];
+                                         fr_store4(dst + (long)p * E.N, c, E.N, true, v);
+                                         if (!shared) return;
+                                         for (int q = p + 1; q % top != 0; ++q)
+                                           if (expert_of(idx[q], E.experts) == e) fr_store4(dst + (long)q * E.N, c, E.N, true, v);
+                                       });
 }
 
 // out[row] = sum_k wts[row, k] d[row, k] + shared[row] * (sigmoid(sg[row]) or 1)
