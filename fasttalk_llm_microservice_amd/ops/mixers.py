@@ -131,7 +131,7 @@ def _few_rows_pays(rows: int, n: int, k: int, act: Optional[str] = None) -> bool
         else:
             longest = 2048 if rows <= 32 and not 12288 < n < 16384 else 0
     elif rows <= 16:
-        longest = max(4096, min(8192, 2 * n))
+        longest = max(4096, min(8192, (4 if rows <= 8 else 2) * n))
     else:
         longest = 4096 if rows <= 32 or n >= 512 else 1024
     return k <= longest
