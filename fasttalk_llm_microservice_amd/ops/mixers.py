@@ -102,7 +102,8 @@ def _few_rows(x, w) -> bool:
 
 def _few_rows_pays(rows: int, n: int, k: int, act: Optional[str] = None) -> bool:
     """Where the few-rows kernel is at least level with the vendor's product and, with ``act``, the activation's kernel
-    (``n`` rows of w: a gated form's two matrices).  Its waves take long sums in a chain and share one read of X per
+    (``n`` rows of w: a gated form's two matrices), or behind by a microsecond or so: it takes 5 us on the host where the
+    vendor's call takes 20, which counts in steps that are not replayed.  Its waves take long sums in a chain and share one read of X per
     workgroup, so it loses with k, the sooner the more rows there are; most columns below 16384 go to workgroups of four
     waves, whose chains are twice as long.  us at 1 / 16 / 32 / 64 rows, the vendor's beside it (weights from HBM):
       n = 2048, k = 4096      8 9 11 14 (15 15 12 14)        k = 12288   19 21 28 39 (19 19 24 34)
@@ -131,9 +132,11 @@ def _few_rows_pays(rows: int, n: int, k: int, act: Optional[str] = None) -> bool
         else:
             longest = 2048 if rows <= 32 and not 12288 < n < 16384 else 0
     elif rows <= 16:
-        longest = max(4096, min(8192, (4 if rows <= 8 else 2) * n))
+        longest = max(4096, min(8192, 4 * n))
+    elif rows <= 32:
+        longest = 6144 if n >= 2048 else 4096
     else:
-        longest = 4096 if rows <= 32 or n >= 512 else 1024
+        longest = 4096 if n >= 512 else 2048
     return k <= longest
 
 
