@@ -132,12 +132,13 @@ latent_decode_kernel(float* __restrict__ ws_acc, float* __restrict__ ws_ml, cons
     }
     __syncthreads();
     const float mn = fmaxf(fmaxf(m, fmaxf(tile_max[0][n], tile_max[1][n])), fmaxf(tile_max[2][n], tile_max[3][n]));
-    const float alpha = expf(m - mn);         // 0 at the first tile (m = -inf)
+    const float mu = mn == -INFINITY ? 0.f : mn;      // (scores of -inf, sums that overflow, have weight 0, also alone)
+    const float alpha = expf(m - mu);         // 0 at the first tile (m = -inf)
     if (wave < 4) {
       float sum = 0.f;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        x[e] = expf(x[e] - mn);               // exp(-inf) = 0 for the masked keys
+        x[e] = expf(x[e] - mu);               // exp(-inf) = 0 for the masked keys
         sum += x[e];
       }
       uint2 hi, mid, lo;

@@ -43,3 +43,34 @@ def test_latent_decode(lens, pos0, heads, page, known, sink):
         bound = 2 ** -16 * (p @ k[:, :RANK].abs()) + 1e-7
         assert bool(((got[:, a:b].double() - p @ k[:, :RANK]).abs() <= bound).all())
         a = b
+
+
+@pytest.mark.parametrize("sink", [False, True])
+@pytest.mark.parametrize("known", [False, True])
+@pytest.mark.parametrize("first,last", [(64, 128), (128, 130), (0, 70)])     # a slice of 64, the last slice's two, a first one
+def test_scores_that_overflow(first, last, known, sink):
+    """Scores of -inf (products of 1e20 and -1e20) throughout a slice of the keys: weight 0, as exp(-inf)."""
+    kv, heads, page = 130, 16, 16
+    g = torch.Generator(device=DEV).manual_seed(7)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=DEV)      # noqa: E731
+    seg, _ = make_seg([1], [kv - 1], [0], block_size=page)
+    seg = to_dev(seg)
+    seg.max_kv = kv if known else 0
+    blocks = seg.block_tables[0, :(kv + page - 1) // page].long()
+    keys = rnd(blocks.numel() * page, RANK + DR)
+    keys[:, -1] = 0
+    keys[first:last, -1] = -1e20
+    cache = torch.zeros(int(blocks.max()) + 1, page, RANK + DR, device=DEV)
+    cache[blocks] = keys.view(-1, page, RANK + DR)
+    cache = cache.bfloat16()
+    qa, qr, scale = rnd(heads, 1, RANK), rnd(1, heads, DR), 0.07
+    qr[..., -1] = 1e20
+    sinks = rnd(heads) if sink else None
+    got = M.latent_attention(qa, qr, cache, seg, scale, RANK, sink=sinks)[:, 0].double()
+    k = keys.bfloat16().double()[:kv]
+    sc = (qa[:, 0].double() @ k[:, :RANK].t() + qr[0].double() @ k[:, RANK:].t()) * scale
+    if sink:
+        sc = torch.cat([sc, sinks.double()[:, None]], -1)
+    p = sc.softmax(-1)[:, :kv]
+    # as above
+    assert bool(((got - p @ k[:, :RANK]).abs() <= 2 ** -16 * (p @ k[:, :RANK].abs()) + 1e-7).all())
