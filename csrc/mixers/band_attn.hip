@@ -131,7 +131,7 @@ band_attn_kernel(BandArgs A) {
   };
   auto pages = [&](int tile) {
 #pragma unroll
-    for (int u = 0; u < NT; ++u) blk[u] = table[min(key_of(u, tile), last) >> A.page_shift];
+    for (int u = 0; u < NT; ++u) blk[u] = table[max(min(key_of(u, tile), last), 0) >> A.page_shift];   // (last: -1 without keys)
   };
   auto fetch = [&](int tile) {
 #pragma unroll

@@ -186,3 +186,22 @@ def test_infinite_queries(kind, n):
     got = M.window_attention_products(out, q, kc, vc, seg, sp, 32) if n >= 32 else M.window_attention(q, kc, vc, seg, sp, out=out)
     assert bool(want.isfinite().all())
     assert float((got.double() - want).norm() / want.norm()) < 1e-6       # fp32 sums, as test_against_64_bits
+
+
+@pytest.mark.parametrize("opt", [{}, dict(sink=0.5), dict(window=40, keep_first=3), dict(sigmoid=True)])
+def test_segments_without_keys(opt):
+    """A long segment whose context is empty (the first, so that nothing lies before its pages' ids): zeros."""
+    g = torch.Generator().manual_seed(4)
+    sp = M.WindowSpec(**{**dict(heads=4, kv_heads=2, dk=64, dv=64, window=0, scale=0.125), **opt})
+    seg, blocks = segments([33, 40, 3], [0, 9, 5], 4, g)
+    seg.host[2][0] = 0
+    seg.kv_len[0] = 0
+    kc, vc = (torch.randn(blocks, 4, 128, generator=g).to(DEV, torch.bfloat16) for _ in range(2))
+    q = torch.randn(76, 256, generator=g).to(DEV)
+    out = torch.full((76, 4, 64), 7.0, device=DEV)
+    assert M.band_attention_ok(out, q, kc, vc, seg, sp) and M._band_pays(seg, sp, 32)
+    got = M.window_attention_products(out, q, kc, vc, seg, sp, 32)
+    want = reference(q, kc, vc, seg, sp, 40)
+    assert bool((got[:33] == 0).all()) and bool((got[73:] == 7.0).all())
+    # fp32 sums of a few dozen terms
+    assert float((got[33:73].double() - want[33:73]).norm()) < 1e-6 * float(want.norm())
