@@ -91,46 +91,32 @@ __device__ __forceinline__ void split_bf16x3(float a, float b, uint32_t& hi, uin
   lo = ft::pack2(a1 - __uint_as_float(mid << 16), b1 - __uint_as_float(mid & 0xffff0000u));
 }
 
-// the same for any two values: one that is infinite is its hi part alone, one that bf16 would round to infinity has the
-// largest finite hi part
+// the same for any two values: of one that is infinite, or that bf16 would round to infinity, the largest finite hi part, and
+// what is left is mid (infinite itself, with nothing in lo, or exact)
 __device__ __forceinline__ void split_any_bf16x3(float a, float b, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
   constexpr float kMax = 3.38953139e38f;
-  const auto inf = [](float x) { return fabsf(x) == INFINITY; };
-  const auto in_range = [&](float x) { return fabsf(x) > kMax && !inf(x) ? copysignf(kMax, x) : x; };
-  hi = ft::pack2(in_range(a), in_range(b));
-  const float a1 = inf(a) ? 0.f : a - __uint_as_float(hi << 16), b1 = inf(b) ? 0.f : b - __uint_as_float(hi & 0xffff0000u);
+  const auto cut = [](float x) { return fminf(fmaxf(x, -kMax), kMax); };
+  hi = ft::pack2(cut(a), cut(b));
+  const float a1 = a - __uint_as_float(hi << 16), b1 = b - __uint_as_float(hi & 0xffff0000u);
   mid = ft::pack2(a1, b1);
-  lo = ft::pack2(a1 - __uint_as_float(mid << 16), b1 - __uint_as_float(mid & 0xffff0000u));
+  const float a2 = cut(a1), b2 = cut(b1);
+  const uint32_t m = ft::pack2(a2, b2);
+  lo = ft::pack2(a2 - __uint_as_float(m << 16), b2 - __uint_as_float(m & 0xffff0000u));
 }
 
-// the parts of this lane's 8 entries of each of KS pieces of 32 (src: the lane's first), as matrix operands.  (Which way
-// they are split is asked once per wave: a decode row without keys takes 7.8 us so, 8.0 always in the general form, 7.6 in
-// the short one.)
+// the parts of this lane's 8 entries of each of KS pieces of 32 (src: the lane's first), as matrix operands.  (Any value, with no
+// question asked: a branch between this and the short form has the entries waited for behind the keys' loads, a decode
+// row of 540 keys 19 to 20 us, 18.3 so and with the short form alone.)
 template <int KS>
 __device__ __forceinline__ void split_queries(const float* src, uint4 (&part)[3][KS]) {
-  float4 x[KS][2];
-  float top = 0.f;
 #pragma unroll
-  for (int s = 0; s < KS; ++s)
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      x[s][i] = *reinterpret_cast<const float4*>(src + 32 * s + 4 * i);
-      top = fmaxf(fmaxf(fmaxf(top, fabsf(x[s][i].x)), fabsf(x[s][i].y)), fmaxf(fabsf(x[s][i].z), fabsf(x[s][i].w)));
-    }
-  auto run = [&](auto split) {
-#pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      const float4 u = x[s][0], v = x[s][1];
-      split(u.x, u.y, part[0][s].x, part[1][s].x, part[2][s].x);
-      split(u.z, u.w, part[0][s].y, part[1][s].y, part[2][s].y);
-      split(v.x, v.y, part[0][s].z, part[1][s].z, part[2][s].z);
-      split(v.z, v.w, part[0][s].w, part[1][s].w, part[2][s].w);
-    }
-  };
-  if (__any(top > 3.38953139e38f))
-    run([](float a, float b, uint32_t& hi, uint32_t& mid, uint32_t& lo) { split_any_bf16x3(a, b, hi, mid, lo); });
-  else
-    run([](float a, float b, uint32_t& hi, uint32_t& mid, uint32_t& lo) { split_bf16x3(a, b, hi, mid, lo); });
+  for (int s = 0; s < KS; ++s) {
+    const float4 u = *reinterpret_cast<const float4*>(src + 32 * s), v = *reinterpret_cast<const float4*>(src + 32 * s + 4);
+    split_any_bf16x3(u.x, u.y, part[0][s].x, part[1][s].x, part[2][s].x);
+    split_any_bf16x3(u.z, u.w, part[0][s].y, part[1][s].y, part[2][s].y);
+    split_any_bf16x3(v.x, v.y, part[0][s].z, part[1][s].z, part[2][s].z);
+    split_any_bf16x3(v.z, v.w, part[0][s].w, part[1][s].w, part[2][s].w);
+  }
 }
 
 // a wave's own LDS writes, to be read by its other lanes
