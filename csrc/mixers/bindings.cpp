@@ -53,11 +53,11 @@ int mx_chunk_rows();
 int mx_chunk_key_pad(int dk);
 int mx_head_delta_chunks(float* o, const float* q, const float* k, const float* v, const float* lg, const float* beta,
                          float* state, float* ws_s, float* ws_w, float* ws_k, float* ws_u, float* ws_g,
-                         const int* start, const int* pos0, const int* slot, int num_segs, int max_rows, int heads,
+                         const int* start, const int* pos0, const int* slot, long rows, int num_segs, int max_rows, int heads,
                          int kv_heads, int dk, int dv, int num_slots, int min_rows, hipStream_t s);
 int mx_retention_chunks(float* o, const void* p, int bf16, long stride, const float* table, int table_rows,
                         int rot_dims, int interleaved, const double* log_decay, float* state, float* ws_s,
-                        const int* start, const int* pos0, const int* slot, int num_segs, int max_rows, int heads,
+                        const int* start, const int* pos0, const int* slot, long rows, int num_segs, int max_rows, int heads,
                         int dk, int dv, int num_slots, int min_rows, hipStream_t s);
 int mx_act_glu(void* out, const void* gu, int bf16, long gu_stride, long rows, int ff, int act, hipStream_t s);
 int mx_row_max_width();
@@ -149,12 +149,12 @@ int mx_channel_delta_chunks(float* o, const float* qn, const float* kn, const fl
                             const void* qkv, int bf16, long stride, const void* a, long a_stride,
                             const void* b, long b_stride, const float* a_log, const float* dt_bias, float* state,
                             float* ws_s, float* ws_p, float* ws_q, float* ws_k, float* ws_g, float* ws_w, float* ws_u,
-                            const int* start, const int* pos0, const int* slot, int num_segs, int max_rows, int heads,
+                            const int* start, const int* pos0, const int* slot, long rows, int num_segs, int max_rows, int heads,
                             int kv_heads, int dk, int dv, int num_slots, int min_rows, hipStream_t s);
 int mx_channel_linear_chunks(float* o, const void* qkv, int bf16, long stride, const void* a, long a_stride,
                              const float* a_bias, float tau, float* state, float* ws_s, float* ws_p, float* ws_q,
                              float* ws_k, float* ws_g, const int* start, const int* pos0, const int* slot,
-                             int num_segs, int max_rows, int heads, int dk, int dv, int num_slots, int min_rows,
+                             long rows, int num_segs, int max_rows, int heads, int dk, int dv, int num_slots, int min_rows,
                              hipStream_t s);
 int mx_latent_kv_write(const void* dkv, int bf16, long stride, const float* w, float eps, const float* table,
                        int table_rows, int dims, const int* positions, const int* slots, void* cache,
@@ -540,7 +540,7 @@ void gated_delta_rule(Tensor o, Tensor qkv, Tensor a, Tensor b, Tensor a_log, Te
                               state.data_ptr<float>(), ws.s.data_ptr<float>(), ws.p.data_ptr<float>(),
                               ws.q.data_ptr<float>(), ws.k.data_ptr<float>(), ws.g.data_ptr<float>(),
                               ws.w.data_ptr<float>(), ws.u.data_ptr<float>(), start.data_ptr<int>(),
-                              pos0.data_ptr<int>(), slot.data_ptr<int>(), (int)num_segs, (int)max_rows, (int)heads,
+                              pos0.data_ptr<int>(), slot.data_ptr<int>(), t, (int)num_segs, (int)max_rows, (int)heads,
                               (int)kv_heads, (int)dk, (int)dv, (int)state.size(0), (int)chunk_from, stream()),
       "delta rule chunks");
 }
@@ -597,7 +597,7 @@ void head_delta_rule(Tensor o, Tensor q, Tensor k, Tensor v, Tensor lg, Tensor b
                            lg.data_ptr<float>(), beta.data_ptr<float>(), state.data_ptr<float>(),
                            ws_s.data_ptr<float>(), ws_w.data_ptr<float>(), ws_k.data_ptr<float>(),
                            ws_u.data_ptr<float>(), ws_g.data_ptr<float>(), start.data_ptr<int>(), pos0.data_ptr<int>(),
-                           slot.data_ptr<int>(), (int)num_segs, (int)max_rows, (int)heads, (int)kvh, (int)dk, (int)dv,
+                           slot.data_ptr<int>(), t, (int)num_segs, (int)max_rows, (int)heads, (int)kvh, (int)dk, (int)dv,
                            (int)state.size(0), (int)chunk_from, stream()), "delta rule chunks");
 }
 
@@ -627,7 +627,7 @@ void retention(Tensor o, Tensor p, OptT table, int64_t rot_dims, bool interleave
   chk(mx_retention_chunks(o.data_ptr<float>(), p.data_ptr(), bf(p), p.stride(0), rope.table, rope.rows, rope.dims,
                           interleaved ? 1 : 0, log_decay.data_ptr<double>(), state.data_ptr<float>(),
                           ws_s.data_ptr<float>(), start.data_ptr<int>(), pos0.data_ptr<int>(), slot.data_ptr<int>(),
-                          (int)num_segs, (int)max_rows, (int)heads, (int)dk, (int)dv, (int)state.size(0),
+                          t, (int)num_segs, (int)max_rows, (int)heads, (int)dk, (int)dv, (int)state.size(0),
                           (int)chunk_from, stream()), "retention chunks");
 }
 
@@ -683,7 +683,7 @@ void gated_linear_attention(Tensor o, Tensor qkv, Tensor a, Tensor a_bias, doubl
                                a_bias.data_ptr<float>(), (float)tau, state.data_ptr<float>(), ws.s.data_ptr<float>(),
                                ws.p.data_ptr<float>(), ws.q.data_ptr<float>(), ws.k.data_ptr<float>(),
                                ws.g.data_ptr<float>(), start.data_ptr<int>(), pos0.data_ptr<int>(),
-                               slot.data_ptr<int>(), (int)num_segs, (int)max_rows, (int)heads, (int)dk, (int)dv,
+                               slot.data_ptr<int>(), t, (int)num_segs, (int)max_rows, (int)heads, (int)dk, (int)dv,
                                (int)state.size(0), (int)chunk_from, stream()), "linear attention chunks");
 }
 

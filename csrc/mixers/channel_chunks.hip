@@ -90,15 +90,16 @@ __global__ void __launch_bounds__(kPrepThreads)
 channel_prep_kernel(float* __restrict__ ws_p, float* __restrict__ ws_q, float* __restrict__ ws_k,
                     float* __restrict__ ws_g, float* __restrict__ ws_w, float* __restrict__ ws_u, ChannelIn in,
                     const int* __restrict__ start, const int* __restrict__ pos0, const int* __restrict__ slot, int heads,
-                    int dk, int dv, int num_slots, int min_rows, int vec) {
+                    int dk, int dv, int num_slots, ChunkSteps st, int vec) {
   constexpr int DKP = 16 * DKT, LDK = DKP + 4;
   extern __shared__ __attribute__((aligned(16))) float lds[];
   float *kb = lds, *qb = kb + kC * LDK, *gb = qb + kC * LDK;       // rows of k, q, decays; later k u, q c, k c
   float *ab = gb + kC * LDK, *pb = ab + kC * kPLD;                 // pair weights of k (times beta) and of q
   float *bt = pb + kC * kPLD, *bs = bt + 4 * DKP;                  // block products, beta
   Chunk c;
-  if (!find_chunk(c, blockIdx.x, blockIdx.z, start, pos0, slot, min_rows, num_slots)) return;
-  const int h = blockIdx.y;
+  int seg, idx;
+  if (!find_chunk(c, blockIdx.x / heads, st, seg, idx, start, pos0, slot, num_slots)) return;
+  const int h = blockIdx.x % heads;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lo = lane & 15, hi = lane >> 4, half = wave >> 2;
   auto stage = [&](auto type, auto rows) {
@@ -351,25 +352,27 @@ channel_prep_kernel(float* __restrict__ ws_p, float* __restrict__ ws_q, float* _
   }
 }
 
-// grid (chunks, heads * ceil(dv / 64), segments): o of the chunk's rows, wave w rows 16 w .. 16 w + 15
+// a workgroup per chunk, head and 64 columns: o of the chunk's rows, wave w rows 16 w .. 16 w + 15
 template <int DKT, bool DELTA, typename TV>
 __global__ void __launch_bounds__(256)
 channel_out_kernel(float* __restrict__ o, ChannelIn in, const float* __restrict__ ws_s, const float* __restrict__ ws_p,
                    const float* __restrict__ ws_q, const float* __restrict__ ws_u, const int* __restrict__ start,
                    const int* __restrict__ pos0, const int* __restrict__ slot, int heads, int dk, int dv, int num_slots,
-                   int min_rows, int vec) {
+                   ChunkSteps st, int vec) {
   __shared__ __attribute__((aligned(16))) float vb[2][kC * kVLD];
-  const int vt = (dv + 63) / 64;
-  const int h = blockIdx.y / vt, col0 = blockIdx.y % vt * 64;
+  const int vt = (dv + 63) / 64, unit = blockIdx.x % (heads * vt);
+  const int h = unit / vt, col0 = unit % vt * 64;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lo = lane & 15, hi = lane >> 4;
   Chunk c;
-  if (!find_chunk(c, blockIdx.x, blockIdx.z, start, pos0, slot, min_rows, num_slots)) {
+  int s, idx;
+  if (!find_chunk(c, blockIdx.x / (heads * vt), st, s, idx, start, pos0, slot, num_slots)) {
+    if (s < 0) return;
     // a padding segment's rows are zeros
-    const int s = blockIdx.z, r0 = start[s], n = start[s + 1] - r0;
-    if (n >= min_rows && (slot[s] < 0 || slot[s] >= num_slots))
+    const int r0 = start[s], n = start[s + 1] - r0;
+    if (n >= st.min_rows && (slot[s] < 0 || slot[s] >= num_slots))
       for (int e = tid; e < kC * 64; e += 256) {
-        const int t = blockIdx.x * kC + (e >> 6), cc = col0 + (e & 63);
+        const int t = idx * kC + (e >> 6), cc = col0 + (e & 63);
         if (t < n && cc < dv) o[((long)(r0 + t) * heads + h) * dv + cc] = 0.f;
       }
     return;
@@ -440,11 +443,11 @@ struct ChannelWs {
 
 template <bool DELTA, typename T>
 int channel_run(float* o, const ChannelIn& in, const ChannelWs& ws, float* state, const int* start, const int* pos0,
-                const int* slot, int num_segs, int max_rows, int heads, int dk, int dv, int num_slots, int min_rows,
+                const int* slot, long rows, int num_segs, int max_rows, int heads, int dk, int dv, int num_slots, int min_rows,
                 int vec, hipStream_t s) {
-  const int chunks = (max_rows + kC - 1) / kC;
+  const ChunkGrid g(rows, max_rows, min_rows, num_segs);
   const long outs = (long)heads * ((dv + 63) / 64);
-  if (heads > 65535 || outs > 65535 || num_segs > 65535) return -2;
+  if (!g.fits(outs)) return -2;
   // whole quads of q, k and g at aligned addresses
   const int quads = dk % 4 == 0 && in.q_stride % 4 == 0 && in.k_stride % 4 == 0 && in.g_stride % 4 == 0 &&
                     ((uintptr_t)in.q | (uintptr_t)in.k | (uintptr_t)in.g) % (4 * (DELTA && in.a_log == nullptr ? sizeof(float) : sizeof(T))) == 0;
@@ -456,17 +459,17 @@ int channel_run(float* o, const ChannelIn& in, const ChannelWs& ws, float* state
       rc = (int)hipFuncSetAttribute(reinterpret_cast<const void*>(prep), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
       if (rc != 0) return;
     }
-    hipLaunchKernelGGL(prep, dim3(chunks, heads, num_segs), dim3(kPrepThreads), lds, s, ws.p, ws.q, ws.k, ws.g, ws.w,
-                       ws.u, in, start, pos0, slot, heads, dk, dv, num_slots, min_rows, quads);
-    const dim3 cgrid(heads, (dv + 15) / 16, num_segs);
+    hipLaunchKernelGGL(prep, g.grid(heads), dim3(kPrepThreads), lds, s, ws.p, ws.q, ws.k, ws.g, ws.w,
+                       ws.u, in, start, pos0, slot, heads, dk, dv, num_slots, g.steps, quads);
+    const dim3 cgrid(heads, (dv + 15) / 16, g.longs);
     if (dk == 16 * DKT && dv % 16 == 0)
       hipLaunchKernelGGL((chunk_carry_kernel<DKT, true, true, DELTA, T>), cgrid, dim3(256), 0, s, ws.s, ws.w, ws.k, ws.u,
-                         ws.g, (const T*)in.v, in.v_stride, state, start, pos0, slot, heads, dk, dv, num_slots, min_rows);
+                         ws.g, (const T*)in.v, in.v_stride, state, start, pos0, slot, heads, dk, dv, num_slots, g.steps);
     else
       hipLaunchKernelGGL((chunk_carry_kernel<DKT, false, true, DELTA, T>), cgrid, dim3(256), 0, s, ws.s, ws.w, ws.k, ws.u,
-                         ws.g, (const T*)in.v, in.v_stride, state, start, pos0, slot, heads, dk, dv, num_slots, min_rows);
-    hipLaunchKernelGGL((channel_out_kernel<DKT, DELTA, T>), dim3(chunks, (unsigned)outs, num_segs), dim3(256), 0, s, o, in,
-                       ws.s, ws.p, ws.q, ws.u, start, pos0, slot, heads, dk, dv, num_slots, min_rows, vec);
+                         ws.g, (const T*)in.v, in.v_stride, state, start, pos0, slot, heads, dk, dv, num_slots, g.steps);
+    hipLaunchKernelGGL((channel_out_kernel<DKT, DELTA, T>), g.grid(outs), dim3(256), 0, s, o, in,
+                       ws.s, ws.p, ws.q, ws.u, start, pos0, slot, heads, dk, dv, num_slots, g.steps, vec);
   });
   return rc != 0 ? rc : (int)hipGetLastError();
 }
@@ -483,7 +486,7 @@ extern "C" int mx_channel_delta_chunks(float* o, const float* qn, const float* k
                                        const void* b, long b_stride, const float* a_log, const float* dt_bias,
                                        float* state, float* ws_s, float* ws_p, float* ws_q, float* ws_k, float* ws_g,
                                        float* ws_w, float* ws_u, const int* start, const int* pos0, const int* slot,
-                                       int num_segs, int max_rows, int heads, int kv_heads, int dk, int dv,
+                                       long rows, int num_segs, int max_rows, int heads, int kv_heads, int dk, int dv,
                                        int num_slots, int min_rows, hipStream_t s) {
   if (num_segs <= 0 || max_rows < min_rows) return 0;
   if (dk < 1 || dk > 128 || dv < 1 || kv_heads < 1 || heads % kv_heads || min_rows < 1) return -1;
@@ -511,14 +514,14 @@ extern "C" int mx_channel_delta_chunks(float* o, const float* qn, const float* k
     in.q_scale = 1.f;
   }
   const ChannelWs ws{ws_s, ws_p, ws_q, ws_k, ws_g, ws_w, ws_u};
-  MX_DISPATCH_T(bf16, return (channel_run<true, T>(o, in, ws, state, start, pos0, slot, num_segs, max_rows, heads, dk, dv,
+  MX_DISPATCH_T(bf16, return (channel_run<true, T>(o, in, ws, state, start, pos0, slot, rows, num_segs, max_rows, heads, dk, dv,
                                                    num_slots, min_rows, 0, s)));
 }
 
 extern "C" int mx_channel_linear_chunks(float* o, const void* qkv, int bf16, long stride, const void* a, long a_stride,
                                         const float* a_bias, float tau, float* state, float* ws_s, float* ws_p,
                                         float* ws_q, float* ws_k, float* ws_g, const int* start, const int* pos0,
-                                        const int* slot, int num_segs, int max_rows, int heads, int dk, int dv,
+                                        const int* slot, long rows, int num_segs, int max_rows, int heads, int dk, int dv,
                                         int num_slots, int min_rows, hipStream_t s) {
   if (num_segs <= 0 || max_rows < min_rows) return 0;
   if (dk < 1 || dk > 128 || dv < 1 || heads < 1 || min_rows < 1 || !(tau > 0.f)) return -1;
@@ -537,6 +540,6 @@ extern "C" int mx_channel_linear_chunks(float* o, const void* qkv, int bf16, lon
   in.q_scale = 1.0f / sqrtf((float)dk);
   const int vec = dk % 4 == 0 && dv % 4 == 0 && stride % 4 == 0 && ((uintptr_t)qkv) % (4 * es) == 0;
   const ChannelWs ws{ws_s, ws_p, ws_q, ws_k, ws_g, nullptr, nullptr};
-  MX_DISPATCH_T(bf16, return (channel_run<false, T>(o, in, ws, state, start, pos0, slot, num_segs, max_rows, heads, dk,
+  MX_DISPATCH_T(bf16, return (channel_run<false, T>(o, in, ws, state, start, pos0, slot, rows, num_segs, max_rows, heads, dk,
                                                        dv, num_slots, min_rows, vec, s)));
 }

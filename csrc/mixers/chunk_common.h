@@ -3,6 +3,7 @@
 // triangular matrix.
 #pragma once
 
+#include <algorithm>
 #include <type_traits>
 
 #include "mx_common.h"
@@ -79,6 +80,32 @@ __device__ __forceinline__ bool find_chunk(Chunk& c, int idx, int s, const int* 
   return true;
 }
 
+// A step's chunk kernels run over its chunks and not over as many per segment as its longest one has: a prompt beside 64
+// decode rows would be one chunk in a hundred, and every empty workgroup waits for the LDS of a full one.  The counts are
+// bounds from the step's rows; which segment a workgroup has it finds itself, unless all have the same number.
+struct ChunkSteps {
+  int num_segs, min_rows, per_seg;     // per_seg: chunks of every segment, or 0
+};
+// workgroup `item` of a unit: its segment and chunk; false if there is none (s: -1 if there is no such segment)
+__device__ __forceinline__ bool find_chunk(Chunk& c, int item, const ChunkSteps& st, int& s, int& idx, const int* start,
+                                           const int* pos0, const int* slot, int num_slots) {
+  if (st.per_seg > 0) {
+    s = item / st.per_seg, idx = item % st.per_seg;
+  } else {
+    s = -1;
+    if (!segment_block(start, st.num_segs, st.min_rows, 1, kC, item, s, idx)) return false;
+    s = __builtin_amdgcn_readfirstlane(s), idx = __builtin_amdgcn_readfirstlane(idx);
+  }
+  return find_chunk(c, idx, s, start, pos0, slot, st.min_rows, num_slots);
+}
+// the i-th of `longs` segments that have chunks (-1: none)
+__device__ __forceinline__ int long_segment(int i, int longs, const ChunkSteps& st, const int* start) {
+  if (longs == st.num_segs) return i;
+  int s = -1, block;
+  if (!segment_block(start, st.num_segs, st.min_rows, 1, 1 << 30, i, s, block)) return -1;
+  return __builtin_amdgcn_readfirstlane(s);
+}
+
 // ab [kC][kPLD]: A below the diagonal (nothing else is read) -> T = (I + A)^-1, the blocks above the
 // diagonal blocks left as they are.  The first four of WAVES waves work; what they read of the diagonal
 // blocks of A has been written by the wave itself or before a barrier.
@@ -150,7 +177,7 @@ __device__ __forceinline__ void inverse_column(const float (&tf)[4][16], const f
 }
 
 // ---------------------------------------------------------------------------------
-// grid (heads, ceil(dv / 16), segments), four waves: the state's 16 columns, chunk after chunk.
+// grid (heads, ceil(dv / 16), long segments), four waves: the state's 16 columns, chunk after chunk.
 // (Heads come first so that, 8 XCDs taking workgroups in turn, the column tiles of a head
 // tend to share one XCD's L2: they all read the same operands.)
 // Wave w holds the 16-row tiles w IT .. w IT + IT - 1 in accumulators; accumulator register r of
@@ -168,12 +195,13 @@ __global__ void __launch_bounds__(256)
 chunk_carry_kernel(float* __restrict__ ws_s, const float* __restrict__ ws_w, const float* __restrict__ ws_k,
                    float* __restrict__ ws_u, const float* __restrict__ ws_g, const TV* __restrict__ v_rows,
                    long v_stride, float* __restrict__ state, const int* __restrict__ start, const int* __restrict__ pos0, const int* __restrict__ slot, int heads,
-                   int dk, int dv, int num_slots, int min_rows) {
+                   int dk, int dv, int num_slots, ChunkSteps st) {
   constexpr int IT = DKT < 4 ? 1 : DKT / 4;
   __shared__ f32x4 part[SOLVED ? 4 : 1][4][64], whole[2][4][64];
   Chunk c;
-  if (!find_chunk(c, 0, blockIdx.z, start, pos0, slot, min_rows, num_slots)) return;
-  const int h = blockIdx.x, rows = start[blockIdx.z + 1] - start[blockIdx.z];
+  const int seg = long_segment(blockIdx.z, gridDim.z, st, start);
+  if (seg < 0 || !find_chunk(c, 0, seg, start, pos0, slot, st.min_rows, num_slots)) return;
+  const int h = blockIdx.x, rows = start[seg + 1] - start[seg];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, lo = lane & 15, hi = lane >> 4;
   const int col = blockIdx.y * 16 + lo;
   const bool live = FULL || col < dv;
@@ -302,6 +330,26 @@ chunk_carry_kernel(float* __restrict__ ws_s, const float* __restrict__ ws_w, con
 }
 
 }  // namespace mx
+
+// The launches of a step of `rows` rows, segments of up to max_rows, those of at least min_rows in chunks.  grid(units): a
+// workgroup per chunk and unit (head, or head and 64 columns), units fastest: workgroups go to the 8 XCDs in turn, so with
+// chunks fastest segments of a multiple of eight put their first chunks, a short one's only ones, on the same XCD.  us, delta
+// rule / linear attention / scan: 64 heads of 128 x 64, a segment of 1000 rows and ten of 100 436 261 221, with chunks
+// fastest 1533 834 223 (walks 688 428 222); 128 of 64 x 32, one of 1000 beside 64 of one row 365 255 163, with a workgroup
+// for every chunk that a segment could have 574 458 298 (429 253 181).
+struct ChunkGrid {
+  mx::ChunkSteps steps;
+  long items;
+  int longs;
+  ChunkGrid(long rows, int max_rows, int min_rows, int num_segs) {
+    const int most = (max_rows + mx::kC - 1) / mx::kC;
+    longs = (int)std::max(1L, std::min((long)num_segs, rows / min_rows));
+    items = std::min((long)most * num_segs, rows / mx::kC + longs);
+    steps = {num_segs, min_rows, items == (long)most * num_segs ? most : 0};
+  }
+  bool fits(long units) const { return units <= 65535 && longs <= 65535 && items * units <= 0x7fffffffL; }
+  dim3 grid(long units) const { return dim3((unsigned)(items * units)); }
+};
 
 // calls f with the key size's tile count as a constant
 template <typename F>

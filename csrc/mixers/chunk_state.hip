@@ -118,7 +118,7 @@ __device__ __forceinline__ void stage_row_scale(float* rs, const ChunkIn& in, lo
 }
 
 // ---------------------------------------------------------------------------------
-// grid (chunks, heads * ceil(dv / 64), segments): L = sum_j e^{G_last - G_j} k_j v_j^T into the
+// a workgroup per chunk, head and 64 columns: L = sum_j e^{G_last - G_j} k_j v_j^T into the
 // chunk's workspace [dk, dv] (v times its row factor); totals[chunk, head] = e^{G_last} if wanted.
 // Wave w: columns 16 w .. 16 w + 15 of the 64, all rows.
 // ---------------------------------------------------------------------------------
@@ -126,15 +126,16 @@ template <typename T, int DKT>
 __global__ void __launch_bounds__(256)
 state_add_kernel(float* __restrict__ ws_s, float* __restrict__ totals, ChunkIn in, const int* __restrict__ start,
                  const int* __restrict__ pos0, const int* __restrict__ slot, int heads, int dk, int dv, int num_slots,
-                 int min_rows, int vec) {
+                 ChunkSteps st, int vec) {
   constexpr int DKP = 16 * DKT, LDK = DKP + 16;
   __shared__ __attribute__((aligned(16))) float kb[kC * LDK], vb[kC * kVLD];
   __shared__ double G[kC];
   __shared__ float rs[kC];
+  const int vt = (dv + 63) / 64, unit = blockIdx.x % (heads * vt);
+  const int h = unit / vt, col0 = unit % vt * 64;
   Chunk c;
-  if (!find_chunk(c, blockIdx.x, blockIdx.z, start, pos0, slot, min_rows, num_slots)) return;
-  const int vt = (dv + 63) / 64;
-  const int h = blockIdx.y / vt, col0 = blockIdx.y % vt * 64;
+  int seg, idx;
+  if (!find_chunk(c, blockIdx.x / (heads * vt), st, seg, idx, start, pos0, slot, num_slots)) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, lo = lane & 15, hi = lane >> 4;
   stage_log_decay(G, in, c.row0, c.cnt, heads, h);
   stage_row_scale(rs, in, c.row0, c.cnt, heads, h);
@@ -166,18 +167,19 @@ state_add_kernel(float* __restrict__ ws_s, float* __restrict__ totals, ChunkIn i
     }
 }
 
-// grid (ceil(dk dv / 256), heads, segments): workspaces hold every chunk's own contribution L_c
+// grid (ceil(dk dv / 256), heads, long segments): workspaces hold every chunk's own contribution L_c
 // and become its incoming state; the last one goes to the slot.  A chunk's decay: totals[chunk, head],
 // or the head's fixed one per row.
 __global__ void __launch_bounds__(256)
 state_carry_kernel(float* __restrict__ ws_s, const double* __restrict__ log_decay, const float* __restrict__ totals,
                    float* __restrict__ state, const int* __restrict__ start, const int* __restrict__ pos0,
-                   const int* __restrict__ slot, int heads, int size, int num_slots, int min_rows) {
+                   const int* __restrict__ slot, int heads, int size, int num_slots, ChunkSteps st) {
   Chunk c;
-  if (!find_chunk(c, 0, blockIdx.z, start, pos0, slot, min_rows, num_slots)) return;
+  const int seg = long_segment(blockIdx.z, gridDim.z, st, start);
+  if (seg < 0 || !find_chunk(c, 0, seg, start, pos0, slot, st.min_rows, num_slots)) return;
   const int h = blockIdx.y, e = blockIdx.x * 256 + threadIdx.x;
   if (e >= size) return;
-  const int n = start[blockIdx.z + 1] - start[blockIdx.z];
+  const int n = start[seg + 1] - start[seg];
   float* sp = state + ((long)c.slot * heads + h) * size + e;
   float S = c.pos > 0 ? *sp : 0.f;
   float full = 0.f, last = 0.f;
@@ -207,29 +209,31 @@ state_carry_kernel(float* __restrict__ ws_s, const double* __restrict__ log_deca
 }
 
 // ---------------------------------------------------------------------------------
-// grid (chunks, heads * ceil(dv / 64), segments): o of the chunk's rows.  Wave w: rows 16 w ..
+// a workgroup per chunk, head and 64 columns: o of the chunk's rows.  Wave w: rows 16 w ..
 // 16 w + 15, 64 columns; its q rows stay in registers as left-hand operands.
 // ---------------------------------------------------------------------------------
 template <typename T, int DKT>
 __global__ void __launch_bounds__(256)
 chunk_out_kernel(float* __restrict__ o, ChunkIn in, const float* __restrict__ ws_s, const int* __restrict__ start,
                  const int* __restrict__ pos0, const int* __restrict__ slot, int heads, int dk, int dv, int num_slots,
-                 int min_rows, int vec) {
+                 ChunkSteps st, int vec) {
   constexpr int DKP = 16 * DKT, LDK = DKP + 4;
   constexpr int KB = kC * LDK > 64 * kPLD ? kC * LDK : 64 * kPLD;
   __shared__ __attribute__((aligned(16))) float kb[KB], vb[kC * kVLD];
   __shared__ double G[kC];
   __shared__ float rs[kC];
-  const int vt = (dv + 63) / 64;
-  const int h = blockIdx.y / vt, col0 = blockIdx.y % vt * 64;
+  const int vt = (dv + 63) / 64, unit = blockIdx.x % (heads * vt);
+  const int h = unit / vt, col0 = unit % vt * 64;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, lo = lane & 15, hi = lane >> 4;
   Chunk c;
-  if (!find_chunk(c, blockIdx.x, blockIdx.z, start, pos0, slot, min_rows, num_slots)) {
+  int s, idx;
+  if (!find_chunk(c, blockIdx.x / (heads * vt), st, s, idx, start, pos0, slot, num_slots)) {
+    if (s < 0) return;
     // a padding segment's rows are zeros
-    const int s = blockIdx.z, r0 = start[s], n = start[s + 1] - r0;
-    if (n >= min_rows && (slot[s] < 0 || slot[s] >= num_slots))
+    const int r0 = start[s], n = start[s + 1] - r0;
+    if (n >= st.min_rows && (slot[s] < 0 || slot[s] >= num_slots))
       for (int e = tid; e < kC * 64; e += 256) {
-        const int t = blockIdx.x * kC + (e >> 6), cc = col0 + (e & 63);
+        const int t = idx * kC + (e >> 6), cc = col0 + (e & 63);
         if (t < n && cc < dv) o[((long)(r0 + t) * heads + h) * dv + cc] = 0.f;
       }
     return;
@@ -336,7 +340,7 @@ chunk_out_kernel(float* __restrict__ o, ChunkIn in, const float* __restrict__ ws
 }
 
 // ---------------------------------------------------------------------------------
-// grid (chunks, heads, segments), 256 threads.  Leaves per chunk and head, as fragments: -W,
+// a workgroup per chunk and head, 256 threads.  Leaves per chunk and head, as fragments: -W,
 // e^{G_last - G_j} k_j and U; and e^{G_last}.
 // ---------------------------------------------------------------------------------
 template <int DKT>
@@ -344,15 +348,16 @@ __global__ void __launch_bounds__(256)
 delta_solve_kernel(float* __restrict__ ws_w, float* __restrict__ ws_k, float* __restrict__ ws_u,
                    float* __restrict__ ws_g, ChunkIn in, const float* __restrict__ beta, const int* __restrict__ start,
                    const int* __restrict__ pos0, const int* __restrict__ slot, int heads, int dk, int dv, int num_slots,
-                   int min_rows, int vec) {
+                   ChunkSteps st, int vec) {
   constexpr int DKP = 16 * DKT, LDK = DKP + 4;
   // ab: A, block by block replaced by T = (I + A)^-1 (blocks above the diagonal are never read)
   __shared__ __attribute__((aligned(16))) float kb[kC * LDK], ab[kC * kPLD];
   __shared__ double G[kC];
   __shared__ float bs[kC], eg[kC], el[kC];
   Chunk c;
-  if (!find_chunk(c, blockIdx.x, blockIdx.z, start, pos0, slot, min_rows, num_slots)) return;
-  const int h = blockIdx.y;
+  int seg, idx;
+  if (!find_chunk(c, blockIdx.x / heads, st, seg, idx, start, pos0, slot, num_slots)) return;
+  const int h = blockIdx.x % heads;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, lo = lane & 15, hi = lane >> 4;
   stage_log_decay(G, in, c.row0, c.cnt, heads, h);
   if (tid >= 64 && tid < 128) bs[tid - 64] = tid - 64 < c.cnt ? beta[(c.row0 + tid - 64) * heads + h] : 0.f;
@@ -434,17 +439,17 @@ extern "C" int mx_chunk_key_pad(int dk) { return dk <= 16 ? 16 : dk <= 32 ? 32 :
 
 template <typename T>
 static void launch_out(float* o, const ChunkIn& in, const float* ws_s, const int* start, const int* pos0,
-                       const int* slot, dim3 grid, int heads, int dk, int dv, int num_slots, int min_rows, int vec,
+                       const int* slot, const ChunkGrid& g, int heads, int dk, int dv, int num_slots, int vec,
                        hipStream_t s) {
   key_tiles(dk, [&](auto t) {
-    hipLaunchKernelGGL((chunk_out_kernel<T, decltype(t)::value>), grid, dim3(256), 0, s, o, in, ws_s, start, pos0, slot,
-                       heads, dk, dv, num_slots, min_rows, vec);
+    hipLaunchKernelGGL((chunk_out_kernel<T, decltype(t)::value>), g.grid((long)heads * ((dv + 63) / 64)), dim3(256), 0, s, o, in,
+                       ws_s, start, pos0, slot, heads, dk, dv, num_slots, g.steps, vec);
   });
 }
 
 extern "C" int mx_retention_chunks(float* o, const void* p, int bf16, long stride, const float* table, int table_rows,
                                    int rot_dims, int interleaved, const double* log_decay, float* state, float* ws_s,
-                                   const int* start, const int* pos0, const int* slot, int num_segs, int max_rows,
+                                   const int* start, const int* pos0, const int* slot, long rows, int num_segs, int max_rows,
                                    int heads, int dk, int dv, int num_slots, int min_rows, hipStream_t s) {
   if (num_segs <= 0 || max_rows < min_rows) return 0;
   if (dk < 1 || dk > mx_chunk_max_dk() || dv < 1 || heads < 1 || min_rows < 1) return -1;
@@ -460,15 +465,16 @@ extern "C" int mx_retention_chunks(float* o, const void* p, int bf16, long strid
   in.table_rows = table_rows; in.rot_dims = rot_dims; in.interleaved = interleaved;
   in.k_scale = 1.0f / sqrtf((float)dk);
   const int vec = dk % 4 == 0 && dv % 4 == 0 && stride % 4 == 0 && ((uintptr_t)p) % (4 * es) == 0;
-  const dim3 grid((max_rows + kC - 1) / kC, heads * ((dv + 63) / 64), num_segs);
-  if (grid.y > 65535 || grid.z > 65535) return -2;
+  const ChunkGrid g(rows, max_rows, min_rows, num_segs);
+  const long units = (long)heads * ((dv + 63) / 64);
+  if (!g.fits(units)) return -2;
   MX_DISPATCH_T(bf16, key_tiles(dk, [&](auto t) {
-    hipLaunchKernelGGL((state_add_kernel<T, decltype(t)::value>), grid, dim3(256), 0, s, ws_s, nullptr, in, start, pos0,
-                       slot, heads, dk, dv, num_slots, min_rows, vec);
+    hipLaunchKernelGGL((state_add_kernel<T, decltype(t)::value>), g.grid(units), dim3(256), 0, s, ws_s, nullptr, in, start, pos0,
+                       slot, heads, dk, dv, num_slots, g.steps, vec);
   }));
-  hipLaunchKernelGGL(state_carry_kernel, dim3((dk * dv + 255) / 256, heads, num_segs), dim3(256), 0, s, ws_s, log_decay,
-                     nullptr, state, start, pos0, slot, heads, dk * dv, num_slots, min_rows);
-  MX_DISPATCH_T(bf16, (launch_out<T>(o, in, ws_s, start, pos0, slot, grid, heads, dk, dv, num_slots, min_rows, vec, s)));
+  hipLaunchKernelGGL(state_carry_kernel, dim3((dk * dv + 255) / 256, heads, g.longs), dim3(256), 0, s, ws_s, log_decay,
+                     nullptr, state, start, pos0, slot, heads, dk * dv, num_slots, g.steps);
+  MX_DISPATCH_T(bf16, (launch_out<T>(o, in, ws_s, start, pos0, slot, g, heads, dk, dv, num_slots, vec, s)));
   return (int)hipGetLastError();
 }
 
@@ -508,24 +514,25 @@ extern "C" int mx_ssd_chunks(float* y, const void* xbc, int bf16, long stride, c
   in.skip = d_skip;
   in.k_scale = 1.f;
   const int vec = n % 4 == 0 && dv % 4 == 0 && stride % 4 == 0 && ((uintptr_t)xbc) % (4 * es) == 0;
-  const dim3 grid((max_rows + kC - 1) / kC, heads * ((dv + 63) / 64), num_segs);
-  if (grid.y > 65535 || grid.z > 65535) return -2;
+  const ChunkGrid g(rows, max_rows, min_rows, num_segs);
+  const long units = (long)heads * ((dv + 63) / 64);
+  if (!g.fits(units)) return -2;
   MX_DISPATCH_T(bf16, hipLaunchKernelGGL((ssd_steps_kernel<T>), dim3((unsigned)((rows * heads + 255) / 256)), dim3(256),
                                          0, s, ws_h, ws_h + rows * heads, (const T*)dt, dt_stride, a_log, dt_bias, rows,
                                          heads));
   MX_DISPATCH_T(bf16, key_tiles(n, [&](auto t) {
-    hipLaunchKernelGGL((state_add_kernel<T, decltype(t)::value>), grid, dim3(256), 0, s, ws_s, ws_g, in, start, pos0,
-                       slot, heads, n, dv, num_slots, min_rows, vec);
+    hipLaunchKernelGGL((state_add_kernel<T, decltype(t)::value>), g.grid(units), dim3(256), 0, s, ws_s, ws_g, in, start, pos0,
+                       slot, heads, n, dv, num_slots, g.steps, vec);
   }));
-  hipLaunchKernelGGL(state_carry_kernel, dim3((n * dv + 255) / 256, heads, num_segs), dim3(256), 0, s, ws_s, nullptr,
-                     ws_g, state, start, pos0, slot, heads, n * dv, num_slots, min_rows);
-  MX_DISPATCH_T(bf16, (launch_out<T>(y, in, ws_s, start, pos0, slot, grid, heads, n, dv, num_slots, min_rows, vec, s)));
+  hipLaunchKernelGGL(state_carry_kernel, dim3((n * dv + 255) / 256, heads, g.longs), dim3(256), 0, s, ws_s, nullptr,
+                     ws_g, state, start, pos0, slot, heads, n * dv, num_slots, g.steps);
+  MX_DISPATCH_T(bf16, (launch_out<T>(y, in, ws_s, start, pos0, slot, g, heads, n, dv, num_slots, vec, s)));
   return (int)hipGetLastError();
 }
 
 extern "C" int mx_head_delta_chunks(float* o, const float* q, const float* k, const float* v, const float* lg,
                                     const float* beta, float* state, float* ws_s, float* ws_w, float* ws_k, float* ws_u,
-                                    float* ws_g, const int* start, const int* pos0, const int* slot, int num_segs,
+                                    float* ws_g, const int* start, const int* pos0, const int* slot, long rows, int num_segs,
                                     int max_rows, int heads, int kv_heads, int dk, int dv, int num_slots, int min_rows,
                                     hipStream_t s) {
   if (num_segs <= 0 || max_rows < min_rows) return 0;
@@ -539,25 +546,24 @@ extern "C" int mx_head_delta_chunks(float* o, const float* q, const float* k, co
   in.k_scale = 1.f;
   const int vec = dk % 4 == 0 && dv % 4 == 0 && (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v) % 16) == 0;
   if (((uintptr_t)ws_w | (uintptr_t)ws_k | (uintptr_t)ws_u) % 16) return -3;
-  const int chunks = (max_rows + kC - 1) / kC;
-  if (heads > 65535 || (long)heads * ((dv + 63) / 64) > 65535 || num_segs > 65535) return -2;
+  const ChunkGrid g(rows, max_rows, min_rows, num_segs);
+  if (!g.fits((long)heads * ((dv + 63) / 64))) return -2;
   key_tiles(dk, [&](auto t) {
-    hipLaunchKernelGGL((delta_solve_kernel<decltype(t)::value>), dim3(chunks, heads, num_segs), dim3(256), 0, s, ws_w,
-                       ws_k, ws_u, ws_g, in, beta, start, pos0, slot, heads, dk, dv, num_slots, min_rows, vec);
+    hipLaunchKernelGGL((delta_solve_kernel<decltype(t)::value>), g.grid(heads), dim3(256), 0, s, ws_w,
+                       ws_k, ws_u, ws_g, in, beta, start, pos0, slot, heads, dk, dv, num_slots, g.steps, vec);
     constexpr int DKT = decltype(t)::value;
-    const dim3 cgrid(heads, (dv + 15) / 16, num_segs);
+    const dim3 cgrid(heads, (dv + 15) / 16, g.longs);
     if (dk == 16 * DKT && dv % 16 == 0)
       hipLaunchKernelGGL((chunk_carry_kernel<DKT, true, false, true, float>), cgrid, dim3(256), 0, s, ws_s, ws_w, ws_k,
                          ws_u, ws_g, (const float*)nullptr, 0L, state, start,
-                         pos0, slot, heads, dk, dv, num_slots, min_rows);
+                         pos0, slot, heads, dk, dv, num_slots, g.steps);
     else
       hipLaunchKernelGGL((chunk_carry_kernel<DKT, false, false, true, float>), cgrid, dim3(256), 0, s, ws_s, ws_w, ws_k,
                          ws_u, ws_g, (const float*)nullptr, 0L, state, start,
-                         pos0, slot, heads, dk, dv, num_slots, min_rows);
+                         pos0, slot, heads, dk, dv, num_slots, g.steps);
   });
   in.v = ws_u;                     // the solved rows take the values' place
   in.v_frags = 1;
-  launch_out<float>(o, in, ws_s, start, pos0, slot, dim3(chunks, heads * ((dv + 63) / 64), num_segs), heads, dk, dv,
-                    num_slots, min_rows, vec, s);
+  launch_out<float>(o, in, ws_s, start, pos0, slot, g, heads, dk, dv, num_slots, vec, s);
   return (int)hipGetLastError();
 }

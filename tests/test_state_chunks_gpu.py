@@ -52,7 +52,9 @@ def check(run, want_state, want, dv, monkeypatch):
     return got
 
 
-SHAPES = [([64], [0]), ([31, 32, 1, 65], [0, 5, 9, 0]), ([127, 200, 40], [64, 0, 3]), ([520], [0])]
+# (the last: workgroups that look for their segment among more than 64, a long one of padding rows)
+SHAPES = [([64], [0]), ([31, 32, 1, 65], [0, 5, 9, 0]), ([127, 200, 40], [64, 0, 3]), ([520], [0]),
+          ([40, 65] + [1] * 66 + [513], [0, 3] + [7] * 66 + [2])]
 
 
 @pytest.mark.parametrize("dt_", [torch.float32, torch.bfloat16])
