@@ -422,35 +422,63 @@ SSD_CHUNK_ROWS = 256
 NO_CHUNKS = 1 << 30
 
 
-def _chunk_counts(seg: Segments, rows: int):
-    """(chunks of 64 rows, rows) of the segments of at least ``rows`` rows."""
-    lens = [b - a for a, b in zip(seg.host[0][:-1], seg.host[0][1:]) if b - a >= rows]
-    return sum((n + 63) // 64 for n in lens), sum(lens)
+def _chunks_pay(seg: Segments, least: int, heads: int, dk: int, dv: int, cols: int, walk, launch: float, link: float,
+                short_entry: float, products) -> bool:
+    """Whether a step's segments of ``least`` rows or more run in chunks (and only the others in walks): by the time, us, of
+    both forms, fitted to 2238 steps of 1 to 65 segments, 1 to 128 heads of 8 x 8 to 128 x 256 (the form chosen takes 1.004 to
+    1.008 times the better one's time in the mean, 1.25 times or more in one step of a
+    hundred; the chunks' a tenth up, their fit is the coarser).
+    A walk takes a row after the other, ``cols`` state columns a workgroup and a few hundred workgroups at a time (``walk``:
+    launch, a row and more per dk, workgroups at a time and fewer per dk, a state's entry, a row's preparation per head).
+    Chunks take ``launch``, ``products`` (of chunks times heads, dk, tiles of 64 columns), ``link`` for each of the longest
+    segment's in the carry and, after the walk of the others, ``short_entry`` for an entry of those states."""
+    if seg.host is None or seg.max_rows < least:
+        return True
+    lens = [b - a for a, b in zip(seg.host[0][:-1], seg.host[0][1:])]
+    short = [n for n in lens if n < least]
+
+    def walked(lens):
+        begin, row, row_dk, room, room_dk, entry, prep = walk
+        busy = sum(lens) * heads * (-(-dv // cols)) / max(room - room_dk * dk, 50.0)
+        return begin + (row + row_dk * dk) * (max(lens) ** 4 + busy ** 4) ** 0.25 + \
+            heads * (entry * len(lens) * dk * dv + prep * sum(lens))
+
+    pad = 16 if dk <= 16 else 32 if dk <= 32 else 64 if dk <= 64 else 128
+    chunked = launch + link * ((max(lens) + 63) // 64) + \
+        products(heads * sum((n + 63) // 64 for n in lens if n >= least), pad, -(-dv // 64))
+    if short:
+        chunked += walked(short) + short_entry * heads * len(short) * dk * dv
+    return 1.1 * chunked <= walked(lens)
+
+
+def _turns(units: int, turn: int, share: float) -> float:
+    """``units`` workgroups, ``share`` of their time in whole turns of the chip."""
+    return (1 - share) * units + share * turn * -(-units // turn)
 
 
 def _delta_chunks_pay(seg: Segments, heads: int, dk: int, dv: int) -> bool:
-    """Many segments of narrow heads fill the chip with walks, whose work per row is the smaller one then.  us, chunks
-    (walks): 32 heads of 64 x 64, 16 and 64 segments of 100 rows 124 489 (113 403), 32 of 256 472 (497); of 16 x 32 79 264
-    (51 130), 266 (168); 16 heads of 128 x 128 135 554 (261 1057).  A row costs a walk r us, `slots` walks of 32 columns at
-    a time; a head's chunk c us of the chip."""
-    if seg.host is None or seg.max_rows < CHANNEL_CHUNK_ROWS:
-        return True
-    chunks, rows = _chunk_counts(seg, CHANNEL_CHUNK_ROWS)
-    r, slots, c = 0.2 + 0.0026 * dk, 480 - 1.75 * dk, 0.05 + 0.0005 * dk + 8.5e-6 * dk * dk
-    walked = rows * heads * ((dv + 31) // 32) / slots
-    return walked <= seg.max_rows or r * walked >= c * chunks * heads
+    """us, chunks (walks): 32 heads of 64 x 64, 16 and 64 segments of 100 rows 124 489 (113 403), 32 of 256 472 (497); of
+    16 x 32 79 264 (51 130), 266 (168); 16 heads of 128 x 128 135 554 (261 1057)."""
+    return _chunks_pay(seg, CHANNEL_CHUNK_ROWS, heads, dk, dv, 32, (7.0, 0.18, 0.0025, 940, 5.5, 1.8e-6, 6.4e-4), 11, 1.0,
+                       2.2e-6, lambda n, pad, tall: _turns(n, 256 if pad >= 64 else 512, 0.3) *
+                       (0.041 + 4.9e-6 * pad * pad + tall * (3.3e-4 * pad + 0.013)))
+
+
+def _linear_chunks_pay(seg: Segments, heads: int, dk: int, dv: int) -> bool:
+    """The same of linear attention: 128 heads of 64 x 16, 32 segments of 130 rows 625 (248); 128 of 8 x 8, 8 of 130 67 (44);
+    64 of 32 x 32 55 (44); 16 of 128 x 128, one of 200 43 (70); 4 of 64 x 128, two of 130 23 (36)."""
+    return _chunks_pay(seg, CHANNEL_CHUNK_ROWS, heads, dk, dv, 16, (5.6, 0.12, 0.0014, 600, 1.4, 5.2e-6, 1.3e-5), 10, 0.71,
+                       2.8e-6, lambda n, pad, tall: _turns(n, 256 if pad >= 64 else 512, 0.3) *
+                       (0.0068 + 3.1e-6 * pad * pad + tall * (2.8e-4 * pad + 0.0089)))
 
 
 def _ssd_chunks_pay(seg: Segments, heads: int, n: int, dv: int) -> bool:
-    """The same of the state-space scan, with walks of 16 columns and both forms' whole times, the chunk form's a tenth
-    up: 16 heads of 128 x 128, 32 segments of 256 rows 420 (388), four of 2000 370 (459), of 128 x 256, 4 heads, eight of
-    300 95 (78); 32 of 64 x 64 82 (74), 32 of 256 193 (201); of 16 x 32 99 (87)."""
-    if seg.host is None or seg.max_rows < SSD_CHUNK_ROWS:
-        return True
-    chunks, rows = _chunk_counts(seg, SSD_CHUNK_ROWS)
-    walked = rows * heads * ((dv + 15) // 16) / (900 - 2.6 * n)
-    chunked = (0.012 + 0.0006 * n) * ((dv + 63) // 64) * chunks * heads
-    return 1.1 * (12 + chunked) <= 12 + (0.127 + 0.00065 * n) * max(seg.max_rows, walked)
+    """The same of the state-space scan: 16 heads of 128 x 128, 32 segments of 256 rows 420 (388), four of 2000 370 (459), one
+    of 300 beside 64 decode rows 120 (86); of 128 x 256, 4 heads, eight of 300 95 (78); 32 of 64 x 64 82 (74), 32 of 256
+    193 (201); of 16 x 32 99 (87); 128 heads of 16 x 32, one of 3000 beside 64 decode rows 187 (436)."""
+    return _chunks_pay(seg, SSD_CHUNK_ROWS, heads, n, dv, 16, (5.0, 0.13, 5.7e-4, 1100, 4.3, 1.2e-6, 0), 14, 0.28,
+                       3.1e-6, lambda n, pad, tall: _turns(n * tall, 512 if pad >= 64 else 768, 0.42) *
+                       (0.015 + 2.4e-4 * pad + 2e-6 * pad * pad))
 
 
 def head_delta_rule(q, k, v, log_decay, beta, state, seg: Segments) -> torch.Tensor:
@@ -503,9 +531,10 @@ def gated_linear_attention(qkv, a, a_bias, tau: float, state, seg: Segments, hea
     Returns o fp32 [T, heads*dv]."""
     if qkv.is_cuda:
         o = torch.empty(qkv.shape[0], heads * dv, dtype=torch.float32, device=qkv.device)
+        chunk = CHANNEL_CHUNK_ROWS if _linear_chunks_pay(seg, heads, dk, dv) else NO_CHUNKS
         native_mixers().gated_linear_attention(o, qkv, a, a_bias, float(tau), state, seg.start, seg.pos0,
                                                seg.slot, seg.num, seg.max_rows, heads, dk, dv,
-                                               _walk_below(seg, CHANNEL_CHUNK_ROWS), CHANNEL_CHUNK_ROWS)
+                                               _walk_below(seg, chunk), chunk)
         return o
     return ref.gated_linear_attention(qkv, a, a_bias, tau, state, seg, heads, dk, dv)
 

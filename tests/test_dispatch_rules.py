@@ -98,3 +98,20 @@ def test_delta_rule_of_long_segments(heads, dk, dv, lens, chunks, walks):
 def test_state_space_scan_of_long_segments(heads, n, dv, lens, chunks, walks):
     taken = chunks if M._ssd_chunks_pay(unlike(lens), heads, n, dv) else walks
     assert taken <= 1.1 * min(chunks, walks)
+
+
+@pytest.mark.parametrize("heads,dk,dv,lens,chunks,walks", [
+    (128, 64, 16, [130] * 32, 625, 248), (128, 64, 8, [200] * 16, 414, 188), (128, 32, 8, [130] * 16, 159, 78),
+    (64, 128, 64, [1000] + [100] * 10, 261, 428), (32, 64, 64, [1000] + [1] * 64, 122, 254), (4, 64, 128, [130] * 2, 23, 36),
+    (16, 128, 32, [100] + [1] * 64, 72, 48), (64, 32, 64, [900] * 8, 288, 481), (16, 128, 128, [200], 43, 70)])
+def test_linear_attention_of_long_segments(heads, dk, dv, lens, chunks, walks):
+    taken = chunks if M._linear_chunks_pay(unlike(lens), heads, dk, dv) else walks
+    assert taken <= 1.1 * min(chunks, walks)
+
+
+@pytest.mark.parametrize("rule,heads,dk,dv,lens,chunks,walks", [
+    (M._delta_chunks_pay, 64, 128, 64, [1000] + [100] * 10, 436, 688), (M._delta_chunks_pay, 16, 64, 128, [100] + [1] * 64, 72, 47),
+    (M._delta_chunks_pay, 32, 64, 64, [1000] + [1] * 64, 133, 364), (M._ssd_chunks_pay, 16, 128, 128, [300] + [1] * 64, 120, 86),
+    (M._ssd_chunks_pay, 128, 16, 32, [3000] + [1] * 64, 187, 436), (M._ssd_chunks_pay, 32, 64, 64, [1000] + [1] * 64, 84, 174)])
+def test_prompts_beside_short_segments(rule, heads, dk, dv, lens, chunks, walks):
+    assert (chunks if rule(unlike(lens), heads, dk, dv) else walks) <= 1.1 * min(chunks, walks)

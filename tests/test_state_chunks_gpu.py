@@ -37,6 +37,7 @@ def walk(seg, state, step):
 
 def check(run, want_state, want, dv, monkeypatch):
     """run() -> (outputs, states), once in chunk form and once row by row."""
+    monkeypatch.setattr(M, "_chunks_pay", lambda *a: True)
     both = []
     for rows in (32, 1 << 30):
         monkeypatch.setattr(M, "CHANNEL_CHUNK_ROWS", rows)
@@ -207,6 +208,7 @@ def test_state_space_forgets_at_once(first, monkeypatch):
     xbc = torch.randn(T, heads * dv + 2 * n, generator=g).to(DEV)
     dt, bias, skip = torch.randn(T, heads, generator=g).to(DEV), torch.zeros(heads, device=DEV), torch.ones(heads, device=DEV)
     a_log, s0 = torch.tensor([first, 0.0], device=DEV), torch.randn(1, heads, n, dv, generator=g).to(DEV)
+    monkeypatch.setattr(M, "_chunks_pay", lambda *a: True)
     out = []
     for rows in (64, 1 << 30):
         monkeypatch.setattr(M, "SSD_CHUNK_ROWS", rows)
