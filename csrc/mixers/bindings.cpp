@@ -831,6 +831,20 @@ void latent_attention(Tensor out, Tensor qa, Tensor qr, Tensor cache, Tensor sta
     int64_t rows = std::max<int64_t>(1, std::min<int64_t>(t, num_segs * std::max<int64_t>(1, std::min(max_rows, skip_from > 0 ? skip_from - 1 : max_rows))));
     const bool units = mx_latent_decode_fits((int)rank, (int)dr, bf(cache)) != 0;
     int64_t splits = std::max<int64_t>(1, std::min<int64_t>(units ? 32 : 16, (units ? 512 : 256) / rows));
+    if (units && heads > 16 && splits > 1) {
+      // a workgroup per 16 heads and one a CU (its LDS), empty slices' too: as many slices as the fewest turns of the 256
+      // CUs hold that they fill to nine tenths.  us without / so, no context known: 128 heads, 64 rows of 20 keys 119 28 (the
+      // general kernel 105), of 600 174 89, of 4000 527 475; 40 heads, 64 rows of 20 49 29, of 4000 204 194
+      const int64_t wgs = rows * ((heads + 15) / 16);
+      int64_t best = 1;
+      double filled = 0;
+      for (int64_t turns = 1, s = 0; s < splits && filled < 0.9; ++turns) {
+        s = std::min(splits, turns * 256 / wgs);
+        const double f = (double)(s * wgs) / (double)((s * wgs + 255) / 256 * 256);
+        if (s > 0 && f > filled) best = s, filled = f;
+      }
+      splits = best;
+    }
     if (max_kv > 0) splits = std::max<int64_t>(1, std::min(splits, (max_kv + 63) / 64));
     while (splits > 1 && t * splits * heads * rank * 4 > (256LL << 20)) splits /= 2;
     auto f32 = qa.options();
