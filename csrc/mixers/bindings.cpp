@@ -1338,7 +1338,10 @@ void ssd_scan(Tensor y, Tensor xbc, Tensor dt, Tensor a_log, Tensor dt_bias, Ten
   check_segs(start, pos0, slot, num_segs);
   TORCH_CHECK(chunk_from >= 1, "state-space rows");
   max_rows = std::min(max_rows, t);     // (a bound may be given)
-  if (max_rows == 1 && mx_state_step_fits(y.data_ptr<float>(), state.data_ptr<float>(), (int)n, (int)dv)) {
+  // (states so small that most of the step's threads have no entry stay with the walk: 128 heads of 24 x 16, 256 rows 64 us,
+  // 54 so; of 64 x 8, 32 x 16 or 8 x 32 the step is about level, beyond faster)
+  if (max_rows == 1 && (n * dv > 512 || dv >= 32) &&
+      mx_state_step_fits(y.data_ptr<float>(), state.data_ptr<float>(), (int)n, (int)dv)) {
     chk(mx_state_step(2, y.data_ptr<float>(), xbc.data_ptr(), bf(xbc), xbc.stride(0), dt.data_ptr(), dt.stride(0), nullptr,
                       0, a_log.data_ptr<float>(), dt_bias.data_ptr<float>(), d_skip.data_ptr<float>(), 0.f,
                       state.data_ptr<float>(), start.data_ptr<int>(), pos0.data_ptr<int>(), slot.data_ptr<int>(),
