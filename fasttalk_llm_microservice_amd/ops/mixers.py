@@ -692,9 +692,9 @@ def latent_attention_products(out, qa, qr, cache, seg: Segments, scale: float, r
     heads = qa.shape[0]
     bs = cache.shape[1]
     width = cache.shape[2]
-    if latent_prefill_ok(qa, cache, rank, dtype) and qa.dtype == qr.dtype == out.dtype == torch.float32 \
-            and _plain16(out, qa, qr, cache) and _device_segments(seg) \
-            and _latent_prefill_pays(seg, heads, min_rows):
+    if latent_prefill_ok(qa, cache, rank, dtype) and _latent_prefill_pays(seg, heads, min_rows) \
+            and qa.dtype == qr.dtype == out.dtype == torch.float32 \
+            and _plain16(out, qa, qr, cache) and _device_segments(seg):
         ns = [n for n in (b - a for a, b in zip(start[:-1], start[1:])) if n >= min_rows]
         native_mixers().latent_prefill(out, qa, qr, cache, seg.start, seg.pos0, seg.kv_len, seg.block_tables, seg.num,
                                        len(ns), sum(ns), float(scale), rank, min_rows, sink)
