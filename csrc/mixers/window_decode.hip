@@ -4,17 +4,18 @@
 // fp32 queries and weights stay fp32: each is the exact sum of three bf16 parts, keys and values are bf16 already,
 // so three v_mfma_f32_16x16x32_bf16 per operand pair form the products of an fp32 multiply, summed in fp32.
 //
-// A workgroup owns one row and one key head (and score map) with the up to 16 query heads that share it; its eight
-// waves take 32 keys in turn, so a key is read once for all its heads.  S^T = K Q^T and O^T = V^T P^T, a column
+// A workgroup owns one row and one key head (and score map) with the up to 16 query heads that share it; its waves
+// (eight, fewer where there are many groups) take 32 keys in turn, so a key is read once for all its heads.  S^T = K Q^T and O^T = V^T P^T, a column
 // per head: keys go straight from memory to operands, values through a wave's own LDS strip (ds_read_b64_tr_b16),
 // and weights need no exchange.  The next 32 keys load under the softmax and the sums.  The waves' (maximum, sum,
 // sums) meet in LDS at the end: one launch, whatever the length.
 // Bound by a wave's chain for few rows, by the read of the keys for many.  In running models, 16 heads of 128 on 4
 // key heads: one row, 900 keys in a block of 1024 or with a table 25 us (general kernel, a workgroup per head: 50),
-// 540 keys with sigmoid weights 18 (33), two maps of 64 16 (33); 32 rows of 540 24 (56).  A row takes 7.8 us however few its
-// keys (general kernel: 5.8 with one, 6.3 with ten, 9.4 with a hundred), and one query head a key head wastes fifteen
-// columns of sixteen: 64 rows of 16 such heads 32 us at 100 keys (19), 139 at 1000 (158), 385 at 8000 (545).  Lengths are not
-// known on the host where a step is replayed, so sizes alone choose.
+// 540 keys with sigmoid weights 18 (33), two maps of 64 16 (33); 32 rows of 540 24 (56).  With the keys in the L2 a row takes
+// 7.7 to 9.3 us however few they are (general kernel: 6 to 7 with one, 10 with a hundred), and one query head a key head
+// wastes fifteen columns of sixteen: 64 rows of 16 such heads 18 us at 100 keys (20), 162 at 1500 (228), 600 at 6000 (823).
+// (Eight waves for all of them and a merge that read every wave's part, an entry a thread: 32 at 100 keys; 16 heads a
+// group, one key: 12.4, now 9.3.)  Lengths are not known on the host where a step is replayed, so sizes alone choose.
 #include "mx_common.h"
 
 namespace mx {
@@ -49,15 +50,15 @@ __device__ __forceinline__ wd_f32x4 wd_mfma(const uint4& a, const uint4& b, wd_f
                                                  0, 0, 0);
 }
 
-constexpr int kWdWaves = 8, kWdKeys = 32, kWdMaxRep = 16;
+constexpr int kWdKeys = 32, kWdMaxRep = 16;
 
-template <int DK, int DV>
-__global__ void __launch_bounds__(64 * kWdWaves, 2)
+template <int DK, int DV, int WV>
+__global__ void __launch_bounds__(64 * WV, 2)
 window_decode_kernel(WindowArgs A) {
   constexpr int KS = DK / 32, DT = DV / 16, PV = DV / 8, VL = kWdKeys * PV / 64;
   constexpr int kStrip = kWdKeys * DV * 2, kMerge = kWdMaxRep * DV * 4;      // bytes per wave
-  __shared__ __attribute__((aligned(16))) uint8_t lds[kWdWaves * (kStrip > kMerge ? kStrip : kMerge)];
-  __shared__ float ml[kWdWaves][2][kWdMaxRep];
+  __shared__ __attribute__((aligned(16))) uint8_t lds[WV * (kStrip > kMerge ? kStrip : kMerge)];
+  __shared__ float ml[WV][2][kWdMaxRep];
   const int row = blockIdx.x, gk = blockIdx.y;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 15, g4 = lane >> 4;
@@ -80,7 +81,7 @@ window_decode_kernel(WindowArgs A) {
     return blk >= 0 && blk < A.num_blocks ? blk * A.block_size + j % A.block_size : -1;
   };
   uint4 k[2][KS], v[VL];
-  constexpr int kStep = kWdWaves * kWdKeys;
+  constexpr int kStep = WV * kWdKeys;
   auto look = [&](int c0, int (&slot)[2]) {    // lane n of each group: keys n and 16 + n
 #pragma unroll
     for (int t = 0; t < 2; ++t) slot[t] = slot_of(c0 + 16 * t + n);
@@ -214,30 +215,32 @@ window_decode_kernel(WindowArgs A) {
   }
   // the waves' parts
   __syncthreads();
+  const int waves = max(1, min(WV, (nkeys + kWdKeys - 1) / kWdKeys));       // that have seen a key
   l_ = ft::kgroups_sum(l_);
   float* mine = reinterpret_cast<float*>(lds) + (long)wave * rep * DV;
-  if (n < rep) {
+  if (n < rep && wave < waves) {
 #pragma unroll
     for (int t = 0; t < DT; ++t)
       *reinterpret_cast<float4*>(mine + n * DV + 16 * t + 4 * g4) = make_float4(o[t][0], o[t][1], o[t][2], o[t][3]);
     if (g4 == 0) ml[wave][0][n] = mx_, ml[wave][1][n] = l_;
   }
   __syncthreads();
-  for (int e = tid; e < rep * DV; e += 64 * kWdWaves) {
-    const int h = e / DV;
-    float top = -INFINITY, l = 0.f, y = 0.f;
-#pragma unroll
-    for (int w = 0; w < kWdWaves; ++w) top = fmaxf(top, ml[w][0][h]);
-#pragma unroll
-    for (int w = 0; w < kWdWaves; ++w) {
+  const float4* parts = reinterpret_cast<const float4*>(lds);
+  for (int e = tid; e < rep * (DV / 4); e += 64 * WV) {
+    const int h = e / (DV / 4);
+    float top = -INFINITY, l = 0.f;
+    float4 y = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int w = 0; w < waves; ++w) top = fmaxf(top, ml[w][0][h]);
+    for (int w = 0; w < waves; ++w) {
       const float f = A.sigmoid ? 1.f : ml[w][0][h] == -INFINITY ? 0.f : expf(ml[w][0][h] - top);
+      const float4 p = parts[w * rep * (DV / 4) + e];
       l += f * ml[w][1][h];
-      y += f * reinterpret_cast<const float*>(lds)[(long)w * rep * DV + e];
+      y.x += f * p.x, y.y += f * p.y, y.z += f * p.z, y.w += f * p.w;
     }
-    y = A.sigmoid ? y : l > 0.f ? y / l : 0.f;
-    const long at = ((long)row * hq + (kvh * rep + h) * A.maps + map) * DV + e % DV;
-    if (A.out_bf16) st((bf16_t*)A.out, at, y);
-    else ((float*)A.out)[at] = y;
+    if (!A.sigmoid) y = l > 0.f ? make_float4(y.x / l, y.y / l, y.z / l, y.w / l) : make_float4(0.f, 0.f, 0.f, 0.f);
+    const long at = ((long)row * hq + (kvh * rep + h) * A.maps + map) * DV + 4 * (e % (DV / 4));
+    if (A.out_bf16) *reinterpret_cast<uint2*>((bf16_t*)A.out + at) = make_uint2(ft::pack2(y.x, y.y), ft::pack2(y.z, y.w));
+    else *reinterpret_cast<float4*>((float*)A.out + at) = y;
   }
 }
 
@@ -265,10 +268,24 @@ extern "C" int mx_window_decode(void* out, int out_bf16, const float* q, const v
   const WindowArgs A{out, out_bf16, q, (const bf16_t*)k_cache, (const bf16_t*)v_cache, start, pos0, kv_len, bt, bt_stride, num_segs,
                      heads, maps, kv_heads, window, scale, sigmoid, r1, r2, pb, block_size, num_blocks, skip_from, softcap,
                      has_sink, sink, sinks, blocks, keep_first, dist_bias, nd};
-  const dim3 grid((unsigned)total_rows, (unsigned)(kv_heads * maps)), block(64 * kWdWaves);
-  if (dk == 128 && dv == 128) hipLaunchKernelGGL((window_decode_kernel<128, 128>), grid, block, 0, s, A);
-  else if (dk == 64 && dv == 128) hipLaunchKernelGGL((window_decode_kernel<64, 128>), grid, block, 0, s, A);
-  else if (dk == 128) hipLaunchKernelGGL((window_decode_kernel<128, 64>), grid, block, 0, s, A);
-  else hipLaunchKernelGGL((window_decode_kernel<64, 64>), grid, block, 0, s, A);
+  const long groups = total_rows * kv_heads * maps;
+  const dim3 grid((unsigned)total_rows, (unsigned)(kv_heads * maps));
+  // eight waves are a CU's registers: fewer share a group's keys where that leaves groups waiting.  us with 8 / 4 / 2 waves,
+  // 16 heads of 128 with a key head each: 64 rows (1024 groups) of 30 keys 27 15 9, of 300 56 42 34, of 1500 178 173 155; 32
+  // rows (512) of 20 15 9 9, of 600 41 34 47; 4 key heads, 64 rows (256) of 30 9 9 9, of 400 20 23 30, of 6000 161 226 331
+  const int wv = groups <= 256 ? 8 : groups <= 512 ? 4 : 2;
+#define WD_WAVES(DK, DV, WV) hipLaunchKernelGGL((window_decode_kernel<DK, DV, WV>), grid, dim3(64 * WV), 0, s, A)
+#define WD_GO(DK, DV)                     \
+  do {                                    \
+    if (wv == 8) WD_WAVES(DK, DV, 8);     \
+    else if (wv == 4) WD_WAVES(DK, DV, 4); \
+    else WD_WAVES(DK, DV, 2);             \
+  } while (0)
+  if (dk == 128 && dv == 128) WD_GO(128, 128);
+  else if (dk == 64 && dv == 128) WD_GO(64, 128);
+  else if (dk == 128) WD_GO(128, 64);
+  else WD_GO(64, 64);
+#undef WD_GO
+#undef WD_WAVES
   return (int)hipGetLastError();
 }

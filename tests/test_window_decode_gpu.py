@@ -22,6 +22,9 @@ def cases():
     yield "sigmoid, distance", f(2, 1, 128, 128, 150), dict(sigmoid=True, terms=True), [1, 1], [31, 400]
     yield "sink per head, one key head each", f(2, 2, 128, 128, 33), dict(sinks=True), [1, 7], [640, 0]
     yield "sixteen heads, cap, sink per head", f(32, 2, 128, 128, 200), dict(softcap=8.0, sinks=True, keep_first=3), [1, 2], [450, 31]
+    many = lambda n: [(37 * i) % 290 + (i == 5) for i in range(n)]   # noqa: E731
+    yield "many groups (four waves)", f(16, 8, 128, 128, 0), dict(sinks=True, softcap=20.0), [1] * 33, many(33)
+    yield "many groups (two waves)", f(8, 8, 64, 128, 0), dict(table=40), [1] * 60 + [3, 2], many(62)
     yield "seventeen heads a group (general kernel)", f(17, 1, 64, 64, 0), {}, [1], [300]
 
 
