@@ -18,6 +18,8 @@
 // group, one key: 12.4, now 9.3.)  Lengths are not known on the host where a step is replayed, so sizes alone choose.
 #include "mx_common.h"
 
+#include <type_traits>
+
 namespace mx {
 
 typedef __bf16 wd_bf16x8 __attribute__((ext_vector_type(8)));
@@ -225,22 +227,45 @@ window_decode_kernel(WindowArgs A) {
     if (g4 == 0) ml[wave][0][n] = mx_, ml[wave][1][n] = l_;
   }
   __syncthreads();
-  const float4* parts = reinterpret_cast<const float4*>(lds);
-  for (int e = tid; e < rep * (DV / 4); e += 64 * WV) {
-    const int h = e / (DV / 4);
-    float top = -INFINITY, l = 0.f;
-    float4 y = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int w = 0; w < waves; ++w) top = fmaxf(top, ml[w][0][h]);
-    for (int w = 0; w < waves; ++w) {
-      const float f = A.sigmoid ? 1.f : ml[w][0][h] == -INFINITY ? 0.f : expf(ml[w][0][h] - top);
-      const float4 p = parts[w * rep * (DV / 4) + e];
-      l += f * ml[w][1][h];
-      y.x += f * p.x, y.y += f * p.y, y.z += f * p.z, y.w += f * p.w;
+  // (all of the waves: a constant, every read in flight; four columns a thread where the entries are more than the threads)
+  auto merge = [&](auto count, auto cols) {
+    constexpr int C = decltype(cols)::value;
+    for (int e = tid; e < rep * (DV / C); e += 64 * WV) {
+      const int h = e / (DV / C);
+      float top = -INFINITY, l = 0.f, y[C];
+#pragma unroll
+      for (int c = 0; c < C; ++c) y[c] = 0.f;
+#pragma unroll
+      for (int w = 0; w < count; ++w) top = fmaxf(top, ml[w][0][h]);
+#pragma unroll
+      for (int w = 0; w < count; ++w) {
+        const float f = A.sigmoid ? 1.f : ml[w][0][h] == -INFINITY ? 0.f : expf(ml[w][0][h] - top);
+        const float* p = reinterpret_cast<const float*>(lds) + (long)w * rep * DV + e * C;
+        l += f * ml[w][1][h];
+#pragma unroll
+        for (int c = 0; c < C; ++c) y[c] += f * p[c];
+      }
+#pragma unroll
+      for (int c = 0; c < C; ++c) y[c] = A.sigmoid ? y[c] : l > 0.f ? y[c] / l : 0.f;
+      const long at = ((long)row * hq + (kvh * rep + h) * A.maps + map) * DV + C * (e % (DV / C));
+      if constexpr (C == 4) {
+        if (A.out_bf16) *reinterpret_cast<uint2*>((bf16_t*)A.out + at) = make_uint2(ft::pack2(y[0], y[1]), ft::pack2(y[2], y[3]));
+        else *reinterpret_cast<float4*>((float*)A.out + at) = make_float4(y[0], y[1], y[2], y[3]);
+      } else {
+        if (A.out_bf16) st((bf16_t*)A.out, at, y[0]);
+        else ((float*)A.out)[at] = y[0];
+      }
     }
-    if (!A.sigmoid) y = l > 0.f ? make_float4(y.x / l, y.y / l, y.z / l, y.w / l) : make_float4(0.f, 0.f, 0.f, 0.f);
-    const long at = ((long)row * hq + (kvh * rep + h) * A.maps + map) * DV + 4 * (e % (DV / 4));
-    if (A.out_bf16) *reinterpret_cast<uint2*>((bf16_t*)A.out + at) = make_uint2(ft::pack2(y.x, y.y), ft::pack2(y.z, y.w));
-    else *reinterpret_cast<float4*>((float*)A.out + at) = y;
+  };
+  const std::integral_constant<int, 1> one;
+  const std::integral_constant<int, 4> four;
+  const std::integral_constant<int, WV> all;
+  if (rep * DV > 64 * WV) {
+    if (waves == WV) merge(all, four);
+    else merge(waves, four);
+  } else {
+    if (waves == WV) merge(all, one);
+    else merge(waves, one);
   }
 }
 
