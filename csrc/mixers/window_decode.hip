@@ -5,10 +5,10 @@
 // so three v_mfma_f32_16x16x32_bf16 per operand pair form the products of an fp32 multiply, summed in fp32.
 //
 // A workgroup owns one row and one key head (and score map) with the up to 16 query heads that share it; its waves
-// (eight, fewer where there are many groups) take 32 keys in turn, so a key is read once for all its heads.  S^T = K Q^T and O^T = V^T P^T, a column
-// per head: keys go straight from memory to operands, values through a wave's own LDS strip (ds_read_b64_tr_b16),
-// and weights need no exchange.  The next 32 keys load under the softmax and the sums.  The waves' (maximum, sum,
-// sums) meet in LDS at the end: one launch, whatever the length.
+// (eight, fewer where there are many groups) take 32 keys in turn, so a key is read once for all its heads.
+// S^T = K Q^T and O^T = V^T P^T, a column per head: keys go straight from memory to operands, values through a wave's
+// own LDS strip (ds_read_b64_tr_b16), and weights need no exchange.  The next 32 keys load under the softmax and the
+// sums.  The waves' (maximum, sum, sums) meet in LDS at the end: one launch, whatever the length.
 // Bound by a wave's chain for few rows, by the read of the keys for many.  In running models, 16 heads of 128 on 4
 // key heads: one row, 900 keys in a block of 1024 or with a table 25 us (general kernel, a workgroup per head: 50),
 // 540 keys with sigmoid weights 18 (33), two maps of 64 16 (33); 32 rows of 540 24 (56).  With the keys in the L2 a row takes
