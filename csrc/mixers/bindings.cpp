@@ -15,8 +15,13 @@ int mx_embed_rows(float* out, const int* ids, const void* table, int bf16, int r
 int mx_layer_norm(float* x, const void* y, int y_bf16, long y_stride, const float* w, const float* b, void* out,
                   void* cast, int out_bf16, int rows, int width, float eps, hipStream_t s);
 int mx_tanh_cap(float* x, long n, float cap, hipStream_t s);
-int mx_grouped_gemm(void* C, const void* A, const int* rows, const void* W, const int* offs, int groups, long M, int N,
-                    int K, int act, float limit, hipStream_t s);
+int mx_grouped_gemm(void* C, const void* A, long a_rows, const int* rows, const void* W, const int* offs, int groups, long M,
+                    int N, int K, int act, float limit, hipStream_t s);
+int mx_tile_gemm_fits(long M, int N, int K, long a_stride, int glu);
+float mx_tile_gemm_us(long M, int N, int K, int glu);
+int mx_tile_gemm(void* C, long c_stride, const void* A, long a_stride, long a_rows, const int* rows, const void* W,
+                 const void* bias, const int* offs, int groups, long M, int N, int K, int act, float limit, int form,
+                 hipStream_t s);
 int mx_pair_sort(int* offs, int* sorted_row, int* place, const int* idx, long rows, int top, int experts, hipStream_t s);
 int mx_experts_merge(float* out, const void* d, const int* place, const float* wts, const void* shared, const void* h,
                      long h_stride, const void* gate_w, long rows, int top, int width, hipStream_t s);
@@ -407,7 +412,7 @@ void grouped_gemm(Tensor out, Tensor a, Tensor w, Tensor offs) {
   TORCH_CHECK(out.is_cuda() && out.is_contiguous() && out.scalar_type() == at::kBFloat16 && out.dim() == 2 &&
               out.size(0) == a.size(0) && out.size(1) == w.size(1), "out: bf16 [M, N]");
   TORCH_CHECK(a.size(1) % 8 == 0 && a.size(1) >= 8, "K must be a multiple of 8");
-  chk(mx_grouped_gemm(out.data_ptr(), a.data_ptr(), nullptr, w.data_ptr(), offs.data_ptr<int>(), (int)w.size(0),
+  chk(mx_grouped_gemm(out.data_ptr(), a.data_ptr(), a.size(0), nullptr, w.data_ptr(), offs.data_ptr<int>(), (int)w.size(0),
                       a.size(0), (int)w.size(1), (int)a.size(1), 0, 0.f, stream()), "grouped_gemm");
 }
 
@@ -1021,6 +1026,27 @@ void experts_few(Tensor out, Tensor h, Tensor idx, Tensor wts, Tensor wgu, Tenso
                      (float)shared_limit, stream()), "experts_few");
 }
 
+double tile_gemm_us(int64_t rows, int64_t n, int64_t k, bool glu) { return mx_tile_gemm_us(rows, (int)n, (int)k, glu); }
+
+// form: one of tile_gemm.hip's, or below 0 the one that it takes by itself
+void tile_gemm(Tensor y, Tensor x, Tensor w, OptT bias, int64_t act, double limit, int64_t form) {
+  check_rows(x, "x");
+  check_rows(y, "y");
+  const bool glu = act >= 1 && act <= 4;
+  TORCH_CHECK(x.scalar_type() == at::kBFloat16 && y.scalar_type() == at::kBFloat16 && w.is_cuda() &&
+              w.scalar_type() == at::kBFloat16 && w.dim() == 2 && w.is_contiguous() && x.size(1) == w.size(1) && act >= 0 &&
+              act <= 5, "tile_gemm: bf16 rows and weights");
+  TORCH_CHECK(y.size(0) == x.size(0) && y.size(1) * (glu ? 2 : 1) == w.size(0) && x.size(0) <= 0x3fffffff, "tile_gemm: shapes");
+  if (x.size(0) == 0 || y.size(1) == 0) return;
+  TORCH_CHECK(mx_tile_gemm_fits(x.size(0), (int)y.size(1), (int)x.size(1), x.stride(0), glu), "tile_gemm: sizes");
+  if (bias)
+    TORCH_CHECK(bias->is_cuda() && bias->scalar_type() == at::kBFloat16 && bias->is_contiguous() &&
+                bias->numel() == w.size(0), "tile_gemm: bias");
+  chk(mx_tile_gemm(y.data_ptr(), y.stride(0), x.data_ptr(), x.stride(0), x.size(0), nullptr, w.data_ptr(),
+                   bias ? bias->data_ptr() : nullptr, nullptr, 1, x.size(0), (int)y.size(1), (int)x.size(1), (int)act,
+                   (float)limit, (int)form, stream()), "tile_gemm");
+}
+
 void experts_many(Tensor out, Tensor h, Tensor idx, Tensor wts, Tensor wgu, Tensor wdown, double limit, int64_t act,
                   OptT shared, OptT gate_w) {
   check_f32(out, "out");
@@ -1043,9 +1069,9 @@ void experts_many(Tensor out, Tensor h, Tensor idx, Tensor wts, Tensor wgu, Tens
   int *row = sorted.data_ptr<int>(), *place = row + pairs, *offs = place + pairs;
   Tensor y = at::empty({pairs, ff}, h.options()), d = at::empty({pairs, width}, h.options());
   chk(mx_pair_sort(offs, row, place, idx.data_ptr<int>(), t, (int)top, experts, stream()), "pair_sort");
-  chk(mx_grouped_gemm(y.data_ptr(), h.data_ptr(), row, wgu.data_ptr(), offs, experts, pairs, (int)ff, (int)width,
+  chk(mx_grouped_gemm(y.data_ptr(), h.data_ptr(), t, row, wgu.data_ptr(), offs, experts, pairs, (int)ff, (int)width,
                       (int)act, (float)limit, stream()), "grouped_gemm");
-  chk(mx_grouped_gemm(d.data_ptr(), y.data_ptr(), nullptr, wdown.data_ptr(), offs, experts, pairs, (int)width, (int)ff,
+  chk(mx_grouped_gemm(d.data_ptr(), y.data_ptr(), pairs, nullptr, wdown.data_ptr(), offs, experts, pairs, (int)width, (int)ff,
                       0, 0.f, stream()), "grouped_gemm");
   chk(mx_experts_merge(out.data_ptr<float>(), d.data_ptr(), place, wts.data_ptr<float>(),
                        shared ? shared->data_ptr() : nullptr, h.data_ptr(), h.stride(0),
@@ -1560,6 +1586,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("moe_topk", &moe_topk);
   m.def("moe_pairs", &moe_pairs);
   m.def("few_rows_gemm", &few_rows_gemm);
+  m.def("tile_gemm", &tile_gemm);
+  m.def("tile_gemm_us", &tile_gemm_us);
   m.def("moe_route_softmax", &moe_route_softmax);
   m.def("moe_route", &moe_route);
   m.def("moe_route_fits", &moe_route_fits);

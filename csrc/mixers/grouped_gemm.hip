@@ -18,11 +18,9 @@
 // taller tile empty).  The tiles run group by group, bands of eight row tiles with their columns after each
 // other, and each XCD (workgroup id mod 8) takes one contiguous eighth of that order, so the tiles in flight on
 // an XCD share an expert's rows and columns in its L2.
-// Bound by the L2's rate on tall groups (128 x 128 tiles with all operands resident in L2 still take 200 of the
-// 254 us below; 128 x 256 tiles with one workgroup a CU, 264), by the read of the matrices on short ones.
-// 16384 pairs of 32 experts, 2048 -> 2 x 1024 gated, 137 GFLOP: 195 us (700 TFLOP/s) in a running model, 254
-// with cold operands; one step of loads in flight, a barrier between reads and products and tiles in grid
-// order: 242 in the model.  1800 pairs, same matrices (268 MB): 78 us in the model, was 98.
+// Serves short groups, where it is bound by the read of the matrices, and rows that are no whole stages of tile_gemm.hip's:
+// tall groups go there (mx_grouped_gemm has the line and both sides).  1800 pairs of 32 experts, 2048 -> 2 x 1024 gated (268 MB):
+// 78 us in a model, with one step of loads in flight, a barrier between reads and products and tiles in grid order 98.
 #include "few_rows.h"
 
 #include <type_traits>
@@ -345,15 +343,29 @@ experts_merge_kernel(float* __restrict__ out, const bf16_t* __restrict__ d, cons
 
 using namespace mx;
 
-// act: few_rows.h (0: none).  rows: A's row of every sorted row, or null.
-extern "C" int mx_grouped_gemm(void* C, const void* A, const int* rows, const void* W, const int* offs, int groups, long M,
-                               int N, int K, int act, float limit, hipStream_t s) {
+extern "C" int mx_tile_gemm_fits(long M, int N, int K, long a_stride, int glu);
+extern "C" int mx_tile_gemm(void* C, long c_stride, const void* A, long a_stride, long a_rows, const int* rows, const void* W,
+                            const void* bias, const int* offs, int groups, long M, int N, int K, int act, float limit, int form,
+                            hipStream_t s);
+extern "C" int mx_tile_form_128();
+extern "C" int mx_tile_form_256();
+
+// act: few_rows.h (0: none).  a_rows: rows of A (M without an index).  rows: A's row of every sorted row, or null.
+extern "C" int mx_grouped_gemm(void* C, const void* A, long a_rows, const int* rows, const void* W, const int* offs, int groups,
+                               long M, int N, int K, int act, float limit, hipStream_t s) {
   if (M <= 0 || N <= 0 || groups <= 0) return 0;
   if (K < 8 || K % 8 || M > 0x7fffffffL || act < kFrStore || act > kFrReluSq) return -1;
   if (((uintptr_t)A) % 16 || ((uintptr_t)W) % 16) return -2;
   const bool glu = act >= kFrGelu && act <= kFrClamp;
   const int vec = N % 4 == 0 && ((uintptr_t)C) % 8 == 0;
   if ((M + 63) / 64 + groups > 65535) return -3;
+  // Tall groups take tile_gemm.hip's tiles, 256 x 256 or, up to 120 rows a group, 128 x 128.  us, 32 groups of 2048 -> 2 x 1024
+  // (gated), here with 64-row tiles / 128-row tiles / there with 128 / 256:  38 rows a group 64 - 70 80; 56: 71 - 69 80;
+  // 75: 76 - 70 80; 97: - 70 70 83; 125: - 89 81 81; 175: - 115 103 83; 250: - 130 120 119; 512: - 220 205 174;
+  // 128 groups of 768 -> 2048: 38 rows 97 - 111, 62: 116 - 117, 87: 145 - 125 130, 125: - 158 156 136
+  if (M >= 50L * groups && mx_tile_gemm_fits(a_rows, N, K, K, glu))
+    return mx_tile_gemm(C, N, A, K, a_rows, rows, W, nullptr, offs, groups, M, N, K, act, limit,
+                        M >= 120L * groups ? mx_tile_form_256() : mx_tile_form_128(), s);
   // 128-row tiles once the groups fill them on average
   const bool tall = M >= 96L * groups;
   const int cols = 128 / (glu ? 2 : 1), col_tiles = (N + cols - 1) / cols;

@@ -7,7 +7,7 @@
 // counted are a tenth of the cycles).
 #pragma once
 #include "mx_common.h"
-#include "../kernels/ft_lds.h"
+#include "ft_lds.h"
 
 namespace mx {
 

@@ -876,7 +876,7 @@ class MoEFF:
                 w1, wdown = self.shared
                 if self.shared_gate:
                     w1, gate_w = w1[:-1], w1[-1]
-                shared = M.linear(self._act(M.linear(h, w1), self.shared_limit), wdown)
+                shared = M.linear(M.linear_act(h, w1, self.act, self.shared_limit), wdown)
             return M.experts_many(h, idx, wts, self.wgu, self.wdown, self.act, self.limit, shared, gate_w)
         if self.shared is not None and not self.shared_gate:
             # an ungated shared expert's output is what the chosen experts' are added to

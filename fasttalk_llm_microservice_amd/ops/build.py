@@ -153,7 +153,8 @@ def build_kernels(force: bool = False, jobs: int = 8, verbose: bool = True,
 MIXER_FLAGS = NO_PK_F32
 # per kernel file, as KERNEL_FLAGS: accumulators that the vector units rescale between products
 MIXER_KERNEL_FLAGS = {"band_attn": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
-                      "latent_prefill": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
+                      "latent_prefill": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+                      "tile_gemm": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
 
 
 def build_mixers(force: bool = False, jobs: int = 8, verbose: bool = True) -> Path:

@@ -21,6 +21,7 @@ a longer one), with the position of its first row, its state slot and its block 
 from __future__ import annotations
 
 import dataclasses
+import functools
 import importlib
 import os
 import threading
@@ -93,11 +94,50 @@ FEW_ROWS = 64
 FEW_ACTS = {None: 0, "gelu_tanh": 1, "relu": 2, "silu": 3, "clamp_glu": 4, "relu_sq": 5, "silu_glu": 3}
 
 
-def _few_rows(x, w) -> bool:
-    """bf16 rows and weights of whole 16-byte pieces, at most FEW_ROWS rows, on a GPU."""
+def _piece_rows(x, w) -> bool:
+    """bf16 rows and weights of whole 16-byte pieces on a GPU."""
     return bool(x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2
-                and 1 <= x.shape[0] <= FEW_ROWS and x.shape[1] % 8 == 0 and x.shape[1] >= 8 and x.stride(1) == 1
+                and x.shape[0] >= 1 and x.shape[1] % 8 == 0 and x.shape[1] >= 8 and x.stride(1) == 1
                 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and w.is_contiguous())
+
+
+def _few_rows(x, w) -> bool:
+    """The same, at most FEW_ROWS rows."""
+    return x.shape[0] <= FEW_ROWS and _piece_rows(x, w)
+
+
+@functools.lru_cache(maxsize=8192)
+def _tile_gemm_pays(rows: int, n: int, k: int, act: Optional[str] = None) -> bool:
+    """Where a product of more than FEW_ROWS rows runs in the kernels of csrc/mixers/tile_gemm.hip (``n`` rows of w; with
+    ``act`` in their epilogue): k of whole 64 and an expected time that is near the vendor's, which lies between 6 and 20 us
+    above that of its operations at 1.3 PFLOP/s, and the activation's kernel, which takes 4 us and its bytes at 3.5 TB/s.  Up to
+    1024 rows a step is issued by the host, where a call of the vendor's product takes 21 us and this one 5, so the kernel may
+    be behind by a few; beyond, the sooner full tiles keep the vendor's product at its rate, the less.  us at 100 / 300 / 777 /
+    2048 / 4096 rows, the vendor's (with the activation) beside it:
+      n = 2048, k = 2048     7 10 14 22 40 (9 11 15 23 35)         k = 8192            22 31 49 90 128 (21 33 47 74 118)
+      n = 10272, k = 2048    18 21 47 92 155 (18 26 41 96 180)     n = 64              6 7 7 7 8 (8 8 8 9 10)
+      gated, 2 x 8192, k = 2048    20 34 55 109 225 (28 40 66 137 270)
+      n = 4096, k = 14336    44 93 121 215 338 (50 76 115 204 316)"""
+    if rows <= FEW_ROWS or k % 64 or k < 64:
+        return False
+    glu = act is not None and act != "relu_sq"
+    out = n // 2 if glu else n
+    if max(rows * k, n * k) * 2 > 0xffffffff or out < 1:
+        return False
+    spare = (20 if rows <= 1024 else 7) + (0 if act is None else 4 + rows * out * (6 if glu else 4) / 3.5e6)
+    return native_mixers().tile_gemm_us(rows, out, k, glu) <= spare + 2.0 * rows * n * k / (1.3e9 if rows <= 1024 else 1.35e9)
+
+
+def _tile_gemm(x, w, bias, act: Optional[str] = None, limit: float = 0.0):
+    """The product where :func:`_tile_gemm_pays`, else None."""
+    if x.dim() != 2 or x.shape[0] <= FEW_ROWS or not _piece_rows(x, w) \
+            or x.stride(0) * x.shape[0] * 2 > 0xffffffff or not _tile_gemm_pays(x.shape[0], w.shape[0], x.shape[1], act) \
+            or (bias is not None and not (bias.dtype == torch.bfloat16 and bias.is_contiguous())):
+        return None
+    n = w.shape[0] if act is None or act == "relu_sq" else w.shape[0] // 2
+    y = torch.empty(x.shape[0], n, dtype=x.dtype, device=x.device)
+    native_mixers().tile_gemm(y, x, w, bias, FEW_ACTS[act], float(limit), -1)
+    return y
 
 
 def _few_rows_pays(rows: int, n: int, k: int, act: Optional[str] = None) -> bool:
@@ -146,7 +186,8 @@ def linear(x, w, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
         y = torch.empty(x.shape[0], w.shape[0], dtype=x.dtype, device=x.device)
         native_mixers().few_rows_gemm(y, x, w, bias, 0, 0.0)
         return y
-    return torch.nn.functional.linear(x, w, bias)
+    y = _tile_gemm(x, w, bias)
+    return torch.nn.functional.linear(x, w, bias) if y is None else y
 
 
 def linear_f32(x, w) -> torch.Tensor:
@@ -160,18 +201,21 @@ def linear_f32(x, w) -> torch.Tensor:
 
 def linear_act(x, w, act: str, limit: float = 0.0) -> torch.Tensor:
     """act of x w^T: w = [gate | up] rows for the gated forms ("gelu_tanh", "relu", "silu",
-    "clamp_glu" with ``limit``), one matrix for "relu_sq".  Where the few-rows kernel pays, one
-    kernel, the products stay fp32 up to the activation's result."""
+    "clamp_glu" with ``limit``), one matrix for "relu_sq".  Where the few-rows kernel or the tiles pay,
+    one kernel, the products stay fp32 up to the activation's result."""
     if _few_rows(x, w) and _few_rows_pays(x.shape[0], w.shape[0], x.shape[1], act):
         n = w.shape[0] if act == "relu_sq" else w.shape[0] // 2
         y = torch.empty(x.shape[0], n, dtype=x.dtype, device=x.device)
         native_mixers().few_rows_gemm(y, x, w, None, FEW_ACTS[act], float(limit))
         return y
+    y = _tile_gemm(x, w, None, act, limit)
+    if y is not None:
+        return y
     u = torch.nn.functional.linear(x, w)
     if act == "relu_sq":
         return relu_sq(u)
-    return clamp_swiglu(u, limit) if act == "clamp_glu" else {"gelu_tanh": gelu_glu, "relu": relu_glu,
-                                                              "silu": silu_glu}[act](u)
+    return clamp_swiglu(u, limit) if act == "clamp_glu" else {"gelu_tanh": gelu_glu, "relu": relu_glu, "silu": silu_glu,
+                                                              "silu_glu": silu_glu}[act](u)
 
 
 # ---------------------------------------------------------------------------------
