@@ -229,29 +229,32 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void packed_gemm_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// 256 x 256 "phased" variant (guide §5 "The 256² 8-phase template", adapted to
-// the packed W image): each k-tile (64) is computed in 4 phases, one C quadrant
-// (64 x 32 per wave) per phase, and the operand halves (A rows 0-127 / 128-255,
-// W columns 0-127 / 128-255, 16 KiB each) are re-filled as soon as the last
-// phase that reads them is over, so with only two LDS slots the next-but-one
-// tile's halves are in flight while this tile computes.  Waves sit 2 (M) x 4 (N)
-// and own rows {mq * 128 + wm * 64 + [0, 64)} x cols {nq * 128 + wn * 32 + [0, 32)}
-// for quadrants (mq, nq), so every wave reads the same half in the same phase:
-//   phase:        P0          P1          P2          P3
-//   quadrant:   Alo.Blo     Alo.Bhi     Ahi.Blo     Ahi.Bhi
-//   LDS reads:  Alo, Blo    Bhi         Ahi         -      (kept in registers)
-//   DMA issue:  -           Alo,Blo     Bhi         Ahi    of tile t+2
-// A half is refilled with tile t+2 one phase after its only read, so two whole
-// tiles stay in flight with two LDS slots (6 phases between a half's DMA and its
-// first read).  Each phase: counted vmcnt for the data the NEXT phase reads,
-// this phase's ds_reads and DMA, s_barrier, MFMA cluster (setprio 1), s_barrier.
+// 256 x 256 tiles, eight waves in two groups half a phase apart: while one group's
+// products run, the other's LDS reads and DMA do (waves w and w + 4 share a SIMD).
+// A 64-deep stage takes four phases, a quarter's products each (waves sit 2 (M) x 4
+// (N); a wave owns 64 rows x 32 columns of each quarter of the tile):
+//   phase:     0              1                 2              3
+//   quarter:   Alo.Blo        Alo.Bhi           Ahi.Blo        Ahi.Bhi
+//   LDS reads: Alo (3 of 4)   Bhi, Ahi's 4th    Ahi (3 of 4)   Blo, Alo's 4th of stage t + 1
+//   DMA:       Blo            Alo               Bhi            Ahi           of stage t + 2
+// A half is refilled where the phase before read last, so with two slots four to six
+// phases lie between a DMA and its read.  Every phase: the DMA that the next one
+// reads has landed (counted vmcnt; a barrier lies between), reads, DMA, barrier,
+// products, barrier.  Six LDS reads a phase: the LDS delivers a wave's eight in the
+// time of its 16 products, and eight, four, eight, four a phase took 7 % longer.
+// W is the left operand, so a lane ends with four neighbouring columns of a row;
+// bf16 results leave through LDS in whole rows (written four columns a lane: 4 %).
+// us at M = 4096, back to back (packed_gemm_kernel's 256 x 256 tiles): gate_up with
+// SiLU 691, 1392 TFLOP/s (809); down 338 (414); qkv 170 (220); o 97 (124); M = 1024:
+// down in four splits 96 (110), gate_up 188 (227).  Bound by the matrix units at the
+// clock that the card's power leaves them, less the first loads and the epilogue of
+// a tile (9 us of 4096 x 4096 x 4096's 97).
 template <int EPI>
 __global__ __launch_bounds__(512, 1) void packed_gemm8_kernel(
     const uint16_t* __restrict__ x, int x_stride, int M, const uint16_t* __restrict__ wpk, int N,
     int K, int k_slice, uint16_t* __restrict__ out, int out_stride, float* __restrict__ ws) {
   constexpr int HALF = 16384;              // bytes per operand half-tile
   constexpr int SLOT = 4 * HALF;           // Alo | Ahi | Blo | Bhi
-  constexpr int ALO = 0, AHI = HALF, BLO = 2 * HALF, BHI = 3 * HALF;
   __shared__ __attribute__((aligned(16))) uint8_t smem[2 * SLOT];
 
   const int lane = lane_id(), w = wave_id();
@@ -263,7 +266,12 @@ __global__ __launch_bounds__(512, 1) void packed_gemm8_kernel(
   const int orig = blockIdx.x;
   const int q = total / 8, r = total % 8, xcd = orig % 8;
   const int wgid = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + orig / 8;
-  const int tn = wgid / mt_tiles, tm = wgid % mt_tiles;
+  // bands of eight row tiles, columns after each other, rows fastest: the tiles in
+  // flight on an XCD share rows and columns in its L2
+  const int nt_tiles = total / mt_tiles;
+  const int band = wgid / (8 * nt_tiles), in = wgid - band * 8 * nt_tiles;
+  const int tall = min(8, mt_tiles - 8 * band);
+  const int tn = in / tall, tm = 8 * band + in % tall;
   const int m0 = tm * 256, n0 = tn * 256;
   const int s = blockIdx.y;
   const int kbeg = s * k_slice;
@@ -287,169 +295,174 @@ __global__ __launch_bounds__(512, 1) void packed_gemm8_kernel(
       const int nt = min((n0 >> 4) + hf * 8 + (piece >> 1), ntiles_all - 1);
       b_src[hf][i] = wpk + ((size_t)nt * ksteps + (kbeg >> 6)) * 1024 + (piece & 1) * 512 + lane * 8;
     }
-  auto issue_a = [&](int hf, int t) {
-    const uint32_t base = lds0 + (t & 1) * SLOT + (hf ? AHI : ALO);
+  auto load_a = [&](int hf, int t) {
+    const uint32_t base = lds0 + (t & 1) * SLOT + hf * HALF;
 #pragma unroll
     for (int i = 0; i < 2; ++i) glds16(a_src[hf][i] + t * 64, base + (w + 8 * i) * 1024);
   };
-  auto issue_b = [&](int hf, int t) {
-    const uint32_t base = lds0 + (t & 1) * SLOT + (hf ? BHI : BLO);
+  auto load_b = [&](int hf, int t) {
+    const uint32_t base = lds0 + (t & 1) * SLOT + (2 + hf) * HALF;
 #pragma unroll
     for (int i = 0; i < 2; ++i) glds16(b_src[hf][i] + (size_t)t * 1024, base + (w + 8 * i) * 1024);
   };
 
-  // fragment offsets inside a half: A rows wm*64 + i*16 + l15, W n-tiles wn*2 + j
-  uint32_t a_off[4][2];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int rl = wm * 64 + i * 16 + l15;
-#pragma unroll
-    for (int h = 0; h < 2; ++h) a_off[i][h] = rl * 128 + (((2 * g + h) ^ ((rl >> 1) & 5)) * 16);
-  }
-  const uint32_t b_off = (wn * 2) * 2048 + lane * 16;
+  // fragments: A rows wm * 64 + i * 16 + l15 of a half, half k-step h in chunk 2 g + h;
+  // W n-tile wn * 2 + j of a half, in fragment order
+  const int swz = (l15 >> 1) & 5;
+  const uint8_t* as = smem + (wm * 64 + l15) * 128;
+  const int get[2] = {((2 * g) ^ swz) * 16, ((2 * g + 1) ^ swz) * 16};
+  const uint8_t* bs = smem + 2 * HALF + wn * 4096 + lane * 16;
 
-  pg_floatx4 acc[8][4];
+  pg_floatx4 acc[2][2][2][4];
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
+  for (int a = 0; a < 2; ++a)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = pg_floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[a][b][j][i] = pg_floatx4{0.f, 0.f, 0.f, 0.f};
 
-  uint4 alo[4][2], ahi[4][2], blo[2][2], bhi[2][2];
-  auto read_a = [&](uint4 (&a)[4][2], uint32_t base) {
+  uint4 a3[3][2], a4[2][2], blo[2][2], bhi[2][2];   // a4: the fourth row tile of Alo and Ahi
+  auto read_a = [&](int hf, int t) {
+    const uint8_t* p = as + (t & 1) * SLOT + hf * HALF;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      a[i][0] = ds_read16(base + a_off[i][0]);
-      a[i][1] = ds_read16(base + a_off[i][1]);
-    }
-  };
-  auto read_b = [&](uint4 (&b)[2][2], uint32_t base) {
+    for (int i = 0; i < 3; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      b[j][0] = ds_read16(base + b_off + j * 2048);
-      b[j][1] = ds_read16(base + b_off + j * 2048 + 1024);
-    }
+      for (int h = 0; h < 2; ++h) a3[i][h] = *reinterpret_cast<const uint4*>(p + get[h] + i * 2048);
   };
-  auto quad = [&](uint4 (&a)[4][2], uint4 (&b)[2][2], int mq, int nq) {
+  auto read_a4 = [&](int hf, int t) {
+    const uint8_t* p = as + (t & 1) * SLOT + hf * HALF + 3 * 2048;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) a4[hf][h] = *reinterpret_cast<const uint4*>(p + get[h]);
+  };
+  auto read_b = [&](uint4 (&b)[2][2], int hf, int t) {
+    const uint8_t* p = bs + (t & 1) * SLOT + hf * HALF;
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) b[j][h] = *reinterpret_cast<const uint4*>(p + j * 2048 + h * 1024);
+  };
+  auto quad = [&](uint4 (&b)[2][2], int mq, int nq) {
+    lgkm_wait<0>();   // (before the barrier: what these reads read is refilled behind it)
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          pg_floatx4& c = acc[mq][nq][j][i];
+          c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              pg_frag(b[j][h]), pg_frag(i == 3 ? a4[mq][h] : a3[i < 3 ? i : 0][h]), c, 0, 0, 0);
+        }
+    __builtin_amdgcn_s_setprio(0);
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // LEFT: stages behind this one (2: two or more)
+  auto stage = [&](auto left, int t) {
+    constexpr int LEFT = decltype(left)::value;
+    vm_wait<LEFT >= 1 ? 8 : 0>();                            // Ahi, Bhi of t
+    read_a(0, t);
+    if constexpr (LEFT >= 2) load_b(0, t + 2);
+    quad(blo, 0, 0);
+    read_b(bhi, 1, t);
+    read_a4(1, t);
+    if constexpr (LEFT >= 2) load_a(0, t + 2);
+    quad(bhi, 0, 1);
+    if constexpr (LEFT >= 1) vm_wait<LEFT >= 2 ? 8 : 4>();   // Blo, Alo of t + 1
+    read_a(1, t);
+    if constexpr (LEFT >= 2) load_b(1, t + 2);
+    quad(blo, 1, 0);
+    if constexpr (LEFT >= 1) {
+      read_b(blo, 0, t + 1);
+      read_a4(0, t + 1);
+    }
+    if constexpr (LEFT >= 2) load_a(1, t + 2);
+    quad(bhi, 1, 1);
+  };
+
+  load_b(0, 0);
+  load_a(0, 0);
+  load_b(1, 0);
+  load_a(1, 0);
+  if (nk > 1) {
+    load_b(0, 1);
+    load_a(0, 1);
+    load_b(1, 1);
+    load_a(1, 1);
+    vm_wait<12>();   // stage 0's Blo, Alo
+  } else {
+    vm_wait<4>();
+  }
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+  read_b(blo, 0, 0);
+  read_a4(0, 0);
+  lgkm_wait<0>();
+  if (wm == 1) __builtin_amdgcn_s_barrier();   // the second group: one barrier behind
+  for (int t = 0; t + 2 < nk; ++t) stage(std::integral_constant<int, 2>{}, t);
+  if (nk > 1) stage(std::integral_constant<int, 1>{}, nk - 2);
+  stage(std::integral_constant<int, 0>{}, nk - 1);
+  if (wm == 0) __builtin_amdgcn_s_barrier();
+
+  // lane (g, l15) holds columns 4 g .. 4 g + 3 of row l15 of each 16 x 16 tile
+  if constexpr (EPI == kPgSlab) {
+    float* slab = ws + (size_t)s * M * N;
+#pragma unroll
+    for (int mq = 0; mq < 2; ++mq)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int m = m0 + mq * 128 + wm * 64 + i * 16 + l15;
+        if (m >= M) continue;
+#pragma unroll
+        for (int nq = 0; nq < 2; ++nq)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            const int n = n0 + nq * 128 + wn * 32 + j * 16 + 4 * g;
+            const pg_floatx4& c = acc[mq][nq][j][i];
+            if (n < N)
+              *reinterpret_cast<float4*>(slab + (size_t)m * N + n) = make_float4(c[0], c[1], c[2], c[3]);
+          }
+      }
+    return;
+  }
+  constexpr int OC = EPI == kPgSilu ? 128 : 256;   // output columns of the tile
+  constexpr int RS = OC * 2 + 16;                  // bytes of a staged row
+  const int out_cols = EPI == kPgSilu ? N >> 1 : N;
+  const int oc0 = EPI == kPgSilu ? n0 >> 1 : n0;
+#pragma unroll
+  for (int mq = 0; mq < 2; ++mq) {
+    if (mq) __syncthreads();
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        pg_floatx4& c = acc[mq * 4 + i][nq * 2 + j];
-        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pg_frag(a[i][0]), pg_frag(b[j][0]), c, 0, 0, 0);
-        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pg_frag(a[i][1]), pg_frag(b[j][1]), c, 0, 0, 0);
-      }
-    __builtin_amdgcn_s_setprio(0);
-  };
-  auto dep_a = [&](uint4 (&a)[4][2]) {
+      for (int nq = 0; nq < 2; ++nq)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      dep(a[i][0]);
-      dep(a[i][1]);
-    }
-  };
-  auto dep_b = [&](uint4 (&b)[2][2]) {
+        for (int j = 0; j < (EPI == kPgSilu ? 1 : 2); ++j) {
+          float v[4];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      dep(b[j][0]);
-      dep(b[j][1]);
-    }
-  };
-
-  // prologue: tiles 0 and 1 whole (issue order = the steady-state order)
-  issue_a(0, 0);
-  issue_b(0, 0);
-  issue_b(1, 0);
-  issue_a(1, 0);
-  if (nk > 1) {
-    issue_a(0, 1);
-    issue_b(0, 1);
-    issue_b(1, 1);
-    issue_a(1, 1);
-    vm_wait<12>();  // tile 0's Alo, Blo
-  } else {
-    vm_wait<0>();
-  }
-  __builtin_amdgcn_s_barrier();
-
-  for (int t = 0; t < nk; ++t) {
-    const uint32_t base = lds0 + (t & 1) * SLOT;
-    const bool steady = t + 2 < nk;   // every issue of the schedule happens
-    // ---- P0: reads Alo, Blo (quadrant 0,0); retire Bhi(t) for P1
-    if (steady) vm_wait<10>(); else vm_wait<0>();
-    read_a(alo, base + ALO);
-    read_b(blo, base + BLO);
-    __builtin_amdgcn_s_barrier();
-    lgkm_wait<0>();
-    dep_a(alo);
-    dep_b(blo);
-    quad(alo, blo, 0, 0);
-    __builtin_amdgcn_s_barrier();
-    // ---- P1: reads Bhi (0,1); Alo/Blo(t) are in registers -> refill with tile t+2;
-    // retire Ahi(t) for P2
-    if (steady) vm_wait<8>(); else vm_wait<0>();
-    read_b(bhi, base + BHI);
-    if (t + 2 < nk) {
-      issue_a(0, t + 2);
-      issue_b(0, t + 2);
-    }
-    __builtin_amdgcn_s_barrier();
-    lgkm_wait<0>();
-    dep_b(bhi);
-    quad(alo, bhi, 0, 1);
-    __builtin_amdgcn_s_barrier();
-    // ---- P2: reads Ahi (1,0); Bhi(t) free -> Bhi(t+2)
-    read_a(ahi, base + AHI);
-    if (t + 2 < nk) issue_b(1, t + 2);
-    __builtin_amdgcn_s_barrier();
-    lgkm_wait<0>();
-    dep_a(ahi);
-    quad(ahi, blo, 1, 0);
-    __builtin_amdgcn_s_barrier();
-    // ---- P3: (1,1) from registers; Ahi(t) free -> Ahi(t+2); retire Alo/Blo(t+1)
-    if (steady) vm_wait<10>(); else vm_wait<0>();
-    if (t + 2 < nk) issue_a(1, t + 2);
-    __builtin_amdgcn_s_barrier();
-    quad(ahi, bhi, 1, 1);
-    __builtin_amdgcn_s_barrier();
-  }
-
-  // epilogue: acc[mq * 4 + i][nq * 2 + j] -> rows m0 + mq*128 + wm*64 + i*16 + 4g + rr,
-  // cols n0 + nq*128 + wn*32 + j*16 + l15
-  if (EPI == kPgSilu) {
-    const int half_n = N >> 1;
-#pragma unroll
-    for (int mi = 0; mi < 8; ++mi)
-#pragma unroll
-      for (int nq = 0; nq < 2; ++nq) {
-        const int col = ((n0 + nq * 128 + wn * 32) >> 1) + l15;
-#pragma unroll
-        for (int rr = 0; rr < 4; ++rr) {
-          const int m = m0 + (mi >> 2) * 128 + wm * 64 + (mi & 3) * 16 + 4 * g + rr;
-          if (m < M && col < half_n) {
-            const float gv = acc[mi][nq * 2][rr], uv = acc[mi][nq * 2 + 1][rr];
-            out[(size_t)m * out_stride + col] = f32_to_bf16(gv / (1.f + __expf(-gv)) * uv);
+          for (int e = 0; e < 4; ++e) {
+            v[e] = acc[mq][nq][j][i][e];
+            if constexpr (EPI == kPgSilu) v[e] = v[e] / (1.f + __expf(-v[e])) * acc[mq][nq][1][i][e];
           }
+          const int c = (EPI == kPgSilu ? nq * 64 + wn * 16 : nq * 128 + wn * 32 + j * 16) + 4 * g;
+          *reinterpret_cast<uint2*>(smem + (wm * 64 + i * 16 + l15) * RS + c * 2) =
+              make_uint2(pack2(v[0], v[1]), pack2(v[2], v[3]));
         }
-      }
-  } else {
-    float* slab = ws + (size_t)s * M * N;
+    __syncthreads();
+    constexpr int CPR = OC / 8;   // 16-B chunks per row
 #pragma unroll
-    for (int mi = 0; mi < 8; ++mi)
-#pragma unroll
-      for (int nj = 0; nj < 4; ++nj) {
-        const int n = n0 + (nj >> 1) * 128 + wn * 32 + (nj & 1) * 16 + l15;
-#pragma unroll
-        for (int rr = 0; rr < 4; ++rr) {
-          const int m = m0 + (mi >> 2) * 128 + wm * 64 + (mi & 3) * 16 + 4 * g + rr;
-          if (m < M && n < N) {
-            if (EPI == kPgSlab)
-              slab[(size_t)m * N + n] = acc[mi][nj][rr];
-            else
-              out[(size_t)m * out_stride + n] = f32_to_bf16(acc[mi][nj][rr]);
-          }
-        }
-      }
+    for (int e = threadIdx.x; e < 128 * CPR; e += 512) {
+      const int rl = e / CPR, c = (e % CPR) * 8, m = m0 + mq * 128 + rl;
+      const uint4 v = *reinterpret_cast<const uint4*>(smem + rl * RS + c * 2);
+      if (m < M && oc0 + c < out_cols)
+        *reinterpret_cast<uint4*>(out + (size_t)m * out_stride + oc0 + c) = v;
+    }
   }
 }
 
@@ -684,6 +697,8 @@ extern "C" int ft_packed_gemm(const void* x, int x_stride, int M, const void* wp
   if ((epi == 1) != (splits > 1)) return -4;
   if (epi == 1 && ws == nullptr) return -4;
   const int k_slice = K / splits;
+  const bool whole = epi == 1 || (out_stride % 8 == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0);
+  if (cfg == 3 && !whole) cfg = 0;   // (the same sums, written column by column)
   int bm, bn;
   switch (cfg) {
     case 0: bm = 256; bn = 256; break;
@@ -702,10 +717,7 @@ extern "C" int ft_packed_gemm(const void* x, int x_stride, int M, const void* wp
   }
   const int tiles = ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
   dim3 grid(tiles, splits), block(cfg == 4 ? 256 : 512);
-  if (cfg >= 10) {
-    // pg32 (BK 32 ring): bf16 / SiLU epilogues store 16-B row chunks
-    if (epi != 1 && (out_stride % 8 != 0 || (reinterpret_cast<uintptr_t>(out) & 15) != 0)) return -6;
-  }
+  if (cfg >= 10 && !whole) return -6;   // pg32 (BK 32 ring): bf16 / SiLU epilogues store 16-B row chunks
 #define FT_PG(CFG, WM, WN, MT, NT, S)                                                          \
   if (cfg == CFG) {                                                                            \
     if (epi == 0)                                                                              \

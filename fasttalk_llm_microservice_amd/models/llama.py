@@ -154,15 +154,22 @@ MAX_SPLITS = 4
 # step to 192 / 384 MFMA rows instead of 256 / 512 -- profiles/pg_probe_192_r04.log:
 # gate_up 54.8 vs 67.8 us at 145 rows, 81.4 vs 102.4 at 300, 88.2 vs 105.3 at 384;
 # down 36.2 vs 43.7 / 54.3 vs 63.8 / 57.5 vs 66.3; LM head 233 vs 263 / 376 vs 463.
+# Above 384 rows: cfg 3, 256x256 in phases, with as many splits as leave one round of
+# workgroups (us, the tile it replaces beside it): qkv 50 vs 57 at 768 rows and 57 vs 65
+# at 1280 (2 splits), 78 vs 99 at 1536, 170 vs 218 at 4096; o 53 vs 66 at 1280 (2), 85 vs
+# 105 at 3000; gate_up 98 vs 122 at 512, 280 vs 329 at 1536; down 82 vs 95 at 640 (4),
+# 140 vs 192 at 1280 (2), 286 vs 363 at 3000; LM head 429 vs 523 at 512, 1579 vs 1830 at
+# 2048.  (o at 513-1024 rows keeps two splits: four take 34 vs 40 us but leave the
+# residual-add kernel twice the slabs.)
 PG_PLAN = {
-    "qkv": ((128, 1, 8), (192, 6, 4), (256, 2, 4), (384, 6, 2), (512, 2, 2), (2047, 0, 2),
-            (1 << 30, 2, 1)),
-    "o": ((128, 2, 8), (192, 6, 8), (256, 1, 8), (384, 6, 4), (512, 2, 4), (2047, 1, 2),
-          (1 << 30, 0, 1)),
-    "gu": ((128, 1, 2), (192, 6, 1), (256, 2, 1), (384, 5, 1), (1 << 30, 0, 1)),
-    "down": ((128, 1, 16), (192, 6, 8), (256, 1, 8), (384, 5, 8), (512, 0, 8), (2047, 0, 4),
-             (1 << 30, 3, 1)),
-    "lm": ((128, 1, 1), (192, 5, 1), (256, 3, 1), (384, 5, 1), (1 << 30, 0, 1)),
+    "qkv": ((128, 1, 8), (192, 6, 4), (256, 2, 4), (384, 6, 2), (512, 2, 2), (1280, 3, 2),
+            (1 << 30, 3, 1)),
+    "o": ((128, 2, 8), (192, 6, 8), (256, 1, 8), (384, 6, 4), (512, 2, 4), (1024, 1, 2),
+          (2047, 3, 2), (1 << 30, 3, 1)),
+    "gu": ((128, 1, 2), (192, 6, 1), (256, 2, 1), (384, 5, 1), (1 << 30, 3, 1)),
+    "down": ((128, 1, 16), (192, 6, 8), (256, 1, 8), (384, 5, 8), (512, 3, 8), (1024, 3, 4),
+             (2047, 3, 2), (1 << 30, 3, 1)),
+    "lm": ((128, 1, 1), (192, 5, 1), (256, 3, 1), (384, 5, 1), (1 << 30, 3, 1)),
 }
 PG_MAX_SLAB_ROWS = 2048
 # hipBLASLt detours removed in round 5: unpacking the packed image into a row-major
