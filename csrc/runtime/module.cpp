@@ -10,6 +10,7 @@ namespace py = pybind11;
 using namespace ftrt;
 
 void register_json_fsm(py::module_& m);
+void register_step_inputs(py::module_& m);
 
 // The bindings are a plain function so csrc/tools/rt_sanitize.cpp can register the
 // same module inside an ASan/UBSan-instrumented executable that embeds Python.
@@ -72,6 +73,7 @@ void ftrt_register(py::module_& m) {
       .def_property_readonly("vocab_size", &Detokenizer::vocab_size);
 
   register_json_fsm(m);
+  register_step_inputs(m);
 }
 
 #ifndef FTRT_EMBEDDED

@@ -845,12 +845,16 @@ class LLMEngine:
                 r += n
             wanted = [base[rid] + int(w) for rid, _, want in entries for w in want]
             # the step gathers ascending, distinct rows; the caller's order is restored here
-            uniq, inverse = np.unique(np.asarray(wanted, dtype=np.int64), return_inverse=True)
-            batch.logit_rows = uniq.tolist()
+            inverse = None
+            if any(a >= b for a, b in zip(wanted, wanted[1:])):
+                uniq, inverse = np.unique(np.asarray(wanted, dtype=np.int64), return_inverse=True)
+                batch.logit_rows = uniq.tolist()
+            else:
+                batch.logit_rows = wanted
             self._executing = batch
             logits = self.runner.execute(batch, None, logits_only=True)
             self._executing = None
-            logits = logits[inverse] if len(wanted) else logits
+            logits = logits if inverse is None else logits[inverse]
             sched.post_step(batch)
             self.stats["given_steps"] += 1
         for rid in end:

@@ -24,6 +24,7 @@ from ..models.config import ModelConfig
 from ..models.llama import AttnMeta
 from ..models.registry import build_model
 from ..parallel.comm import SINGLE, TPComm
+from ..runtime import rt
 from .config import EngineConfig
 from .scheduler import ScheduledBatch
 
@@ -88,47 +89,52 @@ class _Uploader:
         self.device = device
         self.pin = pin
         self.host = [torch.zeros(0, dtype=torch.int32) for _ in range(2)]
+        self.words = [h.numpy() for h in self.host]
         self.events = [None, None]
         self.dev = torch.zeros(0, dtype=torch.int32, device=device)
         self.k = 0
 
     def __call__(self, arrays):
         arrs = [np.ascontiguousarray(a) for a in arrays]
-        offs, n = [], 0
+        offs, cut, n = [], [], 0              # (cut: field, gap, field, gap, ..)
         for a in arrs:
+            if a.dtype.itemsize not in (4, 8):
+                raise TypeError(f"upload: unsupported dtype {a.dtype}")
             offs.append(n)
-            w = (a.nbytes + 3) // 4
-            n += (w + self.ALIGN - 1) // self.ALIGN * self.ALIGN
-        n = max(n, self.ALIGN)
+            w = a.nbytes // 4
+            gap = -w % self.ALIGN
+            cut += (w, gap)
+            n += w + gap
+        if n < self.ALIGN:
+            cut += (0, self.ALIGN - n)
+            n = self.ALIGN
         k = self.k
         self.k ^= 1
         if self.events[k] is not None:
             self.events[k].synchronize()
         if self.host[k].numel() < n:
             self.host[k] = torch.zeros(2 * n, dtype=torch.int32, pin_memory=self.pin)
+            self.words[k] = self.host[k].numpy()
         if self.dev.numel() < n:
             # the old buffer may still feed queued kernels: the caching allocator only
             # reuses its memory after the stream has passed this point
             self.dev = torch.zeros(2 * n, dtype=torch.int32, device=self.device)
-        hb = self.host[k].numpy().view(np.uint8)
-        for a, o in zip(arrs, offs):
-            hb[4 * o:4 * o + a.nbytes] = a.reshape(-1).view(np.uint8)
-        self.dev[:n].copy_(self.host[k][:n], non_blocking=True)
+        hw = self.words[k]
+        for a, o, w in zip(arrs, offs, cut[::2]):
+            hw[o:o + w] = a.reshape(-1).view(np.int32)
+        dev = self.dev[:n]
+        dev.copy_(self.host[k][:n], non_blocking=True)
         if self.pin:
             ev = self.events[k] or torch.cuda.Event()
             ev.record()
             self.events[k] = ev
         outs = []
-        for a, o in zip(arrs, offs):
-            w = (a.nbytes + 3) // 4
-            v = self.dev[o:o + w]
+        for a, v in zip(arrs, dev.split(cut)[::2]):
             if a.dtype.itemsize == 8:
                 v = v.view(torch.int64 if a.dtype.kind in "iu" else torch.float64)
             elif a.dtype == np.float32:
                 v = v.view(torch.float32)
-            elif a.dtype.itemsize != 4:
-                raise TypeError(f"upload: unsupported dtype {a.dtype}")
-            outs.append(v.view(a.shape) if a.ndim != 1 else v)
+            outs.append(v if a.ndim == 1 else v.view(a.shape))
         return outs
 
 
@@ -1097,48 +1103,10 @@ class ModelRunner:
         return h.host[:h.n].tolist()
 
     def _decode_fill(self, seqs, nb: int, st: "_Staging") -> int:
-        """Writes a decode step's inputs into a pinned staging set."""
-        n = len(seqs)
-        mb = self.max_decode_batch
-        hs = st.hs
-        ids = hs[0:mb]
-        pos = hs[mb:2 * mb]
-        slots = hs[2 * mb:3 * mb]
-        sl = hs[3 * mb:4 * mb]
-        bt = st.hbt
-        bs = self.bs
-        maxblk = 1
-        for i, s in enumerate(seqs):
-            p = s.n_tokens - 1 + s.inflight   # steps queued ahead of this one
-            ids[i] = s.last_token  # replaced on the device when queued ahead
-            pos[i] = p
-            slots[i] = s.block_ids[p // bs] * bs + p % bs
-            sl[i] = p + 1
-            nbk = len(s.block_ids)
-            bt[i, :nbk] = s.block_ids
-            maxblk = max(maxblk, nbk)
-        if self.stateful:
-            ss = hs[6 * mb:7 * mb]
-            for i, s in enumerate(seqs):
-                ss[i] = s.state_slot
-            ss[n:nb] = -1   # padding rows touch no state
-        temp, topp, topk, seeds, steps = self._sampling_arrays(seqs)
-        hs[4 * mb:4 * mb + n] = topk
-        hs[5 * mb:5 * mb + n] = steps
-        st.hf[:n] = temp
-        st.hf[mb:mb + n] = topp
-        st.hseed[:n] = seeds
-        if nb > n:  # padding rows: no KV write, empty context (no attention work), greedy
-            ids[n:nb] = 0
-            pos[n:nb] = 0
-            slots[n:nb] = -1
-            sl[n:nb] = 0
-            bt[n:nb, 0] = 0
-            hs[4 * mb + n:4 * mb + nb] = 0
-            hs[5 * mb + n:5 * mb + nb] = 0
-            st.hf[n:nb] = 0.0
-            st.hf[mb + n:mb + nb] = 1.0
-        return maxblk
+        """Writes a decode step's inputs into a pinned staging set (csrc/runtime/step_inputs.cpp); returns
+        the widest block table."""
+        return rt().fill_decode(list(seqs), self.bs, self.max_decode_batch, nb, self.stateful, st.hs, st.hbt, st.hf,
+                                st.hseed)
 
     def _gap_mark(self, start: bool, kind: str = "d"):
         ev = torch.cuda.Event(enable_timing=True)
