@@ -17,6 +17,20 @@ int mx_layer_norm(float* x, const void* y, int y_bf16, long y_stride, const floa
 int mx_tanh_cap(float* x, long n, float cap, hipStream_t s);
 int mx_grouped_gemm(void* C, const void* A, long a_rows, const int* rows, const void* W, const int* offs, int groups, long M,
                     int N, int K, int act, float limit, hipStream_t s);
+int mx_norm_route_fits(int width, int experts);
+int mx_norm_route(int* idx, float* wts, void* h, float* x, const void* y, int y_bf16, long y_stride,
+                  int layer, const float* wb, const float* w, const float* b, float eps, const float* router, const float* bias, long rows,
+                  int experts, int width, int top, int mode, float scale, int groups, int keep, hipStream_t s);
+int mx_expert_rows_fit(int width);
+int mx_add_rms_norm_experts(float* x, const float* d, const float* wts, const float* shared, const float* gate, int top,
+                            const float* wb, const float* add_vec, const float* next_w, void* out, void* cast, int out_bf16,
+                            int rows, int width, float eps, hipStream_t s);
+int mx_layer_norm_experts(float* x, const float* d, const float* wts, const float* shared, const float* gate, int top,
+                          const float* w, const float* b, void* cast, int rows, int width, float eps, hipStream_t s);
+int mx_add_norm_shift_experts(float* x, const float* d, const float* wts, const float* shared, const float* gate, int top,
+                              const float* wb, const float* w, const float* shift, void* out, float* state, int num_slots,
+                              const int* start, const int* pos0, const int* slot, int num_segs, int rows, int width,
+                              float eps, hipStream_t s);
 int mx_tile_gemm_fits(long M, int N, int K, long a_stride, int glu);
 float mx_tile_gemm_us(long M, int N, int K, int glu);
 int mx_tile_gemm(void* C, long c_stride, const void* A, long a_stride, long a_rows, const int* rows, const void* W,
@@ -986,9 +1000,12 @@ void few_rows_gemm(Tensor y, Tensor x, Tensor w, OptT bias, int64_t act, double 
                        (int)x.size(1), (int)act, (float)limit, stream()), "few_rows_gemm");
 }
 
-void experts_few(Tensor out, Tensor h, Tensor idx, Tensor wts, Tensor wgu, Tensor wdown, double limit, int64_t act,
-                 OptT shared_w, OptT shared_down, double shared_limit, bool shared_gate) {
-  check_f32(out, "out");
+// without out: the results not yet summed come back, (d [rows * top, width], the shared expert's [rows, width], its gate's
+// logits [rows]), for add_rms_norm_experts and its like
+std::tuple<Tensor, OptT, OptT> experts_few(OptT out, Tensor h, Tensor idx, Tensor wts, Tensor wgu, Tensor wdown, double limit,
+                                           int64_t act, OptT shared_w, OptT shared_down, double shared_limit,
+                                           bool shared_gate) {
+  if (out) check_f32(*out, "out");
   check_rows(h, "h");
   check_i32(idx, "idx");
   check_f32(wts, "wts");
@@ -999,7 +1016,7 @@ void experts_few(Tensor out, Tensor h, Tensor idx, Tensor wts, Tensor wgu, Tenso
   TORCH_CHECK(h.scalar_type() == at::kBFloat16 && bf16(wgu) && bf16(wdown) && wgu.dim() == 3 && wdown.dim() == 3 &&
               wgu.size(0) == wdown.size(0) && wgu.size(2) == width && wdown.size(1) == width &&
               wgu.size(1) == mult * wdown.size(2), "experts_few: expert weights");
-  TORCH_CHECK(idx.dim() == 2 && idx.size(0) == t && wts.numel() == t * top && out.numel() == t * width &&
+  TORCH_CHECK(idx.dim() == 2 && idx.size(0) == t && wts.numel() == t * top && (!out || out->numel() == t * width) &&
               t <= mx_few_rows_max() && top >= 1, "experts_few: shapes");
   const int64_t ff = wdown.size(2);
   int64_t fs = 0;
@@ -1010,20 +1027,122 @@ void experts_few(Tensor out, Tensor h, Tensor idx, Tensor wts, Tensor wgu, Tenso
     fs = shared_down->size(1);
     TORCH_CHECK(shared_w->size(0) == mult * fs + (shared_gate ? 1 : 0), "experts_few: shared expert's rows");
   }
-  Tensor y = at::empty({t * top, ff}, h.options()), d = at::empty({t * top, width}, out.options());
+  Tensor y = at::empty({t * top, ff}, h.options()), d = at::empty({t * top, width}, wts.options());
   Tensor ys, ds, sg;
   if (shared_w) {
     ys = at::empty({t, fs}, h.options());
-    ds = at::empty({t, width}, out.options());
-    if (shared_gate) sg = at::empty({t}, out.options());
+    ds = at::empty({t, width}, wts.options());
+    if (shared_gate) sg = at::empty({t}, wts.options());
   }
-  chk(mx_experts_few(out.data_ptr<float>(), y.data_ptr(), d.data_ptr<float>(), h.data_ptr(), h.stride(0),
+  chk(mx_experts_few(out ? out->data_ptr<float>() : nullptr, y.data_ptr(), d.data_ptr<float>(), h.data_ptr(), h.stride(0),
                      idx.data_ptr<int>(), wts.data_ptr<float>(), wgu.data_ptr(), wdown.data_ptr(), (int)t, (int)top,
                      (int)wgu.size(0), (int)ff, (int)width, (float)limit, (int)act,
                      shared_w ? ys.data_ptr() : nullptr, shared_w ? ds.data_ptr<float>() : nullptr,
                      shared_w && shared_gate ? sg.data_ptr<float>() : nullptr,
                      shared_w ? shared_w->data_ptr() : nullptr, shared_w ? shared_down->data_ptr() : nullptr, (int)fs,
                      (float)shared_limit, stream()), "experts_few");
+  return {d, shared_w ? OptT(ds) : OptT(), shared_w && shared_gate ? OptT(sg) : OptT()};
+}
+
+// experts' results not yet summed, of `rows` rows
+struct Experts {
+  const float *d, *wts, *shared, *gate;
+  int top;
+};
+Experts check_experts(const Tensor& d, const Tensor& wts, const OptT& shared, const OptT& gate, int64_t rows, int64_t width) {
+  check_f32(d, "experts' results");
+  check_f32(wts, "experts' weights");
+  TORCH_CHECK(wts.dim() == 2 && wts.size(0) == rows && wts.size(1) >= 1 && d.dim() == 2 && d.size(0) == rows * wts.size(1) &&
+              d.size(1) == width, "experts' results");
+  if (shared) {
+    check_f32(*shared, "shared expert's rows");
+    TORCH_CHECK(shared->numel() == rows * width, "shared expert's rows");
+  }
+  if (gate) {
+    check_f32(*gate, "shared expert's gate");
+    TORCH_CHECK(shared && gate->numel() == rows, "shared expert's gate");
+  }
+  return {d.data_ptr<float>(), wts.data_ptr<float>(), shared ? shared->data_ptr<float>() : nullptr,
+          gate ? gate->data_ptr<float>() : nullptr, (int)wts.size(1)};
+}
+const float* row_weight(const OptT& w, int64_t width) {
+  if (!w) return nullptr;
+  check_f32(*w, "norm weight");
+  TORCH_CHECK(w->numel() == width, "norm weight");
+  return w->data_ptr<float>();
+}
+
+void add_rms_norm_experts(Tensor x, Tensor d, Tensor wts, OptT shared, OptT gate, OptT wb, OptT add_vec, OptT next_w, OptT out,
+                          OptT cast, double eps) {
+  check_f32(x, "residual");
+  TORCH_CHECK(x.dim() == 2 && mx_expert_rows_fit((int)x.size(1)), "residual");
+  const int64_t rows = x.size(0), width = x.size(1);
+  const Experts e = check_experts(d, wts, shared, gate, rows, width);
+  TORCH_CHECK((bool)next_w == (bool)out, "next_w and out go together");
+  int obf = 0;
+  for (const OptT* t : {&out, &cast}) {
+    if (!*t) continue;
+    TORCH_CHECK((*t)->is_cuda() && is_act(**t) && (*t)->is_contiguous() && (*t)->sizes() == x.sizes(), "out / cast");
+    obf = bf(**t);
+  }
+  TORCH_CHECK(!out || !cast || out->scalar_type() == cast->scalar_type(), "out and cast share a dtype");
+  chk(mx_add_rms_norm_experts(x.data_ptr<float>(), e.d, e.wts, e.shared, e.gate, e.top, row_weight(wb, width),
+                              row_weight(add_vec, width), row_weight(next_w, width), out ? out->data_ptr() : nullptr,
+                              cast ? cast->data_ptr() : nullptr, obf, (int)rows, (int)width, (float)eps, stream()),
+      "add_rms_norm_experts");
+}
+
+void layer_norm_experts(Tensor x, Tensor d, Tensor wts, OptT shared, OptT gate, Tensor w, Tensor b, Tensor cast, double eps) {
+  check_f32(x, "residual");
+  TORCH_CHECK(x.dim() == 2 && mx_expert_rows_fit((int)x.size(1)), "residual");
+  const int64_t rows = x.size(0), width = x.size(1);
+  const Experts e = check_experts(d, wts, shared, gate, rows, width);
+  TORCH_CHECK(cast.is_cuda() && cast.scalar_type() == at::kBFloat16 && cast.is_contiguous() && cast.sizes() == x.sizes(), "cast");
+  chk(mx_layer_norm_experts(x.data_ptr<float>(), e.d, e.wts, e.shared, e.gate, e.top, row_weight(w, width),
+                            row_weight(b, width), cast.data_ptr(), (int)rows, (int)width, (float)eps, stream()),
+      "layer_norm_experts");
+}
+
+// decode rows: every segment has one row at most
+void add_norm_shift_experts(Tensor x, Tensor d, Tensor wts, OptT shared, OptT gate, Tensor wb, Tensor w, Tensor shift, Tensor out,
+                            Tensor state, Tensor start, Tensor pos0, Tensor slot, int64_t num_segs, double eps) {
+  check_f32(x, "residual");
+  check_f32(state, "shift state");
+  TORCH_CHECK(x.dim() == 2 && mx_expert_rows_fit((int)x.size(1)), "residual");
+  const int64_t rows = x.size(0), width = x.size(1);
+  const Experts e = check_experts(d, wts, shared, gate, rows, width);
+  TORCH_CHECK(state.dim() == 2 && state.size(0) >= 1 && state.size(1) == width, "shift state");
+  TORCH_CHECK(out.is_cuda() && out.scalar_type() == at::kBFloat16 && out.is_contiguous() && out.sizes() == x.sizes(), "out");
+  check_segs(start, pos0, slot, num_segs);
+  chk(mx_add_norm_shift_experts(x.data_ptr<float>(), e.d, e.wts, e.shared, e.gate, e.top, row_weight(wb, width),
+                                row_weight(w, width), row_weight(shift, width), out.data_ptr(), state.data_ptr<float>(),
+                                (int)state.size(0), start.data_ptr<int>(), pos0.data_ptr<int>(), slot.data_ptr<int>(),
+                                (int)num_segs, (int)rows, (int)width, (float)eps, stream()), "add_norm_shift_experts");
+}
+
+bool norm_route_fits(int64_t width, int64_t experts) { return mx_norm_route_fits((int)width, (int)experts); }
+
+// layer: h = x += layer_norm(y) * w + b; else x += rms_norm(y) * wb (or y), h = rms_norm(x) * w.  bf16 rows; see mx_norm_route
+void norm_route(Tensor idx, Tensor wts, Tensor h, Tensor x, Tensor y, bool layer, OptT wb, Tensor w, OptT b, double eps,
+                Tensor router, OptT bias, int64_t top, int64_t mode, double scale, int64_t groups, int64_t keep) {
+  check_f32(x, "residual");
+  check_rows(y, "y");
+  check_f32(router, "router");
+  check_i32(idx, "idx");
+  check_f32(wts, "wts");
+  TORCH_CHECK(x.dim() == 2 && router.dim() == 2 && router.size(1) == x.size(1), "norm_route: router");
+  const int64_t rows = x.size(0), width = x.size(1), experts = router.size(0);
+  TORCH_CHECK(norm_route_fits(width, experts) && y.sizes() == x.sizes() &&
+              h.is_cuda() && h.scalar_type() == at::kBFloat16 && h.is_contiguous() && h.sizes() == x.sizes(), "norm_route: rows");
+  TORCH_CHECK(idx.numel() == rows * top && wts.numel() == rows * top && layer == (bool)b && !(layer && wb), "norm_route shapes");
+  if (bias) {
+    check_f32(*bias, "router bias");
+    TORCH_CHECK(bias->numel() == experts, "router bias");
+  }
+  chk(mx_norm_route(idx.data_ptr<int>(), wts.data_ptr<float>(), h.data_ptr(), x.data_ptr<float>(), y.data_ptr(), bf(y),
+                    y.stride(0), layer, row_weight(wb, width), row_weight(w, width), row_weight(b, width), (float)eps,
+                    router.data_ptr<float>(), bias ? bias->data_ptr<float>() : nullptr, rows, (int)experts, (int)width,
+                    (int)top, (int)mode, (float)scale, (int)groups, (int)keep, stream()), "norm_route");
 }
 
 double tile_gemm_us(int64_t rows, int64_t n, int64_t k, bool glu) { return mx_tile_gemm_us(rows, (int)n, (int)k, glu); }
@@ -1586,6 +1705,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("moe_topk", &moe_topk);
   m.def("moe_pairs", &moe_pairs);
   m.def("few_rows_gemm", &few_rows_gemm);
+  m.def("expert_rows_fit", [](int64_t width) { return (bool)mx_expert_rows_fit((int)width); });
+  m.def("add_rms_norm_experts", &add_rms_norm_experts);
+  m.def("layer_norm_experts", &layer_norm_experts);
+  m.def("add_norm_shift_experts", &add_norm_shift_experts);
+  m.def("norm_route_fits", &norm_route_fits);
+  m.def("norm_route", &norm_route);
   m.def("tile_gemm", &tile_gemm);
   m.def("tile_gemm_us", &tile_gemm_us);
   m.def("moe_route_softmax", &moe_route_softmax);

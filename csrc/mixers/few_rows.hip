@@ -380,6 +380,7 @@ extern "C" int mx_experts_few(float* out, void* y, float* d, const void* h, long
   else EX_GO(4);
 #undef EX_GO
 #undef EX_FIRST
+  if (out == nullptr) return (int)hipGetLastError();       // (the step behind sums them: rows.hip, ExpertRows)
   hipLaunchKernelGGL(experts_combine_kernel, dim3((unsigned)((width + 255) / 256), (unsigned)rows), dim3(256), 0, s,
                      out, d, wts, sh ? ds : nullptr, sg, top, width);
   return (int)hipGetLastError();

@@ -8,7 +8,7 @@
 // by the softmax over just those, or by their sigmoids divided by the sum of those, times a
 // factor; there, too, the choice may be limited to the best groups, a group's score being the
 // sum of its two largest sigmoids.
-#include "mx_common.h"
+#include "route_choice.h"
 
 namespace mx {
 
@@ -166,6 +166,31 @@ moe_top_logits_kernel(int* __restrict__ idx, float* __restrict__ wts, const floa
   chosen_weights(wts + row * top, val, top, lane, sigmoid, scale);
 }
 
+// One wave: ch [experts] holds a row's logits; its choice by any of the routers, one expert after the other.  val
+// [top, or experts for softmax over all, + groups] is scratch.  Lane 0's LDS writes are made visible to the wave's other lanes
+// by a wave-level fence.
+__device__ __forceinline__ void choose_in_turn(int* idx, float* wts, float* ch, float* val, const float* bias, int experts,
+                                               int top, int mode, float scale, int groups, int keep, int lane) {
+  if (mode == kRouteSoftmaxAll) {
+    choose_softmax_all(idx, wts, ch, val, val + experts, bias, experts, top, groups, keep, lane);
+    return;
+  }
+  if (keep < groups) limit_to_best_groups(ch, val + top, experts, groups, keep, lane);
+  for (int k = 0; k < top; ++k) {
+    Best b{-INFINITY, 1 << 30};
+    for (int e = lane; e < experts; e += 64) b = better(b, Best{ch[e], e});
+    b = wave_best(b);
+    const int e = b.i < experts ? b.i : 0;
+    if (lane == 0) {
+      idx[k] = e;
+      val[k] = b.v;
+      ch[e] = -INFINITY;
+    }
+    wave_lds_fence();
+  }
+  chosen_weights(wts, val, top, lane, mode == kRouteSigmoid, scale);
+}
+
 // four consecutive activations as fp32
 __device__ __forceinline__ void load4(const float* p, float* v) {
   const float4 u = *reinterpret_cast<const float4*>(p);
@@ -184,7 +209,6 @@ __device__ __forceinline__ void load4(const bf16_t* p, float* v) {
 // per expert in turn with the lanes along the width (four elements per lane and pass when
 // the rows allow 16-byte loads, several passes in flight); then wave 0 chooses as above.
 constexpr int kRouteWaves = 16;
-enum { kRouteSoftmaxTop = 0, kRouteSigmoid = 1, kRouteSoftmaxAll = 2 };     // bias: the selection bias in the last
 
 template <typename T>
 __global__ void __launch_bounds__(64 * kRouteWaves)
@@ -216,28 +240,189 @@ moe_route_top_logits_kernel(int* __restrict__ idx, float* __restrict__ wts, cons
   }
   __syncthreads();
   if (wave != 0) return;
-  if (mode == kRouteSoftmaxAll) {
-    choose_softmax_all(idx + row * top, wts + row * top, ch, val, val + experts, bias, experts, top, groups, keep, lane);
-    return;
-  }
-  // one wave from here on: lane 0's LDS writes are made visible to the wave's other lanes
-  // by a wave-level fence instead of a workgroup barrier
-  if (keep < groups) limit_to_best_groups(ch, val + top, experts, groups, keep, lane);
-  for (int k = 0; k < top; ++k) {
-    Best b{-INFINITY, 1 << 30};
-    for (int e = lane; e < experts; e += 64) b = better(b, Best{ch[e], e});
-    b = wave_best(b);
-    const int e = b.i < experts ? b.i : 0;
-    if (lane == 0) {
-      idx[row * top + k] = e;
-      val[k] = b.v;
-      ch[e] = -INFINITY;
+  choose_in_turn(idx + row * top, wts + row * top, ch, val, bias, experts, top, mode, scale, groups, keep, lane);
+}
+
+// The same for bf16 rows of whole 256 and up to 64 experts, optionally behind the norm step that makes the rows: one workgroup of
+// sixteen waves per row.  A wave's router rows (an expert in turn, the lanes along the width) are on their way while the
+// norm's reductions run, and a row passes to the products through LDS.
+//   NORM 0: h given;  1: x += rms_norm(y) * wb (y as it is without wb), h = rms_norm(x) * w;  2: x += layer_norm(y) * w + b, h = x
+// Bound by what one CU draws of the router (256 KB for 32 experts of 2048) behind that chain, then by the choice.  Width 2048, 32
+// experts, in a decode step: layer norm and router of 32 rows 10.4 us (4.7 + 10.4 in two launches), RMS norms and router of 8
+// rows with groups 12.9 (3.9 + 12.7); with the router asked for before the row 1.2 more.
+constexpr int kRoutePieces = 8;              // 16-byte pieces of the router a lane asks for at a time; two such in flight
+
+struct RouteRows {
+  int* idx;
+  float* wts;
+  bf16_t* h;                                 // read (NORM 0), else written, dense
+  long h_stride;
+  float* x;
+  const void* y;                             // TY
+  long y_stride;
+  const float *wb, *w, *b;
+  const float *router, *bias;
+  int experts, width, top, mode, groups, keep;
+  float eps, scale;
+};
+
+template <int NORM, int C, typename TY>
+__global__ void __launch_bounds__(64 * kRouteWaves)
+route_rows_kernel(RouteRows R) {
+  constexpr int NT = 64 * kRouteWaves;
+  extern __shared__ __attribute__((aligned(16))) float row_s[];
+  __shared__ float red[kRouteWaves], z_s[64];
+  const long row = blockIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), width = R.width;
+  const int passes = width / 256;
+  using Raw = typename std::conditional<sizeof(TY) == 2, uint2, float4>::type;
+  // (loads come back in the order they were asked for: the row's before the router's)
+  float v[C][4], t[C][4], w[C][4], u[C][4];
+  Raw yr[C];
+  uint2 hr[C];
+  const float* wb = NORM == 2 ? R.w : R.wb;
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    const int i = min((c * NT + tid) * 4, width - 4);
+    if constexpr (NORM == 0) {
+      hr[c] = *reinterpret_cast<const uint2*>(R.h + row * R.h_stride + i);
+    } else {
+      yr[c] = *reinterpret_cast<const Raw*>((const TY*)R.y + row * R.y_stride + i);
+      load4(R.x + row * width + i, v[c]);
+      load4((wb != nullptr ? wb : R.w) + i, w[c]);
+      load4((NORM == 2 ? R.b : R.w) + i, u[c]);
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   }
-  chosen_weights(wts + row * top, val, top, lane, mode == kRouteSigmoid, scale);
+  const bool biased = R.bias != nullptr && R.mode != kRouteSoftmaxAll;
+  const float bias = (biased ? R.bias : R.router)[min(lane, R.experts - 1)];
+  float4 ahead[2][kRoutePieces];
+  int fe = wave, fp = 0;                     // the expert and piece to ask for next
+  // (no branch around a load: behind one the wait for the row would be a wait for all; pieces past an end are read twice)
+  auto fetch = [&](float4 (&a)[kRoutePieces]) {
+    const float* p = R.router + (long)min(fe, R.experts - 1) * width + lane * 4;
+#pragma unroll
+    for (int i = 0; i < kRoutePieces; ++i) a[i] = *reinterpret_cast<const float4*>(p + min(fp + i, passes - 1) * 256);
+    fp += kRoutePieces;
+    if (fp >= passes) fp = 0, fe += kRouteWaves;
+  };
+  fetch(ahead[0]);
+  fetch(ahead[1]);
+  __builtin_amdgcn_sched_barrier(0);
+  auto keep_row = [&](int i, const float (&v)[4]) {
+    *reinterpret_cast<float4*>(row_s + i) = make_float4(v[0], v[1], v[2], v[3]);
+  };
+  if constexpr (NORM == 0) {
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+      if ((c * NT + tid) * 4 < width) {
+        ft::unpack2(hr[c].x, v[c][0], v[c][1]);
+        ft::unpack2(hr[c].y, v[c][2], v[c][3]);
+        keep_row((c * NT + tid) * 4, v[c]);
+      }
+  } else {
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      if constexpr (sizeof(TY) == 2) {
+        ft::unpack2(yr[c].x, t[c][0], t[c][1]);
+        ft::unpack2(yr[c].y, t[c][2], t[c][3]);
+      } else {
+        t[c][0] = yr[c].x, t[c][1] = yr[c].y, t[c][2] = yr[c].z, t[c][3] = yr[c].w;
+      }
+      if ((c * NT + tid) * 4 >= width)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v[c][k] = t[c][k] = w[c][k] = u[c][k] = 0.f;
+    }
+    float sum = 0.f;
+    if constexpr (NORM == 2) {
+#pragma unroll
+      for (int c = 0; c < C; ++c) sum += (t[c][0] + t[c][1]) + (t[c][2] + t[c][3]);
+      const float mean = block_sum<NT>(sum, red) / (float)width;
+      sum = 0.f;
+#pragma unroll
+      for (int c = 0; c < C; ++c)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          t[c][k] = (c * NT + tid) * 4 < width ? t[c][k] - mean : 0.f;
+          sum += t[c][k] * t[c][k];
+        }
+    } else if (wb != nullptr) {
+#pragma unroll
+      for (int c = 0; c < C; ++c)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) sum += t[c][k] * t[c][k];
+    }
+    if (wb != nullptr) {
+      const float r = 1.0f / sqrtf(block_sum<NT>(sum, red) / (float)width + R.eps);
+#pragma unroll
+      for (int c = 0; c < C; ++c)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) t[c][k] = NORM == 2 ? t[c][k] * r * w[c][k] + u[c][k] : t[c][k] * (r * w[c][k]);
+    }
+    sum = 0.f;
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        v[c][k] += t[c][k];
+        sum += v[c][k] * v[c][k];
+      }
+    const float r = NORM == 2 ? 1.f : 1.0f / sqrtf(block_sum<NT>(sum, red) / (float)width + R.eps);
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      const int i = (c * NT + tid) * 4;
+      if (i >= width) continue;
+      *reinterpret_cast<float4*>(R.x + row * width + i) = make_float4(v[c][0], v[c][1], v[c][2], v[c][3]);
+      uint2 o;
+      if constexpr (NORM == 2) {
+        o = make_uint2(ft::pack2(v[c][0], v[c][1]), ft::pack2(v[c][2], v[c][3]));
+      } else {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v[c][k] *= r * u[c][k];
+        o = make_uint2(ft::pack2(v[c][0], v[c][1]), ft::pack2(v[c][2], v[c][3]));
+      }
+      *reinterpret_cast<uint2*>(R.h + row * width + i) = o;
+      float q[4];                            // (the router reads the rounded row)
+      ft::unpack2(o.x, q[0], q[1]);
+      ft::unpack2(o.y, q[2], q[3]);
+      keep_row(i, q);
+    }
+  }
+  __syncthreads();
+  int e = wave, pass = 0;
+  float acc = 0.f;
+  auto products = [&](const float4 (&a)[kRoutePieces]) {
+#pragma unroll
+    for (int i = 0; i < kRoutePieces; ++i) {
+      if (pass + i >= passes) break;
+      const float4 x = *reinterpret_cast<const float4*>(row_s + (pass + i) * 256 + lane * 4);
+      acc += x.x * a[i].x + x.y * a[i].y + x.z * a[i].z + x.w * a[i].w;
+    }
+    pass += kRoutePieces;
+    if (pass < passes) return;
+    acc = ft::wave_sum(acc);
+    if (lane == 0) z_s[e] = acc;
+    acc = 0.f;
+    pass = 0;
+    e += kRouteWaves;
+  };
+  while (e < R.experts) {
+    products(ahead[0]);
+    if (e >= R.experts) break;
+    if (fe < R.experts) fetch(ahead[0]);
+    products(ahead[1]);
+    if (fe < R.experts) fetch(ahead[1]);
+  }
+  __syncthreads();
+  if (wave != 0) return;
+  const float z = lane < R.experts ? z_s[lane] + (biased ? bias : 0.f) : 0.f;
+  if (lane < R.experts) z_s[lane] = z;       // (for the choice in turn)
+  wave_lds_fence();
+  if (__any(z != z))                         // (which experts a row with a NaN names is the sequential choice's matter)
+    choose_in_turn(R.idx + row * R.top, R.wts + row * R.top, z_s, row_s, R.bias, R.experts, R.top, R.mode, R.scale, R.groups,
+                   R.keep, lane);
+  else
+    choose_in_lanes(R.idx + row * R.top, R.wts + row * R.top, z, R.bias, R.experts, R.top, R.mode, R.scale, R.groups, R.keep,
+                    lane);
 }
 
 // All routers with their logits computed here, for any number of bf16 rows: one workgroup of sixteen waves per 16
@@ -312,61 +497,49 @@ moe_route_tile_kernel(int* __restrict__ idx, float* __restrict__ wts, const bf16
   __syncthreads();
   const long row = row0 + wave;
   if (row >= rows) return;
-  const bool on = lane < experts;
   float z = 0.f;
 #pragma unroll
   for (int w = 0; w < kRouteWaves; ++w) z += part[w][wave][min(lane, 16 * NE - 1)];
-  if (mode != kRouteSoftmaxAll && bias != nullptr && on) z += bias[lane];
-  if (!on) z = -INFINITY;
-  // ch: what the choice goes by; p: the softmax over all
-  float p = 0.f, ch = z;
-  if (mode == kRouteSoftmaxAll) {
-    const float top_z = ft::wave_max(z);
-    p = on ? expf(z - top_z) : 0.f;
-    p = p / ft::wave_sum(p);
-    ch = on ? p + bias[lane] : -INFINITY;
-  }
-  if (!(ch == ch)) ch = -INFINITY;          // (the order must hold every expert once)
-  auto at = [&](float v, int e) { return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), e)); };
-  if (keep < groups) {
-    const int gsz = experts / groups, g = lane / gsz;
-    float score = -INFINITY;
-    for (int o = 0, e = 0; o < groups; ++o) {
-      float a = -INFINITY, b = -INFINITY;    // the two largest of group o
-      for (int j = 0; j < gsz; ++j, ++e) {
-        const float v = at(ch, e);
-        b = v > a ? a : fmaxf(b, v);
-        a = fmaxf(a, v);
-      }
-      if (mode != kRouteSoftmaxAll) a = sigmoidf_(a) + (gsz > 1 ? sigmoidf_(b) : 0.f);
-      score = o == g ? a : score;
-    }
-    int better_groups = 0;
-    for (int o = 0; o < groups; ++o) {
-      const float v = at(score, o * gsz);
-      better_groups += v > score || (v == score && o < g);
-    }
-    if (better_groups >= keep) ch = -INFINITY;
-  }
-  int place = 0;
-  for (int e = 0; e < experts; ++e) {
-    const float v = at(ch, e);
-    place += v > ch || (v == ch && e < lane);
-  }
-  const bool chosen = on && place < top;
-  float w = p;
-  if (mode != kRouteSoftmaxAll) {
-    const float first = ft::wave_max(chosen ? ch : -INFINITY);
-    w = !chosen ? 0.f : mode == kRouteSigmoid ? sigmoidf_(ch) : expf(ch - first);
-    w = w / (ft::wave_sum(w) + (mode == kRouteSigmoid ? 1e-20f : 0.f)) * scale;
-  }
-  if (chosen) {
-    idx[row * top + place] = lane;
-    wts[row * top + place] = w;
-  }
+  if (mode != kRouteSoftmaxAll && bias != nullptr && lane < experts) z += bias[lane];
+  choose_in_lanes(idx + row * top, wts + row * top, z, bias, experts, top, mode, scale, groups, keep, lane);
+}
+
+// (rows of 32 KB in LDS at most)
+static bool route_rows_fit(int width, int experts) {
+  return width >= 256 && width <= 8192 && width % 256 == 0 && experts >= 1 && experts <= 64;
 }
 
 }  // namespace mx
+
+extern "C" int mx_norm_route_fits(int width, int experts) { return mx::route_rows_fit(width, experts); }
+
+// The norm step in front of a router and the router, bf16 rows out: layer 0: x += rms_norm(y) * wb (wb null: y), h = rms_norm(x) * w;
+// 1: x += layer_norm(y) * w + b, h = x.  Modes as below.
+extern "C" int mx_norm_route(int* idx, float* wts, void* h, float* x, const void* y, int y_bf16, long y_stride,
+                             int layer, const float* wb, const float* w, const float* b, float eps, const float* router, const float* bias, long rows,
+                             int experts, int width, int top, int mode, float scale, int groups, int keep, hipStream_t s) {
+  if (rows <= 0) return 0;
+  if (!mx::route_rows_fit(width, experts) || top < 1 || top > experts || mode < 0 || mode > 2 || (mode == 2 && bias == nullptr) ||
+      rows > 0x7fffffffL || y_stride % 4) return -1;
+  if (groups < 1 || experts % groups || keep < 1 || keep > groups || top > experts / groups * keep) return -1;
+  if (((uintptr_t)h | (uintptr_t)x | (uintptr_t)wb | (uintptr_t)w | (uintptr_t)b | (uintptr_t)router) % 16 || ((uintptr_t)y) % (y_bf16 ? 8 : 16))
+    return -2;
+  const mx::RouteRows R{idx, wts, (mx::bf16_t*)h, width, x, y, y_stride, wb, w, b, router, bias, experts, width,
+                        top, mode, groups, keep, eps, scale};
+#define MX_NR(NORM, C)                                                                                                     \
+  MX_DISPATCH_T(y_bf16, hipLaunchKernelGGL((mx::route_rows_kernel<NORM, C, T>), dim3((unsigned)rows), dim3(64 * mx::kRouteWaves), \
+                                           width * 4, s, R))
+#define MX_NR_C(NORM)                  \
+  do {                                 \
+    if (width <= 4096) MX_NR(NORM, 1); \
+    else MX_NR(NORM, 2);               \
+  } while (0)
+  if (layer) MX_NR_C(2);
+  else MX_NR_C(1);
+#undef MX_NR_C
+#undef MX_NR
+  return (int)hipGetLastError();
+}
 
 // mode 0: moe_top_logits by softmax, 1: by sigmoids, 2: moe_topk (bias: the selection bias)
 extern "C" int mx_moe_route_few(int* idx, float* wts, const void* h, int bf16, long h_stride,
@@ -380,6 +553,15 @@ extern "C" int mx_moe_route_few(int* idx, float* wts, const void* h, int bf16, l
   const long es = bf16 ? 2 : 4;
   const int vec = width % 4 == 0 && h_stride % 4 == 0 && ((uintptr_t)h) % (4 * es) == 0 &&
                   ((uintptr_t)router) % 16 == 0;
+  if (bf16 && vec && mx::route_rows_fit(width, experts)) {
+    const mx::RouteRows R{idx, wts, (mx::bf16_t*)const_cast<void*>(h), h_stride, nullptr, nullptr, 0, nullptr, nullptr, nullptr,
+                          router, bias, experts, width, top, mode, groups, keep, 0.f, scale};
+    if (width <= 4096)
+      hipLaunchKernelGGL((mx::route_rows_kernel<0, 1, mx::bf16_t>), dim3((unsigned)rows), dim3(64 * mx::kRouteWaves), width * 4, s, R);
+    else
+      hipLaunchKernelGGL((mx::route_rows_kernel<0, 2, mx::bf16_t>), dim3((unsigned)rows), dim3(64 * mx::kRouteWaves), width * 4, s, R);
+    return (int)hipGetLastError();
+  }
   MX_DISPATCH_T(bf16, hipLaunchKernelGGL((mx::moe_route_top_logits_kernel<T>), dim3((unsigned)rows),
                                          dim3(64 * mx::kRouteWaves), lds, s, idx, wts, (const T*)h, h_stride, router,
                                          bias, experts, width, top, vec, mode, scale, groups, keep));

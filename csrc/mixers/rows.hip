@@ -234,6 +234,43 @@ __device__ __forceinline__ void store_row(T* p, const float (&v)[C][4], int widt
   }
 }
 
+// What a norm kernel adds to the residual: a row of a tensor, or of the experts' results not yet summed
+// (few_rows.hip: experts_down), sum_k w[row, k] d[row, k] + shared[row] * (sigmoid(gate[row]) or 1), which saves
+// a launch and its rows' way through memory (4.6 us a layer of a decode step).
+template <typename T>
+struct RowsOf {
+  const T* p;
+  long stride;
+  __device__ __forceinline__ bool any() const { return p != nullptr; }
+  template <int NT, int C>
+  __device__ __forceinline__ void load(float (&v)[C][4], long row, int width, int vec) const {
+    load_row<T, NT, C>(v, p + row * stride, width, vec);
+  }
+};
+struct ExpertRows {
+  const float *d, *wts, *shared, *gate;       // [rows * top, width], [rows, top], [rows, width] or null, [rows] or null
+  int top;
+  __device__ __forceinline__ bool any() const { return true; }
+  template <int NT, int C>
+  __device__ __forceinline__ void load(float (&v)[C][4], long row, int width, int) const {      // (width: whole fours)
+    const float* w = wts + row * top;
+    const float g = shared != nullptr && gate != nullptr ? sigmoidf_(gate[row]) : 1.f;
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      const int i = (c * NT + threadIdx.x) * 4;
+      v[c][0] = v[c][1] = v[c][2] = v[c][3] = 0.f;
+      if (i >= width) continue;
+      auto add = [&](const float* p, float f) {
+        const float4 u = *reinterpret_cast<const float4*>(p + i);
+        v[c][0] += f * u.x, v[c][1] += f * u.y, v[c][2] += f * u.z, v[c][3] += f * u.w;
+      };
+#pragma unroll 4
+      for (int k = 0; k < top; ++k) add(d + (row * top + k) * width, w[k]);
+      if (shared != nullptr) add(shared + row * width, g);
+    }
+  }
+};
+
 // sums of two values over a block; every thread gets both
 template <int NT>
 __device__ __forceinline__ void block_sum2(float& a, float& b, float (*red)[2]) {
@@ -268,17 +305,17 @@ __device__ __forceinline__ float sum_sq(const float (&v)[C][4]) {
 // reductions for few rows, by the rows' bytes for many.  Width 2048: layer norm of 32 rows 4.7 us, of 2000 12
 // (values read entry by entry, again for each pass: 10 and 16); scaled add and norm of 777 rows 6 (10); mean of two norms
 // 5 (9).
-template <typename TY, typename TO, int NT, int C>
+template <typename Y, typename TO, int NT, int C>
 __global__ void __launch_bounds__(NT)
-layer_norm_row_kernel(float* __restrict__ x, const TY* __restrict__ y, long y_stride, const float* __restrict__ w,
+layer_norm_row_kernel(float* __restrict__ x, Y y, const float* __restrict__ w,
                       const float* __restrict__ b, TO* __restrict__ out, TO* __restrict__ cast, int width, float eps,
                       int vec) {
   __shared__ float red[NT / 64];
   const long row = blockIdx.x;
   float v[C][4], u[C][4], wv[C][4], bv[C][4];
   load_row<float, NT, C>(v, x + row * width, width, vec);
-  if (y != nullptr) {
-    load_row<TY, NT, C>(u, y + row * y_stride, width, vec);
+  if (y.any()) {
+    y.template load<NT, C>(u, row, width, vec);
   } else {
 #pragma unroll
     for (int c = 0; c < C; ++c)
@@ -306,7 +343,7 @@ layer_norm_row_kernel(float* __restrict__ x, const TY* __restrict__ y, long y_st
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       u[c][k] = u[c][k] * r * wv[c][k] + bv[c][k];
-      if (out == nullptr && y != nullptr) u[c][k] += v[c][k];
+      if (out == nullptr && y.any()) u[c][k] += v[c][k];
     }
   if (out != nullptr) {
     store_row<TO, NT, C>(out + row * width, u, width, vec);
@@ -372,17 +409,17 @@ dual_rms_mean_row_kernel(float* __restrict__ out, const T* __restrict__ a, long 
 
 // residual (fp32, in place): x += rms_norm(y) * wb (y as it is without wb) (+ add_vec);
 // out = rms_norm(x) * next_w (TO);  cast = x (TO).  Every part is optional.
-template <typename TY, typename TO, int NT, int C>
+template <typename Y, typename TO, int NT, int C>
 __global__ void __launch_bounds__(NT)
-add_rms_norm_kernel(float* __restrict__ x, const TY* __restrict__ y, long y_stride, const float* __restrict__ wb,
+add_rms_norm_kernel(float* __restrict__ x, Y y, const float* __restrict__ wb,
                     const float* __restrict__ add_vec, const float* __restrict__ next_w, TO* __restrict__ out,
                     TO* __restrict__ cast, int width, float eps, int vec) {
   __shared__ float red[NT / 64];
   const long row = blockIdx.x;
   float v[C][4], t[C][4], w[C][4];
   load_row<float, NT, C>(v, x + row * width, width, vec);
-  if (y != nullptr) {
-    load_row<TY, NT, C>(t, y + row * y_stride, width, vec);
+  if (y.any()) {
+    y.template load<NT, C>(t, row, width, vec);
     if (wb != nullptr) {
       load_row<float, NT, C>(w, wb, width, vec);
       const float r = 1.0f / sqrtf(block_sum<NT>(sum_sq<C>(t), red) / (float)width + eps);
@@ -403,7 +440,7 @@ add_rms_norm_kernel(float* __restrict__ x, const TY* __restrict__ y, long y_stri
 #pragma unroll
       for (int k = 0; k < 4; ++k) v[c][k] += w[c][k];
   }
-  if (y != nullptr || add_vec != nullptr) store_row<float, NT, C>(x + row * width, v, width, vec);
+  if (y.any() || add_vec != nullptr) store_row<float, NT, C>(x + row * width, v, width, vec);
   if (cast != nullptr) store_row<TO, NT, C>(cast + row * width, v, width, vec);
   if (out != nullptr) {
     load_row<float, NT, C>(w, next_w, width, vec);
@@ -426,10 +463,10 @@ add_rms_norm_kernel(float* __restrict__ x, const TY* __restrict__ y, long y_stri
 // one-row segment also leaves its h in the slot; shift_state_kernel does that for longer ones
 // afterwards (a slot may still be read by the segment's first row here).
 // ---------------------------------------------------------------------------------
-template <typename TY, typename TO, int NT, int C>
+template <typename Y, typename TO, int NT, int C>
 __global__ void __launch_bounds__(NT)
-add_norm_shift_kernel(float* x_out, const float* x_in, const TY* __restrict__ y, long y_stride,
-                      const float* __restrict__ wb, const float* __restrict__ w, const float* __restrict__ shift,
+add_norm_shift_kernel(float* x_out, const float* x_in, Y y, const float* __restrict__ wb, const float* __restrict__ w,
+                      const float* __restrict__ shift,
                       TO* __restrict__ out, float* state, int num_slots, const int* __restrict__ start,
                       const int* __restrict__ pos0, const int* __restrict__ slot, int num_segs, int width,
                       float eps, int vec) {
@@ -448,10 +485,10 @@ add_norm_shift_kernel(float* x_out, const float* x_in, const TY* __restrict__ y,
   float xa[C][4], xp[C][4], t[C][4];
   load_row<float, NT, C>(xa, x_in + row * width, width, vec);
   if (rel > 0) load_row<float, NT, C>(xp, x_in + (row - 1) * width, width, vec);
-  if (y != nullptr) {
+  if (y.any()) {
     float yp[C][4];
-    load_row<TY, NT, C>(t, y + row * y_stride, width, vec);
-    if (rel > 0) load_row<TY, NT, C>(yp, y + (row - 1) * y_stride, width, vec);
+    y.template load<NT, C>(t, row, width, vec);
+    if (rel > 0) y.template load<NT, C>(yp, row - 1, width, vec);
     float sa = sum_sq<C>(t), sb = rel > 0 ? sum_sq<C>(yp) : 0.f;
     block_sum2<NT>(sa, sb, red);
     const float ra = 1.0f / sqrtf(sa / (float)width + eps), rb = 1.0f / sqrtf(sb / (float)width + eps);
@@ -739,8 +776,9 @@ static void launch_layer_norm(float* x, const void* y, long ys, const float* w, 
                   ((uintptr_t)out | (uintptr_t)cast) % (4 * sizeof(TO)) == 0;
   if (row_in_registers(rows, width, vec)) {
     row_chunks(width, [&](auto c) {
-      hipLaunchKernelGGL((layer_norm_row_kernel<TY, TO, kRowThreads, decltype(c)::value>), dim3(rows), dim3(kRowThreads),
-                         0, s, x, (const TY*)y, ys, w, b, (TO*)out, (TO*)cast, width, eps, vec);
+      hipLaunchKernelGGL((layer_norm_row_kernel<RowsOf<TY>, TO, kRowThreads, decltype(c)::value>), dim3(rows),
+                         dim3(kRowThreads), 0, s, x, RowsOf<TY>{(const TY*)y, ys}, w, b, (TO*)out, (TO*)cast, width, eps,
+                         vec);
     });
     return;
   }
@@ -770,8 +808,9 @@ static void launch_add_rms(float* x, const void* y, long ys, const float* wb, co
                   ((uintptr_t)x | (uintptr_t)wb | (uintptr_t)av | (uintptr_t)nw) % 16 == 0 &&
                   ((uintptr_t)out | (uintptr_t)cast) % (4 * sizeof(TO)) == 0;
   row_chunks(width, [&](auto c) {
-    hipLaunchKernelGGL((add_rms_norm_kernel<TY, TO, kRowThreads, decltype(c)::value>), dim3(rows), dim3(kRowThreads), 0,
-                       s, x, (const TY*)y, ys, wb, av, nw, (TO*)out, (TO*)cast, width, eps, vec);
+    hipLaunchKernelGGL((add_rms_norm_kernel<RowsOf<TY>, TO, kRowThreads, decltype(c)::value>), dim3(rows),
+                       dim3(kRowThreads), 0, s, x, RowsOf<TY>{(const TY*)y, ys}, wb, av, nw, (TO*)out, (TO*)cast, width, eps,
+                       vec);
   });
 }
 
@@ -787,6 +826,62 @@ extern "C" int mx_add_rms_norm(float* x, const void* y, int y_bf16, long y_strid
     if (out_bf16) launch_add_rms<float, bf16_t>(x, y, y_stride, wb, add_vec, next_w, out, cast, rows, width, eps, s);
     else launch_add_rms<float, float>(x, y, y_stride, wb, add_vec, next_w, out, cast, rows, width, eps, s);
   }
+  return (int)hipGetLastError();
+}
+
+// widths of the forms below
+extern "C" int mx_expert_rows_fit(int width) { return width % 8 == 0 && width > 1024 && width <= kRowMaxWidth; }
+
+// the three norm steps with the experts' unsummed results as y; bf16 (cast, out) or fp32 results
+extern "C" int mx_add_rms_norm_experts(float* x, const float* d, const float* wts, const float* shared, const float* gate,
+                                       int top, const float* wb, const float* add_vec, const float* next_w, void* out,
+                                       void* cast, int out_bf16, int rows, int width, float eps, hipStream_t s) {
+  if (rows <= 0) return 0;
+  if (!mx_expert_rows_fit(width) || top < 1) return -1;
+  if (((uintptr_t)d | (uintptr_t)shared) % 16) return -2;
+  const int vec = ((uintptr_t)x | (uintptr_t)wb | (uintptr_t)add_vec | (uintptr_t)next_w | (uintptr_t)out | (uintptr_t)cast) % 16 == 0;
+  const ExpertRows y{d, wts, shared, gate, top};
+  row_chunks(width, [&](auto c) {
+    if (out_bf16)
+      hipLaunchKernelGGL((add_rms_norm_kernel<ExpertRows, bf16_t, kRowThreads, decltype(c)::value>), dim3(rows),
+                         dim3(kRowThreads), 0, s, x, y, wb, add_vec, next_w, (bf16_t*)out, (bf16_t*)cast, width, eps, vec);
+    else
+      hipLaunchKernelGGL((add_rms_norm_kernel<ExpertRows, float, kRowThreads, decltype(c)::value>), dim3(rows),
+                         dim3(kRowThreads), 0, s, x, y, wb, add_vec, next_w, (float*)out, (float*)cast, width, eps, vec);
+  });
+  return (int)hipGetLastError();
+}
+
+extern "C" int mx_layer_norm_experts(float* x, const float* d, const float* wts, const float* shared, const float* gate,
+                                     int top, const float* w, const float* b, void* cast, int rows, int width, float eps,
+                                     hipStream_t s) {
+  if (rows <= 0) return 0;
+  if (!mx_expert_rows_fit(width) || top < 1) return -1;
+  if (((uintptr_t)d | (uintptr_t)shared) % 16) return -2;
+  const int vec = ((uintptr_t)x | (uintptr_t)w | (uintptr_t)b | (uintptr_t)cast) % 16 == 0;
+  const ExpertRows y{d, wts, shared, gate, top};
+  row_chunks(width, [&](auto c) {
+    hipLaunchKernelGGL((layer_norm_row_kernel<ExpertRows, bf16_t, kRowThreads, decltype(c)::value>), dim3(rows),
+                       dim3(kRowThreads), 0, s, x, y, w, b, (bf16_t*)nullptr, (bf16_t*)cast, width, eps, vec);
+  });
+  return (int)hipGetLastError();
+}
+
+// decode rows: segments of one row at most, x in place
+extern "C" int mx_add_norm_shift_experts(float* x, const float* d, const float* wts, const float* shared, const float* gate,
+                                         int top, const float* wb, const float* w, const float* shift, void* out,
+                                         float* state, int num_slots, const int* start, const int* pos0, const int* slot,
+                                         int num_segs, int rows, int width, float eps, hipStream_t s) {
+  if (rows <= 0 || num_segs <= 0) return 0;
+  if (!mx_expert_rows_fit(width) || top < 1) return -1;
+  if (((uintptr_t)d | (uintptr_t)shared) % 16) return -2;
+  const int vec = ((uintptr_t)x | (uintptr_t)wb | (uintptr_t)w | (uintptr_t)shift | (uintptr_t)out | (uintptr_t)state) % 16 == 0;
+  const ExpertRows y{d, wts, shared, gate, top};
+  row_chunks(width, [&](auto c) {
+    hipLaunchKernelGGL((add_norm_shift_kernel<ExpertRows, bf16_t, kRowThreads, decltype(c)::value>), dim3(rows),
+                       dim3(kRowThreads), 0, s, x, x, y, wb, w, shift, (bf16_t*)out, state, num_slots, start, pos0, slot,
+                       num_segs, width, eps, vec);
+  });
   return (int)hipGetLastError();
 }
 
@@ -997,9 +1092,9 @@ static void launch_shift(float* x_out, const float* x_in, const void* y, long ys
                    (uintptr_t)state) % 16 == 0 && ((uintptr_t)out) % (4 * sizeof(TO)) == 0;
   row_chunks(width, [&](auto c) {
     constexpr int C = decltype(c)::value;
-    hipLaunchKernelGGL((add_norm_shift_kernel<TY, TO, kRowThreads, C>), dim3(rows), dim3(kRowThreads), 0, s, x_out,
-                       x_in, (const TY*)y, ys, wb, w, shift, (TO*)out, state, num_slots, start, pos0, slot, num_segs,
-                       width, eps, vec);
+    hipLaunchKernelGGL((add_norm_shift_kernel<RowsOf<TY>, TO, kRowThreads, C>), dim3(rows), dim3(kRowThreads), 0, s, x_out,
+                       x_in, RowsOf<TY>{(const TY*)y, ys}, wb, w, shift, (TO*)out, state, num_slots, start, pos0, slot,
+                       num_segs, width, eps, vec);
     if (max_rows > 1)
       hipLaunchKernelGGL((shift_state_kernel<kRowThreads, C>), dim3(num_segs), dim3(kRowThreads), 0, s, state,
                          num_slots, x_out, w, start, slot, width, eps, vec);

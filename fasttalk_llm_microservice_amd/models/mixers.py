@@ -861,14 +861,26 @@ class MoEFF:
             return M.clamp_swiglu(u, self.limit if limit is None else limit)
         return M.silu_glu(u) if self.act == "silu_glu" else M.relu_sq(u)
 
-    def __call__(self, h, ctx=None) -> torch.Tensor:
+    def norm_route(self, x, y, wb, w, b, eps: float, dtype):
+        """The norm step in front of this mixture (see :func:`..ops.mixers.norm_route`) with its router, for few rows:
+        (h, (idx, wts)), or None where that launch does not take them."""
+        if dtype != torch.bfloat16 or x.shape[0] > self.PAIR_ROWS or not M.norm_route_fits(x, y, wb, w, b, self.router):
+            return None
+        grouped, limited = self.routing == "grouped_softmax", self.routing != "top_logits"
+        return M.norm_route(x, y, wb, w, b, eps, self.router, self.correction if grouped else self.router_bias, self.top,
+                            self.routing, 1.0 if grouped else self.route_scale, self.groups if limited else 1,
+                            self.keep if limited else 1)
+
+    def __call__(self, h, ctx=None, routed=None, parts: bool = False):
+        """``routed``: the choice (idx, wts), if :meth:`norm_route` made it; ``parts``: the result may be
+        :class:`..ops.mixers.ExpertParts`."""
         t, width = h.shape
         if t <= self.PAIR_ROWS and M.experts_few_ok(h, self.wgu, self.wdown, self.shared) and \
                 M.experts_few_pays(t * self.top, self.e, self.wdown[0].numel(), self.shared is not None):
             # decode-size steps: a matrix is read once for all rows, nothing read back on the host
-            idx, wts = self.route(h)
+            idx, wts = routed or self.route(h)
             return M.experts_few(h, idx, wts, self.wgu, self.wdown, self.act, self.limit, self.shared,
-                                 self.shared_limit if self.shared is not None else 0.0, self.shared_gate)
+                                 self.shared_limit if self.shared is not None else 0.0, self.shared_gate, parts)
         if t > self.PAIR_ROWS and M.experts_many_ok(h, self.wgu, self.wdown):
             idx, wts = self.route(h)
             shared = gate_w = None
@@ -883,7 +895,7 @@ class MoEFF:
             out = M.linear(self._act(M.linear(h, self.shared[0]), self.shared_limit), self.shared[1]).float()
         else:
             out = torch.zeros(t, width, dtype=torch.float32, device=h.device)
-        idx, wts = self.route(h)
+        idx, wts = routed or self.route(h)
         if t <= self.PAIR_ROWS:
             # few pairs, fp32, or rows that are not whole 16-byte pieces: per-pair weight streaming
             M.moe_pairs(out, h, idx, wts, self.wgu, self.wdown, self.limit, self.act)

@@ -43,7 +43,7 @@ import torch.nn.functional as F
 from ..ops import mixers as M
 from ..parallel.comm import SINGLE, TPComm
 from . import weights as W
-from .mixers import StepContext
+from .mixers import MoEFF, StepContext
 
 
 @dataclasses.dataclass
@@ -254,18 +254,16 @@ class StackedModel:
                                               "without post-norms")
                 wb = L.norm1b
                 if L.ff is not None:
-                    h, _ = M.add_rms_norm_rows(x, y, L.norm1b, eps, next_w=L.norm2, out_dtype=dt)
-                    y, wb = L.ff(h, ctx), L.norm2b
+                    y, wb = self._norm_ff(x, y, L.norm1b, L.norm2, None, L.ff, ctx, seg.max_rows <= 1), L.norm2b
                 x, h = M.add_norm_shift_rows(x, y, wb, self.layers[nxt[0]].norm1, nshift, eps, dt, prev_h[r + 1], seg)
                 if tap is not None:
                     tap.append(x.clone())
                 continue
-            h, xc = M.add_rms_norm_rows(x, y, L.norm1b, eps,
-                                        add_vec=nvec if last else None,
-                                        next_w=L.norm2 if L.ff is not None else (nw if last else None),
-                                        out_dtype=dt, want_cast=L.ff is None and L.side is not None)
-            if L.ff is not None:
-                y = L.ff(h, ctx)
+            if L.ff is None:
+                h, xc = M.add_rms_norm_rows(x, y, L.norm1b, eps, add_vec=nvec if last else None,
+                                            next_w=nw if last else None, out_dtype=dt, want_cast=L.side is not None)
+            else:
+                y = self._norm_ff(x, y, L.norm1b, L.norm2, None, L.ff, ctx)
                 last = L.side is None
                 h, xc = M.add_rms_norm_rows(x, y, L.norm2b, eps, add_vec=nvec if last else None,
                                             next_w=nw if last else None, out_dtype=dt,
@@ -281,6 +279,20 @@ class StackedModel:
         if rows.shape[0] == 0:
             return rows.to(dt)
         return M.rms_norm_rows(rows, self.final_norm, eps, dt)
+
+    def _norm_ff(self, x, y, wb, w, b, ff, ctx, parts: bool = True):
+        """A layer's add and norm between its mixer and its feed-forward, and that: x += rms_norm(y) * wb and ff of
+        rms_norm(x) * w, or, with b, x += layer_norm(y) * w + b and ff of x.  The result is a norm step's ``y``."""
+        eps, dt = self.cfg.rms_norm_eps, self.dtype
+        if isinstance(ff, MoEFF):
+            got = ff.norm_route(x, y, wb, w, b, eps, dt)
+            if got is not None:
+                return ff(got[0], ctx, got[1], parts)
+        if b is not None:
+            h = M.add_layer_norm_rows(x, y, w, b, eps, dt)
+        else:
+            h, _ = M.add_rms_norm_rows(x, y, wb, eps, next_w=w, out_dtype=dt)
+        return ff(h, ctx)
 
     def _embed(self, input_ids, ctx, caches: StackedCache) -> torch.Tensor:
         """fp32 residual rows: embedding table, plus the pair table's rows if there is one."""
@@ -306,9 +318,12 @@ class StackedModel:
             if mark is not None and r == mark[0]:
                 mark[1].record()
             L = self.layers[li]
-            h = M.add_layer_norm_rows(x, L.mixer(h, ctx, caches.per_run[r]), L.norm1b, L.bias1, eps, dt)
-            if L.ff is not None:
-                h = M.add_layer_norm_rows(x, L.ff(h, ctx), L.norm2b, L.bias2, eps, dt)
+            y = L.mixer(h, ctx, caches.per_run[r])
+            if L.ff is None:
+                h = M.add_layer_norm_rows(x, y, L.norm1b, L.bias1, eps, dt)
+            else:
+                y = self._norm_ff(x, y, None, L.norm1b, L.bias1, L.ff, ctx)
+                h = M.add_layer_norm_rows(x, y, L.norm2b, L.bias2, eps, dt)
             if tap is not None:
                 tap.append(x.clone())
         idx = meta.logits_indices

@@ -1,0 +1,93 @@
+"""Decode rows of a mixture layer: the norm step and the router behind it in one launch (csrc/mixers/moe_route.hip
+route_rows_kernel), and the norm steps that sum the experts' results themselves (csrc/mixers/rows.hip ExpertRows)."""
+import pytest
+import torch
+
+from fasttalk_llm_microservice_amd.ops import mixers as M
+from fasttalk_llm_microservice_amd.ops import mixers_ref as R
+from test_mixer_kernels_gpu import DEV, rnd
+
+pytestmark = pytest.mark.gpu
+
+
+# one pass and several, a router of fewer and more pieces than are in flight, one and two pieces of a row per thread
+@pytest.mark.parametrize("routing,form", [("grouped_softmax", "rms"), ("top_logits", "layer"), ("top_sigmoid", "plain")])
+@pytest.mark.parametrize("rows,width,experts,top,groups,keep,ydt", [
+    (1, 256, 1, 1, 1, 1, torch.bfloat16), (3, 2048, 17, 4, 1, 1, torch.float32), (64, 2048, 32, 4, 4, 2, torch.bfloat16),
+    (2, 4096, 64, 8, 8, 4, torch.bfloat16), (5, 4352, 33, 3, 3, 2, torch.float32), (2, 8192, 64, 64, 64, 64, torch.bfloat16)])
+def test_norm_route(routing, form, rows, width, experts, top, groups, keep, ydt):
+    if routing == "top_logits":
+        groups = keep = 1
+    g = torch.Generator().manual_seed(rows + width)
+    x, y = rnd(rows, width, g=g), rnd(rows, width + 8, dt=ydt, g=g)[:, :width]
+    w, wb, b = (1 + rnd(width, g=g, scale=0.1), rnd(width, g=g), rnd(width, g=g))
+    router, bias = rnd(experts, width, g=g, scale=width ** -0.5), rnd(experts, g=g, scale=0.1)
+    wb, b = (wb if form == "rms" else None), (b if form == "layer" else None)
+    d = [None if t is None else t.to(DEV) for t in (x, y, wb, w, b, router, bias)]
+    assert M.norm_route_fits(*d[:6])
+    h, (idx, wts) = M.norm_route(*d[:5], 1e-5, *d[5:], top, routing, 1.7, groups, keep)
+    if form == "layer":
+        want = R.add_layer_norm_rows(x, y, w, b, 1e-5, torch.float32)
+    else:
+        want, _ = R.add_rms_norm_rows(x, y, wb, 1e-5, None, w, torch.float32, False)
+    torch.testing.assert_close(d[0].cpu(), x, rtol=1e-5, atol=1e-5)          # fp32 sums in another order
+    torch.testing.assert_close(h.float().cpu(), want, rtol=2 ** -8, atol=1e-5)      # one rounding to bf16
+    z = h.cpu().double() @ router.double().t()
+    if routing == "grouped_softmax":
+        i64, w64 = R.moe_topk(z.float(), bias, top, groups, keep)
+    else:
+        z = (z + bias.double()).float()
+        i64, w64 = R.moe_top_sigmoid(z, top, 1.7, groups, keep) if routing == "top_sigmoid" else R.moe_top_logits(z, top)
+        w64 = w64 * (1.7 if routing == "top_logits" else 1.0)
+    # fp32 logits of a few thousand terms: a choice may only differ between experts that are as good as level
+    same = idx.cpu() == i64.int()
+    by = z.float() if routing != "grouped_softmax" else torch.softmax(z.float(), -1) + bias
+    level = by.gather(1, idx.cpu().long()) - by.gather(1, i64.long())
+    assert bool((same | (level.abs() < 2e-5)).all())
+    torch.testing.assert_close(wts.cpu(), w64.float(), rtol=2e-4, atol=1e-5)
+
+
+def test_router_of_rows_with_nan_names_the_same_experts():
+    g = torch.Generator().manual_seed(1)
+    h, router, bias = rnd(3, 512, dt=torch.bfloat16, g=g).to(DEV), rnd(12, 512, g=g).to(DEV), rnd(12, g=g).to(DEV)
+    h[1, 5] = float("nan")
+    idx, wts = M.moe_route_top_logits(h, router, bias, 3)
+    i32, w32 = M.moe_route_top_logits(h.float(), router, bias, 3)            # (the kernel of fp32 rows)
+    assert torch.equal(idx, i32)
+    torch.testing.assert_close(wts, w32, rtol=1e-5, atol=1e-7, equal_nan=True)
+
+
+@pytest.mark.parametrize("rows,width,top", [(1, 1032, 1), (3, 2048, 4), (5, 4096, 8), (2, 16384, 5)])
+@pytest.mark.parametrize("shared", ["no", "as it is", "gated"])
+def test_norm_steps_sum_the_experts(rows, width, top, shared):
+    g = torch.Generator().manual_seed(rows * top)
+    d, wts = rnd(rows * top, width, g=g).to(DEV), rnd(rows, top, g=g).abs().to(DEV)
+    ds = rnd(rows, width, g=g).to(DEV) if shared != "no" else None
+    gate = rnd(rows, g=g).to(DEV) if shared == "gated" else None
+    parts = M.ExpertParts(d, wts, ds, gate)
+    y = (wts[:, :, None] * d.view(rows, top, width)).sum(1)
+    if ds is not None:
+        y = y + ds * (torch.sigmoid(gate)[:, None] if gate is not None else 1.0)
+    x, w, wb, b, add = rnd(rows, width, g=g), rnd(width, g=g), rnd(width, g=g), rnd(width, g=g), rnd(width, g=g)
+    w, wb, b, add = (t.to(DEV) for t in (w, wb, b, add))
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)      # noqa: E731
+    # a sequence's first token, one further on, and a row without a slot
+    pos, slot = [0, 7, 3, 5, 9][:rows], [2, 0, -1, 4, 1][:rows]
+    seg = M.Segments(start=i32(list(range(rows + 1))), pos0=i32(pos), slot=i32(slot), kv_len=i32([p + 1 for p in pos]),
+                     block_tables=i32([[0]] * rows), num=rows, max_rows=1)
+    state = rnd(5, width, g=g)
+    states = [state.to(DEV), state.to(DEV)]
+    calls = [lambda x, y: M.add_rms_norm_rows(x, y, wb, 1e-5, add, w, torch.bfloat16, True),
+             lambda x, y: M.add_rms_norm_rows(x, y, None, 1e-5, None, w, torch.bfloat16),
+             lambda x, y: M.add_rms_norm_rows(x, y, wb, 1e-5, None, None, torch.bfloat16),
+             lambda x, y: M.add_layer_norm_rows(x, y, w, b, 1e-5, torch.bfloat16),
+             lambda x, y: M.add_norm_shift_rows(x, y, wb, w, b, 1e-5, torch.bfloat16, states[isinstance(y, torch.Tensor)], seg)]
+    for call in calls:
+        xs = [x.to(DEV), x.to(DEV)]
+        got, want = call(xs[0], parts), call(xs[1], y)
+        torch.testing.assert_close(xs[0], xs[1], rtol=1e-5, atol=2e-5)       # fp32 sums in another order
+        for a, c in zip(*(t if isinstance(t, tuple) else (t,) for t in (got, want))):
+            assert (a is None) == (c is None)
+            if a is not None:
+                torch.testing.assert_close(a.float(), c.float(), rtol=2 ** -7, atol=1e-4)    # a rounding to bf16 on each side
+    torch.testing.assert_close(*states, rtol=1e-5, atol=1e-4)
