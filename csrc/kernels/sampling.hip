@@ -172,6 +172,11 @@ constexpr int kChunks = kSlots / 8;  // 16 chunks of 8 ids per lane
 // multi-workgroup sampler (samp_*_kernel below)
 constexpr int kSlices = 32;
 constexpr int kSlThreads = 256;
+// Up to this many rows the draw and the above-masses are one launch, every slice's workgroup
+// with the whole draw: 256 workgroups, one a CU.  us a step of 8 rows of 131072 bf16 (50000 fp32)
+// at top-p 0.9 21.5 (17.1), in two launches 23.6 (19.1); of 16 rows, two workgroups a CU, 34.8
+// (28.2) and 24.3 (19.8).
+constexpr int kAboveRows = 8;
 // top-k rows with k <= kTopkMax take the multi-workgroup top-k path: each slice
 // keeps its own top-k candidates (the global top-k is a subset of their union)
 constexpr int kTopkMax = 64;
@@ -498,6 +503,7 @@ __device__ __forceinline__ int wave_sum_int(int v) {
 }
 
 // max over the workgroup (<= 16 waves), s: >= waves ints of LDS
+template <int NW>
 __device__ __forceinline__ uint32_t wave_max_u32_wg(uint32_t v, int* s) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v = max(v, (uint32_t)__shfl_xor((int)v, o, 64));
@@ -505,7 +511,7 @@ __device__ __forceinline__ uint32_t wave_max_u32_wg(uint32_t v, int* s) {
   if (lane_id() == 0) s[wave_id()] = (int)v;
   __syncthreads();
   uint32_t m = 0u;
-  for (int w = 0; w < (int)(blockDim.x >> 6); ++w) m = max(m, (uint32_t)s[w]);
+  for (int w = 0; w < NW; ++w) m = max(m, (uint32_t)s[w]);
   return m;
 }
 
@@ -515,8 +521,8 @@ __device__ __forceinline__ bool mw_topk_row(const int* top_k, const float* tempe
   return topk_row(top_k, row, vocab) && top_k[row] <= kTopkMax && temperature[row] > 0.f;
 }
 
-// largest t with count(key >= t) >= kk over NK register keys per thread of the
-// workgroup (4-ary search on the 16-bit key, 3 counts per pass); kk >= 1
+// largest t with count(key >= t) >= kk over NK register keys per thread of
+// kSlThreads (4-ary search on the 16-bit key, 3 counts per pass); kk >= 1
 template <int NK>
 __device__ __forceinline__ uint32_t wg_kth_key(const uint32_t (&key)[NK], int kk, int* s3) {
   uint32_t t = 0u;
@@ -534,12 +540,11 @@ __device__ __forceinline__ uint32_t wg_kth_key(const uint32_t (&key)[NK], int kk
 #pragma unroll
       for (int q = 0; q < 3; ++q) s3[3 * wave_id() + q] = c[q];
     __syncthreads();
-    const int nw = blockDim.x >> 6;
     uint32_t nt = t;
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
       int tot = 0;
-      for (int w = 0; w < nw; ++w) tot += s3[3 * w + q];
+      for (int w = 0; w < kSlThreads / 64; ++w) tot += s3[3 * w + q];
       if (tot >= kk) nt = t + ((uint32_t)(q + 1) << shift);
     }
     t = nt;
@@ -574,14 +579,14 @@ __device__ __forceinline__ void wg_argmax(uint32_t& k, int& idx, uint32_t* su, i
     }
 }
 
+template <int NW>
 __device__ __forceinline__ float wg_sum(float v, float* sf) {
   v = wave_sum(v);
   __syncthreads();
   if (lane_id() == 0) sf[wave_id()] = v;
   __syncthreads();
   float t = 0.f;
-  const int nw = blockDim.x >> 6;
-  for (int w = 0; w < nw; ++w) t += sf[w];
+  for (int w = 0; w < NW; ++w) t += sf[w];
   return t;
 }
 
@@ -700,7 +705,7 @@ __global__ __launch_bounds__(kSlThreads) void samp_stats_kernel(
 #pragma unroll
       for (int j = 0; j < 8; ++j) z += key[j] > kNegInfKey ? exp2f((key_to_f32(key[j]) - Mp) * cexp) : 0.f;
     }
-    Zp = wg_sum(z, sf);
+    Zp = wg_sum<kSlThreads / 64>(z, sf);
   }
   if (threadIdx.x == 0) {
     st[0] = Mp;
@@ -710,7 +715,184 @@ __global__ __launch_bounds__(kSlThreads) void samp_stats_kernel(
   }
 }
 
+// slice p's mass of ids strictly more likely than each candidate (keys ck); kSlThreads threads call it
 template <typename T>
+__device__ __forceinline__ void above_mass(const T* x, const uint32_t* mrow, int vocab, int p, float M, float cexp,
+                                           const uint32_t* ck, float* wr, float* sf) {
+  uint32_t kc[kCand], kmin = 0xffffffffu;
+#pragma unroll
+  for (int c = 0; c < kCand; ++c) {
+    kc[c] = ck[c];
+    kmin = min(kmin, kc[c]);
+  }
+  const int S = slice_len(vocab);
+  const int beg = p * S, end = min(vocab, beg + S);
+  float a[kCand] = {};
+  for (int base = beg + threadIdx.x * 8; base < end; base += kSlThreads * 8) {
+    uint32_t key[8];
+    load_keys8<T>(x, mrow, base, vocab, key);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float e = key[j] > kmin ? exp2f((key_to_f32(key[j]) - M) * cexp) : 0.f;
+#pragma unroll
+      for (int c = 0; c < kCand; ++c) a[c] += key[j] > kc[c] ? e : 0.f;
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < kCand; ++c) {
+    a[c] = wg_sum<kSlThreads / 64>(a[c], sf);
+    if (threadIdx.x == 0) wr[kWsAbove + kCand * p + c] = a[c];
+  }
+}
+
+// Top-k rows (k <= kTopkMax, temperature > 0), one workgroup per row: merge the
+// slices' candidates, keep key >= t* (t* = largest key with count(key >= t*) >= k,
+// the single-workgroup kernel's rule: ties at the threshold stay), then top-p over
+// the kept ids (an id is in the nucleus iff the mass of strictly more likely kept
+// ids is < top_p * Z) and one inverse-CDF draw in (key desc, id asc) order over a
+// rank-ordered prefix sum -- deterministic whatever order the candidates were
+// appended in.  Rows whose
+// candidates or kept set overflow go to the one-workgroup kernel (flag 2).
+// (kSlThreads threads call it)
+__device__ __forceinline__ void draw_topk(
+    int row, int* __restrict__ out_tokens, int vocab, const float* __restrict__ temperature,
+    const float* __restrict__ top_p, const int* __restrict__ top_k,
+    const long long* __restrict__ seeds, const int* __restrict__ steps, float* __restrict__ ws) {
+  constexpr int NC = kSlices * kTopkMax / kSlThreads;   // candidates per thread
+  __shared__ int s_off[kSlices + 1];
+  constexpr int kNW = kSlThreads / 64;
+  __shared__ int s3[3 * kNW];
+  __shared__ float sf[kNW];
+  __shared__ int s_nk, s_bad, s_pick, s_last;
+  __shared__ uint32_t s_k[kTopkKept];
+  __shared__ int s_i[kTopkKept];
+  __shared__ float s_e[kTopkKept];
+  __shared__ float s_c[kTopkKept];
+  const int tid = threadIdx.x;
+  float* wr = ws + (long)row * kWsRow;
+  int* flag = reinterpret_cast<int*>(wr + kWsFlag);
+  const int* cnt = reinterpret_cast<const int*>(wr + kWsTkCnt);
+  if (tid == 0) {
+    int o = 0, bad = 0;
+    for (int p = 0; p < kSlices; ++p) {
+      s_off[p] = o;
+      bad |= cnt[p] < 0;
+      o += max(cnt[p], 0);
+    }
+    s_off[kSlices] = o;
+    s_bad = bad;
+    s_nk = 0;
+    s_pick = -1;
+    s_last = -1;
+  }
+  __syncthreads();
+  if (s_bad) {
+    if (tid == 0) *flag = 2;
+    return;
+  }
+  const int C = s_off[kSlices];
+  uint32_t key[NC];
+  int id[NC];
+#pragma unroll
+  for (int j = 0; j < NC; ++j) {
+    const int c = tid + kSlThreads * j;
+    key[j] = 0u;
+    id[j] = 0;
+    if (c < C) {
+      int p = 0;
+      while (s_off[p + 1] <= c) ++p;
+      const float* e = wr + kWsTk + 2 * kTopkMax * p + 2 * (c - s_off[p]);
+      key[j] = __float_as_uint(e[0]);
+      id[j] = __float_as_int(e[1]);
+    }
+  }
+  const int kk = min(top_k[row], C);
+  if (kk == 0) {   // everything masked
+    if (tid == 0) {
+      out_tokens[row] = FT_CHECK_IDX(0, vocab, kCkSampled, row);
+      *flag = 0;
+    }
+    return;
+  }
+  const uint32_t th = wg_kth_key<NC>(key, kk, s3);
+#pragma unroll
+  for (int j = 0; j < NC; ++j)
+    if (key[j] >= th && key[j] > kNegInfKey) {
+      const int slot = atomicAdd(&s_nk, 1);
+      if (slot < kTopkKept) {
+        s_k[slot] = key[j];
+        s_i[slot] = id[j];
+      }
+    }
+  __syncthreads();
+  const int nk = s_nk;
+  if (nk > kTopkKept) {
+    if (tid == 0) *flag = 2;
+    return;
+  }
+  const float cexp = 1.4426950408889634f / temperature[row];
+  const uint32_t kmax = wave_max_u32_wg<kNW>(tid < nk ? s_k[tid] : 0u, s3);
+  const float M = key_to_f32(kmax);
+  const float e = tid < nk ? exp2f((key_to_f32(s_k[tid]) - M) * cexp) : 0.f;
+  if (tid < nk) s_e[tid] = e;
+  const float Z = wg_sum<kNW>(e, sf);   // (its barriers also publish s_e)
+  const float tp = top_p[row];
+  // strictly-more-likely mass and (key desc, id asc) rank of this thread's kept id
+  float above = 0.f;
+  int rank = 0;
+  const uint32_t mk = tid < nk ? s_k[tid] : 0u;
+  const int mi = tid < nk ? s_i[tid] : 0;
+  for (int j = 0; j < nk; ++j) {
+    const uint32_t kj = s_k[j];
+    if (kj > mk) above += s_e[j];
+    rank += (kj > mk || (kj == mk && s_i[j] < mi)) ? 1 : 0;
+  }
+  const bool member = tid < nk && (tp >= 1.f || above < tp * Z);
+  __syncthreads();
+  // nucleus masses in (key desc, id asc) rank order (the ranks are a permutation of
+  // 0..nk-1), then ONE prefix sum over that order: the members' intervals
+  // [cum, cum + e) tile [0, Zn) exactly and every sum has a fixed order, whatever
+  // order the candidates were appended in (a seeded draw reproduces bit for bit)
+  if (tid < nk) s_e[rank] = member ? e : 0.f;
+  __syncthreads();
+  float incl = tid < nk ? s_e[tid] : 0.f;   // the mass of rank tid, then its inclusive prefix
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const float y = __shfl_up(incl, o, 64);
+    if (lane_id() >= o) incl += y;
+  }
+  if (lane_id() == 63) sf[wave_id()] = incl;
+  __syncthreads();
+  float wbase = 0.f;
+  for (int w = 0; w < wave_id(); ++w) wbase += sf[w];
+  float Zn = 0.f;
+  for (int w = 0; w < kSlThreads / 64; ++w) Zn += sf[w];
+  float excl = __shfl_up(incl, 1, 64);
+  if (lane_id() == 0) excl = 0.f;
+  // the start of rank tid's interval; an interval ends where the next one starts, so
+  // consecutive boundaries tile [0, Zn) with no gap or overlap under any rounding
+  if (tid < nk) s_c[tid] = wbase + excl;
+  __syncthreads();
+  const float cum = member ? s_c[rank] : 0.f;
+  const uint64_t s0 =
+      splitmix64((uint64_t)seeds[row] ^ (0x632BE59BD9B4E019ull * (uint64_t)(steps[row] + 1)));
+  const uint64_t h = splitmix64(s0);
+  const float T = ((float)(h >> 40) + 0.5f) * (1.0f / 16777216.0f) * Zn;
+  const float hi = rank + 1 < nk ? s_c[rank + 1] : Zn;   // the next rank's start
+  if (member && e > 0.f && T >= cum && T < hi) s_pick = mi;
+  if (member) atomicMax(&s_last, rank);   // rounding tail: the last-ranked member
+  __syncthreads();
+  if (s_pick < 0 && member && rank == s_last) s_pick = mi;
+  __syncthreads();
+  if (tid == 0) {
+    out_tokens[row] = FT_CHECK_IDX(s_pick, vocab, kCkSampled, row);
+    *flag = 0;
+  }
+}
+
+// ABOVE: for few rows, one workgroup per row and slice, each with the whole draw and then
+// its own slice's above-mass (K2 and K3 in one launch; slice 0's writes what the accept step reads).
+template <typename T, bool ABOVE>
 __global__ __launch_bounds__(kSampThreads) void samp_draw_kernel(
     int* __restrict__ out_tokens, const T* __restrict__ logits, long stride, int vocab,
     const float* __restrict__ temperature, const float* __restrict__ top_p,
@@ -720,15 +902,21 @@ __global__ __launch_bounds__(kSampThreads) void samp_draw_kernel(
   static_assert(kSlices <= 64, "one lane per slice");
   // top-p rows: candidate r is searched by threads [r * per, (r + 1) * per), per = kSampThreads /
   // kCand; without a nucleus only candidate 0 is drawn, by the whole workgroup
-  __shared__ float s_scan[kSampThreads / 64];
+  __shared__ float s_scan[kSampThreads / 64], s_sum[kSlThreads / 64];
   __shared__ float s_M, s_cexp, s_tgt[kCand];
   __shared__ int s_ps[kCand], s_done, s_last[kCand], s_found[kCand];
-  const int row = blockIdx.x, tid = threadIdx.x, lane = lane_id();
+  __shared__ uint32_t s_ck[kCand];
+  const int row = ABOVE ? blockIdx.y : blockIdx.x, part = ABOVE ? blockIdx.x : 0;
+  const int tid = threadIdx.x, lane = lane_id();
+  const bool writes = part == 0;
   float* wr = ws + (long)row * kWsRow;
   int* flag = reinterpret_cast<int*>(wr + kWsFlag);
   if (topk_row(top_k, row, vocab)) {
-    // multi-workgroup top-k rows: samp_topk_kernel sets the flag; others: one-WG path
-    if (tid == 0 && !mw_topk_row(top_k, temperature, row, vocab)) *flag = 2;
+    if (!writes || tid >= kSlThreads) return;   // (waves that have ended are in no barrier's count)
+    if (mw_topk_row(top_k, temperature, row, vocab))
+      draw_topk(row, out_tokens, vocab, temperature, top_p, top_k, seeds, steps, ws);
+    else if (tid == 0)
+      *flag = 2;   // one-WG path
     return;
   }
   const float tp = top_p[row];
@@ -765,9 +953,11 @@ __global__ __launch_bounds__(kSampThreads) void samp_draw_kernel(
     const bool done = temp <= 0.f || besti == 0x7fffffff || bestk <= kNegInfKey;
     if (done) {
       if (lane == 0) {
+        s_done = 1;
+      }
+      if (lane == 0 && writes) {
         out_tokens[row] = FT_CHECK_IDX((besti == 0x7fffffff) ? 0 : besti, vocab, kCkSampled, row);
         *flag = 0;
-        s_done = 1;
       }
     } else {
       const float cexp = 1.4426950408889634f / temp;
@@ -803,12 +993,16 @@ __global__ __launch_bounds__(kSampThreads) void samp_draw_kernel(
         s_M = M;
         s_cexp = cexp;
         s_done = 0;
-        wr[kWsMZ] = M;
-        wr[kWsMZ + 1] = Z;
 #pragma unroll
-        for (int c = 0; c < kCand; ++c) {   // defined even if a search finds nothing
-          wr[kWsCand + 2 * c] = __uint_as_float(bestk);
-          wr[kWsCand + 2 * c + 1] = __int_as_float(besti);
+        for (int c = 0; c < kCand; ++c) s_ck[c] = bestk;   // defined even if a search finds nothing
+        if (writes) {
+          wr[kWsMZ] = M;
+          wr[kWsMZ + 1] = Z;
+#pragma unroll
+          for (int c = 0; c < kCand; ++c) {
+            wr[kWsCand + 2 * c] = __uint_as_float(bestk);
+            wr[kWsCand + 2 * c + 1] = __int_as_float(besti);
+          }
         }
       }
     }
@@ -886,18 +1080,24 @@ __global__ __launch_bounds__(kSampThreads) void samp_draw_kernel(
       pk = lastkey;
     }
     if (pick >= 0 && atomicCAS(&s_found[r], 0, 1) == 0) {
-      wr[kWsCand + 2 * r] = __uint_as_float(pk);
-      wr[kWsCand + 2 * r + 1] = __int_as_float(pick);
+      s_ck[r] = pk;
+      if (writes) {
+        wr[kWsCand + 2 * r] = __uint_as_float(pk);
+        wr[kWsCand + 2 * r + 1] = __int_as_float(pick);
+      }
     }
   }
   __syncthreads();
-  if (tid == 0) {
+  if (tid == 0 && writes) {
     if (tp >= 1.f) {   // no nucleus: the first draw is the sample
       out_tokens[row] = FT_CHECK_IDX(__float_as_int(wr[kWsCand + 1]), vocab, kCkSampled, row);
       *flag = 0;
     } else {
-      *flag = 3;   // samp_above_kernel + the accept step decide
+      *flag = 3;   // the above-masses + the accept step decide
     }
+  }
+  if constexpr (ABOVE) {
+    if (tp < 1.f && tid < kSlThreads) above_mass<T>(x, mrow, vocab, part, M, cexp, s_ck, wr, s_sum);
   }
 }
 
@@ -906,181 +1106,14 @@ __global__ __launch_bounds__(kSlThreads) void samp_above_kernel(
     const T* __restrict__ logits, long stride, int vocab, const float* __restrict__ temperature,
     const uint32_t* __restrict__ allow_mask, int mask_words, float* __restrict__ ws) {
   __shared__ float sf[kSlThreads / 64];
-  const int row = blockIdx.y, p = blockIdx.x;
+  __shared__ uint32_t s_ck[kCand];
+  const int row = blockIdx.y;
   float* wr = ws + (long)row * kWsRow;
   if (*reinterpret_cast<const int*>(wr + kWsFlag) != 3) return;
-  const T* x = logits + (long)row * stride;
-  const uint32_t* mrow = allow_mask ? allow_mask + (long)row * mask_words : nullptr;
-  const float M = wr[kWsMZ];
-  const float cexp = 1.4426950408889634f / temperature[row];
-  uint32_t kc[kCand], kmin = 0xffffffffu;
-#pragma unroll
-  for (int c = 0; c < kCand; ++c) {
-    kc[c] = __float_as_uint(wr[kWsCand + 2 * c]);
-    kmin = min(kmin, kc[c]);
-  }
-  const int S = slice_len(vocab);
-  const int beg = p * S, end = min(vocab, beg + S);
-  float a[kCand] = {};
-  for (int base = beg + threadIdx.x * 8; base < end; base += kSlThreads * 8) {
-    uint32_t key[8];
-    load_keys8<T>(x, mrow, base, vocab, key);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float e = key[j] > kmin ? exp2f((key_to_f32(key[j]) - M) * cexp) : 0.f;
-#pragma unroll
-      for (int c = 0; c < kCand; ++c) a[c] += key[j] > kc[c] ? e : 0.f;
-    }
-  }
-#pragma unroll
-  for (int c = 0; c < kCand; ++c) {
-    a[c] = wg_sum(a[c], sf);
-    if (threadIdx.x == 0) wr[kWsAbove + kCand * p + c] = a[c];
-  }
-}
-
-// Top-k rows (k <= kTopkMax, temperature > 0), one workgroup per row: merge the
-// slices' candidates, keep key >= t* (t* = largest key with count(key >= t*) >= k,
-// the single-workgroup kernel's rule: ties at the threshold stay), then top-p over
-// the kept ids (an id is in the nucleus iff the mass of strictly more likely kept
-// ids is < top_p * Z) and one inverse-CDF draw in (key desc, id asc) order over a
-// rank-ordered prefix sum -- deterministic whatever order the candidates were
-// appended in.  Rows whose
-// candidates or kept set overflow go to the one-workgroup kernel (flag 2).
-__global__ __launch_bounds__(kSlThreads) void samp_topk_kernel(
-    int* __restrict__ out_tokens, int vocab, const float* __restrict__ temperature,
-    const float* __restrict__ top_p, const int* __restrict__ top_k,
-    const long long* __restrict__ seeds, const int* __restrict__ steps, float* __restrict__ ws) {
-  constexpr int NC = kSlices * kTopkMax / kSlThreads;   // candidates per thread
-  __shared__ int s_off[kSlices + 1];
-  __shared__ int s3[3 * (kSlThreads / 64)];
-  __shared__ float sf[kSlThreads / 64];
-  __shared__ int s_nk, s_bad, s_pick, s_last;
-  __shared__ uint32_t s_k[kTopkKept];
-  __shared__ int s_i[kTopkKept];
-  __shared__ float s_e[kTopkKept];
-  __shared__ float s_c[kTopkKept];
-  const int row = blockIdx.x, tid = threadIdx.x;
-  if (!mw_topk_row(top_k, temperature, row, vocab)) return;
-  float* wr = ws + (long)row * kWsRow;
-  int* flag = reinterpret_cast<int*>(wr + kWsFlag);
-  const int* cnt = reinterpret_cast<const int*>(wr + kWsTkCnt);
-  if (tid == 0) {
-    int o = 0, bad = 0;
-    for (int p = 0; p < kSlices; ++p) {
-      s_off[p] = o;
-      bad |= cnt[p] < 0;
-      o += max(cnt[p], 0);
-    }
-    s_off[kSlices] = o;
-    s_bad = bad;
-    s_nk = 0;
-    s_pick = -1;
-    s_last = -1;
-  }
+  if (threadIdx.x < kCand) s_ck[threadIdx.x] = __float_as_uint(wr[kWsCand + 2 * threadIdx.x]);
   __syncthreads();
-  if (s_bad) {
-    if (tid == 0) *flag = 2;
-    return;
-  }
-  const int C = s_off[kSlices];
-  uint32_t key[NC];
-  int id[NC];
-#pragma unroll
-  for (int j = 0; j < NC; ++j) {
-    const int c = tid + kSlThreads * j;
-    key[j] = 0u;
-    id[j] = 0;
-    if (c < C) {
-      int p = 0;
-      while (s_off[p + 1] <= c) ++p;
-      const float* e = wr + kWsTk + 2 * kTopkMax * p + 2 * (c - s_off[p]);
-      key[j] = __float_as_uint(e[0]);
-      id[j] = __float_as_int(e[1]);
-    }
-  }
-  const int kk = min(top_k[row], C);
-  if (kk == 0) {   // everything masked
-    if (tid == 0) {
-      out_tokens[row] = FT_CHECK_IDX(0, vocab, kCkSampled, row);
-      *flag = 0;
-    }
-    return;
-  }
-  const uint32_t th = wg_kth_key<NC>(key, kk, s3);
-#pragma unroll
-  for (int j = 0; j < NC; ++j)
-    if (key[j] >= th && key[j] > kNegInfKey) {
-      const int slot = atomicAdd(&s_nk, 1);
-      if (slot < kTopkKept) {
-        s_k[slot] = key[j];
-        s_i[slot] = id[j];
-      }
-    }
-  __syncthreads();
-  const int nk = s_nk;
-  if (nk > kTopkKept) {
-    if (tid == 0) *flag = 2;
-    return;
-  }
-  const float cexp = 1.4426950408889634f / temperature[row];
-  const uint32_t kmax = wave_max_u32_wg(tid < nk ? s_k[tid] : 0u, s3);
-  const float M = key_to_f32(kmax);
-  const float e = tid < nk ? exp2f((key_to_f32(s_k[tid]) - M) * cexp) : 0.f;
-  if (tid < nk) s_e[tid] = e;
-  const float Z = wg_sum(e, sf);   // (its barriers also publish s_e)
-  const float tp = top_p[row];
-  // strictly-more-likely mass and (key desc, id asc) rank of this thread's kept id
-  float above = 0.f;
-  int rank = 0;
-  const uint32_t mk = tid < nk ? s_k[tid] : 0u;
-  const int mi = tid < nk ? s_i[tid] : 0;
-  for (int j = 0; j < nk; ++j) {
-    const uint32_t kj = s_k[j];
-    if (kj > mk) above += s_e[j];
-    rank += (kj > mk || (kj == mk && s_i[j] < mi)) ? 1 : 0;
-  }
-  const bool member = tid < nk && (tp >= 1.f || above < tp * Z);
-  __syncthreads();
-  // nucleus masses in (key desc, id asc) rank order (the ranks are a permutation of
-  // 0..nk-1), then ONE prefix sum over that order: the members' intervals
-  // [cum, cum + e) tile [0, Zn) exactly and every sum has a fixed order, whatever
-  // order the candidates were appended in (a seeded draw reproduces bit for bit)
-  if (tid < nk) s_e[rank] = member ? e : 0.f;
-  __syncthreads();
-  float incl = tid < nk ? s_e[tid] : 0.f;   // the mass of rank tid, then its inclusive prefix
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const float y = __shfl_up(incl, o, 64);
-    if (lane_id() >= o) incl += y;
-  }
-  if (lane_id() == 63) sf[wave_id()] = incl;
-  __syncthreads();
-  float wbase = 0.f;
-  for (int w = 0; w < wave_id(); ++w) wbase += sf[w];
-  float Zn = 0.f;
-  for (int w = 0; w < kSlThreads / 64; ++w) Zn += sf[w];
-  float excl = __shfl_up(incl, 1, 64);
-  if (lane_id() == 0) excl = 0.f;
-  // the start of rank tid's interval; an interval ends where the next one starts, so
-  // consecutive boundaries tile [0, Zn) with no gap or overlap under any rounding
-  if (tid < nk) s_c[tid] = wbase + excl;
-  __syncthreads();
-  const float cum = member ? s_c[rank] : 0.f;
-  const uint64_t s0 =
-      splitmix64((uint64_t)seeds[row] ^ (0x632BE59BD9B4E019ull * (uint64_t)(steps[row] + 1)));
-  const uint64_t h = splitmix64(s0);
-  const float T = ((float)(h >> 40) + 0.5f) * (1.0f / 16777216.0f) * Zn;
-  const float hi = rank + 1 < nk ? s_c[rank + 1] : Zn;   // the next rank's start
-  if (member && e > 0.f && T >= cum && T < hi) s_pick = mi;
-  if (member) atomicMax(&s_last, rank);   // rounding tail: the last-ranked member
-  __syncthreads();
-  if (s_pick < 0 && member && rank == s_last) s_pick = mi;
-  __syncthreads();
-  if (tid == 0) {
-    out_tokens[row] = FT_CHECK_IDX(s_pick, vocab, kCkSampled, row);
-    *flag = 0;
-  }
+  above_mass<T>(logits + (long)row * stride, allow_mask ? allow_mask + (long)row * mask_words : nullptr, vocab, blockIdx.x,
+                wr[kWsMZ], 1.4426950408889634f / temperature[row], s_ck, wr, sf);
 }
 
 }  // namespace ft
@@ -1104,14 +1137,18 @@ extern "C" int ft_sample(int* out_tokens, const void* logits, int logits_is_bf16
       hipLaunchKernelGGL(ft::samp_stats_kernel<TT>, dim3(ft::kSlices, batch), dim3(ft::kSlThreads),\
                          0, stream, lg, logit_stride, vocab, temperature, top_k, allow_mask,     \
                          mask_words, ws);                                                        \
-      hipLaunchKernelGGL(ft::samp_draw_kernel<TT>, dim3(batch), dim3(ft::kSampThreads), 0, stream,\
-                         out_tokens, lg, logit_stride, vocab, temperature, top_p, top_k, seeds,  \
-                         steps, allow_mask, mask_words, ws);                                     \
-      hipLaunchKernelGGL(ft::samp_above_kernel<TT>, dim3(ft::kSlices, batch), dim3(ft::kSlThreads),\
-                         0, stream, lg, logit_stride, vocab, temperature, allow_mask, mask_words, \
-                         ws);                                                                    \
-      hipLaunchKernelGGL(ft::samp_topk_kernel, dim3(batch), dim3(ft::kSlThreads), 0, stream,     \
-                         out_tokens, vocab, temperature, top_p, top_k, seeds, steps, ws);        \
+      if (batch <= ft::kAboveRows) {                                                             \
+        hipLaunchKernelGGL((ft::samp_draw_kernel<TT, true>), dim3(ft::kSlices, batch),           \
+                           dim3(ft::kSampThreads), 0, stream, out_tokens, lg, logit_stride, vocab, \
+                           temperature, top_p, top_k, seeds, steps, allow_mask, mask_words, ws); \
+      } else {                                                                                   \
+        hipLaunchKernelGGL((ft::samp_draw_kernel<TT, false>), dim3(batch), dim3(ft::kSampThreads), \
+                           0, stream, out_tokens, lg, logit_stride, vocab, temperature, top_p,   \
+                           top_k, seeds, steps, allow_mask, mask_words, ws);                     \
+        hipLaunchKernelGGL(ft::samp_above_kernel<TT>, dim3(ft::kSlices, batch),                  \
+                           dim3(ft::kSlThreads), 0, stream, lg, logit_stride, vocab, temperature, \
+                           allow_mask, mask_words, ws);                                          \
+      }                                                                                          \
       flags = reinterpret_cast<int*>(ws + ft::kWsFlag);                                          \
     }                                                                                            \
   }
