@@ -13,7 +13,7 @@ extern "C" {
 int mx_embed_rows(float* out, const int* ids, const void* table, int bf16, int rows, int width, int vocab,
                   float scale, const int* positions, const float* freqs, hipStream_t s);
 int mx_layer_norm(float* x, const void* y, int y_bf16, long y_stride, const float* w, const float* b, void* out,
-                  void* cast, int out_bf16, int rows, int width, float eps, hipStream_t s);
+                  void* cast, int out_bf16, const float* next_w, const float* next_b, int rows, int width, float eps, hipStream_t s);
 int mx_tanh_cap(float* x, long n, float cap, hipStream_t s);
 int mx_grouped_gemm(void* C, const void* A, long a_rows, const int* rows, const void* W, const int* offs, int groups, long M,
                     int N, int K, int act, float limit, hipStream_t s);
@@ -26,7 +26,8 @@ int mx_add_rms_norm_experts(float* x, const float* d, const float* wts, const fl
                             const float* wb, const float* add_vec, const float* next_w, void* out, void* cast, int out_bf16,
                             int rows, int width, float eps, hipStream_t s);
 int mx_layer_norm_experts(float* x, const float* d, const float* wts, const float* shared, const float* gate, int top,
-                          const float* w, const float* b, void* cast, int rows, int width, float eps, hipStream_t s);
+                          const float* w, const float* b, void* cast, const float* next_w, const float* next_b, int rows,
+                          int width, float eps, hipStream_t s);
 int mx_add_norm_shift_experts(float* x, const float* d, const float* wts, const float* shared, const float* gate, int top,
                               const float* wb, const float* w, const float* shift, void* out, float* state, int num_slots,
                               const int* start, const int* pos0, const int* slot, int num_segs, int rows, int width,
@@ -304,7 +305,14 @@ void embed_rows(Tensor out, Tensor ids, Tensor table, double scale, OptT positio
 }
 
 // x (fp32 residual) with y: x += ln(y), cast = x; without y: out = ln(x), or, without out, x = ln(x), cast = x
-void layer_norm(Tensor x, OptT y, Tensor w, Tensor b, OptT out, OptT cast, double eps) {
+const float* row_weight(const OptT& w, int64_t width) {
+  if (!w) return nullptr;
+  check_f32(*w, "norm weight");
+  TORCH_CHECK(w->numel() == width, "norm weight");
+  return w->data_ptr<float>();
+}
+
+void layer_norm(Tensor x, OptT y, Tensor w, Tensor b, OptT out, OptT cast, OptT next_w, OptT next_b, double eps) {
   check_f32(x, "residual");
   TORCH_CHECK(x.dim() == 2, "residual 2-D");
   const int64_t rows = x.size(0), width = x.size(1);
@@ -312,6 +320,7 @@ void layer_norm(Tensor x, OptT y, Tensor w, Tensor b, OptT out, OptT cast, doubl
   check_f32(b, "norm bias");
   TORCH_CHECK(w.numel() == width && b.numel() == width, "norm weight / bias size");
   TORCH_CHECK(!(y && out), "out goes without y");
+  TORCH_CHECK((bool)next_w == (bool)next_b && (!next_w || (cast && !out)), "next norm: weight, bias and cast");
   const void* yp = nullptr;
   int ybf = 0;
   long ys = 0;
@@ -332,7 +341,8 @@ void layer_norm(Tensor x, OptT y, Tensor w, Tensor b, OptT out, OptT cast, doubl
   if (out) op = out->data_ptr();
   if (cast) cp = cast->data_ptr();
   chk(mx_layer_norm(x.data_ptr<float>(), yp, ybf, ys, w.data_ptr<float>(), b.data_ptr<float>(), op, cp, obf,
-                    (int)rows, (int)width, (float)eps, stream()), "layer_norm");
+                    row_weight(next_w, width), row_weight(next_b, width), (int)rows, (int)width, (float)eps, stream()),
+      "layer_norm");
 }
 
 void tanh_cap(Tensor x, double cap) {
@@ -989,7 +999,7 @@ void few_rows_gemm(Tensor y, Tensor x, Tensor w, OptT bias, int64_t act, double 
   check_rows(y, "y");
   const bool glu = act >= 1 && act <= 4;
   TORCH_CHECK(x.scalar_type() == at::kBFloat16 && w.is_cuda() && w.scalar_type() == at::kBFloat16 && w.dim() == 2 &&
-              w.is_contiguous() && x.size(1) == w.size(1) && act >= 0 && act <= 5, "few_rows_gemm: bf16 rows and weights");
+              w.is_contiguous() && x.size(1) == w.size(1) && act >= 0 && act <= 6, "few_rows_gemm: bf16 rows and weights");
   TORCH_CHECK(y.size(0) == x.size(0) && y.size(1) * (glu ? 2 : 1) == w.size(0) && x.size(0) <= mx_few_rows_max(),
               "few_rows_gemm: shapes");
   if (bias)
@@ -1065,12 +1075,6 @@ Experts check_experts(const Tensor& d, const Tensor& wts, const OptT& shared, co
   return {d.data_ptr<float>(), wts.data_ptr<float>(), shared ? shared->data_ptr<float>() : nullptr,
           gate ? gate->data_ptr<float>() : nullptr, (int)wts.size(1)};
 }
-const float* row_weight(const OptT& w, int64_t width) {
-  if (!w) return nullptr;
-  check_f32(*w, "norm weight");
-  TORCH_CHECK(w->numel() == width, "norm weight");
-  return w->data_ptr<float>();
-}
 
 void add_rms_norm_experts(Tensor x, Tensor d, Tensor wts, OptT shared, OptT gate, OptT wb, OptT add_vec, OptT next_w, OptT out,
                           OptT cast, double eps) {
@@ -1092,14 +1096,16 @@ void add_rms_norm_experts(Tensor x, Tensor d, Tensor wts, OptT shared, OptT gate
       "add_rms_norm_experts");
 }
 
-void layer_norm_experts(Tensor x, Tensor d, Tensor wts, OptT shared, OptT gate, Tensor w, Tensor b, Tensor cast, double eps) {
+void layer_norm_experts(Tensor x, Tensor d, Tensor wts, OptT shared, OptT gate, Tensor w, Tensor b, Tensor cast, OptT next_w,
+                        OptT next_b, double eps) {
   check_f32(x, "residual");
   TORCH_CHECK(x.dim() == 2 && mx_expert_rows_fit((int)x.size(1)), "residual");
   const int64_t rows = x.size(0), width = x.size(1);
   const Experts e = check_experts(d, wts, shared, gate, rows, width);
   TORCH_CHECK(cast.is_cuda() && cast.scalar_type() == at::kBFloat16 && cast.is_contiguous() && cast.sizes() == x.sizes(), "cast");
+  TORCH_CHECK((bool)next_w == (bool)next_b, "next norm: weight and bias");
   chk(mx_layer_norm_experts(x.data_ptr<float>(), e.d, e.wts, e.shared, e.gate, e.top, row_weight(w, width),
-                            row_weight(b, width), cast.data_ptr(), (int)rows, (int)width, (float)eps, stream()),
+                            row_weight(b, width), cast.data_ptr(), row_weight(next_w, width), row_weight(next_b, width), (int)rows, (int)width, (float)eps, stream()),
       "layer_norm_experts");
 }
 

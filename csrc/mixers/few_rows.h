@@ -88,7 +88,7 @@ __device__ __forceinline__ void few_rows_core(fr_f32x4 (&acc)[NT][NB], const bf1
 }
 
 // what is done to a column's sum(s)
-enum { kFrStore = 0, kFrGelu = 1, kFrRelu = 2, kFrSilu = 3, kFrClamp = 4, kFrReluSq = 5 };
+enum { kFrStore = 0, kFrGelu = 1, kFrRelu = 2, kFrSilu = 3, kFrClamp = 4, kFrReluSq = 5, kFrTanhCap = 6 };
 
 // 1 / (1 + e^-x) in eight instructions, for epilogues that a whole tile waits for (with the library's exp, tanh and division
 // 22 of 131 us of 2048 x 2048 -> 2 x 8192): e^-x = 2^t (1 + r ln 2), t + r = -x log2(e) with r what t's rounding lost.  Results

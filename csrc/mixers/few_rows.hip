@@ -82,6 +82,12 @@ few_rows_gemm_kernel(TO* __restrict__ Y, long y_stride, const bf16_t* __restrict
 #pragma unroll
         for (int i = 0; i < 4; ++i) v[i] = fr_act(act, limit, v[i], 0.f);
       }
+      if constexpr (sizeof(TO) == 4) {           // logits: as tanh_cap_kernel, 5 us less than behind the product
+        if (act == kFrTanhCap) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) v[i] = isfinite(v[i]) ? limit * tanhf(v[i] / limit) : v[i];
+        }
+      }
     }
     fr_store4(Y + r * y_stride, c, N, vec != 0, v);
   }
@@ -332,7 +338,8 @@ extern "C" int mx_few_rows_max() { return kFewRows; }
 extern "C" int mx_few_rows_gemm(void* Y, int y_f32, long y_stride, const void* X, long x_stride, int rows,
                                 const void* W, const void* bias, int N, int K, int act, float limit, hipStream_t s) {
   if (rows <= 0 || N <= 0) return 0;
-  if (rows > kFewRows || K < 8 || K % 8 || x_stride % 8 || act < kFrStore || act > kFrReluSq) return -1;
+  if (rows > kFewRows || K < 8 || K % 8 || x_stride % 8 || act < kFrStore || act > kFrTanhCap || (act == kFrTanhCap && !y_f32))
+    return -1;
   if (((uintptr_t)X) % 16 || ((uintptr_t)W) % 16) return -2;
   const bool glu = act >= kFrGelu && act <= kFrClamp;
   if (glu && (bias != nullptr || y_f32)) return -3;

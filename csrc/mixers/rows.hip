@@ -308,11 +308,31 @@ __device__ __forceinline__ float sum_sq(const float (&v)[C][4]) {
 template <typename Y, typename TO, int NT, int C>
 __global__ void __launch_bounds__(NT)
 layer_norm_row_kernel(float* __restrict__ x, Y y, const float* __restrict__ w,
-                      const float* __restrict__ b, TO* __restrict__ out, TO* __restrict__ cast, int width, float eps,
-                      int vec) {
+                      const float* __restrict__ b, TO* __restrict__ out, TO* __restrict__ cast,
+                      const float* __restrict__ next_w, const float* __restrict__ next_b, int width, float eps, int vec) {
   __shared__ float red[NT / 64];
   const long row = blockIdx.x;
   float v[C][4], u[C][4], wv[C][4], bv[C][4];
+  auto norm = [&] {                          // u <- its layer norm, times wv plus bv
+    float sum = 0.f;
+#pragma unroll
+    for (int c = 0; c < C; ++c) sum += (u[c][0] + u[c][1]) + (u[c][2] + u[c][3]);
+    const float mean = block_sum<NT>(sum, red) / (float)width;
+    float ss = 0.f;
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const bool in = (c * NT + (int)threadIdx.x) * 4 + k < width;
+        u[c][k] = in ? u[c][k] - mean : 0.f;
+        ss += u[c][k] * u[c][k];
+      }
+    const float r = 1.0f / sqrtf(block_sum<NT>(ss, red) / (float)width + eps);
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) u[c][k] = u[c][k] * r * wv[c][k] + bv[c][k];
+  };
   load_row<float, NT, C>(v, x + row * width, width, vec);
   if (y.any()) {
     y.template load<NT, C>(u, row, width, vec);
@@ -324,31 +344,21 @@ layer_norm_row_kernel(float* __restrict__ x, Y y, const float* __restrict__ w,
   }
   load_row<float, NT, C>(wv, w, width, vec);
   load_row<float, NT, C>(bv, b, width, vec);
-  float sum = 0.f;
+  norm();
+  if (out == nullptr && y.any())
 #pragma unroll
-  for (int c = 0; c < C; ++c) sum += (u[c][0] + u[c][1]) + (u[c][2] + u[c][3]);
-  const float mean = block_sum<NT>(sum, red) / (float)width;
-  float ss = 0.f;
+    for (int c = 0; c < C; ++c)
 #pragma unroll
-  for (int c = 0; c < C; ++c)
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const bool in = (c * NT + (int)threadIdx.x) * 4 + k < width;
-      u[c][k] = in ? u[c][k] - mean : 0.f;
-      ss += u[c][k] * u[c][k];
-    }
-  const float r = 1.0f / sqrtf(block_sum<NT>(ss, red) / (float)width + eps);
-#pragma unroll
-  for (int c = 0; c < C; ++c)
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      u[c][k] = u[c][k] * r * wv[c][k] + bv[c][k];
-      if (out == nullptr && y.any()) u[c][k] += v[c][k];
-    }
+      for (int k = 0; k < 4; ++k) u[c][k] += v[c][k];
   if (out != nullptr) {
     store_row<TO, NT, C>(out + row * width, u, width, vec);
   } else {
     store_row<float, NT, C>(x + row * width, u, width, vec);
+    if (next_w != nullptr) {
+      load_row<float, NT, C>(wv, next_w, width, vec);
+      load_row<float, NT, C>(bv, next_b, width, vec);
+      norm();
+    }
     if (cast != nullptr) store_row<TO, NT, C>(cast + row * width, u, width, vec);
   }
 }
@@ -770,32 +780,39 @@ static bool row_in_registers(int rows, int width, int vec) {
 
 template <typename TY, typename TO>
 static void launch_layer_norm(float* x, const void* y, long ys, const float* w, const float* b, void* out,
-                              void* cast, int rows, int width, float eps, hipStream_t s) {
+                              void* cast, const float* nw, const float* nb, int rows, int width, float eps,
+                              hipStream_t s) {
   const int vec = width % 4 == 0 && (y == nullptr || (ys % 4 == 0 && ((uintptr_t)y) % (4 * sizeof(TY)) == 0)) &&
-                  ((uintptr_t)x | (uintptr_t)w | (uintptr_t)b) % 16 == 0 &&
+                  ((uintptr_t)x | (uintptr_t)w | (uintptr_t)b | (uintptr_t)nw | (uintptr_t)nb) % 16 == 0 &&
                   ((uintptr_t)out | (uintptr_t)cast) % (4 * sizeof(TO)) == 0;
   if (row_in_registers(rows, width, vec)) {
     row_chunks(width, [&](auto c) {
       hipLaunchKernelGGL((layer_norm_row_kernel<RowsOf<TY>, TO, kRowThreads, decltype(c)::value>), dim3(rows),
-                         dim3(kRowThreads), 0, s, x, RowsOf<TY>{(const TY*)y, ys}, w, b, (TO*)out, (TO*)cast, width, eps,
-                         vec);
+                         dim3(kRowThreads), 0, s, x, RowsOf<TY>{(const TY*)y, ys}, w, b, (TO*)out, (TO*)cast, nw, nb,
+                         width, eps, vec);
     });
     return;
   }
   hipLaunchKernelGGL((layer_norm_kernel<TY, TO, 256>), dim3(rows), dim3(256), 0, s, x, (const TY*)y, ys, w, b,
-                     (TO*)out, (TO*)cast, width, eps);
+                     (TO*)out, nw != nullptr ? (TO*)nullptr : (TO*)cast, width, eps);
+  if (nw != nullptr)
+    hipLaunchKernelGGL((layer_norm_kernel<float, TO, 256>), dim3(rows), dim3(256), 0, s, x, (const float*)nullptr, 0L, nw, nb,
+                       (TO*)cast, (TO*)nullptr, width, eps);
 }
 
+// next_w, next_b: cast is the layer norm by these of the new residual
 extern "C" int mx_layer_norm(float* x, const void* y, int y_bf16, long y_stride, const float* w, const float* b,
-                             void* out, void* cast, int out_bf16, int rows, int width, float eps, hipStream_t s) {
+                             void* out, void* cast, int out_bf16, const float* next_w,
+                             const float* next_b, int rows, int width, float eps, hipStream_t s) {
   if (rows <= 0) return 0;
-  if (y != nullptr && out != nullptr) return -1;
+  if ((y != nullptr && out != nullptr) || (next_w != nullptr && (next_b == nullptr || cast == nullptr || out != nullptr)))
+    return -1;
   if (y_bf16) {
-    if (out_bf16) launch_layer_norm<bf16_t, bf16_t>(x, y, y_stride, w, b, out, cast, rows, width, eps, s);
-    else launch_layer_norm<bf16_t, float>(x, y, y_stride, w, b, out, cast, rows, width, eps, s);
+    if (out_bf16) launch_layer_norm<bf16_t, bf16_t>(x, y, y_stride, w, b, out, cast, next_w, next_b, rows, width, eps, s);
+    else launch_layer_norm<bf16_t, float>(x, y, y_stride, w, b, out, cast, next_w, next_b, rows, width, eps, s);
   } else {
-    if (out_bf16) launch_layer_norm<float, bf16_t>(x, y, y_stride, w, b, out, cast, rows, width, eps, s);
-    else launch_layer_norm<float, float>(x, y, y_stride, w, b, out, cast, rows, width, eps, s);
+    if (out_bf16) launch_layer_norm<float, bf16_t>(x, y, y_stride, w, b, out, cast, next_w, next_b, rows, width, eps, s);
+    else launch_layer_norm<float, float>(x, y, y_stride, w, b, out, cast, next_w, next_b, rows, width, eps, s);
   }
   return (int)hipGetLastError();
 }
@@ -853,16 +870,16 @@ extern "C" int mx_add_rms_norm_experts(float* x, const float* d, const float* wt
 }
 
 extern "C" int mx_layer_norm_experts(float* x, const float* d, const float* wts, const float* shared, const float* gate,
-                                     int top, const float* w, const float* b, void* cast, int rows, int width, float eps,
-                                     hipStream_t s) {
+                                     int top, const float* w, const float* b, void* cast, const float* next_w,
+                                     const float* next_b, int rows, int width, float eps, hipStream_t s) {
   if (rows <= 0) return 0;
   if (!mx_expert_rows_fit(width) || top < 1) return -1;
   if (((uintptr_t)d | (uintptr_t)shared) % 16) return -2;
-  const int vec = ((uintptr_t)x | (uintptr_t)w | (uintptr_t)b | (uintptr_t)cast) % 16 == 0;
+  const int vec = ((uintptr_t)x | (uintptr_t)w | (uintptr_t)b | (uintptr_t)next_w | (uintptr_t)next_b | (uintptr_t)cast) % 16 == 0;
   const ExpertRows y{d, wts, shared, gate, top};
   row_chunks(width, [&](auto c) {
     hipLaunchKernelGGL((layer_norm_row_kernel<ExpertRows, bf16_t, kRowThreads, decltype(c)::value>), dim3(rows),
-                       dim3(kRowThreads), 0, s, x, y, w, b, (bf16_t*)nullptr, (bf16_t*)cast, width, eps, vec);
+                       dim3(kRowThreads), 0, s, x, y, w, b, (bf16_t*)nullptr, (bf16_t*)cast, next_w, next_b, width, eps, vec);
   });
   return (int)hipGetLastError();
 }

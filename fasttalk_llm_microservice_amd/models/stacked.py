@@ -232,6 +232,7 @@ class StackedModel:
         nruns = len(self.runs)
         mark = self.mark_at
         prev_h = caches.extra.get("prev_h")
+        every = meta.logits_indices.numel() == x.shape[0]      # the final norm rides in the last layer's last add
         for r, (li, step) in enumerate(self.runs):
             if mark is not None and r == mark[0]:
                 mark[1].record()
@@ -245,6 +246,8 @@ class StackedModel:
             nxt = self.runs[r + 1] if r + 1 < nruns else None
             nvec = self.loop_step[nxt[1]] if nxt is not None and nxt[1] is not None and fuse_step else None
             nw = self.layers[nxt[0]].norm1 if nxt is not None and (fuse_step or nxt[1] is None) else None
+            if nxt is None and every:
+                nw = self.final_norm
             last = L.ff is None and L.side is None
             nshift = self.layers[nxt[0]].shift if nxt is not None else None
             if nshift is not None:
@@ -274,11 +277,18 @@ class StackedModel:
                                            out_dtype=dt)
             if tap is not None:
                 tap.append(x.clone())
-        idx = meta.logits_indices
-        rows = x.index_select(0, idx) if idx.numel() != x.shape[0] else x
+        if every and nruns:
+            return h
+        return self._final_rows(x, meta, every)
+
+    def _final_rows(self, x, meta, every: bool) -> torch.Tensor:
+        """The final norm by itself, of the rows whose logits are wanted."""
+        rows = x if every else x.index_select(0, meta.logits_indices)
         if rows.shape[0] == 0:
-            return rows.to(dt)
-        return M.rms_norm_rows(rows, self.final_norm, eps, dt)
+            return rows.to(self.dtype)
+        if self.norm_style == "layer_post":
+            return M.layer_norm_rows(rows, self.final_norm, self.final_bias, self.cfg.rms_norm_eps, self.dtype)
+        return M.rms_norm_rows(rows, self.final_norm, self.cfg.rms_norm_eps, self.dtype)
 
     def _norm_ff(self, x, y, wb, w, b, ff, ctx, parts: bool = True):
         """A layer's add and norm between its mixer and its feed-forward, and that: x += rms_norm(y) * wb and ff of
@@ -314,23 +324,24 @@ class StackedModel:
         h = M.add_layer_norm_rows(x, None, self.embed_norm[0], self.embed_norm[1], eps, dt) \
             if self.embed_norm is not None else (x if dt == torch.float32 else x.to(dt))
         tap, mark = self.layer_tap, self.mark_at
+        every, nruns = meta.logits_indices.numel() == x.shape[0], len(self.runs)
         for r, (li, _) in enumerate(self.runs):
             if mark is not None and r == mark[0]:
                 mark[1].record()
             L = self.layers[li]
             y = L.mixer(h, ctx, caches.per_run[r])
+            # the final norm rides in the last layer's last one
+            nxt = (self.final_norm, self.final_bias) if every and r + 1 == nruns else None
             if L.ff is None:
-                h = M.add_layer_norm_rows(x, y, L.norm1b, L.bias1, eps, dt)
+                h = M.add_layer_norm_rows(x, y, L.norm1b, L.bias1, eps, dt, nxt)
             else:
                 y = self._norm_ff(x, y, None, L.norm1b, L.bias1, L.ff, ctx)
-                h = M.add_layer_norm_rows(x, y, L.norm2b, L.bias2, eps, dt)
+                h = M.add_layer_norm_rows(x, y, L.norm2b, L.bias2, eps, dt, nxt)
             if tap is not None:
                 tap.append(x.clone())
-        idx = meta.logits_indices
-        rows = x.index_select(0, idx) if idx.numel() != x.shape[0] else x
-        if rows.shape[0] == 0:
-            return rows.to(dt)
-        return M.layer_norm_rows(rows, self.final_norm, self.final_bias, eps, dt)
+        if every and nruns:
+            return h
+        return self._final_rows(x, meta, every)
 
     def _forward_shared_pre(self, input_ids, meta, ctx, caches: StackedCache) -> torch.Tensor:
         dt, eps, mult = self.dtype, self.cfg.rms_norm_eps, self.residual_mult
@@ -339,36 +350,38 @@ class StackedModel:
         nruns = len(self.runs)
         h = M.add_scaled_rms_norm_rows(x, None, None, mult, self.layers[self.runs[0][0]].norm1, eps, dt) \
             if nruns else None
+        every = meta.logits_indices.numel() == x.shape[0]
         for r, (li, _) in enumerate(self.runs):
             if mark is not None and r == mark[0]:
                 mark[1].record()
             L = self.layers[li]
             y = L.mixer(h, ctx, caches.per_run[r])
             f = L.ff(h, ctx) if L.ff is not None else None
-            nw = self.layers[self.runs[r + 1][0]].norm1 if r + 1 < nruns else None
+            # (behind the last layer the final norm, if every row's logits are wanted)
+            nw = self.layers[self.runs[r + 1][0]].norm1 if r + 1 < nruns else self.final_norm if every else None
             h = M.add_scaled_rms_norm_rows(x, y, f, mult, nw, eps, dt)
             if tap is not None:
                 tap.append(x.clone())
-        idx = meta.logits_indices
-        rows = x.index_select(0, idx) if idx.numel() != x.shape[0] else x
-        if rows.shape[0] == 0:
-            return rows.to(dt)
-        return M.rms_norm_rows(rows, self.final_norm, eps, dt)
+        if every and nruns:
+            return h
+        return self._final_rows(x, meta, every)
 
     def compute_logits(self, h: torch.Tensor) -> torch.Tensor:
         """fp32 logits [rows, vocab rounded up to a multiple of 8]; columns past the
         vocabulary are -inf.  With ``logit_softcap`` c > 0 the logits are c tanh(z / c)."""
-        logits = self._head_product(h)
-        if self.logit_scale != 1.0:
+        scaled = self.logit_scale != 1.0
+        logits = self._head_product(h, 0.0 if scaled else self.logit_softcap)
+        if scaled:
             logits *= self.logit_scale
-        if self.logit_softcap:
-            M.tanh_cap_(logits, self.logit_softcap)
+            if self.logit_softcap:
+                M.tanh_cap_(logits, self.logit_softcap)
         if self.vocab_pad:
             logits[:, self.cfg.vocab_size:] = float("-inf")
         return logits
 
-    def _head_product(self, h: torch.Tensor) -> torch.Tensor:
+    def _head_product(self, h: torch.Tensor, cap: float = 0.0) -> torch.Tensor:
         if h.dtype == torch.float32:
-            return F.linear(h, self.head)
+            y = F.linear(h, self.head)
+            return M.tanh_cap_(y, cap) if cap else y
         # bf16 operands, fp32 accumulation and fp32 output
-        return M.linear_f32(h, self.head)
+        return M.linear_f32(h, self.head, cap)

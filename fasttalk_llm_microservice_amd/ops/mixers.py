@@ -91,6 +91,7 @@ def _device_segments(seg: Segments) -> bool:
 # step's; the vendor's tiles fill up beyond)
 FEW_ROWS = 64
 # activations of the few-rows kernels and the sorted experts (csrc/mixers/few_rows.h)
+FEW_TANH_CAP = 6       # linear_f32 with a cap
 FEW_ACTS = {None: 0, "gelu_tanh": 1, "relu": 2, "silu": 3, "clamp_glu": 4, "relu_sq": 5, "silu_glu": 3}
 
 
@@ -190,13 +191,14 @@ def linear(x, w, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     return torch.nn.functional.linear(x, w, bias) if y is None else y
 
 
-def linear_f32(x, w) -> torch.Tensor:
-    """x w^T with fp32 accumulation and fp32 output."""
+def linear_f32(x, w, cap: float = 0.0) -> torch.Tensor:
+    """x w^T with fp32 accumulation and fp32 output, through :func:`tanh_cap_` if there is a ``cap``."""
     if _few_rows(x, w) and _few_rows_pays(x.shape[0], w.shape[0], x.shape[1]):
         y = torch.empty(x.shape[0], w.shape[0], dtype=torch.float32, device=x.device)
-        native_mixers().few_rows_gemm(y, x, w, None, 0, 0.0)
+        native_mixers().few_rows_gemm(y, x, w, None, FEW_TANH_CAP if cap else 0, float(cap))
         return y
-    return mm_f32(x, w.t())
+    y = mm_f32(x, w.t())
+    return tanh_cap_(y, cap) if cap else y
 
 
 def linear_act(x, w, act: str, limit: float = 0.0) -> torch.Tensor:
@@ -244,7 +246,7 @@ def layer_norm_rows(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor, eps: floa
     rounded to ``out_dtype``; x is left as it is."""
     if x.is_cuda:
         out = torch.empty(x.shape, dtype=out_dtype, device=x.device)
-        native_mixers().layer_norm(x, None, w, b, out, None, eps)
+        native_mixers().layer_norm(x, None, w, b, out, None, None, None, eps)
         return out
     return ref.layer_norm_rows(x, w, b, eps, out_dtype)
 
@@ -260,20 +262,22 @@ class ExpertParts(NamedTuple):
 
 
 def add_layer_norm_rows(residual: torch.Tensor, y: Optional[torch.Tensor], w: torch.Tensor, b: torch.Tensor,
-                        eps: float, out_dtype) -> torch.Tensor:
+                        eps: float, out_dtype, next_norm: Optional[tuple] = None) -> torch.Tensor:
     """residual (fp32, in place) += layer_norm(y) * w + b, or, without y, residual <-
     layer_norm(residual) * w + b.  Returns the new residual in ``out_dtype`` (the residual
-    itself when that is fp32): what the next sublayer of a post-norm stack reads.  y may be :class:`ExpertParts`."""
+    itself when that is fp32): what the next sublayer of a post-norm stack reads; with ``next_norm`` (weight, bias) its layer
+    norm by these instead.  y may be :class:`ExpertParts`."""
     if isinstance(y, ExpertParts):
         cast = torch.empty(residual.shape, dtype=out_dtype, device=residual.device)
-        native_mixers().layer_norm_experts(residual, *y, w, b, cast, eps)
+        native_mixers().layer_norm_experts(residual, *y, w, b, cast, *(next_norm or (None, None)), eps)
         return cast
     if residual.is_cuda:
-        cast = None if out_dtype == torch.float32 else \
+        cast = None if out_dtype == torch.float32 and next_norm is None else \
             torch.empty(residual.shape, dtype=out_dtype, device=residual.device)
-        native_mixers().layer_norm(residual, y, w, b, None, cast, eps)
+        native_mixers().layer_norm(residual, y, w, b, None, cast, *(next_norm or (None, None)), eps)
         return residual if cast is None else cast
-    return ref.add_layer_norm_rows(residual, y, w, b, eps, out_dtype)
+    h = ref.add_layer_norm_rows(residual, y, w, b, eps, out_dtype)
+    return h if next_norm is None else ref.layer_norm_rows(residual, *next_norm, eps, out_dtype)
 
 
 def tanh_cap_(x: torch.Tensor, cap: float) -> torch.Tensor:

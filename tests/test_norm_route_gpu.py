@@ -91,3 +91,31 @@ def test_norm_steps_sum_the_experts(rows, width, top, shared):
             if a is not None:
                 torch.testing.assert_close(a.float(), c.float(), rtol=2 ** -7, atol=1e-4)    # a rounding to bf16 on each side
     torch.testing.assert_close(*states, rtol=1e-5, atol=1e-4)
+
+
+# in registers and not (rows / width), experts' results
+@pytest.mark.parametrize("rows,width", [(1, 1032), (7, 2048), (3, 16392), (2, 30)])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+def test_layer_norm_behind_the_last_one(rows, width, dt):
+    g = torch.Generator().manual_seed(width)
+    x, y = rnd(rows, width, g=g).to(DEV), rnd(rows, width, g=g).to(DEV)
+    w, b, nw, nb = (rnd(width, g=g).to(DEV) for _ in range(4))
+    x2 = x.clone()
+    got = M.add_layer_norm_rows(x, y, w, b, 1e-5, dt, (nw, nb))
+    M.add_layer_norm_rows(x2, y, w, b, 1e-5, dt)
+    assert torch.equal(x, x2)
+    assert got.dtype == dt and torch.equal(got, M.layer_norm_rows(x2, nw, nb, 1e-5, dt))       # the same sums
+    if dt == torch.bfloat16 and 1024 < width <= 16384:
+        parts = M.ExpertParts(y, torch.ones(rows, 1, device=DEV), None, None)
+        x3 = (x2 - M.layer_norm_rows(y, w, b, 1e-5, torch.float32))
+        got = M.add_layer_norm_rows(x3, parts, w, b, 1e-5, dt, (nw, nb))
+        want = M.layer_norm_rows(x3, nw, nb, 1e-5, torch.float32)
+        torch.testing.assert_close(got.float(), want, rtol=2 ** -8, atol=1e-5)                 # one rounding to bf16
+
+
+@pytest.mark.parametrize("rows,n", [(1, 8), (33, 4104)])
+def test_capped_logits(rows, n):
+    g = torch.Generator().manual_seed(n)
+    x, w = rnd(rows, 256, dt=torch.bfloat16, g=g).to(DEV), rnd(n, 256, dt=torch.bfloat16, g=g).to(DEV)
+    z = M.linear_f32(x, w)
+    assert torch.equal(M.linear_f32(x, w, 30.0), M.tanh_cap_(z.clone(), 30.0))
