@@ -17,6 +17,12 @@ int mx_layer_norm(float* x, const void* y, int y_bf16, long y_stride, const floa
 int mx_tanh_cap(float* x, long n, float cap, hipStream_t s);
 int mx_grouped_gemm(void* C, const void* A, long a_rows, const int* rows, const void* W, const int* offs, int groups, long M,
                     int N, int K, int act, float limit, hipStream_t s);
+int mx_head_product_fits(int K, int N);
+int mx_latent_q_absorb(float* qa, float* qr, const void* q, int bf16, long stride, const float* wuk, const float* table,
+                       int table_rows, int dims, const int* positions, int rows, int heads, int K, int N, int dr,
+                       int interleaved, hipStream_t s);
+int mx_head_values(void* out, int out_bf16, const float* o, const float* wuv, const void* gate, long gate_stride,
+                   int rows, int heads, int K, int N, hipStream_t s);
 int mx_norm_route_fits(int width, int experts);
 int mx_norm_route(int* idx, float* wts, void* h, float* x, const void* y, int y_bf16, long y_stride,
                   int layer, const float* wb, const float* w, const float* b, float eps, const float* router, const float* bias, long rows,
@@ -1674,9 +1680,48 @@ void heads_to_rows(const Tensor& out, const Tensor& o, const OptT& inv, const Op
 void scaled_heads_gate(Tensor out, Tensor o, Tensor inv, OptT gate) { heads_to_rows(out, o, inv, gate, false); }
 void head_gate(Tensor out, Tensor o, Tensor gate) { heads_to_rows(out, o, {}, gate, true); }
 
+bool head_product_fits(int64_t k, int64_t n) { return mx_head_product_fits((int)k, (int)n) != 0; }
+
+// few rows: latent_q_rope with its unrotated part taken through wuk [heads][dn][rank], fp32
+void latent_q_absorb(Tensor qa, Tensor qr, Tensor q, Tensor wuk, Tensor table, int64_t dims, Tensor positions, int64_t dr,
+                     bool interleaved) {
+  check_f32(qa, "qa");
+  check_f32(qr, "qr");
+  check_rows(q, "q");
+  check_f32(wuk, "wuk");
+  check_f32(table, "rope table");
+  check_i32(positions, "positions");
+  TORCH_CHECK(wuk.dim() == 3 && head_product_fits(wuk.size(1), wuk.size(2)), "wuk");
+  const int64_t t = q.size(0), heads = wuk.size(0), dn = wuk.size(1), rank = wuk.size(2);
+  TORCH_CHECK(dr >= 0 && q.size(1) == heads * (dn + dr) && qa.numel() == heads * t * rank && qr.numel() == t * heads * dr &&
+              dims % 2 == 0 && dims <= dr && table.dim() == 2 && table.size(1) == dims && positions.numel() >= t &&
+              t <= 0x7fffffff, "latent_q_absorb shapes");
+  chk(mx_latent_q_absorb(qa.data_ptr<float>(), qr.data_ptr<float>(), q.data_ptr(), bf(q), q.stride(0), wuk.data_ptr<float>(),
+                         table.data_ptr<float>(), (int)table.size(0), (int)dims, positions.data_ptr<int>(), (int)t, (int)heads,
+                         (int)dn, (int)rank, (int)dr, interleaved ? 1 : 0, stream()), "latent_q_absorb");
+}
+
+// few rows: o [heads][T][rank] through wuv [heads][rank][dv], gated per head, as rows
+void head_values(Tensor out, Tensor o, Tensor wuv, OptT gate) {
+  check_f32(o, "o");
+  check_f32(wuv, "wuv");
+  TORCH_CHECK(o.dim() == 3 && wuv.dim() == 3 && wuv.size(0) == o.size(0) && wuv.size(1) == o.size(2) &&
+              head_product_fits(wuv.size(1), wuv.size(2)), "head_values: o / wuv");
+  const int64_t heads = o.size(0), t = o.size(1), dv = wuv.size(2);
+  TORCH_CHECK(out.is_cuda() && out.is_contiguous() && is_act(out) && out.dim() == 2 && out.size(0) == t &&
+              out.size(1) == heads * dv && t <= 0x7fffffff, "out");
+  long gs = 0;
+  const void* gp = gate_rows(gate, out, t, heads, &gs);
+  chk(mx_head_values(out.data_ptr(), bf(out), o.data_ptr<float>(), wuv.data_ptr<float>(), gp, gs, (int)t, (int)heads,
+                     (int)o.size(2), (int)dv, stream()), "head_values");
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  m.def("head_product_fits", &head_product_fits);
+  m.def("latent_q_absorb", &latent_q_absorb);
+  m.def("head_values", &head_values);
   m.def("embed_rows", &embed_rows);
   m.def("add_rms_norm", &add_rms_norm);
   m.def("layer_norm", &layer_norm);

@@ -207,7 +207,7 @@ struct ConvWalk {
 };
 
 // sum_sp w[sp] acc[sp * stride + c] for a wave that owns columns [c0, c0 + 256) of n: w is lane
-// sp's value (slices <= 64; a slice of weight 0 is not read).  VEC (n and stride multiples of 4,
+// sp's value (slices <= 64, 0 beyond them; a slice of weight 0 adds nothing).  VEC (n and stride multiples of 4,
 // 16-byte aligned): several slices per pass, 16-byte loads; out(c, value) is called once per
 // column by one lane.
 template <bool VEC, typename F>
@@ -220,16 +220,24 @@ __device__ __forceinline__ void merge_slices(const float* __restrict__ acc, long
     while (lpp < pieces) lpp <<= 1;              // lanes per slice
     const int per = 64 / lpp, sub = lane / lpp, pc = lane & (lpp - 1);
     float v[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 8
-    for (int s0 = 0; s0 < slices; s0 += per) {
-      const int sp = s0 + sub;
-      const float ws = __shfl(w, min(sp, 63));
-      if (sp < slices && ws != 0.f && pc < pieces) {
-        const float4 a = *reinterpret_cast<const float4*>(acc + sp * stride + c0 + 4 * pc);
-        v[0] += ws * a.x;
-        v[1] += ws * a.y;
-        v[2] += ws * a.z;
-        v[3] += ws * a.w;
+    // eight passes' loads at a time without a branch among them (with one per slice 32 slices of 512 columns took 14 us,
+    // so 6); a slice of weight 0 may hold anything and adds nothing
+    const unsigned long long some = __builtin_amdgcn_ballot_w64(w != 0.f);
+    for (int s0 = 0; s0 < slices; s0 += 8 * per) {
+      if (((some >> s0) & (8 * per < 64 ? (1ull << (8 * per)) - 1 : ~0ull)) == 0) continue;
+      float4 a[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        a[u] = *reinterpret_cast<const float4*>(acc + min(s0 + u * per + sub, slices - 1) * stride + c0 + 4 * min(pc, pieces - 1));
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int sp = s0 + u * per + sub;
+        const float ws = __shfl(w, min(sp, 63));
+        const bool on = sp < slices && ws != 0.f;
+        v[0] = on ? v[0] + ws * a[u].x : v[0];
+        v[1] = on ? v[1] + ws * a[u].y : v[1];
+        v[2] = on ? v[2] + ws * a[u].z : v[2];
+        v[3] = on ? v[3] + ws * a[u].w : v[3];
       }
     }
     for (int off = lpp; off < 64; off <<= 1) {

@@ -128,9 +128,8 @@ class LatentAttention:
         else:
             M.latent_kv_write(dkv, self.dkv_norm, self.eps, self.table, self.rot_dims, ctx.positions,
                               ctx.slot_mapping, cache, self.rank, self.interleaved)
-        qn, qr = M.latent_q_rope(q, self.table, self.rot_dims, ctx.positions, self.heads, self.dn,
-                                 self.dr, self.interleaved)
-        qa = torch.bmm(qn.transpose(0, 1), self.wuk)                 # [heads, T, rank]
+        qa, qr = M.latent_q_absorb(q, self.wuk, self.table, self.rot_dims, ctx.positions, self.heads, self.dn,
+                                   self.dr, self.interleaved)         # [heads, T, rank]
         seg = ctx.seg
         if seg.host is not None and seg.max_rows >= self.PRODUCT_ROWS:
             # prefill chunks in tiles; short segments and decode rows (if any) keep the per-row
@@ -143,11 +142,7 @@ class LatentAttention:
                                         self.PRODUCT_ROWS, self.dtype, self.sink)
         else:
             ol = M.latent_attention(qa, qr, cache, seg, self.scale, self.rank, sink=self.sink)
-        o = torch.bmm(ol, self.wuvT)                                  # [heads, T, vdim]
-        if self.gated:
-            return M.linear(M.head_gate(o, qd[:, self.n_down:], self.dtype), self.wo)
-        o = o.transpose(0, 1).reshape(t, self.heads * self.dv).to(self.dtype)
-        return M.linear(o, self.wo)
+        return M.linear(M.head_values(ol, self.wuvT, qd[:, self.n_down:] if self.gated else None, self.dtype), self.wo)
 
 
 class ChannelDelta:

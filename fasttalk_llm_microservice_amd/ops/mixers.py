@@ -662,6 +662,47 @@ def latent_q_rope(q, table, rot_dims: int, positions, heads: int, dn: int, dr: i
     return ref.latent_q_rope(q, table, rot_dims, positions, heads, dn, dr, interleaved)
 
 
+# rows up to which a fp32 matrix per head goes through head_product.hip: it takes eight rows at a time, the library's batched
+# product all of them, in two launches with what is around it.  us of both products at 3 8 16 24 32 rows (rotation, gate and
+# rounding in the second): 16 heads, 128 -> 512 -> 128: 8 11 17 24 31 (library 23 23 22 22 22); 128 heads 15 22 36 52 65
+# (59 60 59 65 62); 40 heads, 64 -> 256 -> 64: 7 10 16 22 27 (19 20 20 22 22)
+HEAD_PRODUCT_ROWS = 16
+
+
+def _head_product(rows: int, w) -> bool:
+    """Whether the kernels of few rows (csrc/mixers/head_product.hip) take a fp32 matrix per head."""
+    return bool(w.is_cuda and rows <= HEAD_PRODUCT_ROWS and w.dtype == torch.float32 and w.is_contiguous()
+                and w.data_ptr() % 16 == 0 and native_mixers().head_product_fits(w.shape[1], w.shape[2]))
+
+
+def latent_q_absorb(q, wuk, table, rot_dims: int, positions, heads: int, dn: int, dr: int, interleaved: bool = False):
+    """:func:`latent_q_rope` and the unrotated parts' way into latent space: (fp32 [heads, T, rank] = q W_uk per head, ``wuk``
+    fp32 [heads, dn, rank]; the rotated parts fp32 [T, heads, dr]).  One launch for few rows."""
+    t = q.shape[0]
+    if _head_product(t, wuk) and q.stride(1) == 1 and q.stride(0) % 4 == 0 and (dn + dr) % 4 == 0 \
+            and q.data_ptr() % (4 * q.element_size()) == 0:
+        qa = torch.empty(heads, t, wuk.shape[2], dtype=torch.float32, device=q.device)
+        qr = torch.empty(t, heads, dr, dtype=torch.float32, device=q.device)
+        native_mixers().latent_q_absorb(qa, qr, q, wuk, table, rot_dims, positions, dr, bool(interleaved))
+        return qa, qr
+    qn, qr = latent_q_rope(q, table, rot_dims, positions, heads, dn, dr, interleaved)
+    return torch.bmm(qn.transpose(0, 1), wuk), qr
+
+
+def head_values(ol, wuv, gate, out_dtype) -> torch.Tensor:
+    """Latent-space sums ``ol`` fp32 [heads, T, rank] through ``wuv`` fp32 [heads, rank, dv], times sigmoid(gate[t, h]) if there
+    is a ``gate`` [T, heads], as rows [T, heads * dv] in ``out_dtype``.  One launch for few rows."""
+    heads, t = ol.shape[:2]
+    if _head_product(t, wuv) and ol.is_contiguous():
+        out = torch.empty(t, heads * wuv.shape[2], dtype=out_dtype, device=ol.device)
+        native_mixers().head_values(out, ol, wuv, gate)
+        return out
+    o = torch.bmm(ol, wuv)                                               # [heads, T, dv]
+    if gate is not None:
+        return head_gate(o, gate, out_dtype)
+    return o.transpose(0, 1).reshape(t, heads * wuv.shape[2]).to(out_dtype)
+
+
 def latent_attention(qa, qr, cache, seg: Segments, scale: float, rank: int,
                      skip_from: int = 0, out: Optional[torch.Tensor] = None,
                      sink: Optional[torch.Tensor] = None) -> torch.Tensor:
