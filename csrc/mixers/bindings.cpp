@@ -231,7 +231,7 @@ int mx_band_attn(void* out, int out_bf16, const float* q, const void* k_cache, c
                  long long_rows, int heads, int maps, int kv_heads, int dk, int dv, int window, float scale, int sigmoid,
                  const float* r1, const float* r2, const float* pb, int block_size, int num_blocks, int min_rows,
                  float softcap, int has_sink, float sink, const float* sinks, int blocks, int keep_first,
-                 const float* dist_bias, int nd, hipStream_t s);
+                 const float* dist_bias, int nd, int groups, hipStream_t s);
 int mx_few_rows_gemm(void* Y, int y_f32, long y_stride, const void* X, long x_stride, int rows, const void* W,
                      const void* bias, int N, int K, int act, float limit, hipStream_t s);
 int mx_experts_few(float* out, void* y, float* d, const void* h, long h_stride, const int* idx, const float* wts,
@@ -1406,7 +1406,7 @@ void band_attention(Tensor out, Tensor q, Tensor k_cache, Tensor v_cache, Tensor
                     Tensor bt, int64_t num_segs, int64_t long_segs, int64_t long_rows, int64_t heads, int64_t maps,
                     int64_t kv_heads, int64_t dk, int64_t dv, int64_t window, double scale, bool sigmoid, OptT r1,
                     OptT r2, OptT pb, int64_t min_rows, double softcap, c10::optional<double> sink, OptT sinks,
-                    bool blocks, int64_t keep_first, OptT dist_bias) {
+                    bool blocks, int64_t keep_first, OptT dist_bias, int64_t groups) {
   TORCH_CHECK(out.is_cuda() && is_act(out) && out.is_contiguous(), "out: fp32 / bf16 rows");
   check_f32(q, "q");
   TORCH_CHECK(keep_first >= 0 && (!blocks || window >= 1) && min_rows >= 1, "band attention mask");
@@ -1435,7 +1435,7 @@ void band_attention(Tensor out, Tensor q, Tensor k_cache, Tensor v_cache, Tensor
                    (int)min_rows, (float)softcap, sink || sinks ? 1 : 0, sink ? (float)*sink : 0.f,
                    opt_f32(sinks, hq, "sinks"), blocks ? 1 : 0, (int)keep_first,
                    dist_bias ? dist_bias->data_ptr<float>() : nullptr, dist_bias ? (int)dist_bias->size(0) : 0,
-                   stream()), "band_attention");
+                   (int)groups, stream()), "band_attention");
 }
 
 void band_weights(Tensor S, int64_t rows, int64_t first_pos, int64_t key0, int64_t heads, int64_t maps,

@@ -1032,10 +1032,10 @@ def band_attention_ok(out, q, k_cache, v_cache, seg: Segments, spec: WindowSpec)
 def _band_pays(seg: Segments, sp: WindowSpec, min_rows: int) -> bool:
     """A workgroup of the one kernel owns 64 (row, query head) pairs and walks their keys, so a few rows behind a long
     context leave the chip idle, where the products' widened copies and library kernels fill it: 64 rows of 16 heads of
-    128 on 4 key heads at position 8000 take 297 us and the products 138, at 30000 1075 and 562; 32 at 2000 82 and 101, 300
-    at 4000 165 and 235, 2000 from 0 112 and 518.  A key costs the walk 36 ns (plain; 50 to 58 with a cap, a table or
-    sigmoids), 340 walks at a time; the products, whose 25 launches take 100 us to issue, the reads of the cache and the
-    pairs' sums."""
+    128 on 4 key heads at position 8000 take 165 us and the products 149, at 30000 591 and 570; 64 at 2000 52 and 115, 300
+    at 4000 96 and 252, 2000 from 0 70 and 474.  The line is drawn for a walk of 36 ns a key (plain; 50 to 58 with a cap, a
+    table or sigmoids), 340 walks at a time, half as fast as it is now, so it errs towards the products, by up to their 100
+    us; those: 25 launches that take 100 us to issue, the reads of the cache and the pairs' sums."""
     start, _, kv_len = seg.host
     wide, rep = (sp.dk + sp.dv) / 256, sp.heads // sp.kv_heads
     kind = 33 if sp.sigmoid else 30 if sp.dist_bias is not None else 28 if sp.softcap > 0 else 14
@@ -1050,6 +1050,28 @@ def _band_pays(seg: Segments, sp: WindowSpec, min_rows: int) -> bool:
         total += keys * sp.kv_heads * sp.maps * (-(-n * rep // 64))
         products += max(100.0, 20 + 1e-3 * keys * (a + b * n) * (0.8 if sp.sigmoid else 1.0))
     return 10 + 1e-3 * (kind + 22 * wide) * max(longest, total / 340) <= products
+
+
+def _band_groups(seg: Segments, sp: WindowSpec, min_rows: int) -> int:
+    """Groups of waves in a workgroup of the one kernel.  Two walk a block's tiles of 64 keys in turn, 1.3 us a tile where one
+    takes 1.7 to 2; but one leaves room for a second workgroup on the CU, which hides its own start and end (8 and 11 us) and
+    gets 1.35 us a tile out of the CU where two groups get 1.5.  So two where the longest walk is what counts: us with one / two,
+    16 heads of 128 on 4 key heads: 300 rows 15.7 16.5, 600 23.5 22.1, 777 30 28, 1000 37 33, 2048 74 70, 4096 206 216, 8192 699
+    772; 64 at 2000 64 52, at 30000 822 608; 1500 at 3000 160 169; 16 of 100 16 25, five of 258 to 542 30 35; 2048 in a window
+    of 512 35 45, of two maps 96 107."""
+    start, _, kv_len = seg.host
+    rep, heads = sp.heads // sp.kv_heads, sp.kv_heads * sp.maps
+    longest = tiles = groups = 0.0
+    for n, kv in zip((y - x for x, y in zip(start[:-1], start[1:])), kv_len):
+        if n < min_rows:
+            continue
+        top, mean, blocks = kv, kv - n / 2, -(-n * rep // 64) * heads
+        if sp.window > 0:
+            top, mean = min(top, sp.window), min(mean, sp.window / 2 if sp.blocks and kv > sp.window else sp.window)
+        longest = max(longest, top / 64)
+        tiles += blocks * max(1.0, mean / 64)
+        groups += blocks
+    return 2 if longest > 5 and tiles / 256 + 4 * max(0.0, groups / 256 - 1) < 1.2 * longest else 1
 
 
 def window_attention_products(out, q, k_cache, v_cache, seg: Segments, spec: WindowSpec, min_rows: int):
@@ -1072,7 +1094,7 @@ def window_attention_products(out, q, k_cache, v_cache, seg: Segments, spec: Win
                                        seg.num, len(ns), sum(ns), sp.heads, sp.maps, sp.kv_heads, sp.dk, sp.dv,
                                        sp.window, float(sp.scale), bool(sp.sigmoid), sp.r1, sp.r2, sp.pb, min_rows,
                                        float(sp.softcap), *_sink_args(sp.sink), bool(sp.blocks), int(sp.keep_first),
-                                       sp.dist_bias)
+                                       sp.dist_bias, _band_groups(seg, sp, min_rows))
         return out
     rep = sp.heads // sp.kv_heads
     gk = sp.kv_heads * sp.maps

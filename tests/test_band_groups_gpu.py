@@ -1,0 +1,59 @@
+"""The one-pass attention of long segments with one and with two groups of waves to a workgroup (csrc/mixers/band_attn.hip)
+against 64 bits: no, one, an odd and an even number of key tiles, tiles without keys of theirs, a scale below zero."""
+import pytest
+import torch
+
+from fasttalk_llm_microservice_amd.ops import mixers as M
+from test_band_attention_gpu import DEV, cases, reference, segments
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("name,sizes,opt,lens,pos0", [c for c in cases() if c[0] in (
+    "causal, cap, sink 0", "window, kept, table", "sigmoid, distance", "two maps", "blocks")] + [
+    ("one tile", dict(heads=4, kv_heads=1, dk=128, dv=128, window=0), {}, [64, 1], [0, 0]),
+    ("three tiles, a sink each", dict(heads=4, kv_heads=4, dk=64, dv=128, window=0), dict(sinks=True), [33, 129], [159, 0]),
+    ("below zero", dict(heads=2, kv_heads=2, dk=64, dv=64, window=0), dict(scale=-0.125), [140], [70])],
+    ids=lambda v: v if isinstance(v, str) else "")
+def test_groups(name, sizes, opt, lens, pos0, monkeypatch):
+    g = torch.Generator().manual_seed(len(name))
+    rnd = lambda *s: torch.randn(*s, generator=g)   # noqa: E731
+    opt, hq = dict(opt), sizes["heads"] * opt.get("maps", 1)
+    table, terms, sinks = opt.pop("table", 0), opt.pop("terms", False), opt.pop("sinks", False)
+    if table:
+        opt["dist_bias"] = (0.5 * rnd(table, hq)).to(DEV)
+    if terms:
+        opt.update({k: torch.rand(hq, generator=g).to(DEV) for k in ("r1", "r2", "pb")})
+    if sinks:
+        opt["sink"] = rnd(hq).to(DEV)
+    sp = M.WindowSpec(**{"scale": sizes["dk"] ** -0.5, **sizes, **opt})
+    seg, blocks = segments(lens, pos0, 16, g)
+    kc = rnd(blocks, 16, sp.kv_heads * sp.maps * sp.dk).to(DEV, torch.bfloat16)
+    vc = rnd(blocks, 16, sp.kv_heads * sp.dv).to(DEV, torch.bfloat16)
+    q = (2.0 * rnd(sum(lens), hq * sp.dk)).to(DEV)
+    want = reference(q, kc, vc, seg, sp, 32)
+    # what a page holds past the last key counts for nothing
+    for s in range(seg.num):
+        kv = seg.host[2][s]
+        if kv % 16:
+            page = int(seg.block_tables[s, kv // 16])
+            kc[page, kv % 16:] = float("nan")
+            vc[page, kv % 16:] = float("nan")
+    rows = torch.cat([torch.full((n,), n >= 32) for n in lens]).to(DEV)
+    norm = float(want[rows].norm())
+    monkeypatch.setattr(M, "_band_pays", lambda *a: True)
+    for groups in (1, 2):
+        monkeypatch.setattr(M, "_band_groups", lambda *a: groups)
+        got = M.window_attention_products(torch.full((q.shape[0], hq, sp.dv), 7.0, device=DEV), q, kc, vc, seg, sp, 32)
+        assert bool((got[~rows] == 7.0).all())
+        # fp32 sums of a few hundred terms: about 2^-22
+        assert float((got.double() - want)[rows].norm()) / norm < 1e-6
+
+
+@pytest.mark.parametrize("rows,count,pos,window,groups", [(300, 1, 0, 0, 1), (777, 1, 0, 0, 2), (2048, 1, 0, 0, 2),
+                                                          (8192, 1, 0, 0, 1), (64, 1, 8000, 0, 2), (100, 16, 0, 0, 1),
+                                                          (2048, 1, 0, 512, 1)])
+def test_rule(rows, count, pos, window, groups):
+    start = [i * rows for i in range(count + 1)]
+    seg = M.Segments(None, None, None, None, None, count, rows, pos + rows, host=(start, [pos] * count, [pos + rows] * count))
+    assert M._band_groups(seg, M.WindowSpec(heads=16, kv_heads=4, dk=128, dv=128, window=window, scale=1.0), 32) == groups
