@@ -220,6 +220,13 @@ def prefill_partials(nkv: int, head_dim: int, max_partials: int = PREFILL_MAX_PA
 # plans one round instead of two (4 x 150 new over 1.5k: 46.9 vs 58.9 us)
 PREFILL_ITEM_TILES = float(os.environ.get("FT_PREFILL_ITEM_TILES", "2.0"))
 PREFILL_MAX_ROUNDS = 4
+# for plans of uneven items, in tiles (2 us each): an item's start and end, the merge of split ones, and a split item's
+# partial sums per key / value head.  us of plans that cut at so many tiles, 32 heads on 8: 2048 tokens at 9 12 16 24 and
+# whole 84 68 68 63 72 (9: two items a CU); 1500 at 6 8 10 14 whole 53 54 53 46 54; 1000 at 4 6 8 whole 41 32
+# 33 39; 777 at 4 6 8 whole 28 30 31 33; 5 x 400 at 4 6 whole 35 31 24; 3000 at 18 24 32 whole 122 115 103 102
+PREFILL_UNEVEN_ITEM = 4.0
+PREFILL_MERGE = 3.0
+PREFILL_PARTIAL = 0.025
 PREFILL_ROUND_BLIND = os.environ.get("FT_PREFILL_ROUND_BLIND", "0") == "1"
 
 
@@ -250,7 +257,8 @@ def build_prefill_tiles(q_lens, tile_tokens: int, seq_lens=None, nkv: int = 8, n
     LDS), so the grid executes in rounds of ``num_cus`` workgroups (= num_cus / nkv
     items): for 1..PREFILL_MAX_ROUNDS rounds the smallest chunk (>= min_split_tiles
     tiles) whose items fit is found and the plan with the least estimated makespan
-    (rounds x (longest item + PREFILL_ITEM_TILES)) wins.  The earlier plan aimed at
+    (rounds x (longest item + PREFILL_ITEM_TILES)) wins; of ranges that differ by
+    more than 2x see PREFILL_UNEVEN_ITEM.  The earlier plan aimed at
     ~2 workgroups per CU and rounded every block's split up, e.g. 520 workgroups for
     5 prompts x 107 tokens over 3k: a third round for 8 workgroups."""
     blocks = []
@@ -285,12 +293,20 @@ def build_prefill_tiles(q_lens, tile_tokens: int, seq_lens=None, nkv: int = 8, n
     chunk = 0
     nk_lo = min(n for _, _, n in blocks) if blocks else 0
     nk_hi = max(n for _, _, n in blocks) if blocks else 0
-    # the round model assumes near-equal items: a causal prompt's early blocks (a few
-    # tiles each) make the greedy dispatch far from it (1 x 2048 fresh tokens ran 103
-    # vs 91 us on the round-aware plan), so ranges that differ by more than 2x keep
-    # the round-blind split (profiles/prefill_round_plan_r03.log)
-    blind = PREFILL_ROUND_BLIND or nk_lo * 2 < nk_hi
-    if seq_lens is not None and blocks and blind:
+    # the round model assumes near-equal items; where ranges differ by more than 2x (a causal prompt's
+    # early blocks) the items start longest first, and the time is that of the longest one or of all of them
+    # evenly over the CUs
+    if seq_lens is not None and blocks and nk_lo * 2 < nk_hi and not PREFILL_ROUND_BLIND:
+        total, f = sum(n for _, _, n in blocks), PREFILL_UNEVEN_ITEM
+        best = max(nk_hi + f, (total + f * len(blocks)) / per_round)       # whole
+        if best > (total + f * len(blocks)) / per_round + PREFILL_MERGE:
+            cuts = [c for c in sorted({-(-nk_hi // k) for k in (2, 3, 4, 5, 6, 8, 12, 16, 24, 32)}) if c >= min_split_tiles]
+            ns = -(-np.array([n for _, _, n in blocks]) // np.array(cuts or [nk_hi])[:, None])
+            for c, n, part in zip(cuts, ns.sum(1).tolist(), (ns * (ns > 1)).sum(1).tolist()):
+                cost = max(c + f, (total + f * n) / per_round) + PREFILL_MERGE + PREFILL_PARTIAL * nkv * part
+                if cost < best and part <= max_partials:
+                    best, chunk = cost, c
+    elif seq_lens is not None and blocks and PREFILL_ROUND_BLIND:
         # the round-2 plan (~2 workgroups per CU, per-block round-up), for A/B runs
         target = 2 * per_round
         total = sum(n for _, _, n in blocks)
@@ -311,7 +327,7 @@ def build_prefill_tiles(q_lens, tile_tokens: int, seq_lens=None, nkv: int = 8, n
             if ok.any():
                 best = int(c[ok][np.argmin(cost[ok])])
                 chunk = best if best < top else 0
-    slots = 0
+    slots, sizes = 0, []
     for b, s, nkt in blocks:
         ns = -(-nkt // chunk) if chunk else 1
         if ns > 1 and slots + ns <= max_partials:
@@ -319,9 +335,16 @@ def build_prefill_tiles(q_lens, tile_tokens: int, seq_lens=None, nkv: int = 8, n
             for j in range(ns):
                 lo, hi = j * nkt // ns, (j + 1) * nkt // ns
                 items.append((b, s, (lo << 16) | hi, slots + j))
+                sizes.append(hi - lo)
             slots += ns
         else:
             items.append((b, s, 0xFFFF, -1))
+            sizes.append(nkt)
+    # the longest first: workgroups start in this order, and one that starts last ends last (4096 tokens of one prompt, us a
+    # layer: 280 with the longest last, 180)
+    if len(items) * nkv > num_cus:
+        order = sorted(range(len(items)), key=sizes.__getitem__, reverse=True)
+        items = [items[i] for i in order]
     return items, combine
 
 
