@@ -833,7 +833,8 @@ class MoEFF:
             self.shared_limit = float(shared_limit or 0.0)
 
     def route(self, h):
-        grouped, few = self.routing == "grouped_softmax", h.shape[0] <= self.PAIR_ROWS
+        grouped = self.routing == "grouped_softmax"
+        few = h.shape[0] <= self.PAIR_ROWS or M.moe_route_by_row(h, self.router)
         if not few and M.moe_route_fits(h, self.router_parts, self.e):
             limited = self.routing != "top_logits"
             return M.moe_route(h, self.router_parts, self.correction if grouped else self.router_bias, self.e, self.top,
@@ -859,7 +860,7 @@ class MoEFF:
     def norm_route(self, x, y, wb, w, b, eps: float, dtype):
         """The norm step in front of this mixture (see :func:`..ops.mixers.norm_route`) with its router, for few rows:
         (h, (idx, wts)), or None where that launch does not take them."""
-        if dtype != torch.bfloat16 or x.shape[0] > self.PAIR_ROWS or not M.norm_route_fits(x, y, wb, w, b, self.router):
+        if dtype != torch.bfloat16 or not M.norm_route_fits(x, y, wb, w, b, self.router):
             return None
         grouped, limited = self.routing == "grouped_softmax", self.routing != "top_logits"
         return M.norm_route(x, y, wb, w, b, eps, self.router, self.correction if grouped else self.router_bias, self.top,
@@ -877,7 +878,7 @@ class MoEFF:
             return M.experts_few(h, idx, wts, self.wgu, self.wdown, self.act, self.limit, self.shared,
                                  self.shared_limit if self.shared is not None else 0.0, self.shared_gate, parts)
         if t > self.PAIR_ROWS and M.experts_many_ok(h, self.wgu, self.wdown):
-            idx, wts = self.route(h)
+            idx, wts = routed or self.route(h)
             shared = gate_w = None
             if self.shared is not None:
                 w1, wdown = self.shared

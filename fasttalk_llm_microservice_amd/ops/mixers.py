@@ -1358,17 +1358,32 @@ def moe_route_softmax(h, router, correction, top: int, groups: int, keep: int):
 
 def moe_route_softmax_pays(experts: int) -> bool:
     """Where :func:`moe_route_softmax`, a workgroup per row that takes the experts sixteen at a time, beats a library
-    product and :func:`moe_topk`: 32 experts 10 us (17 for 64 rows of 2048), 64 15 (18), 128 25 (20)."""
+    product and :func:`moe_topk`: 32 experts 9 us (17 for 64 rows of 2048), 64 10 (18), 128 25 (20)."""
     return experts <= 64
 
 
 ROUTE_MODES = {"top_logits": 0, "top_sigmoid": 1, "grouped_softmax": 2}
 
 
+# Rows up to which a workgroup a row routes (csrc/mixers/moe_route.hip route_rows_kernel; beyond, a workgroup for sixteen with
+# the router on the matrix units), alone and with the norm step in front: two such workgroups fit a CU, and one.  us, 32 experts
+# of 2048 (64 of 2048, 8 of 4096), rows / sixteen a workgroup: 256 rows 9.2 15.4 (11 17, 6.0 9.8), 512 12.8 15.5 (17 17, 9.2
+# 11.1), 777 19.8 15.7 (28 17, 15 12); with the norm 256 rows 11.3 19.1 (13 21, 8.4 14.6), 300 20.5 19.5 (23 21, 14.6 15.3).
+ROUTE_ROWS = 512
+NORM_ROUTE_ROWS = 256
+
+
+def moe_route_by_row(h, router) -> bool:
+    """Whether a workgroup a row is the faster router (:func:`moe_route_top_logits`, :func:`moe_route_softmax`)."""
+    return bool(h.is_cuda and h.shape[0] <= ROUTE_ROWS and h.dtype == torch.bfloat16 and h.stride(1) == 1 and h.stride(0) % 4 == 0
+                and h.data_ptr() % 8 == 0 and router.data_ptr() % 16 == 0
+                and native_mixers().norm_route_fits(h.shape[1], router.shape[0]))
+
+
 def norm_route_fits(x, y, wb, w, b, router) -> bool:
-    """Whether :func:`norm_route` takes these rows: bf16 or fp32 sublayer outputs y on a GPU, at most 64 experts (a lane
-    each), widths of whole 256 up to 8192 (a row in LDS), all at 16-byte addresses."""
-    return bool(y.is_cuda and x.is_contiguous() and y.dim() == 2 and y.shape == x.shape
+    """Whether :func:`norm_route` takes these rows: up to NORM_ROUTE_ROWS bf16 or fp32 sublayer outputs y on a GPU, at most 64
+    experts (a lane each), widths of whole 256 up to 8192 (a row in LDS), all at 16-byte addresses."""
+    return bool(y.is_cuda and y.shape[0] <= NORM_ROUTE_ROWS and x.is_contiguous() and y.dim() == 2 and y.shape == x.shape
                 and y.stride(1) == 1 and y.stride(0) % 4 == 0 and y.data_ptr() % (4 * y.element_size()) == 0
                 and all(t is None or t.data_ptr() % 16 == 0 for t in (x, wb, w, b, router))
                 and native_mixers().norm_route_fits(x.shape[1], router.shape[0]))

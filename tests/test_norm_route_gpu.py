@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 # one pass and several, a router of fewer and more pieces than are in flight, one and two pieces of a row per thread
 @pytest.mark.parametrize("routing,form", [("grouped_softmax", "rms"), ("top_logits", "layer"), ("top_sigmoid", "plain")])
 @pytest.mark.parametrize("rows,width,experts,top,groups,keep,ydt", [
-    (1, 256, 1, 1, 1, 1, torch.bfloat16), (3, 2048, 17, 4, 1, 1, torch.float32), (64, 2048, 32, 4, 4, 2, torch.bfloat16),
+    (1, 256, 1, 1, 1, 1, torch.bfloat16), (256, 512, 6, 2, 1, 1, torch.bfloat16), (3, 2048, 17, 4, 1, 1, torch.float32), (64, 2048, 32, 4, 4, 2, torch.bfloat16),
     (2, 4096, 64, 8, 8, 4, torch.bfloat16), (5, 4352, 33, 3, 3, 2, torch.float32), (2, 8192, 64, 64, 64, 64, torch.bfloat16)])
 def test_norm_route(routing, form, rows, width, experts, top, groups, keep, ydt):
     if routing == "top_logits":
@@ -119,3 +119,29 @@ def test_capped_logits(rows, n):
     x, w = rnd(rows, 256, dt=torch.bfloat16, g=g).to(DEV), rnd(n, 256, dt=torch.bfloat16, g=g).to(DEV)
     z = M.linear_f32(x, w)
     assert torch.equal(M.linear_f32(x, w, 30.0), M.tanh_cap_(z.clone(), 30.0))
+
+
+@pytest.mark.parametrize("routing", ["grouped_softmax", "top_logits", "top_sigmoid"])
+@pytest.mark.parametrize("rows", [65, 256, 257, 512, 513])
+def test_layer_routes_alike_by_either_kernel(rows, routing):
+    """A mixture's choice where a workgroup takes a row and where it takes sixteen, and behind its norm step."""
+    from fasttalk_llm_microservice_amd.models.mixers import MoEFF
+    g = torch.Generator().manual_seed(rows)
+    sizes = {"router": (12, 2048), "correction": (12,), "router.b": (12,)}
+    size = lambda n: sizes.get(n, (2048, 16) if n.endswith("down") else (16, 2048))      # noqa: E731
+    groups, keep = (1, 1) if routing == "top_logits" else (4, 2)
+    moe = MoEFF(lambda n: rnd(*size(n), g=g, scale=2048 ** -0.5), 12, 3, 7.0, groups, keep, None, torch.bfloat16, DEV, routing=routing)
+    h = rnd(rows, 2048, dt=torch.bfloat16, g=g).to(DEV)
+    idx, wts = moe.route(h)
+    limited = routing != "top_logits"
+    i2, w2 = M.moe_route(h, moe.router_parts, moe.correction if routing == "grouped_softmax" else moe.router_bias, 12, 3, routing,
+                         1.0, groups if limited else 1, keep if limited else 1)
+    near = (wts - w2).abs().max(1).values < 1e-4       # fp32 logits of 2048 terms in another order: level experts may change places
+    assert bool((torch.equal(idx, i2) or float((idx != i2).any(1).float().mean()) < 0.01)) and bool(near.all())
+    x, y, w = rnd(rows, 2048, g=g).to(DEV), rnd(rows, 2048, g=g).to(DEV), torch.ones(2048, device=DEV)
+    got = moe.norm_route(x, y, None, w, None, 1e-5, torch.bfloat16)
+    assert (got is not None) == (rows <= 256)
+    if got is not None:
+        i3, w3 = moe.route(got[0])
+        assert torch.equal(i3, got[1][0])
+        torch.testing.assert_close(w3, got[1][1], rtol=1e-5, atol=1e-7)
