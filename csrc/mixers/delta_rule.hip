@@ -55,8 +55,8 @@ __global__ void short_conv_kernel(T* __restrict__ out, const T* __restrict__ x, 
 
 // The same for TAPS taps and rows of whole 16-byte pieces: a thread owns the V channels of a piece over
 // kConvRows rows, all their loads in flight at once and each input read once per thread instead of once
-// per tap.  Bound by the read and write of the rows: 4096 rows of 6144 channels, bf16, 34 us
-// (one thread per value, 143).  A segment that fits one tile leaves its history here, longer ones to
+// per tap.  Bound by the read and write of the rows: 4096 rows of 6144 channels, bf16, 32 us
+// (one thread per value, 143), half of it for the sigmoids.  A segment that fits one tile leaves its history here, longer ones to
 // conv_hist_kernel (another workgroup may still read the old history).
 constexpr int kConvRows = 8;
 
