@@ -401,7 +401,7 @@ channel_out_kernel(float* __restrict__ o, ChannelIn in, const float* __restrict_
     for (int e = 0; e < 4; ++e)
 #pragma unroll
       for (int ct = 0; ct < 4; ++ct)
-        O[ct] = mma(qf[i][e], vb[i / 4][(16 * (i % 4) + 4 * e + hi) * kVLD + 16 * ct + lo], O[ct]);
+        O[ct] = mma(qf[i][e], vb[i / 4][swizzled<kVLD>(16 * (i % 4) + 4 * e + hi, 16 * ct + lo)], O[ct]);
   __syncthreads();
   float* wb = vb[0];
   if constexpr (DELTA) {
@@ -412,7 +412,7 @@ channel_out_kernel(float* __restrict__ o, ChannelIn in, const float* __restrict_
     for (int m = 0; m < 4; ++m) {
       const f32x4 u = fp[(tile * 4 + m) * 64 + lane];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) wb[(16 * m + 4 * hi + r) * kVLD + 16 * wave + lo] = u[r];
+      for (int r = 0; r < 4; ++r) wb[swizzled<kVLD>(16 * m + 4 * hi + r, 16 * wave + lo)] = u[r];
     }
   } else {
     stage_cols<TV>(wb, (const TV*)in.v + c.row0 * in.v_stride + (long)h * dv, in.v_stride, c.cnt, col0, dv, vec);
@@ -424,7 +424,7 @@ channel_out_kernel(float* __restrict__ o, ChannelIn in, const float* __restrict_
 #pragma unroll
     for (int e = 0; e < 4; ++e)
 #pragma unroll
-      for (int ct = 0; ct < 4; ++ct) O[ct] = mma(pf[b][e], wb[(16 * b + 4 * e + hi) * kVLD + 16 * ct + lo], O[ct]);
+      for (int ct = 0; ct < 4; ++ct) O[ct] = mma(pf[b][e], wb[swizzled<kVLD>(16 * b + 4 * e + hi, 16 * ct + lo)], O[ct]);
   }
 #pragma unroll
   for (int r = 0; r < 4; ++r) {

@@ -12,7 +12,11 @@ namespace mx {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 constexpr int kC = 64;          // rows per chunk
-constexpr int kVLD = 80;        // floats between rows of a staged [rows][64 columns] tile
+// entry (row, col) of a staged tile of `ld` floats a row, 16-column blocks exchanged by the row: lanes (hi, lo) that read rows
+// 4 s + hi, columns lo fall on all 64 banks, without padding (which cost chunk_out and state_add the third workgroup a CU)
+template <int LD>
+__device__ __forceinline__ int swizzled(int row, int col) { return row * LD + (col ^ ((row & 3) << 4)); }
+constexpr int kVLD = 64;        // of a [rows][64 columns] tile
 constexpr int kPLD = 68;        // floats between rows of a staged [16][64] strip
 
 __device__ __forceinline__ f32x4 mma(float a, float b, f32x4 c) {
@@ -42,21 +46,47 @@ __device__ __forceinline__ void load4(const bf16_t* p, float* v) {
   ft::unpack2(u.y, v[2], v[3]);
 }
 
-// rows [0, cnt) x 64 columns from col0 of a [., dv] array into LDS [kC][kVLD], zeros elsewhere
+// Four neighbouring entries of a row on their way to LDS: what is fetched is put later, so a workgroup asks for all of a tile
+// at once, and for the next one before it needs it (chunk_out of 2048 rows, 64 heads of 128 x 64, with loads behind a branch
+// each, one after the other, 104 us; so 81; with three workgroups a CU 73).
+template <typename T>
+using Four = typename std::conditional<sizeof(T) == 2, uint2, float4>::type;
+__device__ __forceinline__ float4 widen(const float4& u) { return u; }
+__device__ __forceinline__ float4 widen(const uint2& u) {
+  float4 v;
+  ft::unpack2(u.x, v.x, v.y);
+  ft::unpack2(u.y, v.z, v.w);
+  return v;
+}
+
+// rows [0, cnt) x 64 columns from col0 of a [., dv] array (dv in whole fours), by 256 threads; rows past the end read the last
+template <typename T>
+__device__ __forceinline__ void fetch_cols(Four<T> (&u)[4], const T* src, long stride, int cnt, int col0, int dv) {
+#pragma unroll
+  for (int n = 0; n < 4; ++n) {
+    const int e = threadIdx.x + 256 * n, t = min(e >> 4, cnt - 1), c = min(col0 + (e & 15) * 4, dv - 4);
+    u[n] = *reinterpret_cast<const Four<T>*>(src + t * stride + c);
+  }
+}
+// into LDS [kC][kVLD] (swizzled), zeros elsewhere
+template <typename F>
+__device__ __forceinline__ void put_cols(float* dst, const F (&u)[4], int cnt, int col0, int dv) {
+#pragma unroll
+  for (int n = 0; n < 4; ++n) {
+    const int e = threadIdx.x + 256 * n, t = e >> 4, c = (e & 15) * 4;
+    *reinterpret_cast<float4*>(dst + swizzled<kVLD>(t, c)) = t < cnt && col0 + c < dv ? widen(u[n]) : make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+}
 template <typename T>
 __device__ __forceinline__ void stage_cols(float* dst, const T* src, long stride, int cnt, int col0, int dv, int vec) {
-  const int tid = threadIdx.x;
   if (vec) {
-    for (int e = tid; e < kC * 16; e += 256) {
-      const int t = e >> 4, c = (e & 15) * 4;
-      float v[4] = {0.f, 0.f, 0.f, 0.f};
-      if (t < cnt && col0 + c < dv) load4(src + t * stride + col0 + c, v);
-      *reinterpret_cast<float4*>(dst + t * kVLD + c) = make_float4(v[0], v[1], v[2], v[3]);
-    }
+    Four<T> u[4];
+    fetch_cols<T>(u, src, stride, cnt, col0, dv);
+    put_cols(dst, u, cnt, col0, dv);
   } else {
-    for (int e = tid; e < kC * 64; e += 256) {
+    for (int e = threadIdx.x; e < kC * 64; e += 256) {
       const int t = e >> 6, c = e & 63;
-      dst[t * kVLD + c] = t < cnt && col0 + c < dv ? ld(src, t * stride + col0 + c) : 0.f;
+      dst[swizzled<kVLD>(t, c)] = t < cnt && col0 + c < dv ? ld(src, t * stride + col0 + c) : 0.f;
     }
   }
 }

@@ -54,10 +54,31 @@ struct ChunkIn {
   const float* skip;                   // o += skip[h] v, null: none
 };
 
-// rows [0, cnt) of one head of q or k into LDS [kC][LDK], rotated, times scale; zeros past cnt
-// and past dk (up to DKP)
+// rows [0, cnt) of one head of q or k (dk in whole fours, DKP of them padded), by 256 threads; rows past the end read the last
 template <typename T, int DKP>
-__device__ __forceinline__ void stage_head(float* dst, int LDK, const T* src, long stride, int cnt, int dk,
+__device__ __forceinline__ void fetch_head(Four<T> (&u)[DKP / 16], const T* src, long stride, int cnt, int dk) {
+#pragma unroll
+  for (int n = 0; n < DKP / 16; ++n) {
+    const int e = threadIdx.x + 256 * n, t = min(e / (DKP / 4), cnt - 1), i = min(e % (DKP / 4) * 4, dk - 4);
+    u[n] = *reinterpret_cast<const Four<T>*>(src + t * stride + i);
+  }
+}
+// times scale into LDS, entry (row, column) at `at`, zeros elsewhere
+template <typename F, int DKP, typename At>
+__device__ __forceinline__ void put_head(float* dst, At at, const F (&u)[DKP / 16], int cnt, int dk, float scale) {
+#pragma unroll
+  for (int n = 0; n < DKP / 16; ++n) {
+    const int e = threadIdx.x + 256 * n, t = e / (DKP / 4), i = e % (DKP / 4) * 4;
+    const float4 v = widen(u[n]);
+    const float f = t < cnt && i < dk ? scale : 0.f;
+    *reinterpret_cast<float4*>(dst + at(t, i)) = f != 0.f ? make_float4(v.x * f, v.y * f, v.z * f, v.w * f) : make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+}
+
+// rows [0, cnt) of one head of q or k into LDS, rotated, times scale; zeros past cnt
+// and past dk (up to DKP)
+template <typename T, int DKP, typename At>
+__device__ __forceinline__ void stage_head(float* dst, At at, const T* src, long stride, int cnt, int dk,
                                            const float* table, int table_rows, int rot, int interleaved, int pos,
                                            float scale, int vec) {
   const int tid = threadIdx.x;
@@ -78,23 +99,19 @@ __device__ __forceinline__ void stage_head(float* dst, int LDK, const T* src, lo
         const int a = interleaved ? 2 * i : i, b = interleaved ? 2 * i + 1 : i + half;
         const float c = cs[i], sn = cs[half + i];
         const float x = ld(src, tt * stride + a), y = ld(src, tt * stride + b);
-        dst[t * LDK + a] = (x * c - y * sn) * f;
-        dst[t * LDK + b] = (y * c + x * sn) * f;
+        dst[at(t, a)] = (x * c - y * sn) * f;
+        dst[at(t, b)] = (y * c + x * sn) * f;
       }
     }
   }
   if (vec && d0 == 0) {
-    for (int e = tid; e < kC * (DKP / 4); e += 256) {
-      const int t = e / (DKP / 4), i = e % (DKP / 4) * 4;
-      float v[4] = {0.f, 0.f, 0.f, 0.f};
-      if (t < cnt && i < dk) load4(src + t * stride + i, v);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) dst[t * LDK + i + j] = v[j] * scale;
-    }
+    Four<T> u[DKP / 16];
+    fetch_head<T, DKP>(u, src, stride, cnt, dk);
+    put_head<Four<T>, DKP>(dst, at, u, cnt, dk, scale);
     return;
   }
   for (int t = t0; t < kC; t += 8)
-    for (int i = d0 + l0; i < DKP; i += 32) dst[t * LDK + i] = t < cnt && i < dk ? ld(src, t * stride + i) * scale : 0.f;
+    for (int i = d0 + l0; i < DKP; i += 32) dst[at(t, i)] = t < cnt && i < dk ? ld(src, t * stride + i) * scale : 0.f;
 }
 
 // G[t] = sum of the chunk's log decays up to t (wave 0; 64 rows)
@@ -127,7 +144,8 @@ __global__ void __launch_bounds__(256)
 state_add_kernel(float* __restrict__ ws_s, float* __restrict__ totals, ChunkIn in, const int* __restrict__ start,
                  const int* __restrict__ pos0, const int* __restrict__ slot, int heads, int dk, int dv, int num_slots,
                  ChunkSteps st, int vec) {
-  constexpr int DKP = 16 * DKT, LDK = DKP + 16;
+  constexpr int DKP = 16 * DKT, LDK = DKT >= 4 ? DKP : DKP + 16;       // (fewer blocks than there are to exchange: padded)
+  auto at = [](int row, int col) { return DKT >= 4 ? swizzled<LDK>(row, col) : row * LDK + col; };
   __shared__ __attribute__((aligned(16))) float kb[kC * LDK], vb[kC * kVLD];
   __shared__ double G[kC];
   __shared__ float rs[kC];
@@ -139,7 +157,7 @@ state_add_kernel(float* __restrict__ ws_s, float* __restrict__ totals, ChunkIn i
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, lo = lane & 15, hi = lane >> 4;
   stage_log_decay(G, in, c.row0, c.cnt, heads, h);
   stage_row_scale(rs, in, c.row0, c.cnt, heads, h);
-  stage_head<T, DKP>(kb, LDK, (const T*)in.k + c.row0 * in.k_stride + (long)(h / in.rep) * dk, in.k_stride, c.cnt, dk,
+  stage_head<T, DKP>(kb, at, (const T*)in.k + c.row0 * in.k_stride + (long)(h / in.rep) * dk, in.k_stride, c.cnt, dk,
                      in.table, in.table_rows, in.rot_dims, in.interleaved, c.pos, in.k_scale, vec);
   stage_cols<T>(vb, (const T*)in.v + c.row0 * in.v_stride + (long)h * dv, in.v_stride, c.cnt, col0, dv, vec);
   __syncthreads();
@@ -151,9 +169,9 @@ state_add_kernel(float* __restrict__ ws_s, float* __restrict__ totals, ChunkIn i
 #pragma unroll 4
   for (int s = 0; s < kC / 4; ++s) {
     const int j = 4 * s + hi;
-    const float b = vb[j * kVLD + 16 * wave + lo] * (expf((float)(gl - G[j])) * rs[j]);
+    const float b = vb[swizzled<kVLD>(j, 16 * wave + lo)] * (expf((float)(gl - G[j])) * rs[j]);
 #pragma unroll
-    for (int i = 0; i < DKT; ++i) acc[i] = mma(kb[j * LDK + 16 * i + lo], b, acc[i]);
+    for (int i = 0; i < DKT; ++i) acc[i] = mma(kb[at(j, 16 * i + lo)], b, acc[i]);
   }
   const int col = col0 + 16 * wave + lo;
   if (col >= dv) return;
@@ -218,6 +236,7 @@ chunk_out_kernel(float* __restrict__ o, ChunkIn in, const float* __restrict__ ws
                  const int* __restrict__ pos0, const int* __restrict__ slot, int heads, int dk, int dv, int num_slots,
                  ChunkSteps st, int vec) {
   constexpr int DKP = 16 * DKT, LDK = DKP + 4;
+  auto at = [](int row, int col) { return row * LDK + col; };
   constexpr int KB = kC * LDK > 64 * kPLD ? kC * LDK : 64 * kPLD;
   __shared__ __attribute__((aligned(16))) float kb[KB], vb[kC * kVLD];
   __shared__ double G[kC];
@@ -242,10 +261,21 @@ chunk_out_kernel(float* __restrict__ o, ChunkIn in, const float* __restrict__ ws
   const float* S = ws_s + ((c.ws * heads + h) * dk) * (long)dv;
   stage_log_decay(G, in, c.row0, c.cnt, heads, h);
   stage_row_scale(rs, in, c.row0, c.cnt, heads, h);
-  stage_head<T, DKP>(kb, LDK, (const T*)in.q + c.row0 * in.q_stride + hoff, in.q_stride, c.cnt, dk, in.table,
+  stage_head<T, DKP>(kb, at, (const T*)in.q + c.row0 * in.q_stride + hoff, in.q_stride, c.cnt, dk, in.table,
                      in.table_rows, in.rot_dims, in.interleaved, c.pos, 1.f, vec);
   const int svec = dv % 4 == 0;
-  stage_cols<float>(vb, S, dv, dk, col0, dv, svec);         // rows 0 .. 63 of the incoming state
+  stage_cols<float>(vb, S, dv, min(dk, kC), col0, dv, svec);         // rows 0 .. 63 of the incoming state
+  // what follows is asked for now: rows 64 .. of the state, the keys and the values
+  const T* const kp = (const T*)in.k + c.row0 * in.k_stride + hoff;
+  const T* const vp = (const T*)in.v + c.row0 * in.v_stride + (long)h * dv;
+  const bool plain = vec && (in.table == nullptr || in.rot_dims == 0), rows_v = vec && !in.v_frags;
+  Four<float> s_next[4];
+  Four<T> k_next[DKT], v_next[4];
+  if constexpr (DKT > 4) {
+    if (svec) fetch_cols<float>(s_next, S + 64L * dv, dv, dk - 64, col0, dv);
+  }
+  if (plain) fetch_head<T, DKP>(k_next, kp, in.k_stride, c.cnt, dk);
+  if (rows_v) fetch_cols<T>(v_next, vp, in.v_stride, c.cnt, col0, dv);
   __syncthreads();
   float qf[4 * DKT];
 #pragma unroll
@@ -256,19 +286,23 @@ chunk_out_kernel(float* __restrict__ o, ChunkIn in, const float* __restrict__ ws
 #pragma unroll
   for (int s = 0; s < (DKT < 4 ? 4 * DKT : 16); ++s)
 #pragma unroll
-    for (int ct = 0; ct < 4; ++ct) O[ct] = mma(qf[s], vb[(4 * s + hi) * kVLD + 16 * ct + lo], O[ct]);
+    for (int ct = 0; ct < 4; ++ct) O[ct] = mma(qf[s], vb[swizzled<kVLD>(4 * s + hi, 16 * ct + lo)], O[ct]);
   __syncthreads();
   if constexpr (DKT > 4) {                                   // rows 64 .. of the state
-    stage_cols<float>(vb, S + 64L * dv, dv, dk - 64, col0, dv, svec);
+    if (svec) put_cols(vb, s_next, dk - 64, col0, dv);
+    else stage_cols<float>(vb, S + 64L * dv, dv, dk - 64, col0, dv, 0);
     __syncthreads();
 #pragma unroll
     for (int s = 16; s < 4 * DKT; ++s)
 #pragma unroll
-      for (int ct = 0; ct < 4; ++ct) O[ct] = mma(qf[s], vb[(4 * (s - 16) + hi) * kVLD + 16 * ct + lo], O[ct]);
+      for (int ct = 0; ct < 4; ++ct) O[ct] = mma(qf[s], vb[swizzled<kVLD>(4 * (s - 16) + hi, 16 * ct + lo)], O[ct]);
     __syncthreads();
   }
-  stage_head<T, DKP>(kb, LDK, (const T*)in.k + c.row0 * in.k_stride + hoff, in.k_stride, c.cnt, dk, in.table,
-                     in.table_rows, in.rot_dims, in.interleaved, c.pos, in.k_scale, vec);
+  if (plain)
+    put_head<Four<T>, DKP>(kb, at, k_next, c.cnt, dk, in.k_scale);
+  else
+    stage_head<T, DKP>(kb, at, kp, in.k_stride, c.cnt, dk, in.table, in.table_rows, in.rot_dims, in.interleaved, c.pos,
+                       in.k_scale, vec);
   if (in.v_frags) {
     const int tiles = (dv + 15) / 16;
     const float4* fp = (const float4*)in.v + (c.ws * heads + h) * (long)tiles * 256;
@@ -279,11 +313,13 @@ chunk_out_kernel(float* __restrict__ o, ChunkIn in, const float* __restrict__ ws
         const float4 u = fp[(tile * 4 + m) * 64 + lane];
         const float v[4] = {u.x, u.y, u.z, u.w};
 #pragma unroll
-        for (int r = 0; r < 4; ++r) vb[(16 * m + 4 * hi + r) * kVLD + 16 * ct + lo] = v[r];
+        for (int r = 0; r < 4; ++r) vb[swizzled<kVLD>(16 * m + 4 * hi + r, 16 * ct + lo)] = v[r];
       }
     }
+  } else if (rows_v) {
+    put_cols(vb, v_next, c.cnt, col0, dv);
   } else {
-    stage_cols<T>(vb, (const T*)in.v + c.row0 * in.v_stride + (long)h * dv, in.v_stride, c.cnt, col0, dv, vec);
+    stage_cols<T>(vb, vp, in.v_stride, c.cnt, col0, dv, 0);
   }
   double gr[4];
 #pragma unroll
@@ -323,7 +359,7 @@ chunk_out_kernel(float* __restrict__ o, ChunkIn in, const float* __restrict__ ws
     for (int s = 4 * jt; s < 4 * jt + 4; ++s) {
       const float a = strip[lo * kPLD + 4 * s + hi];
 #pragma unroll
-      for (int ct = 0; ct < 4; ++ct) O[ct] = mma(a, vb[(4 * s + hi) * kVLD + 16 * ct + lo], O[ct]);
+      for (int ct = 0; ct < 4; ++ct) O[ct] = mma(a, vb[swizzled<kVLD>(4 * s + hi, 16 * ct + lo)], O[ct]);
     }
   }
 #pragma unroll
@@ -335,7 +371,7 @@ chunk_out_kernel(float* __restrict__ o, ChunkIn in, const float* __restrict__ ws
 #pragma unroll
     for (int ct = 0; ct < 4; ++ct)
       if (col0 + 16 * ct + lo < dv)
-        op[col0 + 16 * ct + lo] = in.skip != nullptr ? O[ct][r] + sk * vb[t * kVLD + 16 * ct + lo] : O[ct][r];
+        op[col0 + 16 * ct + lo] = in.skip != nullptr ? O[ct][r] + sk * vb[swizzled<kVLD>(t, 16 * ct + lo)] : O[ct][r];
   }
 }
 
@@ -350,6 +386,7 @@ delta_solve_kernel(float* __restrict__ ws_w, float* __restrict__ ws_k, float* __
                    const int* __restrict__ pos0, const int* __restrict__ slot, int heads, int dk, int dv, int num_slots,
                    ChunkSteps st, int vec) {
   constexpr int DKP = 16 * DKT, LDK = DKP + 4;
+  auto at = [](int row, int col) { return row * LDK + col; };
   // ab: A, block by block replaced by T = (I + A)^-1 (blocks above the diagonal are never read)
   __shared__ __attribute__((aligned(16))) float kb[kC * LDK], ab[kC * kPLD];
   __shared__ double G[kC];
@@ -361,7 +398,7 @@ delta_solve_kernel(float* __restrict__ ws_w, float* __restrict__ ws_k, float* __
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, lo = lane & 15, hi = lane >> 4;
   stage_log_decay(G, in, c.row0, c.cnt, heads, h);
   if (tid >= 64 && tid < 128) bs[tid - 64] = tid - 64 < c.cnt ? beta[(c.row0 + tid - 64) * heads + h] : 0.f;
-  stage_head<float, DKP>(kb, LDK, (const float*)in.k + c.row0 * in.k_stride + (long)(h / in.rep) * dk, in.k_stride, c.cnt,
+  stage_head<float, DKP>(kb, at, (const float*)in.k + c.row0 * in.k_stride + (long)(h / in.rep) * dk, in.k_stride, c.cnt,
                          dk, nullptr, 0, 0, 0, 0, 1.f, vec);
   __syncthreads();
   if (tid < kC) {
