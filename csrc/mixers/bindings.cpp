@@ -17,6 +17,10 @@ int mx_layer_norm(float* x, const void* y, int y_bf16, long y_stride, const floa
 int mx_tanh_cap(float* x, long n, float cap, hipStream_t s);
 int mx_grouped_gemm(void* C, const void* A, long a_rows, const int* rows, const void* W, const int* offs, int groups, long M,
                     int N, int K, int act, float limit, hipStream_t s);
+int mx_few_rows_pair(void* Y, void* Y2, long y_stride, const void* X, const void* X2, long x_stride, int rows,
+                     const void* W, const void* W2, int N, int K, hipStream_t s);
+int mx_few_rows_side_gate(void* Y, long y_stride, const void* X, long x_stride, int rows, const void* W, int N, int K,
+                          const void* table, long table_stride, const int* ids, int vocab, hipStream_t s);
 int mx_head_product_fits(int K, int N);
 int mx_latent_q_absorb(float* qa, float* qr, const void* q, int bf16, long stride, const float* wuk, const float* table,
                        int table_rows, int dims, const int* positions, int rows, int heads, int K, int N, int dr,
@@ -1016,6 +1020,33 @@ void few_rows_gemm(Tensor y, Tensor x, Tensor w, OptT bias, int64_t act, double 
                        (int)x.size(1), (int)act, (float)limit, stream()), "few_rows_gemm");
 }
 
+void check_few(const Tensor& y, const Tensor& x, const Tensor& w) {
+  check_rows(x, "x");
+  TORCH_CHECK(x.scalar_type() == at::kBFloat16 && w.is_cuda() && w.scalar_type() == at::kBFloat16 && w.dim() == 2 &&
+              w.is_contiguous() && x.size(1) == w.size(1) && y.is_cuda() && y.is_contiguous() &&
+              y.scalar_type() == at::kBFloat16 && y.dim() == 2 && y.size(0) == x.size(0) && y.size(1) == w.size(0) &&
+              x.size(0) <= mx_few_rows_max(), "few rows: bf16 rows and weights");
+}
+
+// two products of the same sizes and strides in one launch
+void few_rows_pair(Tensor y, Tensor y2, Tensor x, Tensor x2, Tensor w, Tensor w2) {
+  check_few(y, x, w);
+  check_few(y2, x2, w2);
+  TORCH_CHECK(y.sizes() == y2.sizes() && x.sizes() == x2.sizes() && x.stride(0) == x2.stride(0), "few_rows_pair: two alike");
+  chk(mx_few_rows_pair(y.data_ptr(), y2.data_ptr(), y.stride(0), x.data_ptr(), x2.data_ptr(), x.stride(0), (int)x.size(0),
+                       w.data_ptr(), w2.data_ptr(), (int)w.size(0), (int)w.size(1), stream()), "few_rows_pair");
+}
+
+void few_rows_side_gate(Tensor y, Tensor x, Tensor w, Tensor table, Tensor ids, int64_t col0) {
+  check_few(y, x, w);
+  check_i32(ids, "ids");
+  TORCH_CHECK(table.is_cuda() && table.scalar_type() == at::kBFloat16 && table.dim() == 2 && table.stride(1) == 1 &&
+              table.size(0) >= 1 && col0 >= 0 && col0 + w.size(0) <= table.size(1) && ids.numel() >= x.size(0), "side table / ids");
+  chk(mx_few_rows_side_gate(y.data_ptr(), y.stride(0), x.data_ptr(), x.stride(0), (int)x.size(0), w.data_ptr(), (int)w.size(0),
+                            (int)w.size(1), (const char*)table.data_ptr() + 2 * col0, table.stride(0), ids.data_ptr<int>(),
+                            (int)table.size(0), stream()), "few_rows_side_gate");
+}
+
 // without out: the results not yet summed come back, (d [rows * top, width], the shared expert's [rows, width], its gate's
 // logits [rows]), for add_rms_norm_experts and its like
 std::tuple<Tensor, OptT, OptT> experts_few(OptT out, Tensor h, Tensor idx, Tensor wts, Tensor wgu, Tensor wdown, double limit,
@@ -1756,6 +1787,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("moe_topk", &moe_topk);
   m.def("moe_pairs", &moe_pairs);
   m.def("few_rows_gemm", &few_rows_gemm);
+  m.def("few_rows_pair", &few_rows_pair);
+  m.def("few_rows_side_gate", &few_rows_side_gate);
   m.def("expert_rows_fit", [](int64_t width) { return (bool)mx_expert_rows_fit((int)width); });
   m.def("add_rms_norm_experts", &add_rms_norm_experts);
   m.def("layer_norm_experts", &layer_norm_experts);

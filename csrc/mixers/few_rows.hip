@@ -34,15 +34,29 @@ __device__ __forceinline__ void few_rows_sum(const float4* red, int t, int b, in
   }
 }
 
+// What rides in a launch of a plain product, which at decode sizes is 4.6 us by itself: a second product of the same sizes and
+// strides (workgroups of blockIdx.y = 1), or a token-side gate behind the sums, gelu(v) * table[ids[row], column].
+struct FewRowsRider {
+  const bf16_t *X2, *W2;
+  void* Y2;
+  const bf16_t* table;
+  const int* ids;
+  long table_stride;
+  int vocab;
+};
+
 // ---------------------------------------------------------------------------------
 // one workgroup of WV waves per P tiles of 16 output columns (GLU: P tiles of the gate and the
 // same of the up matrix).
 // ---------------------------------------------------------------------------------
-template <int P, bool GLU, int NB, int WV, int U, typename TO>
+template <int P, bool GLU, int NB, int WV, int U, typename TO, bool RIDE>
 __global__ void __launch_bounds__(64 * WV)
 few_rows_gemm_kernel(TO* __restrict__ Y, long y_stride, const bf16_t* __restrict__ X, long x_stride, int rows,
                      const bf16_t* __restrict__ W, const bf16_t* __restrict__ bias, int N, int K, int act, float limit,
-                     int vec) {
+                     int vec, FewRowsRider R) {
+  if constexpr (RIDE) {
+    if (blockIdx.y != 0) X = R.X2, W = R.W2, Y = (TO*)R.Y2;
+  }
   constexpr int NT = GLU ? 2 * P : P;
   extern __shared__ float4 red[];                // few_rows_lds bytes: X stages, then partial sums
   const int tid = threadIdx.x, lane = tid & 63;
@@ -81,6 +95,14 @@ few_rows_gemm_kernel(TO* __restrict__ Y, long y_stride, const bf16_t* __restrict
       if (act == kFrReluSq) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) v[i] = fr_act(act, limit, v[i], 0.f);
+      }
+      if constexpr (RIDE) {
+        if (R.table != nullptr) {
+          const int id = R.ids[r];
+          const bf16_t* g = R.table + (long)(id < 0 || id >= R.vocab ? 0 : id) * R.table_stride + c;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) v[i] = c + i < N ? gelu_tanh_(v[i]) * ft::bf16_to_f32(g[i]) : 0.f;
+        }
       }
       if constexpr (sizeof(TO) == 4) {           // logits: as tanh_cap_kernel, 5 us less than behind the product
         if (act == kFrTanhCap) {
@@ -291,19 +313,20 @@ experts_combine_kernel(float* __restrict__ out, const float* __restrict__ d, con
   out[row * width + c] = v;
 }
 
-template <int P, bool GLU, int NB, int WV, int U, typename TO>
+template <int P, bool GLU, int NB, int WV, int U, typename TO, bool RIDE>
 int few_rows_launch(void* Y, long y_stride, const void* X, long x_stride, int rows, const void* W, const void* bias,
-                    int N, int K, int act, float limit, int vec, hipStream_t s) {
+                    int N, int K, int act, float limit, int vec, const FewRowsRider& R, hipStream_t s) {
   constexpr int NT = GLU ? 2 * P : P;
   constexpr int kRed = WV * NT * NB * 1024, kX = WV * kFrStage<NB, U>, lds = kRed > kX ? kRed : kX;
-  auto kernel = few_rows_gemm_kernel<P, GLU, NB, WV, U, TO>;
+  auto kernel = few_rows_gemm_kernel<P, GLU, NB, WV, U, TO, RIDE>;
   if constexpr (lds > 64 * 1024) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     if (e != hipSuccess) return (int)e;
   }
-  hipLaunchKernelGGL(kernel, dim3((unsigned)((N + 16 * P - 1) / (16 * P))), dim3(64 * WV), lds, s, (TO*)Y, y_stride,
-                     (const bf16_t*)X, x_stride, rows, (const bf16_t*)W, (const bf16_t*)bias, N, K, act, limit, vec);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)((N + 16 * P - 1) / (16 * P)), R.W2 != nullptr ? 2 : 1), dim3(64 * WV), lds, s,
+                     (TO*)Y, y_stride, (const bf16_t*)X, x_stride, rows, (const bf16_t*)W, (const bf16_t*)bias, N, K, act, limit, vec,
+                     R);
   return (int)hipGetLastError();
 }
 
@@ -315,11 +338,11 @@ int few_rows_launch(void* Y, long y_stride, const void* X, long x_stride, int ro
 //   N = 32768: four tiles share an X fragment   26.9 27.7 29.0 34.2  (35.1 33.5 35.2 36.2; 24.0 at 5.6 TB/s)
 //   gated, 2 x 8192: 4 waves                    15.7 15.7 17.5 21.8  (18 + 5 for the activation)
 // Below 1024 columns of X a wave has one step or none: four waves.
-template <bool GLU, int NB, typename TO>
+template <bool GLU, int NB, typename TO, bool RIDE = false>
 int few_rows_pick(void* Y, long y_stride, const void* X, long x_stride, int rows, const void* W, const void* bias,
-                  int N, int K, int act, float limit, int vec, hipStream_t s) {
+                  int N, int K, int act, float limit, int vec, const FewRowsRider& R, hipStream_t s) {
 #define FR_RUN(P, WV, U) \
-  few_rows_launch<P, GLU, NB, WV, U, TO>(Y, y_stride, X, x_stride, rows, W, bias, N, K, act, limit, vec, s)
+  few_rows_launch<P, GLU, NB, WV, U, TO, RIDE>(Y, y_stride, X, x_stride, rows, W, bias, N, K, act, limit, vec, R, s)
   if constexpr (GLU) {
     return FR_RUN(1, 4, NB == 4 ? 2 : 1);
   } else {
@@ -346,13 +369,40 @@ extern "C" int mx_few_rows_gemm(void* Y, int y_f32, long y_stride, const void* X
   const int es = y_f32 ? 4 : 2;
   const int vec = y_stride % 4 == 0 && ((uintptr_t)Y) % (4 * es) == 0;
   const int nb = rows <= 16 ? 1 : rows <= 32 ? 2 : 4;
+  const FewRowsRider R{};
 #define FR_GO(GLU, TO)                                                                                               \
-  (nb == 1   ? few_rows_pick<GLU, 1, TO>(Y, y_stride, X, x_stride, rows, W, bias, N, K, act, limit, vec, s)          \
-   : nb == 2 ? few_rows_pick<GLU, 2, TO>(Y, y_stride, X, x_stride, rows, W, bias, N, K, act, limit, vec, s)          \
-             : few_rows_pick<GLU, 4, TO>(Y, y_stride, X, x_stride, rows, W, bias, N, K, act, limit, vec, s))
+  (nb == 1   ? few_rows_pick<GLU, 1, TO>(Y, y_stride, X, x_stride, rows, W, bias, N, K, act, limit, vec, R, s)       \
+   : nb == 2 ? few_rows_pick<GLU, 2, TO>(Y, y_stride, X, x_stride, rows, W, bias, N, K, act, limit, vec, R, s)       \
+             : few_rows_pick<GLU, 4, TO>(Y, y_stride, X, x_stride, rows, W, bias, N, K, act, limit, vec, R, s))
   if (glu) return FR_GO(true, bf16_t);
   return y_f32 ? FR_GO(false, float) : FR_GO(false, bf16_t);
 #undef FR_GO
+}
+
+// bf16 products with a rider: Y = X W^T and Y2 = X2 W2^T, of the same sizes and strides
+extern "C" int mx_few_rows_pair(void* Y, void* Y2, long y_stride, const void* X, const void* X2, long x_stride, int rows,
+                                const void* W, const void* W2, int N, int K, hipStream_t s) {
+  if (rows <= 0 || N <= 0) return 0;
+  if (rows > kFewRows || K < 8 || K % 8 || x_stride % 8 || W2 == nullptr) return -1;
+  if (((uintptr_t)X | (uintptr_t)X2 | (uintptr_t)W | (uintptr_t)W2) % 16) return -2;
+  const int vec = y_stride % 4 == 0 && ((uintptr_t)Y | (uintptr_t)Y2) % 8 == 0;
+  const FewRowsRider R{(const bf16_t*)X2, (const bf16_t*)W2, Y2, nullptr, nullptr, 0, 0};
+  if (rows <= 16) return few_rows_pick<false, 1, bf16_t, true>(Y, y_stride, X, x_stride, rows, W, nullptr, N, K, kFrStore, 0.f, vec, R, s);
+  if (rows <= 32) return few_rows_pick<false, 2, bf16_t, true>(Y, y_stride, X, x_stride, rows, W, nullptr, N, K, kFrStore, 0.f, vec, R, s);
+  return few_rows_pick<false, 4, bf16_t, true>(Y, y_stride, X, x_stride, rows, W, nullptr, N, K, kFrStore, 0.f, vec, R, s);
+}
+
+// Y = gelu(X W^T) * table[ids[row], 0 .. N), ids outside 0 .. vocab as 0
+extern "C" int mx_few_rows_side_gate(void* Y, long y_stride, const void* X, long x_stride, int rows, const void* W, int N, int K,
+                                     const void* table, long table_stride, const int* ids, int vocab, hipStream_t s) {
+  if (rows <= 0 || N <= 0) return 0;
+  if (rows > kFewRows || K < 8 || K % 8 || x_stride % 8 || table == nullptr || vocab < 1) return -1;
+  if (((uintptr_t)X | (uintptr_t)W) % 16) return -2;
+  const int vec = y_stride % 4 == 0 && ((uintptr_t)Y) % 8 == 0;
+  const FewRowsRider R{nullptr, nullptr, nullptr, (const bf16_t*)table, ids, table_stride, vocab};
+  if (rows <= 16) return few_rows_pick<false, 1, bf16_t, true>(Y, y_stride, X, x_stride, rows, W, nullptr, N, K, kFrStore, 0.f, vec, R, s);
+  if (rows <= 32) return few_rows_pick<false, 2, bf16_t, true>(Y, y_stride, X, x_stride, rows, W, nullptr, N, K, kFrStore, 0.f, vec, R, s);
+  return few_rows_pick<false, 4, bf16_t, true>(Y, y_stride, X, x_stride, rows, W, nullptr, N, K, kFrStore, 0.f, vec, R, s);
 }
 
 extern "C" int mx_experts_few(float* out, void* y, float* d, const void* h, long h_stride, const int* idx,

@@ -39,6 +39,10 @@ __device__ __forceinline__ float sigmoidf_(float x) {
   return x == x ? fmaf(fmaf(-d, q, 1.f), q, q) : x;
 }
 
+__device__ __forceinline__ float gelu_tanh_(float z) {
+  return 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
+}
+
 // softplus with the usual linear branch for large arguments
 __device__ __forceinline__ float softplusf_(float x) { return x > 20.0f ? x : log1pf(expf(x)); }
 

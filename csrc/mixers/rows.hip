@@ -750,9 +750,6 @@ __global__ void clamp_swiglu_kernel(T* __restrict__ out, const T* __restrict__ g
   });
 }
 
-__device__ __forceinline__ float gelu_tanh_(float z) {
-  return 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
-}
 
 // rows [gate (ff) | up (ff)]: out = act(gate) * up, act = gelu_tanh (0), relu (1) or silu (2)
 template <typename T>

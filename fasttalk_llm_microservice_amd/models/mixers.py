@@ -155,16 +155,15 @@ class ChannelDelta:
             raise ValueError("heads must be a multiple of kv_heads")
         self.heads, self.kvh, self.dk, self.dv, self.taps = heads, kv_heads, dim, vdim, taps
         self.eps, self.dtype = eps, dtype
-        self.wqkv = torch.cat([get("q"), get("k"), get("v")], 0).to(device, dtype).contiguous()
-        self.channels = self.wqkv.shape[0]
+        q, k, v, a1, g1, b = (get(n) for n in ("q", "k", "v", "a1", "g1", "b"))
+        self.channels = q.shape[0] + k.shape[0] + v.shape[0]
         self.conv_w = torch.cat([get("q.conv"), get("k.conv"), get("v.conv")], 0) \
             .to(device, torch.float32).contiguous()
         if self.conv_w.shape != (self.channels, taps):
             raise ValueError("convolution weights do not fit the projections")
-        a1, g1, b = get("a1"), get("g1"), get("b")
         self.ra, self.rg = a1.shape[0], g1.shape[0]
-        # the two low-rank down-projections and beta's projection in one product
-        self.wlo = torch.cat([a1, g1, b], 0).to(device, dtype).contiguous()
+        # q, k and v, the two low-rank down-projections and beta's projection
+        self.win = _product_rows([q, k, v, a1, g1, b], dtype, device)
         self.wa2 = get("a2").to(device, dtype).contiguous()
         self.wg2 = get("g2").to(device, dtype).contiguous()
         self.a_log = get("A_log").to(device, torch.float32)
@@ -183,11 +182,14 @@ class ChannelDelta:
 
     def __call__(self, h, ctx: StepContext, state) -> torch.Tensor:
         s_rec, s_conv = state
-        qkv = M.linear(h, self.wqkv)
-        lo = M.linear(h, self.wlo)
-        a = M.linear(lo[:, :self.ra], self.wa2)
-        gp = M.linear(lo[:, self.ra:self.ra + self.rg], self.wg2)
-        b = lo[:, self.ra + self.rg:]
+        c = self.channels
+        if h.shape[0] <= M.FEW_ROWS:      # decode steps: one product, a launch less
+            p = M.linear(h, self.win)
+            qkv, lo = p[:, :c], p[:, c:]
+        else:
+            qkv, lo = M.linear(h, self.win[:c]), M.linear(h, self.win[c:])
+        a, gp = M.linear_pair(lo[:, :self.ra], self.wa2, lo[:, self.ra:self.ra + self.rg], self.wg2)
+        b = lo[:, self.ra + self.rg:self.ra + self.rg + self.heads]
         qkv = M.short_conv_silu(qkv, self.conv_w, s_conv, ctx.seg)
         o = M.gated_delta_rule(qkv, a, b, self.a_log, self.dt_bias, s_rec, ctx.seg, self.heads,
                                self.kvh, self.dk, self.dv)
@@ -938,5 +940,5 @@ class TokenSide:
         self.norm = get("norm").to(device, torch.float32)
 
     def __call__(self, xc, ctx: StepContext) -> torch.Tensor:
-        g = M.side_gate(M.linear(xc, self.gate), self.table, ctx.ids, self.col0, self.dim)
+        g = M.linear_side_gate(xc, self.gate, self.table, ctx.ids, self.col0, self.dim)
         return M.linear(g, self.proj)

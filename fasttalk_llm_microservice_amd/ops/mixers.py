@@ -191,6 +191,27 @@ def linear(x, w, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     return torch.nn.functional.linear(x, w, bias) if y is None else y
 
 
+def linear_pair(x, w, x2, w2):
+    """(:func:`linear` of x and w, of x2 and w2); one launch where the kernel of few rows takes both and they are alike in sizes
+    and strides."""
+    if x.shape == x2.shape and w.shape == w2.shape and x.stride() == x2.stride() and _few_rows(x, w) and _few_rows(x2, w2) \
+            and _few_rows_pays(x.shape[0], w.shape[0], x.shape[1]):
+        y, y2 = (torch.empty(x.shape[0], w.shape[0], dtype=x.dtype, device=x.device) for _ in range(2))
+        native_mixers().few_rows_pair(y, y2, x, x2, w, w2)
+        return y, y2
+    return linear(x, w), linear(x2, w2)
+
+
+def linear_side_gate(x, w, table, ids, col0: int, sd: int):
+    """:func:`side_gate` of x w^T; one launch, the product fp32 up to the gate's result, for few rows."""
+    if _few_rows(x, w) and _few_rows_pays(x.shape[0], w.shape[0], x.shape[1]) and table.dtype == torch.bfloat16 \
+            and table.stride(1) == 1 and ids.dtype == torch.int32:
+        y = torch.empty(x.shape[0], sd, dtype=x.dtype, device=x.device)
+        native_mixers().few_rows_side_gate(y, x, w, table, ids, col0)
+        return y
+    return side_gate(linear(x, w), table, ids, col0, sd)
+
+
 def linear_f32(x, w, cap: float = 0.0) -> torch.Tensor:
     """x w^T with fp32 accumulation and fp32 output, through :func:`tanh_cap_` if there is a ``cap``."""
     if _few_rows(x, w) and _few_rows_pays(x.shape[0], w.shape[0], x.shape[1]):
