@@ -13,10 +13,10 @@ what a token costs in pages.
 
 Each class takes its sizes and constants as constructor arguments and a ``get(name)``
 callable that returns a weight tensor ([out, in] for projections), so a model file only
-describes which sublayers it stacks.  Matrix products of many rows are vendor GEMMs
-(``F.linear`` / ``torch.bmm``) in the compute dtype with fp32 accumulation, those of decode steps
-the few-rows kernels (``ops.mixers.linear``); everything around them runs in the HIP kernels
-(GPU) or their PyTorch twins (CPU backend).
+describes which sublayers it stacks.  Matrix products run in the compute dtype with fp32
+accumulation (``ops.mixers.linear``): those of decode steps in the few-rows kernels, those of many rows
+in the tile kernels or, where those do not pay, the vendor's; everything around them runs in the HIP
+kernels (GPU) or their PyTorch twins (CPU backend).
 """
 from __future__ import annotations
 
