@@ -90,33 +90,22 @@ __device__ __forceinline__ void few_rows_core(fr_f32x4 (&acc)[NT][NB], const bf1
 // what is done to a column's sum(s)
 enum { kFrStore = 0, kFrGelu = 1, kFrRelu = 2, kFrSilu = 3, kFrClamp = 4, kFrReluSq = 5, kFrTanhCap = 6 };
 
-// 1 / (1 + e^-x) in eight instructions, for epilogues that a whole tile waits for (with the library's exp, tanh and division
-// 22 of 131 us of 2048 x 2048 -> 2 x 8192): e^-x = 2^t (1 + r ln 2), t + r = -x log2(e) with r what t's rounding lost.  Results
-// are rounded to bf16 behind it; before that they are within 3.4 units in the last place (mean 0.3 to 0.5) where the library's
-// are within 2.6 (0.25 to 0.5).
-__device__ __forceinline__ float fr_sigmoid(float x) {
-  constexpr float kHi = 1.44269502162933349609375f, kLo = 1.92596299112661746887e-8f, kLn2 = 0.693147182f;
-  const float t = -x * kHi, r = fmaf(-x, kHi, -t) - x * kLo;
-  const float e = __builtin_amdgcn_exp2f(t);
-  // (r of an infinite t is NaN: what it would correct is 0 or infinite)
-  return __builtin_amdgcn_rcpf(1.f + (fabsf(t) < 150.f ? fmaf(e, r * kLn2, e) : e));
-}
-
-// gated forms take the gate's and the up matrix's sums; relu^2 takes one.  0.5 (1 + tanh z) = sigmoid(2 z)
+// gated forms take the gate's and the up matrix's sums; relu^2 takes one.  0.5 (1 + tanh z) = sigmoid(2 z).  One sigmoid for
+// all: with one in each case of a switch tile_gemm.hip's epilogue is too long for the compiler to unroll, its sums lie in
+// memory, and 2048 x 2048 -> 2 x 8192 takes 189 us instead of 113.
 __device__ __forceinline__ float fr_act(int act, float limit, float g, float u) {
-  switch (act) {
-    case kFrGelu: return g * fr_sigmoid(1.5957691216057308f * (g + 0.044715f * g * g * g)) * u;
-    case kFrRelu: return fmaxf(g, 0.f) * u;
-    case kFrSilu: return g * fr_sigmoid(g) * u;
-    case kFrClamp: {
-      const float a = fminf(g, limit), b = fminf(fmaxf(u, -limit), limit);
-      return a * fr_sigmoid(1.702f * a) * (b + 1.0f);
-    }
-    default: {
-      const float r = fmaxf(g, 0.f);
-      return r * r;
-    }
+  if (act == kFrReluSq) {
+    const float r = fmaxf(g, 0.f);
+    return r * r;
   }
+  float a = g, z = g, b = u;
+  if (act == kFrGelu) z = 1.5957691216057308f * (g + 0.044715f * g * g * g);
+  if (act == kFrClamp) {
+    a = fminf(g, limit);
+    z = 1.702f * a;
+    b = fminf(fmaxf(u, -limit), limit) + 1.0f;
+  }
+  return (act == kFrRelu ? fmaxf(g, 0.f) : a * sigmoidf_(z)) * b;
 }
 
 // four neighbouring columns n0 .. n0 + 3 of one output row
