@@ -904,7 +904,7 @@ __global__ __launch_bounds__(kSampThreads) void samp_draw_kernel(
   // kCand; without a nucleus only candidate 0 is drawn, by the whole workgroup
   __shared__ float s_scan[kSampThreads / 64], s_sum[kSlThreads / 64];
   __shared__ float s_M, s_cexp, s_tgt[kCand];
-  __shared__ int s_ps[kCand], s_done, s_last[kCand], s_found[kCand];
+  __shared__ int s_ps[kCand], s_done, s_last[kCand], s_first[kCand];
   __shared__ uint32_t s_ck[kCand];
   const int row = ABOVE ? blockIdx.y : blockIdx.x, part = ABOVE ? blockIdx.x : 0;
   const int tid = threadIdx.x, lane = lane_id();
@@ -1009,7 +1009,7 @@ __global__ __launch_bounds__(kSampThreads) void samp_draw_kernel(
   }
   if (tid < kCand) {
     s_last[tid] = -1;
-    s_found[tid] = 0;
+    s_first[tid] = kSampThreads;
   }
   __syncthreads();
   if (s_done) return;
@@ -1050,7 +1050,12 @@ __global__ __launch_bounds__(kSampThreads) void samp_draw_kernel(
   const float excl = wbase + incl - mass;
   const bool mine = mass > 0.f &&
                     ((tgt >= excl && tgt < excl + mass) || (lt == s_last[r] && tgt >= excl + mass));
-  if (mine) {
+  // the ranges are fp32 sums and may overlap by a unit in the last place, across waves: the lowest thread's id is the
+  // candidate (the first to finish may be another one in every workgroup that draws the row, and with ABOVE their masses
+  // are added up)
+  if (mine) atomicMin(&s_first[r], lt);
+  __syncthreads();
+  if (mine && lt == s_first[r]) {
     float a = excl;
     int pick = -1, lastk = -1;
     uint32_t pk = 0u, lastkey = 0u;
@@ -1079,7 +1084,7 @@ __global__ __launch_bounds__(kSampThreads) void samp_draw_kernel(
       pick = lastk;
       pk = lastkey;
     }
-    if (pick >= 0 && atomicCAS(&s_found[r], 0, 1) == 0) {
+    if (pick >= 0) {
       s_ck[r] = pk;
       if (writes) {
         wr[kWsCand + 2 * r] = __uint_as_float(pk);
