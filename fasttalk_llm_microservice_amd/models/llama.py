@@ -155,14 +155,15 @@ MAX_SPLITS = 4
 # gate_up 54.8 vs 67.8 us at 145 rows, 81.4 vs 102.4 at 300, 88.2 vs 105.3 at 384;
 # down 36.2 vs 43.7 / 54.3 vs 63.8 / 57.5 vs 66.3; LM head 233 vs 263 / 376 vs 463.
 # Above 384 rows: cfg 3, 256x256 in phases, with as many splits as leave one round of
-# workgroups (us, the tile it replaces beside it): qkv 50 vs 57 at 768 rows and 57 vs 65
-# at 1280 (2 splits), 78 vs 99 at 1536, 170 vs 218 at 4096; o 53 vs 66 at 1280 (2), 85 vs
-# 105 at 3000; gate_up 98 vs 122 at 512, 280 vs 329 at 1536; down 82 vs 95 at 640 (4),
+# workgroups (us, the tile it replaces beside it): qkv 50 vs 57 at 768 rows, 56 vs 69 at
+# 1280 and 97 vs 108 at 1536 (2 splits below 2048 rows: the sums reach the rotation in
+# fp32; one split takes 75 at 1536, but rounds them to bf16 first), 170 vs 218 at 4096; o
+# 53 vs 66 at 1280 (2), 85 vs 105 at 3000; gate_up 98 vs 122 at 512, 280 vs 329 at 1536; down 82 vs 95 at 640 (4),
 # 140 vs 192 at 1280 (2), 286 vs 363 at 3000; LM head 429 vs 523 at 512, 1579 vs 1830 at
 # 2048.  (o at 513-1024 rows keeps two splits: four take 34 vs 40 us but leave the
 # residual-add kernel twice the slabs.)
 PG_PLAN = {
-    "qkv": ((128, 1, 8), (192, 6, 4), (256, 2, 4), (384, 6, 2), (512, 2, 2), (1280, 3, 2),
+    "qkv": ((128, 1, 8), (192, 6, 4), (256, 2, 4), (384, 6, 2), (512, 2, 2), (2047, 3, 2),
             (1 << 30, 3, 1)),
     "o": ((128, 2, 8), (192, 6, 8), (256, 1, 8), (384, 6, 4), (512, 2, 4), (1024, 1, 2),
           (2047, 3, 2), (1 << 30, 3, 1)),

@@ -177,3 +177,9 @@ def test_w4_plan_uses_mh_above_48_rows():
     assert llama.w4_cfg("o", 50, 8192, 8192) == (4, 2, 0)
     assert llama.w4_cfg("qkv", 50, 6144, 4096) == (2, 4, 4)
     assert llama.w4_cfg("down", 50, 8192, 28672) == llama.W4_PLAN["down"][64]
+
+
+@pytest.mark.parametrize("proj,k", [("qkv", 4096), ("o", 4096), ("down", 14336)])
+def test_sums_below_2048_rows_stay_fp32(proj, k):
+    """Two splits or more leave fp32 slabs that the rotation or the residual add sums; one rounds to bf16 in front of it."""
+    assert all(llama.pg_cfg(proj, rows, k)[1] > 1 for rows in range(65, 2048))
