@@ -19,7 +19,7 @@
 // instructions (the score times log2(e) in one fused step, masks only on tiles that need them, loads
 // without branches; 1150 before that, which took three times the products' time).  16 heads of 128 on 4
 // key heads, us, before -> now: 2048 rows causal 115 -> 70, 4096 334 -> 206 (0.5 PFLOP/s of bf16 products),
-// 777 37 -> 28, with a distance table 50 -> 29, with sigmoids of 2048 157 -> 79, five prompts of 258 to 542
+// 777 37 -> 28, with a distance table 51 -> 32, with sigmoids of 2048 157 -> 79, five prompts of 258 to 542
 // with a cap 51 -> 39; two fp32 products through memory with a weights kernel between them, gathers
 // and layout changes around them, take 140 to 500 us and 25 launches per segment.
 #include "mx_common.h"
@@ -54,6 +54,15 @@ struct BandArgs {
 __device__ __forceinline__ ba_f32x4 ba_mfma(const uint4& a, const uint4& b, ba_f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(ba_bf16x8, a), __builtin_bit_cast(ba_bf16x8, b), c,
                                                  0, 0, 0);
+}
+
+// e^x for x <= 0, the argument's rounding in base 2 made good; 0 far below; NaN stays NaN
+__device__ __forceinline__ float ba_exp(float x) {
+  x = x < -150.f ? -150.f : x;
+  const float t = x * 1.44269502f;
+  const float r = fmaf(x, 1.44269502f, -t) + x * 1.92596303e-8f;
+  const float e = __builtin_amdgcn_exp2f(t);
+  return fmaf(e, r * 0.693147181f, e);
 }
 
 // 1 / (1 + e^-x): the argument's rounding in base 2 and the reciprocal's made good.  (sigmoidf_ reduces the argument first, for
@@ -129,11 +138,14 @@ band_attn_kernel(BandArgs A) {
   const float pbias = A.pb != nullptr ? A.pb[a] : 0.f;
   const float cap = A.softcap, icap = cap > 0.f ? (KIND == kBandCap ? A.scale / cap : 1.f / cap) : 0.f;
   const float sink = A.sinks != nullptr ? A.sinks[a] : A.sink_all;
-  // a score is v vmul in base 2 with v what the score terms leave (products, tanh, or the score itself)
+  // Without terms a score is v vmul in base 2, v the product or tanh.  With terms it stays as it is: a bias may be the type's
+  // lowest value, which has no multiple, and log2(e) rounded once for all would be a larger error than ba_exp's.
+  constexpr bool kTwo = KIND == kBandPlain || KIND == kBandCap;
   constexpr float kLog2e = 1.44269502f;
-  const float vmul = KIND == kBandPlain ? A.scale2 : KIND == kBandCap ? cap * kLog2e : kLog2e;
+  const float vmul = KIND == kBandPlain ? A.scale2 : KIND == kBandCap ? cap * kLog2e : 1.f;
+  auto weight = [](float x) { return kTwo ? __builtin_amdgcn_exp2f(x) : ba_exp(x); };
   const bool sinks = A.has_sink && grp == 0;
-  float mx_ = sinks ? sink * kLog2e : -INFINITY, l_ = sinks && g4 == 0 ? 1.f : 0.f;
+  float mx_ = sinks ? (kTwo ? sink * kLog2e : sink) : -INFINITY, l_ = sinks && g4 == 0 ? 1.f : 0.f;
   ba_f32x4 o[DT];
 #pragma unroll
   for (int t = 0; t < DT; ++t) o[t] = ba_f32x4{0.f, 0.f, 0.f, 0.f};
@@ -262,7 +274,7 @@ band_attn_kernel(BandArgs A) {
           for (int e = 1; e < 16; ++e) tmax = fmaxf(tmax, sc[e >> 2][e & 3]);
           tmax = ft::kgroups_max(tmax) * vmul;
           if (__ballot(tmax > mx_)) {                          // (rare once the first tiles have been seen)
-            const float nm = fmaxf(mx_, tmax), f = mx_ == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mx_ - nm);
+            const float nm = fmaxf(mx_, tmax), f = mx_ == -INFINITY ? 0.f : weight(mx_ - nm);
             l_ *= f;
 #pragma unroll
             for (int t = 0; t < DT; ++t)
@@ -285,7 +297,7 @@ band_attn_kernel(BandArgs A) {
           for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-              sc[kt][v] = __builtin_amdgcn_exp2f(fmaf(sc[kt][v], vmul, -mu));
+              sc[kt][v] = weight(kTwo ? fmaf(sc[kt][v], vmul, -mu) : sc[kt][v] - mu);
               l_ += sc[kt][v];
             }
         }
@@ -330,7 +342,7 @@ band_attn_kernel(BandArgs A) {
     if (grp != 0) return;
     if (!sigmoid) {
       const float m2 = ml[tid], l2 = ml[256 + tid], nm = fmaxf(mx_, m2), mu = nm == -INFINITY ? 0.f : nm;
-      f = __builtin_amdgcn_exp2f(mx_ - mu), f2 = __builtin_amdgcn_exp2f(m2 - mu);
+      f = weight(mx_ - mu), f2 = weight(m2 - mu);
       l_ = l_ * f + l2 * f2;
     }
   }

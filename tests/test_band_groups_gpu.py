@@ -7,6 +7,7 @@ from fasttalk_llm_microservice_amd.ops import mixers as M
 from test_band_attention_gpu import DEV, cases, reference, segments
 
 pytestmark = pytest.mark.gpu
+LOW = torch.finfo(torch.float32).min
 
 
 @pytest.mark.parametrize("name,sizes,opt,lens,pos0", [c for c in cases() if c[0] in (
@@ -57,3 +58,39 @@ def test_rule(rows, count, pos, window, groups):
     start = [i * rows for i in range(count + 1)]
     seg = M.Segments(None, None, None, None, None, count, rows, pos + rows, host=(start, [pos] * count, [pos + rows] * count))
     assert M._band_groups(seg, M.WindowSpec(heads=16, kv_heads=4, dk=128, dv=128, window=window, scale=1.0), 32) == groups
+
+
+@pytest.mark.parametrize("groups", [1, 2])
+@pytest.mark.parametrize("opt", [{}, dict(softcap=5.0), dict(sink=LOW), dict(terms=True)], ids=str)
+def test_lowest_biases(groups, opt, monkeypatch):
+    """A distance table that masks with the type's lowest value: rows that see masked keys only weigh them all alike, others
+    not at all."""
+    opt = dict(opt)
+    g = torch.Generator().manual_seed(2)
+    if opt.pop("terms", False):
+        opt.update({k: torch.rand(4, generator=g).to(DEV) for k in ("r1", "r2")})
+    table = torch.full((300, 4), LOW, device=DEV)
+    table[:, 1] = 0.25                        # a head that sees all
+    table[3:, 2] = 0.5                        # one that does from a distance of 3 on: the first three rows see masked keys only
+    table[:3, 3] = -0.5                       # one that sees no further: its first tiles are masked
+    sp = M.WindowSpec(heads=4, kv_heads=2, dk=64, dv=64, window=0, scale=0.125, dist_bias=table, **opt)
+    seg, blocks = segments([150, 70], [0, 0], 16, g)
+    kc, vc = (torch.randn(blocks, 16, 128, generator=g).to(DEV, torch.bfloat16) for _ in range(2))
+    q = torch.randn(220, 4, 64, generator=g).to(DEV)
+    want = reference(q.view(220, 256), kc, vc, seg, sp, 32)
+    alike = torch.zeros(220, 4, dtype=torch.bool, device=DEV)          # (64 bits tell such scores apart: their mean instead)
+    alike[:, 0] = True
+    alike[:3, 2] = alike[150:153, 2] = True
+    for s, (a, b) in enumerate(((0, 150), (150, 220))):
+        v = vc[seg.block_tables[s].long()].reshape(-1, 2, 64).double()
+        mean = v.cumsum(0)[:b - a] / torch.arange(1, b - a + 1, device=DEV)[:, None, None]
+        mean = mean.repeat_interleave(2, 1)
+        want[a:b][alike[a:b]] = mean[alike[a:b]]
+    if "sink" in opt:                        # the sink is as low: one more that weighs the same
+        n = torch.cat([torch.arange(1, 151), torch.arange(1, 71)]).to(DEV)[:, None, None].double()
+        want = torch.where(alike[:, :, None], want * n / (n + 1), want)
+    monkeypatch.setattr(M, "_band_pays", lambda *a: True)
+    monkeypatch.setattr(M, "_band_groups", lambda *a: groups)
+    got = M.window_attention_products(torch.zeros(220, 4, 64, device=DEV), q.view(220, 256), kc, vc, seg, sp, 32)
+    # fp32 sums of a few hundred terms: about 2^-22
+    assert float((got.double() - want).norm() / want.norm()) < 1e-6
