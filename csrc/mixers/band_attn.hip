@@ -19,7 +19,7 @@
 // instructions (the score times log2(e) in one fused step, masks only on tiles that need them, loads
 // without branches; 1150 before that, which took three times the products' time).  16 heads of 128 on 4
 // key heads, us, before -> now: 2048 rows causal 115 -> 70, 4096 334 -> 206 (0.5 PFLOP/s of bf16 products),
-// 777 37 -> 28, with a distance table 51 -> 32, with sigmoids of 2048 157 -> 79, five prompts of 258 to 542
+// 777 37 -> 28, with a distance table 51 -> 32, with sigmoids of 2048 159 -> 83, five prompts of 258 to 542
 // with a cap 51 -> 39; two fp32 products through memory with a weights kernel between them, gathers
 // and layout changes around them, take 140 to 500 us and 25 launches per segment.
 #include "mx_common.h"
@@ -63,17 +63,6 @@ __device__ __forceinline__ float ba_exp(float x) {
   const float r = fmaf(x, 1.44269502f, -t) + x * 1.92596303e-8f;
   const float e = __builtin_amdgcn_exp2f(t);
   return fmaf(e, r * 0.693147181f, e);
-}
-
-// 1 / (1 + e^-x): the argument's rounding in base 2 and the reciprocal's made good.  (sigmoidf_ reduces the argument first, for
-// 0.03 of a unit in the last place on average, far below the score's own error, and 5 us of 72.)
-__device__ __forceinline__ float ba_sigmoid(float x) {
-  const float c = fminf(fmaxf(x, -88.f), 88.f);            // (e^88 is finite; NaN: below)
-  const float t = c * -1.44269502f;
-  const float r = fmaf(c, -1.44269502f, -t) - c * 1.92596303e-8f;
-  const float e = __builtin_amdgcn_exp2f(t), d = 1.f + fmaf(e, r * 0.693147181f, e);
-  const float q = __builtin_amdgcn_rcpf(d);
-  return x == x ? fmaf(fmaf(-d, q, 1.f), q, q) : x;
 }
 
 // the score terms a kernel is built for (run-time tests per score cost as much as the products: a
@@ -134,7 +123,7 @@ band_attn_kernel(BandArgs A) {
     return q < head_tiles ? q : band0 + q - head_tiles;
   };
 
-  const float c1 = use_terms ? A.r1[a] * 0.693147181f : 0.f, c2 = use_terms ? A.r2[a] : 0.f;
+  const float c1 = use_terms ? A.r1[a] : 0.f, c2 = use_terms ? A.r2[a] : 0.f;
   const float pbias = A.pb != nullptr ? A.pb[a] : 0.f;
   const float cap = A.softcap, icap = cap > 0.f ? (KIND == kBandCap ? A.scale / cap : 1.f / cap) : 0.f;
   const float sink = A.sinks != nullptr ? A.sinks[a] : A.sink_all;
@@ -213,9 +202,9 @@ band_attn_kernel(BandArgs A) {
         if constexpr (kAny) {
           if (use_cap) z = cap * tanh_(z * icap);
         }
-        if (use_terms) z -= c1 * __builtin_amdgcn_logf(1.0f + c2 * (float)max(d, 0));
+        if (use_terms) z -= c1 * logf(1.0f + c2 * (float)max(d, 0));
         if (use_dist) z += A.dist_bias[min(max(d, 0), A.nd - 1) * hq + a];
-        if (sigmoid) z = ba_sigmoid(z + pbias);
+        if (sigmoid) z = sigmoidf_(z + pbias);
         sc[kt][v] = z;
       }
     if (whole) return;

@@ -94,3 +94,22 @@ def test_lowest_biases(groups, opt, monkeypatch):
     got = M.window_attention_products(torch.zeros(220, 4, 64, device=DEV), q.view(220, 256), kc, vc, seg, sp, 32)
     # fp32 sums of a few hundred terms: about 2^-22
     assert float((got.double() - want).norm() / want.norm()) < 1e-6
+
+
+@pytest.mark.parametrize("lens,pos0", [([300], [0]), ([64], [3000])])
+@pytest.mark.parametrize("groups", [1, 2])
+def test_distance_terms_are_as_exact_as_the_products(lens, pos0, groups, monkeypatch):
+    """Scores that are mostly logarithms of the distance: no further from 64 bits than the fp32 products with the library's."""
+    g = torch.Generator().manual_seed(5)
+    r1, r2 = (0.5 + torch.rand(4, generator=g)).to(DEV), (0.5 + torch.rand(4, generator=g)).to(DEV)
+    sp = M.WindowSpec(heads=4, kv_heads=1, dk=128, dv=128, window=0, scale=128 ** -0.5, r1=r1, r2=r2)
+    seg, blocks = segments(lens, pos0, 16, g)
+    kc, vc = (torch.randn(blocks, 16, 128, generator=g).to(DEV, torch.bfloat16) for _ in range(2))
+    q = (0.05 * torch.randn(sum(lens), 512, generator=g)).to(DEV)
+    want = reference(q, kc, vc, seg, sp, 1)
+    monkeypatch.setattr(M, "_band_pays", lambda *a: True)
+    monkeypatch.setattr(M, "_band_groups", lambda *a: groups)
+    new, old = (M.window_attention_products(torch.zeros(sum(lens), 4, 128, device=DEV), q, k, v, seg, sp, 1)
+                for k, v in ((kc, vc), (kc.float(), vc.float())))
+    e_new, e_old = (float((x.double() - want).norm() / want.norm()) for x in (new, old))
+    assert e_new < 1.05 * e_old, (e_new, e_old)
