@@ -331,7 +331,7 @@ band_attn_kernel(BandArgs A) {
     if (grp != 0) return;
     if (!sigmoid) {
       const float m2 = ml[tid], l2 = ml[256 + tid], nm = fmaxf(mx_, m2), mu = nm == -INFINITY ? 0.f : nm;
-      f = weight(mx_ - mu), f2 = weight(m2 - mu);
+      f = mx_ == mu ? 1.f : weight(mx_ - mu), f2 = m2 == mu ? 1.f : weight(m2 - mu);     // (a sink may be infinite)
       l_ = l_ * f + l2 * f2;
     }
   }

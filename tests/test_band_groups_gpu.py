@@ -113,3 +113,24 @@ def test_distance_terms_are_as_exact_as_the_products(lens, pos0, groups, monkeyp
                 for k, v in ((kc, vc), (kc.float(), vc.float())))
     e_new, e_old = (float((x.double() - want).norm() / want.norm()) for x in (new, old))
     assert e_new < 1.05 * e_old, (e_new, e_old)
+
+
+@pytest.mark.parametrize("groups", [1, 2])
+@pytest.mark.parametrize("opt", [{}, dict(softcap=5.0), dict(table=True)], ids=str)
+@pytest.mark.parametrize("sink", [float("inf"), torch.finfo(torch.float32).max, LOW, -float("inf")])
+def test_extreme_sinks(groups, opt, sink, monkeypatch):
+    """A sink far above all scores takes all of the weight, one far below none."""
+    g = torch.Generator().manual_seed(6)
+    extra = dict(dist_bias=torch.randn(40, 4, generator=g).to(DEV)) if opt.get("table") else opt
+    sp = M.WindowSpec(heads=4, kv_heads=2, dk=64, dv=64, window=0, scale=0.125, sink=sink, **extra)
+    seg, blocks = segments([150, 70], [0, 9], 16, g)
+    kc, vc = (torch.randn(blocks, 16, 128, generator=g).to(DEV, torch.bfloat16) for _ in range(2))
+    q = torch.randn(220, 256, generator=g).to(DEV)
+    monkeypatch.setattr(M, "_band_pays", lambda *a: True)
+    monkeypatch.setattr(M, "_band_groups", lambda *a: groups)
+    got = M.window_attention_products(torch.full((220, 4, 64), 7.0, device=DEV), q, kc, vc, seg, sp, 32)
+    if sink > 0:
+        assert bool((got == 0).all())
+    else:
+        want = reference(q, kc, vc, seg, M.WindowSpec(heads=4, kv_heads=2, dk=64, dv=64, window=0, scale=0.125, **extra), 32)
+        assert float((got.double() - want).norm() / want.norm()) < 1e-6       # fp32 sums of a few hundred terms: about 2^-22
