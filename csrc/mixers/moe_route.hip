@@ -264,7 +264,11 @@ struct RouteRows {
   const float *router, *bias;
   int experts, width, top, mode, groups, keep;
   float eps, scale;
+  int in_turn;                               // rows with logits that are no finite numbers: experts by choose_in_turn
 };
+// Which experts such a row names does not hang on the kernel that its step takes: up to 64 rows those of the routers above, beyond
+// those of the router for sixteen rows a workgroup where that serves (widths of whole 2048)
+static bool route_in_turn(long rows, int width) { return rows <= 64 || width % 2048 != 0; }
 
 template <int NORM, int C, typename TY>
 __global__ void __launch_bounds__(64 * kRouteWaves)
@@ -417,7 +421,9 @@ route_rows_kernel(RouteRows R) {
   const float z = lane < R.experts ? z_s[lane] + (biased ? bias : 0.f) : 0.f;
   if (lane < R.experts) z_s[lane] = z;       // (for the choice in turn)
   wave_lds_fence();
-  if (__any(z != z))                         // (which experts a row with a NaN names is the sequential choice's matter)
+  // (ties and NaN have another order there)
+  const bool odd = !(fabsf(z) < INFINITY) || (R.mode == kRouteSoftmaxAll && !(fabsf(R.bias[min(lane, R.experts - 1)]) < INFINITY));
+  if (R.in_turn && __any(odd))
     choose_in_turn(R.idx + row * R.top, R.wts + row * R.top, z_s, row_s, R.bias, R.experts, R.top, R.mode, R.scale, R.groups,
                    R.keep, lane);
   else
@@ -525,7 +531,7 @@ extern "C" int mx_norm_route(int* idx, float* wts, void* h, float* x, const void
   if (((uintptr_t)h | (uintptr_t)x | (uintptr_t)wb | (uintptr_t)w | (uintptr_t)b | (uintptr_t)router) % 16 || ((uintptr_t)y) % (y_bf16 ? 8 : 16))
     return -2;
   const mx::RouteRows R{idx, wts, (mx::bf16_t*)h, width, x, y, y_stride, wb, w, b, router, bias, experts, width,
-                        top, mode, groups, keep, eps, scale};
+                        top, mode, groups, keep, eps, scale, mx::route_in_turn(rows, width)};
 #define MX_NR(NORM, C)                                                                                                     \
   MX_DISPATCH_T(y_bf16, hipLaunchKernelGGL((mx::route_rows_kernel<NORM, C, T>), dim3((unsigned)rows), dim3(64 * mx::kRouteWaves), \
                                            width * 4, s, R))
@@ -555,7 +561,8 @@ extern "C" int mx_moe_route_few(int* idx, float* wts, const void* h, int bf16, l
                   ((uintptr_t)router) % 16 == 0;
   if (bf16 && vec && mx::route_rows_fit(width, experts)) {
     const mx::RouteRows R{idx, wts, (mx::bf16_t*)const_cast<void*>(h), h_stride, nullptr, nullptr, 0, nullptr, nullptr, nullptr,
-                          router, bias, experts, width, top, mode, groups, keep, 0.f, scale};
+                          router, bias, experts, width, top, mode, groups, keep, 0.f, scale,
+                          mx::route_in_turn(rows, width)};
     if (width <= 4096)
       hipLaunchKernelGGL((mx::route_rows_kernel<0, 1, mx::bf16_t>), dim3((unsigned)rows), dim3(64 * mx::kRouteWaves), width * 4, s, R);
     else
