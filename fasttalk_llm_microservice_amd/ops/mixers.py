@@ -130,13 +130,16 @@ def _tile_gemm_pays(rows: int, n: int, k: int, act: Optional[str] = None) -> boo
 
 
 def _tile_gemm(x, w, bias, act: Optional[str] = None, limit: float = 0.0):
-    """The product where :func:`_tile_gemm_pays`, else None."""
-    if x.dim() != 2 or x.shape[0] <= FEW_ROWS or not _piece_rows(x, w) \
+    """The product where :func:`_tile_gemm_pays`, else None: also where rows overlap, w is one row or a gated form's two matrices
+    and one row more, or the bias is broadcast."""
+    if x.dim() != 2 or w.dim() != 2 or x.shape[0] <= FEW_ROWS or not _piece_rows(x, w) or x.stride(0) < x.shape[1] \
             or x.stride(0) * x.shape[0] * 2 > 0xffffffff or not _tile_gemm_pays(x.shape[0], w.shape[0], x.shape[1], act) \
-            or (bias is not None and not (bias.dtype == torch.bfloat16 and bias.is_contiguous())):
+            or (bias is not None and not (bias.dtype == torch.bfloat16 and bias.is_contiguous() and bias.shape == w.shape[:1])):
         return None
-    n = w.shape[0] if act is None or act == "relu_sq" else w.shape[0] // 2
-    y = torch.empty(x.shape[0], n, dtype=x.dtype, device=x.device)
+    glu = act is not None and act != "relu_sq"
+    if glu and w.shape[0] % 2:
+        return None
+    y = torch.empty(x.shape[0], w.shape[0] // 2 if glu else w.shape[0], dtype=x.dtype, device=x.device)
     native_mixers().tile_gemm(y, x, w, bias, FEW_ACTS[act], float(limit), -1)
     return y
 
