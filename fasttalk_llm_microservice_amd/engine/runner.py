@@ -23,6 +23,7 @@ from .. import ops
 from ..models.config import ModelConfig
 from ..models.llama import AttnMeta
 from ..models.registry import build_model
+from ..ops.mixers import replayed_step
 from ..parallel.comm import SINGLE, TPComm
 from ..runtime import rt
 from .config import EngineConfig
@@ -1294,13 +1295,13 @@ class ModelRunner:
 
         s = torch.cuda.Stream(self.device)
         s.wait_stream(torch.cuda.current_stream(self.device))
-        with torch.cuda.stream(s):
+        with torch.cuda.stream(s), replayed_step():
             samp(fwd())  # warm-up (allocator, lazy init)
         torch.cuda.current_stream(self.device).wait_stream(s)
         if self.graph_pool is None:
             self.graph_pool = torch.cuda.graph_pool_handle()
         gf = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(gf, pool=self.graph_pool):
+        with torch.cuda.graph(gf, pool=self.graph_pool), replayed_step():
             lg = fwd()
         self._fwd_logits[nb] = lg
         gs = torch.cuda.CUDAGraph()
@@ -1330,13 +1331,13 @@ class ModelRunner:
         self.d_sslots[:nb].fill_(-1)
         s = torch.cuda.Stream(self.device)
         s.wait_stream(torch.cuda.current_stream(self.device))
-        with torch.cuda.stream(s), self._long_waits():
+        with torch.cuda.stream(s), self._long_waits(), replayed_step():
             self._graph_body(nb)  # warm-up (allocator, lazy init)
         torch.cuda.current_stream(self.device).wait_stream(s)
         if self.graph_pool is None:
             self.graph_pool = torch.cuda.graph_pool_handle()
         g = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(g, pool=self.graph_pool):
+        with torch.cuda.graph(g, pool=self.graph_pool), replayed_step():
             self._graph_body(nb, keep=True)
         self.d_slots[:nb].copy_(saved[0])
         self.d_seq_lens[:nb].copy_(saved[1])

@@ -20,6 +20,7 @@ a longer one), with the position of its first row, its state slot and its block 
 """
 from __future__ import annotations
 
+import contextlib
 import dataclasses
 import functools
 import importlib
@@ -129,6 +130,29 @@ def _tile_gemm_pays(rows: int, n: int, k: int, act: Optional[str] = None) -> boo
     return native_mixers().tile_gemm_us(rows, out, k, glu) <= spare + 2.0 * rows * n * k / (1.3e9 if rows <= 1024 else 1.35e9)
 
 
+_replayed = threading.local()
+
+
+@contextlib.contextmanager
+def replayed_step():
+    """What this thread issues inside is captured, or warms up what is: no call of its replays costs the host anything."""
+    before = getattr(_replayed, "on", False)
+    _replayed.on = True
+    try:
+        yield
+    finally:
+        _replayed.on = before
+
+
+def _tile_gemm_behind(n: int, k: int, act: Optional[str]) -> bool:
+    """Where :func:`_tile_gemm_pays` lets the tiles be behind the vendor's product for its host time: few columns, and long
+    sums of few tiles.  A :func:`replayed_step` has none to save and leaves these to the vendor's.  us in a graph at 65 / 128 /
+    256 rows, the vendor's beside it: n = 256, k = 2048 6.5 6.5 6.5 (5.6 8.2 8.3); 64 6.2 6.4 6.5 (5.8 5.9 5.7); 2048, 8192 19.8
+    24.7 24.0 (19.9 20.5 26.1); 14336, 4096 32.7 34.8 43.4 (29.4 32.5 50.0); kept: 2048, 2048 7.2 7.5 7.6 (8.8 8.8 9.8); 1024, 1024
+    5.2 5.3 5.2 (5.6 5.6 8.3); 8192, 2048 12.0 13.4 17.2 (13.5 15.5 24.6); gated, 2 x 8192, k = 2048 20.9 21.0 26.2 (22.5 24.6 34.1)."""
+    return act is None and (n < 1024 or k >= 4096)
+
+
 def _tile_gemm(x, w, bias, act: Optional[str] = None, limit: float = 0.0):
     """The product where :func:`_tile_gemm_pays`, else None: also where rows overlap, w is one row or a gated form's two matrices
     and one row more, or the bias is broadcast."""
@@ -137,7 +161,7 @@ def _tile_gemm(x, w, bias, act: Optional[str] = None, limit: float = 0.0):
             or (bias is not None and not (bias.dtype == torch.bfloat16 and bias.is_contiguous() and bias.shape == w.shape[:1])):
         return None
     glu = act is not None and act != "relu_sq"
-    if glu and w.shape[0] % 2:
+    if (glu and w.shape[0] % 2) or (getattr(_replayed, "on", False) and _tile_gemm_behind(*w.shape, act)):
         return None
     y = torch.empty(x.shape[0], w.shape[0] // 2 if glu else w.shape[0], dtype=x.dtype, device=x.device)
     native_mixers().tile_gemm(y, x, w, bias, FEW_ACTS[act], float(limit), -1)
