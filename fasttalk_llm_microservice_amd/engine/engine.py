@@ -854,7 +854,8 @@ class LLMEngine:
             self._executing = batch
             logits = self.runner.execute(batch, None, logits_only=True)
             self._executing = None
-            logits = logits if inverse is None else logits[inverse]
+            # (on the CPU a view of rows that are padded)
+            logits = np.ascontiguousarray(logits) if inverse is None else logits[inverse]
             sched.post_step(batch)
             self.stats["given_steps"] += 1
         for rid in end:

@@ -75,6 +75,15 @@ def test_state_slots_gate_admission(tmp_path):
     assert eng.scheduler.slots.num_free() == 2 and eng.bm.num_free() == 8
 
 
+def test_replayed_logits_are_dense(tmp_path):
+    """Rows of the vocabulary's width, one after the other, whatever order is wanted (the model's own are padded)."""
+    d, cfg, _ = C.make_model("b", 3, tmp_path)
+    eng = C.make_engine(d, "cpu", seqs=2, pages=8)
+    for i, want in enumerate(([3], [0, 2, 3], [3, 0], [1, 1])):
+        lg = eng.replay_step([(f"r{i}", C.tokens(4, cfg["vocab"], 1), want)], end=[f"r{i}"])
+        assert lg.shape == (len(want), cfg["vocab"]) and lg.flags.c_contiguous and lg.dtype.name == "float32"
+
+
 def test_replay_order_and_idle_steps(tmp_path):
     """Wanted rows come back in the caller's order whatever the step's row order is; a
     request may sit out a step; an entry without tokens and a step without entries run
