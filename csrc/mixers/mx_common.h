@@ -20,10 +20,11 @@ __device__ __forceinline__ float ld(const bf16_t* p, long i) { return ft::bf16_t
 __device__ __forceinline__ void st(float* p, long i, float v) { p[i] = v; }
 __device__ __forceinline__ void st(bf16_t* p, long i, float v) { p[i] = ft::f32_to_bf16(v); }
 
-// 1 / (1 + e^-x), as exact as the library's exponential and division (2.6 units in the last place at most, 0.43 on average in
-// -8 .. 8, the same in both) in half their instructions
+// 1 / (1 + e^-x), as exact as the library's exponential and division (2.7 units in the last place at most, 0.45 on average in
+// -8 .. 8, the same in both) in half their instructions.  The denominator is formed 2^-24 times as large: e^104 has a
+// reciprocal, so results are right down to the smallest numbers, and 0 below.
 __device__ __forceinline__ float sigmoidf_(float x) {
-  const float c = fminf(fmaxf(x, -88.f), 88.f);                  // (e^88 is finite; NaN: below)
+  const float c = fminf(fmaxf(x, -104.f), 88.f);                 // (NaN: below)
   float t, f;                                                    // e^-x = 2^(t + r), r what t's rounding lost
   {
 #pragma clang fp contract(off)
@@ -34,9 +35,9 @@ __device__ __forceinline__ float sigmoidf_(float x) {
 #pragma clang fp contract(off)
     f = t - n;
   }
-  const float d = 1.f + __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(f + r), (int)n);
+  const float d = 0x1p-24f + __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(f + r), (int)n - 24);
   const float q = __builtin_amdgcn_rcpf(d);
-  return x == x ? fmaf(fmaf(-d, q, 1.f), q, q) : x;
+  return x == x ? 0x1p-24f * fmaf(fmaf(-d, q, 1.f), q, q) : x;
 }
 
 __device__ __forceinline__ float gelu_tanh_(float z) {

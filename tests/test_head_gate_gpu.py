@@ -27,3 +27,15 @@ def test_head_rms_gate(rows, heads, dv, dt, off):
         # fp32 sums of up to 256 terms and a few roundings; bf16: one rounding of the result
         torch.testing.assert_close(got.double()[fin], want.view(rows, -1)[fin], rtol=2 ** -8 if dt == torch.bfloat16 else 2e-6, atol=1e-30)
         assert bool(torch.isinf(got[~fin]).all())
+
+
+def test_sigmoid_in_its_tail():
+    """z sigmoid(z) in fp32: within a few units in the last place as far as the sigmoid is any number, half the smallest one's
+    step times |z| below the normal numbers, -0 beyond."""
+    z = torch.cat([torch.linspace(-104.5, -30, 1 << 16), torch.linspace(-30, 110, 1 << 16), torch.tensor([-1e5, -1e30, -3.4e38])]).to(DEV)
+    got = M.silu_glu(torch.stack([z, torch.ones_like(z)], 1).contiguous())[:, 0].double()
+    want = z.double() * torch.sigmoid(z.double())
+    err = (got - want).abs()
+    # the exponential's, the sum's and the reciprocal's roundings, and that of the product: 4 units of 2^-24 at most
+    bound = want.abs() * 2.0 ** -22 + z.double().abs().clamp(max=105.0) * 2.0 ** -149
+    assert bool((err <= bound).all()), (float(z[(err - bound).argmax()]), float((err / bound).max()))
