@@ -1080,13 +1080,18 @@ def band_attention_ok(out, q, k_cache, v_cache, seg: Segments, spec: WindowSpec)
 def _band_pays(seg: Segments, sp: WindowSpec, min_rows: int) -> bool:
     """A workgroup of the one kernel owns 64 (row, query head) pairs and walks their keys, so a few rows behind a long
     context leave the chip idle, where the products' widened copies and library kernels fill it: 64 rows of 16 heads of
-    128 on 4 key heads at position 8000 take 165 us and the products 149, at 30000 591 and 570; 64 at 2000 52 and 115, 300
-    at 4000 96 and 252, 2000 from 0 70 and 474.  The line is drawn for a walk of 36 ns a key (plain; 50 to 58 with a cap, a
-    table or sigmoids), 340 walks at a time, half as fast as it is now, so it errs towards the products, by up to their 100
-    us; those: 25 launches that take 100 us to issue, the reads of the cache and the pairs' sums."""
+    128 on 4 key heads at position 8000 take 174 us and the products 144, at 30000 609 and 566; 32 at 2000 54 and 122, 300
+    at 4000 101 and 245, 2000 from 0 72 and 510.  A key costs the longest walk 20 ns (26 with a table or sigmoids, 31 with a cap;
+    38 with distance terms in a softmax, 48 to 79 with terms that only the general form of the kernel has), a CU one walk at
+    a time; the products, whose 25 launches take 100 us to issue, the reads of the cache and the pairs' sums, by an estimate
+    that is up to a fifth above them near the line."""
     start, _, kv_len = seg.host
     wide, rep = (sp.dk + sp.dv) / 256, sp.heads // sp.kv_heads
-    kind = 33 if sp.sigmoid else 30 if sp.dist_bias is not None else 28 if sp.softcap > 0 else 14
+    cap, table, terms = sp.softcap > 0, sp.dist_bias is not None, sp.r1 is not None
+    if (cap or table) if sp.sigmoid else (terms or (cap and table)):
+        kind = 26 + 13 * cap + 19 * table + 9 * bool(sp.sigmoid)
+    else:
+        kind = (20 if terms else 14) if sp.sigmoid else 14 if table else 19 if cap else 8
     a = 4 + 4 * sp.kv_heads * (sp.maps * sp.dk + sp.dv) / 1024
     b = sp.heads * sp.maps * (0.0053 + 0.0049 * wide)
     longest = total = products = 0.0
@@ -1097,7 +1102,7 @@ def _band_pays(seg: Segments, sp: WindowSpec, min_rows: int) -> bool:
         longest = max(longest, keys)
         total += keys * sp.kv_heads * sp.maps * (-(-n * rep // 64))
         products += max(100.0, 20 + 1e-3 * keys * (a + b * n) * (0.8 if sp.sigmoid else 1.0))
-    return 10 + 1e-3 * (kind + 22 * wide) * max(longest, total / 340) <= products
+    return 10 + 1e-3 * (kind + 12 * wide) * max(longest, total / 256) <= 0.92 * products
 
 
 def _band_groups(seg: Segments, sp: WindowSpec, min_rows: int) -> int:

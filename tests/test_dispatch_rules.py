@@ -15,23 +15,32 @@ SPECS = {
     "plain": CAUSAL, "cap": dict(CAUSAL, softcap=30.0), "table": dict(CAUSAL, dist_bias=True),
     "sigmoid": dict(CAUSAL, sigmoid=True), "narrow": dict(heads=8, kv_heads=8, dk=64, dv=64, window=0),
     "window": dict(CAUSAL, window=1024), "two maps": dict(CAUSAL, dk=64, window=1024, maps=2),
-    "wide blocks": dict(heads=16, kv_heads=16, dk=128, dv=128, window=4096, blocks=True),
+    "wide blocks": dict(heads=16, kv_heads=16, dk=128, dv=128, window=4096, blocks=True), "terms": dict(CAUSAL, r1=True),
+    "sigmoid terms": dict(CAUSAL, sigmoid=True, r1=True), "cap table": dict(CAUSAL, softcap=30.0, dist_bias=True),
 }
 
 
 @pytest.mark.parametrize("spec,rows,count,pos,one,products", [
-    ("plain", 32, 1, 0, 11, 99), ("plain", 32, 1, 2000, 82, 101), ("plain", 64, 1, 8000, 297, 138),
-    ("plain", 64, 1, 30000, 1074, 562), ("plain", 300, 1, 4000, 165, 235), ("plain", 300, 1, 30000, 1090, 1930),
-    ("plain", 1000, 1, 30000, 1121, 5143), ("plain", 2000, 1, 0, 112, 518), ("plain", 40, 8, 700, 37, 768),
-    ("plain", 32, 4, 15000, 545, 776), ("plain", 33, 1, 120000, 4219, 1580),
-    ("cap", 64, 1, 8000, 409, 138), ("cap", 300, 1, 4000, 227, 240), ("cap", 32, 4, 15000, 759, 790),
-    ("table", 32, 1, 2000, 120, 104), ("table", 64, 1, 30000, 1555, 589), ("table", 1000, 1, 30000, 1592, 5763),
-    ("sigmoid", 32, 1, 2000, 117, 103), ("sigmoid", 64, 1, 30000, 1619, 477), ("sigmoid", 32, 4, 15000, 817, 648),
-    ("sigmoid", 1000, 1, 30000, 1682, 3701), ("sigmoid", 300, 1, 0, 25, 103),
-    ("narrow", 64, 1, 8000, 208, 124), ("narrow", 300, 1, 4000, 117, 165), ("narrow", 64, 1, 30000, 749, 340),
-    ("narrow", 1000, 1, 30000, 776, 2111), ("window", 64, 1, 8000, 48, 100), ("window", 300, 1, 4000, 49, 136),
-    ("two maps", 64, 1, 8000, 42, 107), ("wide blocks", 64, 1, 8000, 152, 99), ("wide blocks", 300, 1, 4000, 158, 255),
-    ("wide blocks", 2000, 1, 0, 117, 436)])
+    ("plain", 32, 1, 0, 11, 118), ("plain", 32, 1, 2000, 54, 122), ("plain", 64, 1, 8000, 174, 144),
+    ("plain", 64, 1, 30000, 609, 566), ("plain", 300, 1, 4000, 101, 245), ("plain", 300, 1, 30000, 623, 1937),
+    ("plain", 1000, 1, 30000, 664, 5150), ("plain", 2000, 1, 0, 72, 510), ("plain", 40, 8, 700, 29, 806),
+    ("plain", 32, 4, 15000, 312, 771), ("plain", 33, 1, 120000, 2381, 1599), ("cap", 64, 1, 8000, 258, 142),
+    ("cap", 300, 1, 4000, 145, 243), ("cap", 32, 4, 15000, 463, 780), ("table", 32, 1, 2000, 65, 116),
+    ("table", 64, 1, 30000, 771, 617), ("table", 1000, 1, 30000, 801, 5784), ("sigmoid", 32, 1, 2000, 66, 104),
+    ("sigmoid", 64, 1, 30000, 806, 478), ("sigmoid", 32, 4, 15000, 408, 650), ("sigmoid", 1000, 1, 30000, 839, 3703),
+    ("sigmoid", 300, 1, 0, 22, 108), ("narrow", 64, 1, 8000, 119, 128), ("narrow", 300, 1, 4000, 70, 169),
+    ("narrow", 64, 1, 30000, 412, 338), ("narrow", 1000, 1, 30000, 429, 2111), ("window", 64, 1, 8000, 34, 105),
+    ("window", 300, 1, 4000, 36, 139), ("two maps", 64, 1, 8000, 29, 108), ("wide blocks", 64, 1, 8000, 91, 103),
+    ("wide blocks", 300, 1, 4000, 95, 259), ("wide blocks", 2000, 1, 0, 72, 441), ("plain", 64, 1, 4000, 93, 103),
+    ("plain", 128, 1, 8000, 173, 227), ("plain", 128, 1, 30000, 607, 746), ("plain", 32, 1, 8000, 172, 124),
+    ("plain", 100, 1, 3000, 75, 119), ("cap", 64, 1, 4000, 137, 106), ("cap", 128, 1, 8000, 259, 229),
+    ("cap", 200, 1, 8000, 260, 384), ("cap", 32, 1, 2000, 74, 107), ("table", 64, 1, 8000, 219, 149),
+    ("table", 128, 1, 8000, 219, 232), ("sigmoid", 64, 1, 8000, 223, 122), ("sigmoid", 128, 1, 8000, 227, 196),
+    ("sigmoid", 250, 1, 20000, 549, 687), ("narrow", 64, 1, 4000, 66, 97), ("narrow", 128, 1, 8000, 121, 136),
+    ("narrow", 200, 1, 8000, 121, 189), ("terms", 64, 1, 8000, 325, 135), ("terms", 300, 1, 4000, 181, 245),
+    ("sigmoid terms", 64, 1, 8000, 270, 119), ("sigmoid terms", 300, 1, 4000, 152, 216),
+    ("cap table", 64, 1, 8000, 564, 146), ("cap table", 300, 1, 4000, 311, 258), ("plain", 64, 4, 8000, 174, 520),
+    ("cap", 2000, 1, 8000, 572, 2913), ("plain", 48, 16, 1500, 49, 1428)])
 def test_long_windowed_segments(spec, rows, count, pos, one, products):
     sp = M.WindowSpec(scale=1.0, **SPECS[spec])
     taken = one if M._band_pays(segments(rows, count, pos), sp, 32) else products
