@@ -528,8 +528,9 @@ extern "C" int ft_prefill_attention(void* out, int out_stride, const void* q, in
   // Workgroups start in the order of their numbers, and the items come longest first.  Where they take several rounds of the
   // 256 CUs (one workgroup each) all heads of an item come before the next item, so that the last ones to start are the
   // shortest of any head, and an XCD keeps few heads' keys: 32 on 8 heads of 128, us, a head at a time / so: 4096 tokens
-  // 278 / 180, 1500 68 / 62, 4 x 1024 over 4096 382 / 357, 5 x 400 40 / 36.  In one round the heads apart are better, each
-  // XCD reading several: 777 tokens 27.4 / 29.1, 500 over 1000 32.7 / 36.5.
+  // 278 / 180 (167 with the ranges planned for this order, 195 in a model's step behind a product), 1500 68 / 62, 4 x 1024
+  // over 4096 382 / 357, 5 x 400 40 / 36.  In one round the heads apart are better, each XCD reading several: 777 tokens
+  // 27.4 / 29.1, 500 over 1000 32.7 / 36.5.
   const bool heads_first = (long)num_tiles * nkv > 256 && (long)num_tiles * nkv <= 0x7fffffffL;
   dim3 grid(heads_first ? num_tiles * nkv : num_tiles, heads_first ? 1 : nkv), block(512);
 #define FT_PF_CASE(DD, GG)                                                                   \

@@ -341,7 +341,7 @@ def build_prefill_tiles(q_lens, tile_tokens: int, seq_lens=None, nkv: int = 8, n
             items.append((b, s, 0xFFFF, -1))
             sizes.append(nkt)
     # the longest first: workgroups start in this order, and one that starts last ends last (4096 tokens of one prompt, us a
-    # layer: 280 with the longest last, 180)
+    # layer: 278 with the longest last, 180; 167 with the plan above)
     if len(items) * nkv > num_cus:
         order = sorted(range(len(items)), key=sizes.__getitem__, reverse=True)
         items = [items[i] for i in order]
