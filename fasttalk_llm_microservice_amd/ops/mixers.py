@@ -115,8 +115,8 @@ def _tile_gemm_pays(rows: int, n: int, k: int, act: Optional[str] = None) -> boo
     above that of its operations at 1.3 PFLOP/s, and the activation's kernel, which takes 4 us and its bytes at 3.5 TB/s.  Up to
     1024 rows a step is issued by the host, where a call of the vendor's product takes 21 us and this one 5, so the kernel may
     be behind by a few (2 to 4 us of 25 to 35 from 640 rows on; at most 13 of 82 were seen: gated 2 x 6144, k = 4096, 640
-    rows); captured steps: :func:`_tile_gemm_behind`.  Beyond, the sooner full tiles keep the vendor's product at its rate, the less.  us at 100 / 300 / 777 /
-    2048 / 4096 rows, the vendor's (with the activation) beside it:
+    rows); captured steps: :func:`_tile_gemm_behind`.  Beyond, the sooner full tiles keep the vendor's product at its rate, the
+    less.  us at 100 / 300 / 777 / 2048 / 4096 rows, the vendor's (with the activation) beside it:
       n = 2048, k = 2048     7 10 14 22 40 (9 11 15 23 35)         k = 8192            22 31 49 90 128 (21 33 47 74 118)
       n = 10272, k = 2048    18 21 47 92 155 (18 26 41 96 180)     n = 64              6 7 7 7 8 (8 8 8 9 10)
       gated, 2 x 8192, k = 2048    20 34 55 109 225 (28 40 66 137 270)
