@@ -18,8 +18,8 @@
 // taller tile empty).  The tiles run group by group, bands of eight row tiles with their columns after each
 // other, and each XCD (workgroup id mod 8) takes one contiguous eighth of that order, so the tiles in flight on
 // an XCD share an expert's rows and columns in its L2.
-// Serves short groups, where it is bound by the read of the matrices, and rows that are no whole stages of tile_gemm.hip's:
-// tall groups go there (mx_grouped_gemm has the line and both sides).  1800 pairs of 32 experts, 2048 -> 2 x 1024 gated (268 MB):
+// Serves short groups of small sets, where it is bound by the read of the matrices, and rows that are no whole stages of
+// tile_gemm.hip's: the others go there (mx_grouped_gemm has the lines and both sides).  1800 pairs of 32 experts, 2048 -> 2 x 1024 gated (268 MB):
 // 78 us in a model, with one step of loads in flight, a barrier between reads and products and tiles in grid order 98.
 #include "few_rows.h"
 
@@ -349,6 +349,7 @@ extern "C" int mx_tile_gemm(void* C, long c_stride, const void* A, long a_stride
                             hipStream_t s);
 extern "C" int mx_tile_form_128();
 extern "C" int mx_tile_form_256();
+extern "C" int mx_tile_form_groups();
 
 // act: few_rows.h (0: none).  a_rows: rows of A (M without an index).  rows: A's row of every sorted row, or null.
 extern "C" int mx_grouped_gemm(void* C, const void* A, long a_rows, const int* rows, const void* W, const int* offs, int groups,
@@ -359,13 +360,24 @@ extern "C" int mx_grouped_gemm(void* C, const void* A, long a_rows, const int* r
   const bool glu = act >= kFrGelu && act <= kFrClamp;
   const int vec = N % 4 == 0 && ((uintptr_t)C) % 8 == 0;
   if ((M + 63) / 64 + groups > 65535) return -3;
-  // Tall groups take tile_gemm.hip's tiles, 256 x 256 or, up to 120 rows a group, 128 x 128.  us, 32 groups of 2048 -> 2 x 1024
-  // (gated), here with 64-row tiles / 128-row tiles / there with 128 / 256:  38 rows a group 64 - 70 80; 56: 71 - 69 80;
-  // 75: 76 - 70 80; 97: - 70 70 83; 125: - 89 81 81; 175: - 115 103 83; 250: - 130 120 119; 512: - 220 205 174;
-  // 128 groups of 768 -> 2048: 38 rows 97 - 111, 62: 116 - 117, 87: 145 - 125 130, 125: - 158 156 136
-  if (M >= 50L * groups && mx_tile_gemm_fits(a_rows, N, K, K, glu))
-    return mx_tile_gemm(C, N, A, K, a_rows, rows, W, nullptr, offs, groups, M, N, K, act, limit,
-                        M >= 120L * groups ? mx_tile_form_256() : mx_tile_form_128(), s);
+  // tile_gemm.hip's tiles wherever rows are whole stages, by what fills the card.  us, 64-row tiles here / 128 x 128 / 256 x 256 /
+  // 256 x 256 with shorter last pieces, matrices from HBM:
+  //   32 groups of 2048 -> 2 x 1024 (gated)  8 rows a group: 64 70 82 52; 56: 71 69 80 53; 125: - 86 81 61; 234: - 122 119 84; 512: -
+  //   207 186 145;  128 of 768 -> 2048  4: 78 101 116 82; 28: 90 107 119 89; 88: - 129 137 112; 117: - 139 145 120
+  //   16 of 1024 -> 2 x 256, 2 columns of tiles each  16: 12.7 - - 16.0; 300: - - 29.4 30.0;  4 of 512 -> 2 x 512  50: 8.8 - - 9.5
+  // Short k of few rows is the 64-row kernel's (32 of 1024 -> 2048, 8 rows: 26 and 28), and matrices that the last level cache does
+  // not hold are read twice where most groups are one tile and a piece (8 of 4096 -> 2 x 4096, 350 rows: 213 and 221; 64 of 4096
+  // -> 2 x 1408, 375: 598 and 623; 268 MB of them, 375: 119 and 113).
+  if (mx_tile_gemm_fits(a_rows, N, K, K, glu)) {
+    const long wide = (long)groups * ((N + (glu ? 127 : 255)) / (glu ? 128 : 256)), w_bytes = 2L * groups * N * K * (glu ? 2 : 1);
+    const bool twice = w_bytes >= 512L << 20 && M > 256L * groups && M < 420L * groups;
+    int form = -1;
+    if (wide >= 128 && !twice && (K > 1024 || M >= 25L * groups)) form = mx_tile_form_groups();
+    else if (M >= 120L * groups) form = mx_tile_form_256();
+    else if (M >= 50L * groups) form = mx_tile_form_128();
+    if (form >= 0)
+      return mx_tile_gemm(C, N, A, K, a_rows, rows, W, nullptr, offs, groups, M, N, K, act, limit, form, s);
+  }
   // 128-row tiles once the groups fill them on average
   const bool tall = M >= 96L * groups;
   const int cols = 128 / (glu ? 2 : 1), col_tiles = (N + cols - 1) / cols;

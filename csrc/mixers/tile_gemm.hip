@@ -9,7 +9,7 @@
 // the same 16 of the up matrix, so a lane has both sums and the activation is part of the epilogue.  Results leave through
 // LDS, whole rows of the tile at a time (written four columns a lane, 4096 x 4096 -> 2 x 14336 takes 700 us instead of 656).
 //
-// Three kernels, for different numbers of tiles (the table of forms below has their times):
+// Four kernels, for different numbers of tiles (the table of forms below has the times of three):
 //   tile_phase_kernel  256 x 256, eight waves in two groups half a phase apart: while one group's products run, the other's
 //                      LDS reads and loads do (all eight in step, 4096 x 2048 -> 2 x 8192 takes 259 us instead of 225).
 //                      Bound by the matrix units at the clock that the card's power leaves them: 4096 x 4096 -> 2 x 14336
@@ -20,6 +20,11 @@
 //   tile_split_kernel  64 x 64 and smaller, eight waves that share a tile and split its k, each staging its own: few tiles,
 //                      where the chain of stages with a barrier each is what takes the time (300 x 2048 -> 2048: 10 us, the ring
 //                      14, the vendor 11).
+//   tile_groups_kernel 256 x 256 for the whole tiles of each group and 128 or 64 x 256 for what is left of it, the whole ones
+//                      first: 512 rows an expert are two tiles and a few rows for every other expert.  Bound by the matrix units or,
+//                      up to a hundred rows a group, by the read of the matrices (5.4 TB/s).  us before and now, 32 experts: 4096
+//                      rows, top 4, of 2048 -> 2 x 1024 and back 186 + 104, 145 + 86; 1872, of 2048 -> 1536 and back 65 + 92, 61 + 71;
+//                      300, top 6, of 2048 -> 2 x 1024 71, 53.
 #include "few_rows.h"
 #include "ft_lds.h"
 
@@ -146,6 +151,18 @@ __device__ __forceinline__ unsigned tile_w_off(const TileArgs& P, int n0, int r,
   return (unsigned)((GLU && (r & 16) ? P.N : 0) + col) * P.w_bytes + (unsigned)(((lane & 7) ^ ((r >> 1) & 5)) * 16);
 }
 
+// SPREAD: every XCD begins k at another eighth of it.  Rows of 4 KB put one stage of all rows into few of the memory's channels,
+// and with the workgroups all at the same stage those are what the read waits for: 32 matrices of 2 x 1024 x 2048 with up to 64 rows
+// each 71 us (3.8 TB/s) in step, 50 (5.4) spread; 234 rows each 97 and 84.  Tiles of one XCD stay in step, since they share rows in
+// its L2.  Products of one matrix read it at that rate from a few rows on and gain nothing.
+__device__ __forceinline__ int tile_first_stage(int nk) { return (int)(blockIdx.x & 7) * nk / 8; }
+template <bool SPREAD>
+__device__ __forceinline__ int tile_stage_at(int t, int k0, int nk) {
+  if constexpr (!SPREAD) return t;
+  t += k0;
+  return t >= nk ? t - nk : t;
+}
+
 template <bool GLU>
 __device__ __forceinline__ void tile_result(const TileArgs& P, int col, const fr_f32x4& x, const fr_f32x4& up, float (&v)[4]) {
 #pragma unroll
@@ -199,22 +216,20 @@ __device__ __forceinline__ void tile_out(const TileArgs& P, char* smem, int row0
 // slots.  Every phase: the loads that the next one reads have landed (counted; a barrier lies between), reads, loads,
 // barrier, products, barrier.  The second group of waves runs one barrier behind the first.
 // ---------------------------------------------------------------------------------
-template <bool GLU>
-__global__ void __launch_bounds__(512, 1)
-tile_phase_kernel(TileArgs P) {
-  constexpr int QM = 4, QN = 2, HM = 32 * QM, HN = 64 * QN, BM = 2 * HM, BN = 2 * HN;
+constexpr int kPhaseLds = 131072;
+
+template <bool GLU, bool SPREAD = false>
+__device__ __forceinline__ void tile_phase(const TileArgs& P, const TileAt& at, char* smem) {
+  constexpr int QM = 4, QN = 2, HM = 32 * QM, HN = 64 * QN, BN = 2 * HN;
   constexpr int PA = HM / 64, PB = HN / 64;                         // loads a wave and half
   constexpr int kA = HM * 128, kB = HN * 128, kSlot = 2 * (kA + kB);
   constexpr int OC = GLU ? BN / 2 : BN;
-  static_assert(HM * (OC * 2 + 16) <= 2 * kSlot, "results fit");
-  __shared__ __attribute__((aligned(16))) char smem[2 * kSlot];
+  static_assert(2 * kSlot == kPhaseLds && HM * (OC * 2 + 16) <= 2 * kSlot, "results fit");
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 2, wn = wave & 3, l15 = lane & 15, g4 = lane >> 4;
-  TileAt at;
-  if (!tile_at<BM>(P, lane, at)) return;
   const int n0 = at.ct * OC;
   const bf16_t* W = P.W + (long)at.g * P.N * (GLU ? 2 : 1) * P.K;
-  const int nk = P.K / kTK;
+  const int nk = P.K / kTK, k0 = SPREAD ? tile_first_stage(nk) : 0;
   const uint32_t lds0 = ft::lds_off(smem);
   unsigned ap[2][PA], wp[2][PB];
 #pragma unroll
@@ -225,14 +240,16 @@ tile_phase_kernel(TileArgs P) {
     for (int p = 0; p < PB; ++p) wp[h][p] = tile_w_off<GLU>(P, n0, h * HN + (wave + 8 * p) * 8 + (lane >> 3), lane);
   }
   auto load_a = [&](int h, int t) {
+    const int k = tile_stage_at<SPREAD>(t, k0, nk);
     const uint32_t dst = lds0 + (t & 1) * kSlot + h * kA + wave * 1024;
 #pragma unroll
-    for (int p = 0; p < PA; ++p) tile_dma(P.A + t * kTK, ap[h][p], dst + p * 8192);
+    for (int p = 0; p < PA; ++p) tile_dma(P.A + k * kTK, ap[h][p], dst + p * 8192);
   };
   auto load_w = [&](int h, int t) {
+    const int k = tile_stage_at<SPREAD>(t, k0, nk);
     const uint32_t dst = lds0 + (t & 1) * kSlot + 2 * kA + h * kB + wave * 1024;
 #pragma unroll
-    for (int p = 0; p < PB; ++p) tile_dma(W + t * kTK, wp[h][p], dst + p * 8192);
+    for (int p = 0; p < PB; ++p) tile_dma(W + k * kTK, wp[h][p], dst + p * 8192);
   };
   fr_f32x4 acc[2][2][QN][QM];
 #pragma unroll
@@ -336,26 +353,33 @@ tile_phase_kernel(TileArgs P) {
   }
 }
 
+template <bool GLU>
+__global__ void __launch_bounds__(512, 1)
+tile_phase_kernel(TileArgs P) {
+  __shared__ __attribute__((aligned(16))) char smem[kPhaseLds];
+  TileAt at;
+  if (tile_at<256>(P, threadIdx.x & 63, at)) tile_phase<GLU>(P, at, smem);
+}
+
 // ---------------------------------------------------------------------------------
 // WM x WN waves of MT x NT tiles of 16, a ring of S stages.  The operands of a stage's second half are read under its first
 // half's products and the next stage's first half under the second's, a barrier a stage.
 // ---------------------------------------------------------------------------------
-template <int WM, int WN, int MT, int NT, int S, bool GLU>
-__global__ void __launch_bounds__(64 * WM * WN, 1)
-tile_ring_kernel(TileArgs P) {
+template <int WM, int WN, int MT, int NT, int S>
+constexpr int kRingLds = S * (WM * MT + WN * NT) * 16 * 128;
+
+template <int WM, int WN, int MT, int NT, int S, bool GLU, bool SPREAD = false>
+__device__ __forceinline__ void tile_ring(const TileArgs& P, const TileAt& at, char* smem) {
   constexpr int NW = WM * WN, BM = WM * MT * 16, BN = WN * NT * 16;
   constexpr int PA = BM / (8 * NW), PB = BN / (8 * NW), PW = PA + PB;
   constexpr int kStage = (BM + BN) * 128, OC = GLU ? BN / 2 : BN;
   static_assert(BM % (8 * NW) == 0 && BN % (8 * NW) == 0 && (!GLU || NT % 2 == 0), "");
   static_assert(BM * (OC * 2 + 16) <= S * kStage && S >= 3, "");
-  __shared__ __attribute__((aligned(16))) char smem[S * kStage];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WN, wn = wave % WN, l15 = lane & 15, g4 = lane >> 4;
-  TileAt at;
-  if (!tile_at<BM>(P, lane, at)) return;
   const int n0 = at.ct * OC;
   const bf16_t* W = P.W + (long)at.g * P.N * (GLU ? 2 : 1) * P.K;
-  const int nk = P.K / kTK;
+  const int nk = P.K / kTK, k0 = SPREAD ? tile_first_stage(nk) : 0;
   const uint32_t lds0 = ft::lds_off(smem);
   unsigned ap[PA], wp[PB];
 #pragma unroll
@@ -364,8 +388,9 @@ tile_ring_kernel(TileArgs P) {
   for (int p = 0; p < PB; ++p) wp[p] = tile_w_off<GLU>(P, n0, (wave + NW * p) * 8 + (lane >> 3), lane);
   auto load1 = [&](int t, int slot, int p) {
     const uint32_t dst = lds0 + slot * kStage + wave * 1024;
-    if (p < PA) tile_dma(P.A + t * kTK, ap[p < PA ? p : 0], dst + p * NW * 1024);
-    else tile_dma(W + t * kTK, wp[p < PA ? 0 : p - PA], dst + BM * 128 + (p - PA) * NW * 1024);
+    const int k = tile_stage_at<SPREAD>(t, k0, nk);
+    if (p < PA) tile_dma(P.A + k * kTK, ap[p < PA ? p : 0], dst + p * NW * 1024);
+    else tile_dma(W + k * kTK, wp[p < PA ? 0 : p - PA], dst + BM * 128 + (p - PA) * NW * 1024);
   };
   fr_f32x4 acc[NT][MT];
 #pragma unroll
@@ -456,6 +481,86 @@ tile_ring_kernel(TileArgs P) {
       for (int i = 0; i < NT; i += GLU ? 2 : 1)
         write((wm * MT + j) * 16 + l15, (wn * NT + i) * 16 / (GLU ? 2 : 1) + 4 * g4, acc[i][j], acc[GLU ? i + 1 : i][j]);
   });
+}
+
+template <int WM, int WN, int MT, int NT, int S, bool GLU>
+__global__ void __launch_bounds__(64 * WM * WN, 1)
+tile_ring_kernel(TileArgs P) {
+  __shared__ __attribute__((aligned(16))) char smem[kRingLds<WM, WN, MT, NT, S>];
+  TileAt at;
+  if (tile_at<WM * MT * 16>(P, threadIdx.x & 63, at)) tile_ring<WM, WN, MT, NT, S, GLU>(P, at, smem);
+}
+
+// ---------------------------------------------------------------------------------
+// Groups in tiles of 256 rows and, for a last piece of at most 128 or 64 rows, of that many, which take half and a third of
+// a whole one's time.
+// ---------------------------------------------------------------------------------
+// As tile_at, the groups' whole tiles (a last piece of more than 128 rows is one) before all shorter ones: the workgroups
+// that are dispatched last take the least time.
+__device__ __forceinline__ bool tile_at_groups(const TileArgs& P, int lane, TileAt& at, bool& shorter) {
+  const int x = blockIdx.x & 7, cols = P.col_tiles;
+  int i = blockIdx.x >> 3, lo = 0, hi = 0, whole = 0, part = 0;
+  // lane's group's whole and short tiles; the sums over lanes up to it come back as whole * 128 + short (at most 64 of them)
+  auto span = [&](int k) {
+    lo = k > 0 && k < P.groups ? min(max(P.offs[k - 1], 0), P.M) : 0;
+    hi = k < P.groups ? min(max(P.offs[k], lo), P.M) : lo;
+    const int last = (hi - lo) & 255;
+    whole = ((hi - lo) >> 8) + (last > 128 ? 1 : 0);
+    part = last > 0 && last <= 128 ? 1 : 0;
+    int upto = whole * 128 + part;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int y = __shfl_up(upto, o, 64);
+      upto += lane >= o ? y : 0;
+    }
+    return upto;
+  };
+  int wholes = 0, parts = 0, upto = 0;
+  for (int g0 = 0; g0 < P.groups; g0 += 64) {
+    upto = span(g0 + lane);
+    const int sum = __shfl(upto, 63, 64);
+    wholes += sum >> 7, parts += sum & 127;
+  }
+  long all = (long)wholes * cols, per = (all + 7) / 8;
+  shorter = i >= per;
+  if (shorter) i -= (int)per, all = (long)parts * cols, per = (all + 7) / 8;
+  const long t = x * per + i;
+  if (i >= per || t >= all) return false;
+  const int tile = (int)(t / cols);
+  int base = 0, g = 0;
+  uint64_t past = 0;
+  auto mine = [&](int v) { return shorter ? v & 127 : v >> 7; };
+  for (;; g += 64) {                            // (ends: tile < the sum of all)
+    if (P.groups > 64) upto = span(g + lane);
+    past = __ballot(base + mine(upto) > tile);
+    if (past != 0 || g + 64 >= P.groups) break;
+    base += mine(__shfl(upto, 63, 64));
+  }
+  const int k = past != 0 ? __builtin_ctzll(past) : 63;
+  lo = __builtin_amdgcn_readlane(lo, k);
+  hi = __builtin_amdgcn_readlane(hi, k);
+  const int n = __builtin_amdgcn_readlane(shorter ? part : whole, k);
+  const int first = base + mine(__builtin_amdgcn_readlane(upto, k)) - n;
+  const int r = (int)(t - (long)first * cols), band = r / (8 * cols), in = r - band * 8 * cols, tall = min(8, n - 8 * band);
+  at.g = __builtin_amdgcn_readfirstlane(g + k);
+  at.ct = __builtin_amdgcn_readfirstlane(in / tall);
+  at.row0 = __builtin_amdgcn_readfirstlane(shorter ? hi - ((hi - lo) & 255) : lo + (8 * band + in % tall) * 256);
+  at.end = __builtin_amdgcn_readfirstlane(hi);
+  return true;
+}
+
+template <bool GLU>
+__global__ void __launch_bounds__(512, 1)
+tile_groups_kernel(TileArgs P) {
+  constexpr int k64 = kRingLds<1, 8, 4, 2, 4>, k128 = kRingLds<2, 4, 4, 4, 3>;
+  constexpr int kRing = k64 > k128 ? k64 : k128;
+  __shared__ __attribute__((aligned(16))) char smem[kRing > kPhaseLds ? kRing : kPhaseLds];
+  TileAt at;
+  bool shorter;
+  if (!tile_at_groups(P, threadIdx.x & 63, at, shorter)) return;
+  if (!shorter) tile_phase<GLU, true>(P, at, smem);
+  else if (at.end - at.row0 > 64) tile_ring<2, 4, 4, 4, 3, GLU, true>(P, at, smem);
+  else tile_ring<1, 8, 4, 2, 4, GLU, true>(P, at, smem);
 }
 
 // ---------------------------------------------------------------------------------
@@ -557,7 +662,7 @@ tile_split_kernel(TileArgs P) {
 // the second part for what all CUs share (rates of the L2 and of memory, the card's power).  Fitted to 504 products of 65 to 4096
 // rows, weights from HBM, N and K of 64 to 14336 (residuals 4 to 11 %); the form chosen takes 1.006 times the best one's
 // time in the mean, 1.2 times at most.
-enum TileForm { kTile256x256, kTile256x128, kTile192x128, kTile128x128, kTile64x128, kTile64x64, kTile64x32, kTile32x64, kTileForms };
+enum TileForm { kTile256x256, kTile256x128, kTile192x128, kTile128x128, kTile64x128, kTile64x64, kTile64x32, kTile32x64, kTileForms, kTileGroups = kTileForms };
 struct TileSize {
   int rows, cols;
   float begin, tile, stage, all_stage, all_tile;
@@ -585,6 +690,14 @@ int tile_pick(long M, int N, int K, bool glu, float* us) {
 
 template <bool GLU>
 int tile_launch(TileArgs& P, int form, hipStream_t s) {
+  if (form == kTileGroups) {
+    P.col_tiles = (P.N + (GLU ? 127 : 255)) / (GLU ? 128 : 256);
+    const long tiles = (P.M / 256 + (long)P.groups) * P.col_tiles;       // (a group has n / 256 rounded up)
+    if (P.offs == nullptr || tiles > 0x7fffff00L) return -3;
+    // (both sorts of tiles are eighths, rounded up)
+    hipLaunchKernelGGL((tile_groups_kernel<GLU>), dim3((unsigned)((tiles + 21) / 8 * 8)), dim3(512), 0, s, P);
+    return (int)hipGetLastError();
+  }
   const TileSize& z = kTileSizes[form];
   const int oc = z.cols / (GLU ? 2 : 1);
   P.col_tiles = (P.N + oc - 1) / oc;
@@ -630,7 +743,7 @@ extern "C" int mx_tile_gemm(void* C, long c_stride, const void* A, long a_stride
                             hipStream_t s) {
   if (M <= 0 || N <= 0 || groups <= 0) return 0;
   const bool glu = act >= kFrGelu && act <= kFrClamp;
-  if (act < kFrStore || act > kFrReluSq || form >= kTileForms || M > 0x3fffffffL) return -1;
+  if (act < kFrStore || act > kFrReluSq || form > kTileGroups || M > 0x3fffffffL) return -1;
   if (!mx_tile_gemm_fits(a_rows, N, K, a_stride, glu)) return -1;
   if (((uintptr_t)A) % 16 || ((uintptr_t)W) % 16) return -2;
   if (glu && bias != nullptr) return -4;
@@ -644,3 +757,4 @@ extern "C" int mx_tile_gemm(void* C, long c_stride, const void* A, long a_stride
 // the forms that grouped_gemm.hip takes
 extern "C" int mx_tile_form_128() { return kTile128x128; }
 extern "C" int mx_tile_form_256() { return kTile256x256; }
+extern "C" int mx_tile_form_groups() { return kTileGroups; }

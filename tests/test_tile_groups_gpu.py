@@ -1,0 +1,63 @@
+"""Grouped products in tiles of 256 rows with shorter last pieces (csrc/mixers/tile_gemm.hip, tile_groups_kernel) against the same
+sums in 64 bits: group sizes at the edges of each tile, one to a few stages of k (every XCD begins at another of them), more
+groups than a wave has lanes, plain, gated and through an index."""
+import pytest
+import torch
+
+from fasttalk_llm_microservice_amd.ops import mixers as M
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+EDGES = [0, 1, 63, 64, 65, 127, 128, 129, 255, 256, 257, 320, 321, 384, 385, 512, 513]
+
+
+def rnd(seed, *shape, scale=1.0):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    return (torch.randn(*shape, generator=g, device=DEV) * scale).bfloat16()
+
+
+def close(got, want, k, slope=1.0):
+    """bf16 output: half a unit in the last place, plus fp32 sums of k terms of order 1 through an activation of this slope."""
+    err = (got.double() - want).abs()
+    bound = want.abs() * 2.0 ** -8 + slope * (k ** 0.5 * 2.0 ** -22 + 2.0 ** -20)
+    assert bool((err <= bound).all()), float((err - bound).max())
+
+
+@pytest.mark.parametrize("counts", [EDGES, [3] * 70 + [700] + [0] * 5 + [40] * 60, [0] * 63 + [130] + [0] * 64 + [1]])
+@pytest.mark.parametrize("k", [64, 192, 576, 1088])
+def test_plain_groups(counts, k):
+    e = len(counts)
+    n = 8 * (-(-128 // e) * 256 // 8) - 248          # 128 tiles of columns or more over all groups, the last one 8 wide
+    rows = sum(counts)
+    if k <= 1024 and rows < 25 * e:                  # (few rows of short k are another kernel's)
+        counts = [c * 40 for c in counts]
+        rows *= 40
+    a, w = rnd(e, rows, k), rnd(e + 1, e, n, k, scale=k ** -0.5)
+    got = M.grouped_mm(a, w, torch.tensor(counts).cumsum(0).int().to(DEV))
+    s = 0
+    for g, c in enumerate(counts):
+        close(got[s:s + c], a[s:s + c].double() @ w[g].double().t(), k)
+        s += c
+
+
+@pytest.mark.parametrize("rows,experts,top", [(70, 16, 2), (300, 16, 4), (900, 16, 4), (2100, 16, 3)])
+@pytest.mark.parametrize("act", ["silu_glu", "relu_sq"])
+def test_experts(rows, experts, top, act):
+    """The two products of experts_many one after the other, the first through the index of sorted rows."""
+    width, ff = 2048, 1088                           # (9 tiles of gated columns; the second product's k is 17 stages)
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    h = rnd(rows, rows, width)
+    wgu = rnd(1, experts, (2 if act == "silu_glu" else 1) * ff, width, scale=width ** -0.5)
+    wdown = rnd(2, experts, width, ff, scale=ff ** -0.5)
+    idx = torch.rand(rows, experts, generator=g, device=DEV).topk(top).indices.int().contiguous()
+    wts = torch.rand(rows, top, generator=g, device=DEV)
+    got = M.experts_many(h, idx, wts, wgu, wdown, act)
+    want, size = torch.zeros(rows, width, dtype=torch.float64, device=DEV), torch.zeros(rows, width, dtype=torch.float64, device=DEV)
+    for e in range(experts):
+        u = h.double() @ wgu[e].double().t()
+        y = u.relu() ** 2 if act == "relu_sq" else u[:, :ff] * torch.sigmoid(u[:, :ff]) * u[:, ff:]
+        w = (wts.double() * (idx == e)).sum(1, keepdim=True)
+        want += w * (y @ wdown[e].double().t())
+        size += w * (y.abs() @ wdown[e].double().abs().t())
+    # two bf16 roundings, each half a unit in the eighth bit: 2^-8 of each term of the second product and of its sum
+    assert bool(((got.double() - want).abs() <= 2.0 ** -7 * size + 1e-5).all())
