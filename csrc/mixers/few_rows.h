@@ -37,8 +37,9 @@ constexpr int kFrStage = NB * 16 * kFrRow<U>;
 
 // acc[t][b] += W rows of tile t times X rows of block b, over this wave's share of k.  wp: the lane's
 // row of each tile; xrow(r): row r < rows of X; stage: this wave's kFrStage bytes.  All pieces are 16
-// bytes (K a multiple of 8); those past the wave's share count as zeros.
-template <int NT, int NB, int WV, int U, typename XR>
+// bytes (K a multiple of 8); those past the wave's share count as zeros.  AHEAD: a round's loads are in
+// flight under the products of the one before, for workgroups that have a CU to themselves.
+template <int NT, int NB, int WV, int U, bool AHEAD = false, typename XR>
 __device__ __forceinline__ void few_rows_core(fr_f32x4 (&acc)[NT][NB], const bf16_t* const (&wp)[NT], XR xrow, int rows,
                                               int K, char* stage, int wave, int lane) {
   constexpr int LPR = U * 8, RPI = 64 / LPR, XI = NB * 16 / RPI;   // lanes a row, rows a load, loads a round
@@ -46,8 +47,8 @@ __device__ __forceinline__ void few_rows_core(fr_f32x4 (&acc)[NT][NB], const bf1
   const int per = (((K + 63) >> 6) + WV - 1) / WV * 64;
   const int kend = min((wave + 1) * per, K);
   const int sr = lane / LPR, sk = (lane % LPR) * 8;
-  for (int k0 = wave * per; k0 < kend; k0 += 64 * U) {
-    uint4 x[XI], w[U][NT][2];
+  uint4 x[XI], w[U][NT][2];
+  auto fetch = [&](int k0) {
 #pragma unroll
     for (int i = 0; i < XI; ++i) {
       const int r = i * RPI + sr;
@@ -64,11 +65,25 @@ __device__ __forceinline__ void few_rows_core(fr_f32x4 (&acc)[NT][NB], const bf1
           w[u][t][j] = uint4{0, 0, 0, 0};
           if (k < kend) w[u][t][j] = *reinterpret_cast<const uint4*>(wp[t] + k);
         }
+  };
+  if constexpr (AHEAD) fetch(wave * per);
+  for (int k0 = wave * per; k0 < kend; k0 += 64 * U) {
+    if constexpr (!AHEAD) fetch(k0);
     wave_lds_fence();                            // the last round's operands have been read
 #pragma unroll
     for (int i = 0; i < XI; ++i) {
       const int r = i * RPI + sr;
       if (r < rows) *reinterpret_cast<uint4*>(stage + r * kFrRow<U> + sk * 2) = x[i];
+    }
+    uint4 now[U][NT][2];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) now[u][t][j] = w[u][t][j];
+    if constexpr (AHEAD) {
+      if (k0 + 64 * U < kend) fetch(k0 + 64 * U);
     }
     wave_lds_fence();
 #pragma unroll
@@ -82,7 +97,7 @@ __device__ __forceinline__ void few_rows_core(fr_f32x4 (&acc)[NT][NB], const bf1
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll
-          for (int b = 0; b < NB; ++b) acc[t][b] = fr_mfma(w[u][t][j], xb[b], acc[t][b]);
+          for (int b = 0; b < NB; ++b) acc[t][b] = fr_mfma(now[u][t][j], xb[b], acc[t][b]);
       }
   }
 }

@@ -118,7 +118,7 @@ few_rows_gemm_kernel(TO* __restrict__ Y, long y_stride, const bf16_t* __restrict
 // ---------------------------------------------------------------------------------
 // Experts of few rows.  A workgroup owns one tile of 16 (two) columns of one expert's matrix and
 // serves every row that chose the expert: the matrix is read once however many rows share it.
-// blockIdx.y: expert; == experts: the shared expert, which serves all rows.
+// blockIdx.y: expert (expert_in_slot); the last row: the shared expert, which serves all rows.
 // Bound by the stream of the chosen experts' matrices.  32 rows, top 4 of 32 experts of 1536 (relu^2)
 // and a shared one: 44 + 50 us for 214 MB each, 4.9 and 4.3 TB/s, where one read per (row, choice)
 // took 105 + 101 us; 16 rows, top 6 of 32 gated experts of 1024: 54 + 30 us, before 112 + 54.
@@ -128,9 +128,23 @@ struct ExpertSet {
   const bf16_t* shared;   // [shared rows][K_shared], or null
   int experts, K, N;      // N: output columns (GLU: of gate and of up each)
   int shared_K, shared_N;
+  int slots;              // workgroups' rows of the grid before the shared expert's: the experts, or the most that can be chosen
 };
 
 __device__ __forceinline__ int expert_of(int v, int experts) { return v < 0 || v >= experts ? 0 : v; }
+
+// Expert of a row of the grid: itself, or where there are fewer rows than experts the slot-th of the chosen ones (none: -1).
+// One row, top 6 of 32 experts: 6 x 64 workgroups instead of 32 x 64, most of which end after they have read the choices.
+__device__ __forceinline__ int expert_in_slot(const int* __restrict__ idx, int pairs, const ExpertSet& E, int slot) {
+  if (E.slots == E.experts) return slot;         // (E.experts <= 64 otherwise)
+  const int lane = threadIdx.x & 63;
+  uint64_t m = 0;
+  for (int p = lane; p < pairs; p += 64) m |= 1ull << expert_of(idx[p], E.experts);
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) m |= __shfl_xor((unsigned long long)m, o, 64);
+  for (int i = 0; i < slot; ++i) m &= m - 1;
+  return m != 0 ? __builtin_amdgcn_readfirstlane(__builtin_ctzll(m)) : -1;
+}
 
 // the (row, choice) pairs that chose expert e -> list, ascending, the first `room` of them; returns how many there are.
 // `once`: a row's first pair only.  All threads of the workgroup call it.
@@ -172,8 +186,12 @@ __device__ __forceinline__ int rows_of(const int* __restrict__ idx, int pairs, i
   return count;
 }
 
+// steps of k a round (expert_tile_any)
+template <int MB>
+constexpr int kExpSteps = MB == 1 ? 2 : 1;
+
 // the tile's sums for the listed rows: f(entry row in the list, column, sums, up sums)
-template <int P, bool GLU, int NB, int WV, int U, typename F>
+template <int P, bool GLU, int NB, int WV, int U, bool AHEAD, typename F>
 __device__ __forceinline__ void expert_tile(float4* red, const bf16_t* W, int N, int K, int n0, const bf16_t* X,
                                             long x_stride, const int* list, int count, int div, int wave, int lane,
                                             F out) {
@@ -186,7 +204,7 @@ __device__ __forceinline__ void expert_tile(float4* red, const bf16_t* W, int N,
   for (int t = 0; t < NT; ++t)
 #pragma unroll
     for (int b = 0; b < NB; ++b) acc[t][b] = fr_f32x4{0.f, 0.f, 0.f, 0.f};
-  few_rows_core<NT, NB, WV, U>(acc, wp, [&](int r) { return X + (long)(list[r] / div) * x_stride; }, count, K,
+  few_rows_core<NT, NB, WV, U, AHEAD>(acc, wp, [&](int r) { return X + (long)(list[r] / div) * x_stride; }, count, K,
                                reinterpret_cast<char*>(red) + wave * kFrStage<NB, U>, wave, lane);
   __syncthreads();
   few_rows_park<NT, NB, WV>(red, acc, wave, lane);
@@ -202,14 +220,18 @@ __device__ __forceinline__ void expert_tile(float4* red, const bf16_t* W, int N,
   }
 }
 
-// blocks of 16 rows that the listed rows fill, at most MB
+// blocks of 16 rows that the listed rows fill, at most MB.  Steps of at most 16 rows name few experts, whose tiles leave a
+// CU one to three workgroups: two steps of k a round, and the next one's loads under it.  us of both products and the shared
+// expert's, one step a round / so: 3 rows, top 4 of 32 gated experts of 1024 44 / 37.5; 4 rows and a shared one of 2048 55 / 45;
+// 8 of 1536 (relu^2) 67 / 64; 16 rows 73 / 74.  With more rows the CU is full and the registers cost more (64 rows, top 6: 85 / 93).
 template <int P, bool GLU, int WV, int MB, typename F>
 __device__ __forceinline__ void expert_tile_any(float4* red, const bf16_t* W, int N, int K, int n0, const bf16_t* X,
                                                 long x_stride, const int* list, int count, int div, int wave, int lane,
                                                 F out) {
-  if (MB == 1 || count <= 16) expert_tile<P, GLU, 1, WV, 1>(red, W, N, K, n0, X, x_stride, list, count, div, wave, lane, out);
-  else if (MB == 2 || count <= 32) expert_tile<P, GLU, 2, WV, 1>(red, W, N, K, n0, X, x_stride, list, count, div, wave, lane, out);
-  else expert_tile<P, GLU, MB, WV, 1>(red, W, N, K, n0, X, x_stride, list, count, div, wave, lane, out);
+  if (MB == 1) expert_tile<P, GLU, 1, WV, kExpSteps<1>, true>(red, W, N, K, n0, X, x_stride, list, count, div, wave, lane, out);
+  else if (count <= 16) expert_tile<P, GLU, 1, WV, 1, false>(red, W, N, K, n0, X, x_stride, list, count, div, wave, lane, out);
+  else if (MB == 2 || count <= 32) expert_tile<P, GLU, 2, WV, 1, false>(red, W, N, K, n0, X, x_stride, list, count, div, wave, lane, out);
+  else expert_tile<P, GLU, MB, WV, 1, false>(red, W, N, K, n0, X, x_stride, list, count, div, wave, lane, out);
 }
 
 // y[pair] = act(first matrices of the pair's expert times its row of h); ys[row] the same of the
@@ -218,7 +240,7 @@ __device__ __forceinline__ void expert_tile_any(float4* red, const bf16_t* W, in
 constexpr int kExpWaves = 4;
 // X stages and partial sums (two tiles) of a tile with MB blocks of rows
 template <int MB>
-constexpr int kExpLds = kExpWaves * (kFrStage<MB, 1> > 2048 * MB ? kFrStage<MB, 1> : 2048 * MB);
+constexpr int kExpLds = kExpWaves * (kFrStage<MB, kExpSteps<MB>> > 2048 * MB ? kFrStage<MB, kExpSteps<MB>> : 2048 * MB);
 
 template <bool GLU, int MB>
 __global__ void __launch_bounds__(64 * kExpWaves)
@@ -230,9 +252,11 @@ experts_first_kernel(bf16_t* __restrict__ y, bf16_t* __restrict__ ys, float* __r
   __shared__ int list[kFewRows], counts[kExpWaves];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int e = blockIdx.y, n0 = blockIdx.x * 16 * P;
-  if (e < E.experts) {
+  const int n0 = blockIdx.x * 16 * P;
+  if ((int)blockIdx.y < E.slots) {
     if (n0 >= E.N) return;
+    const int e = expert_in_slot(idx, rows * top, E, blockIdx.y);
+    if (e < 0) return;
     bool shared;
     const int count = rows_of<kExpWaves>(idx, rows * top, top, E.experts, e, 16 * MB, list, counts, shared);
     if (count == 0) return;
@@ -273,12 +297,15 @@ experts_down_kernel(float* __restrict__ d, float* __restrict__ ds, const bf16_t*
   __shared__ int list[kFewRows], counts[kExpWaves];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int e = blockIdx.y, n0 = blockIdx.x * 16 * P;
+  const int n0 = blockIdx.x * 16 * P;
+  const bool routed = (int)blockIdx.y < E.slots;
+  const int e = routed ? expert_in_slot(idx, rows * top, E, blockIdx.y) : 0;
+  if (e < 0) return;
   float* dst = d;
   const bf16_t *W = E.w + (long)e * E.N * E.K, *X = y;
   int K = E.K, count = rows;
   bool shared = false;
-  if (e < E.experts) {
+  if (routed) {
     count = rows_of<kExpWaves>(idx, rows * top, top, E.experts, e, 16 * MB, list, counts, shared);
     if (count == 0) return;
   } else {
@@ -419,9 +446,10 @@ extern "C" int mx_experts_few(float* out, void* y, float* d, const void* h, long
   const int cols = glu ? 16 : 32;
   const bool sh = shared_w != nullptr;
   const int tiles = (ff + cols - 1) / cols, tiles_s = sh ? (shared_ff + cols - 1) / cols + (sg != nullptr) : 0;
-  ExpertSet first{(const bf16_t*)wgu, (const bf16_t*)shared_w, experts, width, ff, width, shared_ff};
-  const dim3 g1((unsigned)(tiles > tiles_s ? tiles : tiles_s), (unsigned)(experts + (sh ? 1 : 0))), block(64 * kExpWaves);
-  ExpertSet down{(const bf16_t*)wdown, (const bf16_t*)shared_down, experts, ff, width, shared_ff, width};
+  const int slots = experts <= 64 && rows * top < experts ? rows * top : experts;
+  ExpertSet first{(const bf16_t*)wgu, (const bf16_t*)shared_w, experts, width, ff, width, shared_ff, slots};
+  const dim3 g1((unsigned)(tiles > tiles_s ? tiles : tiles_s), (unsigned)(slots + (sh ? 1 : 0))), block(64 * kExpWaves);
+  ExpertSet down{(const bf16_t*)wdown, (const bf16_t*)shared_down, experts, ff, width, shared_ff, width, slots};
   const dim3 g2((unsigned)((width + 31) / 32), g1.y);
 #define EX_FIRST(GLU, MB)                                                                                              \
   hipLaunchKernelGGL((experts_first_kernel<GLU, MB>), g1, block, 0, s, (bf16_t*)y, (bf16_t*)ys, sg, (const bf16_t*)h, \
