@@ -5,6 +5,7 @@
 // extern "C" launcher on the caller's current HIP stream, so ops are
 // hipGraph-capturable (no allocation, no synchronisation).
 #include <torch/extension.h>
+#include <pybind11/numpy.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime.h>
 
@@ -901,6 +902,27 @@ void set_kernel_checks(torch::Tensor word) {
 }
 #endif
 
+// Views of an int32 image on the device in the types and shapes of the host arrays that were packed into it, array i from word
+// offs[i] on (a step's twelve to twenty take 6 us so, 16 as calls from Python).
+std::vector<at::Tensor> cut_words(at::Tensor image, std::vector<int64_t> offs, py::list arrays) {
+  TORCH_CHECK(image.scalar_type() == at::kInt && image.dim() == 1 && image.is_contiguous() && offs.size() == arrays.size(),
+              "cut_words: an int32 image and a word offset per array");
+  std::vector<at::Tensor> out;
+  out.reserve(offs.size());
+  for (size_t i = 0; i < offs.size(); ++i) {
+    const auto a = py::cast<py::array>(arrays[i]);
+    const int64_t size = a.itemsize(), words = a.size() * size / 4;
+    TORCH_CHECK((size == 4 || size == 8) && offs[i] >= 0 && offs[i] + words <= image.numel(), "cut_words: array ", i);
+    const char kind = a.dtype().kind();
+    const auto type = size == 8 ? (kind == 'i' || kind == 'u' ? at::kLong : at::kDouble) : kind == 'f' ? at::kFloat : at::kInt;
+    at::Tensor v = image.narrow(0, offs[i], words);
+    if (type != at::kInt) v = v.view(type);
+    if (a.ndim() != 1) v = v.view(std::vector<int64_t>(a.shape(), a.shape() + a.ndim()));
+    out.push_back(v);
+  }
+  return out;
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -911,6 +933,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
 #else
   m.attr("kernel_checks") = false;
 #endif
+  m.def("cut_words", &cut_words);
   m.def("rmsnorm", &rmsnorm);
   m.def("fused_add_rmsnorm", &fused_add_rmsnorm);
   m.def("silu_mul", &silu_mul);

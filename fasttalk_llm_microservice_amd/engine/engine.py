@@ -825,7 +825,8 @@ class LLMEngine:
         for rid, toks, _ in entries:
             seq = sched.by_id.get(rid)
             if seq is None:
-                seq = Sequence(rid, list(toks), SamplingParams(temperature=0.0, max_tokens=1 << 30))
+                seq = Sequence(rid, toks if type(toks) is list else list(toks),
+                               SamplingParams(temperature=0.0, max_tokens=1 << 30))     # (copies them)
                 sched.admit_given(seq)
             else:
                 for t in toks:

@@ -96,41 +96,31 @@ class _Uploader:
         self.k = 0
 
     def __call__(self, arrays):
-        arrs = [np.ascontiguousarray(a) for a in arrays]
-        offs, cut, n = [], [], 0              # (cut: field, gap, field, gap, ..)
-        for a in arrs:
-            if a.dtype.itemsize not in (4, 8):
-                raise TypeError(f"upload: unsupported dtype {a.dtype}")
-            offs.append(n)
-            w = a.nbytes // 4
-            gap = -w % self.ALIGN
-            cut += (w, gap)
-            n += w + gap
-        if n < self.ALIGN:
-            cut += (0, self.ALIGN - n)
-            n = self.ALIGN
+        arrs = list(arrays)
         k = self.k
         self.k ^= 1
         if self.events[k] is not None:
             self.events[k].synchronize()
-        if self.host[k].numel() < n:
+        n, offs = rt().pack_words(arrs, self.words[k], self.ALIGN)
+        if n > self.words[k].size:
             self.host[k] = torch.zeros(2 * n, dtype=torch.int32, pin_memory=self.pin)
             self.words[k] = self.host[k].numpy()
+            n, offs = rt().pack_words(arrs, self.words[k], self.ALIGN)
         if self.dev.numel() < n:
             # the old buffer may still feed queued kernels: the caching allocator only
             # reuses its memory after the stream has passed this point
             self.dev = torch.zeros(2 * n, dtype=torch.int32, device=self.device)
-        hw = self.words[k]
-        for a, o, w in zip(arrs, offs, cut[::2]):
-            hw[o:o + w] = a.reshape(-1).view(np.int32)
         dev = self.dev[:n]
         dev.copy_(self.host[k][:n], non_blocking=True)
         if self.pin:
             ev = self.events[k] or torch.cuda.Event()
             ev.record()
             self.events[k] = ev
+        if dev.is_cuda:
+            return ops.native().cut_words(dev, offs, arrs)
         outs = []
-        for a, v in zip(arrs, dev.split(cut)[::2]):
+        for a, o in zip(arrs, offs):
+            v = dev[o:o + a.nbytes // 4]
             if a.dtype.itemsize == 8:
                 v = v.view(torch.int64 if a.dtype.kind in "iu" else torch.float64)
             elif a.dtype == np.float32:
@@ -555,62 +545,16 @@ class ModelRunner:
         starts = [a for a, n in zip(batch.prefill_start or [None] * len(batch.prefill_seqs),
                                     batch.prefill_tokens) if n > 0]
         psamp = [sm for sm, n in zip(batch.prefill_sample, batch.prefill_tokens) if n > 0]
-        bs = self.bs
         nd = len(dseqs)
-        ids, pos, slots = [], [], []
-        host: Dict[str, object] = {"nd": nd}
-        # decode rows
-        if nd:
-            d_ids = np.empty(nd, np.int32)
-            d_pos = np.empty(nd, np.int32)
-            d_slot = np.empty(nd, np.int32)
-            d_bt = np.zeros((nd, max(len(s.block_ids) for s in dseqs)), np.int32)
-            for i, s in enumerate(dseqs):
-                p = s.n_tokens - 1 + s.inflight   # queued ahead: ids come from the device
-                d_ids[i] = s.last_token
-                d_pos[i] = p
-                d_slot[i] = s.block_ids[p // bs] * bs + p % bs
-                d_bt[i, : len(s.block_ids)] = s.block_ids
-            ids.append(d_ids)
-            pos.append(d_pos)
-            slots.append(d_slot)
-            host["d_bt"] = d_bt
-            host["d_sl"] = d_pos + 1
-        # prefill rows
-        seq_lens = np.empty(len(pseqs), np.int32)
-        qsl = np.zeros(len(pseqs) + 1, np.int32)
-        maxb = max([len(s.block_ids) for s in pseqs] or [1])
-        bt = np.zeros((max(1, len(pseqs)), maxb), np.int32)
-        for i, (s, n, a) in enumerate(zip(pseqs, ntoks, starts)):
-            if a is None:
-                a = s.num_computed
-            ids.append(s.tokens[a:a + n])
-            p = np.arange(a, a + n, dtype=np.int32)
-            pos.append(p)
-            blk = np.asarray(s.block_ids, dtype=np.int32)
-            bt[i, : len(blk)] = blk
-            slots.append(blk[p // bs] * bs + p % bs)
-            seq_lens[i] = a + n
-            qsl[i + 1] = qsl[i] + n
+        # rows, block tables and (models with state) one segment per scheduled sequence, decode rows first
+        host: Dict[str, object] = rt().mixed_rows(list(dseqs), pseqs, ntoks, starts or [None] * len(pseqs), self.bs,
+                                                  bool(self.stateful))
+        host["nd"] = nd
+        qsl = host["qsl"]
         if self.stateful:
             tiles, combine = [], []
-            # one segment per scheduled sequence, decode rows first (ops.mixers.Segments)
-            ns = nd + len(pseqs)
-            sg_bt = np.zeros((max(1, ns), max([len(s.block_ids) for s in dseqs + pseqs] or [1])),
-                             np.int32)
-            for i, s in enumerate(dseqs + pseqs):
-                sg_bt[i, : len(s.block_ids)] = s.block_ids
-            d_pos0 = pos[0] if nd else np.zeros(0, np.int32)
-            p_pos0 = np.asarray([seq_lens[i] - ntoks[i] for i in range(len(pseqs))], np.int32)
-            host.update(
-                sg_start=np.concatenate([np.arange(nd, dtype=np.int32), nd + qsl]).astype(np.int32),
-                sg_pos0=np.concatenate([d_pos0, p_pos0]).astype(np.int32),
-                sg_slot=np.asarray([s.state_slot for s in dseqs + pseqs] or [0], np.int32),
-                sg_len=np.concatenate([d_pos0 + 1, seq_lens]).astype(np.int32) if ns
-                else np.zeros(1, np.int32),
-                sg_bt=sg_bt, num_segs=ns, max_rows=max([1] * bool(nd) + ntoks + [0]),
-                max_kv=int(max([0] + [int(x) for x in d_pos0 + 1] + [int(x) for x in seq_lens])))
         else:
+            seq_lens = host["seq_lens"]
             tiles, combine = ops.build_prefill_tiles(
                 ntoks, ops.prefill_tile_tokens(self.attn_dims[0], self.attn_dims[1]),
                 seq_lens=seq_lens if self.pf_part_o is not None else None, nkv=self.attn_dims[1],
@@ -620,9 +564,7 @@ class ModelRunner:
         lrows = list(range(nd)) + [nd + int(qsl[i + 1]) - 1 for i, sm in enumerate(psamp) if sm]
         if batch.logit_rows is not None:
             lrows = list(batch.logit_rows)
-        host.update(ids=np.concatenate(ids).astype(np.int32), pos=np.concatenate(pos).astype(np.int32),
-                    slots=np.concatenate(slots).astype(np.int32), lrows=np.asarray(lrows, np.int64),
-                    bt=bt, seq_lens=seq_lens, qsl=qsl, tiles=np.asarray(tiles, np.int32).reshape(-1),
+        host.update(lrows=np.asarray(lrows, np.int64), tiles=np.asarray(tiles, np.int32).reshape(-1),
                     num_tiles=len(tiles), combine=np.asarray(combine, np.int32).reshape(-1),
                     num_combine=len(combine),
                     num_partials=sum(c[3] for c in combine))

@@ -8,6 +8,7 @@ from typing import Any, Callable, List, Optional
 
 import numpy as np
 
+from ..runtime import rt
 from .sampling_params import SamplingParams
 
 
@@ -48,7 +49,10 @@ class Sequence:
         self.prompt_len = len(prompt_ids)
         cap = max(64, len(prompt_ids) + min(params.max_tokens, 4096) + 1)
         self._tok = np.zeros(cap, dtype=np.int32)
-        self._tok[: len(prompt_ids)] = prompt_ids
+        if type(prompt_ids) is list:
+            rt().fill_ids(self._tok, prompt_ids)
+        else:
+            self._tok[: len(prompt_ids)] = prompt_ids
         self.n_tokens = len(prompt_ids)
         self.status = SeqStatus.WAITING
         self.block_ids: List[int] = []
