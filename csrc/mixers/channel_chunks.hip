@@ -112,7 +112,7 @@ channel_prep_kernel(float* __restrict__ ws_p, float* __restrict__ ws_q, float* _
     const float rate = R == kDelta ? expf(in.a_log[h]) : 0.f;
     auto decay = [&](float z, int i) {
       if constexpr (R == kReady) return z;
-      else if constexpr (R == kDelta) return expf(-rate * softplusf_(z + bias[i]));
+      else if constexpr (R == kDelta) return delta_decay(z + bias[i], rate);
       else return gla_decay(z + bias[i], in.inv_tau);
     };
     auto unit = [](float square) { return 1.0f / sqrtf(square + 1e-6f); };

@@ -96,6 +96,24 @@ __device__ __forceinline__ float gla_decay(float z, float inv_tau) {
   return __expf(-sp * inv_tau);
 }
 
+// exp(-rate softplus(z)) on the hardware's exp2 and log2, a third of the instructions of the library's expf and log1pf and nearer:
+// softplus(z) = max(z, 0) + log(1 + e), e = exp(-|z|), with what 1 + e drops of e added back; what the roundings of that sum and of
+// the products with rate and log2 e drop goes into the result at the end.  Largest and mean error in units in the last place, z in
+// -12 .. 12, rate in e^-3 .. e^3: 46 and 0.6 (library: 138 and 2.4).  channel_prep, 4096 rows of 16 heads of 128: 134 us and now 109.
+__device__ __forceinline__ float delta_decay(float z, float rate) {
+  constexpr float kL = 1.4426950408889634f, kLo = 1.925963033500e-8f, kLn2 = 0.6931471805599453f;
+  const float e = __builtin_amdgcn_exp2f(-kL * fabsf(z)), u = 1.0f + e, m = fmaxf(z, 0.0f);
+  const float l = fmaf(__builtin_amdgcn_logf(u), kLn2, (e - (u - 1.0f)) * __builtin_amdgcn_rcpf(u));
+  const float sp = m + l;
+  float y = rate * sp, low = fmaf(rate, sp, -y) + rate * (l - (sp - m));
+  if (!(y <= 200.0f)) y = y > 200.0f ? 200.0f : y, low = 0.f;          // (a NaN stays one)
+  const float t = y * -kL;
+  low = fmaf(y, -kLo, fmaf(y, -kL, -t)) - kL * low;
+  const int down = t < -100.0f ? 64 : 0;            // (exp2 has no denormal results)
+  const float r = __builtin_amdgcn_exp2f(t + (float)down);
+  return ldexpf(fmaf(r * kLn2, low, r), -down);
+}
+
 // tanh without branches: the Taylor polynomial up to |x| = 1/4, (1 - e^-2|x|) / (1 + e^-2|x|) beyond
 __device__ __forceinline__ float tanh_(float x) {
   const float a = fabsf(x), q = a * a;
