@@ -146,6 +146,11 @@ int mx_ssd_scan(float* y, const void* xbc, int bf16, long x_stride, const void* 
                 const float* a_log, const float* dt_bias, const float* d_skip, float* state, const int* start,
                 const int* pos0, const int* slot, int num_segs, int heads, int groups, int n, int dv, int num_slots,
                 int skip_from, hipStream_t s);
+int mx_state_scan_takes(const void* y, const void* xbc, int bf16, long stride, int heads, int groups, int n, int dv, int max_rows);
+int mx_state_scan_floats();
+int mx_state_scan(float* y, float* ws, const void* xbc, long stride, const void* dt, long dt_stride, const float* a_log, const float* dt_bias,
+                  const float* d_skip, float* state, long rows, const int* start, const int* pos0, const int* slot, int num_segs,
+                  int max_rows, int heads, int groups, int n, int dv, int num_slots, int min_rows, hipStream_t s);
 int mx_ssd_chunks(float* y, const void* xbc, int bf16, long stride, const void* dt, long dt_stride, const float* a_log,
                   const float* dt_bias, const float* d_skip, float* state, float* ws_s, float* ws_g, float* ws_h,
                   long rows, const int* start, const int* pos0, const int* slot, int num_segs, int max_rows, int heads,
@@ -1506,6 +1511,13 @@ void diff_combine(Tensor out, Tensor a, Tensor gate, double lam, double post, do
                       (int)heads, (int)dv, (float)lam, (float)post, (float)eps, stream()), "diff_combine");
 }
 
+// whether ssd_scan takes these rows' long segments in state_scan.hip's chunks
+bool state_scan_takes(Tensor y, Tensor xbc, int64_t heads, int64_t groups, int64_t n, int64_t dv, int64_t max_rows) {
+  return xbc.is_cuda() && y.is_cuda() && xbc.dim() == 2 && xbc.stride(1) == 1 && y.scalar_type() == at::kFloat &&
+         mx_state_scan_takes(y.data_ptr(), xbc.data_ptr(), bf(xbc), xbc.stride(0), (int)heads, (int)groups, (int)n, (int)dv,
+                             (int)std::min(max_rows, xbc.size(0)));
+}
+
 void ssd_scan(Tensor y, Tensor xbc, Tensor dt, Tensor a_log, Tensor dt_bias, Tensor d_skip, Tensor state,
               Tensor start, Tensor pos0, Tensor slot, int64_t num_segs, int64_t max_rows, int64_t heads, int64_t groups,
               int64_t n, int64_t dv, bool walk, int64_t chunk_from) {
@@ -1545,6 +1557,15 @@ void ssd_scan(Tensor y, Tensor xbc, Tensor dt, Tensor a_log, Tensor dt_bias, Ten
                     (int)num_segs, (int)heads, (int)groups, (int)n, (int)dv, (int)state.size(0),
                     chunks ? (int)chunk_from : 0, stream()), "ssd_scan");
   if (!chunks) return;
+  if (mx_state_scan_takes(y.data_ptr<float>(), xbc.data_ptr(), bf(xbc), xbc.stride(0), (int)heads, (int)groups, (int)n, (int)dv,
+                          (int)max_rows)) {
+    Tensor ws = at::empty({chunk_bound(t, num_segs) * heads * mx_state_scan_floats()}, y.options());
+    chk(mx_state_scan(y.data_ptr<float>(), ws.data_ptr<float>(), xbc.data_ptr(), xbc.stride(0), dt.data_ptr(), dt.stride(0), a_log.data_ptr<float>(),
+                      dt_bias.data_ptr<float>(), d_skip.data_ptr<float>(), state.data_ptr<float>(), t, start.data_ptr<int>(),
+                      pos0.data_ptr<int>(), slot.data_ptr<int>(), (int)num_segs, (int)max_rows, (int)heads, (int)groups, (int)n,
+                      (int)dv, (int)state.size(0), (int)chunk_from, stream()), "state-space scan in chunks");
+    return;
+  }
   const int64_t nc = chunk_bound(t, num_segs);
   Tensor ws_s = at::empty({nc, heads, n, dv}, y.options()), ws_g = at::empty({nc, heads}, y.options());
   Tensor ws_h = at::empty({2, t, heads}, y.options());
@@ -1824,6 +1845,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   });
   m.def("diff_combine", &diff_combine);
   m.def("ssd_scan", &ssd_scan);
+  m.def("state_scan_takes", &state_scan_takes);
   m.def("gate_group_norm", &gate_group_norm);
   m.def("window_max_dv", []() { return (int64_t)mx_window_max_dv(); });
   m.def("ssd_max_state", []() { return (int64_t)mx_ssd_max_state(); });

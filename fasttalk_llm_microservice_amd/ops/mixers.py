@@ -540,6 +540,9 @@ CHUNK_ROWS = 32
 # 245), state space 40 41 46 98 (19 28 49 169; four segments of 200: 108, walk 97)
 CHANNEL_CHUNK_ROWS = 96
 SSD_CHUNK_ROWS = 256
+# of the state-space scan where its chunks take one launch for the weights and one for the walk over them (csrc/mixers/state_scan.hip):
+# us, 32 heads of 128 x 128, a row at a time beside it: one segment of 40 rows 14 16, of 64 12 18, eight of 40 40 49, 64 of 33 244 264
+SCAN_ROWS = 64
 NO_CHUNKS = 1 << 30
 
 
@@ -896,7 +899,10 @@ def ssd_scan(xbc, dt, a_log, dt_bias, d_skip, state, seg: Segments, heads: int, 
     position 0) and left at the segment's last row.  Returns y fp32 [T, heads*dv]."""
     if xbc.is_cuda:
         y = torch.empty(xbc.shape[0], heads * dv, dtype=torch.float32, device=xbc.device)
-        chunk = SSD_CHUNK_ROWS if _ssd_chunks_pay(seg, heads, n, dv) else NO_CHUNKS
+        if native_mixers().state_scan_takes(y, xbc, heads, groups, n, dv, seg.max_rows):
+            chunk = SCAN_ROWS
+        else:
+            chunk = SSD_CHUNK_ROWS if _ssd_chunks_pay(seg, heads, n, dv) else NO_CHUNKS
         native_mixers().ssd_scan(y, xbc, dt, a_log, dt_bias, d_skip, state, seg.start, seg.pos0, seg.slot,
                                  seg.num, seg.max_rows, heads, groups, n, dv, _walk_below(seg, chunk), chunk)
         return y

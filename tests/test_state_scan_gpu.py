@@ -1,0 +1,77 @@
+"""The state-space scan's chunks on the bf16 matrix units (csrc/mixers/state_scan.hip) against the recurrence in 64 bits: chunk
+edges, segments beside each other and beside short ones, states that go on, padding segments, decays from none to all."""
+import pytest
+import torch
+
+from fasttalk_llm_microservice_amd.ops import mixers as M
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+N = 128
+
+
+def case(lens, heads, groups, dv, seed=0, shift=-3.0, wide=0):
+    g = torch.Generator(device=DEV).manual_seed(seed + sum(lens))
+    rnd = lambda *s: torch.randn(*s, generator=g, device=DEV)   # noqa: E731
+    t, width = sum(lens), heads * dv + 2 * groups * N
+    xbc = (rnd(t, width + wide) * 0.7).bfloat16()[:, :width]
+    return (xbc, rnd(t, heads + 3).bfloat16()[:, :heads], rnd(heads).abs(), rnd(heads) + shift, rnd(heads),
+            rnd(len(lens), heads, N, dv))
+
+
+def reference(xbc, dt, a_log, dt_bias, skip, state, lens, pos, heads, groups, dv):
+    t = xbc.shape[0]
+    x, b, c = xbc.double().split([heads * dv, groups * N, groups * N], 1)
+    x, (b, c) = x.view(t, heads, dv), (z.view(t, groups, N).repeat_interleave(heads // groups, 1) for z in (b, c))
+    step = torch.nn.functional.softplus(dt.double() + dt_bias.double())
+    decay = torch.exp(-torch.exp(a_log.double()) * step)
+    y, out, size, r = torch.zeros(t, heads, dv, dtype=torch.float64, device=DEV), [], 0.0, 0
+    for i, n in enumerate(lens):
+        s = state[i].double() * (pos[i] > 0)
+        for k in range(r, r + n):
+            s = s * decay[k][:, None, None] + b[k][:, :, None] * (step[k][:, None] * x[k])[:, None]
+            y[k] = torch.einsum("hnv,hn->hv", s, c[k]) + skip.double()[:, None] * x[k]
+        r += n
+        size = max(size, float(s.abs().max()))
+        out.append(s)
+    return y.reshape(t, -1), torch.stack(out), size
+
+
+def run(args, lens, pos, heads, groups, dv, slots=None, least=64):
+    xbc, dt, a_log, dt_bias, skip, state = args
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)   # noqa: E731
+    start = [sum(lens[:i]) for i in range(len(lens) + 1)]
+    y, state = torch.full((xbc.shape[0], heads * dv), 7.0, device=DEV), state.clone()
+    assert M.native_mixers().state_scan_takes(y, xbc, heads, groups, N, dv, max(lens))
+    M.native_mixers().ssd_scan(y, xbc, dt, a_log, dt_bias, skip, state, i32(start), i32(pos), i32(slots or list(range(len(lens)))),
+                               len(lens), max(lens), heads, groups, N, dv, min(lens) < least, least)
+    return y, state
+
+
+@pytest.mark.parametrize("lens,pos", [([64], [0]), ([65], [5]), ([127, 128, 129], [0, 3, 0]), ([1000], [9]), ([64, 1, 40, 200, 1], [0, 7, 0, 1, 2]),
+                                      ([192], [0]), ([257, 80], [4, 0])])
+@pytest.mark.parametrize("heads,groups,dv", [(4, 2, 16), (2, 1, 48), (3, 3, 128)])
+@pytest.mark.parametrize("shift", [-3.0, 3.0, -30.0])
+def test_rows(lens, pos, heads, groups, dv, shift):
+    """(a shift of 3: most decays are below e^-3; of -30: nothing decays and nothing is added)"""
+    args = case(lens, heads, groups, dv, shift=shift, wide=8)
+    y, state = run(args, lens, pos, heads, groups, dv)
+    want, left, size = reference(*args, lens, pos, heads, groups, dv)
+    # fp32 sums of 128 products with the state and up to 64 with pair weights, each of them exact to 2^-24 of its size
+    bound = 2.0 ** -21 * (size * 128 ** 0.5 * 4 + float(want.abs().max()))
+    assert float((y.double() - want).abs().max()) <= bound
+    assert float((state.double() - left).abs().max()) <= 2.0 ** -21 * max(size, 1.0)
+
+
+def test_padding_segments_and_infinite_rows():
+    heads, groups, dv, lens = 4, 2, 32, [100, 70, 130]
+    args = case(lens, heads, groups, dv)
+    good, states = run(args, lens, [0, 0, 0], heads, groups, dv)
+    y, left = run(args, lens, [0, 0, 0], heads, groups, dv, slots=[0, -1, 2])
+    assert torch.equal(y[:100], good[:100]) and torch.equal(y[170:], good[170:]) and bool((y[100:170] == 0).all())
+    assert torch.equal(left[1], args[5][1]) and torch.equal(left[0], states[0])
+    # rows before an infinite one do not see it, nor do other segments and heads
+    args[0][100 + 16, 5] = float("inf")
+    y, _ = run(args, lens, [0, 0, 0], heads, groups, dv)
+    assert torch.equal(y[:116], good[:116]) and torch.equal(y[170:], good[170:])
+    assert torch.equal(y[:, dv:], good[:, dv:]) and not bool(torch.isfinite(y[116:170, 5]).any())
