@@ -51,6 +51,7 @@ int ft_w4_gemm_xr(const void* x, int x_stride, int M, const uint32_t* wq, const 
 int ft_w4_gemm_mh(const void* x, int x_stride, int M, const uint32_t* wq, const void* sz, int N, int K,
                   float* ws, void* out, int out_stride, int splits, int ring, int silu,
                   hipStream_t stream);
+int ft_host_copy(void* dst, const void* src, long words, hipStream_t stream);
 int ft_kv_swap(const uint64_t* ptrs_dev, int ncache, const int* ids_dev, int n, void* staging,
                long block_elems, int to_staging, int num_blocks, hipStream_t stream);
 int ft_skinny_gemm_xc(const void* x, int x_stride, int M, const void* w, int N, int K, float* ws,
@@ -902,6 +903,20 @@ void set_kernel_checks(torch::Tensor word) {
 }
 #endif
 
+// dst = src, one of them on the device and the other in pinned host memory that outlives the copy (ordered on the current stream)
+void host_copy(at::Tensor dst, at::Tensor src) {
+  TORCH_CHECK(dst.is_contiguous() && src.is_contiguous() && dst.scalar_type() == src.scalar_type() && dst.numel() == src.numel() &&
+              src.element_size() % 4 == 0 && dst.is_cuda() != src.is_cuda(), "host_copy: alike, contiguous, words");
+  if (src.numel() == 0) return;
+  hipPointerAttribute_t attr{};
+  void* host = dst.is_cuda() ? src.data_ptr() : dst.data_ptr();
+  const bool pinned = hipPointerGetAttributes(&attr, host) == hipSuccess && attr.type == hipMemoryTypeHost && attr.devicePointer != nullptr;
+  if (!pinned) (void)hipGetLastError();
+  TORCH_CHECK(pinned, "host_copy: pinned host memory");
+  check_rc(ft_host_copy(dst.is_cuda() ? dst.data_ptr() : attr.devicePointer, src.is_cuda() ? src.data_ptr() : attr.devicePointer,
+                        src.numel() * (src.element_size() / 4), cur_stream()), "host_copy");
+}
+
 // Views of an int32 image on the device in the types and shapes of the host arrays that were packed into it, array i from word
 // offs[i] on (a step's twelve to twenty take 6 us so, 16 as calls from Python).
 std::vector<at::Tensor> cut_words(at::Tensor image, std::vector<int64_t> offs, py::list arrays) {
@@ -934,6 +949,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.attr("kernel_checks") = false;
 #endif
   m.def("cut_words", &cut_words);
+  m.def("host_copy", &host_copy);
   m.def("rmsnorm", &rmsnorm);
   m.def("fused_add_rmsnorm", &fused_add_rmsnorm);
   m.def("silu_mul", &silu_mul);

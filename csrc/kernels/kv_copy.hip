@@ -72,5 +72,34 @@ extern "C" int ft_kv_swap(const uint64_t* ptrs_dev, int ncache, const int* ids_d
   return static_cast<int>(hipGetLastError());
 }
 
+// A step's inputs from pinned host memory, or its results into it, by a kernel over the link: `words` of 4 bytes.  Bound by the link's
+// latency and, from a few hundred KB on, its rate.  A runtime copy of this size is a launch of its own kind, and the queue
+// passes from it to a graph and back only after 6 to 11 us: a decode step's 16 to 130 KB cost 13 to 16 us less so.
+namespace ft {
+
+__global__ __launch_bounds__(256) void host_copy_kernel(uint32_t* __restrict__ dst, const uint32_t* __restrict__ src, long words,
+                                                        int vec) {
+  const long at = blockIdx.x * 256L + threadIdx.x, step = gridDim.x * 256L;
+  if (vec) {
+    for (long i = at; i < words / 4; i += step)
+      reinterpret_cast<uint4*>(dst)[i] = reinterpret_cast<const uint4*>(src)[i];
+    if (at < words % 4) dst[words / 4 * 4 + at] = src[words / 4 * 4 + at];
+  } else {
+    for (long i = at; i < words; i += step) dst[i] = src[i];
+  }
+}
+
+}  // namespace ft
+
+extern "C" int ft_host_copy(void* dst, const void* src, long words, hipStream_t stream) {
+  if (words <= 0) return 0;
+  if (((uintptr_t)dst | (uintptr_t)src) % 4) return -1;
+  const int vec = ((uintptr_t)dst | (uintptr_t)src) % 16 == 0;
+  const long groups = (words / (vec ? 4 : 1) + 255) / 256;
+  hipLaunchKernelGGL(ft::host_copy_kernel, dim3((unsigned)(groups < 1 ? 1 : groups > 256 ? 256 : groups)), dim3(256), 0, stream,
+                     (uint32_t*)dst, (const uint32_t*)src, words, vec);
+  return static_cast<int>(hipGetLastError());
+}
+
 // checked build: this unit's error-word / limits hook (ft_common.h)
 FT_CHECK_HOOK(kv_copy)

@@ -37,11 +37,60 @@ constexpr int kFrStage = NB * 16 * kFrRow<U>;
 
 // acc[t][b] += W rows of tile t times X rows of block b, over this wave's share of k.  wp: the lane's
 // row of each tile; xrow(r): row r < rows of X; stage: this wave's kFrStage bytes.  All pieces are 16
-// bytes (K a multiple of 8); those past the wave's share count as zeros.  AHEAD: a round's loads are in
-// flight under the products of the one before, for workgroups that have a CU to themselves.
-template <int NT, int NB, int WV, int U, bool AHEAD = false, typename XR>
+// bytes (K a multiple of 8); those past the wave's share count as zeros.
+template <int NT, int NB, int WV, int U, typename XR>
 __device__ __forceinline__ void few_rows_core(fr_f32x4 (&acc)[NT][NB], const bf16_t* const (&wp)[NT], XR xrow, int rows,
                                               int K, char* stage, int wave, int lane) {
+  constexpr int LPR = U * 8, RPI = 64 / LPR, XI = NB * 16 / RPI;   // lanes a row, rows a load, loads a round
+  const int n = lane & 15, q = lane >> 4;
+  const int per = (((K + 63) >> 6) + WV - 1) / WV * 64;
+  const int kend = min((wave + 1) * per, K);
+  const int sr = lane / LPR, sk = (lane % LPR) * 8;
+  for (int k0 = wave * per; k0 < kend; k0 += 64 * U) {
+    uint4 x[XI], w[U][NT][2];
+#pragma unroll
+    for (int i = 0; i < XI; ++i) {
+      const int r = i * RPI + sr;
+      x[i] = uint4{0, 0, 0, 0};
+      if (r < rows && k0 + sk < kend) x[i] = *reinterpret_cast<const uint4*>(xrow(r) + k0 + sk);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const int k = k0 + 64 * u + 16 * q + 8 * j;
+          w[u][t][j] = uint4{0, 0, 0, 0};
+          if (k < kend) w[u][t][j] = *reinterpret_cast<const uint4*>(wp[t] + k);
+        }
+    wave_lds_fence();                            // the last round's operands have been read
+#pragma unroll
+    for (int i = 0; i < XI; ++i) {
+      const int r = i * RPI + sr;
+      if (r < rows) *reinterpret_cast<uint4*>(stage + r * kFrRow<U> + sk * 2) = x[i];
+    }
+    wave_lds_fence();
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        uint4 xb[NB];
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+          xb[b] = *reinterpret_cast<const uint4*>(stage + (16 * b + n) * kFrRow<U> + u * 128 + q * 32 + j * 16);
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+          for (int b = 0; b < NB; ++b) acc[t][b] = fr_mfma(w[u][t][j], xb[b], acc[t][b]);
+      }
+  }
+}
+
+// The same with a round's loads in flight under the products of the one before, for workgroups that have a CU to themselves.
+template <int NT, int NB, int WV, int U, typename XR>
+__device__ __forceinline__ void few_rows_core_ahead(fr_f32x4 (&acc)[NT][NB], const bf16_t* const (&wp)[NT], XR xrow, int rows,
+                                                    int K, char* stage, int wave, int lane) {
   constexpr int LPR = U * 8, RPI = 64 / LPR, XI = NB * 16 / RPI;   // lanes a row, rows a load, loads a round
   const int n = lane & 15, q = lane >> 4;
   const int per = (((K + 63) >> 6) + WV - 1) / WV * 64;
@@ -66,9 +115,8 @@ __device__ __forceinline__ void few_rows_core(fr_f32x4 (&acc)[NT][NB], const bf1
           if (k < kend) w[u][t][j] = *reinterpret_cast<const uint4*>(wp[t] + k);
         }
   };
-  if constexpr (AHEAD) fetch(wave * per);
+  fetch(wave * per);
   for (int k0 = wave * per; k0 < kend; k0 += 64 * U) {
-    if constexpr (!AHEAD) fetch(k0);
     wave_lds_fence();                            // the last round's operands have been read
 #pragma unroll
     for (int i = 0; i < XI; ++i) {
@@ -82,9 +130,7 @@ __device__ __forceinline__ void few_rows_core(fr_f32x4 (&acc)[NT][NB], const bf1
       for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int j = 0; j < 2; ++j) now[u][t][j] = w[u][t][j];
-    if constexpr (AHEAD) {
-      if (k0 + 64 * U < kend) fetch(k0 + 64 * U);
-    }
+    if (k0 + 64 * U < kend) fetch(k0 + 64 * U);
     wave_lds_fence();
 #pragma unroll
     for (int u = 0; u < U; ++u)

@@ -204,8 +204,10 @@ __device__ __forceinline__ void expert_tile(float4* red, const bf16_t* W, int N,
   for (int t = 0; t < NT; ++t)
 #pragma unroll
     for (int b = 0; b < NB; ++b) acc[t][b] = fr_f32x4{0.f, 0.f, 0.f, 0.f};
-  few_rows_core<NT, NB, WV, U, AHEAD>(acc, wp, [&](int r) { return X + (long)(list[r] / div) * x_stride; }, count, K,
-                               reinterpret_cast<char*>(red) + wave * kFrStage<NB, U>, wave, lane);
+  const auto row = [&](int r) { return X + (long)(list[r] / div) * x_stride; };
+  char* const stage = reinterpret_cast<char*>(red) + wave * kFrStage<NB, U>;
+  if constexpr (AHEAD) few_rows_core_ahead<NT, NB, WV, U>(acc, wp, row, count, K, stage, wave, lane);
+  else few_rows_core<NT, NB, WV, U>(acc, wp, row, count, K, stage, wave, lane);
   __syncthreads();
   few_rows_park<NT, NB, WV>(red, acc, wave, lane);
   __syncthreads();

@@ -76,6 +76,15 @@ def _input_views(buf: torch.Tensor, mb: int, max_blocks: int):
             buf[12 * mb:].view(mb, max_blocks))
 
 
+def _copy(dst: torch.Tensor, src: torch.Tensor, pinned: bool):
+    """Queues a copy between the device and host memory, which stays until the stream has passed it; ``pinned``: by a kernel,
+    which a graph's first launch follows at once."""
+    if pinned:
+        ops.native().host_copy(dst, src)
+    else:
+        dst.copy_(src, non_blocking=True)
+
+
 class _Uploader:
     """Eager (mixed decode + prefill) step inputs in ONE host -> device copy: the
     numpy arrays are packed into a pinned int32 image (64-B aligned fields, int64
@@ -111,7 +120,7 @@ class _Uploader:
             # reuses its memory after the stream has passed this point
             self.dev = torch.zeros(2 * n, dtype=torch.int32, device=self.device)
         dev = self.dev[:n]
-        dev.copy_(self.host[k][:n], non_blocking=True)
+        _copy(dev, self.host[k][:n], self.pin)
         if self.pin:
             ev = self.events[k] or torch.cuda.Event()
             ev.record()
@@ -638,7 +647,7 @@ class ModelRunner:
             if not self.is_gpu:
                 return logits.numpy()
             out = torch.empty(logits.shape, dtype=torch.float32, pin_memory=True)
-            out.copy_(logits, non_blocking=True)
+            _copy(out, logits.contiguous(), True)
             self._wait()
             return out.numpy()
         if not has_logits:
@@ -1101,7 +1110,7 @@ class ModelRunner:
         nw = IN_HEAD * self.max_decode_batch + nb * self.max_blocks_per_seq
         if self._gaps is not None:   # g: a split step, closed by its sampler (sample_launch)
             self._gap_mark(True, "g" if fwd_only else "d")
-        self.d_in[:nw].copy_(st.h_in[:nw], non_blocking=True)
+        _copy(self.d_in[:nw], st.h_in[:nw], self.is_gpu)
         if from_device:  # the previous step's sampled ids feed this step
             if gather is None:
                 self.d_input_ids[:nb].copy_(self.d_out[:nb])
