@@ -22,6 +22,10 @@ int mx_few_rows_pair(void* Y, void* Y2, long y_stride, const void* X, const void
 int mx_few_rows_side_gate(void* Y, long y_stride, const void* X, long x_stride, int rows, const void* W, int N, int K,
                           const void* table, long table_stride, const int* ids, int vocab, hipStream_t s);
 int mx_head_product_fits(int K, int N);
+int mx_head_tiles_fits(int K, int N);
+int mx_latent_q_tiles(float*, float*, const void*, int, long, const void*, const float*, int, int, const int*, int, int, int, int, int,
+                      int, hipStream_t);
+int mx_head_values_tiles(void*, int, const float*, const void*, const void*, long, int, int, int, int, hipStream_t);
 int mx_latent_q_absorb(float* qa, float* qr, const void* q, int bf16, long stride, const float* wuk, const float* table,
                        int table_rows, int dims, const int* positions, int rows, int heads, int K, int N, int dr,
                        int interleaved, hipStream_t s);
@@ -1732,46 +1736,67 @@ void heads_to_rows(const Tensor& out, const Tensor& o, const OptT& inv, const Op
 void scaled_heads_gate(Tensor out, Tensor o, Tensor inv, OptT gate) { heads_to_rows(out, o, inv, gate, false); }
 void head_gate(Tensor out, Tensor o, Tensor gate) { heads_to_rows(out, o, {}, gate, true); }
 
+bool head_tiles_fits(int64_t k, int64_t n) { return mx_head_tiles_fits((int)k, (int)n) != 0; }
 bool head_product_fits(int64_t k, int64_t n) { return mx_head_product_fits((int)k, (int)n) != 0; }
 
-// few rows: latent_q_rope with its unrotated part taken through wuk [heads][dn][rank], fp32
+void check_head_weight(const Tensor& w, bool tiles) {
+  if (!tiles) {
+    check_f32(w, "head matrices");
+    TORCH_CHECK(w.dim() == 3 && head_product_fits(w.size(1), w.size(2)), "head matrices");
+    return;
+  }
+  TORCH_CHECK(w.is_cuda() && w.is_contiguous() && w.scalar_type() == at::kBFloat16 && w.dim() == 5 && w.size(3) == 2 &&
+              w.size(4) == 512, "head matrices in tiles");
+}
+
+// latent_q_rope with its unrotated part taken through wuk [heads][dn][rank]: few rows, and fp32; or (tiles) many rows, bf16 values in
+// head_tiles.hip's order, [heads][rank / 32][dn / 32][2][512]
 void latent_q_absorb(Tensor qa, Tensor qr, Tensor q, Tensor wuk, Tensor table, int64_t dims, Tensor positions, int64_t dr,
-                     bool interleaved) {
+                     bool interleaved, bool tiles) {
   check_f32(qa, "qa");
   check_f32(qr, "qr");
   check_rows(q, "q");
-  check_f32(wuk, "wuk");
   check_f32(table, "rope table");
   check_i32(positions, "positions");
-  TORCH_CHECK(wuk.dim() == 3 && head_product_fits(wuk.size(1), wuk.size(2)), "wuk");
-  const int64_t t = q.size(0), heads = wuk.size(0), dn = wuk.size(1), rank = wuk.size(2);
+  check_head_weight(wuk, tiles);
+  const int64_t t = q.size(0), heads = wuk.size(0), dn = tiles ? wuk.size(2) * 32 : wuk.size(1);
+  const int64_t rank = tiles ? wuk.size(1) * 32 : wuk.size(2);
   TORCH_CHECK(dr >= 0 && q.size(1) == heads * (dn + dr) && qa.numel() == heads * t * rank && qr.numel() == t * heads * dr &&
               dims % 2 == 0 && dims <= dr && table.dim() == 2 && table.size(1) == dims && positions.numel() >= t &&
               t <= 0x7fffffff, "latent_q_absorb shapes");
-  chk(mx_latent_q_absorb(qa.data_ptr<float>(), qr.data_ptr<float>(), q.data_ptr(), bf(q), q.stride(0), wuk.data_ptr<float>(),
-                         table.data_ptr<float>(), (int)table.size(0), (int)dims, positions.data_ptr<int>(), (int)t, (int)heads,
-                         (int)dn, (int)rank, (int)dr, interleaved ? 1 : 0, stream()), "latent_q_absorb");
+  const auto run = [&](auto f, auto w) {
+    chk(f(qa.data_ptr<float>(), qr.data_ptr<float>(), q.data_ptr(), bf(q), q.stride(0), w, table.data_ptr<float>(),
+          (int)table.size(0), (int)dims, positions.data_ptr<int>(), (int)t, (int)heads, (int)dn, (int)rank, (int)dr,
+          interleaved ? 1 : 0, stream()), "latent_q_absorb");
+  };
+  if (tiles) run(mx_latent_q_tiles, (const void*)wuk.data_ptr());
+  else run(mx_latent_q_absorb, (const float*)wuk.data_ptr<float>());
 }
 
-// few rows: o [heads][T][rank] through wuv [heads][rank][dv], gated per head, as rows
-void head_values(Tensor out, Tensor o, Tensor wuv, OptT gate) {
+// o [heads][T][rank] through wuv [heads][rank][dv] (tiles: as above, [heads][dv / 32][rank / 32][2][512]), gated per head, as rows
+void head_values(Tensor out, Tensor o, Tensor wuv, OptT gate, bool tiles) {
   check_f32(o, "o");
-  check_f32(wuv, "wuv");
-  TORCH_CHECK(o.dim() == 3 && wuv.dim() == 3 && wuv.size(0) == o.size(0) && wuv.size(1) == o.size(2) &&
-              head_product_fits(wuv.size(1), wuv.size(2)), "head_values: o / wuv");
-  const int64_t heads = o.size(0), t = o.size(1), dv = wuv.size(2);
+  check_head_weight(wuv, tiles);
+  TORCH_CHECK(o.dim() == 3 && wuv.size(0) == o.size(0) && (tiles ? wuv.size(2) * 32 : wuv.size(1)) == o.size(2),
+              "head_values: o / wuv");
+  const int64_t heads = o.size(0), t = o.size(1), dv = tiles ? wuv.size(1) * 32 : wuv.size(2);
   TORCH_CHECK(out.is_cuda() && out.is_contiguous() && is_act(out) && out.dim() == 2 && out.size(0) == t &&
               out.size(1) == heads * dv && t <= 0x7fffffff, "out");
   long gs = 0;
   const void* gp = gate_rows(gate, out, t, heads, &gs);
-  chk(mx_head_values(out.data_ptr(), bf(out), o.data_ptr<float>(), wuv.data_ptr<float>(), gp, gs, (int)t, (int)heads,
-                     (int)o.size(2), (int)dv, stream()), "head_values");
+  const auto run = [&](auto f, auto w) {
+    chk(f(out.data_ptr(), bf(out), o.data_ptr<float>(), w, gp, gs, (int)t, (int)heads, (int)o.size(2), (int)dv, stream()),
+        "head_values");
+  };
+  if (tiles) run(mx_head_values_tiles, (const void*)wuv.data_ptr());
+  else run(mx_head_values, (const float*)wuv.data_ptr<float>());
 }
 
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("head_product_fits", &head_product_fits);
+  m.def("head_tiles_fits", &head_tiles_fits);
   m.def("latent_q_absorb", &latent_q_absorb);
   m.def("head_values", &head_values);
   m.def("embed_rows", &embed_rows);

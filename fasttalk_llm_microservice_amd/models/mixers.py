@@ -101,6 +101,7 @@ class LatentAttention:
         self.wuk = get("uk").to(device, torch.float32).view(heads, dim, kv_rank).contiguous()
         self.wuvT = get("uv").to(device, torch.float32).view(heads, vdim, kv_rank) \
             .transpose(1, 2).contiguous()
+        self.wuk_tiles, self.wuvT_tiles = M.head_tiles(self.wuk), M.head_tiles(self.wuvT)
         self.wo = get("o").to(device, dtype).contiguous()
         self.table = M.rope_table(max_pos, rot_dims, rot_base, device=device)
 
@@ -129,7 +130,7 @@ class LatentAttention:
             M.latent_kv_write(dkv, self.dkv_norm, self.eps, self.table, self.rot_dims, ctx.positions,
                               ctx.slot_mapping, cache, self.rank, self.interleaved)
         qa, qr = M.latent_q_absorb(q, self.wuk, self.table, self.rot_dims, ctx.positions, self.heads, self.dn,
-                                   self.dr, self.interleaved)         # [heads, T, rank]
+                                   self.dr, self.interleaved, self.wuk_tiles)         # [heads, T, rank]
         seg = ctx.seg
         if seg.host is not None and seg.max_rows >= self.PRODUCT_ROWS:
             # prefill chunks in tiles; short segments and decode rows (if any) keep the per-row
@@ -142,7 +143,7 @@ class LatentAttention:
                                         self.PRODUCT_ROWS, self.dtype, self.sink)
         else:
             ol = M.latent_attention(qa, qr, cache, seg, self.scale, self.rank, sink=self.sink)
-        return M.linear(M.head_values(ol, self.wuvT, qd[:, self.n_down:] if self.gated else None, self.dtype), self.wo)
+        return M.linear(M.head_values(ol, self.wuvT, qd[:, self.n_down:] if self.gated else None, self.dtype, self.wuvT_tiles), self.wo)
 
 
 class ChannelDelta:

@@ -719,6 +719,11 @@ def latent_q_rope(q, table, rot_dims: int, positions, heads: int, dn: int, dr: i
 # rounding in the second): 16 heads, 128 -> 512 -> 128: 8 11 17 24 31 (library 23 23 22 22 22); 128 heads 15 22 36 52 65
 # (59 60 59 65 62); 40 heads, 64 -> 256 -> 64: 7 10 16 22 27 (19 20 20 22 22)
 HEAD_PRODUCT_ROWS = 16
+# rows from which the values' product goes through head_tiles.hip where the matrix allows it; the queries' always does.  us of
+# queries + values, 16 heads, 128 -> 512 -> 128, 1 4 8 16 64 rows: 2.9 + 4.7, 3.0 + 4.8, 3.2 + 4.9, 3.4 + 5.1, 4.8 + 6.1 (head_product.hip
+# 3.1 + 3.2, 3.8 + 4.4, 4.7 + 6.1, 7.4 + 10.2; library 10.6 + 20.1 at 64); 300 and 4096 rows 7.5 + 11 and 44 + 34 (library 17 + 14 and
+# 104 + 89)
+HEAD_TILES_ROWS = 5
 
 
 def _head_product(rows: int, w) -> bool:
@@ -727,27 +732,49 @@ def _head_product(rows: int, w) -> bool:
                 and w.data_ptr() % 16 == 0 and native_mixers().head_product_fits(w.shape[1], w.shape[2]))
 
 
-def latent_q_absorb(q, wuk, table, rot_dims: int, positions, heads: int, dn: int, dr: int, interleaved: bool = False):
+def head_tiles(w) -> Optional[torch.Tensor]:
+    """Matrices ``w`` fp32 [heads, K, N] in the order in which csrc/mixers/head_tiles.hip reads them, bf16 [heads, N / 32, K / 32,
+    2, 512], if that holds them: all values are finite bf16 ones (a bf16 checkpoint's); else None."""
+    if not w.is_cuda or w.dtype != torch.float32 or not native_mixers().head_tiles_fits(w.shape[1], w.shape[2]):
+        return None
+    b = w.to(torch.bfloat16)
+    if not bool(((b.float() == w) & w.isfinite()).all()):
+        return None
+    h, k, n = w.shape
+    # K = (step, hi, e), N = (pair, tile, lo): a lane (hi, lo) holds 8 entries of column lo of a tile
+    b = b.view(h, k // 32, 4, 8, n // 32, 2, 16).permute(0, 4, 1, 5, 2, 6, 3)
+    return b.reshape(h, n // 32, k // 32, 2, 512).contiguous()
+
+
+def latent_q_absorb(q, wuk, table, rot_dims: int, positions, heads: int, dn: int, dr: int, interleaved: bool = False,
+                    tiles: Optional[torch.Tensor] = None):
     """:func:`latent_q_rope` and the unrotated parts' way into latent space: (fp32 [heads, T, rank] = q W_uk per head, ``wuk``
-    fp32 [heads, dn, rank]; the rotated parts fp32 [T, heads, dr]).  One launch for few rows."""
+    fp32 [heads, dn, rank]; the rotated parts fp32 [T, heads, dr]).  One launch for few rows, and for all of them with ``tiles``
+    = :func:`head_tiles` of ``wuk``."""
     t = q.shape[0]
-    if _head_product(t, wuk) and q.stride(1) == 1 and q.stride(0) % 4 == 0 and (dn + dr) % 4 == 0 \
-            and q.data_ptr() % (4 * q.element_size()) == 0:
+
+    def reads(n):                                # whether q can be read n entries at a time
+        return q.stride(1) == 1 and q.stride(0) % n == 0 and (dn + dr) % n == 0 and q.data_ptr() % (n * q.element_size()) == 0
+
+    tiled = tiles is not None and reads(16 // q.element_size())
+    if tiled or (_head_product(t, wuk) and reads(4)):
         qa = torch.empty(heads, t, wuk.shape[2], dtype=torch.float32, device=q.device)
         qr = torch.empty(t, heads, dr, dtype=torch.float32, device=q.device)
-        native_mixers().latent_q_absorb(qa, qr, q, wuk, table, rot_dims, positions, dr, bool(interleaved))
+        native_mixers().latent_q_absorb(qa, qr, q, tiles if tiled else wuk, table, rot_dims, positions, dr, bool(interleaved), tiled)
         return qa, qr
     qn, qr = latent_q_rope(q, table, rot_dims, positions, heads, dn, dr, interleaved)
     return torch.bmm(qn.transpose(0, 1), wuk), qr
 
 
-def head_values(ol, wuv, gate, out_dtype) -> torch.Tensor:
+def head_values(ol, wuv, gate, out_dtype, tiles: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Latent-space sums ``ol`` fp32 [heads, T, rank] through ``wuv`` fp32 [heads, rank, dv], times sigmoid(gate[t, h]) if there
-    is a ``gate`` [T, heads], as rows [T, heads * dv] in ``out_dtype``.  One launch for few rows."""
+    is a ``gate`` [T, heads], as rows [T, heads * dv] in ``out_dtype``.  One launch for few rows, and for all of them with
+    ``tiles`` = :func:`head_tiles` of ``wuv``."""
     heads, t = ol.shape[:2]
-    if _head_product(t, wuv) and ol.is_contiguous():
+    tiled = tiles is not None and t >= HEAD_TILES_ROWS
+    if ol.is_contiguous() and (tiled or _head_product(t, wuv)):
         out = torch.empty(t, heads * wuv.shape[2], dtype=out_dtype, device=ol.device)
-        native_mixers().head_values(out, ol, wuv, gate)
+        native_mixers().head_values(out, ol, tiles if tiled else wuv, gate, tiled)
         return out
     o = torch.bmm(ol, wuv)                                               # [heads, T, dv]
     if gate is not None:
