@@ -675,8 +675,10 @@ extern "C" int mx_conv_attn_prep(float* q_out, const void* qkv, int bf16, long s
   const int channels = nq + nk + nv;
   const int chunks = (nq + nk) / head_dim + (nv + head_dim - 1) / head_dim;
   if (head_dim > 512 || rows > 0x7fffffffL || (chunks + 3) / 4 > 65535) return -3;
-  // rows per wave: a few once there are enough of them
-  const int rb = rows >= 256 && head_dim <= 256 && taps <= 4 ? 8 : 1;
+  // rows per wave: a few once there are enough of them, as many as leave every CU some waves (a wave's rows are a chain).  us with 1 2
+  // 4 8, 24 heads of 128: 300 rows 9.4 8.8 10.4 14.3, 500 12.1 10.8 11.7 15.4, 777 16.5 13.5 13.0 15.6, 1000 21 17 14 18, 1500 30 25
+  // 21.5 20.9, 4096 66 56 43 38 (64 4.7 6.7 11 19)
+  const int rb = rows < 256 || head_dim > 256 || taps > 4 ? 1 : rows < 640 ? 2 : rows < 1280 ? 4 : 8;
   const int nu = head_dim <= 64 ? 1 : head_dim <= 128 ? 2 : head_dim <= 256 ? 4 : 8;
   const dim3 grid((unsigned)((rows + rb - 1) / rb), (unsigned)((chunks + 3) / 4)), block(256);
 #define MX_CPREP(T, TC, TAPS, NU, RB)                                                                            \
@@ -684,15 +686,23 @@ extern "C" int mx_conv_attn_prep(float* q_out, const void* qkv, int bf16, long s
                      nk, nv, conv_w, taps, hist, start, pos0, slot, num_segs, num_state_slots, wq, wk, eps,       \
                      head_dim, slots, (TC*)k_cache, (TC*)v_cache, num_slots, rot_dims > 0 ? table : nullptr,      \
                      table_rows, rot_dims, interleaved)
+#define MX_CPRB(T, TC, RB)                             \
+  do {                                                 \
+    if (nu == 1) MX_CPREP(T, TC, 4, 1, RB);            \
+    else if (nu == 2) MX_CPREP(T, TC, 4, 2, RB);       \
+    else MX_CPREP(T, TC, 4, 4, RB);                    \
+  } while (0)
 #define MX_CPN(T, TC)                                  \
   do {                                                 \
     if (taps > 4) {                                    \
       if (nu <= 4) MX_CPREP(T, TC, 16, 4, 1);          \
       else MX_CPREP(T, TC, 16, 8, 1);                  \
     } else if (rb == 8) {                              \
-      if (nu == 1) MX_CPREP(T, TC, 4, 1, 8);           \
-      else if (nu == 2) MX_CPREP(T, TC, 4, 2, 8);      \
-      else MX_CPREP(T, TC, 4, 4, 8);                   \
+      MX_CPRB(T, TC, 8);                               \
+    } else if (rb == 4) {                              \
+      MX_CPRB(T, TC, 4);                               \
+    } else if (rb == 2) {                              \
+      MX_CPRB(T, TC, 2);                               \
     } else {                                           \
       if (nu <= 2) MX_CPREP(T, TC, 4, 2, 1);           \
       else if (nu == 4) MX_CPREP(T, TC, 4, 4, 1);      \
@@ -703,6 +713,7 @@ extern "C" int mx_conv_attn_prep(float* q_out, const void* qkv, int bf16, long s
   else if (!bf16 && !cache_bf16) MX_CPN(float, float);
   else return -4;                        // the cache is kept in the activations' dtype
 #undef MX_CPN
+#undef MX_CPRB
 #undef MX_CPREP
   int rc = (int)hipGetLastError();
   if (rc == 0 && taps > 1 && max_rows > 1)
