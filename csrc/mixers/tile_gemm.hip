@@ -564,6 +564,42 @@ tile_groups_kernel(TileArgs P) {
 }
 
 // ---------------------------------------------------------------------------------
+// One group's tiles of 256 x 256 while they make whole rounds over the chip's 256 CUs, and the last ones, up to 128, as halves of
+// 128 rows, a CU each: a round of those takes 0.7 of a whole one (their fragment reads bind them, as the ring's).  Bit for bit
+// the whole tiles' results.  us, whole tiles alone and the vendor's product beside it: 4096 x 2048 -> 6144 87 (96, 89), 2048 x 2048 ->
+// 10272 82 (90, 96), 2002 x 512 -> 9568 31 (36, 46).
+// ---------------------------------------------------------------------------------
+constexpr int kCus = 256;
+
+template <bool GLU>
+__global__ void __launch_bounds__(512, 1)
+tile_tail_kernel(TileArgs P) {
+  constexpr int kRing = kRingLds<2, 4, 4, 4, 3>;
+  __shared__ __attribute__((aligned(16))) char smem[kRing > kPhaseLds ? kRing : kPhaseLds];
+  const int n = (P.M + 255) / 256, cols = P.col_tiles, all = n * cols, whole = all / kCus * kCus, halves = 2 * (all - whole);
+  const int x = blockIdx.x & 7, per = (halves + 7) / 8;
+  int i = blockIdx.x >> 3, t, down = 0;
+  const bool half = i >= whole / 8;
+  if (half) {
+    i -= whole / 8;
+    const int u = x * per + i;
+    if (i >= per || u >= halves) return;
+    t = whole + u / 2, down = u % 2 * 128;
+  } else {
+    t = x * (whole / 8) + i;
+  }
+  const int band = t / (8 * cols), in = t - band * 8 * cols, tall = min(8, n - 8 * band);
+  TileAt at;
+  at.g = 0;
+  at.ct = __builtin_amdgcn_readfirstlane(in / tall);
+  at.row0 = __builtin_amdgcn_readfirstlane((8 * band + in % tall) * 256 + down);
+  at.end = P.M;
+  if (at.row0 >= P.M) return;
+  if (half) tile_ring<2, 4, 4, 4, 3, GLU>(P, at, smem);
+  else tile_phase<GLU, false>(P, at, smem);
+}
+
+// ---------------------------------------------------------------------------------
 // KW waves that share a tile of MT x NT tiles of 16: wave w takes the stages w, w + KW, .. and stages its own operands
 // (no barrier before the sums meet in LDS, in wave order).
 // ---------------------------------------------------------------------------------
@@ -661,8 +697,8 @@ tile_split_kernel(TileArgs P) {
 //   begin + R (tile + nk * stage) + r (all_tile + nk * all_stage)
 // the second part for what all CUs share (rates of the L2 and of memory, the card's power).  Fitted to 504 products of 65 to 4096
 // rows, weights from HBM, N and K of 64 to 14336 (residuals 4 to 11 %); the form chosen takes 1.006 times the best one's
-// time in the mean, 1.2 times at most.
-enum TileForm { kTile256x256, kTile256x128, kTile192x128, kTile128x128, kTile64x128, kTile64x64, kTile64x32, kTile32x64, kTileForms, kTileGroups = kTileForms };
+// time in the mean, 1.2 times at most.  kTileTail: whole tiles' rounds, and its last one's fitted beside them.
+enum TileForm { kTile256x256, kTile256x128, kTile192x128, kTile128x128, kTile64x128, kTile64x64, kTile64x32, kTile32x64, kTileForms, kTileGroups = kTileForms, kTileTail };
 struct TileSize {
   int rows, cols;
   float begin, tile, stage, all_stage, all_tile;
@@ -673,7 +709,8 @@ constexpr TileSize kTileSizes[kTileForms] = {
     {64, 128, 2.4f, 0.3f, 0.326f, 0.059f, 1.5f},  {64, 64, 3.2f, 0.5f, 0.184f, 0.050f, 1.4f},
     {64, 32, 2.0f, 1.1f, 0.107f, 0.054f, 0.6f},   {32, 64, 2.0f, 0.9f, 0.127f, 0.040f, 0.8f}};
 
-int tile_pick(long M, int N, int K, bool glu, float* us) {
+// (groups: of unknown rows, in the forms that take them)
+int tile_pick(long M, int N, int K, bool glu, bool groups, float* us) {
   int best = 0;
   float least = 3e38f;
   for (int f = 0; f < kTileForms; ++f) {
@@ -683,6 +720,13 @@ int tile_pick(long M, int N, int K, bool glu, float* us) {
     const float r = tiles / 256.f, whole = (float)((tiles + 255) / 256), nk = K / 64.f;
     const float t = z.begin + whole * (z.tile + nk * z.stage) + r * (z.all_tile + nk * z.all_stage);
     if (t < least) least = t, best = f;
+  }
+  const long tiles = ((M + 255) / 256) * ((N + (glu ? 127 : 255)) / (glu ? 128 : 256)), last = tiles % kCus;
+  if (!groups && tiles > kCus && last > 0 && last <= kCus / 2) {
+    const TileSize& z = kTileSizes[kTile256x256];
+    const float r = tiles / 256.f, nk = K / 64.f;
+    const float t = z.begin + (tiles / kCus) * (z.tile + nk * z.stage) + 3.8f + nk * 0.685f + r * (z.all_tile + nk * z.all_stage);
+    if (t < least) least = t, best = kTileTail;
   }
   if (us != nullptr) *us = least;
   return best;
@@ -696,6 +740,13 @@ int tile_launch(TileArgs& P, int form, hipStream_t s) {
     if (P.offs == nullptr || tiles > 0x7fffff00L) return -3;
     // (both sorts of tiles are eighths, rounded up)
     hipLaunchKernelGGL((tile_groups_kernel<GLU>), dim3((unsigned)((tiles + 21) / 8 * 8)), dim3(512), 0, s, P);
+    return (int)hipGetLastError();
+  }
+  if (form == kTileTail) {
+    P.col_tiles = (P.N + (GLU ? 127 : 255)) / (GLU ? 128 : 256);
+    const long tiles = (P.M + 255L) / 256 * P.col_tiles, whole = tiles / kCus * kCus;
+    if (P.offs != nullptr || tiles > 0x3fffff00L) return -3;
+    hipLaunchKernelGGL((tile_tail_kernel<GLU>), dim3((unsigned)(whole + (2 * (tiles - whole) + 7) / 8 * 8)), dim3(512), 0, s, P);
     return (int)hipGetLastError();
   }
   const TileSize& z = kTileSizes[form];
@@ -727,7 +778,7 @@ using namespace mx;
 // us that a product is expected to take
 extern "C" float mx_tile_gemm_us(long M, int N, int K, int glu) {
   float us;
-  tile_pick(M, N, K, glu != 0, &us);
+  tile_pick(M, N, K, glu != 0, false, &us);
   return us;
 }
 
@@ -743,14 +794,14 @@ extern "C" int mx_tile_gemm(void* C, long c_stride, const void* A, long a_stride
                             hipStream_t s) {
   if (M <= 0 || N <= 0 || groups <= 0) return 0;
   const bool glu = act >= kFrGelu && act <= kFrClamp;
-  if (act < kFrStore || act > kFrReluSq || form > kTileGroups || M > 0x3fffffffL) return -1;
+  if (act < kFrStore || act > kFrReluSq || form > kTileTail || M > 0x3fffffffL) return -1;
   if (!mx_tile_gemm_fits(a_rows, N, K, a_stride, glu)) return -1;
   if (((uintptr_t)A) % 16 || ((uintptr_t)W) % 16) return -2;
   if (glu && bias != nullptr) return -4;
   TileArgs P{(bf16_t*)C, (const bf16_t*)A, rows, (const bf16_t*)W, (const bf16_t*)bias, offs, c_stride,
              (unsigned)(a_stride * 2), (unsigned)(K * 2), groups, (int)M, N, K, 0, act, 0, limit};
   P.vec = c_stride % 8 == 0 && N % 8 == 0 && ((uintptr_t)C) % 16 == 0 ? 2 : c_stride % 4 == 0 && ((uintptr_t)C) % 8 == 0 ? 1 : 0;
-  if (form < 0) form = tile_pick(M, N, K, glu, nullptr);
+  if (form < 0) form = tile_pick(M, N, K, glu, offs != nullptr, nullptr);
   return glu ? tile_launch<true>(P, form, s) : tile_launch<false>(P, form, s);
 }
 

@@ -118,7 +118,7 @@ def _tile_gemm_pays(rows: int, n: int, k: int, act: Optional[str] = None) -> boo
     rows); captured steps: :func:`_tile_gemm_behind`.  Beyond, the sooner full tiles keep the vendor's product at its rate, the
     less.  us at 100 / 300 / 777 / 2048 / 4096 rows, the vendor's (with the activation) beside it:
       n = 2048, k = 2048     7 10 14 22 40 (9 11 15 23 35)         k = 8192            22 31 49 90 128 (21 33 47 74 118)
-      n = 10272, k = 2048    18 21 47 92 155 (18 26 41 96 180)     n = 64              6 7 7 7 8 (8 8 8 9 10)
+      n = 10272, k = 2048    18 21 47 82 155 (18 26 41 96 180)     n = 64              6 7 7 7 8 (8 8 8 9 10)
       gated, 2 x 8192, k = 2048    20 34 55 109 225 (28 40 66 137 270)
       n = 4096, k = 14336    44 93 121 215 338 (50 76 115 204 316)"""
     if rows <= FEW_ROWS or k % 64 or k < 64:
@@ -127,6 +127,11 @@ def _tile_gemm_pays(rows: int, n: int, k: int, act: Optional[str] = None) -> boo
     out = n // 2 if glu else n
     if max(rows * k, n * k) * 2 > 0xffffffff or out < 1:
         return False
+    tiles = -(-rows // 256) * -(-n // 256)
+    if act is None and rows > 1024 and 300 <= tiles <= 384 and 1792 <= k <= 2560 and tiles * 65536 <= 1.06 * rows * n:
+        # the vendor's product has the last, part round of its large tiles too: a round and a part in the form that halves those takes
+        # 0.80 to 1.01 of its time at k = 2048 (eleven products; 0.87 to 1.05 at 2560; fewer tiles, or k = 1536, up to 1.14)
+        return True
     spare = (20 if rows <= 1024 else 7) + (0 if act is None else 4 + rows * out * (6 if glu else 4) / 3.5e6)
     return native_mixers().tile_gemm_us(rows, out, k, glu) <= spare + 2.0 * rows * n * k / (1.3e9 if rows <= 1024 else 1.35e9)
 
