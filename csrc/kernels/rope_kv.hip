@@ -1,7 +1,7 @@
 // K4: fused rotary embedding + paged KV-cache write.
 //
 // Input is the fused QKV GEMM output [T, (nq + 2 nkv) * D].  One workgroup per
-// token; each lane handles 8 rotary pairs (element i and i + D/2, the Llama
+// token rotates its q and k heads; each lane handles 8 rotary pairs (element i and i + D/2, the Llama
 // "rotate_half" convention) with 16-B loads/stores.  Q is rotated in place (the
 // attention kernels read it with the QKV row stride, so there is no extra copy),
 // K is rotated and written straight into the paged cache, V is copied into the
@@ -18,6 +18,66 @@
 
 namespace ft {
 
+// V into its transposed blocks: a workgroup a key head of 16 tokens, which change places in LDS, so that eight tokens of a
+// dim whose slots follow each other (any eight of a block, in a prompt) leave as one store, two lanes a dim's row of 16.
+// Bound by memory: with the rotation, 4096 tokens of 32 query and 8 key heads of 128 17 us (100 MB), 1024 5.5; token by token,
+// each dim a store of 2 bytes to a line of its own, 32 and 10.9.  Slots in no order 25 us (40), one token level.
+constexpr int kVTokens = 16;
+
+template <int D, bool KV8>
+__device__ __forceinline__ void v_block_write(const uint16_t* __restrict__ qkv, int qkv_stride, const int* __restrict__ slot_mapping,
+                                              void* __restrict__ v_cache, int tokens, int nq, int nkv, int block_size, int num_slots,
+                                              int t0, int kh) {
+  constexpr int P = D + 8;                     // a row's pitch: the two halves of the tokens in different banks
+  __shared__ __attribute__((aligned(16))) uint16_t rows[kVTokens * P];
+  __shared__ int at[kVTokens];
+  const int tid = threadIdx.x;
+  if (tid < kVTokens) {
+    const int t = t0 + tid;
+    int slot = t < tokens ? slot_mapping[t] : -1;
+    if (slot >= 0) slot = FT_CHECK_IDX(slot, num_slots, kCkSlot, t);
+    at[tid] = slot;
+  }
+  if (tid < kVTokens * (D / 8)) {
+    const int j = tid / (D / 8), c = tid % (D / 8), t = min(t0 + j, tokens - 1);
+    *reinterpret_cast<uint4*>(rows + j * P + c * 8) =
+        *reinterpret_cast<const uint4*>(qkv + (size_t)t * qkv_stride + (nq + nkv + kh) * D + c * 8);
+  }
+  __syncthreads();
+  if (tid >= 2 * D) return;
+  const int d = tid >> 1, j0 = (tid & 1) * 8, first = at[j0];
+  uint32_t w[4];
+  bool row = first >= 0 && (first | block_size) % 8 == 0 && reinterpret_cast<uintptr_t>(v_cache) % 16 == 0;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const uint32_t v = rows[(j0 + j) * P + d];
+    w[j / 2] = j % 2 ? w[j / 2] | v << 16 : v;
+    row = row && at[j0 + j] == first + j;
+  }
+  uint2 q8{};
+  if constexpr (KV8) {
+    float f[8];
+    load8(make_uint4(w[0], w[1], w[2], w[3]), f);
+    q8 = fp8x8_pack(f);
+  }
+  if (row) {
+    const int blk = first / block_size, off = first - blk * block_size;
+    const size_t e = (((size_t)blk * nkv + kh) * D + d) * block_size + off;
+    if constexpr (KV8) *reinterpret_cast<uint2*>(reinterpret_cast<uint8_t*>(v_cache) + e) = q8;
+    else *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(v_cache) + e) = make_uint4(w[0], w[1], w[2], w[3]);
+    return;
+  }
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const int slot = at[j0 + j];
+    if (slot < 0) continue;
+    const int blk = slot / block_size, off = slot - blk * block_size;
+    const size_t e = (((size_t)blk * nkv + kh) * D + d) * block_size + off;
+    if constexpr (KV8) reinterpret_cast<uint8_t*>(v_cache)[e] = (uint8_t)((j < 4 ? q8.x : q8.y) >> (8 * (j & 3)));
+    else reinterpret_cast<uint16_t*>(v_cache)[e] = (uint16_t)(w[j / 2] >> (16 * (j & 1)));
+  }
+}
+
 // KV8: fp8 (e4m3) caches, same layouts with 1-byte elements (ft_common.h fp8x*)
 template <int D, bool KV8>
 __global__ __launch_bounds__(256) void rope_kv_kernel(uint16_t* __restrict__ qkv, int qkv_stride,
@@ -27,7 +87,12 @@ __global__ __launch_bounds__(256) void rope_kv_kernel(uint16_t* __restrict__ qkv
                                                       void* __restrict__ k_cache,
                                                       void* __restrict__ v_cache, int nq,
                                                       int nkv, int block_size, int cos_rows,
-                                                      int num_slots) {
+                                                      int num_slots, int tokens) {
+  if ((int)blockIdx.x >= tokens) {
+    const int u = (int)blockIdx.x - tokens;
+    v_block_write<D, KV8>(qkv, qkv_stride, slot_mapping, v_cache, tokens, nq, nkv, block_size, num_slots, u / nkv * kVTokens, u % nkv);
+    return;
+  }
   constexpr int HALF = D / 2;
   constexpr int CPH = HALF / 8;  // 8-pair chunks per head
   const int t = blockIdx.x;
@@ -79,33 +144,6 @@ __global__ __launch_bounds__(256) void rope_kv_kernel(uint16_t* __restrict__ qkv
       }
     }
   }
-  if (slot >= 0) {
-    const int blk = slot / block_size, off = slot - blk * block_size;
-    const int nv = nkv * (D / 8);
-    const uint4* vsrc = reinterpret_cast<const uint4*>(row + (nq + nkv) * D);
-    for (int item = threadIdx.x; item < nv; item += blockDim.x) {
-      const int kh = item / (D / 8), c = item - kh * (D / 8);
-      // V blocks are transposed ([D][block_size]): dims c*8.. of this token
-      const size_t e = (((size_t)blk * nkv + kh) * D + c * 8) * block_size + off;
-      const uint4 v = vsrc[item];
-      if constexpr (KV8) {
-        float f[8];
-        load8(v, f);
-        const uint2 q8 = fp8x8_pack(f);
-        uint8_t* vp = reinterpret_cast<uint8_t*>(v_cache) + e;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) vp[j * block_size] = (uint8_t)(((j < 4 ? q8.x : q8.y) >> (8 * (j & 3))) & 0xffu);
-      } else {
-        uint16_t* vp = reinterpret_cast<uint16_t*>(v_cache) + e;
-        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          vp[(2 * j) * block_size] = (uint16_t)(w[j] & 0xffffu);
-          vp[(2 * j + 1) * block_size] = (uint16_t)(w[j] >> 16);
-        }
-      }
-    }
-  }
 }
 
 }  // namespace ft
@@ -116,11 +154,13 @@ extern "C" int ft_rope_kv_write(void* qkv, int qkv_stride, const int* positions,
                                 int block_size, int cos_rows, int num_slots, int kv8,
                                 hipStream_t stream) {
   if (tokens <= 0) return 0;
-  dim3 grid(tokens), block(256);
+  const long v_blocks = (tokens + ft::kVTokens - 1L) / ft::kVTokens * nkv;
+  if (tokens + v_blocks > 0x7fffffffL) return -2;
+  dim3 grid((unsigned)(tokens + v_blocks)), block(256);
 #define FT_ROPE(DD, K8)                                                                     \
   hipLaunchKernelGGL((ft::rope_kv_kernel<DD, K8>), grid, block, 0, stream, (uint16_t*)qkv,  \
                      qkv_stride, positions, cos_sin, slot_mapping, k_cache, v_cache, nq, nkv, \
-                     block_size, cos_rows, num_slots)
+                     block_size, cos_rows, num_slots, tokens)
   if (head_dim == 128) {
     if (kv8) FT_ROPE(128, true); else FT_ROPE(128, false);
   } else if (head_dim == 64) {
