@@ -24,7 +24,8 @@
 // 101, and 30 where it takes 17); the carry by its chain.  4096 rows, 16 heads of 128 x 128, delta rule:
 // 101 + 159 + 46 us, the walk 2080; 777 rows, linear attention: 17 + 19 + 16 us, the walk 245.
 // Where no segment of a step is walked, the delta rule's rows come as the projections left them and are normed
-// and their decays formed here (129 us; 101 + 56 for a kernel of its own that writes and reads them again).
+// and their decays formed here (113 us; 129 before delta_decay, when a kernel of its own, which writes and reads them again,
+// made it 101 + 56).
 #include "chunk_common.h"
 
 namespace mx {
