@@ -9,7 +9,7 @@
 // the same 16 of the up matrix, so a lane has both sums and the activation is part of the epilogue.  Results leave through
 // LDS, whole rows of the tile at a time (written four columns a lane, 4096 x 4096 -> 2 x 14336 takes 700 us instead of 656).
 //
-// Four kernels, for different numbers of tiles (the table of forms below has the times of three):
+// Five kernels, for different numbers of tiles (the table of forms below has the times of three):
 //   tile_phase_kernel  256 x 256, eight waves in two groups half a phase apart: while one group's products run, the other's
 //                      LDS reads and loads do (all eight in step, 4096 x 2048 -> 2 x 8192 takes 259 us instead of 225).
 //                      Bound by the matrix units at the clock that the card's power leaves them: 4096 x 4096 -> 2 x 14336
@@ -25,6 +25,7 @@
 //                      up to a hundred rows a group, by the read of the matrices (5.4 TB/s).  us before and now, 32 experts: 4096
 //                      rows, top 4, of 2048 -> 2 x 1024 and back 186 + 104, 145 + 86; 1872, of 2048 -> 1536 and back 65 + 92, 61 + 71;
 //                      300, top 6, of 2048 -> 2 x 1024 71, 53.
+//   tile_tail_kernel   256 x 256 while they fill all CUs, the rest of them as halves (below).
 #include "few_rows.h"
 #include "ft_lds.h"
 
