@@ -14,6 +14,10 @@
 // issue of all of them: 1.0 us a chunk; 14 + 37 us for those 2048 rows.  (All of it in one launch, weights and sums of decays by other
 // waves of the same workgroup, which every 16 columns repeat: 87 us; by the output waves: 86 to 97.)
 //
+// A value of v that is not finite reaches its own row and later ones only: a weight of 0 would take it to the rows before it in its block of
+// 16, so blocks with such a value (`loose`) have them apart from the products (no measurable time where there is none: 2048 rows
+// 59 us both, 777 of them 30.1 and 30.9).
+//
 // Operand layouts (v_mfma_f32_16x16x32_bf16): lane (hi, lo) = (lane / 16, lane % 16) holds row or column lo, inner entries 8 hi ..
 // 8 hi + 7; accumulators hold row 4 hi + r, column lo.  Sums over rows j take j in the order in which accumulators lie, entry i < 4
 // of (hi) row 4 hi + i of a tile of 16, i >= 4 of the next one.
@@ -35,6 +39,9 @@ __device__ __forceinline__ void ss_split(float a, float b, float c, float d, uin
   split_any_bf16x3(a, b, p[0].x, p[1].x, p[2].x);
   split_any_bf16x3(c, d, p[0].y, p[1].y, p[2].y);
 }
+// which of two bf16 are infinite or NaN: in the bits of their signs alone, and as 0xffff of theirs
+__device__ __forceinline__ uint32_t ss_loose(uint32_t u) { return (u & 0x7f807f80u) + 0x00800080u; }
+__device__ __forceinline__ uint32_t ss_not_finite(uint32_t u) { return (ss_loose(u) >> 15 & 0x00010001u) * 0xffffu; }
 // e^x of a sum of log decays, x <= 0, within 2 units in the last place (0 below e^-200)
 __device__ __forceinline__ float ss_exp(double x) {
   constexpr float kL = 1.4426950408889634f, kLo = 1.925963033500e-8f, kLn2 = 0.6931471805599453f;
@@ -151,6 +158,7 @@ state_scan_kernel(float* __restrict__ o, const float* __restrict__ ws, ScanIn in
   __shared__ __attribute__((aligned(16))) char ks[3][kC * 256], vs[3][kC * 32];
   __shared__ __attribute__((aligned(16))) uint2 parts[2][3][4][64][2];       // the state's, as left operands (columns) of q . S
   __shared__ __attribute__((aligned(16))) uint4 scaled[2][2][3][64];         // step e^{G_63 - G_j} v_j's, as right operands (columns)
+  __shared__ uint32_t loose[3][4];                      // lanes with a value of v that is not finite, a block of 16 rows each
   const int h = blockIdx.x, c0 = blockIdx.y * kSsCols;
   const int seg = long_segment(blockIdx.z, gridDim.z, st, start);
   if (seg < 0) return;
@@ -213,7 +221,11 @@ state_scan_kernel(float* __restrict__ o, const float* __restrict__ ws, ScanIn in
         *reinterpret_cast<uint4*>(ks[b] + j * 256 + ((lt & 15) ^ (j & 15)) * 16) = x;
       }
       if ((lt >> 1) >= left) vr = uint4{0, 0, 0, 0};
-      if (lt < 2 * kC) *reinterpret_cast<uint4*>(vs[b] + lt * 16) = vr;
+      if (lt < 2 * kC) {
+        *reinterpret_cast<uint4*>(vs[b] + lt * 16) = vr;
+        const uint64_t m = __ballot(((ss_loose(vr.x) | ss_loose(vr.y) | ss_loose(vr.z) | ss_loose(vr.w)) & 0x80008000u) != 0);
+        if ((lane & 31) == 0) loose[b][lt >> 5] = (uint32_t)(m >> lane);
+      }
     };
     fetch(0);
     put(0, 0);
@@ -331,6 +343,7 @@ state_scan_kernel(float* __restrict__ o, const float* __restrict__ ws, ScanIn in
       f0 = fn;
       fetch(idx + 1);
       f32x4 O[3], pv[3];
+      const uint32_t apart = loose[b][wave];
 #pragma unroll
       for (int z = 0; z < 3; ++z) O[z] = pv[z] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -345,7 +358,54 @@ state_scan_kernel(float* __restrict__ o, const float* __restrict__ ws, ScanIn in
 #pragma unroll
         for (int z = 2; z >= 0; --z) pv[z] = ss_mma(v, w[p][z], pv[z]);
       }
-      const f32x4 y = ((O[2] + O[1]) + O[0]) * f0 + ((pv[2] + pv[1]) + pv[0]);
+      const bool again = __builtin_amdgcn_readfirstlane(apart) != 0;
+      if (again) {
+        // One of the block's own rows is not finite, and a weight of 0 takes it to the rows before it: the sums again without such
+        // values of the block, which then go to the rows from them on.
+#pragma unroll
+        for (int z = 0; z < 3; ++z) pv[z] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+          if (2 * p > wave) continue;
+          uint4 v = read_v(vb, p);
+          if (2 * p + 1 > wave) v.z = v.w = 0;
+          if (p == wave >> 1) {
+            if (wave & 1) v.z &= ~ss_not_finite(v.z), v.w &= ~ss_not_finite(v.w);
+            else v.x &= ~ss_not_finite(v.x), v.y &= ~ss_not_finite(v.y);
+          }
+#pragma unroll
+          for (int z = 2; z >= 0; --z) pv[z] = ss_mma(v, w[p][z], pv[z]);
+        }
+      }
+      f32x4 y = ((O[2] + O[1]) + O[0]) * f0 + ((pv[2] + pv[1]) + pv[0]);
+      if (again) {
+        // lane (hi, lo) has the weights of row t and rows 4 hi .. 4 hi + 3 of the block
+        float own[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          own[r] = 0.f;
+#pragma unroll
+          for (int z = 2; z >= 0; --z) {
+            const uint32_t first = wave >> 1 ? (r < 2 ? w[1][z].x : w[1][z].y) : r < 2 ? w[0][z].x : w[0][z].y;
+            const uint32_t second = wave >> 1 ? (r < 2 ? w[1][z].z : w[1][z].w) : r < 2 ? w[0][z].z : w[0][z].w;
+            const uint32_t x = wave & 1 ? second : first;
+            own[r] += __uint_as_float(r & 1 ? x & 0xffff0000u : x << 16);
+          }
+        }
+#pragma unroll 1
+        for (int g = 0; g < 4; ++g) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int j = 4 * g + r;
+            const float wj = __shfl(own[r], 16 * g + lo, 64);
+            const uint2 u = *reinterpret_cast<const uint2*>(vb + (16 * wave + j) * 32 + 8 * hi);
+            const uint32_t m[2] = {ss_not_finite(u.x), ss_not_finite(u.y)}, x[2] = {u.x, u.y};
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if (j <= lo && (m[e >> 1] >> (16 * (e & 1)) & 1)) y[e] += wj * __uint_as_float(e & 1 ? x[e >> 1] & 0xffff0000u : x[e >> 1] << 16);
+          }
+        }
+      }
       if (t < rows - idx * kC) {
         const uint2 own = *reinterpret_cast<const uint2*>(vb + t * 32 + 8 * hi);
         float x[4];

@@ -63,15 +63,39 @@ def test_rows(lens, pos, heads, groups, dv, shift):
     assert float((state.double() - left).abs().max()) <= 2.0 ** -21 * max(size, 1.0)
 
 
-def test_padding_segments_and_infinite_rows():
+def test_padding_segments():
     heads, groups, dv, lens = 4, 2, 32, [100, 70, 130]
     args = case(lens, heads, groups, dv)
     good, states = run(args, lens, [0, 0, 0], heads, groups, dv)
     y, left = run(args, lens, [0, 0, 0], heads, groups, dv, slots=[0, -1, 2])
     assert torch.equal(y[:100], good[:100]) and torch.equal(y[170:], good[170:]) and bool((y[100:170] == 0).all())
     assert torch.equal(left[1], args[5][1]) and torch.equal(left[0], states[0])
-    # rows before an infinite one do not see it, nor do other segments and heads
-    args[0][100 + 16, 5] = float("inf")
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan")])
+@pytest.mark.parametrize("row", [0, 1, 14, 15, 16, 17, 30, 33, 47, 52, 63, 64, 67, 69])
+def test_a_row_that_is_not_finite(bad, row):
+    """Rows before it do not see it, wherever in its chunk it lies, nor do other segments, heads and columns."""
+    heads, groups, dv, lens = 4, 2, 32, [100, 70, 130]
+    args = case(lens, heads, groups, dv)
+    good, _ = run(args, lens, [0, 0, 0], heads, groups, dv)
+    at, n = 100 + row, heads * dv
+    for col, seen in ((5, slice(5, 6)), (n + 3, slice(0, 2 * dv)), (n + groups * N + 3, slice(0, 2 * dv))):     # x, B, C
+        keep = args[0][at, col].clone()
+        args[0][at, col] = bad
+        y, _ = run(args, lens, [0, 0, 0], heads, groups, dv)
+        args[0][at, col] = keep
+        assert torch.equal(y[:at], good[:at]) and torch.equal(y[170:], good[170:])
+        others = torch.ones(n, dtype=torch.bool, device=DEV)
+        others[seen] = False
+        assert torch.equal(y[:, others], good[:, others])
+        own = y[at:170 if col < n + groups * N else at + 1, seen]
+        assert not bool(torch.isfinite(own).any())
+        if col >= n + groups * N:                         # a row of C is its own output's alone
+            assert torch.equal(y[at + 1:], good[at + 1:])
+    args[1][at, 1] = bad if bad > 0 else float("nan")      # (a step of softplus(-inf) is none)
     y, _ = run(args, lens, [0, 0, 0], heads, groups, dv)
-    assert torch.equal(y[:116], good[:116]) and torch.equal(y[170:], good[170:])
-    assert torch.equal(y[:, dv:], good[:, dv:]) and not bool(torch.isfinite(y[116:170, 5]).any())
+    others = [0, 2, 3]
+    assert torch.equal(y[:at], good[:at]) and torch.equal(y[170:], good[170:])
+    assert torch.equal(y.view(-1, heads, dv)[:, others], good.view(-1, heads, dv)[:, others])
+    assert not bool(torch.isfinite(y[at:170].view(-1, heads, dv)[:, 1]).any())
