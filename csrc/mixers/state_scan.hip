@@ -15,8 +15,8 @@
 // waves of the same workgroup, which every 16 columns repeat: 87 us; by the output waves: 86 to 97.)
 //
 // A value of v that is not finite reaches its own row and later ones only: a weight of 0 would take it to the rows before it in its block of
-// 16, so blocks with such a value (`loose`) have them apart from the products (no measurable time where there is none: 2048 rows
-// 59 us both, 777 of them 30.1 and 30.9).
+// 16, so blocks with such a value (`loose`) have them apart from the products (2048 rows 58.8 us so and 59.3
+// without, 777 30.9 and 30.1).
 //
 // Operand layouts (v_mfma_f32_16x16x32_bf16): lane (hi, lo) = (lane / 16, lane % 16) holds row or column lo, inner entries 8 hi ..
 // 8 hi + 7; accumulators hold row 4 hi + r, column lo.  Sums over rows j take j in the order in which accumulators lie, entry i < 4
@@ -42,13 +42,16 @@ __device__ __forceinline__ void ss_split(float a, float b, float c, float d, uin
 // which of two bf16 are infinite or NaN: in the bits of their signs alone, and as 0xffff of theirs
 __device__ __forceinline__ uint32_t ss_loose(uint32_t u) { return (u & 0x7f807f80u) + 0x00800080u; }
 __device__ __forceinline__ uint32_t ss_not_finite(uint32_t u) { return (ss_loose(u) >> 15 & 0x00010001u) * 0xffffu; }
-// e^x of a sum of log decays, x <= 0, within 2 units in the last place (0 below e^-200)
+// e^x of a sum of log decays, x <= 0, within 2 units in the last place of fp32 (which are larger below its smallest normal number)
 __device__ __forceinline__ float ss_exp(double x) {
   constexpr float kL = 1.4426950408889634f, kLo = 1.925963033500e-8f, kLn2 = 0.6931471805599453f;
-  float y = (float)x;
-  y = y < -200.0f ? -200.0f : y;
-  const float t = y * kL, r = __builtin_amdgcn_exp2f(t);
-  return fmaf(r * kLn2, fmaf(y, kLo, fmaf(y, kL, -t)), r);
+  x = x < -200.0 ? -200.0 : x;                     // (a NaN stays one)
+  const float y = (float)x, rest = (float)(x - (double)y), t = y * kL;
+  const int down = t < -100.0f ? 64 : 0;           // (exp2 has no denormal results)
+  const float r = __builtin_amdgcn_exp2f(t + (float)down);
+  // what t dropped of x in units of log2; the sum with `down` is exact
+  const float low = fmaf(rest, kL, fmaf(y, kLo, fmaf(y, kL, -t)));
+  return ldexpf(fmaf(r * kLn2, low, r), -down);
 }
 
 constexpr int kSsKeys = 128, kSsCols = 16;

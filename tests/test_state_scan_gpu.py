@@ -99,3 +99,26 @@ def test_a_row_that_is_not_finite(bad, row):
     assert torch.equal(y[:at], good[:at]) and torch.equal(y[170:], good[170:])
     assert torch.equal(y.view(-1, heads, dv)[:, others], good.view(-1, heads, dv)[:, others])
     assert not bool(torch.isfinite(y[at:170].view(-1, heads, dv)[:, 1]).any())
+
+
+def test_decays_of_any_size():
+    """What a single row leaves to each later one, to a few units in the last place: sums of decays that fp32 does not hold, results
+    below the smallest normal number, within a chunk and over its end."""
+    dv, n, at = 16, 128, 40
+    big, small = 24.5, -14.0                             # softplus(24.5) = 24.5 and softplus(-14) = 8.3e-7 in fp32
+    for steps, x0, c0 in (([big, big, small, small], 1.0, 1.0), ([big, big, small, big, big], 2.0 ** 100, 2.0 ** 20),
+                          ([small] * 3 + [big] + [small] * 60, 1.0, 1.0)):
+        t = at + 1 + len(steps)
+        xbc = torch.zeros(t, dv + 2 * n, device=DEV)
+        xbc[at, :dv], xbc[at, dv], xbc[:, dv + n] = x0, 1.0, c0
+        dt = torch.zeros(t, 1, device=DEV)
+        dt[at + 1:, 0] = torch.tensor(steps)
+        zero = torch.zeros(1, device=DEV)
+        args = (xbc.bfloat16(), dt.bfloat16(), zero, zero, zero, torch.zeros(1, 1, n, dv, device=DEV))
+        y, state = run(args, [t], [0], 1, 1, dv, least=1)
+        step = torch.nn.functional.softplus(dt[:, 0]).double()
+        want = torch.exp(-(step.cumsum(0)[at:] - step[:at + 1].sum())) * step[at] * x0
+        # up to three factors, each within two units in the last place of 2^-24 (of 2^-149 below the smallest normal number), and as
+        # many products of three parts, each rounded once
+        for got, w, f in ((y[at:, 0].double(), want * c0, x0 * c0), (state[0, 0, 0, :1].double(), want[-1:], x0)):
+            assert bool(((got - w).abs() <= 2.0 ** -20 * w + 2.0 ** -148 * f).all()), (got / w - 1).abs().max()
