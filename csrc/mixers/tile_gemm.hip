@@ -152,11 +152,15 @@ __device__ __forceinline__ unsigned tile_w_off(const TileArgs& P, int n0, int r,
   return (unsigned)((GLU && (r & 16) ? P.N : 0) + col) * P.w_bytes + (unsigned)(((lane & 7) ^ ((r >> 1) & 5)) * 16);
 }
 
-// SPREAD: every XCD begins k at another eighth of it.  Rows of 4 KB put one stage of all rows into few of the memory's channels,
+// SPREAD: the groups begin k at its eighths in turn.  Rows of 4 KB put one stage of all rows into few of the memory's channels,
 // and with the workgroups all at the same stage those are what the read waits for: 32 matrices of 2 x 1024 x 2048 with up to 64 rows
-// each 71 us (3.8 TB/s) in step, 50 (5.4) spread; 234 rows each 97 and 84.  Tiles of one XCD stay in step, since they share rows in
-// its L2.  Products of one matrix read it at that rate from a few rows on and gain nothing.
-__device__ __forceinline__ int tile_first_stage(int nk) { return (int)(blockIdx.x & 7) * nk / 8; }
+// each 71 us (3.8 TB/s) in step, 50 (5.4) spread; 234 rows each 97 and 84.  A group's tiles stay in step, since they share rows in
+// an L2 (by columns as well: both products of 2000 rows, top 4, 172 to 200 us).  By the group and not by the XCD: a row's sum is the
+// same wherever its tile lies and whatever rows the other groups have.  Three eighths from a group to the next: an XCD
+// has one or two of them under way, the next one the two after (us of both products, 32 experts of 1024, by XCD / one eighth on / three /
+// g of n at the 8 g / n-th: 4096 rows 262 262 260 266; 300 rows, top 6 95 97 97 95; 64 experts of 1408 256 258 253 257; a group alone of
+// 4096 rows, 2048 -> 2048 45 44 43 46).  Products of one matrix read it at that rate from a few rows on and gain nothing.
+__device__ __forceinline__ int tile_first_stage(int g, int nk) { return (3 * g & 7) * nk / 8; }
 template <bool SPREAD>
 __device__ __forceinline__ int tile_stage_at(int t, int k0, int nk) {
   if constexpr (!SPREAD) return t;
@@ -230,7 +234,7 @@ __device__ __forceinline__ void tile_phase(const TileArgs& P, const TileAt& at, 
   const int wm = wave >> 2, wn = wave & 3, l15 = lane & 15, g4 = lane >> 4;
   const int n0 = at.ct * OC;
   const bf16_t* W = P.W + (long)at.g * P.N * (GLU ? 2 : 1) * P.K;
-  const int nk = P.K / kTK, k0 = SPREAD ? tile_first_stage(nk) : 0;
+  const int nk = P.K / kTK, k0 = SPREAD ? tile_first_stage(at.g, nk) : 0;
   const uint32_t lds0 = ft::lds_off(smem);
   unsigned ap[2][PA], wp[2][PB];
 #pragma unroll
@@ -380,7 +384,7 @@ __device__ __forceinline__ void tile_ring(const TileArgs& P, const TileAt& at, c
   const int wm = wave / WN, wn = wave % WN, l15 = lane & 15, g4 = lane >> 4;
   const int n0 = at.ct * OC;
   const bf16_t* W = P.W + (long)at.g * P.N * (GLU ? 2 : 1) * P.K;
-  const int nk = P.K / kTK, k0 = SPREAD ? tile_first_stage(nk) : 0;
+  const int nk = P.K / kTK, k0 = SPREAD ? tile_first_stage(at.g, nk) : 0;
   const uint32_t lds0 = ft::lds_off(smem);
   unsigned ap[PA], wp[PB];
 #pragma unroll

@@ -1,5 +1,5 @@
 """Grouped products in tiles of 256 rows with shorter last pieces (csrc/mixers/tile_gemm.hip, tile_groups_kernel) against the same
-sums in 64 bits: group sizes at the edges of each tile, one to a few stages of k (every XCD begins at another of them), more
+sums in 64 bits: group sizes at the edges of each tile, one to a few stages of k (the groups begin at another of them in turn), more
 groups than a wave has lanes, plain, gated and through an index."""
 import pytest
 import torch
@@ -61,3 +61,19 @@ def test_experts(rows, experts, top, act):
         size += w * (y.abs() @ wdown[e].double().abs().t())
     # two bf16 roundings, each half a unit in the eighth bit: 2^-8 of each term of the second product and of its sum
     assert bool(((got.double() - want).abs() <= 2.0 ** -7 * size + 1e-5).all())
+
+
+@pytest.mark.parametrize("before,count", [([0, 0, 0], 700), ([300, 40, 900], 1000), ([1, 513, 64], 449)])
+def test_equal_rows(before, count):
+    """A row's result is the same bits wherever its tile lies: in each of its group's, whole or short, and behind others' rows."""
+    k, n, e = 1088, 16 * 256, 16
+    w = rnd(1, e, n, k, scale=k ** -0.5)
+    row = rnd(2, 1, k)
+    counts = [before[i % 3] for i in range(7)] + [count] + [20] * (e - 8)
+    a = row.expand(sum(counts), k).contiguous()
+    got = M.grouped_mm(a, w, torch.tensor(counts).cumsum(0).int().to(DEV))
+    alone = M.grouped_mm(row.expand(e * 30, k).contiguous(), w, torch.tensor([30] * e).cumsum(0).int().to(DEV))
+    s = 0
+    for g, c in enumerate(counts):
+        assert torch.equal(got[s:s + c], alone[30 * g:30 * g + 1].expand(c, n))
+        s += c
