@@ -47,7 +47,7 @@ int mx_add_norm_shift_experts(float* x, const float* d, const float* wts, const 
                               const int* start, const int* pos0, const int* slot, int num_segs, int rows, int width,
                               float eps, hipStream_t s);
 int mx_tile_gemm_fits(long M, int N, int K, long a_stride, int glu);
-float mx_tile_gemm_us(long M, int N, int K, int glu);
+float mx_tile_gemm_us(long M, int N, int K, int glu, int* tail);
 int mx_tile_gemm(void* C, long c_stride, const void* A, long a_stride, long a_rows, const int* rows, const void* W,
                  const void* bias, const int* offs, int groups, long M, int N, int K, int act, float limit, int form,
                  hipStream_t s);
@@ -1197,7 +1197,12 @@ void norm_route(Tensor idx, Tensor wts, Tensor h, Tensor x, Tensor y, bool layer
                     (int)top, (int)mode, (float)scale, (int)groups, (int)keep, stream()), "norm_route");
 }
 
-double tile_gemm_us(int64_t rows, int64_t n, int64_t k, bool glu) { return mx_tile_gemm_us(rows, (int)n, (int)k, glu); }
+// expected us, and whether the last round of tiles is done in halves
+std::pair<double, bool> tile_gemm_us(int64_t rows, int64_t n, int64_t k, bool glu) {
+  int tail = 0;
+  const double us = mx_tile_gemm_us(rows, (int)n, (int)k, glu, &tail);
+  return {us, tail != 0};
+}
 
 // form: one of tile_gemm.hip's, or below 0 the one that it takes by itself
 void tile_gemm(Tensor y, Tensor x, Tensor w, OptT bias, int64_t act, double limit, int64_t form) {

@@ -780,10 +780,11 @@ int tile_launch(TileArgs& P, int form, hipStream_t s) {
 
 using namespace mx;
 
-// us that a product is expected to take
-extern "C" float mx_tile_gemm_us(long M, int N, int K, int glu) {
+// us that a product is expected to take, and (tail, if not null) whether its last round of tiles is done in halves
+extern "C" float mx_tile_gemm_us(long M, int N, int K, int glu, int* tail) {
   float us;
-  tile_pick(M, N, K, glu != 0, false, &us);
+  const int form = tile_pick(M, N, K, glu != 0, false, &us);
+  if (tail != nullptr) *tail = form == kTileTail;
   return us;
 }
 

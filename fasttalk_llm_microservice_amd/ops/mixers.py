@@ -127,13 +127,18 @@ def _tile_gemm_pays(rows: int, n: int, k: int, act: Optional[str] = None) -> boo
     out = n // 2 if glu else n
     if max(rows * k, n * k) * 2 > 0xffffffff or out < 1:
         return False
-    tiles = -(-rows // 256) * -(-n // 256)
-    if act is None and rows > 1024 and 300 <= tiles <= 384 and 1792 <= k <= 2560 and tiles * 65536 <= 1.06 * rows * n:
-        # the vendor's product has the last, part round of its large tiles too: a round and a part in the form that halves those takes
-        # 0.80 to 1.01 of its time at k = 2048 (eleven products; 0.87 to 1.05 at 2560; fewer tiles, or k = 1536, up to 1.14)
-        return True
+    us, tail = native_mixers().tile_gemm_us(rows, out, k, glu)
+    flops_us = 2.0 * rows * n * k / (1.3e9 if rows <= 1024 else 1.35e9)
+    rounds = -(-rows // 256) * -(-n // 256) / 256
+    if tail and act is None and rows > 1024 and n % 8 == 0 and k <= 3072 and rounds < 2:
+        # A round of large tiles and a part, in halves: the vendor's product has that part too, and of what stays empty in it at
+        # least 0.4 shows in its time; these sizes take 0.93 of the expected time.  Of 393 products of 1100 to 4096 rows and k of 512 to
+        # 8192 and 390 drawn ones this takes 85, at 0.92 of the vendor's time in the mean and 1.04 at most.  Left out: columns that
+        # leave in pieces below 16 bytes (up to 1.19), longer sums, whose empty part the vendor's products fill along k (9216 columns of
+        # 2048 rows, k = 2048 / 3072 / 4096 / 8192: 0.94, 1.00, 1.04, 1.08), and two whole rounds and a part (up to 1.05).
+        return 0.93 * us <= 7 + flops_us * (1 + 0.4 * (2 / rounds - 1))
     spare = (20 if rows <= 1024 else 7) + (0 if act is None else 4 + rows * out * (6 if glu else 4) / 3.5e6)
-    return native_mixers().tile_gemm_us(rows, out, k, glu) <= spare + 2.0 * rows * n * k / (1.3e9 if rows <= 1024 else 1.35e9)
+    return us <= spare + flops_us
 
 
 _replayed = threading.local()
