@@ -16,7 +16,7 @@ int mx_layer_norm(float* x, const void* y, int y_bf16, long y_stride, const floa
                   void* cast, int out_bf16, const float* next_w, const float* next_b, int rows, int width, float eps, hipStream_t s);
 int mx_tanh_cap(float* x, long n, float cap, hipStream_t s);
 int mx_grouped_gemm(void* C, const void* A, long a_rows, const int* rows, const void* W, const int* offs, int groups, long M,
-                    int N, int K, int act, float limit, hipStream_t s);
+                    int N, int K, int act, float limit, int form, hipStream_t s);
 int mx_few_rows_pair(void* Y, void* Y2, long y_stride, const void* X, const void* X2, long x_stride, int rows,
                      const void* W, const void* W2, int N, int K, hipStream_t s);
 int mx_few_rows_side_gate(void* Y, long y_stride, const void* X, long x_stride, int rows, const void* W, int N, int K,
@@ -446,8 +446,9 @@ void gather_add_rows(Tensor out, Tensor y, Tensor idx, Tensor w) {
                          out.size(0), (int)idx.size(1), (int)out.size(1), y.size(0), stream()), "gather_add_rows");
 }
 
-// out [M, N] = rows of a [M, K] (sorted by group, group g ends at offs[g]) times w[g]^T, w [G, N, K]; bf16
-void grouped_gemm(Tensor out, Tensor a, Tensor w, Tensor offs) {
+// out [M, N] = rows of a [M, K] (sorted by group, group g ends at offs[g]) times w[g]^T, w [G, N, K]; bf16.  form: below 0 the one
+// that is taken by itself
+void grouped_gemm(Tensor out, Tensor a, Tensor w, Tensor offs, int64_t form) {
   check_i32(offs, "offsets");
   TORCH_CHECK(a.is_cuda() && a.is_contiguous() && a.scalar_type() == at::kBFloat16 && a.dim() == 2, "a: bf16 [M, K]");
   TORCH_CHECK(w.is_cuda() && w.is_contiguous() && w.scalar_type() == at::kBFloat16 && w.dim() == 3 &&
@@ -456,7 +457,7 @@ void grouped_gemm(Tensor out, Tensor a, Tensor w, Tensor offs) {
               out.size(0) == a.size(0) && out.size(1) == w.size(1), "out: bf16 [M, N]");
   TORCH_CHECK(a.size(1) % 8 == 0 && a.size(1) >= 8, "K must be a multiple of 8");
   chk(mx_grouped_gemm(out.data_ptr(), a.data_ptr(), a.size(0), nullptr, w.data_ptr(), offs.data_ptr<int>(), (int)w.size(0),
-                      a.size(0), (int)w.size(1), (int)a.size(1), 0, 0.f, stream()), "grouped_gemm");
+                      a.size(0), (int)w.size(1), (int)a.size(1), 0, 0.f, (int)form, stream()), "grouped_gemm");
 }
 
 void clamp_swiglu(Tensor out, Tensor gu, double limit) {
@@ -1246,9 +1247,9 @@ void experts_many(Tensor out, Tensor h, Tensor idx, Tensor wts, Tensor wgu, Tens
   Tensor y = at::empty({pairs, ff}, h.options()), d = at::empty({pairs, width}, h.options());
   chk(mx_pair_sort(offs, row, place, idx.data_ptr<int>(), t, (int)top, experts, stream()), "pair_sort");
   chk(mx_grouped_gemm(y.data_ptr(), h.data_ptr(), t, row, wgu.data_ptr(), offs, experts, pairs, (int)ff, (int)width,
-                      (int)act, (float)limit, stream()), "grouped_gemm");
+                      (int)act, (float)limit, -1, stream()), "grouped_gemm");
   chk(mx_grouped_gemm(d.data_ptr(), y.data_ptr(), pairs, nullptr, wdown.data_ptr(), offs, experts, pairs, (int)width, (int)ff,
-                      0, 0.f, stream()), "grouped_gemm");
+                      0, 0.f, -1, stream()), "grouped_gemm");
   chk(mx_experts_merge(out.data_ptr<float>(), d.data_ptr(), place, wts.data_ptr<float>(),
                        shared ? shared->data_ptr() : nullptr, h.data_ptr(), h.stride(0),
                        gate_w ? gate_w->data_ptr() : nullptr, t, (int)top, (int)width, stream()), "experts_merge");

@@ -351,9 +351,11 @@ extern "C" int mx_tile_form_128();
 extern "C" int mx_tile_form_256();
 extern "C" int mx_tile_form_groups();
 
-// act: few_rows.h (0: none).  a_rows: rows of A (M without an index).  rows: A's row of every sorted row, or null.
+// act: few_rows.h (0: none).  a_rows: rows of A (M without an index).  rows: A's row of every sorted row, or null.  form: one of
+// tile_gemm.hip's for groups, kTilesHere for the kernel above, or below 0 the one that is taken by itself.
+enum { kTilesHere = 1000 };
 extern "C" int mx_grouped_gemm(void* C, const void* A, long a_rows, const int* rows, const void* W, const int* offs, int groups,
-                               long M, int N, int K, int act, float limit, hipStream_t s) {
+                               long M, int N, int K, int act, float limit, int form, hipStream_t s) {
   if (M <= 0 || N <= 0 || groups <= 0) return 0;
   if (K < 8 || K % 8 || M > 0x7fffffffL || act < kFrStore || act > kFrReluSq) return -1;
   if (((uintptr_t)A) % 16 || ((uintptr_t)W) % 16) return -2;
@@ -365,19 +367,22 @@ extern "C" int mx_grouped_gemm(void* C, const void* A, long a_rows, const int* r
   //   32 groups of 2048 -> 2 x 1024 (gated)  8 rows a group: 64 70 82 52; 56: 71 69 80 53; 125: - 86 81 61; 234: - 122 119 84; 512: -
   //   207 186 145;  128 of 768 -> 2048  4: 78 101 116 82; 28: 90 107 119 89; 88: - 129 137 112; 117: - 139 145 120
   //   16 of 1024 -> 2 x 256, 2 columns of tiles each  16: 12.7 - - 16.0; 300: - - 29.4 30.0;  4 of 512 -> 2 x 512  50: 8.8 - - 9.5
-  // Short k of few rows is the 64-row kernel's (32 of 1024 -> 2048, 8 rows: 26 and 28), and matrices that the last level cache does
-  // not hold are read twice where most groups are one tile and a piece (8 of 4096 -> 2 x 4096, 350 rows: 213 and 221; 64 of 4096
-  // -> 2 x 1408, 375: 598 and 623; 268 MB of them, 375: 119 and 113).
-  if (mx_tile_gemm_fits(a_rows, N, K, K, glu)) {
+  // Short k of few rows is the 64-row kernel's (32 of 1024 -> 2048, 8 rows: 26 and 28).  Matrices that the last level cache does not hold
+  // are read twice where the groups are a whole tile and a short piece, 257 to 384 rows: 256 x 256 / with shorter pieces, 280 320 350
+  // 375 | 400 425 450 475 rows a group on average, uneven: 16 of 4096 -> 4096 (512 MB) 206 214 209 207 | 217 216 214 219 / 209 217 219 218 | 212
+  // 210 212 207; 32 of 2048 -> 4096 (512 MB) 228 230 226 232 | 231 239 236 267 / 227 235 240 231 | 222 226 232 246; 16 of 4096 -> 8192 (1 GB)
+  // 408 417 419 418 | 419 420 423 425 / 407 422 435 440 | 424 414 416 424; 8 of 4096 -> 4096 (256 MB) 102 106 105 104 | 104 108 106
+  // 169 / 101 101 99 102 | 107 104 105 136
+  if (form < 0 && mx_tile_gemm_fits(a_rows, N, K, K, glu)) {
     const long wide = (long)groups * ((N + (glu ? 127 : 255)) / (glu ? 128 : 256)), w_bytes = 2L * groups * N * K * (glu ? 2 : 1);
-    const bool twice = w_bytes >= 512L << 20 && M > 256L * groups && M < 420L * groups;
-    int form = -1;
+    const bool twice = w_bytes >= 512L << 20 && M > 256L * groups && M <= 384L * groups;
     if (wide >= 128 && !twice && (K > 1024 || M >= 25L * groups)) form = mx_tile_form_groups();
     else if (M >= 120L * groups) form = mx_tile_form_256();
     else if (M >= 50L * groups) form = mx_tile_form_128();
-    if (form >= 0)
-      return mx_tile_gemm(C, N, A, K, a_rows, rows, W, nullptr, offs, groups, M, N, K, act, limit, form, s);
   }
+  if (form >= 0 && form != kTilesHere && form != mx_tile_form_groups() && form != mx_tile_form_256() && form != mx_tile_form_128()) return -4;
+  if (form >= 0 && form != kTilesHere)
+    return mx_tile_gemm(C, N, A, K, a_rows, rows, W, nullptr, offs, groups, M, N, K, act, limit, form, s);
   // 128-row tiles once the groups fill them on average
   const bool tall = M >= 96L * groups;
   const int cols = 128 / (glu ? 2 : 1), col_tiles = (N + cols - 1) / cols;

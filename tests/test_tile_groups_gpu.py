@@ -8,6 +8,7 @@ from fasttalk_llm_microservice_amd.ops import mixers as M
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
+GROUPS = 8                       # tile_groups_kernel among tile_gemm.hip's forms
 EDGES = [0, 1, 63, 64, 65, 127, 128, 129, 255, 256, 257, 320, 321, 384, 385, 512, 513]
 
 
@@ -23,17 +24,20 @@ def close(got, want, k, slope=1.0):
     assert bool((err <= bound).all()), float((err - bound).max())
 
 
+def product(a, w, counts):
+    out = torch.full((a.shape[0], w.shape[1]), 7.0, dtype=a.dtype, device=DEV)
+    M.native_mixers().grouped_gemm(out, a, w, torch.tensor(counts).cumsum(0).int().to(DEV), GROUPS)
+    return out
+
+
 @pytest.mark.parametrize("counts", [EDGES, [3] * 70 + [700] + [0] * 5 + [40] * 60, [0] * 63 + [130] + [0] * 64 + [1]])
 @pytest.mark.parametrize("k", [64, 192, 576, 1088])
 def test_plain_groups(counts, k):
     e = len(counts)
     n = 8 * (-(-128 // e) * 256 // 8) - 248          # 128 tiles of columns or more over all groups, the last one 8 wide
     rows = sum(counts)
-    if k <= 1024 and rows < 25 * e:                  # (few rows of short k are another kernel's)
-        counts = [c * 40 for c in counts]
-        rows *= 40
     a, w = rnd(e, rows, k), rnd(e + 1, e, n, k, scale=k ** -0.5)
-    got = M.grouped_mm(a, w, torch.tensor(counts).cumsum(0).int().to(DEV))
+    got = product(a, w, counts)
     s = 0
     for g, c in enumerate(counts):
         close(got[s:s + c], a[s:s + c].double() @ w[g].double().t(), k)
@@ -71,8 +75,8 @@ def test_equal_rows(before, count):
     row = rnd(2, 1, k)
     counts = [before[i % 3] for i in range(7)] + [count] + [20] * (e - 8)
     a = row.expand(sum(counts), k).contiguous()
-    got = M.grouped_mm(a, w, torch.tensor(counts).cumsum(0).int().to(DEV))
-    alone = M.grouped_mm(row.expand(e * 30, k).contiguous(), w, torch.tensor([30] * e).cumsum(0).int().to(DEV))
+    got = product(a, w, counts)
+    alone = product(row.expand(e * 30, k).contiguous(), w, [30] * e)
     s = 0
     for g, c in enumerate(counts):
         assert torch.equal(got[s:s + c], alone[30 * g:30 * g + 1].expand(c, n))
