@@ -319,8 +319,9 @@ extern "C" int mx_conv_delta_prep(float* qn, float* kn, float* vo, float* lg, fl
                                   long rows, int num_slots, int heads, int kv_heads, int dk, int dv, hipStream_t s) {
   if (rows <= 0 || num_segs <= 0) return 0;
   if (taps < 1 || taps > 16 || dk < 1 || dk > mx_head_max_dk() || dv < 1 || kv_heads < 1 || heads % kv_heads) return -1;
-  // rows per wave: a few once there are enough of them.  us with 1 2 4 8, 48 heads of 128: 300 rows 12.0 10.5 10.2 12.6, 500 19 14.3
-  // 12.5 13.7, 777 26 20.7 17.6 16.8, 2000 55 41 33 30 (64 4.6 5.9 8.5 13.6)
+  // rows per wave: a few once there are enough of them.  us with 1 2 4 8, 32 heads of 128 (8 of q and k): 300 rows 12.0 10.5 10.2 12.6, 500
+  // 19 14.3 12.5 13.7, 777 26 20.7 17.6 16.8, 2000 55 41 33 30 (64 4.6 5.9 8.5 13.6); 64 heads: 300 18.5 16.0 15.1 15.5, 500 26 20
+  // 17.4 18.2, 777 37 28 23.9 23.1; 128 heads: 300 31 25 23 27, 500 46 35 31 34, 777 66 48 41 42
   const int rb = rows < 256 ? 1 : rows < 640 && taps <= 4 ? 4 : 8, nu = dk <= 64 ? 1 : dk <= 128 ? 2 : 4;
   const int items = 2 * kv_heads + (heads * dv + 64 * nu - 1) / (64 * nu) + 1;
   if (rows > 0x7fffffffL || (items + 3) / 4 > 65535) return -2;

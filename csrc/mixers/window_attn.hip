@@ -675,10 +675,15 @@ extern "C" int mx_conv_attn_prep(float* q_out, const void* qkv, int bf16, long s
   const int channels = nq + nk + nv;
   const int chunks = (nq + nk) / head_dim + (nv + head_dim - 1) / head_dim;
   if (head_dim > 512 || rows > 0x7fffffffL || (chunks + 3) / 4 > 65535) return -3;
-  // rows per wave: a few once there are enough of them, as many as leave every CU some waves (a wave's rows are a chain).  us with 1 2
-  // 4 8, 24 heads of 128: 300 rows 9.4 8.8 10.4 14.3, 500 12.1 10.8 11.7 15.4, 777 16.5 13.5 13.0 15.6, 1000 21 17 14 18, 1500 30 25
-  // 21.5 20.9, 4096 66 56 43 38 (64 4.7 6.7 11 19)
-  const int rb = rows < 256 || head_dim > 256 || taps > 4 ? 1 : rows < 640 ? 2 : rows < 1280 ? 4 : 8;
+  // rows per wave: as many (up to 8) as leave every CU 16 waves, since a wave's rows are a chain.  us with 1 2 4 8 rows, heads of
+  // 128:  6 (q, k and v): 500 rows 8.3 8.2 9.9 15, 2048 15.0 13.5 13.2 15.9;  24: 300 9.4 8.9 10.5 15, 500 12.0 10.7 11.8 16, 777 16.9
+  // 14.6 13.6 16.3, 1500 29 24 21.5 21.2, 4096 66 56 43 38;  48: 300 13.8 12.4 12.0 16.4, 777 30 26 21.2 21.9;  80: 300 21 18 16.1 17.9,
+  // 640 38 33 27 25;  160: 300 37 31 25.4 24.9, 777 83 70 54 48.  Of these and 80 more it is 0.7 % from the best in the mean, 8 % at
+  // most (by rows alone, 256 / 640 / 1280 of them: 8 %, 75 %)
+  int rb = 1;
+  if (rows >= 256 && head_dim <= 256 && taps <= 4)
+    for (int n = 2; n <= 8; n *= 2)
+      if ((rows + n - 1) / n * chunks >= 16 * 256) rb = n;
   const int nu = head_dim <= 64 ? 1 : head_dim <= 128 ? 2 : head_dim <= 256 ? 4 : 8;
   const dim3 grid((unsigned)((rows + rb - 1) / rb), (unsigned)((chunks + 3) / 4)), block(256);
 #define MX_CPREP(T, TC, TAPS, NU, RB)                                                                            \

@@ -17,15 +17,16 @@ def move(seg, dev):
     return M.Segments(**{**seg.__dict__, **{k: getattr(seg, k).to(dev) for k in ("start", "pos0", "slot", "kv_len", "block_tables")}})
 
 
-@pytest.mark.parametrize("total", [255, 256, 639, 640, 1279, 1280])
+@pytest.mark.parametrize("heads,total", [(3, 255), (3, 256), (3, 639), (3, 640), (28, 272), (28, 274), (62, 255), (62, 256), (62, 504),
+                                         (62, 505), (3, 1639), (3, 1280)])
 @pytest.mark.parametrize("dk,interleaved", [(24, False), (128, True), (200, False)])
-def test_rows_of_a_wave(total, dk, interleaved):
+def test_rows_of_a_wave(heads, total, dk, interleaved):
     g = torch.Generator().manual_seed(total + dk)
     rows = [1, 1, 6, 30]
     rows += [total - sum(rows) - 1, 1]
     pos0, slots = [17, 0, 3, 0, 40, 9], [2, 0, 3, 1, 5, 4]
     seg, slot_map, nb = _segments("cuda", rows, pos0, slots, 16, pad=2)
-    H, G, taps = 3, 1, 4
+    H, G, taps = heads, 1, 4
     nq, nk, nv = H * dk, G * dk, G * dk
     c = nq + nk + nv
     qkv = (0.7 * torch.randn(total, c, generator=g)).bfloat16()
