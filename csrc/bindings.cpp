@@ -6,6 +6,8 @@
 // hipGraph-capturable (no allocation, no synchronisation).
 #include <torch/extension.h>
 #include <pybind11/numpy.h>
+#include <ATen/core/CachingHostAllocator.h>
+#include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime.h>
 
@@ -903,18 +905,23 @@ void set_kernel_checks(torch::Tensor word) {
 }
 #endif
 
-// dst = src, one of them on the device and the other in pinned host memory that outlives the copy (ordered on the current stream)
+// dst = src, one of them on the device and the other in pinned host memory, ordered on the current stream.  The host's may be freed
+// at once: its allocator is told of the stream, as a runtime copy tells it.  Memory that the device caches (non-coherent) is refused: the
+// kernel would read what an earlier copy left in a cache, and the host not see what it wrote.
 void host_copy(at::Tensor dst, at::Tensor src) {
   TORCH_CHECK(dst.is_contiguous() && src.is_contiguous() && dst.scalar_type() == src.scalar_type() && dst.numel() == src.numel() &&
               src.element_size() % 4 == 0 && dst.is_cuda() != src.is_cuda(), "host_copy: alike, contiguous, words");
   if (src.numel() == 0) return;
+  const at::Tensor& host = dst.is_cuda() ? src : dst;
   hipPointerAttribute_t attr{};
-  void* host = dst.is_cuda() ? src.data_ptr() : dst.data_ptr();
-  const bool pinned = hipPointerGetAttributes(&attr, host) == hipSuccess && attr.type == hipMemoryTypeHost && attr.devicePointer != nullptr;
+  const bool pinned = hipPointerGetAttributes(&attr, host.data_ptr()) == hipSuccess && attr.type == hipMemoryTypeHost &&
+                      attr.devicePointer != nullptr && !(attr.allocationFlags & hipHostMallocNonCoherent);
   if (!pinned) (void)hipGetLastError();
-  TORCH_CHECK(pinned, "host_copy: pinned host memory");
+  TORCH_CHECK(pinned, "host_copy: pinned, coherent host memory");
   check_rc(ft_host_copy(dst.is_cuda() ? dst.data_ptr() : attr.devicePointer, src.is_cuda() ? src.data_ptr() : attr.devicePointer,
                         src.numel() * (src.element_size() / 4), cur_stream()), "host_copy");
+  const at::DataPtr& mem = host.storage().data_ptr();
+  at::getHostAllocator(at::kCUDA)->record_event(mem.get(), mem.get_context(), c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().unwrap());
 }
 
 // Views of an int32 image on the device in the types and shapes of the host arrays that were packed into it, array i from word

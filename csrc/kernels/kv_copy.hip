@@ -74,7 +74,9 @@ extern "C" int ft_kv_swap(const uint64_t* ptrs_dev, int ncache, const int* ids_d
 
 // A step's inputs from pinned host memory, or its results into it, by a kernel over the link: `words` of 4 bytes.  Bound by the link's
 // latency and, from a few hundred KB on, its rate.  A runtime copy of this size is a launch of its own kind, and the queue
-// passes from it to a graph and back only after 6 to 11 us: a decode step's 16 to 130 KB cost 13 to 16 us less so.
+// passes from it to a graph and back only after 6 to 11 us: a decode step's 16 to 130 KB cost 13 to 16 us less so.  No fence beside the
+// launch's own: the memory is coherent (the caller looks), which no cache of the device keeps, so its loads see what the host wrote before
+// the launch and the host its stores once the stream has passed.
 namespace ft {
 
 __global__ __launch_bounds__(256) void host_copy_kernel(uint32_t* __restrict__ dst, const uint32_t* __restrict__ src, long words,

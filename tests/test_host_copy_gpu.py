@@ -27,6 +27,28 @@ def test_words(n, off, dtype):
         d.zero_()
 
 
+def test_memory_freed_under_a_copy():
+    """Pinned memory that is freed while a copy is queued is not given to the next tensor before that has run."""
+    n = 1 << 16
+    a = torch.randn(4096, 4096, device="cuda")
+    d = torch.zeros(n, dtype=torch.int32, device="cuda")
+    torch.cuda.synchronize()
+    for to_host in (False, True):
+        h = torch.full((n,), 5, dtype=torch.int32, pin_memory=True)
+        at = h.data_ptr()
+        for _ in range(40):                     # (milliseconds of work in front of the copy)
+            b = a @ a
+        ops.native().host_copy(h, d) if to_host else ops.native().host_copy(d, h)
+        done = torch.cuda.Event()
+        done.record()
+        del h
+        new = torch.full((n,), 9, dtype=torch.int32, pin_memory=True)
+        assert not done.query() and new.data_ptr() != at
+        done.synchronize()
+        assert bool((new == 9).all()) and bool((d == 5).all())
+    del b
+
+
 def test_refused():
     d, pinned = torch.zeros(8, dtype=torch.int32, device="cuda"), torch.zeros(8, dtype=torch.int32, pin_memory=True)
     for a, b in ((d, torch.zeros(8, dtype=torch.int32)), (d, d), (pinned, pinned), (d[:4], pinned), (d[::2], pinned[:4]),
