@@ -905,10 +905,17 @@ void set_kernel_checks(torch::Tensor word) {
 }
 #endif
 
+// The allocator of pinned memory does not hand on t's, once t is freed, before the current stream has passed what is queued by then.
+void host_in_use(at::Tensor t) {
+  const at::DataPtr& mem = t.storage().data_ptr();
+  at::getHostAllocator(at::kCUDA)->record_event(mem.get(), mem.get_context(), c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().unwrap());
+}
+
 // dst = src, one of them on the device and the other in pinned host memory, ordered on the current stream.  The host's may be freed
-// at once: its allocator is told of the stream, as a runtime copy tells it.  Memory that the device caches (non-coherent) is refused: the
+// at once (host_in_use), as after a runtime copy; a caller that waits for the stream before it frees it says `held` and has no
+// event recorded and asked for when it does (20 us of a prompt's step).  Memory that the device caches (non-coherent) is refused: the
 // kernel would read what an earlier copy left in a cache, and the host not see what it wrote.
-void host_copy(at::Tensor dst, at::Tensor src) {
+void host_copy(at::Tensor dst, at::Tensor src, bool held) {
   TORCH_CHECK(dst.is_contiguous() && src.is_contiguous() && dst.scalar_type() == src.scalar_type() && dst.numel() == src.numel() &&
               src.element_size() % 4 == 0 && dst.is_cuda() != src.is_cuda(), "host_copy: alike, contiguous, words");
   if (src.numel() == 0) return;
@@ -920,8 +927,7 @@ void host_copy(at::Tensor dst, at::Tensor src) {
   TORCH_CHECK(pinned, "host_copy: pinned, coherent host memory");
   check_rc(ft_host_copy(dst.is_cuda() ? dst.data_ptr() : attr.devicePointer, src.is_cuda() ? src.data_ptr() : attr.devicePointer,
                         src.numel() * (src.element_size() / 4), cur_stream()), "host_copy");
-  const at::DataPtr& mem = host.storage().data_ptr();
-  at::getHostAllocator(at::kCUDA)->record_event(mem.get(), mem.get_context(), c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().unwrap());
+  if (!held) host_in_use(host);
 }
 
 // Views of an int32 image on the device in the types and shapes of the host arrays that were packed into it, array i from word
@@ -956,7 +962,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.attr("kernel_checks") = false;
 #endif
   m.def("cut_words", &cut_words);
-  m.def("host_copy", &host_copy);
+  m.def("host_copy", &host_copy, py::arg("dst"), py::arg("src"), py::arg("held") = false);
+  m.def("host_in_use", &host_in_use);
   m.def("rmsnorm", &rmsnorm);
   m.def("fused_add_rmsnorm", &fused_add_rmsnorm);
   m.def("silu_mul", &silu_mul);

@@ -77,8 +77,7 @@ def _input_views(buf: torch.Tensor, mb: int, max_blocks: int):
 
 
 def _copy(dst: torch.Tensor, src: torch.Tensor, pinned: bool):
-    """Queues a copy between the device and host memory, which stays until the stream has passed it; ``pinned``: by a kernel,
-    which a graph's first launch follows at once."""
+    """Queues a copy between the device and host memory; ``pinned``: by a kernel, which a graph's first launch follows at once."""
     if pinned:
         ops.native().host_copy(dst, src)
     else:
@@ -647,8 +646,12 @@ class ModelRunner:
             if not self.is_gpu:
                 return logits.numpy()
             out = torch.empty(logits.shape, dtype=torch.float32, pin_memory=True)
-            _copy(out, logits.contiguous(), True)
-            self._wait()
+            ops.native().host_copy(out, logits.contiguous(), held=True)
+            try:
+                self._wait()
+            except BaseException:
+                ops.native().host_in_use(out)     # (freed with the copy still queued)
+                raise
             return out.numpy()
         if not has_logits:
             # a middle chunk of a chunked prefill samples nothing, but its all-reduces

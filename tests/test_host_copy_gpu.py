@@ -33,12 +33,14 @@ def test_memory_freed_under_a_copy():
     a = torch.randn(4096, 4096, device="cuda")
     d = torch.zeros(n, dtype=torch.int32, device="cuda")
     torch.cuda.synchronize()
-    for to_host in (False, True):
+    for to_host, held in ((False, False), (True, False), (True, True)):
         h = torch.full((n,), 5, dtype=torch.int32, pin_memory=True)
         at = h.data_ptr()
         for _ in range(40):                     # (milliseconds of work in front of the copy)
             b = a @ a
-        ops.native().host_copy(h, d) if to_host else ops.native().host_copy(d, h)
+        ops.native().host_copy(*((h, d) if to_host else (d, h)), held=held)
+        if held:                                # (the wait that was to come does not)
+            ops.native().host_in_use(h)
         done = torch.cuda.Event()
         done.record()
         del h
