@@ -446,18 +446,19 @@ void gather_add_rows(Tensor out, Tensor y, Tensor idx, Tensor w) {
                          out.size(0), (int)idx.size(1), (int)out.size(1), y.size(0), stream()), "gather_add_rows");
 }
 
-// out [M, N] = rows of a [M, K] (sorted by group, group g ends at offs[g]) times w[g]^T, w [G, N, K]; bf16.  form: below 0 the one
-// that is taken by itself
-void grouped_gemm(Tensor out, Tensor a, Tensor w, Tensor offs, int64_t form) {
+// out [M, N] = act(rows of a [M, K] (sorted by group, group g ends at offs[g]) times w[g]^T), w [G, N, K], gated forms
+// [G, 2 N, K]; bf16.  form: below 0 the one that is taken by itself
+void grouped_gemm(Tensor out, Tensor a, Tensor w, Tensor offs, int64_t act, double limit, int64_t form) {
   check_i32(offs, "offsets");
+  TORCH_CHECK(act >= 0 && act <= 5, "grouped_gemm: activation");
   TORCH_CHECK(a.is_cuda() && a.is_contiguous() && a.scalar_type() == at::kBFloat16 && a.dim() == 2, "a: bf16 [M, K]");
   TORCH_CHECK(w.is_cuda() && w.is_contiguous() && w.scalar_type() == at::kBFloat16 && w.dim() == 3 &&
               w.size(2) == a.size(1) && offs.numel() == w.size(0), "w: bf16 [G, N, K], offsets [G]");
   TORCH_CHECK(out.is_cuda() && out.is_contiguous() && out.scalar_type() == at::kBFloat16 && out.dim() == 2 &&
-              out.size(0) == a.size(0) && out.size(1) == w.size(1), "out: bf16 [M, N]");
+              out.size(0) == a.size(0) && out.size(1) * (act >= 1 && act <= 4 ? 2 : 1) == w.size(1), "out: bf16 [M, N]");
   TORCH_CHECK(a.size(1) % 8 == 0 && a.size(1) >= 8, "K must be a multiple of 8");
   chk(mx_grouped_gemm(out.data_ptr(), a.data_ptr(), a.size(0), nullptr, w.data_ptr(), offs.data_ptr<int>(), (int)w.size(0),
-                      a.size(0), (int)w.size(1), (int)a.size(1), 0, 0.f, (int)form, stream()), "grouped_gemm");
+                      a.size(0), (int)out.size(1), (int)a.size(1), (int)act, (float)limit, (int)form, stream()), "grouped_gemm");
 }
 
 void clamp_swiglu(Tensor out, Tensor gu, double limit) {

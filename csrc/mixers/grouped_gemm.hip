@@ -18,8 +18,8 @@
 // taller tile empty).  The tiles run group by group, bands of eight row tiles with their columns after each
 // other, and each XCD (workgroup id mod 8) takes one contiguous eighth of that order, so the tiles in flight on
 // an XCD share an expert's rows and columns in its L2.
-// Serves short groups of small sets, where it is bound by the read of the matrices, and rows that are no whole stages of
-// tile_gemm.hip's: the others go there (mx_grouped_gemm has the lines and both sides).  1800 pairs of 32 experts, 2048 -> 2 x 1024 gated (268 MB):
+// Serves short groups that do not fill the card otherwise, where it is bound by the read of the matrices, and rows that are no whole
+// stages of tile_gemm.hip's: the others go there (grouped_form has the lines and both sides).  1800 pairs of 32 experts, 2048 -> 2 x 1024 gated (268 MB):
 // 78 us in a model, with one step of loads in flight, a barrier between reads and products and tiles in grid order 98.
 #include "few_rows.h"
 
@@ -351,9 +351,46 @@ extern "C" int mx_tile_form_128();
 extern "C" int mx_tile_form_256();
 extern "C" int mx_tile_form_groups();
 
+enum { kTilesHere = 1000 };
+
+// The form for rows of whole stages, by rows a group on average and by how far the tiles fill the card (a workgroup a CU in tile_gemm.hip's).
+//
+// By rows alone: 64-row tiles here, 128 x 128 from 50, 256 x 256 from 120.  Short pieces beside whole tiles (tile_groups_kernel) instead
+// while columns do not leave a quarter of the tiles empty, and:
+//  * up to 120 rows, a piece a group: where the last round of pieces over the 256 CUs is full to 144 of them or there are two before it.  Its
+//    time over the other form's, by pieces (groups that have rows, times columns of tiles) 60-100 100-128 150-200 225-256 256-350 350-420
+//    420-512 more:  50 to 90 rows 1.38 1.24 0.86 0.92 1.04 1.00 0.89 0.90;  20 to 50 rows 1.27 1.14 0.89 0.95 1.10 1.00 0.95 1.01;
+//    below 20 1.30 1.18 0.91 1.01 1.12 1.05 1.02 1.07.  In the last two rows only where it is below 1.
+//  * so too with more pieces where a matrix's rows are whole 4 KB, which meet on few of the memory's channels in the other forms (tile_first_stage):
+//    0.80 to 0.95, with more than 768 pieces of below 20 rows 1.07.
+//  * from 120 rows on while whole tiles leave a short last piece or a few groups end just past one: up to 128 rows past whole tiles 0.86 to
+//    0.97, 220 to 255 0.95 to 1.0, between these all are whole tiles and it is behind by the rounding of both sorts (1.01 to 1.04, up to
+//    1.5; rows of 4 KB 0.94).  Of sets of 256 MB and more, which the last level cache does not hold, the short pieces read the matrices a
+//    second time: at 24 to 128 rows past a whole tile 1.05 (320 to 384), 1.05 (560 to 640).
+// Over 4300 products of 2 to 256 groups, 1 to 900 rows each, sizes at random (1500 of them after the lines were drawn): 0.982 of the time by
+// rows alone in the mean, above 1.03 in 68 and above 1.1 in 12 of them.
+static int grouped_form(int groups, long M, int N, int K, bool glu) {
+  const int width = glu ? 128 : 256, cols = (N + width - 1) / width;
+  const float mean = (float)M / groups;
+  const int by_rows = mean >= 120.f ? mx_tile_form_256() : mean >= 50.f ? mx_tile_form_128() : kTilesHere;
+  if (4L * N < 3L * cols * width) return by_rows;
+  const bool in_step = K % 2048 == 0;
+  if (mean < 120.f) {
+    const float pieces = groups * (1.f - expf(-mean)) * cols;              // (rows that choose their groups independently)
+    const int rounds = (int)ceilf(pieces / 256.f);
+    if (rounds <= 2 && pieces - 256.f * (rounds - 1) < 144.f) return by_rows;
+    const bool few = mean >= 20.f ? rounds <= (in_step ? rounds : 2) : in_step ? rounds <= 3 : pieces <= 200.f;
+    return mean >= 50.f || few ? mx_tile_form_groups() : by_rows;
+  }
+  if ((long)groups * cols < 128) return by_rows;
+  const long past = M / groups % 256;
+  if (past >= 128 && past < 220) return in_step ? mx_tile_form_groups() : by_rows;
+  const bool twice = 2L * groups * N * K * (glu ? 2 : 1) >= 256L << 20 && M > 256L * groups && past > 24 && past <= 128;
+  return twice ? by_rows : mx_tile_form_groups();
+}
+
 // act: few_rows.h (0: none).  a_rows: rows of A (M without an index).  rows: A's row of every sorted row, or null.  form: one of
 // tile_gemm.hip's for groups, kTilesHere for the kernel above, or below 0 the one that is taken by itself.
-enum { kTilesHere = 1000 };
 extern "C" int mx_grouped_gemm(void* C, const void* A, long a_rows, const int* rows, const void* W, const int* offs, int groups,
                                long M, int N, int K, int act, float limit, int form, hipStream_t s) {
   if (M <= 0 || N <= 0 || groups <= 0) return 0;
@@ -362,24 +399,7 @@ extern "C" int mx_grouped_gemm(void* C, const void* A, long a_rows, const int* r
   const bool glu = act >= kFrGelu && act <= kFrClamp;
   const int vec = N % 4 == 0 && ((uintptr_t)C) % 8 == 0;
   if ((M + 63) / 64 + groups > 65535) return -3;
-  // tile_gemm.hip's tiles wherever rows are whole stages, by what fills the card.  us, 64-row tiles here / 128 x 128 / 256 x 256 /
-  // 256 x 256 with shorter last pieces, matrices from HBM:
-  //   32 groups of 2048 -> 2 x 1024 (gated)  8 rows a group: 64 70 82 52; 56: 71 69 80 53; 125: - 86 81 61; 234: - 122 119 84; 512: -
-  //   207 186 145;  128 of 768 -> 2048  4: 78 101 116 82; 28: 90 107 119 89; 88: - 129 137 112; 117: - 139 145 120
-  //   16 of 1024 -> 2 x 256, 2 columns of tiles each  16: 12.7 - - 16.0; 300: - - 29.4 30.0;  4 of 512 -> 2 x 512  50: 8.8 - - 9.5
-  // Short k of few rows is the 64-row kernel's (32 of 1024 -> 2048, 8 rows: 26 and 28).  Matrices that the last level cache does not hold
-  // are read twice where the groups are a whole tile and a short piece, 257 to 384 rows: 256 x 256 / with shorter pieces, 280 320 350
-  // 375 | 400 425 450 475 rows a group on average, uneven: 16 of 4096 -> 4096 (512 MB) 206 214 209 207 | 217 216 214 219 / 209 217 219 218 | 212
-  // 210 212 207; 32 of 2048 -> 4096 (512 MB) 228 230 226 232 | 231 239 236 267 / 227 235 240 231 | 222 226 232 246; 16 of 4096 -> 8192 (1 GB)
-  // 408 417 419 418 | 419 420 423 425 / 407 422 435 440 | 424 414 416 424; 8 of 4096 -> 4096 (256 MB) 102 106 105 104 | 104 108 106
-  // 169 / 101 101 99 102 | 107 104 105 136
-  if (form < 0 && mx_tile_gemm_fits(a_rows, N, K, K, glu)) {
-    const long wide = (long)groups * ((N + (glu ? 127 : 255)) / (glu ? 128 : 256)), w_bytes = 2L * groups * N * K * (glu ? 2 : 1);
-    const bool twice = w_bytes >= 512L << 20 && M > 256L * groups && M <= 384L * groups;
-    if (wide >= 128 && !twice && (K > 1024 || M >= 25L * groups)) form = mx_tile_form_groups();
-    else if (M >= 120L * groups) form = mx_tile_form_256();
-    else if (M >= 50L * groups) form = mx_tile_form_128();
-  }
+  if (form < 0 && mx_tile_gemm_fits(a_rows, N, K, K, glu)) form = grouped_form(groups, M, N, K, glu);
   if (form >= 0 && form != kTilesHere && form != mx_tile_form_groups() && form != mx_tile_form_256() && form != mx_tile_form_128()) return -4;
   if (form >= 0 && form != kTilesHere)
     return mx_tile_gemm(C, N, A, K, a_rows, rows, W, nullptr, offs, groups, M, N, K, act, limit, form, s);

@@ -1665,7 +1665,7 @@ def grouped_mm(a, w, offsets, counts=None):
     sizes on the host, read from ``offsets`` when not given)."""
     if grouped_mm_is_one_product(a, w):
         out = torch.empty(a.shape[0], w.shape[1], dtype=a.dtype, device=a.device)
-        native_mixers().grouped_gemm(out, a.contiguous(), w, offsets, -1)
+        native_mixers().grouped_gemm(out, a.contiguous(), w, offsets, 0, 0.0, -1)
         return out
     if counts is None:
         ends = offsets.tolist()

@@ -24,9 +24,9 @@ def close(got, want, k, slope=1.0):
     assert bool((err <= bound).all()), float((err - bound).max())
 
 
-def product(a, w, counts):
-    out = torch.full((a.shape[0], w.shape[1]), 7.0, dtype=a.dtype, device=DEV)
-    M.native_mixers().grouped_gemm(out, a, w, torch.tensor(counts).cumsum(0).int().to(DEV), GROUPS)
+def product(a, w, counts, act=None):
+    out = torch.full((a.shape[0], w.shape[1] // (2 if act else 1)), 7.0, dtype=a.dtype, device=DEV)
+    M.native_mixers().grouped_gemm(out, a, w, torch.tensor(counts).cumsum(0).int().to(DEV), M.FEW_ACTS[act], 0.0, GROUPS)
     return out
 
 
@@ -41,6 +41,18 @@ def test_plain_groups(counts, k):
     s = 0
     for g, c in enumerate(counts):
         close(got[s:s + c], a[s:s + c].double() @ w[g].double().t(), k)
+        s += c
+
+
+@pytest.mark.parametrize("k", [64, 576])
+@pytest.mark.parametrize("n", [8, 136])
+def test_gated_groups(k, n):
+    a, w = rnd(n, sum(EDGES), k), rnd(n + 1, len(EDGES), 2 * n, k, scale=k ** -0.5)
+    got = product(a, w, EDGES, "silu")
+    s = 0
+    for g, c in enumerate(EDGES):
+        u = a[s:s + c].double() @ w[g].double().t()
+        close(got[s:s + c], u[:, :n] * torch.sigmoid(u[:, :n]) * u[:, n:], k, slope=8.0)
         s += c
 
 
