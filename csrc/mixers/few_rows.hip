@@ -8,6 +8,8 @@
 // The core and its layout: few_rows.h.
 #include "few_rows.h"
 
+#include <type_traits>
+
 namespace mx {
 
 constexpr int kFewRows = 64;       // most rows of X
@@ -187,8 +189,8 @@ __device__ __forceinline__ int rows_of(const int* __restrict__ idx, int pairs, i
 }
 
 // steps of k a round (expert_tile_any)
-template <int MB>
-constexpr int kExpSteps = MB == 1 ? 2 : 1;
+template <bool AHEAD>
+constexpr int kExpSteps = AHEAD ? 2 : 1;
 
 // the tile's sums for the listed rows: f(entry row in the list, column, sums, up sums)
 template <int P, bool GLU, int NB, int WV, int U, bool AHEAD, typename F>
@@ -223,14 +225,14 @@ __device__ __forceinline__ void expert_tile(float4* red, const bf16_t* W, int N,
 }
 
 // blocks of 16 rows that the listed rows fill, at most MB.  Steps of at most 16 rows name few experts, whose tiles leave a
-// CU one to three workgroups: two steps of k a round, and the next one's loads under it.  us of both products and the shared
+// CU one to three workgroups: two steps of k a round, and the next one's loads under it (AHEAD).  us of both products and the shared
 // expert's, one step a round / so: 3 rows, top 4 of 32 gated experts of 1024 44 / 37.5; 4 rows and a shared one of 2048 55 / 45;
 // 8 of 1536 (relu^2) 67 / 64; 16 rows 73 / 74.  With more rows the CU is full and the registers cost more (64 rows, top 6: 85 / 93).
-template <int P, bool GLU, int WV, int MB, typename F>
+template <int P, bool GLU, int WV, int MB, bool AHEAD, typename F>
 __device__ __forceinline__ void expert_tile_any(float4* red, const bf16_t* W, int N, int K, int n0, const bf16_t* X,
                                                 long x_stride, const int* list, int count, int div, int wave, int lane,
                                                 F out) {
-  if (MB == 1) expert_tile<P, GLU, 1, WV, kExpSteps<1>, true>(red, W, N, K, n0, X, x_stride, list, count, div, wave, lane, out);
+  if (MB == 1) expert_tile<P, GLU, 1, WV, kExpSteps<AHEAD>, AHEAD>(red, W, N, K, n0, X, x_stride, list, count, div, wave, lane, out);
   else if (count <= 16) expert_tile<P, GLU, 1, WV, 1, false>(red, W, N, K, n0, X, x_stride, list, count, div, wave, lane, out);
   else if (MB == 2 || count <= 32) expert_tile<P, GLU, 2, WV, 1, false>(red, W, N, K, n0, X, x_stride, list, count, div, wave, lane, out);
   else expert_tile<P, GLU, MB, WV, 1, false>(red, W, N, K, n0, X, x_stride, list, count, div, wave, lane, out);
@@ -241,16 +243,16 @@ __device__ __forceinline__ void expert_tile_any(float4* red, const bf16_t* W, in
 // the workgroup past the shared expert's last tile.
 constexpr int kExpWaves = 4;
 // X stages and partial sums (two tiles) of a tile with MB blocks of rows
-template <int MB>
-constexpr int kExpLds = kExpWaves * (kFrStage<MB, kExpSteps<MB>> > 2048 * MB ? kFrStage<MB, kExpSteps<MB>> : 2048 * MB);
+template <int MB, bool AHEAD>
+constexpr int kExpLds = kExpWaves * (kFrStage<MB, kExpSteps<AHEAD>> > 2048 * MB ? kFrStage<MB, kExpSteps<AHEAD>> : 2048 * MB);
 
-template <bool GLU, int MB>
+template <bool GLU, int MB, bool AHEAD>
 __global__ void __launch_bounds__(64 * kExpWaves)
 experts_first_kernel(bf16_t* __restrict__ y, bf16_t* __restrict__ ys, float* __restrict__ sg,
                      const bf16_t* __restrict__ h, long h_stride, int rows, const int* __restrict__ idx, int top,
                      ExpertSet E, int act, float limit, float shared_limit) {
   constexpr int P = GLU ? 1 : 2;
-  __shared__ float4 red[kExpLds<MB> / 16];
+  __shared__ float4 red[kExpLds<MB, AHEAD> / 16];
   __shared__ int list[kFewRows], counts[kExpWaves];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -263,7 +265,7 @@ experts_first_kernel(bf16_t* __restrict__ y, bf16_t* __restrict__ ys, float* __r
     const int count = rows_of<kExpWaves>(idx, rows * top, top, E.experts, e, 16 * MB, list, counts, shared);
     if (count == 0) return;
     const bf16_t* W = E.w + (long)e * E.N * (GLU ? 2 : 1) * E.K;
-    expert_tile_any<P, GLU, kExpWaves, MB>(red, W, E.N, E.K, n0, h, h_stride, list, count, top, wave, lane,
+    expert_tile_any<P, GLU, kExpWaves, MB, AHEAD>(red, W, E.N, E.K, n0, h, h_stride, list, count, top, wave, lane,
                                        [&](int r, int c, float (&v)[4], float (&u)[4]) {
 #pragma unroll
                                          for (int i = 0; i < 4; ++i) v[i] = fr_act(act, limit, v[i], u[i]);
@@ -277,11 +279,11 @@ experts_first_kernel(bf16_t* __restrict__ y, bf16_t* __restrict__ ys, float* __r
   __syncthreads();
   if ((int)blockIdx.x == tiles) {
     const bf16_t* W = E.shared + (long)E.shared_N * (GLU ? 2 : 1) * E.K;
-    expert_tile_any<1, false, kExpWaves, MB>(red, W, 1, E.K, 0, h, h_stride, list, rows, 1, wave, lane,
+    expert_tile_any<1, false, kExpWaves, MB, AHEAD>(red, W, 1, E.K, 0, h, h_stride, list, rows, 1, wave, lane,
                                          [&](int r, int c, float (&v)[4], float (&)[4]) { if (c == 0) sg[r] = v[0]; });
     return;
   }
-  expert_tile_any<P, GLU, kExpWaves, MB>(red, E.shared, E.shared_N, E.K, n0, h, h_stride, list, rows, 1, wave, lane,
+  expert_tile_any<P, GLU, kExpWaves, MB, AHEAD>(red, E.shared, E.shared_N, E.K, n0, h, h_stride, list, rows, 1, wave, lane,
                                      [&](int r, int c, float (&v)[4], float (&u)[4]) {
 #pragma unroll
                                        for (int i = 0; i < 4; ++i) v[i] = fr_act(act, shared_limit, v[i], u[i]);
@@ -290,12 +292,12 @@ experts_first_kernel(bf16_t* __restrict__ y, bf16_t* __restrict__ ys, float* __r
 }
 
 // d[pair] = W_down of the pair's expert times y[pair], ds[row] the shared expert's, fp32
-template <int MB>
+template <int MB, bool AHEAD>
 __global__ void __launch_bounds__(64 * kExpWaves)
 experts_down_kernel(float* __restrict__ d, float* __restrict__ ds, const bf16_t* __restrict__ y,
                     const bf16_t* __restrict__ ys, int rows, const int* __restrict__ idx, int top, ExpertSet E) {
   constexpr int P = 2;
-  __shared__ float4 red[kExpLds<MB> / 16];
+  __shared__ float4 red[kExpLds<MB, AHEAD> / 16];
   __shared__ int list[kFewRows], counts[kExpWaves];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -318,7 +320,7 @@ experts_down_kernel(float* __restrict__ d, float* __restrict__ ds, const bf16_t*
     X = ys;
     K = E.shared_K;
   }
-  expert_tile_any<P, false, kExpWaves, MB>(red, W, E.N, K, n0, X, K, list, count, 1, wave, lane,
+  expert_tile_any<P, false, kExpWaves, MB, AHEAD>(red, W, E.N, K, n0, X, K, list, count, 1, wave, lane,
                                        [&](int r, int c, float (&v)[4], float (&)[4]) {
                                          const int p = list[r];
                                          fr_store4(dst + (long)p * E.N, c, E.N, true, v);
@@ -448,25 +450,44 @@ extern "C" int mx_experts_few(float* out, void* y, float* d, const void* h, long
   const int cols = glu ? 16 : 32;
   const bool sh = shared_w != nullptr;
   const int tiles = (ff + cols - 1) / cols, tiles_s = sh ? (shared_ff + cols - 1) / cols + (sg != nullptr) : 0;
-  const int slots = experts <= 64 && rows * top < experts ? rows * top : experts;
-  ExpertSet first{(const bf16_t*)wgu, (const bf16_t*)shared_w, experts, width, ff, width, shared_ff, slots};
-  const dim3 g1((unsigned)(tiles > tiles_s ? tiles : tiles_s), (unsigned)(slots + (sh ? 1 : 0))), block(64 * kExpWaves);
-  ExpertSet down{(const bf16_t*)wdown, (const bf16_t*)shared_down, experts, ff, width, shared_ff, width, slots};
-  const dim3 g2((unsigned)((width + 31) / 32), g1.y);
-#define EX_FIRST(GLU, MB)                                                                                              \
-  hipLaunchKernelGGL((experts_first_kernel<GLU, MB>), g1, block, 0, s, (bf16_t*)y, (bf16_t*)ys, sg, (const bf16_t*)h, \
-                     h_stride, rows, idx, top, first, act, limit, shared_limit)
-#define EX_GO(MB)                                                                                                   \
-  do {                                                                                                              \
-    if (glu) EX_FIRST(true, MB); else EX_FIRST(false, MB);                                                          \
-    hipLaunchKernelGGL((experts_down_kernel<MB>), g2, block, 0, s, d, ds, (const bf16_t*)y, (const bf16_t*)ys, rows, \
-                       idx, top, down);                                                                          \
-  } while (0)
-  if (rows <= 16) EX_GO(1);
-  else if (rows <= 32) EX_GO(2);
-  else EX_GO(4);
-#undef EX_GO
-#undef EX_FIRST
+  // The lines below are from 700 layers of at most 16 rows, 4 to 128 experts, sizes at random.  Rows of the grid per pair: less than 150
+  // workgroups spared cost up to 0.9 us (the choices are read first), 150 to 300 are level (-3 to 1), 300 to 600 save 0.5, 1000 1.2 and
+  // more 2 to 5.  Loads ahead: 1.01 to 1.12 of the time at 1 to 3 steps of k a wave, whatever the grid; from 4 on 0.94 to 0.99 up to a
+  // workgroup a CU, 0.96 to 0.99 with three and more, between these 1.00 to 1.03 (up to 1.2).  So chosen 0.970 of the time with neither in
+  // the mean, above 1.03 in 3 %.
+  const int pairs = rows * top;
+  const auto slots = [&](int cols) { return experts <= 64 && pairs < experts && (long)(experts - pairs) * cols >= 150 ? pairs : experts; };
+  // workgroups that have rows, where the rows choose their experts independently
+  const float chosen = experts * (1.f - powf(1.f - (float)(top < experts ? top : experts) / experts, (float)rows));
+  const auto ahead = [&](int k, int cols, int shared_cols) {
+    const float groups = chosen * cols + shared_cols;
+    return (k + 63) / 64 > 3 * kExpWaves && (groups <= 256.f || groups > 700.f);
+  };
+  const int tiles_d = (width + 31) / 32;
+  ExpertSet first{(const bf16_t*)wgu, (const bf16_t*)shared_w, experts, width, ff, width, shared_ff, slots(tiles)};
+  ExpertSet down{(const bf16_t*)wdown, (const bf16_t*)shared_down, experts, ff, width, shared_ff, width, slots(tiles_d)};
+  const dim3 g1((unsigned)(tiles > tiles_s ? tiles : tiles_s), (unsigned)(first.slots + (sh ? 1 : 0))), block(64 * kExpWaves);
+  const dim3 g2((unsigned)tiles_d, (unsigned)(down.slots + (sh ? 1 : 0)));
+  const auto go = [&](auto mb, auto first_ahead, auto down_ahead) {
+    constexpr int MB = decltype(mb)::value;
+    constexpr bool AF = decltype(first_ahead)::value, AD = decltype(down_ahead)::value;
+    if (glu)
+      hipLaunchKernelGGL((experts_first_kernel<true, MB, AF>), g1, block, 0, s, (bf16_t*)y, (bf16_t*)ys, sg, (const bf16_t*)h, h_stride, rows,
+                         idx, top, first, act, limit, shared_limit);
+    else
+      hipLaunchKernelGGL((experts_first_kernel<false, MB, AF>), g1, block, 0, s, (bf16_t*)y, (bf16_t*)ys, sg, (const bf16_t*)h, h_stride, rows,
+                         idx, top, first, act, limit, shared_limit);
+    hipLaunchKernelGGL((experts_down_kernel<MB, AD>), g2, block, 0, s, d, ds, (const bf16_t*)y, (const bf16_t*)ys, rows, idx, top, down);
+  };
+  const bool a1 = ahead(width, tiles, tiles_s), a2 = ahead(ff, tiles_d, sh ? tiles_d : 0);
+  using std::bool_constant;
+  using std::integral_constant;
+  if (rows > 32) go(integral_constant<int, 4>{}, bool_constant<false>{}, bool_constant<false>{});
+  else if (rows > 16) go(integral_constant<int, 2>{}, bool_constant<false>{}, bool_constant<false>{});
+  else if (a1 && a2) go(integral_constant<int, 1>{}, bool_constant<true>{}, bool_constant<true>{});
+  else if (a1) go(integral_constant<int, 1>{}, bool_constant<true>{}, bool_constant<false>{});
+  else if (a2) go(integral_constant<int, 1>{}, bool_constant<false>{}, bool_constant<true>{});
+  else go(integral_constant<int, 1>{}, bool_constant<false>{}, bool_constant<false>{});
   if (out == nullptr) return (int)hipGetLastError();       // (the step behind sums them: rows.hip, ExpertRows)
   hipLaunchKernelGGL(experts_combine_kernel, dim3((unsigned)((width + 255) / 256), (unsigned)rows), dim3(256), 0, s,
                      out, d, wts, sh ? ds : nullptr, sg, top, width);

@@ -1,6 +1,7 @@
 """Experts of fewer (row, choice) pairs than experts (csrc/mixers/few_rows.hip: the grid has a row per choice, and the next
 round's loads are in flight under a round's products) against the same sums in 64 bits: up to 64 experts and past them, repeated
-choices, indices outside the experts, k of one round and of uneven ones."""
+choices, indices outside the experts, a grid row per choice in both products, one or none, k of one round and of uneven ones, short (no
+loads ahead) and long in both products and in either."""
 import pytest
 import torch
 
@@ -12,7 +13,7 @@ DEV = "cuda"
 
 @pytest.mark.parametrize("experts", [3, 63, 64, 65])
 @pytest.mark.parametrize("rows,top", [(1, 1), (1, 2), (2, 6), (10, 6), (16, 4)])
-@pytest.mark.parametrize("ff,width,act", [(24, 40, "relu_sq"), (136, 1032, "silu_glu")])
+@pytest.mark.parametrize("ff,width,act", [(24, 40, "relu_sq"), (136, 1032, "silu_glu"), (1048, 1032, "relu_sq"), (1048, 40, "silu_glu")])
 def test_choices(experts, rows, top, ff, width, act):
     g = torch.Generator(device=DEV).manual_seed(experts * rows + top)
     rnd = lambda *s, scale=1.0: (torch.randn(*s, generator=g, device=DEV) * scale).bfloat16()   # noqa: E731
