@@ -6,7 +6,8 @@
 // most of the chip idle and a workgroup's four waves share K instead of owning rows each.
 // Bound by memory, the results of the first and the rows of the second product (4 bytes of rank 512 a row and head): 4096 rows of 16
 // heads, 128 -> 512 with the rotation in 44 us (4.0 TB/s; the library's fp32 product and the rotation's launch 104, the same stores
-// in 64-byte pieces 48), 512 -> 128 with gate and rows in 34 us (4.4 TB/s; the library's, the gate's and the rows' launch 105).
+// in 64-byte pieces 48), 512 -> 128 with gate and rows in 34 us (4.4 TB/s; the library's, the gate's and the rows' launch 105), on their own
+// buffers again and again; in a model's pass, from and to memory that others have used since, 67 and 45.
 // Error against 64 bits 6.0e-8 and 2.4e-7 (library 7.3e-8 and 4.1e-7), SPLIT 4.8e-8 and 8.4e-8 (head_product.hip 4.9e-8, 9.7e-8).
 #include "mx_common.h"
 

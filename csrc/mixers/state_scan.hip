@@ -11,12 +11,12 @@
 // state_scan: waves 4 .. 7 hold the state, 32 rows each, and make the next chunk's of it; waves 0 .. 3 the outputs of 16 rows each,
 // from the state's parts that the others left in LDS; waves 8 .. 11 bring rows, and scale and split v.  A barrier a chunk: while one's
 // outputs are formed, the state of the next is, and the chunks after that are on their way.  Bound by the state's chain and the
-// issue of all of them: 1.0 us a chunk; 14 + 37 us for those 2048 rows.  (All of it in one launch, weights and sums of decays by other
-// waves of the same workgroup, which every 16 columns repeat: 87 us; by the output waves: 86 to 97.)
+// issue of all of them: 1.4 us a chunk; those 2048 rows take 59 us back to back, 15 + 50 in a model's pass.  (All of it in one launch,
+// weights and sums of decays by other waves of the same workgroup, which every 16 columns repeat: 87 us; by the output waves: 86 to 97.)
 //
 // A value of v that is not finite reaches its own row and later ones only: a weight of 0 would take it to the rows before it in its block of
 // 16, so blocks with such a value (`loose`) have them apart from the products (2048 rows 58.8 us so and 59.3
-// without, 777 30.9 and 30.1).
+// without, 777 30.9 and 30.1, 2000 of 8 heads, a chain that leaves most of the chip idle, 49.0 and 47.0).
 //
 // Operand layouts (v_mfma_f32_16x16x32_bf16): lane (hi, lo) = (lane / 16, lane % 16) holds row or column lo, inner entries 8 hi ..
 // 8 hi + 7; accumulators hold row 4 hi + r, column lo.  Sums over rows j take j in the order in which accumulators lie, entry i < 4
@@ -431,8 +431,8 @@ extern "C" int mx_state_scan_floats() { return kSsFloats; }
 // Whether these rows are the kernels': bf16, 128 entries of the state a column, whole 16-byte pieces, and workgroups enough or
 // chunks few enough that the chain of chunks is not what a segment waits for.  us, beside the chunk-parallel form: 16 workgroups (4
 // heads of 128 x 64), 500 / 1000 / 2000 / 4000 rows 21 31 47 94 (32 35 38 53); 32 (4 of 128 x 128), 2000 49 (46); 64 (8 of 128 x
-// 128), 2000 and 4000 49 96 (60 104); 256 (32 of 128 x 128), 64 / 200 / 777 / 2048 / 4096 12 16 32 67 117 (34 40 82 149 251), five of
-// 400 76 (158), 64 of 100 395 (704).
+// 128), 2000 and 4000 49 96 (60 104); 256 (32 of 128 x 128), 64 / 200 / 777 / 2048 / 4096 12 17 32 59 106 (34 40 82 149 251), five of
+// 400 73 (158), 64 of 100 390 (704).
 extern "C" int mx_state_scan_takes(const void* y, const void* xbc, int bf16, long stride, int heads, int groups, int n, int dv,
                                    int max_rows) {
   return bf16 && n == kSsKeys && dv >= 1 && dv % kSsCols == 0 && stride % 8 == 0 && ((uintptr_t)xbc) % 16 == 0 &&
