@@ -1,4 +1,4 @@
-// K4: fused rotary embedding + paged KV-cache write (SURVEY.md §2.4 K4).
+// K4: fused rotary embedding + paged KV-cache write.
 //
 // Input is the fused QKV GEMM output [T, (nq + 2 nkv) * D].  One workgroup per
 // token rotates its q and k heads; each lane handles 8 rotary pairs (element i and i + D/2, the Llama
