@@ -230,6 +230,12 @@ int mx_state_step(int kind, float* o, const void* x, int bf16, long x_stride, co
                   long b_stride, const float* a_log, const float* dt_bias, const float* skip, float inv_tau, float* state,
                   const int* start, const int* pos0, const int* slot, int num_segs, int heads, int kv_heads, int dk, int dv,
                   int num_slots, hipStream_t s);
+int mx_row_step_fits(int kind, int taps, int dk, int dv);
+int mx_row_step(int kind, void* out, int bf16, const void* x, long x_stride, const void* a, long a_stride, const void* b,
+                long b_stride, const void* gate, long gate_stride, const float* conv_w, int taps, float* hist,
+                const float* a_log, const float* dt_bias, float inv_tau, const float* norm, float eps, int silu, float* state,
+                const int* start, const int* pos0, const int* slot, int num_segs, int heads, int dk, int dv, int num_slots,
+                hipStream_t s);
 int mx_latent_decode_fits(int rank, int dr, int cache_bf16);
 int mx_latent_prefill_fits(int rank, int dr, int block_size);
 int mx_latent_prefill(float* out, const float* qa, const float* qr, const void* cache, const int* start, const int* pos0,
@@ -735,6 +741,43 @@ void gated_linear_attention(Tensor o, Tensor qkv, Tensor a, Tensor a_bias, doubl
                                ws.g.data_ptr<float>(), start.data_ptr<int>(), pos0.data_ptr<int>(),
                                slot.data_ptr<int>(), t, (int)num_segs, (int)max_rows, (int)heads, (int)dk, (int)dv,
                                (int)state.size(0), (int)chunk_from, stream()), "linear attention chunks");
+}
+
+// one row per sequence of a recurrent mixer, convolution (none for kind 2), state, head norm and gate (row_step.hip)
+void row_step(int64_t kind, Tensor out, Tensor x, Tensor a, OptT b, Tensor gate, OptT conv_w, OptT hist, OptT a_log, Tensor dt_bias,
+              double tau, Tensor norm, double eps, bool silu, Tensor state, Tensor start, Tensor pos0, Tensor slot,
+              int64_t num_segs, int64_t heads, int64_t dk, int64_t dv) {
+  check_rows(x, "x");
+  check_rows(a, "a");
+  check_rows(gate, "gate");
+  for (const Tensor* t : {&dt_bias, &norm, &state}) check_f32(*t, "row_step");
+  const int64_t t = x.size(0), c = heads * (2 * dk + dv);
+  const bool linear = kind == 2;
+  const int64_t taps = conv_w ? conv_w->size(1) : 0;
+  TORCH_CHECK(kind >= 0 && kind <= 2 && heads >= 1 && mx_row_step_fits((int)kind, (int)taps, (int)dk, (int)dv) && tau > 0, "row_step sizes");
+  TORCH_CHECK((linear ? x.size(1) >= c : x.size(1) == c) && a.size(0) == t && a.size(1) == (kind == 1 ? heads : heads * dk) &&
+              gate.size(0) == t && gate.size(1) == heads * dv && dt_bias.numel() == a.size(1) && norm.numel() == dv &&
+              a.scalar_type() == x.scalar_type() && gate.scalar_type() == x.scalar_type(), "row_step shapes");
+  TORCH_CHECK(out.is_cuda() && out.is_contiguous() && out.scalar_type() == x.scalar_type() && out.dim() == 2 && out.size(0) == t &&
+              out.size(1) == heads * dv, "out");
+  TORCH_CHECK(state.dim() == 4 && state.size(1) == heads && state.size(2) == dk && state.size(3) == dv, "state");
+  if (linear) {
+    TORCH_CHECK(!b && !conv_w && !hist && !a_log, "row_step: linear attention has no convolution, beta or rate");
+  } else {
+    TORCH_CHECK(b && conv_w && hist && a_log, "row_step: convolution, beta and rate");
+    check_rows(*b, "b");
+    for (const OptT* o : {&conv_w, &hist, &a_log}) check_f32(**o, "row_step");
+    TORCH_CHECK(b->size(0) == t && b->size(1) == heads && b->scalar_type() == x.scalar_type() && a_log->numel() == heads &&
+                conv_w->dim() == 2 && conv_w->size(0) == c && hist->dim() == 3 && hist->size(0) == state.size(0) &&
+                hist->size(1) == taps - 1 && hist->size(2) == c, "row_step shapes");
+  }
+  check_segs(start, pos0, slot, num_segs);
+  const auto opt = [](const OptT& o) { return o ? o->data_ptr<float>() : nullptr; };
+  chk(mx_row_step((int)kind, out.data_ptr(), bf(out), x.data_ptr(), x.stride(0), a.data_ptr(), a.stride(0),
+                  b ? b->data_ptr() : nullptr, b ? b->stride(0) : 0, gate.data_ptr(), gate.stride(0), opt(conv_w), (int)taps,
+                  opt(hist), opt(a_log), dt_bias.data_ptr<float>(), 1.0f / (float)tau, norm.data_ptr<float>(), (float)eps,
+                  silu ? 1 : 0, state.data_ptr<float>(), start.data_ptr<int>(), pos0.data_ptr<int>(), slot.data_ptr<int>(),
+                  (int)num_segs, (int)heads, (int)dk, (int)dv, (int)state.size(0), stream()), "row_step");
 }
 
 void pair_embed_add(Tensor x, Tensor ids, Tensor table, int64_t mul_prev, int64_t mul_cur, int64_t buckets,
@@ -1824,6 +1867,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("short_conv_silu", &short_conv_silu);
   m.def("gated_delta_rule", &gated_delta_rule);
   m.def("conv_delta_prep", &conv_delta_prep);
+  m.def("row_step", &row_step);
+  m.def("row_step_fits", [](int64_t kind, int64_t taps, int64_t dk, int64_t dv) {
+    return mx_row_step_fits((int)kind, (int)taps, (int)dk, (int)dv) != 0;
+  });
   m.def("head_delta_rule", &head_delta_rule);
   m.def("retention", &retention);
   m.def("scaled_pair_rows", &scaled_pair_rows);

@@ -191,6 +191,10 @@ class ChannelDelta:
             qkv, lo = M.linear(h, self.win[:c]), M.linear(h, self.win[c:])
         a, gp = M.linear_pair(lo[:, :self.ra], self.wa2, lo[:, self.ra:self.ra + self.rg], self.wg2)
         b = lo[:, self.ra + self.rg:self.ra + self.rg + self.heads]
+        y = M.row_step(M.ROW_CHANNEL, qkv, a, b, gp, self.conv_w, s_conv, self.a_log, self.dt_bias, 1.0, self.norm, self.eps,
+                       False, s_rec, ctx.seg, self.heads, self.kvh, self.dk, self.dv)
+        if y is not None:
+            return M.linear(y, self.wo)
         qkv = M.short_conv_silu(qkv, self.conv_w, s_conv, ctx.seg)
         o = M.gated_delta_rule(qkv, a, b, self.a_log, self.dt_bias, s_rec, ctx.seg, self.heads,
                                self.kvh, self.dk, self.dv)
@@ -237,11 +241,14 @@ class HeadDelta:
         s_rec, s_conv = state
         p = M.linear(h, self.win)
         c, ng, nh = self.channels, self.heads * self.dv, self.heads
-        q, k, v, lg, beta = M.conv_delta_prep(p[:, :c], p[:, c + ng:c + ng + nh], p[:, c + ng + nh:c + ng + 2 * nh],
-                                              self.conv_w, s_conv, self.a_log, self.dt_bias, ctx.seg, nh, self.kvh,
-                                              self.dk, self.dv)
-        o = M.head_delta_rule(q, k, v, lg, beta, s_rec, ctx.seg)
-        y = M.head_rms_gate(o, self.norm, p[:, c:c + ng], self.eps, nh, self.dv, self.dtype, silu=True)
+        qkv, gp, a, b = p[:, :c], p[:, c:c + ng], p[:, c + ng:c + ng + nh], p[:, c + ng + nh:c + ng + 2 * nh]
+        y = M.row_step(M.ROW_HEAD, qkv, a, b, gp, self.conv_w, s_conv, self.a_log, self.dt_bias, 1.0, self.norm, self.eps, True,
+                       s_rec, ctx.seg, nh, self.kvh, self.dk, self.dv)
+        if y is None:
+            q, k, v, lg, beta = M.conv_delta_prep(qkv, a, b, self.conv_w, s_conv, self.a_log, self.dt_bias, ctx.seg, nh,
+                                                  self.kvh, self.dk, self.dv)
+            o = M.head_delta_rule(q, k, v, lg, beta, s_rec, ctx.seg)
+            y = M.head_rms_gate(o, self.norm, gp, self.eps, nh, self.dv, self.dtype, silu=True)
         return M.linear(y, self.wo)
 
 
@@ -585,9 +592,12 @@ class GatedLinearAttention:
     def __call__(self, h, ctx: StepContext, state) -> torch.Tensor:
         p = M.linear(h, self.win)
         a = M.linear(p[:, self.nqkv + self.ng:], self.wa2)
-        o = M.gated_linear_attention(p, a, self.a_bias, self.tau, state, ctx.seg, self.heads, self.dk, self.dv)
-        y = M.head_rms_gate(o, self.norm, p[:, self.nqkv:self.nqkv + self.ng], self.eps, self.heads, self.dv,
-                            self.dtype, silu=True)
+        gp = p[:, self.nqkv:self.nqkv + self.ng]
+        y = M.row_step(M.ROW_LINEAR, p, a, None, gp, None, None, None, self.a_bias, self.tau, self.norm, self.eps, True, state,
+                       ctx.seg, self.heads, self.heads, self.dk, self.dv)
+        if y is None:
+            o = M.gated_linear_attention(p, a, self.a_bias, self.tau, state, ctx.seg, self.heads, self.dk, self.dv)
+            y = M.head_rms_gate(o, self.norm, gp, self.eps, self.heads, self.dv, self.dtype, silu=True)
         return M.linear(y, self.wo)
 
 

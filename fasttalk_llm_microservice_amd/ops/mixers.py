@@ -673,6 +673,26 @@ def gated_linear_attention(qkv, a, a_bias, tau: float, state, seg: Segments, hea
     return ref.gated_linear_attention(qkv, a, a_bias, tau, state, seg, heads, dk, dv)
 
 
+ROW_CHANNEL, ROW_HEAD, ROW_LINEAR = 0, 1, 2
+
+
+def row_step(kind: int, x, a, b, gate, conv_w, conv_state, a_log, dt_bias, tau: float, norm, eps: float, silu: bool, state,
+             seg: Segments, heads: int, kv_heads: int, dk: int, dv: int) -> Optional[torch.Tensor]:
+    """One row per sequence (a decode step) of a recurrent mixer, from its projection to the rows of its output product, in
+    one launch: :func:`short_conv_silu` and :func:`gated_delta_rule` (ROW_CHANNEL), :func:`conv_delta_prep` and
+    :func:`head_delta_rule` (ROW_HEAD) or :func:`gated_linear_attention` (ROW_LINEAR; ``dt_bias`` its a_bias), and
+    :func:`head_rms_gate` in x's dtype.  None where the kernel does not take the step: segments of several rows, heads that
+    share q and k (whose history several workgroups would write), sizes."""
+    if not x.is_cuda or seg.max_rows != 1 or kv_heads != heads or \
+            not native_mixers().row_step_fits(kind, 0 if conv_w is None else conv_w.shape[1], dk, dv) or \
+            state.data_ptr() % 16:
+        return None
+    out = torch.empty(x.shape[0], heads * dv, dtype=x.dtype, device=x.device)
+    native_mixers().row_step(kind, out, x, a, b, gate, conv_w, conv_state, a_log, dt_bias, float(tau), norm, eps, silu, state,
+                             seg.start, seg.pos0, seg.slot, seg.num, heads, dk, dv)
+    return out
+
+
 def head_rms_gate(o, w, gate_pre, eps: float, heads: int, dv: int, out_dtype, silu: bool = False):
     """Per head: o / rms(o) * w * sigmoid(gate_pre) (or * silu(gate_pre)), rounded to
     ``out_dtype``; ``gate_pre`` [T, heads*dv] may be a column range of wider rows."""
