@@ -32,7 +32,7 @@ int mx_latent_q_absorb(float* qa, float* qr, const void* q, int bf16, long strid
 int mx_head_values(void* out, int out_bf16, const float* o, const float* wuv, const void* gate, long gate_stride,
                    int rows, int heads, int K, int N, hipStream_t s);
 int mx_norm_route_fits(int width, int experts);
-int mx_norm_route(int* idx, float* wts, void* h, float* x, const void* y, int y_bf16, long y_stride,
+int mx_norm_route(int* idx, float* wts, void* h, float* x, const void* y, int y_bf16, long y_stride, int parts,
                   int layer, const float* wb, const float* w, const float* b, float eps, const float* router, const float* bias, long rows,
                   int experts, int width, int top, int mode, float scale, int groups, int keep, hipStream_t s);
 int mx_expert_rows_fit(int width);
@@ -222,6 +222,9 @@ int mx_moe_pairs(float* out, void* y, const void* h, int bf16, long h_stride, co
 int mx_moe_topk(int* idx, float* wts, const float* z, const float* corr, long rows, int experts, int top,
                 int groups, int keep, hipStream_t s);
 int mx_few_rows_max();
+int mx_few_rows_parts(int N, int K);
+int mx_few_rows_gemm_parts(float* D, const void* X, long x_stride, int rows, const void* W, const void* bias, int N, int K,
+                           int parts, hipStream_t s);
 int mx_moe_route_fits(const void* h, long h_stride, const void* parts, int experts, int width);
 int mx_moe_route(int* idx, float* wts, const void* h, long h_stride, const void* parts, const float* bias, long rows,
                  int experts, int width, int top, int mode, float scale, int groups, int keep, hipStream_t s);
@@ -1082,6 +1085,20 @@ void check_few(const Tensor& y, const Tensor& x, const Tensor& w) {
               x.size(0) <= mx_few_rows_max(), "few rows: bf16 rows and weights");
 }
 
+// d [rows * parts, n] fp32: the sums of x w^T over parts of k (the first: + bias)
+void few_rows_gemm_parts(Tensor d, Tensor x, Tensor w, OptT bias) {
+  check_rows(x, "x");
+  check_f32(d, "d");
+  const int64_t rows = x.size(0), n = w.size(0);
+  TORCH_CHECK(x.scalar_type() == at::kBFloat16 && w.is_cuda() && w.is_contiguous() && w.scalar_type() == at::kBFloat16 && w.dim() == 2 &&
+              w.size(1) == x.size(1) && rows >= 1 && d.dim() == 2 && d.size(1) == n && d.size(0) >= rows && d.size(0) % rows == 0,
+              "few_rows_gemm_parts shapes");
+  TORCH_CHECK(!bias || (bias->is_cuda() && bias->scalar_type() == at::kBFloat16 && bias->is_contiguous() && bias->numel() == n),
+              "few_rows_gemm_parts bias");
+  chk(mx_few_rows_gemm_parts(d.data_ptr<float>(), x.data_ptr(), x.stride(0), (int)rows, w.data_ptr(), bias ? bias->data_ptr() : nullptr, (int)n, (int)x.size(1),
+                             (int)(d.size(0) / rows), stream()), "few_rows_gemm_parts");
+}
+
 // two products of the same sizes and strides in one launch
 void few_rows_pair(Tensor y, Tensor y2, Tensor x, Tensor x2, Tensor w, Tensor w2) {
   check_few(y, x, w);
@@ -1150,11 +1167,15 @@ struct Experts {
   const float *d, *wts, *shared, *gate;
   int top;
 };
-Experts check_experts(const Tensor& d, const Tensor& wts, const OptT& shared, const OptT& gate, int64_t rows, int64_t width) {
+// (without weights: every one is 1)
+Experts check_experts(const Tensor& d, const OptT& wts, const OptT& shared, const OptT& gate, int64_t rows, int64_t width) {
   check_f32(d, "experts' results");
-  check_f32(wts, "experts' weights");
-  TORCH_CHECK(wts.dim() == 2 && wts.size(0) == rows && wts.size(1) >= 1 && d.dim() == 2 && d.size(0) == rows * wts.size(1) &&
-              d.size(1) == width, "experts' results");
+  TORCH_CHECK(d.dim() == 2 && d.size(1) == width && (rows == 0 || (d.size(0) >= rows && d.size(0) % rows == 0)), "experts' results");
+  const int64_t top = rows == 0 ? 1 : d.size(0) / rows;
+  if (wts) {
+    check_f32(*wts, "experts' weights");
+    TORCH_CHECK(wts->dim() == 2 && wts->size(0) == rows && wts->size(1) == top, "experts' weights");
+  }
   if (shared) {
     check_f32(*shared, "shared expert's rows");
     TORCH_CHECK(shared->numel() == rows * width, "shared expert's rows");
@@ -1163,11 +1184,11 @@ Experts check_experts(const Tensor& d, const Tensor& wts, const OptT& shared, co
     check_f32(*gate, "shared expert's gate");
     TORCH_CHECK(shared && gate->numel() == rows, "shared expert's gate");
   }
-  return {d.data_ptr<float>(), wts.data_ptr<float>(), shared ? shared->data_ptr<float>() : nullptr,
-          gate ? gate->data_ptr<float>() : nullptr, (int)wts.size(1)};
+  return {d.data_ptr<float>(), wts ? wts->data_ptr<float>() : nullptr, shared ? shared->data_ptr<float>() : nullptr,
+          gate ? gate->data_ptr<float>() : nullptr, (int)top};
 }
 
-void add_rms_norm_experts(Tensor x, Tensor d, Tensor wts, OptT shared, OptT gate, OptT wb, OptT add_vec, OptT next_w, OptT out,
+void add_rms_norm_experts(Tensor x, Tensor d, OptT wts, OptT shared, OptT gate, OptT wb, OptT add_vec, OptT next_w, OptT out,
                           OptT cast, double eps) {
   check_f32(x, "residual");
   TORCH_CHECK(x.dim() == 2 && mx_expert_rows_fit((int)x.size(1)), "residual");
@@ -1187,7 +1208,7 @@ void add_rms_norm_experts(Tensor x, Tensor d, Tensor wts, OptT shared, OptT gate
       "add_rms_norm_experts");
 }
 
-void layer_norm_experts(Tensor x, Tensor d, Tensor wts, OptT shared, OptT gate, Tensor w, Tensor b, Tensor cast, OptT next_w,
+void layer_norm_experts(Tensor x, Tensor d, OptT wts, OptT shared, OptT gate, Tensor w, Tensor b, Tensor cast, OptT next_w,
                         OptT next_b, double eps) {
   check_f32(x, "residual");
   TORCH_CHECK(x.dim() == 2 && mx_expert_rows_fit((int)x.size(1)), "residual");
@@ -1201,7 +1222,7 @@ void layer_norm_experts(Tensor x, Tensor d, Tensor wts, OptT shared, OptT gate, 
 }
 
 // decode rows: every segment has one row at most
-void add_norm_shift_experts(Tensor x, Tensor d, Tensor wts, OptT shared, OptT gate, Tensor wb, Tensor w, Tensor shift, Tensor out,
+void add_norm_shift_experts(Tensor x, Tensor d, OptT wts, OptT shared, OptT gate, Tensor wb, Tensor w, Tensor shift, Tensor out,
                             Tensor state, Tensor start, Tensor pos0, Tensor slot, int64_t num_segs, double eps) {
   check_f32(x, "residual");
   check_f32(state, "shift state");
@@ -1219,7 +1240,8 @@ void add_norm_shift_experts(Tensor x, Tensor d, Tensor wts, OptT shared, OptT ga
 
 bool norm_route_fits(int64_t width, int64_t experts) { return mx_norm_route_fits((int)width, (int)experts); }
 
-// layer: h = x += layer_norm(y) * w + b; else x += rms_norm(y) * wb (or y), h = rms_norm(x) * w.  bf16 rows; see mx_norm_route
+// layer: h = x += layer_norm(y) * w + b; else x += rms_norm(y) * wb (or y), h = rms_norm(x) * w.  bf16 rows; see mx_norm_route.
+// y [rows, width], or [rows * 2 or 4, width] fp32: parts of the rows
 void norm_route(Tensor idx, Tensor wts, Tensor h, Tensor x, Tensor y, bool layer, OptT wb, Tensor w, OptT b, double eps,
                 Tensor router, OptT bias, int64_t top, int64_t mode, double scale, int64_t groups, int64_t keep) {
   check_f32(x, "residual");
@@ -1229,15 +1251,16 @@ void norm_route(Tensor idx, Tensor wts, Tensor h, Tensor x, Tensor y, bool layer
   check_f32(wts, "wts");
   TORCH_CHECK(x.dim() == 2 && router.dim() == 2 && router.size(1) == x.size(1), "norm_route: router");
   const int64_t rows = x.size(0), width = x.size(1), experts = router.size(0);
-  TORCH_CHECK(norm_route_fits(width, experts) && y.sizes() == x.sizes() &&
-              h.is_cuda() && h.scalar_type() == at::kBFloat16 && h.is_contiguous() && h.sizes() == x.sizes(), "norm_route: rows");
+  const int64_t parts = rows == 0 ? 1 : y.size(0) / rows;
+  TORCH_CHECK(norm_route_fits(width, experts) && y.size(0) == rows * parts && y.size(1) == width &&
+              (parts == 1 || ((parts == 2 || parts == 4) && !bf(y) && y.is_contiguous())) && h.is_cuda() && h.scalar_type() == at::kBFloat16 && h.is_contiguous() && h.sizes() == x.sizes(), "norm_route: rows");
   TORCH_CHECK(idx.numel() == rows * top && wts.numel() == rows * top && layer == (bool)b && !(layer && wb), "norm_route shapes");
   if (bias) {
     check_f32(*bias, "router bias");
     TORCH_CHECK(bias->numel() == experts, "router bias");
   }
   chk(mx_norm_route(idx.data_ptr<int>(), wts.data_ptr<float>(), h.data_ptr(), x.data_ptr<float>(), y.data_ptr(), bf(y),
-                    y.stride(0), layer, row_weight(wb, width), row_weight(w, width), row_weight(b, width), (float)eps,
+                    y.stride(0), (int)parts, layer, row_weight(wb, width), row_weight(w, width), row_weight(b, width), (float)eps,
                     router.data_ptr<float>(), bias ? bias->data_ptr<float>() : nullptr, rows, (int)experts, (int)width,
                     (int)top, (int)mode, (float)scale, (int)groups, (int)keep, stream()), "norm_route");
 }
@@ -1888,6 +1911,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("moe_pairs", &moe_pairs);
   m.def("few_rows_gemm", &few_rows_gemm);
   m.def("few_rows_pair", &few_rows_pair);
+  m.def("few_rows_gemm_parts", &few_rows_gemm_parts);
+  m.def("few_rows_parts", [](int64_t n, int64_t k) { return (int64_t)mx_few_rows_parts((int)n, (int)k); });
   m.def("few_rows_side_gate", &few_rows_side_gate);
   m.def("expert_rows_fit", [](int64_t width) { return (bool)mx_expert_rows_fit((int)width); });
   m.def("add_rms_norm_experts", &add_rms_norm_experts);

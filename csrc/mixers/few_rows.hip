@@ -1,6 +1,7 @@
 // Products with few rows (decode steps) on the matrix units, weights read in place:
 //   few_rows_gemm   Y[r, n] = sum_k X[r, k] W[n, k] (+ bias[n]), bf16 or fp32 out; or, gated,
 //                   Y[r, c] = act(X W_gate^T, X W_up^T), W = [gate | up]; or relu(X W^T)^2
+//   few_rows_parts  the same product with k cut into parts, a workgroup each: fp32 sums of the parts, which the step behind adds
 //   experts_first   the chosen experts' first matrices (and the shared expert's) with the
 //                   activation, one read of an expert's matrix for all rows that chose it
 //   experts_down    their second matrices, one fp32 row per (row, chosen expert)
@@ -115,6 +116,81 @@ few_rows_gemm_kernel(TO* __restrict__ Y, long y_stride, const bf16_t* __restrict
     }
     fr_store4(Y + r * y_stride, c, N, vec != 0, v);
   }
+}
+
+// ---------------------------------------------------------------------------------
+// D[r, p, n] = the sum over part p of k (the first: + bias[n]), blockIdx.y: products of few columns, whose tiles are half the chip's CUs and each a chain
+// along k.  What reads Y there is a norm, which adds the parts as it reads them (rows.hip: ExpertRows; moe_route.hip).
+// Bound by the read of W, and by the latency of the first loads.  N = 2048, weights from HBM, us at 1 / 16 / 32 / 64 rows, a
+// workgroup a tile beside it:
+//   K = 2048, two parts, 8 waves       4.4 4.4 5.2 6.3    (5.2 5.8 6.9 8.6)
+//   K = 4096, four parts               5.4 6.0 7.2 9.1    (7.3 8.4 10.5 14.0)
+//   K = 8192, four parts               8.4 9.4 11.4 15.2  (11.4 13.5 17.6 24.5)
+//   K = 14336, four parts              12.2 15.4 18.4 25.1 (18.1 23.3 31.2 43.3)
+// ---------------------------------------------------------------------------------
+template <int NB, int WV, int U>
+__global__ void __launch_bounds__(64 * WV)
+few_rows_parts_kernel(float* __restrict__ D, const bf16_t* __restrict__ X, long x_stride, int rows, const bf16_t* __restrict__ W,
+                      const bf16_t* __restrict__ bias, int N, int K, int part) {
+  extern __shared__ float4 red[];                // X stages, then partial sums
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n0 = blockIdx.x * 16, k0 = blockIdx.y * part;
+  const bf16_t* wp[1] = {W + (long)min(n0 + (lane & 15), N - 1) * K + k0};
+  fr_f32x4 acc[1][NB];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) acc[0][b] = fr_f32x4{0.f, 0.f, 0.f, 0.f};
+  few_rows_core<1, NB, WV, U>(acc, wp, [&](int r) { return X + r * x_stride + k0; }, rows, min(part, K - k0),
+                              reinterpret_cast<char*>(red) + wave * kFrStage<NB, U>, wave, lane);
+  __syncthreads();
+  few_rows_park<1, NB, WV>(red, acc, wave, lane);
+  __syncthreads();
+  for (int e = tid; e < NB * 64; e += 64 * WV) {
+    const int el = e & 63, b = e >> 6, r = 16 * b + (el & 15), c = n0 + 4 * (el >> 4);
+    if (r >= rows || c >= N) continue;
+    float v[4];
+    few_rows_sum<1, NB, WV>(red, 0, b, el, v);
+    if (bias != nullptr && blockIdx.y == 0) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] += ft::bf16_to_f32(bias[c + i]);      // (N: whole fours)
+    }
+    fr_store4(D + ((long)r * gridDim.y + blockIdx.y) * N, c, N, true, v);
+  }
+}
+
+template <int NB, int WV, int U>
+int few_rows_parts_launch(float* D, const void* X, long x_stride, int rows, const void* W, const void* bias, int N, int K, int parts, hipStream_t s) {
+  constexpr int kRed = WV * NB * 1024, kX = WV * kFrStage<NB, U>, lds = kRed > kX ? kRed : kX;
+  static_assert(lds <= 160 * 1024, "");
+  auto kernel = few_rows_parts_kernel<NB, WV, U>;
+  if constexpr (lds > 64 * 1024) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (e != hipSuccess) return (int)e;
+  }
+  const int part = ((K + 63) / 64 + parts - 1) / parts * 64;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)((N + 15) / 16), (unsigned)parts), dim3(64 * WV), lds, s, D, (const bf16_t*)X, x_stride,
+                     rows, (const bf16_t*)W, (const bf16_t*)bias, N, K, part);
+  return (int)hipGetLastError();
+}
+
+// Parts of k (1: few_rows_gemm is as fast): until there are two to three workgroups a CU.  From a grid of N = 1280 to 6144, K = 1024 to
+// 14336 and 1 to 64 rows, us of one / two / four / eight parts at 16 rows: N = 1280, K = 8192 13.3 - 8.5 7.2; 2048, 1024 3.7
+// 3.3; 3072, 1024 4.2 4.3; 3072, 4096 9.0 8.4 7.5; 4096, 2048 6.7 6.3 6.2; 4096, 8192 15.6 15.6 16.3.  Every part is a row more
+// for the step behind to read, so where a few per cent are all there is to gain (4096 columns on) k stays whole.
+int few_rows_parts(int N, int K) {
+  if (N > 3584 || K < 1024 || (N > 2048 && K < 2048)) return 1;
+  return K >= 4096 || N > 2048 ? 4 : 2;
+}
+
+// Waves and steps in flight: where the columns fill the chip four waves with one step are the best at all rows; below, shares of k of
+// 512 or less are one round of loads for eight waves, and with more rows X's way through LDS counts (four waves).
+template <int NB>
+int few_rows_parts_pick(float* D, const void* X, long x_stride, int rows, const void* W, const void* bias, int N, int K, int parts, hipStream_t s) {
+#define FR_PARTS(WV, U) few_rows_parts_launch<NB, WV, U>(D, X, x_stride, rows, W, bias, N, K, parts, s)
+  if (N > 2048) return FR_PARTS(4, 1);
+  if (parts <= 2) return K < 2048 || NB == 4 ? FR_PARTS(8, 1) : FR_PARTS(8, 2);
+  return NB == 1 ? FR_PARTS(8, 1) : FR_PARTS(4, 2);
+#undef FR_PARTS
 }
 
 // ---------------------------------------------------------------------------------
@@ -408,6 +484,20 @@ extern "C" int mx_few_rows_gemm(void* Y, int y_f32, long y_stride, const void* X
   if (glu) return FR_GO(true, bf16_t);
   return y_f32 ? FR_GO(false, float) : FR_GO(false, bf16_t);
 #undef FR_GO
+}
+
+extern "C" int mx_few_rows_parts(int N, int K) { return few_rows_parts(N, K); }
+
+// D [rows][parts][N]: parts as mx_few_rows_parts says, or fewer than K has steps of 64
+extern "C" int mx_few_rows_gemm_parts(float* D, const void* X, long x_stride, int rows, const void* W, const void* bias,
+                                      int N, int K, int parts, hipStream_t s) {
+  if (rows <= 0 || N <= 0) return 0;
+  if (rows > kFewRows || K < 8 || K % 8 || x_stride % 8 || N % 4 || parts < 1 || parts > 65535) return -1;
+  if (((((K + 63) / 64) + parts - 1) / parts) * 64L * (parts - 1) >= K) return -1;       // (a part without any k)
+  if (((uintptr_t)X | (uintptr_t)W | (uintptr_t)D) % 16) return -2;
+  if (rows <= 16) return few_rows_parts_pick<1>(D, X, x_stride, rows, W, bias, N, K, parts, s);
+  if (rows <= 32) return few_rows_parts_pick<2>(D, X, x_stride, rows, W, bias, N, K, parts, s);
+  return few_rows_parts_pick<4>(D, X, x_stride, rows, W, bias, N, K, parts, s);
 }
 
 // bf16 products with a rider: Y = X W^T and Y2 = X2 W2^T, of the same sizes and strides

@@ -258,7 +258,7 @@ struct RouteRows {
   bf16_t* h;                                 // read (NORM 0), else written, dense
   long h_stride;
   float* x;
-  const void* y;                             // TY
+  const void* y;                             // TY; PARTS of them a row: dense, and their sum is the row
   long y_stride;
   const float *wb, *w, *b;
   const float *router, *bias;
@@ -270,7 +270,7 @@ struct RouteRows {
 // those of the router for sixteen rows a workgroup where that serves (widths of whole 2048)
 static bool route_in_turn(long rows, int width) { return rows <= 64 || width % 2048 != 0; }
 
-template <int NORM, int C, typename TY>
+template <int NORM, int C, typename TY, int PARTS = 1>
 __global__ void __launch_bounds__(64 * kRouteWaves)
 route_rows_kernel(RouteRows R) {
   constexpr int NT = 64 * kRouteWaves;
@@ -282,7 +282,7 @@ route_rows_kernel(RouteRows R) {
   using Raw = typename std::conditional<sizeof(TY) == 2, uint2, float4>::type;
   // (loads come back in the order they were asked for: the row's before the router's)
   float v[C][4], t[C][4], w[C][4], u[C][4];
-  Raw yr[C];
+  Raw yr[C][PARTS];
   uint2 hr[C];
   const float* wb = NORM == 2 ? R.w : R.wb;
 #pragma unroll
@@ -291,7 +291,9 @@ route_rows_kernel(RouteRows R) {
     if constexpr (NORM == 0) {
       hr[c] = *reinterpret_cast<const uint2*>(R.h + row * R.h_stride + i);
     } else {
-      yr[c] = *reinterpret_cast<const Raw*>((const TY*)R.y + row * R.y_stride + i);
+#pragma unroll
+      for (int p = 0; p < PARTS; ++p)
+        yr[c][p] = *reinterpret_cast<const Raw*>((const TY*)R.y + (PARTS > 1 ? (row * PARTS + p) * width : row * R.y_stride) + i);
       load4(R.x + row * width + i, v[c]);
       load4((wb != nullptr ? wb : R.w) + i, w[c]);
       load4((NORM == 2 ? R.b : R.w) + i, u[c]);
@@ -327,10 +329,12 @@ route_rows_kernel(RouteRows R) {
 #pragma unroll
     for (int c = 0; c < C; ++c) {
       if constexpr (sizeof(TY) == 2) {
-        ft::unpack2(yr[c].x, t[c][0], t[c][1]);
-        ft::unpack2(yr[c].y, t[c][2], t[c][3]);
+        ft::unpack2(yr[c][0].x, t[c][0], t[c][1]);
+        ft::unpack2(yr[c][0].y, t[c][2], t[c][3]);
       } else {
-        t[c][0] = yr[c].x, t[c][1] = yr[c].y, t[c][2] = yr[c].z, t[c][3] = yr[c].w;
+        t[c][0] = yr[c][0].x, t[c][1] = yr[c][0].y, t[c][2] = yr[c][0].z, t[c][3] = yr[c][0].w;
+#pragma unroll
+        for (int p = 1; p < PARTS; ++p) t[c][0] += yr[c][p].x, t[c][1] += yr[c][p].y, t[c][2] += yr[c][p].z, t[c][3] += yr[c][p].w;
       }
       if ((c * NT + tid) * 4 >= width)
 #pragma unroll
@@ -520,13 +524,13 @@ static bool route_rows_fit(int width, int experts) {
 extern "C" int mx_norm_route_fits(int width, int experts) { return mx::route_rows_fit(width, experts); }
 
 // The norm step in front of a router and the router, bf16 rows out: layer 0: x += rms_norm(y) * wb (wb null: y), h = rms_norm(x) * w;
-// 1: x += layer_norm(y) * w + b, h = x.  Modes as below.
-extern "C" int mx_norm_route(int* idx, float* wts, void* h, float* x, const void* y, int y_bf16, long y_stride,
+// 1: x += layer_norm(y) * w + b, h = x.  parts 2 or 4: y [rows][parts][width] fp32, rows the sums of their parts.  Modes as below.
+extern "C" int mx_norm_route(int* idx, float* wts, void* h, float* x, const void* y, int y_bf16, long y_stride, int parts,
                              int layer, const float* wb, const float* w, const float* b, float eps, const float* router, const float* bias, long rows,
                              int experts, int width, int top, int mode, float scale, int groups, int keep, hipStream_t s) {
   if (rows <= 0) return 0;
   if (!mx::route_rows_fit(width, experts) || top < 1 || top > experts || mode < 0 || mode > 2 || (mode == 2 && bias == nullptr) ||
-      rows > 0x7fffffffL || y_stride % 4) return -1;
+      rows > 0x7fffffffL || y_stride % 4 || !(parts == 1 || ((parts == 2 || parts == 4) && !y_bf16))) return -1;
   if (groups < 1 || experts % groups || keep < 1 || keep > groups || top > experts / groups * keep) return -1;
   if (((uintptr_t)h | (uintptr_t)x | (uintptr_t)wb | (uintptr_t)w | (uintptr_t)b | (uintptr_t)router) % 16 || ((uintptr_t)y) % (y_bf16 ? 8 : 16))
     return -2;
@@ -535,14 +539,25 @@ extern "C" int mx_norm_route(int* idx, float* wts, void* h, float* x, const void
 #define MX_NR(NORM, C)                                                                                                     \
   MX_DISPATCH_T(y_bf16, hipLaunchKernelGGL((mx::route_rows_kernel<NORM, C, T>), dim3((unsigned)rows), dim3(64 * mx::kRouteWaves), \
                                            width * 4, s, R))
-#define MX_NR_C(NORM)                  \
-  do {                                 \
-    if (width <= 4096) MX_NR(NORM, 1); \
-    else MX_NR(NORM, 2);               \
+#define MX_NR_PARTS(NORM, C, PARTS)                                                                                  \
+  hipLaunchKernelGGL((mx::route_rows_kernel<NORM, C, float, PARTS>), dim3((unsigned)rows), dim3(64 * mx::kRouteWaves), \
+                     width * 4, s, R)
+#define MX_NR_P(NORM, C)                            \
+  do {                                              \
+    if (parts == 4) MX_NR_PARTS(NORM, C, 4);        \
+    else if (parts == 2) MX_NR_PARTS(NORM, C, 2);   \
+    else MX_NR(NORM, C);                            \
+  } while (0)
+#define MX_NR_C(NORM)                    \
+  do {                                   \
+    if (width <= 4096) MX_NR_P(NORM, 1); \
+    else MX_NR_P(NORM, 2);               \
   } while (0)
   if (layer) MX_NR_C(2);
   else MX_NR_C(1);
 #undef MX_NR_C
+#undef MX_NR_P
+#undef MX_NR_PARTS
 #undef MX_NR
   return (int)hipGetLastError();
 }

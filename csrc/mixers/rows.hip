@@ -236,7 +236,8 @@ __device__ __forceinline__ void store_row(T* p, const float (&v)[C][4], int widt
 
 // What a norm kernel adds to the residual: a row of a tensor, or of the experts' results not yet summed
 // (few_rows.hip: experts_down), sum_k w[row, k] d[row, k] + shared[row] * (sigmoid(gate[row]) or 1), which saves
-// a launch and its rows' way through memory (4.6 us a layer of a decode step).
+// a launch and its rows' way through memory (4.6 us a layer of a decode step); or, without weights, of a product's parts
+// (few_rows.hip: few_rows_parts).
 template <typename T>
 struct RowsOf {
   const T* p;
@@ -248,12 +249,12 @@ struct RowsOf {
   }
 };
 struct ExpertRows {
-  const float *d, *wts, *shared, *gate;       // [rows * top, width], [rows, top], [rows, width] or null, [rows] or null
+  const float *d, *wts, *shared, *gate;       // [rows * top, width], [rows, top] or null, [rows, width] or null, [rows] or null
   int top;
   __device__ __forceinline__ bool any() const { return true; }
   template <int NT, int C>
   __device__ __forceinline__ void load(float (&v)[C][4], long row, int width, int) const {      // (width: whole fours)
-    const float* w = wts + row * top;
+    const float* w = wts != nullptr ? wts + row * top : nullptr;
     const float g = shared != nullptr && gate != nullptr ? sigmoidf_(gate[row]) : 1.f;
 #pragma unroll
     for (int c = 0; c < C; ++c) {
@@ -265,7 +266,7 @@ struct ExpertRows {
         v[c][0] += f * u.x, v[c][1] += f * u.y, v[c][2] += f * u.z, v[c][3] += f * u.w;
       };
 #pragma unroll 4
-      for (int k = 0; k < top; ++k) add(d + (row * top + k) * width, w[k]);
+      for (int k = 0; k < top; ++k) add(d + (row * top + k) * width, w != nullptr ? w[k] : 1.f);
       if (shared != nullptr) add(shared + row * width, g);
     }
   }

@@ -32,13 +32,15 @@ Get = Callable[[str], torch.Tensor]
 
 class StepContext:
     """What a sublayer needs to know about the step: rows' token ids, positions and
-    cache slots, and the row segments (one per scheduled sequence)."""
+    cache slots, and the row segments (one per scheduled sequence).  ``parts``: a sublayer's rows may
+    come as :class:`..ops.mixers.ExpertParts`, since a norm step reads them."""
 
-    def __init__(self, ids, positions, slot_mapping, seg: M.Segments):
+    def __init__(self, ids, positions, slot_mapping, seg: M.Segments, parts: bool = False):
         self.ids = ids
         self.positions = positions
         self.slot_mapping = slot_mapping
         self.seg = seg
+        self.parts = parts
 
 
 def _state_slots(shapes, num_slots: int, device):
@@ -143,7 +145,8 @@ class LatentAttention:
                                         self.PRODUCT_ROWS, self.dtype, self.sink)
         else:
             ol = M.latent_attention(qa, qr, cache, seg, self.scale, self.rank, sink=self.sink)
-        return M.linear(M.head_values(ol, self.wuvT, qd[:, self.n_down:] if self.gated else None, self.dtype, self.wuvT_tiles), self.wo)
+        y = M.head_values(ol, self.wuvT, qd[:, self.n_down:] if self.gated else None, self.dtype, self.wuvT_tiles)
+        return M.linear_out(y, self.wo, ctx.parts)
 
 
 class ChannelDelta:
@@ -194,12 +197,12 @@ class ChannelDelta:
         y = M.row_step(M.ROW_CHANNEL, qkv, a, b, gp, self.conv_w, s_conv, self.a_log, self.dt_bias, 1.0, self.norm, self.eps,
                        False, s_rec, ctx.seg, self.heads, self.kvh, self.dk, self.dv)
         if y is not None:
-            return M.linear(y, self.wo)
+            return M.linear_out(y, self.wo, ctx.parts)
         qkv = M.short_conv_silu(qkv, self.conv_w, s_conv, ctx.seg)
         o = M.gated_delta_rule(qkv, a, b, self.a_log, self.dt_bias, s_rec, ctx.seg, self.heads,
                                self.kvh, self.dk, self.dv)
         y = M.head_rms_gate(o, self.norm, gp, self.eps, self.heads, self.dv, self.dtype)
-        return M.linear(y, self.wo)
+        return M.linear_out(y, self.wo, ctx.parts)
 
 
 class HeadDelta:
@@ -249,7 +252,7 @@ class HeadDelta:
                                                   self.kvh, self.dk, self.dv)
             o = M.head_delta_rule(q, k, v, lg, beta, s_rec, ctx.seg)
             y = M.head_rms_gate(o, self.norm, gp, self.eps, nh, self.dv, self.dtype, silu=True)
-        return M.linear(y, self.wo)
+        return M.linear_out(y, self.wo, ctx.parts)
 
 
 class WindowedAttention:
@@ -330,7 +333,7 @@ class SigmoidAttention(WindowedAttention):
         q = M.attn_prep(qkv, self.nq, self.nk, self.q_norm, self.k_norm, self.eps, None, 0, self.spec.dk,
                         ctx.positions, ctx.slot_mapping, cache[0], cache[1])
         o = self.attend(q, ctx, cache, self.dtype)
-        return M.linear(o.view(h.shape[0], -1), self.wo)
+        return M.linear_out(o.view(h.shape[0], -1), self.wo, ctx.parts)
 
 
 class DifferentialAttention(WindowedAttention):
@@ -368,7 +371,7 @@ class DifferentialAttention(WindowedAttention):
         a = self.attend(q, ctx, cache)
         o = M.diff_combine(a, qkvg[:, n:], self.lam, 1.0 - self.diff, self.eps, self.spec.heads,
                            self.spec.dv, self.dtype)
-        return M.linear(o, self.wo)
+        return M.linear_out(o, self.wo, ctx.parts)
 
 
 class ConvSinkAttention(WindowedAttention):
@@ -422,7 +425,7 @@ class ConvSinkAttention(WindowedAttention):
         return self.attend(q, ctx, (kc, vc), dtype).view(qkv.shape[0], -1)
 
     def __call__(self, h, ctx: StepContext, cache) -> torch.Tensor:
-        return M.linear(self.rows(M.linear(h, self.wqkv), ctx, cache, self.dtype), self.wo)
+        return M.linear_out(self.rows(M.linear(h, self.wqkv), ctx, cache, self.dtype), self.wo, ctx.parts)
 
 
 class BiasedWindowAttention(WindowedAttention):
@@ -467,7 +470,7 @@ class BiasedWindowAttention(WindowedAttention):
             q = M.attn_prep(p[:, :self.n_in], self.nq, self.nk, self.q_norm, self.k_norm, self.eps, None, 0,
                             self.spec.dk, ctx.positions, ctx.slot_mapping, cache[0], cache[1])
         o = self.attend(q, ctx, cache)
-        return M.linear(M.sigmoid_gate(o.view(h.shape[0], -1), p[:, self.n_in:], self.dtype), self.wo)
+        return M.linear_out(M.sigmoid_gate(o.view(h.shape[0], -1), p[:, self.n_in:], self.dtype), self.wo, ctx.parts)
 
 
 class RotaryBlockAttention(WindowedAttention):
@@ -493,7 +496,7 @@ class RotaryBlockAttention(WindowedAttention):
         q = M.attn_prep(qkv, self.nq, self.nk, None, None, self.eps, self.table, self.rot_dims, self.spec.dk,
                         ctx.positions, ctx.slot_mapping, cache[0], cache[1])
         o = self.attend(q, ctx, cache, self.dtype)
-        return M.linear(o.view(h.shape[0], -1), self.wo)
+        return M.linear_out(o.view(h.shape[0], -1), self.wo, ctx.parts)
 
 
 class TalkingHeadsAttention:
@@ -556,7 +559,7 @@ class TalkingHeadsAttention:
         else:
             o = torch.empty(h.shape[0], self.nq, dtype=self.dtype, device=h.device)
             M.talk_attention(o, q, gate, kc, vc, seg, self.spec)
-        return M.linear(o, self.wo, self.bo)
+        return M.linear_out(o, self.wo, ctx.parts, self.bo)
 
 
 class GatedLinearAttention:
@@ -598,7 +601,7 @@ class GatedLinearAttention:
         if y is None:
             o = M.gated_linear_attention(p, a, self.a_bias, self.tau, state, ctx.seg, self.heads, self.dk, self.dv)
             y = M.head_rms_gate(o, self.norm, gp, self.eps, self.heads, self.dv, self.dtype, silu=True)
-        return M.linear(y, self.wo)
+        return M.linear_out(y, self.wo, ctx.parts)
 
 
 class Retention:
@@ -641,7 +644,7 @@ class Retention:
         p = M.linear(h, self.win)
         y = M.head_rms_gate(self.rows(p, ctx, state), self.unit, p[:, self.nqkv:], self.eps, self.heads, self.dv,
                             self.dtype, silu=True)
-        return M.linear(y, self.wo)
+        return M.linear_out(y, self.wo, ctx.parts)
 
 
 class SideBySideSum:
@@ -672,7 +675,7 @@ class SideBySideSum:
         a = self.left.rows(p[:, :self.n_left], ctx, cache[0])
         o = r.rows(pr, ctx, cache[1])
         y = M.scaled_pair_rows(a, self.left_scale, o, pr[:, r.nqkv:], self.right_scale, r.eps, r.heads, r.dv, self.dtype)
-        return M.linear(y, self.wo)
+        return M.linear_out(y, self.wo, ctx.parts)
 
 
 class SideBySide:
@@ -695,6 +698,8 @@ class SideBySide:
                 self.right.alloc_cache(num_blocks, block_size, dtype, num_slots, device))
 
     def __call__(self, h, ctx: StepContext, cache) -> torch.Tensor:
+        if ctx.parts:                        # (each output passes a norm of its own here)
+            ctx = StepContext(ctx.ids, ctx.positions, ctx.slot_mapping, ctx.seg)
         a = self.left(h, ctx, cache[0])
         b = self.right(h, ctx, cache[1])
         return M.dual_rms_mean(a, b, self.w_left, self.w_right, self.eps, self.scale)
@@ -743,7 +748,7 @@ class StateSpaceMixer:
         y = M.ssd_scan(xbc, p[:, self.inner + self.channels:], self.a_log, self.dt_bias, self.d_skip, s_rec,
                        ctx.seg, self.heads, self.groups, self.n, self.dv)
         y = M.gate_group_norm(y, z, self.norm, self.eps, self.norm_groups, self.dtype)
-        return M.linear(y, self.wo)
+        return M.linear_out(y, self.wo, ctx.parts)
 
 
 class GatedFF:
@@ -757,7 +762,7 @@ class GatedFF:
         self.act, self.limit = act, float(limit)
 
     def __call__(self, h, ctx=None) -> torch.Tensor:
-        return M.linear(M.linear_act(h, self.wgu, self.act, self.limit), self.down)
+        return M.linear_out(M.linear_act(h, self.wgu, self.act, self.limit), self.down, ctx is not None and ctx.parts)
 
 
 class DenseFF:
@@ -768,7 +773,7 @@ class DenseFF:
         self.down = get("down").to(device, dtype).contiguous()
 
     def __call__(self, h, ctx=None) -> torch.Tensor:
-        return M.linear(M.linear_act(h, self.up, "relu_sq"), self.down)
+        return M.linear_out(M.linear_act(h, self.up, "relu_sq"), self.down, ctx is not None and ctx.parts)
 
 
 def _glu_weights(get: Get, prefix: str, dtype, device, extra: Optional[torch.Tensor] = None):

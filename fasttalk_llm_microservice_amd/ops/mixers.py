@@ -229,6 +229,19 @@ def linear(x, w, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     return torch.nn.functional.linear(x, w, bias) if y is None else y
 
 
+def linear_out(x, w, parts: bool, bias: Optional[torch.Tensor] = None):
+    """:func:`linear`, a sublayer's last product; with ``parts`` its result may be :class:`ExpertParts`, the product with k cut
+    into parts that the norm step behind adds up: few columns leave a product of few rows half the chip, in long chains."""
+    if parts and _few_rows(x, w) and x.shape[1] <= 16384 and native_mixers().expert_rows_fit(w.shape[0]) and \
+            (bias is None or (bias.dtype == x.dtype and bias.is_contiguous())):
+        n = native_mixers().few_rows_parts(*w.shape)
+        if n > 1:
+            d = torch.empty(x.shape[0] * n, w.shape[0], dtype=torch.float32, device=x.device)
+            native_mixers().few_rows_gemm_parts(d, x, w, bias)
+            return ExpertParts(d, None, None, None)
+    return linear(x, w, bias)
+
+
 def linear_pair(x, w, x2, w2):
     """(:func:`linear` of x and w, of x2 and w2); one launch where the kernel of few rows takes both and they are alike in sizes
     and strides."""
@@ -313,9 +326,10 @@ def layer_norm_rows(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor, eps: floa
 class ExpertParts(NamedTuple):
     """The outputs of a mixture of few rows not yet summed: row t is sum_k wts[t, k] * d[t * top + k] + shared[t] (times the
     sigmoid of gate[t], if there is one).  The norm steps take it for their ``y`` and sum it as they read it, which saves a
-    launch between the experts and the norm (4.6 us of a decode step per layer)."""
+    launch between the experts and the norm (4.6 us of a decode step per layer).  Without ``wts`` every one is 1: the parts of
+    a product (:func:`linear_out`)."""
     d: torch.Tensor                   # fp32 [rows * top, width]
-    wts: torch.Tensor                 # fp32 [rows, top]
+    wts: Optional[torch.Tensor]       # fp32 [rows, top]
     shared: Optional[torch.Tensor]    # fp32 [rows, width]
     gate: Optional[torch.Tensor]      # fp32 [rows]
 
@@ -1499,7 +1513,12 @@ def moe_route_by_row(h, router) -> bool:
 
 def norm_route_fits(x, y, wb, w, b, router) -> bool:
     """Whether :func:`norm_route` takes these rows: up to NORM_ROUTE_ROWS bf16 or fp32 sublayer outputs y on a GPU, at most 64
-    experts (a lane each), widths of whole 256 up to 8192 (a row in LDS), all at 16-byte addresses."""
+    experts (a lane each), widths of whole 256 up to 8192 (a row in LDS), all at 16-byte addresses; or a product's two or four parts."""
+    if isinstance(y, ExpertParts):
+        return bool(y.wts is None and y.shared is None and x.shape[0] <= NORM_ROUTE_ROWS and x.is_contiguous()
+                    and y.d.shape[0] in (2 * x.shape[0], 4 * x.shape[0])
+                    and all(t is None or t.data_ptr() % 16 == 0 for t in (x, y.d, wb, w, b, router))
+                    and native_mixers().norm_route_fits(x.shape[1], router.shape[0]))
     return bool(y.is_cuda and y.shape[0] <= NORM_ROUTE_ROWS and x.is_contiguous() and y.dim() == 2 and y.shape == x.shape
                 and y.stride(1) == 1 and y.stride(0) % 4 == 0 and y.data_ptr() % (4 * y.element_size()) == 0
                 and all(t is None or t.data_ptr() % 16 == 0 for t in (x, wb, w, b, router))
@@ -1514,7 +1533,7 @@ def norm_route(x, y, wb, w, b, eps: float, router, bias, top: int, routing: str,
     h = torch.empty(x.shape, dtype=torch.bfloat16, device=x.device)
     idx = torch.empty(x.shape[0], top, dtype=torch.int32, device=x.device)
     wts = torch.empty(x.shape[0], top, dtype=torch.float32, device=x.device)
-    native_mixers().norm_route(idx, wts, h, x, y, b is not None, wb, w, b, eps, router, bias, top, ROUTE_MODES[routing],
+    native_mixers().norm_route(idx, wts, h, x, y.d if isinstance(y, ExpertParts) else y, b is not None, wb, w, b, eps, router, bias, top, ROUTE_MODES[routing],
                                float(scale), groups, keep)
     return h, (idx, wts)
 
