@@ -196,10 +196,12 @@ int few_rows_parts_pick(float* D, const void* X, long x_stride, int rows, const 
 // ---------------------------------------------------------------------------------
 // Experts of few rows.  A workgroup owns one tile of 16 (two) columns of one expert's matrix and
 // serves every row that chose the expert: the matrix is read once however many rows share it.
-// blockIdx.y: expert (expert_in_slot); the last row: the shared expert, which serves all rows.
-// Bound by the stream of the chosen experts' matrices.  32 rows, top 4 of 32 experts of 1536 (relu^2)
-// and a shared one: 44 + 50 us for 214 MB each, 4.9 and 4.3 TB/s, where one read per (row, choice)
-// took 105 + 101 us; 16 rows, top 6 of 32 gated experts of 1024: 54 + 30 us, before 112 + 54.
+// blockIdx.y: the shared expert, which serves all rows and whose down matrix may have the longest rows, where there is one; then
+// the experts (expert_in_slot).
+// Bound by the stream of the chosen experts' matrices.  us of the first and the down matrices (forms: mx_experts_few), alone with
+// weights from HBM, as before / now (one form for all with the shared expert last): 32 rows, top 4 of 32 experts of 1536 (relu^2) and a shared one of 3072,
+// 214 MB each 52 + 51, 41 + 41; 16 rows, top 6 of 32 gated experts of 1024 48 + 26, 47 + 25; 8 rows, top 4 of them and a shared one
+// of 2048 37 + 24, 36 + 20; 3 rows 24 + 17, 24 + 14.
 // ---------------------------------------------------------------------------------
 struct ExpertSet {
   const bf16_t* w;        // [experts][rows_w][K]
@@ -264,10 +266,6 @@ __device__ __forceinline__ int rows_of(const int* __restrict__ idx, int pairs, i
   return count;
 }
 
-// steps of k a round (expert_tile_any)
-template <bool AHEAD>
-constexpr int kExpSteps = AHEAD ? 2 : 1;
-
 // the tile's sums for the listed rows: f(entry row in the list, column, sums, up sums)
 template <int P, bool GLU, int NB, int WV, int U, bool AHEAD, typename F>
 __device__ __forceinline__ void expert_tile(float4* red, const bf16_t* W, int N, int K, int n0, const bf16_t* X,
@@ -300,48 +298,42 @@ __device__ __forceinline__ void expert_tile(float4* red, const bf16_t* W, int N,
   }
 }
 
-// blocks of 16 rows that the listed rows fill, at most MB.  Steps of at most 16 rows name few experts, whose tiles leave a
-// CU one to three workgroups: two steps of k a round, and the next one's loads under it (AHEAD).  us of both products and the shared
-// expert's, one step a round / so: 3 rows, top 4 of 32 gated experts of 1024 44 / 37.5; 4 rows and a shared one of 2048 55 / 45;
-// 8 of 1536 (relu^2) 67 / 64; 16 rows 73 / 74.  With more rows the CU is full and the registers cost more (64 rows, top 6: 85 / 93).
-template <int P, bool GLU, int WV, int MB, bool AHEAD, typename F>
+// blocks of 16 rows that the listed rows fill, at most MB
+template <int P, bool GLU, int WV, int MB, int U, bool AHEAD, typename F>
 __device__ __forceinline__ void expert_tile_any(float4* red, const bf16_t* W, int N, int K, int n0, const bf16_t* X,
                                                 long x_stride, const int* list, int count, int div, int wave, int lane,
                                                 F out) {
-  if (MB == 1) expert_tile<P, GLU, 1, WV, kExpSteps<AHEAD>, AHEAD>(red, W, N, K, n0, X, x_stride, list, count, div, wave, lane, out);
-  else if (count <= 16) expert_tile<P, GLU, 1, WV, 1, false>(red, W, N, K, n0, X, x_stride, list, count, div, wave, lane, out);
-  else if (MB == 2 || count <= 32) expert_tile<P, GLU, 2, WV, 1, false>(red, W, N, K, n0, X, x_stride, list, count, div, wave, lane, out);
-  else expert_tile<P, GLU, MB, WV, 1, false>(red, W, N, K, n0, X, x_stride, list, count, div, wave, lane, out);
+  if (MB == 1 || count <= 16) expert_tile<P, GLU, 1, WV, U, AHEAD>(red, W, N, K, n0, X, x_stride, list, count, div, wave, lane, out);
+  else if (MB == 2 || count <= 32) expert_tile<P, GLU, 2, WV, U, AHEAD>(red, W, N, K, n0, X, x_stride, list, count, div, wave, lane, out);
+  else expert_tile<P, GLU, MB, WV, U, AHEAD>(red, W, N, K, n0, X, x_stride, list, count, div, wave, lane, out);
 }
+
+// float4s of X stages and partial sums of WV waves' NT tiles with MB blocks of rows
+template <int NT, int MB, int WV, int U>
+constexpr int kExpLds = WV * (kFrStage<MB, U> > 1024 * NT * MB ? kFrStage<MB, U> : 1024 * NT * MB) / 16;
 
 // y[pair] = act(first matrices of the pair's expert times its row of h); ys[row] the same of the
 // shared expert; with a shared gate (one more row of its matrix) sg[row] = that row's product, by
 // the workgroup past the shared expert's last tile.
-constexpr int kExpWaves = 4;
-// X stages and partial sums (two tiles) of a tile with MB blocks of rows
-template <int MB, bool AHEAD>
-constexpr int kExpLds = kExpWaves * (kFrStage<MB, kExpSteps<AHEAD>> > 2048 * MB ? kFrStage<MB, kExpSteps<AHEAD>> : 2048 * MB);
-
-template <bool GLU, int MB, bool AHEAD>
-__global__ void __launch_bounds__(64 * kExpWaves)
+template <bool GLU, int P, int MB, int WV, int U, bool AHEAD>
+__global__ void __launch_bounds__(64 * WV)
 experts_first_kernel(bf16_t* __restrict__ y, bf16_t* __restrict__ ys, float* __restrict__ sg,
                      const bf16_t* __restrict__ h, long h_stride, int rows, const int* __restrict__ idx, int top,
                      ExpertSet E, int act, float limit, float shared_limit) {
-  constexpr int P = GLU ? 1 : 2;
-  __shared__ float4 red[kExpLds<MB, AHEAD> / 16];
-  __shared__ int list[kFewRows], counts[kExpWaves];
+  __shared__ float4 red[kExpLds<GLU ? 2 * P : P, MB, WV, U>];
+  __shared__ int list[kFewRows], counts[WV];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int n0 = blockIdx.x * 16 * P;
-  if ((int)blockIdx.y < E.slots) {
+  const int n0 = blockIdx.x * 16 * P, slot = (int)blockIdx.y - (E.shared != nullptr ? 1 : 0);
+  if (slot >= 0) {
     if (n0 >= E.N) return;
-    const int e = expert_in_slot(idx, rows * top, E, blockIdx.y);
+    const int e = expert_in_slot(idx, rows * top, E, slot);
     if (e < 0) return;
     bool shared;
-    const int count = rows_of<kExpWaves>(idx, rows * top, top, E.experts, e, 16 * MB, list, counts, shared);
+    const int count = rows_of<WV>(idx, rows * top, top, E.experts, e, 16 * MB, list, counts, shared);
     if (count == 0) return;
     const bf16_t* W = E.w + (long)e * E.N * (GLU ? 2 : 1) * E.K;
-    expert_tile_any<P, GLU, kExpWaves, MB, AHEAD>(red, W, E.N, E.K, n0, h, h_stride, list, count, top, wave, lane,
+    expert_tile_any<P, GLU, WV, MB, U, AHEAD>(red, W, E.N, E.K, n0, h, h_stride, list, count, top, wave, lane,
                                        [&](int r, int c, float (&v)[4], float (&u)[4]) {
 #pragma unroll
                                          for (int i = 0; i < 4; ++i) v[i] = fr_act(act, limit, v[i], u[i]);
@@ -355,11 +347,11 @@ experts_first_kernel(bf16_t* __restrict__ y, bf16_t* __restrict__ ys, float* __r
   __syncthreads();
   if ((int)blockIdx.x == tiles) {
     const bf16_t* W = E.shared + (long)E.shared_N * (GLU ? 2 : 1) * E.K;
-    expert_tile_any<1, false, kExpWaves, MB, AHEAD>(red, W, 1, E.K, 0, h, h_stride, list, rows, 1, wave, lane,
+    expert_tile_any<1, false, WV, MB, U, AHEAD>(red, W, 1, E.K, 0, h, h_stride, list, rows, 1, wave, lane,
                                          [&](int r, int c, float (&v)[4], float (&)[4]) { if (c == 0) sg[r] = v[0]; });
     return;
   }
-  expert_tile_any<P, GLU, kExpWaves, MB, AHEAD>(red, E.shared, E.shared_N, E.K, n0, h, h_stride, list, rows, 1, wave, lane,
+  expert_tile_any<P, GLU, WV, MB, U, AHEAD>(red, E.shared, E.shared_N, E.K, n0, h, h_stride, list, rows, 1, wave, lane,
                                      [&](int r, int c, float (&v)[4], float (&u)[4]) {
 #pragma unroll
                                        for (int i = 0; i < 4; ++i) v[i] = fr_act(act, shared_limit, v[i], u[i]);
@@ -368,25 +360,24 @@ experts_first_kernel(bf16_t* __restrict__ y, bf16_t* __restrict__ ys, float* __r
 }
 
 // d[pair] = W_down of the pair's expert times y[pair], ds[row] the shared expert's, fp32
-template <int MB, bool AHEAD>
-__global__ void __launch_bounds__(64 * kExpWaves)
+template <int P, int MB, int WV, int U>
+__global__ void __launch_bounds__(64 * WV)
 experts_down_kernel(float* __restrict__ d, float* __restrict__ ds, const bf16_t* __restrict__ y,
                     const bf16_t* __restrict__ ys, int rows, const int* __restrict__ idx, int top, ExpertSet E) {
-  constexpr int P = 2;
-  __shared__ float4 red[kExpLds<MB, AHEAD> / 16];
-  __shared__ int list[kFewRows], counts[kExpWaves];
+  __shared__ float4 red[kExpLds<P, MB, WV, U>];
+  __shared__ int list[kFewRows], counts[WV];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int n0 = blockIdx.x * 16 * P;
-  const bool routed = (int)blockIdx.y < E.slots;
-  const int e = routed ? expert_in_slot(idx, rows * top, E, blockIdx.y) : 0;
+  const int n0 = blockIdx.x * 16 * P, slot = (int)blockIdx.y - (E.shared != nullptr ? 1 : 0);
+  const bool routed = slot >= 0;
+  const int e = routed ? expert_in_slot(idx, rows * top, E, slot) : 0;
   if (e < 0) return;
   float* dst = d;
   const bf16_t *W = E.w + (long)e * E.N * E.K, *X = y;
   int K = E.K, count = rows;
   bool shared = false;
   if (routed) {
-    count = rows_of<kExpWaves>(idx, rows * top, top, E.experts, e, 16 * MB, list, counts, shared);
+    count = rows_of<WV>(idx, rows * top, top, E.experts, e, 16 * MB, list, counts, shared);
     if (count == 0) return;
   } else {
     if (tid < rows) list[tid] = tid;
@@ -396,7 +387,7 @@ experts_down_kernel(float* __restrict__ d, float* __restrict__ ds, const bf16_t*
     X = ys;
     K = E.shared_K;
   }
-  expert_tile_any<P, false, kExpWaves, MB, AHEAD>(red, W, E.N, K, n0, X, K, list, count, 1, wave, lane,
+  expert_tile_any<P, false, WV, MB, U, false>(red, W, E.N, K, n0, X, K, list, count, 1, wave, lane,
                                        [&](int r, int c, float (&v)[4], float (&)[4]) {
                                          const int p = list[r];
                                          fr_store4(dst + (long)p * E.N, c, E.N, true, v);
@@ -533,51 +524,63 @@ extern "C" int mx_experts_few(float* out, void* y, float* d, const void* h, long
                               hipStream_t s) {
   if (rows <= 0) return 0;
   if (rows > kFewRows || experts < 1 || experts > 65534 || top < 1 || ff % 8 || width % 8 ||
-      ff < 8 || width < 8 || h_stride % 8 || shared_ff % 8 || act < kFrGelu || act > kFrReluSq) return -1;
+      ff < 8 || width < 8 || h_stride % 8 || shared_ff % 8 || act < kFrGelu || act > kFrReluSq ||
+      (shared_w == nullptr) != (shared_down == nullptr)) return -1;
   if (((uintptr_t)h) % 16 || ((uintptr_t)wgu) % 16 || ((uintptr_t)wdown) % 16 || ((uintptr_t)shared_w) % 16 ||
       ((uintptr_t)shared_down) % 16) return -2;
-  const bool glu = act != kFrReluSq;
-  const int cols = glu ? 16 : 32;
-  const bool sh = shared_w != nullptr;
+  const bool glu = act != kFrReluSq, sh = shared_w != nullptr;
+  // Forms by the rows, us of 32 experts and a shared one (rows of the comment above), tiles a workgroup x waves x steps of k a round:
+  //   first, gated      1 x 4 x 1   1 x 4 x 2, the next round's loads under a round   1 x 8 x 1    (4096 wide, 32 rows: 1 x 8 x 2 241, x 1 248)
+  //     8 rows          41.1        36.4                                               37.9
+  //     32 rows         56.2        -                                                  52.8
+  //     64 rows         61.2        -                                                  64.3
+  //   first, relu^2     2 x 4 x 1   1 x 4 x 2, loads ahead    1 x 8 x 1   1 x 4 x 1
+  //     8 rows          39.5        29.6                      29.6        30.5
+  //     32 rows         50.2        -                         40.8        43.4
+  //     64 rows         55.7        -                         60.9        56.4
+  //   down              2 x 4 x 1   1 x 4 x 2                 2 x 8 x 1   (of 1024 / 1536)
+  //     8 rows          21.7 33     19.8 29.9                 20.4 30.4
+  //     32 rows         29.0 43.4   - 44.6                    29.0 41.3
+  //     64 rows         33.5 48.0   -                         36.7 51.0
+  const bool many = rows > 32;
+  const int p1 = glu || !many ? 1 : 2, p2 = rows <= 16 ? 1 : 2, cols = 16 * p1;
   const int tiles = (ff + cols - 1) / cols, tiles_s = sh ? (shared_ff + cols - 1) / cols + (sg != nullptr) : 0;
+  const int tiles_d = (width + 16 * p2 - 1) / (16 * p2);
   // The lines below are from 700 layers of at most 16 rows, 4 to 128 experts, sizes at random.  Rows of the grid per pair: less than 150
   // workgroups spared cost up to 0.9 us (the choices are read first), 150 to 300 are level (-3 to 1), 300 to 600 save 0.5, 1000 1.2 and
   // more 2 to 5.  Loads ahead: 1.01 to 1.12 of the time at 1 to 3 steps of k a wave, whatever the grid; from 4 on 0.94 to 0.99 up to a
-  // workgroup a CU, 0.96 to 0.99 with three and more, between these 1.00 to 1.03 (up to 1.2).  So chosen 0.970 of the time with neither in
-  // the mean, above 1.03 in 3 %.
+  // workgroup a CU, 0.96 to 0.99 with three and more, between these 1.00 to 1.03 (up to 1.2).
   const int pairs = rows * top;
   const auto slots = [&](int cols) { return experts <= 64 && pairs < experts && (long)(experts - pairs) * cols >= 150 ? pairs : experts; };
   // workgroups that have rows, where the rows choose their experts independently
-  const float chosen = experts * (1.f - powf(1.f - (float)(top < experts ? top : experts) / experts, (float)rows));
-  const auto ahead = [&](int k, int cols, int shared_cols) {
-    const float groups = chosen * cols + shared_cols;
-    return (k + 63) / 64 > 3 * kExpWaves && (groups <= 256.f || groups > 700.f);
-  };
-  const int tiles_d = (width + 31) / 32;
+  const float groups = experts * (1.f - powf(1.f - (float)(top < experts ? top : experts) / experts, (float)rows)) * tiles + tiles_s;
+  const bool ahead = (width + 63) / 64 > 12 && (groups <= 256.f || groups > 700.f);
   ExpertSet first{(const bf16_t*)wgu, (const bf16_t*)shared_w, experts, width, ff, width, shared_ff, slots(tiles)};
   ExpertSet down{(const bf16_t*)wdown, (const bf16_t*)shared_down, experts, ff, width, shared_ff, width, slots(tiles_d)};
-  const dim3 g1((unsigned)(tiles > tiles_s ? tiles : tiles_s), (unsigned)(first.slots + (sh ? 1 : 0))), block(64 * kExpWaves);
+  const dim3 g1((unsigned)(tiles > tiles_s ? tiles : tiles_s), (unsigned)(first.slots + (sh ? 1 : 0)));
   const dim3 g2((unsigned)tiles_d, (unsigned)(down.slots + (sh ? 1 : 0)));
-  const auto go = [&](auto mb, auto first_ahead, auto down_ahead) {
-    constexpr int MB = decltype(mb)::value;
-    constexpr bool AF = decltype(first_ahead)::value, AD = decltype(down_ahead)::value;
-    if (glu)
-      hipLaunchKernelGGL((experts_first_kernel<true, MB, AF>), g1, block, 0, s, (bf16_t*)y, (bf16_t*)ys, sg, (const bf16_t*)h, h_stride, rows,
-                         idx, top, first, act, limit, shared_limit);
-    else
-      hipLaunchKernelGGL((experts_first_kernel<false, MB, AF>), g1, block, 0, s, (bf16_t*)y, (bf16_t*)ys, sg, (const bf16_t*)h, h_stride, rows,
-                         idx, top, first, act, limit, shared_limit);
-    hipLaunchKernelGGL((experts_down_kernel<MB, AD>), g2, block, 0, s, d, ds, (const bf16_t*)y, (const bf16_t*)ys, rows, idx, top, down);
-  };
-  const bool a1 = ahead(width, tiles, tiles_s), a2 = ahead(ff, tiles_d, sh ? tiles_d : 0);
-  using std::bool_constant;
-  using std::integral_constant;
-  if (rows > 32) go(integral_constant<int, 4>{}, bool_constant<false>{}, bool_constant<false>{});
-  else if (rows > 16) go(integral_constant<int, 2>{}, bool_constant<false>{}, bool_constant<false>{});
-  else if (a1 && a2) go(integral_constant<int, 1>{}, bool_constant<true>{}, bool_constant<true>{});
-  else if (a1) go(integral_constant<int, 1>{}, bool_constant<true>{}, bool_constant<false>{});
-  else if (a2) go(integral_constant<int, 1>{}, bool_constant<false>{}, bool_constant<true>{});
-  else go(integral_constant<int, 1>{}, bool_constant<false>{}, bool_constant<false>{});
+#define EX_FIRST(GLU, P, MB, WV, U, AHEAD)                                                                                \
+  hipLaunchKernelGGL((experts_first_kernel<GLU, P, MB, WV, U, AHEAD>), g1, dim3(64 * WV), 0, s, (bf16_t*)y, (bf16_t*)ys, sg, \
+                     (const bf16_t*)h, h_stride, rows, idx, top, first, act, limit, shared_limit)
+#define EX_DOWN(P, MB, WV, U)                                                                                          \
+  hipLaunchKernelGGL((experts_down_kernel<P, MB, WV, U>), g2, dim3(64 * WV), 0, s, d, ds, (const bf16_t*)y, (const bf16_t*)ys, \
+                     rows, idx, top, down)
+#define EX_FIRST_ROWS(GLU)                                \
+  do {                                                    \
+    if (many) EX_FIRST(GLU, GLU ? 1 : 2, 4, 4, 1, false); \
+    else if (rows > 16 && width >= 4096) EX_FIRST(GLU, 1, 2, 8, 2, false); \
+    else if (rows > 16) EX_FIRST(GLU, 1, 2, 8, 1, false); \
+    else if (ahead) EX_FIRST(GLU, 1, 1, 4, 2, true);      \
+    else EX_FIRST(GLU, 1, 1, 4, 1, false);                \
+  } while (0)
+  if (glu) EX_FIRST_ROWS(true);
+  else EX_FIRST_ROWS(false);
+  if (many) EX_DOWN(2, 4, 4, 1);
+  else if (rows > 16) EX_DOWN(2, 2, 8, 1);
+  else EX_DOWN(1, 1, 4, 2);
+#undef EX_FIRST_ROWS
+#undef EX_FIRST
+#undef EX_DOWN
   if (out == nullptr) return (int)hipGetLastError();       // (the step behind sums them: rows.hip, ExpertRows)
   hipLaunchKernelGGL(experts_combine_kernel, dim3((unsigned)((width + 255) / 256), (unsigned)rows), dim3(256), 0, s,
                      out, d, wts, sh ? ds : nullptr, sg, top, width);
