@@ -121,11 +121,11 @@ int mx_gla_scan(float* o, const void* qkv, int bf16, long qkv_stride, const void
 int mx_pair_embed_add(float* x, const int* ids, const void* table, int bf16, int rows, int width, long mul_prev,
                       long mul_cur, int buckets, const int* start, const int* pos0, const int* slot, int num_segs,
                       int* last_tok, int num_slots, const void* embed, int vocab, float scale, hipStream_t s);
-int mx_add_scaled_rms_norm(float* x, const void* y1, int y1_bf16, long y1_stride, const void* y2, int y2_bf16,
-                           long y2_stride, float mult, const float* next_w, void* out, int out_bf16, int rows,
+int mx_add_scaled_rms_norm(float* x, const void* y1, int y1_bf16, long y1_stride, int y1_parts, const void* y2, int y2_bf16,
+                           long y2_stride, int y2_parts, float mult, const float* next_w, void* out, int out_bf16, int rows,
                            int width, float eps, hipStream_t s);
-int mx_dual_rms_mean(float* out, const void* a, long a_stride, const void* b, long b_stride, int bf16,
-                     const float* wa, const float* wb, int rows, int width, float eps, float scale, hipStream_t s);
+int mx_dual_rms_mean(float* out, const void* a, int a_bf16, long a_stride, int a_parts, const void* b, int b_bf16, long b_stride,
+                     int b_parts, const float* wa, const float* wb, int rows, int width, float eps, float scale, hipStream_t s);
 int mx_sigmoid_gate(void* out, int out_bf16, const float* o, const void* g, int g_bf16, long g_stride, long rows,
                     int n, hipStream_t s);
 int mx_attn_prep(float* q_out, const void* qkv, int bf16, long stride, int nq, int nk, int nv, const float* wq,
@@ -223,6 +223,8 @@ int mx_moe_topk(int* idx, float* wts, const float* z, const float* corr, long ro
                 int groups, int keep, hipStream_t s);
 int mx_few_rows_max();
 int mx_few_rows_parts(int N, int K);
+int mx_tile_parts(long M, int N, int K);
+int mx_tile_gemm_parts(float* D, const void* A, long a_stride, const void* W, const void* bias, long M, int N, int K, hipStream_t s);
 int mx_few_rows_gemm_parts(float* D, const void* X, long x_stride, int rows, const void* W, const void* bias, int N, int K,
                            int parts, hipStream_t s);
 int mx_moe_route_fits(const void* h, long h_stride, const void* parts, int experts, int width);
@@ -803,7 +805,14 @@ void pair_embed_add(Tensor x, Tensor ids, Tensor table, int64_t mul_prev, int64_
                         (float)scale, stream()), "pair_embed_add");
 }
 
-void add_scaled_rms_norm(Tensor x, OptT y1, OptT y2, double mult, OptT next_w, OptT out, double eps) {
+// rows [rows, width], or with parts > 1 fp32 [rows * parts, width]
+void check_parts(const Tensor& y, int64_t parts, int64_t rows, int64_t width, const char* what) {
+  check_rows(y, what);
+  TORCH_CHECK(parts >= 1 && parts <= 64 && y.size(0) == rows * parts && y.size(1) == width &&
+              (parts == 1 || (!bf(y) && y.is_contiguous())), what, " shape");
+}
+
+void add_scaled_rms_norm(Tensor x, OptT y1, OptT y2, double mult, OptT next_w, OptT out, double eps, int64_t y1_parts, int64_t y2_parts) {
   check_f32(x, "residual");
   TORCH_CHECK(x.dim() == 2, "residual 2-D");
   const int64_t rows = x.size(0), width = x.size(1);
@@ -812,13 +821,11 @@ void add_scaled_rms_norm(Tensor x, OptT y1, OptT y2, double mult, OptT next_w, O
   int b1 = 0, b2 = 0;
   long s1 = 0, s2 = 0;
   if (y1) {
-    check_rows(*y1, "y1");
-    TORCH_CHECK(y1->size(0) == rows && y1->size(1) == width, "y1 shape");
+    check_parts(*y1, y1_parts, rows, width, "y1");
     p1 = y1->data_ptr(); b1 = bf(*y1); s1 = y1->stride(0);
   }
   if (y2) {
-    check_rows(*y2, "y2");
-    TORCH_CHECK(y2->size(0) == rows && y2->size(1) == width, "y2 shape");
+    check_parts(*y2, y2_parts, rows, width, "y2");
     p2 = y2->data_ptr(); b2 = bf(*y2); s2 = y2->stride(0);
   }
   void* op = nullptr;
@@ -828,22 +835,23 @@ void add_scaled_rms_norm(Tensor x, OptT y1, OptT y2, double mult, OptT next_w, O
     op = out->data_ptr();
     obf = bf(*out);
   }
-  chk(mx_add_scaled_rms_norm(x.data_ptr<float>(), p1, b1, s1, p2, b2, s2, (float)mult,
+  chk(mx_add_scaled_rms_norm(x.data_ptr<float>(), p1, b1, s1, y1 ? (int)y1_parts : 1, p2, b2, s2, y2 ? (int)y2_parts : 1, (float)mult,
                              opt_f32(next_w, width, "next norm weight"), op, obf, (int)rows, (int)width, (float)eps,
                              stream()), "add_scaled_rms_norm");
 }
 
-void dual_rms_mean(Tensor out, Tensor a, Tensor b, Tensor wa, Tensor wb, double eps, double scale) {
+void dual_rms_mean(Tensor out, Tensor a, Tensor b, Tensor wa, Tensor wb, double eps, double scale, int64_t a_parts, int64_t b_parts) {
   check_f32(out, "out");
-  check_rows(a, "a");
-  check_rows(b, "b");
   check_f32(wa, "wa");
   check_f32(wb, "wb");
-  const int64_t rows = a.size(0), width = a.size(1);
-  TORCH_CHECK(b.sizes() == a.sizes() && b.scalar_type() == a.scalar_type() && out.dim() == 2 && out.size(0) == rows &&
-              out.size(1) == width && wa.numel() == width && wb.numel() == width, "dual_rms_mean shapes");
-  chk(mx_dual_rms_mean(out.data_ptr<float>(), a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0), bf(a),
-                       wa.data_ptr<float>(), wb.data_ptr<float>(), (int)rows, (int)width, (float)eps, (float)scale,
+  TORCH_CHECK(out.dim() == 2, "out 2-D");
+  const int64_t rows = out.size(0), width = out.size(1);
+  check_parts(a, a_parts, rows, width, "a");
+  check_parts(b, b_parts, rows, width, "b");
+  TORCH_CHECK((b.scalar_type() == a.scalar_type() || a_parts > 1 || b_parts > 1) && wa.numel() == width && wb.numel() == width,
+              "dual_rms_mean shapes");
+  chk(mx_dual_rms_mean(out.data_ptr<float>(), a.data_ptr(), bf(a), a.stride(0), (int)a_parts, b.data_ptr(), bf(b), b.stride(0),
+                       (int)b_parts, wa.data_ptr<float>(), wb.data_ptr<float>(), (int)rows, (int)width, (float)eps, (float)scale,
                        stream()), "dual_rms_mean");
 }
 
@@ -1097,6 +1105,20 @@ void few_rows_gemm_parts(Tensor d, Tensor x, Tensor w, OptT bias) {
               "few_rows_gemm_parts bias");
   chk(mx_few_rows_gemm_parts(d.data_ptr<float>(), x.data_ptr(), x.stride(0), (int)rows, w.data_ptr(), bias ? bias->data_ptr() : nullptr, (int)n, (int)x.size(1),
                              (int)(d.size(0) / rows), stream()), "few_rows_gemm_parts");
+}
+
+// d [rows * tile_parts, n] fp32: the same of more rows, by tiles
+void tile_gemm_parts(Tensor d, Tensor x, Tensor w, OptT bias) {
+  check_rows(x, "x");
+  check_f32(d, "d");
+  const int64_t rows = x.size(0), n = w.size(0), k = x.size(1);
+  TORCH_CHECK(x.scalar_type() == at::kBFloat16 && w.is_cuda() && w.is_contiguous() && w.scalar_type() == at::kBFloat16 && w.dim() == 2 &&
+              w.size(1) == k && rows >= 1 && rows <= 1024 && n >= 1 && n <= 0x3fffffff && k <= 0x3fffffff && d.dim() == 2 && d.size(1) == n &&
+              d.size(0) == rows * mx_tile_parts(rows, (int)n, (int)k), "tile_gemm_parts shapes");
+  TORCH_CHECK(!bias || (bias->is_cuda() && bias->scalar_type() == at::kBFloat16 && bias->is_contiguous() && bias->numel() == n),
+              "tile_gemm_parts bias");
+  chk(mx_tile_gemm_parts(d.data_ptr<float>(), x.data_ptr(), x.stride(0), w.data_ptr(), bias ? bias->data_ptr() : nullptr, rows, (int)n,
+                         (int)k, stream()), "tile_gemm_parts");
 }
 
 // two products of the same sizes and strides in one launch
@@ -1900,8 +1922,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("head_max_dk", []() { return (int64_t)mx_head_max_dk(); });
   m.def("gated_linear_attention", &gated_linear_attention);
   m.def("pair_embed_add", &pair_embed_add);
-  m.def("add_scaled_rms_norm", &add_scaled_rms_norm);
-  m.def("dual_rms_mean", &dual_rms_mean);
+  m.def("add_scaled_rms_norm", &add_scaled_rms_norm, py::arg("x"), py::arg("y1"), py::arg("y2"), py::arg("mult"), py::arg("next_w"),
+        py::arg("out"), py::arg("eps"), py::arg("y1_parts") = 1, py::arg("y2_parts") = 1);
+  m.def("dual_rms_mean", &dual_rms_mean, py::arg("out"), py::arg("a"), py::arg("b"), py::arg("wa"), py::arg("wb"), py::arg("eps"),
+        py::arg("scale"), py::arg("a_parts") = 1, py::arg("b_parts") = 1);
   m.def("sigmoid_gate", &sigmoid_gate);
   m.def("latent_kv_write", &latent_kv_write);
   m.def("latent_q_rope", &latent_q_rope);
@@ -1912,6 +1936,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("few_rows_gemm", &few_rows_gemm);
   m.def("few_rows_pair", &few_rows_pair);
   m.def("few_rows_gemm_parts", &few_rows_gemm_parts);
+  m.def("tile_gemm_parts", &tile_gemm_parts);
+  m.def("tile_parts", [](int64_t m, int64_t n, int64_t k) { return mx_tile_parts(m, (int)n, (int)k); });
   m.def("few_rows_parts", [](int64_t n, int64_t k) { return (int64_t)mx_few_rows_parts((int)n, (int)k); });
   m.def("few_rows_side_gate", &few_rows_side_gate);
   m.def("expert_rows_fit", [](int64_t width) { return (bool)mx_expert_rows_fit((int)width); });

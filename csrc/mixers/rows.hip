@@ -271,6 +271,18 @@ struct ExpertRows {
     }
   }
 };
+struct AnyRows {                              // either, by the launch: bf16 or fp32 rows, or a product's parts
+  const void* p;
+  int bf16, parts;
+  long stride;
+  __device__ __forceinline__ bool any() const { return p != nullptr; }
+  template <int NT, int C>
+  __device__ __forceinline__ void load(float (&v)[C][4], long row, int width, int vec) const {
+    if (parts > 1) ExpertRows{(const float*)p, nullptr, nullptr, nullptr, parts}.load<NT, C>(v, row, width, vec);
+    else if (bf16) load_row<bf16_t, NT, C>(v, (const bf16_t*)p + row * stride, width, vec);
+    else load_row<float, NT, C>(v, (const float*)p + row * stride, width, vec);
+  }
+};
 
 // sums of two values over a block; every thread gets both
 template <int NT>
@@ -366,25 +378,20 @@ layer_norm_row_kernel(float* __restrict__ x, Y y, const float* __restrict__ w,
 
 template <typename TO, int NT, int C>
 __global__ void __launch_bounds__(NT)
-add_scaled_rms_norm_row_kernel(float* __restrict__ x, const void* __restrict__ y1, int y1_bf16, long y1_stride,
-                               const void* __restrict__ y2, int y2_bf16, long y2_stride, float mult,
+add_scaled_rms_norm_row_kernel(float* __restrict__ x, AnyRows y1, AnyRows y2, float mult,
                                const float* __restrict__ next_w, TO* __restrict__ out, int width, float eps, int vec) {
   __shared__ float red[NT / 64];
   const long row = blockIdx.x;
   float v[C][4], a[C][4], b[C][4], w[C][4];
-  auto side = [&](float (&t)[C][4], const void* y, int bf16, long stride) {
-    if (bf16) load_row<bf16_t, NT, C>(t, (const bf16_t*)y + row * stride, width, vec);
-    else load_row<float, NT, C>(t, (const float*)y + row * stride, width, vec);
-  };
   load_row<float, NT, C>(v, x + row * width, width, vec);
-  if (y1 != nullptr) side(a, y1, y1_bf16, y1_stride);
-  if (y2 != nullptr) side(b, y2, y2_bf16, y2_stride);
+  if (y1.any()) y1.load<NT, C>(a, row, width, vec);
+  if (y2.any()) y2.load<NT, C>(b, row, width, vec);
   if (out != nullptr) load_row<float, NT, C>(w, next_w, width, vec);
-  if (y1 != nullptr) {
+  if (y1.any()) {
 #pragma unroll
     for (int c = 0; c < C; ++c)
 #pragma unroll
-      for (int k = 0; k < 4; ++k) v[c][k] += mult * (y2 != nullptr ? a[c][k] + b[c][k] : a[c][k]);
+      for (int k = 0; k < 4; ++k) v[c][k] += mult * (y2.any() ? a[c][k] + b[c][k] : a[c][k]);
     store_row<float, NT, C>(x + row * width, v, width, vec);
   }
   if (out == nullptr) return;
@@ -396,16 +403,15 @@ add_scaled_rms_norm_row_kernel(float* __restrict__ x, const void* __restrict__ y
   store_row<TO, NT, C>(out + row * width, v, width, vec);
 }
 
-template <typename T, int NT, int C>
+template <int NT, int C>
 __global__ void __launch_bounds__(NT)
-dual_rms_mean_row_kernel(float* __restrict__ out, const T* __restrict__ a, long a_stride, const T* __restrict__ b,
-                         long b_stride, const float* __restrict__ wa, const float* __restrict__ wb, int width, float eps,
-                         float scale, int vec) {
+dual_rms_mean_row_kernel(float* __restrict__ out, AnyRows a, AnyRows b, const float* __restrict__ wa,
+                         const float* __restrict__ wb, int width, float eps, float scale, int vec) {
   __shared__ float red[NT / 64][2];
   const long row = blockIdx.x;
   float u[C][4], v[C][4], p[C][4], q[C][4];
-  load_row<T, NT, C>(u, a + row * a_stride, width, vec);
-  load_row<T, NT, C>(v, b + row * b_stride, width, vec);
+  a.load<NT, C>(u, row, width, vec);
+  b.load<NT, C>(v, row, width, vec);
   load_row<float, NT, C>(p, wa, width, vec);
   load_row<float, NT, C>(q, wb, width, vec);
   float sa = sum_sq<C>(u), sb = sum_sq<C>(v);
@@ -1103,26 +1109,31 @@ extern "C" int mx_pair_embed_add(float* x, const int* ids, const void* table, in
   return (int)hipGetLastError();
 }
 
-extern "C" int mx_add_scaled_rms_norm(float* x, const void* y1, int y1_bf16, long y1_stride, const void* y2,
-                                      int y2_bf16, long y2_stride, float mult, const float* next_w, void* out,
+// whether AnyRows may be read four entries at a time; parts: -1 if they cannot be read
+static int any_rows_vec(const AnyRows& y, int width) {
+  if (y.parts > 1) return y.p != nullptr && !y.bf16 && mx_expert_rows_fit(width) && ((uintptr_t)y.p) % 16 == 0 ? 1 : -1;
+  return y.p == nullptr || (y.stride % 4 == 0 && ((uintptr_t)y.p) % (y.bf16 ? 8 : 16) == 0);
+}
+
+// y1, y2: rows of their stride, or (parts > 1) fp32 [rows * parts, width] whose sums over the parts are the rows
+extern "C" int mx_add_scaled_rms_norm(float* x, const void* y1, int y1_bf16, long y1_stride, int y1_parts, const void* y2,
+                                      int y2_bf16, long y2_stride, int y2_parts, float mult, const float* next_w, void* out,
                                       int out_bf16, int rows, int width, float eps, hipStream_t s) {
   if (rows <= 0) return 0;
   if (y1 == nullptr && (y2 != nullptr || out == nullptr)) return -1;
-  auto fits = [](const void* y, int bf16, long stride) {
-    return y == nullptr || (stride % 4 == 0 && ((uintptr_t)y) % (bf16 ? 8 : 16) == 0);
-  };
-  const int vec = width % 4 == 0 && fits(y1, y1_bf16, y1_stride) && fits(y2, y2_bf16, y2_stride) &&
+  const AnyRows a{y1, y1_bf16, y1_parts, y1_stride}, b{y2, y2_bf16, y2_parts, y2_stride};
+  const int va = any_rows_vec(a, width), vb = any_rows_vec(b, width);
+  if (va < 0 || vb < 0) return -2;
+  const int vec = width % 4 == 0 && va && vb &&
                   ((uintptr_t)x | (uintptr_t)next_w) % 16 == 0 && ((uintptr_t)out) % (out_bf16 ? 8 : 16) == 0;
-  if (row_in_registers(rows, width, vec)) {
+  if (row_in_registers(rows, width, vec) || y1_parts > 1 || y2_parts > 1) {
     row_chunks(width, [&](auto c) {
       if (out_bf16)
         hipLaunchKernelGGL((add_scaled_rms_norm_row_kernel<bf16_t, kRowThreads, decltype(c)::value>), dim3(rows),
-                           dim3(kRowThreads), 0, s, x, y1, y1_bf16, y1_stride, y2, y2_bf16, y2_stride, mult, next_w,
-                           (bf16_t*)out, width, eps, vec);
+                           dim3(kRowThreads), 0, s, x, a, b, mult, next_w, (bf16_t*)out, width, eps, vec);
       else
         hipLaunchKernelGGL((add_scaled_rms_norm_row_kernel<float, kRowThreads, decltype(c)::value>), dim3(rows),
-                           dim3(kRowThreads), 0, s, x, y1, y1_bf16, y1_stride, y2, y2_bf16, y2_stride, mult, next_w,
-                           (float*)out, width, eps, vec);
+                           dim3(kRowThreads), 0, s, x, a, b, mult, next_w, (float*)out, width, eps, vec);
     });
     return (int)hipGetLastError();
   }
@@ -1135,23 +1146,25 @@ extern "C" int mx_add_scaled_rms_norm(float* x, const void* y1, int y1_bf16, lon
   return (int)hipGetLastError();
 }
 
-extern "C" int mx_dual_rms_mean(float* out, const void* a, long a_stride, const void* b, long b_stride, int bf16,
-                                const float* wa, const float* wb, int rows, int width, float eps, float scale,
-                                hipStream_t s) {
+// a, b: as mx_add_scaled_rms_norm's, both bf16 or both fp32 unless in parts
+extern "C" int mx_dual_rms_mean(float* out, const void* a, int a_bf16, long a_stride, int a_parts, const void* b, int b_bf16,
+                                long b_stride, int b_parts, const float* wa, const float* wb, int rows, int width, float eps,
+                                float scale, hipStream_t s) {
   if (rows <= 0) return 0;
-  const int vec = width % 4 == 0 && a_stride % 4 == 0 && b_stride % 4 == 0 &&
-                  ((uintptr_t)a | (uintptr_t)b) % (bf16 ? 8 : 16) == 0 &&
-                  ((uintptr_t)out | (uintptr_t)wa | (uintptr_t)wb) % 16 == 0;
-  if (row_in_registers(rows, width, vec)) {
+  const AnyRows ra{a, a_bf16, a_parts, a_stride}, rb{b, b_bf16, b_parts, b_stride};
+  const int va = any_rows_vec(ra, width), vb = any_rows_vec(rb, width);
+  if (va < 0 || vb < 0) return -2;
+  const int vec = width % 4 == 0 && va && vb && ((uintptr_t)out | (uintptr_t)wa | (uintptr_t)wb) % 16 == 0;
+  if (row_in_registers(rows, width, vec) || a_parts > 1 || b_parts > 1) {
     row_chunks(width, [&](auto c) {
-      MX_DISPATCH_T(bf16, hipLaunchKernelGGL((dual_rms_mean_row_kernel<T, kRowThreads, decltype(c)::value>), dim3(rows),
-                                             dim3(kRowThreads), 0, s, out, (const T*)a, a_stride, (const T*)b, b_stride,
-                                             wa, wb, width, eps, scale, vec));
+      hipLaunchKernelGGL((dual_rms_mean_row_kernel<kRowThreads, decltype(c)::value>), dim3(rows), dim3(kRowThreads), 0, s,
+                         out, ra, rb, wa, wb, width, eps, scale, vec);
     });
     return (int)hipGetLastError();
   }
-  MX_DISPATCH_T(bf16, hipLaunchKernelGGL((dual_rms_mean_kernel<T, 256>), dim3(rows), dim3(256), 0, s, out,
-                                         (const T*)a, a_stride, (const T*)b, b_stride, wa, wb, width, eps, scale));
+  if (a_bf16 != b_bf16) return -1;
+  MX_DISPATCH_T(a_bf16, hipLaunchKernelGGL((dual_rms_mean_kernel<T, 256>), dim3(rows), dim3(256), 0, s, out,
+                                           (const T*)a, a_stride, (const T*)b, b_stride, wa, wb, width, eps, scale));
   return (int)hipGetLastError();
 }
 

@@ -46,6 +46,8 @@ struct TileArgs {
   unsigned a_bytes, w_bytes;         // between rows
   int groups, M, N, K, col_tiles, act, vec;
   float limit;
+  float* parts;                      // PARTS kernels: [M][gridDim.y][N], the sums over a part of k each, instead of C
+  int part_stages;                   // of k in a part
 };
 
 // a workgroup's group, rows row0 .. end - 1 of it and column tile
@@ -180,6 +182,20 @@ __device__ __forceinline__ void tile_result(const TileArgs& P, int col, const fr
       if (P.act == kFrReluSq) v[e] = fr_act(P.act, P.limit, v[e], 0.f);
     }
   }
+}
+
+// a part's sums out, four columns a lane (N in whole fours); the bias goes with the first part
+template <typename F>
+__device__ __forceinline__ void tile_part_out(const TileArgs& P, int row0, int end, int n0, F put) {
+  put([&](int r, int c, const fr_f32x4& x, const fr_f32x4&) {
+    if (row0 + r >= end || n0 + c >= P.N) return;
+    float v[4] = {x[0], x[1], x[2], x[3]};
+    if (P.bias != nullptr && blockIdx.y == 0) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] += ft::bf16_to_f32(P.bias[n0 + c + e]);
+    }
+    *reinterpret_cast<float4*>(P.parts + ((long)(row0 + r) * gridDim.y + blockIdx.y) * P.N + n0 + c) = make_float4(v[0], v[1], v[2], v[3]);
+  });
 }
 
 // ROWS rows of OC results out: put(write) hands every lane's (row of the tile, column of the tile, sums, up sums) to `write`.  Where
@@ -373,7 +389,7 @@ tile_phase_kernel(TileArgs P) {
 template <int WM, int WN, int MT, int NT, int S>
 constexpr int kRingLds = S * (WM * MT + WN * NT) * 16 * 128;
 
-template <int WM, int WN, int MT, int NT, int S, bool GLU, bool SPREAD = false>
+template <int WM, int WN, int MT, int NT, int S, bool GLU, bool SPREAD = false, bool PARTS = false>
 __device__ __forceinline__ void tile_ring(const TileArgs& P, const TileAt& at, char* smem) {
   constexpr int NW = WM * WN, BM = WM * MT * 16, BN = WN * NT * 16;
   constexpr int PA = BM / (8 * NW), PB = BN / (8 * NW), PW = PA + PB;
@@ -383,8 +399,9 @@ __device__ __forceinline__ void tile_ring(const TileArgs& P, const TileAt& at, c
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WN, wn = wave % WN, l15 = lane & 15, g4 = lane >> 4;
   const int n0 = at.ct * OC;
-  const bf16_t* W = P.W + (long)at.g * P.N * (GLU ? 2 : 1) * P.K;
-  const int nk = P.K / kTK, k0 = SPREAD ? tile_first_stage(at.g, nk) : 0;
+  const int t0 = PARTS ? (int)blockIdx.y * P.part_stages : 0;
+  const bf16_t *A = P.A + t0 * kTK, *W = P.W + (long)at.g * P.N * (GLU ? 2 : 1) * P.K + t0 * kTK;
+  const int nk = PARTS ? min(P.part_stages, P.K / kTK - t0) : P.K / kTK, k0 = SPREAD ? tile_first_stage(at.g, nk) : 0;
   const uint32_t lds0 = ft::lds_off(smem);
   unsigned ap[PA], wp[PB];
 #pragma unroll
@@ -394,7 +411,7 @@ __device__ __forceinline__ void tile_ring(const TileArgs& P, const TileAt& at, c
   auto load1 = [&](int t, int slot, int p) {
     const uint32_t dst = lds0 + slot * kStage + wave * 1024;
     const int k = tile_stage_at<SPREAD>(t, k0, nk);
-    if (p < PA) tile_dma(P.A + k * kTK, ap[p < PA ? p : 0], dst + p * NW * 1024);
+    if (p < PA) tile_dma(A + k * kTK, ap[p < PA ? p : 0], dst + p * NW * 1024);
     else tile_dma(W + k * kTK, wp[p < PA ? 0 : p - PA], dst + BM * 128 + (p - PA) * NW * 1024);
   };
   fr_f32x4 acc[NT][MT];
@@ -478,22 +495,27 @@ __device__ __forceinline__ void tile_ring(const TileArgs& P, const TileAt& at, c
   first_half(slot);
 #pragma unroll
   for (int j = 0; j < MT; ++j) product(h1, j);
-  __syncthreads();
-  tile_out<BM, OC, NW, GLU>(P, smem, at.row0, at.end, n0, tid, [&](auto write) {
+  const auto put = [&](auto write) {
 #pragma unroll
     for (int j = 0; j < MT; ++j)
 #pragma unroll
       for (int i = 0; i < NT; i += GLU ? 2 : 1)
         write((wm * MT + j) * 16 + l15, (wn * NT + i) * 16 / (GLU ? 2 : 1) + 4 * g4, acc[i][j], acc[GLU ? i + 1 : i][j]);
-  });
+  };
+  if constexpr (PARTS) {
+    tile_part_out(P, at.row0, at.end, n0, put);
+    return;
+  }
+  __syncthreads();
+  tile_out<BM, OC, NW, GLU>(P, smem, at.row0, at.end, n0, tid, put);
 }
 
-template <int WM, int WN, int MT, int NT, int S, bool GLU>
+template <int WM, int WN, int MT, int NT, int S, bool GLU, bool PARTS = false>
 __global__ void __launch_bounds__(64 * WM * WN, 1)
 tile_ring_kernel(TileArgs P) {
   __shared__ __attribute__((aligned(16))) char smem[kRingLds<WM, WN, MT, NT, S>];
   TileAt at;
-  if (tile_at<WM * MT * 16>(P, threadIdx.x & 63, at)) tile_ring<WM, WN, MT, NT, S, GLU>(P, at, smem);
+  if (tile_at<WM * MT * 16>(P, threadIdx.x & 63, at)) tile_ring<WM, WN, MT, NT, S, GLU, false, PARTS>(P, at, smem);
 }
 
 // ---------------------------------------------------------------------------------
@@ -608,7 +630,7 @@ tile_tail_kernel(TileArgs P) {
 // KW waves that share a tile of MT x NT tiles of 16: wave w takes the stages w, w + KW, .. and stages its own operands
 // (no barrier before the sums meet in LDS, in wave order).
 // ---------------------------------------------------------------------------------
-template <int KW, int MT, int NT, bool GLU>
+template <int KW, int MT, int NT, bool GLU, bool PARTS = false>
 __global__ void __launch_bounds__(64 * KW, 1)
 tile_split_kernel(TileArgs P) {
   constexpr int BM = MT * 16, BN = NT * 16, PA = BM / 8, PB = BN / 8;
@@ -621,8 +643,9 @@ tile_split_kernel(TileArgs P) {
   TileAt at;
   if (!tile_at<BM>(P, lane, at)) return;
   const int n0 = at.ct * OC;
-  const bf16_t* W = P.W + (long)at.g * P.N * (GLU ? 2 : 1) * P.K;
-  const int nk = P.K / kTK;
+  const int t0 = PARTS ? (int)blockIdx.y * P.part_stages : 0;
+  const bf16_t *A = P.A + t0 * kTK, *W = P.W + (long)at.g * P.N * (GLU ? 2 : 1) * P.K + t0 * kTK;
+  const int nk = PARTS ? min(P.part_stages, P.K / kTK - t0) : P.K / kTK;
   const char* mine = smem + wave * kStage;
   const uint32_t lds0 = ft::lds_off(mine);
   unsigned ap[PA], wp[PB];
@@ -632,7 +655,7 @@ tile_split_kernel(TileArgs P) {
   for (int p = 0; p < PB; ++p) wp[p] = tile_w_off<GLU>(P, n0, p * 8 + (lane >> 3), lane);
   auto load = [&](int t) {
 #pragma unroll
-    for (int p = 0; p < PA; ++p) tile_dma(P.A + t * kTK, ap[p], lds0 + p * 1024);
+    for (int p = 0; p < PA; ++p) tile_dma(A + t * kTK, ap[p], lds0 + p * 1024);
 #pragma unroll
     for (int p = 0; p < PB; ++p) tile_dma(W + t * kTK, wp[p], lds0 + BM * 128 + p * 1024);
   };
@@ -692,6 +715,10 @@ tile_split_kernel(TileArgs P) {
     const fr_f32x4 x = sum(GLU ? 2 * n : n, m, l);
     fr_f32x4 up = x;
     if constexpr (GLU) up = sum(2 * n + 1, m, l);
+    if constexpr (PARTS) {
+      tile_part_out(P, row, at.end, col, [&](auto write) { write(0, 0, x, up); });
+      continue;
+    }
     float v[4];
     tile_result<GLU>(P, col, x, up, v);
     fr_store4(P.C + row * P.c_stride, col, P.N, P.vec != 0, v);
@@ -707,6 +734,9 @@ enum TileForm { kTile256x256, kTile256x128, kTile192x128, kTile128x128, kTile64x
 struct TileSize {
   int rows, cols;
   float begin, tile, stage, all_stage, all_tile;
+  float us(long tiles, float nk) const {
+    return begin + (float)((tiles + 255) / 256) * (tile + nk * stage) + tiles / 256.f * (all_tile + nk * all_stage);
+  }
 };
 constexpr TileSize kTileSizes[kTileForms] = {
     {256, 256, 1.7f, 5.8f, 0.885f, 0.503f, 5.6f}, {256, 128, 2.5f, 2.0f, 0.681f, 0.235f, 3.3f},
@@ -722,8 +752,7 @@ int tile_pick(long M, int N, int K, bool glu, bool groups, float* us) {
     const TileSize& z = kTileSizes[f];
     const int oc = z.cols / (glu ? 2 : 1);
     const long tiles = ((M + z.rows - 1) / z.rows) * ((N + oc - 1) / oc);
-    const float r = tiles / 256.f, whole = (float)((tiles + 255) / 256), nk = K / 64.f;
-    const float t = z.begin + whole * (z.tile + nk * z.stage) + r * (z.all_tile + nk * z.all_stage);
+    const float t = z.us(tiles, K / 64.f);
     if (t < least) least = t, best = f;
   }
   const long tiles = ((M + 255) / 256) * ((N + (glu ? 127 : 255)) / (glu ? 128 : 256)), last = tiles % kCus;
@@ -734,6 +763,34 @@ int tile_pick(long M, int N, int K, bool glu, bool groups, float* us) {
     if (t < least) least = t, best = kTileTail;
   }
   if (us != nullptr) *us = least;
+  return best;
+}
+
+// A product of few columns and long sums leaves most of the chip idle: up to 1024 rows of 2048 columns are 16 to 128 tiles.  With
+// k in parts, as fp32 sums that the norm step behind adds, every CU has a tile of a shorter chain.  By the forms' times, which the
+// parts' kernels keep to (60 products of 65 to 1024 rows: 0.6 to 1.08 of the estimate at whole parts), and what the norm step reads
+// beside them, at 6 TB/s.  us in a graph with the norm step, weights from HBM, at 65 / 130 / 300 / 600 / 777 / 1024 rows
+// (the sooner of the whole tiles and the vendor's beside them):
+//   n = 2048, k = 4096    12 15 18 24 28 32 (16 16 23 30 31 34)     k = 8192   18 21 28 36 44 50 (25 25 36 47 52 56)
+//   n = 3072, k = 8192    20 24 35 48 58 69 (26 29 37 56 67 71)     n = 4096, k = 14336   35 38 60 97 116 120 (47 59 79 117 120 134)
+// Left whole: k below 4096 (n = k = 2048: 11 13 18 20 22 beside 11 14 18 19 21), more than 1024 rows, whose parts leave the
+// caches (n = 2048, k = 8192, 2048 rows: 87 beside 76), and less than a tenth to gain (n = k = 4096, 777 rows: 48 beside 43).
+int tile_parts(long M, int N, int K, int* form) {
+  if (M > 1024 || K < 4096 || N % 4) return 1;
+  float least;
+  tile_pick(M, N, K, false, false, &least);
+  least *= 0.9f;
+  int best = 1;
+  for (int f : {kTile256x128, kTile192x128, kTile128x128, kTile64x128, kTile64x64}) {
+    const TileSize& z = kTileSizes[f];
+    const long tiles = ((M + z.rows - 1) / z.rows) * ((N + z.cols - 1) / z.cols);
+    for (int p : {2, 3, 4}) {
+      const int stages = (K / 64 + p - 1) / p;       // (64 at least: no part is without any)
+      if (M <= 256 && p == 3) continue;              // (a norm step that also routes takes two or four)
+      const float t = z.us(tiles * p, (float)stages) + (float)M * N * 4 * (p - 1) / 6e6f;
+      if (t < least) least = t, best = p, *form = f;
+    }
+  }
   return best;
 }
 
@@ -809,6 +866,41 @@ extern "C" int mx_tile_gemm(void* C, long c_stride, const void* A, long a_stride
   P.vec = c_stride % 8 == 0 && N % 8 == 0 && ((uintptr_t)C) % 16 == 0 ? 2 : c_stride % 4 == 0 && ((uintptr_t)C) % 8 == 0 ? 1 : 0;
   if (form < 0) form = tile_pick(M, N, K, glu, offs != nullptr, nullptr);
   return glu ? tile_launch<true>(P, form, s) : tile_launch<false>(P, form, s);
+}
+
+// into how many parts of k a product whose norm step adds them is cut; 1: not
+extern "C" int mx_tile_parts(long M, int N, int K) {
+  int form;
+  return mx_tile_gemm_fits(M, N, K, K, 0) ? tile_parts(M, N, K, &form) : 1;
+}
+
+// D [M][mx_tile_parts][N] fp32: the sums of A W^T over parts of k (the first: + bias)
+extern "C" int mx_tile_gemm_parts(float* D, const void* A, long a_stride, const void* W, const void* bias, long M, int N, int K,
+                                  hipStream_t s) {
+  if (M <= 0 || N <= 0) return 0;
+  if (!mx_tile_gemm_fits(M, N, K, a_stride, 0)) return -1;
+  if (((uintptr_t)A | (uintptr_t)W | (uintptr_t)D) % 16) return -2;
+  int form;
+  const int parts = tile_parts(M, N, K, &form);
+  if (parts < 2) return -1;
+  TileArgs P{nullptr, (const bf16_t*)A, nullptr, (const bf16_t*)W, (const bf16_t*)bias, nullptr, 0, (unsigned)(a_stride * 2),
+             (unsigned)(K * 2), 1, (int)M, N, K, 0, kFrStore, 0, 0.f, D, (K / kTK + parts - 1) / parts};
+  const TileSize& z = kTileSizes[form];
+  P.col_tiles = (N + z.cols - 1) / z.cols;
+  const long tiles = ((M + z.rows - 1L) / z.rows) * P.col_tiles;
+  if (tiles > 0x7ffffff0L) return -3;
+  const dim3 grid((unsigned)((tiles + 7) / 8 * 8), (unsigned)parts), block(512);
+#define TG_GO(...) hipLaunchKernelGGL((__VA_ARGS__), grid, block, 0, s, P)
+  switch (form) {
+    case kTile256x128: TG_GO(tile_ring_kernel<4, 2, 4, 4, 3, false, true>); break;
+    case kTile192x128: TG_GO(tile_ring_kernel<4, 2, 3, 4, 3, false, true>); break;
+    case kTile128x128: TG_GO(tile_ring_kernel<2, 4, 4, 2, 4, false, true>); break;
+    case kTile64x128: TG_GO(tile_ring_kernel<2, 4, 2, 2, 6, false, true>); break;
+    case kTile64x64: TG_GO(tile_split_kernel<8, 4, 4, false, true>); break;
+    default: return -5;
+  }
+#undef TG_GO
+  return (int)hipGetLastError();
 }
 
 // the forms that grouped_gemm.hip takes

@@ -698,11 +698,9 @@ class SideBySide:
                 self.right.alloc_cache(num_blocks, block_size, dtype, num_slots, device))
 
     def __call__(self, h, ctx: StepContext, cache) -> torch.Tensor:
-        if ctx.parts:                        # (each output passes a norm of its own here)
-            ctx = StepContext(ctx.ids, ctx.positions, ctx.slot_mapping, ctx.seg)
         a = self.left(h, ctx, cache[0])
         b = self.right(h, ctx, cache[1])
-        return M.dual_rms_mean(a, b, self.w_left, self.w_right, self.eps, self.scale)
+        return M.dual_rms_mean(a, b, self.w_left, self.w_right, self.eps, self.scale, h.shape[0])
 
 
 class StateSpaceMixer:

@@ -220,9 +220,9 @@ class StackedModel:
         seg = meta.segments
         if seg is None:
             raise ValueError("this model needs the step's row segments (AttnMeta.segments)")
-        # (the norm steps sum parts as they read them; with a token shift, of segments of one row, and not two sublayers' at once)
+        # (the norm steps sum parts as they read them; with a token shift, of segments of one row)
         ctx = StepContext(input_ids, meta.positions, meta.slot_mapping, seg,
-                          parts=self.norm_style != "shared_pre" and (seg.max_rows <= 1 or "prev_h" not in caches.extra))
+                          parts=seg.max_rows <= 1 or "prev_h" not in caches.extra)
         if self.norm_style == "layer_post":
             return self._forward_layer_post(input_ids, meta, ctx, caches)
         if self.norm_style == "shared_pre":

@@ -231,15 +231,23 @@ def linear(x, w, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
 
 def linear_out(x, w, parts: bool, bias: Optional[torch.Tensor] = None):
     """:func:`linear`, a sublayer's last product; with ``parts`` its result may be :class:`ExpertParts`, the product with k cut
-    into parts that the norm step behind adds up: few columns leave a product of few rows half the chip, in long chains."""
-    if parts and _few_rows(x, w) and x.shape[1] <= 16384 and native_mixers().expert_rows_fit(w.shape[0]) and \
-            (bias is None or (bias.dtype == x.dtype and bias.is_contiguous())):
-        n = native_mixers().few_rows_parts(*w.shape)
-        if n > 1:
-            d = torch.empty(x.shape[0] * n, w.shape[0], dtype=torch.float32, device=x.device)
-            native_mixers().few_rows_gemm_parts(d, x, w, bias)
-            return ExpertParts(d, None, None, None)
+    into parts that the norm step behind adds up: few columns leave a product of few rows, or of long sums, half the chip."""
+    n, few = _out_parts(x.shape[0], *w.shape) if parts and x.is_cuda else (1, False)
+    if n > 1 and _piece_rows(x, w) and (bias is None or (bias.dtype == x.dtype and bias.is_contiguous() and bias.shape == w.shape[:1])) \
+            and (few or x.shape[1] <= x.stride(0) <= 0x7fffffff // x.shape[0]):
+        d = torch.empty(x.shape[0] * n, w.shape[0], dtype=torch.float32, device=x.device)
+        (native_mixers().few_rows_gemm_parts if few else native_mixers().tile_gemm_parts)(d, x, w, bias)
+        return ExpertParts(d, None, None, None)
     return linear(x, w, bias)
+
+
+@functools.lru_cache(maxsize=8192)
+def _out_parts(rows: int, n: int, k: int):
+    """(The parts of k of a product whose norm step adds them, whether the kernel of few rows makes them)."""
+    N, few = native_mixers(), rows <= FEW_ROWS
+    if not N.expert_rows_fit(n) or k > (16384 if few else 0x7fffffff // n):
+        return 1, few
+    return (N.few_rows_parts(n, k) if few else N.tile_parts(rows, n, k)), few
 
 
 def linear_pair(x, w, x2, w2):
@@ -391,15 +399,25 @@ def add_rms_norm_rows(residual: torch.Tensor, y: torch.Tensor, wb: Optional[torc
     return ref.add_rms_norm_rows(residual, y, wb, eps, add_vec, next_w, out_dtype, want_cast)
 
 
+def _rows_or_parts(y, rows):
+    """(A norm step's rows or a product's :class:`ExpertParts`, how many a row has)."""
+    if not isinstance(y, ExpertParts):
+        return y, 1
+    if y.wts is not None or y.shared is not None:
+        raise ValueError("a mixture's results where a product's parts are read")
+    return y.d, y.d.shape[0] // rows
+
+
 def add_scaled_rms_norm_rows(residual: torch.Tensor, y1: Optional[torch.Tensor], y2: Optional[torch.Tensor],
                              mult: float, next_w: Optional[torch.Tensor], eps: float, out_dtype):
     """residual (fp32, in place) += mult * (y1 + y2); returns rms_norm(residual) * next_w in
     ``out_dtype`` (None without ``next_w``).  y1 and y2 may be fp32 or bf16 each; y2, or
-    both, may be absent (then only the norm is taken).  The step between the layers of a
+    both, may be absent (then only the norm is taken), or be a product's parts.  The step between the layers of a
     stack whose mixer and feed-forward read one shared norm and are added together."""
     if residual.is_cuda:
         out = torch.empty(residual.shape, dtype=out_dtype, device=residual.device) if next_w is not None else None
-        native_mixers().add_scaled_rms_norm(residual, y1, y2, float(mult), next_w, out, eps)
+        (y1, p1), (y2, p2) = _rows_or_parts(y1, residual.shape[0]), _rows_or_parts(y2, residual.shape[0])
+        native_mixers().add_scaled_rms_norm(residual, y1, y2, float(mult), next_w, out, eps, p1, p2)
         return out
     return ref.add_scaled_rms_norm_rows(residual, y1, y2, mult, next_w, eps, out_dtype)
 
@@ -428,13 +446,14 @@ def add_norm_shift_rows(residual: torch.Tensor, y: Optional[torch.Tensor], wb: O
     return ref.add_norm_shift_rows(residual, y, wb, w, shift, eps, out_dtype, prev_state, seg)
 
 
-def dual_rms_mean(a: torch.Tensor, b: torch.Tensor, wa: torch.Tensor, wb: torch.Tensor, eps: float,
-                  scale: float = 0.5) -> torch.Tensor:
+def dual_rms_mean(a, b, wa: torch.Tensor, wb: torch.Tensor, eps: float, scale: float = 0.5,
+                  rows: Optional[int] = None) -> torch.Tensor:
     """fp32 scale * (rms_norm(a) * wa + rms_norm(b) * wb) of two rows of equal width: the
-    outputs of two mixers that run side by side, each normed on its own."""
-    if a.is_cuda:
-        out = torch.empty(a.shape, dtype=torch.float32, device=a.device)
-        native_mixers().dual_rms_mean(out, a, b, wa, wb, eps, float(scale))
+    outputs of two mixers that run side by side, each normed on its own.  a and b may be a product's parts of ``rows`` rows."""
+    if wa.is_cuda:
+        (a, pa), (b, pb) = _rows_or_parts(a, rows), _rows_or_parts(b, rows)
+        out = torch.empty(a.shape[0] // pa, a.shape[1], dtype=torch.float32, device=a.device)
+        native_mixers().dual_rms_mean(out, a, b, wa, wb, eps, float(scale), pa, pb)
         return out
     return ref.dual_rms_mean(a, b, wa, wb, eps, scale)
 
