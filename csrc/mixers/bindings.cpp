@@ -10,8 +10,11 @@
 #include <hip/hip_runtime.h>
 
 extern "C" {
-int mx_embed_rows(float* out, const int* ids, const void* table, int bf16, int rows, int width, int vocab,
-                  float scale, const int* positions, const float* freqs, hipStream_t s);
+int mx_embed_norm_fits(int width);
+int mx_embed_norm(float* x, const int* ids, const void* table, int bf16, int rows, int width, int vocab, float scale,
+                  const int* positions, const float* freqs, const void* pairs, long mul_prev, long mul_cur, int buckets,
+                  const int* start, const int* pos0, const int* slot, int num_segs, int* last_tok, int num_slots, int norm,
+                  void* out, int out_bf16, const float* w, const float* b, float eps, hipStream_t s);
 int mx_layer_norm(float* x, const void* y, int y_bf16, long y_stride, const float* w, const float* b, void* out,
                   void* cast, int out_bf16, const float* next_w, const float* next_b, int rows, int width, float eps, hipStream_t s);
 int mx_tanh_cap(float* x, long n, float cap, hipStream_t s);
@@ -120,7 +123,7 @@ int mx_gla_scan(float* o, const void* qkv, int bf16, long qkv_stride, const void
                 int num_segs, int max_rows, int heads, int dk, int dv, int num_slots, int skip_from, hipStream_t s);
 int mx_pair_embed_add(float* x, const int* ids, const void* table, int bf16, int rows, int width, long mul_prev,
                       long mul_cur, int buckets, const int* start, const int* pos0, const int* slot, int num_segs,
-                      int* last_tok, int num_slots, const void* embed, int vocab, float scale, hipStream_t s);
+                      int* last_tok, int num_slots, hipStream_t s);
 int mx_add_scaled_rms_norm(float* x, const void* y1, int y1_bf16, long y1_stride, int y1_parts, const void* y2, int y2_bf16,
                            long y2_stride, int y2_parts, float mult, const float* next_w, void* out, int out_bf16, int rows,
                            int width, float eps, hipStream_t s);
@@ -315,23 +318,43 @@ RopeArg rope_arg(const OptT& table, int64_t rot_dims, int64_t head_dim) {
   return r;
 }
 
-void embed_rows(Tensor out, Tensor ids, Tensor table, double scale, OptT positions, OptT freqs) {
-  check_f32(out, "out");
+// pairs: {table, start, pos0, slot, last_tok} and (mul_prev, mul_cur, buckets, segments), or empty; norm 0 none, 1 rms (w), 2 layer (w, b)
+void embed_norm(Tensor x, Tensor ids, Tensor table, double scale, OptT positions, OptT freqs, std::vector<Tensor> pairs,
+                std::vector<int64_t> hash, int64_t norm, OptT out, OptT w, OptT b, double eps) {
+  check_f32(x, "x");
   check_i32(ids, "ids");
   TORCH_CHECK(table.is_cuda() && is_act(table) && table.is_contiguous() && table.dim() == 2, "table");
-  TORCH_CHECK(out.dim() == 2 && out.size(0) == ids.numel() && out.size(1) == table.size(1), "out shape");
+  TORCH_CHECK(x.dim() == 2 && x.size(0) == ids.numel() && x.size(1) == table.size(1), "embedded rows' shape");
+  const int64_t width = x.size(1);
   const int* pp = nullptr;
   const float* fp = nullptr;
   if (freqs) {
     TORCH_CHECK(positions, "positions go with the sinusoid frequencies");
     check_i32(*positions, "positions");
     check_f32(*freqs, "sinusoid frequencies");
-    TORCH_CHECK(positions->numel() >= ids.numel() && freqs->numel() * 2 >= table.size(1), "positions / frequencies size");
+    TORCH_CHECK(positions->numel() >= ids.numel() && freqs->numel() * 2 >= width, "positions / frequencies size");
     pp = positions->data_ptr<int>();
     fp = freqs->data_ptr<float>();
   }
-  chk(mx_embed_rows(out.data_ptr<float>(), ids.data_ptr<int>(), table.data_ptr(), bf(table), (int)ids.numel(),
-                    (int)table.size(1), (int)table.size(0), (float)scale, pp, fp, stream()), "embed_rows");
+  const bool paired = !pairs.empty();
+  if (paired) {
+    TORCH_CHECK(pairs.size() == 5 && hash.size() == 4, "pair table");
+    TORCH_CHECK(pairs[0].is_cuda() && pairs[0].is_contiguous() && pairs[0].dim() == 2 && pairs[0].size(1) == width &&
+                pairs[0].scalar_type() == table.scalar_type() && hash[2] >= 1 && pairs[0].size(0) == hash[2] + 1 && hash[0] >= 0 &&
+                hash[1] >= 0, "pair table shapes");
+    check_segs(pairs[1], pairs[2], pairs[3], hash[3]);
+    check_i32(pairs[4], "last tokens");
+  }
+  TORCH_CHECK(norm >= 0 && norm <= 2 && (norm != 1 || out) && (norm != 0 || !out) && (norm > 0) == (bool)w && (norm == 2) == (bool)b,
+              "embed_norm's norm");
+  TORCH_CHECK(!out || (out->is_cuda() && out->is_contiguous() && is_act(*out) && out->sizes() == x.sizes()), "out");
+  chk(mx_embed_norm(x.data_ptr<float>(), ids.data_ptr<int>(), table.data_ptr(), bf(table), (int)ids.numel(), (int)width,
+                    (int)table.size(0), (float)scale, pp, fp, paired ? pairs[0].data_ptr() : nullptr, paired ? (long)hash[0] : 0,
+                    paired ? (long)hash[1] : 0, paired ? (int)hash[2] : 0, paired ? pairs[1].data_ptr<int>() : nullptr,
+                    paired ? pairs[2].data_ptr<int>() : nullptr, paired ? pairs[3].data_ptr<int>() : nullptr, paired ? (int)hash[3] : 0,
+                    paired ? pairs[4].data_ptr<int>() : nullptr, paired ? (int)pairs[4].numel() : 0, (int)norm,
+                    out ? out->data_ptr() : nullptr, out ? bf(*out) : 0, opt_f32(w, width, "norm weight"),
+                    opt_f32(b, width, "norm bias"), (float)eps, stream()), "embed_norm");
 }
 
 // x (fp32 residual) with y: x += ln(y), cast = x; without y: out = ln(x), or, without out, x = ln(x), cast = x
@@ -786,12 +809,8 @@ void row_step(int64_t kind, Tensor out, Tensor x, Tensor a, OptT b, Tensor gate,
 }
 
 void pair_embed_add(Tensor x, Tensor ids, Tensor table, int64_t mul_prev, int64_t mul_cur, int64_t buckets,
-                    Tensor start, Tensor pos0, Tensor slot, int64_t num_segs, Tensor last_tok, OptT embed,
-                    double scale) {
+                    Tensor start, Tensor pos0, Tensor slot, int64_t num_segs, Tensor last_tok) {
   check_f32(x, "residual");
-  if (embed)
-    TORCH_CHECK(embed->is_cuda() && embed->is_contiguous() && embed->dim() == 2 && embed->size(1) == x.size(1) &&
-                embed->scalar_type() == table.scalar_type(), "embedding table");
   check_i32(ids, "ids");
   check_i32(last_tok, "last tokens");
   TORCH_CHECK(table.is_cuda() && is_act(table) && table.is_contiguous() && table.dim() == 2, "table");
@@ -801,8 +820,7 @@ void pair_embed_add(Tensor x, Tensor ids, Tensor table, int64_t mul_prev, int64_
   chk(mx_pair_embed_add(x.data_ptr<float>(), ids.data_ptr<int>(), table.data_ptr(), bf(table), (int)ids.numel(),
                         (int)table.size(1), (long)mul_prev, (long)mul_cur, (int)buckets, start.data_ptr<int>(),
                         pos0.data_ptr<int>(), slot.data_ptr<int>(), (int)num_segs, last_tok.data_ptr<int>(),
-                        (int)last_tok.numel(), embed ? embed->data_ptr() : nullptr, embed ? (int)embed->size(0) : 0,
-                        (float)scale, stream()), "pair_embed_add");
+                        (int)last_tok.numel(), stream()), "pair_embed_add");
 }
 
 // rows [rows, width], or with parts > 1 fp32 [rows * parts, width]
@@ -1894,7 +1912,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("head_tiles_fits", &head_tiles_fits);
   m.def("latent_q_absorb", &latent_q_absorb);
   m.def("head_values", &head_values);
-  m.def("embed_rows", &embed_rows);
+  m.def("embed_norm", &embed_norm);
+  m.def("embed_norm_fits", [](int64_t width) { return mx_embed_norm_fits((int)width) != 0; });
   m.def("add_rms_norm", &add_rms_norm);
   m.def("layer_norm", &layer_norm);
   m.def("tanh_cap", &tanh_cap);

@@ -36,19 +36,35 @@ __device__ __forceinline__ float ldx(const void* p, int bf16, long i) {
   return bf16 ? ft::bf16_to_f32(((const bf16_t*)p)[i]) : ((const float*)p)[i];
 }
 
-// x (fp32 residual) = embed[cur] * scale + table[hash] per row (without `embed`: x +=
-// table[hash]), hash = (prev * mul_prev + cur * mul_cur) mod
-// buckets with prev the token before the row's own in its sequence: the row above within a
-// segment, last_tok[slot] for a segment's first row (pos0 > 0), and for a sequence's first
-// token row `buckets` instead.  One workgroup per row; pair_last_kernel stores each
-// segment's last token afterwards (a second launch: another row of the segment may still
-// be reading the old one).
+// What a row adds from the table of token pairs: entry hash = (prev * mul_prev + cur * mul_cur) mod buckets, prev the token
+// before the row's own in its sequence: the row above within a segment, last_tok[slot] for a segment's first row (pos0 > 0),
+// and for a sequence's first token entry `buckets` instead.  That first row's workgroup, the only reader of the slot, then
+// leaves the segment's last token there.  -1: none (padding rows).  Every thread of a workgroup calls it.
+struct PairArgs {
+  const void* table;                          // null: no pairs
+  long mul_prev, mul_cur;
+  int buckets, num_segs, num_slots;
+  const int *start, *pos0, *slot;
+  int* last_tok;
+};
+__device__ __forceinline__ long pair_entry(const PairArgs& P, const int* __restrict__ ids, int row) {
+  if (row >= P.start[P.num_segs]) return -1;
+  const int sg = segment_of(P.start, P.num_segs, row), first = P.start[sg], end = P.start[sg + 1], sl = P.slot[sg];
+  if (sl < 0 || sl >= P.num_slots) return -1;
+  long prev = row > first ? ids[row - 1] : P.pos0[sg] > 0 ? P.last_tok[sl] : -1;
+  if (row == first) {
+    __syncthreads();                          // (all have read it)
+    if (threadIdx.x == 0) P.last_tok[sl] = ids[end - 1];
+  }
+  if (prev < 0) return P.buckets;
+  long idx = (prev * P.mul_prev + (long)ids[row] * P.mul_cur) % P.buckets;
+  return idx < 0 ? idx + P.buckets : idx;
+}
+
+// x (fp32 residual) = embed[cur] * scale + table[hash] per row (without `embed`: x += table[hash]).  One workgroup per row.
 template <typename T>
-__global__ void pair_embed_add_kernel(float* __restrict__ x, const int* __restrict__ ids,
-                                      const T* __restrict__ table, int width, long mul_prev, long mul_cur,
-                                      int buckets, const int* __restrict__ start, const int* __restrict__ pos0,
-                                      const int* __restrict__ slot, int num_segs, const int* __restrict__ last_tok,
-                                      int num_slots, const T* __restrict__ embed, int vocab, float scale) {
+__global__ void pair_embed_add_kernel(float* __restrict__ x, const int* __restrict__ ids, PairArgs P, int width,
+                                      const T* __restrict__ embed, int vocab, float scale) {
   const int row = blockIdx.x;
   if (embed != nullptr) {                 // every row gets its embedding row, padding rows too
     int id = ids[row];
@@ -56,35 +72,9 @@ __global__ void pair_embed_add_kernel(float* __restrict__ x, const int* __restri
     for (int i = threadIdx.x; i < width; i += blockDim.x)
       x[(long)row * width + i] = ld(embed, (long)id * width + i) * scale;
   }
-  if (row >= start[num_segs]) return;
-  int lo_s = 0, hi_s = num_segs;
-  while (hi_s - lo_s > 1) {
-    const int mid = (lo_s + hi_s) >> 1;
-    if (start[mid] <= row) lo_s = mid; else hi_s = mid;
-  }
-  const int sg = lo_s;
-  const int sl = slot[sg];
-  if (sl < 0 || sl >= num_slots) return;
-  long prev;
-  if (row > start[sg]) prev = ids[row - 1];
-  else prev = pos0[sg] > 0 ? last_tok[sl] : -1;
-  long idx = buckets;
-  if (prev >= 0) {
-    idx = (prev * mul_prev + (long)ids[row] * mul_cur) % buckets;
-    if (idx < 0) idx += buckets;
-  }
-  for (int i = threadIdx.x; i < width; i += blockDim.x) x[(long)row * width + i] += ld(table, idx * width + i);
-}
-
-__global__ void pair_last_kernel(const int* __restrict__ ids, const int* __restrict__ start,
-                                 const int* __restrict__ slot, int num_segs, int* __restrict__ last_tok,
-                                 int num_slots) {
-  const int sg = blockIdx.x * blockDim.x + threadIdx.x;
-  if (sg >= num_segs) return;
-  const int sl = slot[sg];
-  const int a = start[sg], b = start[sg + 1];
-  if (sl < 0 || sl >= num_slots || b <= a) return;
-  last_tok[sl] = ids[b - 1];
+  const long idx = pair_entry(P, ids, row);
+  if (idx < 0) return;
+  for (int i = threadIdx.x; i < width; i += blockDim.x) x[(long)row * width + i] += ld((const T*)P.table, idx * width + i);
 }
 
 // residual (fp32, in place): x += mult * (y1 + y2);  out = rms_norm(x) * next_w (TO).
@@ -422,6 +412,84 @@ dual_rms_mean_row_kernel(float* __restrict__ out, AnyRows a, AnyRows b, const fl
 #pragma unroll
     for (int k = 0; k < 4; ++k) u[c][k] = scale * (u[c][k] * ra * p[c][k] + v[c][k] * rb * q[c][k]);
   store_row<float, NT, C>(out + row * width, u, width, vec);
+}
+
+// A step's first rows and the norm that reads them, in one launch: x = embed[id] * scale (+ the position's sines and
+// cosines) (+ the row of the pair), then out = rms_norm(x) * w (NORM 1), or x = layer_norm(x) * w + b, out = x (NORM 2),
+// or nothing (0).  A row in registers, as the kernels below: all of an embedding row's reads in flight at once, and a sine and
+// a cosine share their angle's reduction.  Bound by the chain of id, row and sums for few rows, by the rows' bytes for many.
+// In running models, us beside embedding, pairs' last tokens and norm in launches of their own: 1 row 4.4 (8.6), 16 with pairs
+// 7.0 (19), 32 with positions 5.6 (16), 2048 10.8 (17.7).
+struct EmbedArgs {
+  const int* ids;
+  const void* table;
+  int vocab;
+  float scale;
+  const int* positions;                       // with freqs
+  const float* freqs;
+};
+template <typename T, typename TO, int NT, int C, int NORM>
+__global__ void __launch_bounds__(NT)
+embed_norm_kernel(EmbedArgs E, PairArgs P, float* __restrict__ x, TO* __restrict__ out, const float* __restrict__ w,
+                  const float* __restrict__ b, int width, float eps) {
+  __shared__ float red[NT / 64];
+  const int row = blockIdx.x;
+  int id = E.ids[row];
+  if (id < 0 || id >= E.vocab) id = 0;
+  float v[C][4], t[C][4], wv[C][4], bv[C][4];
+  load_row<T, NT, C>(v, (const T*)E.table + (long)id * width, width, 1);
+  if constexpr (NORM > 0) load_row<float, NT, C>(wv, w, width, 1);
+  if constexpr (NORM == 2) load_row<float, NT, C>(bv, b, width, 1);
+  long pair = -1;
+  if (P.table != nullptr) pair = pair_entry(P, E.ids, row);
+  if (pair >= 0) load_row<T, NT, C>(t, (const T*)P.table + pair * width, width, 1);
+  const float p = E.freqs != nullptr ? (float)E.positions[row] : 0.f;
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    const int i = (c * NT + threadIdx.x) * 4;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[c][k] *= E.scale;
+    if (E.freqs != nullptr && i < width) {
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        float sn, cs;
+        sincosf(p * E.freqs[i / 2 + k], &sn, &cs);
+        v[c][2 * k] += sn;
+        v[c][2 * k + 1] += cs;
+      }
+    }
+    if (pair >= 0)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) v[c][k] += t[c][k];
+  }
+  if constexpr (NORM < 2) store_row<float, NT, C>(x + (long)row * width, v, width, 1);
+  if constexpr (NORM == 1) {
+    const float r = 1.0f / sqrtf(block_sum<NT>(sum_sq<C>(v), red) / (float)width + eps);
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) v[c][k] *= r * wv[c][k];
+  } else if constexpr (NORM == 2) {
+    float sum = 0.f, ss = 0.f;
+#pragma unroll
+    for (int c = 0; c < C; ++c) sum += (v[c][0] + v[c][1]) + (v[c][2] + v[c][3]);
+    const float mean = block_sum<NT>(sum, red) / (float)width;
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        v[c][k] = (c * NT + (int)threadIdx.x) * 4 + k < width ? v[c][k] - mean : 0.f;
+        ss += v[c][k] * v[c][k];
+      }
+    const float r = 1.0f / sqrtf(block_sum<NT>(ss, red) / (float)width + eps);
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) v[c][k] = v[c][k] * r * wv[c][k] + bv[c][k];
+    store_row<float, NT, C>(x + (long)row * width, v, width, 1);
+  }
+  if constexpr (NORM > 0)
+    if (out != nullptr) store_row<TO, NT, C>(out + (long)row * width, v, width, 1);
 }
 
 // residual (fp32, in place): x += rms_norm(y) * wb (y as it is without wb) (+ add_vec);
@@ -799,16 +867,6 @@ __global__ void scale_add_rows_kernel(float* __restrict__ out, const TY* __restr
 
 using namespace mx;
 
-extern "C" int mx_embed_rows(float* out, const int* ids, const void* table, int bf16, int rows,
-                             int width, int vocab, float scale, const int* positions, const float* freqs,
-                             hipStream_t s) {
-  if (rows <= 0) return 0;
-  if (freqs != nullptr && positions == nullptr) return -1;
-  MX_DISPATCH_T(bf16, hipLaunchKernelGGL((embed_rows_kernel<T>), dim3(rows), dim3(256), 0, s, out, ids,
-                                         (const T*)table, width, vocab, scale, positions, freqs));
-  return (int)hipGetLastError();
-}
-
 constexpr int kRowThreads = 512;
 constexpr int kRowMaxWidth = kRowThreads * 4 * 8;
 
@@ -820,6 +878,46 @@ static void row_chunks(int width, F f) {
   else if (chunks <= 2) f(std::integral_constant<int, 2>{});
   else if (chunks <= 4) f(std::integral_constant<int, 4>{});
   else f(std::integral_constant<int, 8>{});
+}
+
+// x = embed[id] * scale (+ positions) (+ pairs), then the norm: 0 none, 1 out = rms_norm(x) * w, 2 x = layer_norm(x) * w + b and
+// out (if any) = x; rows that are no whole fours or too wide: only without a norm
+extern "C" int mx_embed_norm_fits(int width) { return width % 4 == 0 && width <= kRowMaxWidth; }
+extern "C" int mx_embed_norm(float* x, const int* ids, const void* table, int bf16, int rows, int width, int vocab, float scale,
+                             const int* positions, const float* freqs, const void* pairs, long mul_prev, long mul_cur, int buckets,
+                             const int* start, const int* pos0, const int* slot, int num_segs, int* last_tok, int num_slots,
+                             int norm, void* out, int out_bf16, const float* w, const float* b, float eps, hipStream_t s) {
+  if (rows <= 0) return 0;
+  if ((freqs != nullptr && positions == nullptr) || norm < 0 || norm > 2 || (pairs != nullptr && buckets < 1)) return -1;
+  if (num_segs < 1) pairs = nullptr;          // (padding rows only)
+  const PairArgs P{pairs, mul_prev, mul_cur, buckets, num_segs, num_slots, start, pos0, slot, last_tok};
+  const int vec = mx_embed_norm_fits(width) && ((uintptr_t)table | (uintptr_t)pairs) % (bf16 ? 8 : 16) == 0 &&
+                  ((uintptr_t)x | (uintptr_t)w | (uintptr_t)b) % 16 == 0 && ((uintptr_t)out) % (out_bf16 ? 8 : 16) == 0;
+  if (!vec) {
+    if (norm != 0) return -2;
+    if (pairs != nullptr && freqs != nullptr) return -3;
+    if (pairs != nullptr) {
+      MX_DISPATCH_T(bf16, hipLaunchKernelGGL((pair_embed_add_kernel<T>), dim3(rows), dim3(256), 0, s, x, ids, P, width,
+                                             (const T*)table, vocab, scale));
+    } else {
+      MX_DISPATCH_T(bf16, hipLaunchKernelGGL((embed_rows_kernel<T>), dim3(rows), dim3(256), 0, s, x, ids, (const T*)table, width,
+                                             vocab, scale, positions, freqs));
+    }
+    return (int)hipGetLastError();
+  }
+  const EmbedArgs E{ids, table, vocab, scale, positions, freqs};
+#define MX_EN(TO, NORM)                                                                                                    \
+  MX_DISPATCH_T(bf16, hipLaunchKernelGGL((embed_norm_kernel<T, TO, kRowThreads, decltype(c)::value, NORM>), dim3(rows),    \
+                                         dim3(kRowThreads), 0, s, E, P, x, (TO*)out, w, b, width, eps))
+  row_chunks(width, [&](auto c) {
+    if (norm == 0) MX_EN(float, 0);
+    else if (norm == 1 && out_bf16) MX_EN(bf16_t, 1);
+    else if (norm == 1) MX_EN(float, 1);
+    else if (out_bf16) MX_EN(bf16_t, 2);
+    else MX_EN(float, 2);
+  });
+#undef MX_EN
+  return (int)hipGetLastError();
 }
 
 // whether these rows go to the kernels that hold a row in registers (layer norm, scaled add, mean of two norms), 512 threads a
@@ -1095,17 +1193,15 @@ extern "C" int mx_scale_add_rows(float* out, const void* y, int y_bf16, const in
   return (int)hipGetLastError();
 }
 
+// x (fp32 residual) += table[hash]
 extern "C" int mx_pair_embed_add(float* x, const int* ids, const void* table, int bf16, int rows, int width,
                                  long mul_prev, long mul_cur, int buckets, const int* start, const int* pos0,
-                                 const int* slot, int num_segs, int* last_tok, int num_slots, const void* embed,
-                                 int vocab, float scale, hipStream_t s) {
+                                 const int* slot, int num_segs, int* last_tok, int num_slots, hipStream_t s) {
   if (rows <= 0 || num_segs <= 0) return 0;
   if (buckets < 1 || width < 1) return -1;
-  MX_DISPATCH_T(bf16, hipLaunchKernelGGL((pair_embed_add_kernel<T>), dim3(rows), dim3(256), 0, s, x, ids,
-                                         (const T*)table, width, mul_prev, mul_cur, buckets, start, pos0, slot,
-                                         num_segs, last_tok, num_slots, (const T*)embed, vocab, scale));
-  hipLaunchKernelGGL(pair_last_kernel, dim3((num_segs + 63) / 64), dim3(64), 0, s, ids, start, slot, num_segs, last_tok,
-                     num_slots);
+  const PairArgs P{table, mul_prev, mul_cur, buckets, num_segs, num_slots, start, pos0, slot, last_tok};
+  MX_DISPATCH_T(bf16, hipLaunchKernelGGL((pair_embed_add_kernel<T>), dim3(rows), dim3(256), 0, s, x, ids, P, width,
+                                         (const T*)nullptr, 0, 1.f));
   return (int)hipGetLastError();
 }
 

@@ -227,11 +227,11 @@ class StackedModel:
             return self._forward_layer_post(input_ids, meta, ctx, caches)
         if self.norm_style == "shared_pre":
             return self._forward_shared_pre(input_ids, meta, ctx, caches)
-        x = self._embed(input_ids, ctx, caches)
+        nruns = len(self.runs)
+        first = self.layers[self.runs[0][0]] if nruns and self.runs[0][1] is None else None
+        x, h = self._embed(input_ids, ctx, caches, first.norm1 if first is not None and first.shift is None else None)
         tap = self.layer_tap
         fuse_step = tap is None
-        h = None
-        nruns = len(self.runs)
         mark = self.mark_at
         prev_h = caches.extra.get("prev_h")
         every = meta.logits_indices.numel() == x.shape[0]      # the final norm rides in the last layer's last add
@@ -306,13 +306,10 @@ class StackedModel:
             h, _ = M.add_rms_norm_rows(x, y, wb, eps, next_w=w, out_dtype=dt)
         return ff(h, ctx)
 
-    def _embed(self, input_ids, ctx, caches: StackedCache) -> torch.Tensor:
-        """fp32 residual rows: embedding table, plus the pair table's rows if there is one."""
-        if self.pair_embed is None:
-            return M.embed_rows(input_ids, self.embed, self.embed_scale)
-        table, mul_prev, mul_cur, buckets = self.pair_embed
-        return M.pair_embed_rows(input_ids, self.embed, self.embed_scale, table, mul_prev, mul_cur, buckets, ctx.seg,
-                                 caches.extra["last_token"])
+    def _embed(self, input_ids, ctx, caches: StackedCache, norm: Optional[torch.Tensor]):
+        """(fp32 residual rows: embedding table, plus the pair table's rows if there is one; their RMS norm times ``norm``, if given)."""
+        pair = self.pair_embed and (*self.pair_embed, ctx.seg, caches.extra["last_token"])
+        return M.embed_norm_rows(input_ids, self.embed, self.embed_scale, self.cfg.rms_norm_eps, self.dtype, norm, pair=pair)
 
     def load_pair_table(self, table: torch.Tensor, buckets: int, mul_prev: int, mul_cur: int):
         table = table.to(self.device, self.dtype).contiguous()
@@ -322,9 +319,10 @@ class StackedModel:
 
     def _forward_layer_post(self, input_ids, meta, ctx, caches: StackedCache) -> torch.Tensor:
         dt, eps = self.dtype, self.cfg.rms_norm_eps
-        x = M.embed_rows(input_ids, self.embed, self.embed_scale, meta.positions, self.pos_freqs)
-        h = M.add_layer_norm_rows(x, None, self.embed_norm[0], self.embed_norm[1], eps, dt) \
-            if self.embed_norm is not None else (x if dt == torch.float32 else x.to(dt))
+        x, h = M.embed_norm_rows(input_ids, self.embed, self.embed_scale, eps, dt, *(self.embed_norm or (None, None)),
+                                 meta.positions, self.pos_freqs)
+        if h is None:
+            h = x if dt == torch.float32 else x.to(dt)
         tap, mark = self.layer_tap, self.mark_at
         every, nruns = meta.logits_indices.numel() == x.shape[0], len(self.runs)
         for r, (li, _) in enumerate(self.runs):
@@ -347,11 +345,9 @@ class StackedModel:
 
     def _forward_shared_pre(self, input_ids, meta, ctx, caches: StackedCache) -> torch.Tensor:
         dt, eps, mult = self.dtype, self.cfg.rms_norm_eps, self.residual_mult
-        x = self._embed(input_ids, ctx, caches)
-        tap, mark = self.layer_tap, self.mark_at
         nruns = len(self.runs)
-        h = M.add_scaled_rms_norm_rows(x, None, None, mult, self.layers[self.runs[0][0]].norm1, eps, dt) \
-            if nruns else None
+        x, h = self._embed(input_ids, ctx, caches, self.layers[self.runs[0][0]].norm1 if nruns else None)
+        tap, mark = self.layer_tap, self.mark_at
         every = meta.logits_indices.numel() == x.shape[0]
         for r, (li, _) in enumerate(self.runs):
             if mark is not None and r == mark[0]:

@@ -311,11 +311,38 @@ def embed_rows(ids: torch.Tensor, table: torch.Tensor, scale: float = 1.0,
     :func:`sinusoid_freqs`) a sinusoidal position vector is added: column 2i gets
     sin(p f_i), column 2i+1 cos(p f_i), angles in fp32."""
     if ids.is_cuda:
-        out = torch.empty(ids.shape[0], table.shape[1], dtype=torch.float32, device=ids.device)
-        native_mixers().embed_rows(out, ids, table, float(scale), positions if pos_freqs is not None else None,
-                                   pos_freqs)
-        return out
+        return _embed_norm(ids, table, scale, positions, pos_freqs, None, 0, None, None, None, 0.0)[0]
     return ref.embed_rows(ids, table, scale, positions, pos_freqs)
+
+
+def _embed_norm(ids, table, scale, positions, freqs, pair, norm, w, b, out_dtype, eps):
+    x = torch.empty(ids.shape[0], table.shape[1], dtype=torch.float32, device=ids.device)
+    out = torch.empty(x.shape, dtype=out_dtype, device=ids.device) if out_dtype is not None else None
+    pairs, hashed = [], []
+    if pair is not None:
+        ptable, mul_prev, mul_cur, buckets, seg, last_tok = pair
+        pairs, hashed = [ptable, seg.start, seg.pos0, seg.slot, last_tok], [int(mul_prev), int(mul_cur), int(buckets), seg.num]
+    native_mixers().embed_norm(x, ids, table, float(scale), positions if freqs is not None else None, freqs, pairs, hashed, norm, out,
+                               w, b, float(eps))
+    return x, out
+
+
+def embed_norm_rows(ids: torch.Tensor, table: torch.Tensor, scale: float, eps: float, out_dtype, w: Optional[torch.Tensor] = None,
+                    b: Optional[torch.Tensor] = None, positions: Optional[torch.Tensor] = None,
+                    pos_freqs: Optional[torch.Tensor] = None, pair: Optional[tuple] = None):
+    """The rows of :func:`embed_rows`, or with ``pair`` (table, mul_prev, mul_cur, buckets, segments, last tokens) of
+    :func:`pair_embed_rows`, and what the first sublayer reads of them, one launch where a row is whole fours: (x, rms_norm(x) * w
+    in ``out_dtype``) with ``w``; with ``b`` as well x itself is layer_norm(x) * w + b and comes in ``out_dtype`` beside it."""
+    width = table.shape[1]
+    if ids.is_cuda and w is not None and native_mixers().embed_norm_fits(width) and \
+            all(t is None or t.data_ptr() % 16 == 0 for t in (table, w, b, None if pair is None else pair[0])):
+        own = b is not None and out_dtype == torch.float32                    # (the residual itself)
+        x, h = _embed_norm(ids, table, scale, positions, pos_freqs, pair, 1 if b is None else 2, w, b, None if own else out_dtype, eps)
+        return x, x if own else h
+    x = embed_rows(ids, table, scale, positions, pos_freqs) if pair is None else pair_embed_rows(ids, table, scale, *pair)
+    if w is None:
+        return x, None
+    return x, rms_norm_rows(x, w, eps, out_dtype) if b is None else add_layer_norm_rows(x, None, w, b, eps, out_dtype)
 
 
 sinusoid_freqs = ref.sinusoid_freqs
@@ -480,7 +507,7 @@ def pair_embed_add(x: torch.Tensor, ids: torch.Tensor, table: torch.Tensor, mul_
     token."""
     if x.is_cuda:
         native_mixers().pair_embed_add(x, ids, table, int(mul_prev), int(mul_cur), int(buckets), seg.start,
-                                       seg.pos0, seg.slot, seg.num, last_tok, None, 1.0)
+                                       seg.pos0, seg.slot, seg.num, last_tok)
         return x
     return ref.pair_embed_add(x, ids, table, mul_prev, mul_cur, buckets, seg, last_tok)
 
@@ -490,10 +517,7 @@ def pair_embed_rows(ids: torch.Tensor, embed: torch.Tensor, scale: float, table:
     """:func:`embed_rows` and :func:`pair_embed_add` in one launch: fp32 rows
     embed[ids] * scale + table[hash(previous token, token)]."""
     if ids.is_cuda:
-        x = torch.empty(ids.shape[0], embed.shape[1], dtype=torch.float32, device=ids.device)
-        native_mixers().pair_embed_add(x, ids, table, int(mul_prev), int(mul_cur), int(buckets), seg.start,
-                                       seg.pos0, seg.slot, seg.num, last_tok, embed, float(scale))
-        return x
+        return _embed_norm(ids, embed, scale, None, None, (table, mul_prev, mul_cur, buckets, seg, last_tok), 0, None, None, None, 0.0)[0]
     return ref.pair_embed_add(ref.embed_rows(ids, embed, scale), ids, table, mul_prev, mul_cur, buckets, seg, last_tok)
 
 
