@@ -148,15 +148,25 @@ __device__ __forceinline__ void split_any_bf16x3(float a, float b, uint32_t& hi,
 // question asked: a branch between this and the short form has the entries waited for behind the keys' loads, a decode
 // row of 540 keys 19 to 20 us, 18.3 so and with the short form alone.)
 template <int KS>
-__device__ __forceinline__ void split_queries(const float* src, uint4 (&part)[3][KS]) {
+__device__ __forceinline__ void split_queries(const float4 (&src)[KS][2], uint4 (&part)[3][KS]) {
 #pragma unroll
   for (int s = 0; s < KS; ++s) {
-    const float4 u = *reinterpret_cast<const float4*>(src + 32 * s), v = *reinterpret_cast<const float4*>(src + 32 * s + 4);
+    const float4 u = src[s][0], v = src[s][1];
     split_any_bf16x3(u.x, u.y, part[0][s].x, part[1][s].x, part[2][s].x);
     split_any_bf16x3(u.z, u.w, part[0][s].y, part[1][s].y, part[2][s].y);
     split_any_bf16x3(v.x, v.y, part[0][s].z, part[1][s].z, part[2][s].z);
     split_any_bf16x3(v.z, v.w, part[0][s].w, part[1][s].w, part[2][s].w);
   }
+}
+
+template <int KS>
+__device__ __forceinline__ void split_queries(const float* src, uint4 (&part)[3][KS]) {
+  float4 raw[KS][2];
+#pragma unroll
+  for (int s = 0; s < KS; ++s)
+#pragma unroll
+    for (int y = 0; y < 2; ++y) raw[s][y] = *reinterpret_cast<const float4*>(src + 32 * s + 4 * y);
+  split_queries<KS>(raw, part);
 }
 
 // a wave's own LDS writes, to be read by its other lanes

@@ -9,11 +9,13 @@
 // S^T = K Q^T and O^T = V^T P^T, a column per head: keys go straight from memory to operands, values through a wave's
 // own LDS strip (ds_read_b64_tr_b16), and weights need no exchange.  The next 32 keys load under the softmax and the
 // sums.  The waves' (maximum, sum, sums) meet in LDS at the end: one launch, whatever the length.
-// Bound by a wave's chain for few rows, by the read of the keys for many.  In running models, 16 heads of 128 on 4
-// key heads: one row, 900 keys in a block of 1024 or with a table 25 us (general kernel, a workgroup per head: 50),
-// 540 keys with sigmoid weights 18 (33), two maps of 64 16 (33); 32 rows of 540 24 (56).  With the keys in the L2 a row takes
-// 7.7 to 9.3 us however few they are (general kernel: 6 to 7 with one, 10 with a hundred), and one query head a key head
-// wastes fifteen columns of sixteen: 64 rows of 16 such heads 18 us at 100 keys (20), 162 at 1500 (228), 600 at 6000 (823).
+// Bound by the vector units for few rows (a step of 32 keys is 700 instructions of a wave beside 48 products, two waves a unit),
+// by the read of the keys for many: so terms that a row has not are skipped for all of its keys at once, whole steps ask for no
+// key's presence, and blocks of a power of two are shifted.  us in a graph at 30 / 300 / 540 / 1024 keys, 16 heads of 128 on 4 key
+// heads: one row 7.4 11 13 18, 64 rows 8.2 16 23 33; two maps of 64, one row 6.9 9.9 11 14 (a look at every term and key by
+// itself: 8.1 13 16 23, 8.6 18 25 36 and 7.3 12 14 19; general kernel, a workgroup per head: 50 a row of 900).  Two steps of keys
+// on their way were no sooner.  One query head a key head wastes fifteen columns of sixteen: 64 rows of 16 such heads 10 us at 30
+// keys, 61 at 540, 328 at 3300.  Lengths are not known on the host where a step is replayed, so sizes alone choose.
 // (Eight waves for all of them and a merge that read every wave's part, an entry a thread: 32 at 100 keys; 16 heads a
 // group, one key: 12.4, now 9.3.)  Lengths are not known on the host where a step is replayed, so sizes alone choose.
 #include "mx_common.h"
@@ -44,7 +46,7 @@ struct WindowArgs {
   const float* sinks;
   int blocks, keep_first;
   const float* dist_bias;
-  int nd;
+  int nd, block_shift;                        // block_size as a power of two, or -1
 };
 
 __device__ __forceinline__ wd_f32x4 wd_mfma(const uint4& a, const uint4& b, wd_f32x4 c) {
@@ -53,6 +55,14 @@ __device__ __forceinline__ wd_f32x4 wd_mfma(const uint4& a, const uint4& b, wd_f
 }
 
 constexpr int kWdKeys = 32, kWdMaxRep = 16;
+
+// e^x, x <= 0: 2^(x log2 e) with the rounding of that product, and of log2 e, in a first-order term; a unit in the last place or so
+__device__ __forceinline__ float wd_exp(float x) {
+  constexpr float kLog2e = 1.44269504f, kLow = 1.92596299e-8f, kLn2 = 0.693147181f;   // (kLow: log2 e - kLog2e)
+  x = fmaxf(x, -160.f);                       // (there 0 already)
+  const float t = x * kLog2e, low = fmaf(x, kLow, fmaf(x, kLog2e, -t)), e = __builtin_amdgcn_exp2f(t);
+  return fmaf(e * low, kLn2, e);
+}
 
 template <int DK, int DV, int WV>
 __global__ void __launch_bounds__(64 * WV, 2)
@@ -77,46 +87,54 @@ window_decode_kernel(WindowArgs A) {
   const int nkeys = ext + max(0, last - first + 1);
   const int* table = A.bt + (long)s * A.bt_stride;
 
-  auto slot_of = [&](int c) {                  // of the c-th key the row sees (none: -1)
-    if (c >= nkeys) return -1;
-    const int j = c < ext ? c : first + c - ext, blk = table[j / A.block_size];
-    return blk >= 0 && blk < A.num_blocks ? blk * A.block_size + j % A.block_size : -1;
-  };
+  // No load of the keys' loop stands behind a branch or is looked at before the next step: the loads come back in order, so
+  // a table entry whose range was checked at once waited for the keys asked for before it, twice a step (22.7 us a row of 1024
+  // keys, 21.2 so).  Keys that there are not read slot 0 and count for nothing.
   uint4 k[2][KS], v[VL];
   constexpr int kStep = WV * kWdKeys;
-  auto look = [&](int c0, int (&slot)[2]) {    // lane n of each group: keys n and 16 + n
+  int slot[2], vslot[VL], blk[2], off[2];      // this step's slots (none: -1), the next one's table entries and places in them
+  auto look = [&](int c0) {                    // lane n of each group: keys n and 16 + n
 #pragma unroll
-    for (int t = 0; t < 2; ++t) slot[t] = slot_of(c0 + 16 * t + n);
-  };
-  auto fetch = [&](const int (&slot)[2]) {
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int x = 0; x < KS; ++x) {
-        k[t][x] = uint4{0, 0, 0, 0};
-        if (slot[t] >= 0) k[t][x] = *reinterpret_cast<const uint4*>(A.kc + slot[t] * nk + (long)gk * DK + 32 * x + 8 * g4);
-      }
-#pragma unroll
-    for (int x = 0; x < VL; ++x) {
-      const int key = (64 * x + lane) / PV, s0 = __shfl(slot[0], key & 15), s1 = __shfl(slot[1], key & 15);
-      const int sl = key < 16 ? s0 : s1;
-      v[x] = uint4{0, 0, 0, 0};
-      if (sl >= 0) v[x] = *reinterpret_cast<const uint4*>(A.vc + sl * nv + (long)kvh * DV + (lane % PV) * 8);
+    for (int t = 0; t < 2; ++t) {
+      const int c = c0 + 16 * t + n, in = min(c, nkeys - 1), j = in < ext ? in : first + in - ext;
+      const int b = A.block_shift >= 0 ? j >> A.block_shift : j / A.block_size;
+      blk[t] = table[b];
+      off[t] = c < nkeys ? j - b * A.block_size : -1;
     }
   };
-  // slots are looked up two steps ahead of their use, so that no load waits for a table entry
-  int slot[2], next[2];
-  look(wave * kWdKeys, slot);
-  look(wave * kWdKeys + kStep, next);
-  fetch(slot);
-
-  // the queries' parts, as right operands: head n, elements 32 x + 8 g4 .. + 7
-  uint4 qp[3][KS];
-  split_queries<KS>(A.q + ((long)row * hq + a) * DK + 8 * g4, qp);
+  auto fetch = [&]() {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      slot[t] = off[t] >= 0 && blk[t] >= 0 && blk[t] < A.num_blocks ? blk[t] * A.block_size + off[t] : -1;
+      const bf16_t* p = A.kc + max(slot[t], 0) * nk + (long)gk * DK + 8 * g4;
+#pragma unroll
+      for (int x = 0; x < KS; ++x) k[t][x] = *reinterpret_cast<const uint4*>(p + 32 * x);
+    }
+#pragma unroll
+    for (int x = 0; x < VL; ++x) {
+      vslot[x] = __shfl(slot[x < VL / 2 ? 0 : 1], ((64 * x + lane) / PV) & 15);
+      v[x] = *reinterpret_cast<const uint4*>(A.vc + max(vslot[x], 0) * nv + (long)kvh * DV + (lane % PV) * 8);
+    }
+  };
+  const float* q = A.q + ((long)row * hq + a) * DK + 8 * g4;
+  float4 raw[KS][2];
+#pragma unroll
+  for (int x = 0; x < KS; ++x)
+#pragma unroll
+    for (int y = 0; y < 2; ++y) raw[x][y] = *reinterpret_cast<const float4*>(q + 32 * x + 4 * y);
   const float c1 = A.r1 != nullptr ? A.r1[a] : 0.f, c2 = A.r1 != nullptr ? A.r2[a] : 0.f;
   const float bias = A.sigmoid && A.pb != nullptr ? A.pb[a] : 0.f;
   const bool sinks = A.has_sink && !A.sigmoid && wave == 0;
   float mx_ = sinks ? (A.sinks != nullptr ? A.sinks[a] : A.sink_all) : -INFINITY, l_ = sinks && g4 == 0 ? 1.f : 0.f;
+  if (nkeys > 0) {
+    look(wave * kWdKeys);
+    fetch();
+    look(wave * kWdKeys + kStep);
+  }
+
+  // the queries' parts, as right operands: head n, elements 32 x + 8 g4 .. + 7
+  uint4 qp[3][KS];
+  split_queries<KS>(raw, qp);
   wd_f32x4 o[DT];                              // columns 16 t + 4 g4 .. of head n
 #pragma unroll
   for (int t = 0; t < DT; ++t) o[t] = wd_f32x4{0.f, 0.f, 0.f, 0.f};
@@ -127,6 +145,12 @@ window_decode_kernel(WindowArgs A) {
 
   for (int c0 = wave * kWdKeys; c0 < nkeys; c0 += kStep) {
     wave_lds_fence();                          // (the last strip has been read)
+    const bool whole = __all(slot[0] >= 0 && slot[1] >= 0);
+    if (!whole) {
+#pragma unroll
+      for (int x = 0; x < VL; ++x)
+        if (vslot[x] < 0) v[x] = uint4{0, 0, 0, 0};
+    }
 #pragma unroll
     for (int x = 0; x < VL; ++x) {
       const int key = (64 * x + lane) / PV;
@@ -161,29 +185,34 @@ window_decode_kernel(WindowArgs A) {
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) has[t][e] = __shfl(slot[t], 4 * g4 + e) >= 0;
-    fetch(next);
+      for (int e = 0; e < 4; ++e) has[t][e] = whole || __shfl(slot[t], 4 * g4 + e) >= 0;
+    fetch();
+    look(c0 + 2 * kStep);
+    auto scores = [&](auto f) {
 #pragma unroll
-    for (int t = 0; t < 2; ++t) slot[t] = next[t];
-    look(c0 + 2 * kStep, next);
-    float top = -INFINITY;
+      for (int t = 0; t < 2; ++t)
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
+        for (int e = 0; e < 4; ++e) sc[t][e] = f(sc[t][e], t, e);
+    };
+    // (a look at each term for all of them: the vector units bound a step, and most rows have none)
+    scores([&](float z, int, int) { return z * A.scale; });
+    if (A.softcap > 0.f) scores([&](float z, int, int) { return A.softcap * tanhf(z / A.softcap); });
+    if (A.r1 != nullptr)
+      scores([&](float z, int t, int e) {
         const int c = c0 + 16 * t + 4 * g4 + e, d = i - (c < ext ? c : first + c - ext);
-        float z = sc[t][e] * A.scale;
-        if (A.softcap > 0.f) z = A.softcap * tanhf(z / A.softcap);
-        if (A.r1 != nullptr) z -= c1 * logf(1.0f + c2 * (float)max(d, 0));
-        if (A.dist_bias != nullptr) z += db[t][e];
-        if (A.sigmoid) z = sigmoidf_(z + bias);
-        if (!has[t][e]) z = A.sigmoid ? 0.f : -INFINITY;
-        sc[t][e] = z;
-        top = fmaxf(top, z);
-      }
+        return z - c1 * logf(1.0f + c2 * (float)max(d, 0));
+      });
+    if (A.dist_bias != nullptr) scores([&](float z, int t, int e) { return z + db[t][e]; });
+    if (A.sigmoid) scores([&](float z, int, int) { return sigmoidf_(z + bias); });
+    if (!whole) {
+      const float none = A.sigmoid ? 0.f : -INFINITY;
+      scores([&](float z, int t, int e) { return has[t][e] ? z : none; });
+    }
     if (!A.sigmoid) {
+      const float top = fmaxf(fmaxf(fmaxf(sc[0][0], sc[0][1]), fmaxf(sc[0][2], sc[0][3])),
+                              fmaxf(fmaxf(sc[1][0], sc[1][1]), fmaxf(sc[1][2], sc[1][3])));
       const float mn = fmaxf(mx_, ft::kgroups_max(top)), mu = mn == -INFINITY ? 0.f : mn;
-      const float f = mx_ == -INFINITY ? 0.f : expf(mx_ - mu);
+      const float f = mx_ == -INFINITY ? 0.f : wd_exp(mx_ - mu);
       l_ *= f;
 #pragma unroll
       for (int t = 0; t < DT; ++t) o[t] *= f;
@@ -192,7 +221,7 @@ window_decode_kernel(WindowArgs A) {
       for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          sc[t][e] = expf(sc[t][e] - mu);
+          sc[t][e] = wd_exp(sc[t][e] - mu);
           l_ += sc[t][e];
         }
     }
@@ -292,7 +321,8 @@ extern "C" int mx_window_decode(void* out, int out_bf16, const float* q, const v
                                 hipStream_t s) {
   const WindowArgs A{out, out_bf16, q, (const bf16_t*)k_cache, (const bf16_t*)v_cache, start, pos0, kv_len, bt, bt_stride, num_segs,
                      heads, maps, kv_heads, window, scale, sigmoid, r1, r2, pb, block_size, num_blocks, skip_from, softcap,
-                     has_sink, sink, sinks, blocks, keep_first, dist_bias, nd};
+                     has_sink, sink, sinks, blocks, keep_first, dist_bias, nd,
+                     block_size & (block_size - 1) ? -1 : __builtin_ctz(block_size)};
   const long groups = total_rows * kv_heads * maps;
   const dim3 grid((unsigned)total_rows, (unsigned)(kv_heads * maps));
   // eight waves are a CU's registers: fewer share a group's keys where that leaves groups waiting.  us with 8 / 4 / 2 waves,
