@@ -356,15 +356,22 @@ latent_combine_kernel(float* __restrict__ out, const float* __restrict__ ws_acc,
     ms = ws_ml[(b0 + (long)lane * heads) * 2];
     ls = ws_ml[(b0 + (long)lane * heads) * 2 + 1];
   }
-  float M = ft::wave_max(ms);
-  if (sink != nullptr) M = fmaxf(M, sink[h]);
-  const float w = ms == -INFINITY ? 0.f : expf(ms - M);
-  float L = ft::wave_sum(w * ls);
-  if (sink != nullptr) L += expf(sink[h] - M);
-  const float inv = L > 0.f ? 1.0f / L : 0.f;
+  float inv = 0.f;
+  auto weight = [&](int) {
+    float M = ft::wave_max(ms);
+    if (sink != nullptr) M = fmaxf(M, sink[h]);
+    const float w = ms == -INFINITY ? 0.f : expf(ms - M);
+    float L = ft::wave_sum(w * ls);
+    if (sink != nullptr) L += expf(sink[h] - M);
+    inv = L > 0.f ? 1.0f / L : 0.f;
+    return w;
+  };
   float* op = out + ((long)h * total_rows + row) * rank;
-  merge_slices<VEC>(ws_acc + b0 * rank, (long)heads * rank, w, splits, (unit % chunks) * 256, rank, lane,
-                    [&](int c, float v) { op[c] = v * inv; });
+  merge_slices<VEC>(ws_acc + b0 * rank, (long)heads * rank, weight, splits, (unit % chunks) * 256, rank, lane,
+                    [&](int c, const float* v, auto count) {
+#pragma unroll
+                      for (int k = 0; k < decltype(count)::value; ++k) op[c + k] = v[k] * inv;
+                    });
 }
 
 // P[r, j] = softmax_j(scale * S[r, j]) over the keys j <= first_pos + (r mod rows_per_head),

@@ -10,6 +10,7 @@
 #include <stdint.h>
 
 #include "ft_common.h"
+#include <type_traits>
 
 namespace mx {
 
@@ -256,12 +257,13 @@ struct ConvWalk {
   }
 };
 
-// sum_sp w[sp] acc[sp * stride + c] for a wave that owns columns [c0, c0 + 256) of n: w is lane
+// sum_sp w[sp] acc[sp * stride + c] for a wave that owns columns [c0, c0 + 256) of n: w, from weight(c), is lane
 // sp's value (slices <= 64, 0 beyond them; a slice of weight 0 adds nothing).  VEC (n and stride multiples of 4,
-// 16-byte aligned): several slices per pass, 16-byte loads; out(c, value) is called once per
-// column by one lane.
-template <bool VEC, typename F>
-__device__ __forceinline__ void merge_slices(const float* __restrict__ acc, long stride, float w, int slices, int c0,
+// 16-byte aligned): several slices per pass, 16-byte loads, the first ones asked for before the weights, which wait for
+// loads of their own; c is the first column that the lane may leave.  out(c, values, count) is called once per
+// column by one lane, four columns at a time (VEC) or one.
+template <bool VEC, typename W, typename F>
+__device__ __forceinline__ void merge_slices(const float* __restrict__ acc, long stride, W weight, int slices, int c0,
                                              int n, int lane, F out) {
   const int cols = min(256, n - c0);
   if constexpr (VEC) {
@@ -270,15 +272,20 @@ __device__ __forceinline__ void merge_slices(const float* __restrict__ acc, long
     while (lpp < pieces) lpp <<= 1;              // lanes per slice
     const int per = 64 / lpp, sub = lane / lpp, pc = lane & (lpp - 1);
     float v[4] = {0.f, 0.f, 0.f, 0.f};
+    float4 a[8];
+    auto load = [&](int s0) {
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        a[u] = *reinterpret_cast<const float4*>(acc + min(s0 + u * per + sub, slices - 1) * stride + c0 + 4 * min(pc, pieces - 1));
+    };
+    load(0);
+    const float w = weight(c0 + 4 * min(pc, pieces - 1));
     // eight passes' loads at a time without a branch among them (with one per slice 32 slices of 512 columns took 14 us,
     // so 6); a slice of weight 0 may hold anything and adds nothing
     const unsigned long long some = __builtin_amdgcn_ballot_w64(w != 0.f);
     for (int s0 = 0; s0 < slices; s0 += 8 * per) {
       if (((some >> s0) & (8 * per < 64 ? (1ull << (8 * per)) - 1 : ~0ull)) == 0) continue;
-      float4 a[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u)
-        a[u] = *reinterpret_cast<const float4*>(acc + min(s0 + u * per + sub, slices - 1) * stride + c0 + 4 * min(pc, pieces - 1));
+      if (s0 > 0) load(s0);
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
         const int sp = s0 + u * per + sub;
@@ -294,11 +301,9 @@ __device__ __forceinline__ void merge_slices(const float* __restrict__ acc, long
 #pragma unroll
       for (int k = 0; k < 4; ++k) v[k] += __shfl_xor(v[k], off);
     }
-    if (sub == 0 && pc < pieces) {
-#pragma unroll
-      for (int k = 0; k < 4; ++k) out(c0 + 4 * pc + k, v[k]);
-    }
+    if (sub == 0 && pc < pieces) out(c0 + 4 * pc, v, std::integral_constant<int, 4>{});
   } else {
+    const float w = weight(c0);
     for (int c = lane; c - lane < cols; c += 64) {
       float v = 0.f;
 #pragma unroll 4
@@ -306,7 +311,7 @@ __device__ __forceinline__ void merge_slices(const float* __restrict__ acc, long
         const float ws = __shfl(w, sp);
         if (c < cols && ws != 0.f) v += ws * acc[sp * stride + c0 + c];
       }
-      if (c < cols) out(c0 + c, v);
+      if (c < cols) out(c0 + c, &v, std::integral_constant<int, 1>{});
     }
   }
 }

@@ -303,12 +303,27 @@ talk_attn_kernel(float* __restrict__ ws_acc, float* __restrict__ ws_ml, const fl
   if constexpr (AHEAD > 0) lpk = AHEAD;
   const int sg = lane & (lpk - 1), sub = lane / lpk, kpp = 64 / lpk;
   const bool has_piece = sg < pieces;
+  // TILED: four key heads' pieces of 128 entries for this lane's key, all of them on their way before the first is used
+  uint4 kr[4][4];
   for (int c0 = begin; c0 < end; c0 += kTalkTile) {
     const int cc = c0 + lane;
     const int j = cc < b.ext ? cc : b.first + cc - b.ext;
     const int slot = blk >= 0 && blk < num_blocks ? blk * block_size + j % block_size : -1;
     blk = page_of(cc + kTalkTile);
     const int slot16 = __shfl(slot, col);      // the key whose scores this lane holds
+    const bf16_t* kp16 = reinterpret_cast<const bf16_t*>(k_cache) + (long)max(slot16, 0) * nk;
+    auto load_keys = [&](int g0, int d0) {
+#pragma unroll
+      for (int gi = 0; gi < 4; ++gi)
+#pragma unroll
+        for (int st = 0; st < 4; ++st) {
+          // entries past the row's end meet zeros of the queries, key heads past the last no score
+          const int d = min(d0 + 32 * st + 8 * qt, dk - 8);
+          kr[gi][st] = piece16(kp16 + (long)min(g0 + gi, kv_heads - 1) * dk + d);
+        }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    if constexpr (TILED) load_keys(4 * half, 0);
     __syncthreads();                                 // q_s is there / the last tile's z_s is no longer read
     // AHEAD: this lane's value pieces of the tile (pass ps: key ps * kpp + sub)
     uint4 vr[AHEAD > 0 ? AHEAD : 1];
@@ -325,7 +340,6 @@ talk_attn_kernel(float* __restrict__ ws_acc, float* __restrict__ ws_ml, const fl
     if constexpr (TILED) {
       const bf16_t* qb = reinterpret_cast<const bf16_t*>(q_s) + n * qrow + 8 * qt;
       const int part = 16 * NB * qrow;
-      const bf16_t* kp = reinterpret_cast<const bf16_t*>(k_cache) + (long)max(slot16, 0) * nk;
       for (int g0 = 4 * half; g0 < kv_heads; g0 += W) {
         f32x4_t acc[NB][4];
 #pragma unroll
@@ -333,15 +347,7 @@ talk_attn_kernel(float* __restrict__ ws_acc, float* __restrict__ ws_ml, const fl
 #pragma unroll
           for (int gi = 0; gi < 4; ++gi) acc[bb][gi] = f32x4_t{0.f, 0.f, 0.f, 0.f};
         for (int d0 = 0; d0 < dk; d0 += 128) {
-          uint4 kr[4][4];
-#pragma unroll
-          for (int gi = 0; gi < 4; ++gi)
-#pragma unroll
-            for (int st = 0; st < 4; ++st) {
-              // entries past the row's end meet zeros of the queries, key heads past the last no score
-              const int d = min(d0 + 32 * st + 8 * qt, dk - 8);
-              kr[gi][st] = piece16(kp + (long)min(g0 + gi, kv_heads - 1) * dk + d);
-            }
+          if (d0 > 0 || g0 > 4 * half) load_keys(g0, d0);
 #pragma unroll
           for (int bb = 0; bb < NB; ++bb) {
             // key heads g0 .. g0 + 3 serve query heads g0 rep .. (g0 + 4) rep - 1
@@ -582,11 +588,14 @@ talk_attn_kernel(float* __restrict__ ws_acc, float* __restrict__ ws_ml, const fl
 }
 
 // one wave per (row, head, 256 columns): merges the slices, divides by the sum (with the sink's
-// term, if there is one), applies the element-wise sigmoid gate (optional) and rounds
+// term, if there is one), applies the element-wise sigmoid gate (optional) and rounds.  Bound by latency: the statistics, the
+// first slices and the gate are asked for together.  With the attention before it, 16 heads of 128 on 4 key heads, us in a graph at
+// 30 / 540 / 3300 keys: 1 row 12 13 16 (13 14 18 with each behind the one before, there and in the keys' loads), 64 rows 13 30 90
+// (15 33 92).
 template <typename TG, typename TO, bool VEC>
 __global__ void __launch_bounds__(256)
 talk_combine_kernel(TO* __restrict__ out, const float* __restrict__ ws_acc, const float* __restrict__ ws_ml,
-                    const TG* __restrict__ gate, long gate_stride, const int* __restrict__ start, int num_segs,
+                    const TG* __restrict__ gate, long gate_stride, int fours, const int* __restrict__ start, int num_segs,
                     long total_rows, int heads, int dv, int skip_from, int splits, int has_sink, float sink_all,
                     const float* __restrict__ sinks) {
   const long pair = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -594,28 +603,55 @@ talk_combine_kernel(TO* __restrict__ out, const float* __restrict__ ws_acc, cons
   const int lane = threadIdx.x & 63;
   const long row = pair / heads;
   const int h = (int)(pair % heads);
-  if (row >= start[num_segs]) return;
   if (skip_from > 0) {
+    if (row >= start[num_segs]) return;
     const int sg = segment_of(start, num_segs, (int)row);
     if (start[sg + 1] - start[sg] >= skip_from) return;
   }
   // lane = slice (splits <= 64)
   const long b0 = row * splits * heads + h;
-  float ms = -INFINITY, ls = 0.f;
-  if (lane < splits) {
-    ms = ws_ml[(b0 + (long)lane * heads) * 2];
-    ls = ws_ml[(b0 + (long)lane * heads) * 2 + 1];
-  }
-  float M = ft::wave_max(ms);
+  const long at_ml = (b0 + (long)min(lane, splits - 1) * heads) * 2;
+  float ms = ws_ml[at_ml], ls = ws_ml[at_ml + 1], inv = 0.f, g[4];
   const float sink = sinks != nullptr ? sinks[h] : sink_all;
-  if (has_sink) M = fmaxf(M, sink);
-  const float w = ms == -INFINITY ? 0.f : expf(ms - M);
-  const float L = ft::wave_sum(w * ls) + (has_sink ? expf(sink - M) : 0.f);
-  const float inv = L > 0.f ? 1.0f / L : 0.f;
-  merge_slices<VEC>(ws_acc + b0 * dv, (long)heads * dv, w, splits, blockIdx.y * 256, dv, lane, [&](int c, float v) {
-    v *= inv;
-    if (gate != nullptr) v *= sigmoidf_(ld(gate, row * gate_stride + (long)h * dv + c));
-    st(out, (row * heads + h) * dv + c, v);
+  const TG* gp = gate + row * gate_stride + (long)h * dv;
+  auto weight = [&](int c) {
+    if (VEC && gate != nullptr) {             // (fours: at whole fours)
+      if (fours && sizeof(TG) == 2) {
+        const uint2 u = *reinterpret_cast<const uint2*>(gp + c);
+        ft::unpack2(u.x, g[0], g[1]);
+        ft::unpack2(u.y, g[2], g[3]);
+      } else {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) g[k] = ld(gp, c + k);
+      }
+    }
+    if (lane >= splits) ms = -INFINITY, ls = 0.f;
+    float M = ft::wave_max(ms);
+    if (has_sink) M = fmaxf(M, sink);
+    const float w = ms == -INFINITY ? 0.f : expf(ms - M);
+    const float L = ft::wave_sum(w * ls) + (has_sink ? expf(sink - M) : 0.f);
+    inv = L > 0.f ? 1.0f / L : 0.f;
+    return w;
+  };
+  const int rows = start[num_segs];
+  merge_slices<VEC>(ws_acc + b0 * dv, (long)heads * dv, weight, splits, blockIdx.y * 256, dv, lane,
+                    [&](int c, const float* v, auto count) {
+    constexpr int N = decltype(count)::value;
+    if (row >= rows) return;
+    float y[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      y[k] = v[k] * inv;
+      if (gate != nullptr) y[k] *= sigmoidf_(N == 4 ? g[k] : ld(gp, c + k));
+    }
+    TO* dst = out + (row * heads + h) * dv + c;
+    if constexpr (N == 4 && sizeof(TO) == 2) {
+      *reinterpret_cast<uint2*>(dst) = make_uint2(ft::pack2(y[0], y[1]), ft::pack2(y[2], y[3]));
+    } else if constexpr (N == 4) {
+      *reinterpret_cast<float4*>(dst) = make_float4(y[0], y[1], y[2], y[3]);
+    } else {
+      st(dst, 0, y[0]);
+    }
   });
 }
 
@@ -826,9 +862,10 @@ extern "C" int mx_talk_attention(void* out, int out_bf16, float* ws_acc, float* 
   const dim3 g2((unsigned)((total_rows * heads + 3) / 4), (unsigned)((dv + 255) / 256));
 #define MX_TC(V)                                                                                                \
   MX_DISPATCH_T(out_bf16, hipLaunchKernelGGL((talk_combine_kernel<T, T, V>), g2, dim3(256), 0, s, (T*)out,      \
-                                             ws_acc, ws_ml, (const T*)gate, gate_stride, start, num_segs,       \
+                                             ws_acc, ws_ml, (const T*)gate, gate_stride, fours, start, num_segs, \
                                              total_rows, heads, dv, skip_from, splits, has_sink, sink_all, sinks))
-  if (dv % 4 == 0 && ((uintptr_t)ws_acc) % 16 == 0) MX_TC(true);
+  const int fours = gate_stride % 4 == 0 && ((uintptr_t)gate) % 8 == 0;
+  if (dv % 4 == 0 && ((uintptr_t)ws_acc) % 16 == 0 && ((uintptr_t)out) % (out_bf16 ? 8 : 16) == 0) MX_TC(true);
   else MX_TC(false);
 #undef MX_TC
   return (int)hipGetLastError();
