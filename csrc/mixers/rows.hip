@@ -182,35 +182,61 @@ __global__ void tanh_cap_kernel(float* __restrict__ x, long n, float cap) {
   }
 }
 
-// A row of a workgroup in registers: 4 C entries per thread, four neighbours at a time (16-byte
-// fp32 or 8-byte bf16 accesses when `vec`), width <= 4 C NT.
-template <typename T, int NT, int C>
-__device__ __forceinline__ void load_row(float (&v)[C][4], const T* p, int width, int vec) {
+// A row of a workgroup in registers: 4 C entries per thread, four neighbours at a time, width <= 4 C NT.  A kernel asks for
+// all rows that it will need and only then looks at the first: `ask` loads, `get` waits and widens.  VEC (16-byte fp32 or
+// 8-byte bf16 pieces, width of whole fours): no load stands behind a branch, since the compiler has every load wait that
+// may write the registers of another side of a branch; columns past the width read the row's last four and count as zeros.
+// Rows of more than 8192 have no registers for that: they load where they are got.
+template <int C>
+constexpr bool kAskAhead = C <= 4;
+template <typename T, bool VEC, int NT, int C>
+struct AskedRow {
+  using Raw = typename std::conditional<!VEC, float4, typename std::conditional<sizeof(T) == 2, uint2, float4>::type>::type;
+  Raw r[C];
+  const T* from;
+  __device__ __forceinline__ void ask(const T* p, int width) {
+    if constexpr (kAskAhead<C>) load(p, width);
+    else from = p;
+  }
+  __device__ __forceinline__ void load(const T* p, int width) {
 #pragma unroll
-  for (int c = 0; c < C; ++c) {
-    const int i = (c * NT + threadIdx.x) * 4;
-    if (vec && i < width) {
-      if constexpr (sizeof(T) == 2) {
-        const uint2 u = *reinterpret_cast<const uint2*>(p + i);
-        ft::unpack2(u.x, v[c][0], v[c][1]);
-        ft::unpack2(u.y, v[c][2], v[c][3]);
+    for (int c = 0; c < C; ++c) {
+      const int i = (c * NT + threadIdx.x) * 4;
+      if constexpr (VEC) {
+        r[c] = *reinterpret_cast<const Raw*>(p + min(i, width - 4));
       } else {
-        const float4 u = *reinterpret_cast<const float4*>(p + i);
-        v[c][0] = u.x; v[c][1] = u.y; v[c][2] = u.z; v[c][3] = u.w;
-      }
-    } else {
+        float v[4];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) v[c][k] = i + k < width ? ld(p, i + k) : 0.f;
+        for (int k = 0; k < 4; ++k) v[k] = i + k < width ? ld(p, i + k) : 0.f;
+        r[c] = make_float4(v[0], v[1], v[2], v[3]);
+      }
     }
   }
-}
+  __device__ __forceinline__ void get(float (&v)[C][4], int width) {
+    if constexpr (!kAskAhead<C>) load(from, width);
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      if constexpr (VEC && sizeof(T) == 2) {
+        ft::unpack2(r[c].x, v[c][0], v[c][1]);
+        ft::unpack2(r[c].y, v[c][2], v[c][3]);
+      } else {
+        v[c][0] = r[c].x, v[c][1] = r[c].y, v[c][2] = r[c].z, v[c][3] = r[c].w;
+      }
+      if constexpr (VEC)
+        if ((c * NT + (int)threadIdx.x) * 4 >= width)
+#pragma unroll
+          for (int k = 0; k < 4; ++k) v[c][k] = 0.f;
+    }
+  }
+};
 
-template <typename T, int NT, int C>
-__device__ __forceinline__ void store_row(T* p, const float (&v)[C][4], int width, int vec) {
+template <typename T, bool VEC, int NT, int C>
+__device__ __forceinline__ void store_row(T* p, const float (&v)[C][4], int width) {
 #pragma unroll
   for (int c = 0; c < C; ++c) {
     const int i = (c * NT + threadIdx.x) * 4;
-    if (vec && i < width) {
+    if constexpr (VEC) {
+      if (i >= width) continue;
       if constexpr (sizeof(T) == 2) {
         *reinterpret_cast<uint2*>(p + i) = make_uint2(ft::pack2(v[c][0], v[c][1]), ft::pack2(v[c][2], v[c][3]));
       } else {
@@ -227,51 +253,156 @@ __device__ __forceinline__ void store_row(T* p, const float (&v)[C][4], int widt
 // What a norm kernel adds to the residual: a row of a tensor, or of the experts' results not yet summed
 // (few_rows.hip: experts_down), sum_k w[row, k] d[row, k] + shared[row] * (sigmoid(gate[row]) or 1), which saves
 // a launch and its rows' way through memory (4.6 us a layer of a decode step); or, without weights, of a product's parts
-// (few_rows.hip: few_rows_parts).
+// (few_rows.hip: few_rows_parts).  Asked<>: as AskedRow; `other` is read in the place of what there is not.
 template <typename T>
 struct RowsOf {
+  static constexpr bool kOneRow = false;
   const T* p;
   long stride;
   __device__ __forceinline__ bool any() const { return p != nullptr; }
-  template <int NT, int C>
-  __device__ __forceinline__ void load(float (&v)[C][4], long row, int width, int vec) const {
-    load_row<T, NT, C>(v, p + row * stride, width, vec);
-  }
+  template <bool VEC, int NT, int C>
+  struct Asked {
+    AskedRow<T, VEC, NT, C> r;
+    __device__ __forceinline__ void ask(const RowsOf& y, long row, int width, const float* other) {
+      r.ask(y.p != nullptr ? y.p + row * y.stride : (const T*)other, width);
+    }
+    __device__ __forceinline__ void pin() {}
+    __device__ __forceinline__ void get(const RowsOf&, float (&v)[C][4], long, int width) { r.get(v, width); }
+  };
 };
 struct ExpertRows {
+  static constexpr bool kOneRow = true;       // (a token shift's: decode rows, segments of one row)
   const float *d, *wts, *shared, *gate;       // [rows * top, width], [rows, top] or null, [rows, width] or null, [rows] or null
   int top;
   __device__ __forceinline__ bool any() const { return true; }
-  template <int NT, int C>
-  __device__ __forceinline__ void load(float (&v)[C][4], long row, int width, int) const {      // (width: whole fours)
-    const float* w = wts != nullptr ? wts + row * top : nullptr;
-    const float g = shared != nullptr && gate != nullptr ? sigmoidf_(gate[row]) : 1.f;
-#pragma unroll
-    for (int c = 0; c < C; ++c) {
-      const int i = (c * NT + threadIdx.x) * 4;
-      v[c][0] = v[c][1] = v[c][2] = v[c][3] = 0.f;
-      if (i >= width) continue;
-      auto add = [&](const float* p, float f) {
-        const float4 u = *reinterpret_cast<const float4*>(p + i);
-        v[c][0] += f * u.x, v[c][1] += f * u.y, v[c][2] += f * u.z, v[c][3] += f * u.w;
-      };
-#pragma unroll 4
-      for (int k = 0; k < top; ++k) add(d + (row * top + k) * width, w != nullptr ? w[k] : 1.f);
-      if (shared != nullptr) add(shared + row * width, g);
+  // (its rows are whole fours at 16 bytes whatever the others are)
+  template <bool VEC, int NT, int C>
+  struct Asked {
+    static constexpr int A = C <= 2 ? 4 : 1;  // of the `top` rows so many at once
+    float4 d[A][C], shared[C];
+    float w[A], gate;
+    __device__ __forceinline__ void ask(const ExpertRows& y, long row, int width, const float*) {
+      if constexpr (kAskAhead<C>) load(y, row, width);
     }
-  }
+    // behind all that is asked for: the compiler moves scalar loads to their use, one wait behind the other
+    __device__ __forceinline__ void pin() {
+      if constexpr (kAskAhead<C>) {
+#pragma unroll
+        for (int k = 0; k < A; ++k) asm volatile("" : "+s"(w[k]));
+        asm volatile("" : "+s"(gate));
+      }
+    }
+    __device__ __forceinline__ void load(const ExpertRows& y, long row, int width) {
+      const float* wp = y.wts != nullptr ? y.wts + row * y.top : y.d;
+      gate = *(y.gate != nullptr ? y.gate + row : y.d);
+#pragma unroll
+      for (int k = 0; k < A; ++k) w[k] = wp[min(k, y.top - 1)];
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        const int i = min((c * NT + (int)threadIdx.x) * 4, width - 4);
+#pragma unroll
+        for (int k = 0; k < A; ++k)
+          d[k][c] = *reinterpret_cast<const float4*>(y.d + (row * y.top + min(k, y.top - 1)) * width + i);
+        shared[c] = *reinterpret_cast<const float4*>((y.shared != nullptr ? y.shared + row * width : y.d) + i);
+      }
+    }
+    __device__ __forceinline__ void get(const ExpertRows& y, float (&v)[C][4], long row, int width) {
+      if constexpr (!kAskAhead<C>) load(y, row, width);
+      const float g = y.gate != nullptr ? sigmoidf_(gate) : 1.f;
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        const int i = (c * NT + (int)threadIdx.x) * 4;
+        const bool in = i < width;
+        v[c][0] = v[c][1] = v[c][2] = v[c][3] = 0.f;
+        auto add = [&](const float4& u, float f) {
+          v[c][0] += f * u.x, v[c][1] += f * u.y, v[c][2] += f * u.z, v[c][3] += f * u.w;
+        };
+#pragma unroll
+        for (int k = 0; k < A; ++k)
+          if (in && k < y.top) add(d[k][c], y.wts != nullptr ? w[k] : 1.f);
+        if (in)
+#pragma unroll 4
+          for (int k = A; k < y.top; ++k)
+            add(*reinterpret_cast<const float4*>(y.d + (row * y.top + k) * width + i), y.wts != nullptr ? y.wts[row * y.top + k] : 1.f);
+        if (in && y.shared != nullptr) add(shared[c], g);
+      }
+    }
+  };
 };
-struct AnyRows {                              // either, by the launch: bf16 or fp32 rows, or a product's parts
+constexpr int kAskedParts = 4;                // of a product's parts so many at once (no product here has more)
+struct AnyRows {                              // either, by the launch: bf16 or fp32 rows, or a product's parts, A at once
   const void* p;
   int bf16, parts;
   long stride;
   __device__ __forceinline__ bool any() const { return p != nullptr; }
-  template <int NT, int C>
-  __device__ __forceinline__ void load(float (&v)[C][4], long row, int width, int vec) const {
-    if (parts > 1) ExpertRows{(const float*)p, nullptr, nullptr, nullptr, parts}.load<NT, C>(v, row, width, vec);
-    else if (bf16) load_row<bf16_t, NT, C>(v, (const bf16_t*)p + row * stride, width, vec);
-    else load_row<float, NT, C>(v, (const float*)p + row * stride, width, vec);
-  }
+  template <bool VEC, int NT, int C, int A>
+  struct Asked {
+    uint2 lo[A][C], hi[A][C];
+    const float* from;
+    __device__ __forceinline__ void ask(const AnyRows& y, long row, int width, const float* other) {
+      if constexpr (kAskAhead<C>) load(y, row, width, other);
+      else from = other;
+    }
+    __device__ __forceinline__ void load(const AnyRows& y, long row, int width, const float* other) {
+      const bool two = y.bf16 && y.p != nullptr, parts = y.parts > 1;
+      const long es = two ? 2 : 4, rest = two ? 0 : 8;       // (half an fp32 piece; a bf16 piece is read twice)
+#pragma unroll
+      for (int k = 0; k < A; ++k) {
+        const char* q = y.p == nullptr ? (const char*)other
+                                       : (const char*)y.p + (parts ? (row * y.parts + min(k, y.parts - 1)) * width : row * y.stride) * es;
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+          const int i = (c * NT + (int)threadIdx.x) * 4;
+          if (VEC || parts) {
+            const char* at = q + min(i, width - 4) * es;
+            lo[k][c] = *reinterpret_cast<const uint2*>(at);
+            hi[k][c] = *reinterpret_cast<const uint2*>(at + rest);
+          } else {
+            uint32_t u[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              u[e] = 0;
+              if (i + e < width) u[e] = two ? (uint32_t)((const uint16_t*)q)[i + e] << 16 : ((const uint32_t*)q)[i + e];
+            }
+            lo[k][c] = make_uint2(u[0], u[1]);
+            hi[k][c] = make_uint2(u[2], u[3]);
+          }
+        }
+      }
+    }
+    __device__ __forceinline__ void get(const AnyRows& y, float (&v)[C][4], long row, int width) {
+      if constexpr (!kAskAhead<C>) load(y, row, width, from);
+      const bool parts = y.parts > 1, packed = VEC && y.bf16 && !parts;
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        auto four = [&](int k, float (&u)[4]) {
+          float b[4];
+          ft::unpack2(lo[k][c].x, b[0], b[1]);
+          ft::unpack2(lo[k][c].y, b[2], b[3]);
+          u[0] = packed ? b[0] : __uint_as_float(lo[k][c].x);
+          u[1] = packed ? b[1] : __uint_as_float(lo[k][c].y);
+          u[2] = packed ? b[2] : __uint_as_float(hi[k][c].x);
+          u[3] = packed ? b[3] : __uint_as_float(hi[k][c].y);
+        };
+        four(0, v[c]);
+#pragma unroll
+        for (int k = 1; k < A; ++k)
+          if (parts && k < y.parts) {
+            float u[4];
+            four(k, u);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[c][e] += u[e];
+          }
+        if (parts)
+          for (int k = A; k < y.parts; ++k) {
+            const float4 u = *reinterpret_cast<const float4*>((const float*)y.p + (row * y.parts + k) * width +
+                                                              min((c * NT + (int)threadIdx.x) * 4, width - 4));
+            v[c][0] += u.x, v[c][1] += u.y, v[c][2] += u.z, v[c][3] += u.w;
+          }
+        if ((VEC || parts) && (c * NT + (int)threadIdx.x) * 4 >= width) v[c][0] = v[c][1] = v[c][2] = v[c][3] = 0.f;
+      }
+    }
+  };
 };
 
 // sums of two values over a block; every thread gets both
@@ -308,14 +439,24 @@ __device__ __forceinline__ float sum_sq(const float (&v)[C][4]) {
 // reductions for few rows, by the rows' bytes for many.  Width 2048: layer norm of 32 rows 4.7 us, of 2000 12
 // (values read entry by entry, again for each pass: 10 and 16); scaled add and norm of 777 rows 6 (10); mean of two norms
 // 5 (9).
-template <typename Y, typename TO, int NT, int C>
+template <typename Y, typename TO, bool VEC, int NT, int C>
 __global__ void __launch_bounds__(NT)
 layer_norm_row_kernel(float* __restrict__ x, Y y, const float* __restrict__ w,
                       const float* __restrict__ b, TO* __restrict__ out, TO* __restrict__ cast,
-                      const float* __restrict__ next_w, const float* __restrict__ next_b, int width, float eps, int vec) {
+                      const float* __restrict__ next_w, const float* __restrict__ next_b, int width, float eps) {
   __shared__ float red[NT / 64];
   const long row = blockIdx.x;
   float v[C][4], u[C][4], wv[C][4], bv[C][4];
+  AskedRow<float, VEC, NT, C> xa, wa, ba, nwa, nba;
+  typename Y::template Asked<VEC, NT, C> ya;
+  const bool next = next_w != nullptr;
+  xa.ask(x + row * width, width);
+  ya.ask(y, row, width, x + row * width);
+  wa.ask(w, width);
+  ba.ask(b, width);
+  nwa.ask(next ? next_w : w, width);
+  nba.ask(next ? next_b : b, width);
+  ya.pin();
   auto norm = [&] {                          // u <- its layer norm, times wv plus bv
     float sum = 0.f;
 #pragma unroll
@@ -336,17 +477,17 @@ layer_norm_row_kernel(float* __restrict__ x, Y y, const float* __restrict__ w,
 #pragma unroll
       for (int k = 0; k < 4; ++k) u[c][k] = u[c][k] * r * wv[c][k] + bv[c][k];
   };
-  load_row<float, NT, C>(v, x + row * width, width, vec);
+  xa.get(v, width);
   if (y.any()) {
-    y.template load<NT, C>(u, row, width, vec);
+    ya.get(y, u, row, width);
   } else {
 #pragma unroll
     for (int c = 0; c < C; ++c)
 #pragma unroll
       for (int k = 0; k < 4; ++k) u[c][k] = v[c][k];
   }
-  load_row<float, NT, C>(wv, w, width, vec);
-  load_row<float, NT, C>(bv, b, width, vec);
+  wa.get(wv, width);
+  ba.get(bv, width);
   norm();
   if (out == nullptr && y.any())
 #pragma unroll
@@ -354,35 +495,42 @@ layer_norm_row_kernel(float* __restrict__ x, Y y, const float* __restrict__ w,
 #pragma unroll
       for (int k = 0; k < 4; ++k) u[c][k] += v[c][k];
   if (out != nullptr) {
-    store_row<TO, NT, C>(out + row * width, u, width, vec);
+    store_row<TO, VEC, NT, C>(out + row * width, u, width);
   } else {
-    store_row<float, NT, C>(x + row * width, u, width, vec);
-    if (next_w != nullptr) {
-      load_row<float, NT, C>(wv, next_w, width, vec);
-      load_row<float, NT, C>(bv, next_b, width, vec);
+    store_row<float, VEC, NT, C>(x + row * width, u, width);
+    if (next) {
+      nwa.get(wv, width);
+      nba.get(bv, width);
       norm();
     }
-    if (cast != nullptr) store_row<TO, NT, C>(cast + row * width, u, width, vec);
+    if (cast != nullptr) store_row<TO, VEC, NT, C>(cast + row * width, u, width);
   }
 }
 
-template <typename TO, int NT, int C>
+// A: parts of y1 and y2 (1: neither is in parts)
+template <typename TO, bool VEC, int A, int NT, int C>
 __global__ void __launch_bounds__(NT)
 add_scaled_rms_norm_row_kernel(float* __restrict__ x, AnyRows y1, AnyRows y2, float mult,
-                               const float* __restrict__ next_w, TO* __restrict__ out, int width, float eps, int vec) {
+                               const float* __restrict__ next_w, TO* __restrict__ out, int width, float eps) {
   __shared__ float red[NT / 64];
   const long row = blockIdx.x;
   float v[C][4], a[C][4], b[C][4], w[C][4];
-  load_row<float, NT, C>(v, x + row * width, width, vec);
-  if (y1.any()) y1.load<NT, C>(a, row, width, vec);
-  if (y2.any()) y2.load<NT, C>(b, row, width, vec);
-  if (out != nullptr) load_row<float, NT, C>(w, next_w, width, vec);
+  AskedRow<float, VEC, NT, C> xa, wa;
+  AnyRows::Asked<VEC, NT, C, kAskAhead<C> ? A : 1> ya, yb;
+  xa.ask(x + row * width, width);
+  ya.ask(y1, row, width, x + row * width);
+  yb.ask(y2, row, width, x + row * width);
+  wa.ask(out != nullptr ? next_w : x + row * width, width);
+  xa.get(v, width);
+  ya.get(y1, a, row, width);
+  yb.get(y2, b, row, width);
+  wa.get(w, width);
   if (y1.any()) {
 #pragma unroll
     for (int c = 0; c < C; ++c)
 #pragma unroll
       for (int k = 0; k < 4; ++k) v[c][k] += mult * (y2.any() ? a[c][k] + b[c][k] : a[c][k]);
-    store_row<float, NT, C>(x + row * width, v, width, vec);
+    store_row<float, VEC, NT, C>(x + row * width, v, width);
   }
   if (out == nullptr) return;
   const float r = 1.0f / sqrtf(block_sum<NT>(sum_sq<C>(v), red) / (float)width + eps);
@@ -390,20 +538,26 @@ add_scaled_rms_norm_row_kernel(float* __restrict__ x, AnyRows y1, AnyRows y2, fl
   for (int c = 0; c < C; ++c)
 #pragma unroll
     for (int k = 0; k < 4; ++k) v[c][k] *= r * w[c][k];
-  store_row<TO, NT, C>(out + row * width, v, width, vec);
+  store_row<TO, VEC, NT, C>(out + row * width, v, width);
 }
 
-template <int NT, int C>
+template <bool VEC, int A, int NT, int C>
 __global__ void __launch_bounds__(NT)
 dual_rms_mean_row_kernel(float* __restrict__ out, AnyRows a, AnyRows b, const float* __restrict__ wa,
-                         const float* __restrict__ wb, int width, float eps, float scale, int vec) {
+                         const float* __restrict__ wb, int width, float eps, float scale) {
   __shared__ float red[NT / 64][2];
   const long row = blockIdx.x;
   float u[C][4], v[C][4], p[C][4], q[C][4];
-  a.load<NT, C>(u, row, width, vec);
-  b.load<NT, C>(v, row, width, vec);
-  load_row<float, NT, C>(p, wa, width, vec);
-  load_row<float, NT, C>(q, wb, width, vec);
+  AskedRow<float, VEC, NT, C> pa, qa;
+  AnyRows::Asked<VEC, NT, C, kAskAhead<C> ? A : 1> ya, yb;
+  ya.ask(a, row, width, wa);
+  yb.ask(b, row, width, wa);
+  pa.ask(wa, width);
+  qa.ask(wb, width);
+  ya.get(a, u, row, width);
+  yb.get(b, v, row, width);
+  pa.get(p, width);
+  qa.get(q, width);
   float sa = sum_sq<C>(u), sb = sum_sq<C>(v);
   block_sum2<NT>(sa, sb, red);
   const float ra = 1.0f / sqrtf(sa / (float)width + eps), rb = 1.0f / sqrtf(sb / (float)width + eps);
@@ -411,7 +565,7 @@ dual_rms_mean_row_kernel(float* __restrict__ out, AnyRows a, AnyRows b, const fl
   for (int c = 0; c < C; ++c)
 #pragma unroll
     for (int k = 0; k < 4; ++k) u[c][k] = scale * (u[c][k] * ra * p[c][k] + v[c][k] * rb * q[c][k]);
-  store_row<float, NT, C>(out + row * width, u, width, vec);
+  store_row<float, VEC, NT, C>(out + row * width, u, width);
 }
 
 // A step's first rows and the norm that reads them, in one launch: x = embed[id] * scale (+ the position's sines and
@@ -437,12 +591,20 @@ embed_norm_kernel(EmbedArgs E, PairArgs P, float* __restrict__ x, TO* __restrict
   int id = E.ids[row];
   if (id < 0 || id >= E.vocab) id = 0;
   float v[C][4], t[C][4], wv[C][4], bv[C][4];
-  load_row<T, NT, C>(v, (const T*)E.table + (long)id * width, width, 1);
-  if constexpr (NORM > 0) load_row<float, NT, C>(wv, w, width, 1);
-  if constexpr (NORM == 2) load_row<float, NT, C>(bv, b, width, 1);
+  AskedRow<T, true, NT, C> va, ta;
+  AskedRow<float, true, NT, C> wa, ba;
+  if constexpr (NORM > 0) wa.ask(w, width);
+  if constexpr (NORM == 2) ba.ask(b, width);
+  va.ask((const T*)E.table + (long)id * width, width);
   long pair = -1;
-  if (P.table != nullptr) pair = pair_entry(P, E.ids, row);
-  if (pair >= 0) load_row<T, NT, C>(t, (const T*)P.table + pair * width, width, 1);
+  if (P.table != nullptr) {
+    pair = pair_entry(P, E.ids, row);
+    ta.ask((const T*)P.table + max(pair, 0L) * width, width);
+    ta.get(t, width);
+  }
+  va.get(v, width);
+  if constexpr (NORM > 0) wa.get(wv, width);
+  if constexpr (NORM == 2) ba.get(bv, width);
   const float p = E.freqs != nullptr ? (float)E.positions[row] : 0.f;
 #pragma unroll
   for (int c = 0; c < C; ++c) {
@@ -462,7 +624,7 @@ embed_norm_kernel(EmbedArgs E, PairArgs P, float* __restrict__ x, TO* __restrict
 #pragma unroll
       for (int k = 0; k < 4; ++k) v[c][k] += t[c][k];
   }
-  if constexpr (NORM < 2) store_row<float, NT, C>(x + (long)row * width, v, width, 1);
+  if constexpr (NORM < 2) store_row<float, true, NT, C>(x + (long)row * width, v, width);
   if constexpr (NORM == 1) {
     const float r = 1.0f / sqrtf(block_sum<NT>(sum_sq<C>(v), red) / (float)width + eps);
 #pragma unroll
@@ -486,27 +648,37 @@ embed_norm_kernel(EmbedArgs E, PairArgs P, float* __restrict__ x, TO* __restrict
     for (int c = 0; c < C; ++c)
 #pragma unroll
       for (int k = 0; k < 4; ++k) v[c][k] = v[c][k] * r * wv[c][k] + bv[c][k];
-    store_row<float, NT, C>(x + (long)row * width, v, width, 1);
+    store_row<float, true, NT, C>(x + (long)row * width, v, width);
   }
   if constexpr (NORM > 0)
-    if (out != nullptr) store_row<TO, NT, C>(out + (long)row * width, v, width, 1);
+    if (out != nullptr) store_row<TO, true, NT, C>(out + (long)row * width, v, width);
 }
 
 // residual (fp32, in place): x += rms_norm(y) * wb (y as it is without wb) (+ add_vec);
 // out = rms_norm(x) * next_w (TO);  cast = x (TO).  Every part is optional.
-template <typename Y, typename TO, int NT, int C>
+// Bound by one latency of memory and the reductions for few rows, by the rows' bytes for many.
+template <typename Y, typename TO, bool VEC, int NT, int C>
 __global__ void __launch_bounds__(NT)
 add_rms_norm_kernel(float* __restrict__ x, Y y, const float* __restrict__ wb,
                     const float* __restrict__ add_vec, const float* __restrict__ next_w, TO* __restrict__ out,
-                    TO* __restrict__ cast, int width, float eps, int vec) {
+                    TO* __restrict__ cast, int width, float eps) {
   __shared__ float red[NT / 64];
   const long row = blockIdx.x;
   float v[C][4], t[C][4], w[C][4];
-  load_row<float, NT, C>(v, x + row * width, width, vec);
+  AskedRow<float, VEC, NT, C> xa, wa, aa, na;
+  typename Y::template Asked<VEC, NT, C> ya;
+  const float* xr = x + row * width;
+  xa.ask(xr, width);
+  ya.ask(y, row, width, xr);
+  wa.ask(wb != nullptr ? wb : xr, width);
+  aa.ask(add_vec != nullptr ? add_vec : xr, width);
+  na.ask(out != nullptr ? next_w : xr, width);
+  ya.pin();
+  xa.get(v, width);
   if (y.any()) {
-    y.template load<NT, C>(t, row, width, vec);
+    ya.get(y, t, row, width);
     if (wb != nullptr) {
-      load_row<float, NT, C>(w, wb, width, vec);
+      wa.get(w, width);
       const float r = 1.0f / sqrtf(block_sum<NT>(sum_sq<C>(t), red) / (float)width + eps);
 #pragma unroll
       for (int c = 0; c < C; ++c)
@@ -519,22 +691,22 @@ add_rms_norm_kernel(float* __restrict__ x, Y y, const float* __restrict__ wb,
       for (int k = 0; k < 4; ++k) v[c][k] += t[c][k];
   }
   if (add_vec != nullptr) {
-    load_row<float, NT, C>(w, add_vec, width, vec);
+    aa.get(w, width);
 #pragma unroll
     for (int c = 0; c < C; ++c)
 #pragma unroll
       for (int k = 0; k < 4; ++k) v[c][k] += w[c][k];
   }
-  if (y.any() || add_vec != nullptr) store_row<float, NT, C>(x + row * width, v, width, vec);
-  if (cast != nullptr) store_row<TO, NT, C>(cast + row * width, v, width, vec);
+  if (y.any() || add_vec != nullptr) store_row<float, VEC, NT, C>(x + row * width, v, width);
+  if (cast != nullptr) store_row<TO, VEC, NT, C>(cast + row * width, v, width);
   if (out != nullptr) {
-    load_row<float, NT, C>(w, next_w, width, vec);
+    na.get(w, width);
     const float r = 1.0f / sqrtf(block_sum<NT>(sum_sq<C>(v), red) / (float)width + eps);
 #pragma unroll
     for (int c = 0; c < C; ++c)
 #pragma unroll
       for (int k = 0; k < 4; ++k) v[c][k] *= r * w[c][k];
-    store_row<TO, NT, C>(out + row * width, v, width, vec);
+    store_row<TO, VEC, NT, C>(out + row * width, v, width);
   }
 }
 
@@ -548,37 +720,47 @@ add_rms_norm_kernel(float* __restrict__ x, Y y, const float* __restrict__ wb,
 // one-row segment also leaves its h in the slot; shift_state_kernel does that for longer ones
 // afterwards (a slot may still be read by the segment's first row here).
 // ---------------------------------------------------------------------------------
-template <typename Y, typename TO, int NT, int C>
+template <typename Y, typename TO, bool VEC, int NT, int C>
 __global__ void __launch_bounds__(NT)
 add_norm_shift_kernel(float* x_out, const float* x_in, Y y, const float* __restrict__ wb, const float* __restrict__ w,
                       const float* __restrict__ shift,
                       TO* __restrict__ out, float* state, int num_slots, const int* __restrict__ start,
                       const int* __restrict__ pos0, const int* __restrict__ slot, int num_segs, int width,
-                      float eps, int vec) {
+                      float eps) {
   __shared__ float red[NT / 64][2];
   const long row = blockIdx.x;
+  AskedRow<float, VEC, NT, C> xr, pr, wbr, wr, sr;
+  typename Y::template Asked<VEC, NT, C> yr, ypr;
+  xr.ask(x_in + row * width, width);
+  yr.ask(y, row, width, x_in + row * width);
+  wbr.ask(wb != nullptr ? wb : w, width);
+  wr.ask(w, width);
+  sr.ask(shift, width);
   int sl = -1, rel = 0, n = 1;
   bool old = false;
   if (row < start[num_segs]) {
     const int sg = segment_of(start, num_segs, (int)row);
-    rel = (int)row - start[sg];
+    if constexpr (!Y::kOneRow) rel = (int)row - start[sg];
     n = start[sg + 1] - start[sg];
     sl = slot[sg];
     if (sl >= num_slots) sl = -1;
     old = sl >= 0 && pos0[sg] > 0;
   }
+  // the row above, or what the state slot holds of it
+  pr.ask(rel > 0 ? x_in + (row - 1) * width : old ? state + (long)sl * width : x_in + row * width, width);
   float xa[C][4], xp[C][4], t[C][4];
-  load_row<float, NT, C>(xa, x_in + row * width, width, vec);
-  if (rel > 0) load_row<float, NT, C>(xp, x_in + (row - 1) * width, width, vec);
+  if (rel > 0 && y.any()) ypr.ask(y, row - 1, width, x_in);
+  yr.pin();
+  xr.get(xa, width);
+  pr.get(xp, width);
   if (y.any()) {
-    float yp[C][4];
-    y.template load<NT, C>(t, row, width, vec);
-    if (rel > 0) y.template load<NT, C>(yp, row - 1, width, vec);
+    float yp[C][4], wv[C][4];
+    yr.get(y, t, row, width);
+    if (rel > 0) ypr.get(y, yp, row - 1, width);
     float sa = sum_sq<C>(t), sb = rel > 0 ? sum_sq<C>(yp) : 0.f;
     block_sum2<NT>(sa, sb, red);
     const float ra = 1.0f / sqrtf(sa / (float)width + eps), rb = 1.0f / sqrtf(sb / (float)width + eps);
-    float wv[C][4];
-    load_row<float, NT, C>(wv, wb, width, vec);
+    wbr.get(wv, width);
 #pragma unroll
     for (int c = 0; c < C; ++c)
 #pragma unroll
@@ -586,49 +768,51 @@ add_norm_shift_kernel(float* x_out, const float* x_in, Y y, const float* __restr
         xa[c][k] += t[c][k] * ra * wv[c][k];
         if (rel > 0) xp[c][k] += yp[c][k] * rb * wv[c][k];
       }
-    store_row<float, NT, C>(x_out + row * width, xa, width, vec);
+    store_row<float, VEC, NT, C>(x_out + row * width, xa, width);
   }
   float sa = sum_sq<C>(xa), sb = rel > 0 ? sum_sq<C>(xp) : 0.f;
   block_sum2<NT>(sa, sb, red);
   const float ra = 1.0f / sqrtf(sa / (float)width + eps), rb = 1.0f / sqrtf(sb / (float)width + eps);
-  load_row<float, NT, C>(t, w, width, vec);
+  wr.get(t, width);
 #pragma unroll
   for (int c = 0; c < C; ++c)
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       xa[c][k] *= ra * t[c][k];
-      xp[c][k] = rel > 0 ? xp[c][k] * (rb * t[c][k]) : 0.f;
+      xp[c][k] = rel > 0 ? xp[c][k] * (rb * t[c][k]) : old ? xp[c][k] : 0.f;
     }
-  if (rel == 0 && old) load_row<float, NT, C>(xp, state + (long)sl * width, width, vec);
-  if (sl >= 0 && n == 1) store_row<float, NT, C>(state + (long)sl * width, xa, width, vec);
-  load_row<float, NT, C>(t, shift, width, vec);
+  if (sl >= 0 && n == 1) store_row<float, VEC, NT, C>(state + (long)sl * width, xa, width);
+  sr.get(t, width);
 #pragma unroll
   for (int c = 0; c < C; ++c)
 #pragma unroll
     for (int k = 0; k < 4; ++k) xa[c][k] += (xp[c][k] - xa[c][k]) * t[c][k];
-  store_row<TO, NT, C>(out + row * width, xa, width, vec);
+  store_row<TO, VEC, NT, C>(out + row * width, xa, width);
 }
 
 // the h of each longer segment's last row, from its x, into the segment's slot; grid segments
-template <int NT, int C>
+template <bool VEC, int NT, int C>
 __global__ void __launch_bounds__(NT)
 shift_state_kernel(float* __restrict__ state, int num_slots, const float* __restrict__ x, const float* __restrict__ w,
-                   const int* __restrict__ start, const int* __restrict__ slot, int width, float eps, int vec) {
+                   const int* __restrict__ start, const int* __restrict__ slot, int width, float eps) {
   __shared__ float red[NT / 64][2];
   const int s = blockIdx.x;
   const int n = start[s + 1] - start[s], sl = slot[s];
   if (n < 2 || sl < 0 || sl >= num_slots) return;
   float xa[C][4], t[C][4];
-  load_row<float, NT, C>(xa, x + (long)(start[s + 1] - 1) * width, width, vec);
+  AskedRow<float, VEC, NT, C> xr, wr;
+  xr.ask(x + (long)(start[s + 1] - 1) * width, width);
+  wr.ask(w, width);
+  xr.get(xa, width);
   float sa = sum_sq<C>(xa), sb = 0.f;
   block_sum2<NT>(sa, sb, red);
   const float ra = 1.0f / sqrtf(sa / (float)width + eps);
-  load_row<float, NT, C>(t, w, width, vec);
+  wr.get(t, width);
 #pragma unroll
   for (int c = 0; c < C; ++c)
 #pragma unroll
     for (int k = 0; k < 4; ++k) xa[c][k] *= ra * t[c][k];
-  store_row<float, NT, C>(state + (long)sl * width, xa, width, vec);
+  store_row<float, VEC, NT, C>(state + (long)sl * width, xa, width);
 }
 
 // one wave per (row, head): out = o / rms(o) * w * sigmoid(gate), or * silu(gate)
@@ -879,6 +1063,14 @@ static void row_chunks(int width, F f) {
   else if (chunks <= 4) f(std::integral_constant<int, 4>{});
   else f(std::integral_constant<int, 8>{});
 }
+// the same and whether rows are read in pieces of four (vec: width of whole fours, all rows aligned)
+template <typename F>
+static void row_chunks(int width, int vec, F f) {
+  row_chunks(width, [&](auto c) {
+    if (vec) f(c, std::true_type{});
+    else f(c, std::false_type{});
+  });
+}
 
 // x = embed[id] * scale (+ positions) (+ pairs), then the norm: 0 none, 1 out = rms_norm(x) * w, 2 x = layer_norm(x) * w + b and
 // out (if any) = x; rows that are no whole fours or too wide: only without a norm
@@ -937,10 +1129,10 @@ static void launch_layer_norm(float* x, const void* y, long ys, const float* w, 
                   ((uintptr_t)x | (uintptr_t)w | (uintptr_t)b | (uintptr_t)nw | (uintptr_t)nb) % 16 == 0 &&
                   ((uintptr_t)out | (uintptr_t)cast) % (4 * sizeof(TO)) == 0;
   if (row_in_registers(rows, width, vec)) {
-    row_chunks(width, [&](auto c) {
-      hipLaunchKernelGGL((layer_norm_row_kernel<RowsOf<TY>, TO, kRowThreads, decltype(c)::value>), dim3(rows),
+    row_chunks(width, vec, [&](auto c, auto v4) {
+      hipLaunchKernelGGL((layer_norm_row_kernel<RowsOf<TY>, TO, decltype(v4)::value, kRowThreads, decltype(c)::value>), dim3(rows),
                          dim3(kRowThreads), 0, s, x, RowsOf<TY>{(const TY*)y, ys}, w, b, (TO*)out, (TO*)cast, nw, nb,
-                         width, eps, vec);
+                         width, eps);
     });
     return;
   }
@@ -975,10 +1167,9 @@ static void launch_add_rms(float* x, const void* y, long ys, const float* wb, co
   const int vec = width % 4 == 0 && (y == nullptr || (ys % 4 == 0 && ((uintptr_t)y) % (4 * sizeof(TY)) == 0)) &&
                   ((uintptr_t)x | (uintptr_t)wb | (uintptr_t)av | (uintptr_t)nw) % 16 == 0 &&
                   ((uintptr_t)out | (uintptr_t)cast) % (4 * sizeof(TO)) == 0;
-  row_chunks(width, [&](auto c) {
-    hipLaunchKernelGGL((add_rms_norm_kernel<RowsOf<TY>, TO, kRowThreads, decltype(c)::value>), dim3(rows),
-                       dim3(kRowThreads), 0, s, x, RowsOf<TY>{(const TY*)y, ys}, wb, av, nw, (TO*)out, (TO*)cast, width, eps,
-                       vec);
+  row_chunks(width, vec, [&](auto c, auto v4) {
+    hipLaunchKernelGGL((add_rms_norm_kernel<RowsOf<TY>, TO, decltype(v4)::value, kRowThreads, decltype(c)::value>), dim3(rows),
+                       dim3(kRowThreads), 0, s, x, RowsOf<TY>{(const TY*)y, ys}, wb, av, nw, (TO*)out, (TO*)cast, width, eps);
   });
 }
 
@@ -1009,13 +1200,13 @@ extern "C" int mx_add_rms_norm_experts(float* x, const float* d, const float* wt
   if (((uintptr_t)d | (uintptr_t)shared) % 16) return -2;
   const int vec = ((uintptr_t)x | (uintptr_t)wb | (uintptr_t)add_vec | (uintptr_t)next_w | (uintptr_t)out | (uintptr_t)cast) % 16 == 0;
   const ExpertRows y{d, wts, shared, gate, top};
-  row_chunks(width, [&](auto c) {
+  row_chunks(width, vec, [&](auto c, auto v4) {
     if (out_bf16)
-      hipLaunchKernelGGL((add_rms_norm_kernel<ExpertRows, bf16_t, kRowThreads, decltype(c)::value>), dim3(rows),
-                         dim3(kRowThreads), 0, s, x, y, wb, add_vec, next_w, (bf16_t*)out, (bf16_t*)cast, width, eps, vec);
+      hipLaunchKernelGGL((add_rms_norm_kernel<ExpertRows, bf16_t, decltype(v4)::value, kRowThreads, decltype(c)::value>), dim3(rows),
+                         dim3(kRowThreads), 0, s, x, y, wb, add_vec, next_w, (bf16_t*)out, (bf16_t*)cast, width, eps);
     else
-      hipLaunchKernelGGL((add_rms_norm_kernel<ExpertRows, float, kRowThreads, decltype(c)::value>), dim3(rows),
-                         dim3(kRowThreads), 0, s, x, y, wb, add_vec, next_w, (float*)out, (float*)cast, width, eps, vec);
+      hipLaunchKernelGGL((add_rms_norm_kernel<ExpertRows, float, decltype(v4)::value, kRowThreads, decltype(c)::value>), dim3(rows),
+                         dim3(kRowThreads), 0, s, x, y, wb, add_vec, next_w, (float*)out, (float*)cast, width, eps);
   });
   return (int)hipGetLastError();
 }
@@ -1028,9 +1219,9 @@ extern "C" int mx_layer_norm_experts(float* x, const float* d, const float* wts,
   if (((uintptr_t)d | (uintptr_t)shared) % 16) return -2;
   const int vec = ((uintptr_t)x | (uintptr_t)w | (uintptr_t)b | (uintptr_t)next_w | (uintptr_t)next_b | (uintptr_t)cast) % 16 == 0;
   const ExpertRows y{d, wts, shared, gate, top};
-  row_chunks(width, [&](auto c) {
-    hipLaunchKernelGGL((layer_norm_row_kernel<ExpertRows, bf16_t, kRowThreads, decltype(c)::value>), dim3(rows),
-                       dim3(kRowThreads), 0, s, x, y, w, b, (bf16_t*)nullptr, (bf16_t*)cast, next_w, next_b, width, eps, vec);
+  row_chunks(width, vec, [&](auto c, auto v4) {
+    hipLaunchKernelGGL((layer_norm_row_kernel<ExpertRows, bf16_t, decltype(v4)::value, kRowThreads, decltype(c)::value>), dim3(rows),
+                       dim3(kRowThreads), 0, s, x, y, w, b, (bf16_t*)nullptr, (bf16_t*)cast, next_w, next_b, width, eps);
   });
   return (int)hipGetLastError();
 }
@@ -1045,10 +1236,10 @@ extern "C" int mx_add_norm_shift_experts(float* x, const float* d, const float* 
   if (((uintptr_t)d | (uintptr_t)shared) % 16) return -2;
   const int vec = ((uintptr_t)x | (uintptr_t)wb | (uintptr_t)w | (uintptr_t)shift | (uintptr_t)out | (uintptr_t)state) % 16 == 0;
   const ExpertRows y{d, wts, shared, gate, top};
-  row_chunks(width, [&](auto c) {
-    hipLaunchKernelGGL((add_norm_shift_kernel<ExpertRows, bf16_t, kRowThreads, decltype(c)::value>), dim3(rows),
+  row_chunks(width, vec, [&](auto c, auto v4) {
+    hipLaunchKernelGGL((add_norm_shift_kernel<ExpertRows, bf16_t, decltype(v4)::value, kRowThreads, decltype(c)::value>), dim3(rows),
                        dim3(kRowThreads), 0, s, x, x, y, wb, w, shift, (bf16_t*)out, state, num_slots, start, pos0, slot,
-                       num_segs, width, eps, vec);
+                       num_segs, width, eps);
   });
   return (int)hipGetLastError();
 }
@@ -1223,14 +1414,19 @@ extern "C" int mx_add_scaled_rms_norm(float* x, const void* y1, int y1_bf16, lon
   const int vec = width % 4 == 0 && va && vb &&
                   ((uintptr_t)x | (uintptr_t)next_w) % 16 == 0 && ((uintptr_t)out) % (out_bf16 ? 8 : 16) == 0;
   if (row_in_registers(rows, width, vec) || y1_parts > 1 || y2_parts > 1) {
-    row_chunks(width, [&](auto c) {
-      if (out_bf16)
-        hipLaunchKernelGGL((add_scaled_rms_norm_row_kernel<bf16_t, kRowThreads, decltype(c)::value>), dim3(rows),
-                           dim3(kRowThreads), 0, s, x, a, b, mult, next_w, (bf16_t*)out, width, eps, vec);
-      else
-        hipLaunchKernelGGL((add_scaled_rms_norm_row_kernel<float, kRowThreads, decltype(c)::value>), dim3(rows),
-                           dim3(kRowThreads), 0, s, x, a, b, mult, next_w, (float*)out, width, eps, vec);
-    });
+    auto go = [&](auto parts) {
+      row_chunks(width, vec, [&](auto c, auto v4) {
+        constexpr int A = decltype(parts)::value, C = decltype(c)::value;
+        if (out_bf16)
+          hipLaunchKernelGGL((add_scaled_rms_norm_row_kernel<bf16_t, decltype(v4)::value, A, kRowThreads, C>), dim3(rows),
+                             dim3(kRowThreads), 0, s, x, a, b, mult, next_w, (bf16_t*)out, width, eps);
+        else
+          hipLaunchKernelGGL((add_scaled_rms_norm_row_kernel<float, decltype(v4)::value, A, kRowThreads, C>), dim3(rows),
+                             dim3(kRowThreads), 0, s, x, a, b, mult, next_w, (float*)out, width, eps);
+      });
+    };
+    if (y1_parts > 1 || y2_parts > 1) go(std::integral_constant<int, kAskedParts>{});
+    else go(std::integral_constant<int, 1>{});
     return (int)hipGetLastError();
   }
   if (out_bf16)
@@ -1252,10 +1448,14 @@ extern "C" int mx_dual_rms_mean(float* out, const void* a, int a_bf16, long a_st
   if (va < 0 || vb < 0) return -2;
   const int vec = width % 4 == 0 && va && vb && ((uintptr_t)out | (uintptr_t)wa | (uintptr_t)wb) % 16 == 0;
   if (row_in_registers(rows, width, vec) || a_parts > 1 || b_parts > 1) {
-    row_chunks(width, [&](auto c) {
-      hipLaunchKernelGGL((dual_rms_mean_row_kernel<kRowThreads, decltype(c)::value>), dim3(rows), dim3(kRowThreads), 0, s,
-                         out, ra, rb, wa, wb, width, eps, scale, vec);
-    });
+    auto go = [&](auto parts) {
+      row_chunks(width, vec, [&](auto c, auto v4) {
+        hipLaunchKernelGGL((dual_rms_mean_row_kernel<decltype(v4)::value, decltype(parts)::value, kRowThreads, decltype(c)::value>),
+                           dim3(rows), dim3(kRowThreads), 0, s, out, ra, rb, wa, wb, width, eps, scale);
+      });
+    };
+    if (a_parts > 1 || b_parts > 1) go(std::integral_constant<int, kAskedParts>{});
+    else go(std::integral_constant<int, 1>{});
     return (int)hipGetLastError();
   }
   if (a_bf16 != b_bf16) return -1;
@@ -1287,14 +1487,14 @@ static void launch_shift(float* x_out, const float* x_in, const void* y, long ys
   const int vec = width % 4 == 0 && (y == nullptr || (ys % 4 == 0 && ((uintptr_t)y) % (4 * sizeof(TY)) == 0)) &&
                   ((uintptr_t)x_in | (uintptr_t)x_out | (uintptr_t)w | (uintptr_t)wb | (uintptr_t)shift |
                    (uintptr_t)state) % 16 == 0 && ((uintptr_t)out) % (4 * sizeof(TO)) == 0;
-  row_chunks(width, [&](auto c) {
+  row_chunks(width, vec, [&](auto c, auto v4) {
     constexpr int C = decltype(c)::value;
-    hipLaunchKernelGGL((add_norm_shift_kernel<RowsOf<TY>, TO, kRowThreads, C>), dim3(rows), dim3(kRowThreads), 0, s, x_out,
+    hipLaunchKernelGGL((add_norm_shift_kernel<RowsOf<TY>, TO, decltype(v4)::value, kRowThreads, C>), dim3(rows), dim3(kRowThreads), 0, s, x_out,
                        x_in, RowsOf<TY>{(const TY*)y, ys}, wb, w, shift, (TO*)out, state, num_slots, start, pos0, slot,
-                       num_segs, width, eps, vec);
+                       num_segs, width, eps);
     if (max_rows > 1)
-      hipLaunchKernelGGL((shift_state_kernel<kRowThreads, C>), dim3(num_segs), dim3(kRowThreads), 0, s, state,
-                         num_slots, x_out, w, start, slot, width, eps, vec);
+      hipLaunchKernelGGL((shift_state_kernel<decltype(v4)::value, kRowThreads, C>), dim3(num_segs), dim3(kRowThreads), 0, s, state,
+                         num_slots, x_out, w, start, slot, width, eps);
   });
 }
 
