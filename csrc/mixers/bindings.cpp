@@ -234,6 +234,11 @@ int mx_moe_route_fits(const void* h, long h_stride, const void* parts, int exper
 int mx_moe_route(int* idx, float* wts, const void* h, long h_stride, const void* parts, const float* bias, long rows,
                  int experts, int width, int top, int mode, float scale, int groups, int keep, hipStream_t s);
 int mx_state_step_fits(const float* o, const float* state, int dk, int dv);
+int mx_group_step_fits(int taps, int heads, int groups, int dk, int dv);
+int mx_group_step(void* out, int bf16, const void* x, long x_stride, const void* z, long z_stride, const void* dt, long dt_stride,
+                  const float* conv_w, const float* conv_b, int taps, float* hist, const float* a_log, const float* dt_bias,
+                  const float* skip, const float* norm, float eps, float* state, const int* start, const int* pos0,
+                  const int* slot, int num_segs, int heads, int groups, int dk, int dv, int num_slots, hipStream_t s);
 int mx_state_step(int kind, float* o, const void* x, int bf16, long x_stride, const void* a, long a_stride, const void* b,
                   long b_stride, const float* a_log, const float* dt_bias, const float* skip, float inv_tau, float* state,
                   const int* start, const int* pos0, const int* slot, int num_segs, int heads, int kv_heads, int dk, int dv,
@@ -806,6 +811,35 @@ void row_step(int64_t kind, Tensor out, Tensor x, Tensor a, OptT b, Tensor gate,
                   opt(hist), opt(a_log), dt_bias.data_ptr<float>(), 1.0f / (float)tau, norm.data_ptr<float>(), (float)eps,
                   silu ? 1 : 0, state.data_ptr<float>(), start.data_ptr<int>(), pos0.data_ptr<int>(), slot.data_ptr<int>(),
                   (int)num_segs, (int)heads, (int)dk, (int)dv, (int)state.size(0), stream()), "row_step");
+}
+
+// one row per sequence of a state-space mixer: convolution, state, gate and group norm (row_step.hip)
+void group_step(Tensor out, Tensor x, Tensor z, Tensor dt, Tensor conv_w, OptT conv_b, Tensor hist, Tensor a_log, Tensor dt_bias,
+                Tensor skip, Tensor norm, double eps, Tensor state, Tensor start, Tensor pos0, Tensor slot, int64_t num_segs,
+                int64_t heads, int64_t groups, int64_t dk, int64_t dv) {
+  for (const Tensor* t : {&x, &z, &dt}) {
+    check_rows(*t, "group_step");
+    TORCH_CHECK(t->scalar_type() == x.scalar_type() && t->size(0) == x.size(0), "group_step rows");
+  }
+  for (const Tensor* t : {&conv_w, &hist, &a_log, &dt_bias, &skip, &norm, &state}) check_f32(*t, "group_step");
+  TORCH_CHECK(conv_w.dim() == 2 && mx_group_step_fits((int)conv_w.size(1), (int)heads, (int)groups, (int)dk, (int)dv), "group_step sizes");
+  const int64_t inner = heads * dv, c = inner + 2 * groups * dk, taps = conv_w.size(1);
+  TORCH_CHECK(x.size(1) == c && z.size(1) == inner && dt.size(1) == heads && conv_w.size(0) == c && a_log.numel() == heads &&
+              dt_bias.numel() == heads && skip.numel() == heads && norm.numel() == inner, "group_step shapes");
+  TORCH_CHECK(out.is_cuda() && out.is_contiguous() && out.scalar_type() == x.scalar_type() && out.dim() == 2 &&
+              out.size(0) == x.size(0) && out.size(1) == inner, "out");
+  TORCH_CHECK(state.dim() == 4 && state.size(1) == heads && state.size(2) == dk && state.size(3) == dv && hist.dim() == 3 &&
+              hist.size(0) == state.size(0) && hist.size(1) == taps - 1 && hist.size(2) == c, "state");
+  if (conv_b) {
+    check_f32(*conv_b, "conv bias");
+    TORCH_CHECK(conv_b->numel() == c, "conv bias");
+  }
+  check_segs(start, pos0, slot, num_segs);
+  chk(mx_group_step(out.data_ptr(), bf(out), x.data_ptr(), x.stride(0), z.data_ptr(), z.stride(0), dt.data_ptr(), dt.stride(0),
+                    conv_w.data_ptr<float>(), conv_b ? conv_b->data_ptr<float>() : nullptr, (int)taps, hist.data_ptr<float>(),
+                    a_log.data_ptr<float>(), dt_bias.data_ptr<float>(), skip.data_ptr<float>(), norm.data_ptr<float>(), (float)eps,
+                    state.data_ptr<float>(), start.data_ptr<int>(), pos0.data_ptr<int>(), slot.data_ptr<int>(), (int)num_segs,
+                    (int)heads, (int)groups, (int)dk, (int)dv, (int)state.size(0), stream()), "group_step");
 }
 
 void pair_embed_add(Tensor x, Tensor ids, Tensor table, int64_t mul_prev, int64_t mul_cur, int64_t buckets,
@@ -1932,6 +1966,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gated_delta_rule", &gated_delta_rule);
   m.def("conv_delta_prep", &conv_delta_prep);
   m.def("row_step", &row_step);
+  m.def("group_step", &group_step);
+  m.def("group_step_fits", [](int64_t taps, int64_t heads, int64_t groups, int64_t dk, int64_t dv) {
+    return mx_group_step_fits((int)taps, (int)heads, (int)groups, (int)dk, (int)dv) != 0;
+  });
   m.def("row_step_fits", [](int64_t kind, int64_t taps, int64_t dk, int64_t dv) {
     return mx_row_step_fits((int)kind, (int)taps, (int)dk, (int)dv) != 0;
   });

@@ -195,9 +195,178 @@ row_step_kernel(RowStepArgs A) {
     *reinterpret_cast<float4*>(out) = make_float4(sum[0], sum[1], sum[2], sum[3]);
 }
 
+// The same of a state-space mixer (ssd.hip): convolution with a bias and silu over x, B and C, S <- g S + B (step x)^T,
+// y = S^T C + skip x, and out = y silu(z) / rms * w over a group of heads.  B and C, their history and the norm belong to a group,
+// so a workgroup owns all heads of one; a wave 32 columns of one head, a lane four of them in every 8th row.
+// Bound for few sequences by what one CU reads and writes (256 KB each of 4 heads of 128 x 128; the chain before the state's
+// loads arrive, convolution and history, costs nothing when it is asked for first: 13.5 us with the compiler's order), for many by
+// the states' bytes.  In running models, 32 heads of 128 x 128 in 8 groups, us a layer at 1 / 8 / 16 / 32 / 48 / 64 sequences:
+// 11.8 14.6 17.8 27 45 52, with a launch each for convolution, state and norm 15.7 21 27 40 57 69.
+constexpr int kGsWaves = 16, kGsCols = 32, kGsMaxDk = 128;
+
+struct GroupStepArgs {
+  void* out;                         // [T, heads * dv], dense
+  const void *x, *z, *dt;            // rows x (heads * dv) | B | C (groups * dk each); the gate; steps, one a head
+  long x_stride, z_stride, dt_stride;
+  const float *conv_w, *conv_b, *a_log, *dt_bias, *skip, *norm;      // conv_b may be null
+  float *hist, *state;
+  const int *start, *pos0, *slot;
+  int heads, groups, dk, dv, num_slots;
+  float eps;
+};
+
+// NR: rows of the state a lane, dk <= 8 NR (FULL: dk = 8 NR)
+template <typename T, int TAPS, int NR, bool FULL>
+__global__ void __launch_bounds__(64 * kGsWaves)
+group_step_kernel(GroupStepArgs A) {
+  constexpr int kOld = TAPS - 1;
+  __shared__ float x_s[kGsWaves * kGsCols], b_s[kGsMaxDk], c_s[kGsMaxDk], sq_s[kGsWaves];
+  const int grp = blockIdx.x, s = blockIdx.y, tid = threadIdx.x, lane = tid & 63, waves = blockDim.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int row = A.start[s], rows = A.start[s + 1] - row, sl = A.slot[s];
+  if (rows <= 0) return;
+  const int dk = A.dk, dv = A.dv, gs = waves * kGsCols, inner = A.heads * dv, rg = lane >> 3;
+  const int col = wave * kGsCols + 4 * (lane & 7), hd = wave * kGsCols / dv, h = grp * (A.heads / A.groups) + hd;
+  T* out = (T*)A.out + (long)row * inner + (long)grp * gs + col;
+  if (sl < 0 || sl >= A.num_slots) {
+    if (rg == 0)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) st(out, j, 0.f);
+    return;
+  }
+  const bool fresh = A.pos0[s] <= 0;
+  // entry e of the group's x | B | C: its channel, a thread each (2 dk <= gs)
+  const int n = gs + 2 * dk, channels = inner + 2 * A.groups * dk, e = min(tid, n - 1);
+  const int ch = e < gs ? grp * gs + e : e < gs + dk ? inner + grp * dk + e - gs : inner + (A.groups + grp - 1) * dk + e - gs;
+  const T xr = ((const T*)A.x + (long)row * A.x_stride)[ch];       // (widened behind the state's loads)
+  float* hist = A.hist + (long)sl * kOld * channels + ch;
+  float old[kOld], cw[TAPS];
+#pragma unroll
+  for (int m = 0; m < kOld; ++m) old[m] = hist[(long)m * channels];
+#pragma unroll
+  for (int j = 0; j < TAPS; ++j) cw[j] = A.conv_w[(long)ch * TAPS + j];
+  const float cb = (A.conv_b != nullptr ? A.conv_b : A.conv_w)[ch];
+  const T dr = ((const T*)A.dt + (long)row * A.dt_stride)[h];
+  float bias = A.dt_bias[h], rate = A.a_log[h], skip = A.skip[h];
+  float nw[4];
+  T zr[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    zr[j] = ((const T*)A.z + (long)row * A.z_stride + (long)grp * gs)[col + j];
+    nw[j] = A.norm[(long)grp * gs + col + j];
+  }
+  float* S = A.state + ((long)sl * A.heads + h) * dk * dv + (col - hd * dv);
+  float4 st_[NR];
+  // (the compiler would move the loads before this behind the state's, to where they are used)
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int r = 0; r < NR; ++r) st_[r] = *reinterpret_cast<const float4*>(S + (long)(FULL ? rg + 8 * r : min(rg + 8 * r, dk - 1)) * dv);
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("" : "+s"(bias), "+s"(rate), "+s"(skip));
+#pragma unroll
+  for (int m = 0; m < kOld; ++m) asm volatile("" : "+v"(old[m]));
+
+  const float xin = ld(&xr, 0), dz = ld(&dr, 0);
+  float y = 0.f;
+#pragma unroll
+  for (int m = 0; m < kOld; ++m) {
+    old[m] = fresh ? 0.f : old[m];
+    y += old[m] * cw[m];
+  }
+  y += xin * cw[TAPS - 1];
+  if (A.conv_b != nullptr) y += cb;
+  y *= sigmoidf_(y);
+  if (tid < n) {
+#pragma unroll
+    for (int m = 0; m < kOld; ++m) hist[(long)m * channels] = m + 1 < kOld ? old[m + 1] : xin;
+    if (tid < gs) x_s[tid] = y;
+    else if (tid < gs + dk) b_s[tid - gs] = y;
+    else c_s[tid - gs - dk] = y;
+  }
+  const float step = softplusf_(dz + bias), decay = expf(-expf(rate) * step);
+  __syncthreads();
+  float v[4], sum[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int j = 0; j < 4; ++j) v[j] = x_s[col + j];
+#pragma unroll
+  for (int r = 0; r < NR; ++r) {
+    const int i = rg + 8 * r;
+    const bool in = FULL || i < dk;
+    const float b = in ? b_s[min(i, kGsMaxDk - 1)] : 0.f, c = in ? c_s[min(i, kGsMaxDk - 1)] : 0.f;
+    float* f = reinterpret_cast<float*>(&st_[r]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      f[j] = (fresh || !in ? 0.f : decay * f[j]) + b * (step * v[j]);
+      sum[j] += f[j] * c;
+    }
+    if (in) *reinterpret_cast<float4*>(S + (long)i * dv) = st_[r];
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    sum[j] = ft::kgroups_sum(sum[j] + __shfl_xor(sum[j], 8)) + skip * v[j];
+    const float gz = ld(&zr[j], 0);
+    sum[j] *= gz * sigmoidf_(gz);
+    ss += sum[j] * sum[j];
+  }
+  ss += __shfl_xor(ss, 1);
+  ss += __shfl_xor(ss, 2);
+  ss += __shfl_xor(ss, 4);
+  if (lane == 0) sq_s[wave] = ss;
+  __syncthreads();
+  if (rg != 0) return;
+  ss = 0.f;
+  for (int w = 0; w < waves; ++w) ss += sq_s[w];
+  const float r = 1.0f / sqrtf(ss / (float)gs + A.eps);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) sum[j] *= r * nw[j];
+  if constexpr (sizeof(T) == 2)
+    *reinterpret_cast<uint2*>(out) = make_uint2(ft::pack2(sum[0], sum[1]), ft::pack2(sum[2], sum[3]));
+  else
+    *reinterpret_cast<float4*>(out) = make_float4(sum[0], sum[1], sum[2], sum[3]);
+}
+
 }  // namespace mx
 
 using namespace mx;
+
+// whether group_step_kernel takes the sizes: a group's heads in one workgroup, no wave's columns in two of them
+extern "C" int mx_group_step_fits(int taps, int heads, int groups, int dk, int dv) {
+  if (groups < 1 || heads < groups || heads % groups || dk < 1 || dv < kGsCols || dv % kGsCols) return 0;
+  const long gs = (long)(heads / groups) * dv;
+  return gs <= kGsWaves * kGsCols && dk <= kGsMaxDk && 2 * dk <= gs && taps >= 2 && taps <= kRsTaps;
+}
+
+// out and state at 16-byte addresses; every segment has one row at most
+extern "C" int mx_group_step(void* out, int bf16, const void* x, long x_stride, const void* z, long z_stride, const void* dt,
+                             long dt_stride, const float* conv_w, const float* conv_b, int taps, float* hist, const float* a_log,
+                             const float* dt_bias, const float* skip, const float* norm, float eps, float* state,
+                             const int* start, const int* pos0, const int* slot, int num_segs, int heads, int groups, int dk,
+                             int dv, int num_slots, hipStream_t s) {
+  if (num_segs <= 0) return 0;
+  if (!mx_group_step_fits(taps, heads, groups, dk, dv)) return -1;
+  if ((((uintptr_t)out) | ((uintptr_t)state)) % 16 || num_segs > 65535) return -2;
+  const GroupStepArgs A{out, x, z, dt, x_stride, z_stride, dt_stride, conv_w, conv_b, a_log, dt_bias, skip, norm, hist, state,
+                        start, pos0, slot, heads, groups, dk, dv, num_slots, eps};
+  const dim3 grid((unsigned)groups, (unsigned)num_segs), block((unsigned)(64 * (heads / groups * dv / kGsCols)));
+#define MX_GS(TAPS, NR)                                                                                                       \
+  do {                                                                                                                        \
+    if (dk == 8 * NR) MX_DISPATCH_T(bf16, hipLaunchKernelGGL((group_step_kernel<T, TAPS, NR, true>), grid, block, 0, s, A));   \
+    else MX_DISPATCH_T(bf16, hipLaunchKernelGGL((group_step_kernel<T, TAPS, NR, false>), grid, block, 0, s, A));               \
+  } while (0)
+#define MX_GS_DK(TAPS)                \
+  do {                                \
+    if (dk <= 32) MX_GS(TAPS, 4);     \
+    else if (dk <= 64) MX_GS(TAPS, 8); \
+    else MX_GS(TAPS, 16);             \
+  } while (0)
+  if (taps == 4) MX_GS_DK(4);
+  else if (taps == 3) MX_GS_DK(3);
+  else MX_GS_DK(2);
+#undef MX_GS_DK
+#undef MX_GS
+  return (int)hipGetLastError();
+}
 
 // whether the kernel takes the sizes: whole fours of columns that one workgroup holds, a convolution of two to four taps (kind 2: none)
 extern "C" int mx_row_step_fits(int kind, int taps, int dk, int dv) {

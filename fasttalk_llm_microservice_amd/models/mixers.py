@@ -740,12 +740,13 @@ class StateSpaceMixer:
     def __call__(self, h, ctx: StepContext, state) -> torch.Tensor:
         s_rec, s_conv = state
         p = M.linear(h, self.win)
-        z = p[:, :self.inner]
-        xbc = M.short_conv_silu(p[:, self.inner:self.inner + self.channels], self.conv_w, s_conv, ctx.seg,
-                                bias=self.conv_b)
-        y = M.ssd_scan(xbc, p[:, self.inner + self.channels:], self.a_log, self.dt_bias, self.d_skip, s_rec,
-                       ctx.seg, self.heads, self.groups, self.n, self.dv)
-        y = M.gate_group_norm(y, z, self.norm, self.eps, self.norm_groups, self.dtype)
+        z, xbc, dt = p.split([self.inner, self.channels, self.heads], 1)
+        y = M.group_step(xbc, z, dt, self.conv_w, self.conv_b, s_conv, self.a_log, self.dt_bias, self.d_skip, self.norm, self.eps,
+                         self.norm_groups, s_rec, ctx.seg, self.heads, self.groups, self.n, self.dv)
+        if y is None:
+            xbc = M.short_conv_silu(xbc, self.conv_w, s_conv, ctx.seg, bias=self.conv_b)
+            y = M.ssd_scan(xbc, dt, self.a_log, self.dt_bias, self.d_skip, s_rec, ctx.seg, self.heads, self.groups, self.n, self.dv)
+            y = M.gate_group_norm(y, z, self.norm, self.eps, self.norm_groups, self.dtype)
         return M.linear_out(y, self.wo, ctx.parts)
 
 

@@ -750,6 +750,20 @@ def row_step(kind: int, x, a, b, gate, conv_w, conv_state, a_log, dt_bias, tau: 
     return out
 
 
+def group_step(xbc, z, dt, conv_w, conv_b, conv_state, a_log, dt_bias, d_skip, norm, eps: float, norm_groups: int, state,
+               seg: Segments, heads: int, groups: int, n: int, dv: int) -> Optional[torch.Tensor]:
+    """One row per sequence (a decode step) of a state-space mixer in one launch: :func:`short_conv_silu`, :func:`ssd_scan` and
+    :func:`gate_group_norm` in xbc's dtype.  None where the kernel does not take the step: segments of several rows, norm groups
+    that are not those of B and C, sizes."""
+    if not xbc.is_cuda or seg.max_rows != 1 or norm_groups != groups or \
+            state.data_ptr() % 16 or not native_mixers().group_step_fits(conv_w.shape[1], heads, groups, n, dv):
+        return None
+    out = torch.empty(xbc.shape[0], heads * dv, dtype=xbc.dtype, device=xbc.device)
+    native_mixers().group_step(out, xbc, z, dt, conv_w, conv_b, conv_state, a_log, dt_bias, d_skip, norm, eps, state, seg.start,
+                               seg.pos0, seg.slot, seg.num, heads, groups, n, dv)
+    return out
+
+
 def head_rms_gate(o, w, gate_pre, eps: float, heads: int, dv: int, out_dtype, silu: bool = False):
     """Per head: o / rms(o) * w * sigmoid(gate_pre) (or * silu(gate_pre)), rounded to
     ``out_dtype``; ``gate_pre`` [T, heads*dv] may be a column range of wider rows."""
