@@ -510,7 +510,7 @@ class TalkingHeadsAttention:
     sigmoid(W_g h) before the output projection.  q, k and the output projection have
     biases.  Pages hold the rotated, normed keys and the raw k rows (the values)."""
 
-    # segments of this many rows or more run as banded products
+    # segments of this many rows or more run as banded products, unless the rows' kernel is the faster one (talk_product_rows)
     PRODUCT_ROWS = 32
 
     def __init__(self, get: Get, width: int, heads: int, kv_heads: int, dim: int, window: int, keep_first: int,
@@ -551,11 +551,14 @@ class TalkingHeadsAttention:
         q = M.rot_norm_prep(p, self.nq, self.nk, self.spec.dk, self.table, self.rot_dims, self.eps, self.q_scale,
                             ctx.positions, ctx.slot_mapping, kc, vc)
         gate = p[:, self.nq + self.nk:]
-        if seg.host is not None and seg.max_rows >= self.PRODUCT_ROWS:
+        least = self.PRODUCT_ROWS
+        if seg.host is not None and seg.max_rows >= least:
+            least = M.talk_product_rows(seg, self.spec, kc, least)
+        if seg.host is not None and seg.max_rows >= least:
             o = torch.zeros(h.shape[0], self.nq, dtype=self.dtype, device=h.device)
-            if min(b - a for a, b in zip(seg.host[0][:-1], seg.host[0][1:])) < self.PRODUCT_ROWS:
-                M.talk_attention(o, q, gate, kc, vc, seg, self.spec, skip_from=self.PRODUCT_ROWS)
-            M.talk_attention_products(o, q, gate, kc, vc, seg, self.spec, self.PRODUCT_ROWS)
+            if min(b - a for a, b in zip(seg.host[0][:-1], seg.host[0][1:])) < least:
+                M.talk_attention(o, q, gate, kc, vc, seg, self.spec, skip_from=least)
+            M.talk_attention_products(o, q, gate, kc, vc, seg, self.spec, least)
         else:
             o = torch.empty(h.shape[0], self.nq, dtype=self.dtype, device=h.device)
             M.talk_attention(o, q, gate, kc, vc, seg, self.spec)

@@ -1402,6 +1402,36 @@ def talk_attention(out, q, gate, k_cache, v_cache, seg: Segments, spec: TalkSpec
     return out
 
 
+# Segments of a prompt whose (row, key) pairs are no more, or whose band is no wider, stay with the rows' kernel, which reads the
+# caches in place, all segments in one launch; the products gather the keys, write all scores and take a dozen launches a
+# segment.  us, 16 heads of 128 on 4 key heads, kernel / products: 64 rows 20 64, 300 44 70, 600 90 118, 1024 175 175, four of 200
+# 67 293, 400 behind 1500 keys 135 187; a window of 1024 and 64 kept, 1000 behind 1500 keys 268 328, 4096 rows 891 1114; no
+# window, 300 behind 3000 (0.95 M pairs) 346 291, 700 behind 1500 (1.3 M) 364 298.  Only forms of the kernel whose waves' heads share a
+# value head (talk_attn.hip, AHEAD) of up to 16 heads: 16 heads on 16, 1100 rows 854 320; 32 on 8, 400 behind 1500 335 297.
+TALK_ROWS_PAIRS = 768 << 10
+TALK_ROWS_BAND = 1152
+
+
+def talk_product_rows(seg: Segments, spec: TalkSpec, k_cache, least: int) -> int:
+    """The rows (``least`` or more) from which a step's segments are left to :func:`talk_attention_products`; the others are
+    :func:`talk_attention`'s.  Needs the segments' host copies."""
+    sp = spec
+    per = 1
+    while 4 * per < sp.heads:                      # heads of a wave
+        per *= 2
+    if not k_cache.is_cuda or k_cache.dtype != torch.bfloat16 or sp.heads > 16 or (sp.heads // sp.kv_heads) % per or \
+            sp.dk % 8 or sp.dv % 8 or max(sp.dk, sp.dv) > 128:
+        return least
+    none = 1 << 30
+    band = sp.window + sp.keep_first if sp.window > 0 else none
+    if band <= TALK_ROWS_BAND:
+        return none
+    start, pos0, kv_len = seg.host
+    rows = [b - a for a, b in zip(start[:-1], start[1:])]
+    return min([n for n, p, kv in zip(rows, pos0, kv_len) if n >= least and n * min(band, (p + 1 + kv) // 2) > TALK_ROWS_PAIRS],
+               default=none)
+
+
 def talk_weights(s, first_pos: int, key0: int, ext: int, spec: TalkSpec):
     """Dot products fp32 [heads, rows, keys] -> unnormalised weights exp(z - max) in place
     (zeros where a key is not visible) and the reciprocals of their row sums, fp32 [heads,
