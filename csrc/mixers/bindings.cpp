@@ -39,6 +39,12 @@ int mx_norm_route(int* idx, float* wts, void* h, float* x, const void* y, int y_
                   int layer, const float* wb, const float* w, const float* b, float eps, const float* router, const float* bias, long rows,
                   int experts, int width, int top, int mode, float scale, int groups, int keep, hipStream_t s);
 int mx_expert_rows_fit(int width);
+int mx_add_rms_norm_sorted(float* x, const void* d, const int* place, const float* wts, const void* shared, const void* h,
+                           long h_stride, const void* gate_w, int top, const float* wb, const float* add_vec, const float* next_w,
+                           void* out, void* cast, int rows, int width, float eps, hipStream_t s);
+int mx_layer_norm_sorted(float* x, const void* d, const int* place, const float* wts, const void* shared, const void* h,
+                         long h_stride, const void* gate_w, int top, const float* w, const float* b, void* cast,
+                         const float* next_w, const float* next_b, int rows, int width, float eps, hipStream_t s);
 int mx_add_rms_norm_experts(float* x, const float* d, const float* wts, const float* shared, const float* gate, int top,
                             const float* wb, const float* add_vec, const float* next_w, void* out, void* cast, int out_bf16,
                             int rows, int width, float eps, hipStream_t s);
@@ -1282,6 +1288,56 @@ void add_rms_norm_experts(Tensor x, Tensor d, OptT wts, OptT shared, OptT gate, 
       "add_rms_norm_experts");
 }
 
+// a mixture's results of the grouped products not yet summed; place: the first rows * top entries
+struct Sorted {
+  const void *d, *shared, *h, *gate_w;
+  const int* place;
+  const float* wts;
+  long h_stride;
+  int top;
+};
+Sorted check_sorted(const Tensor& d, const Tensor& place, const Tensor& wts, const OptT& shared, const Tensor& h, const OptT& gate_w,
+                    int64_t rows, int64_t width) {
+  auto bf16 = [](const Tensor& t) { return t.is_cuda() && t.scalar_type() == at::kBFloat16 && t.is_contiguous(); };
+  check_i32(place, "place");
+  check_f32(wts, "experts' weights");
+  TORCH_CHECK(mx_expert_rows_fit((int)width) && wts.dim() == 2 && wts.size(0) == rows && wts.size(1) >= 1, "experts' weights");
+  const int64_t top = wts.size(1);
+  TORCH_CHECK(bf16(d) && d.dim() == 2 && d.size(0) == rows * top && d.size(1) == width && place.numel() >= rows * top, "experts' results");
+  TORCH_CHECK(bf16(h) && h.dim() == 2 && h.size(0) == rows && h.size(1) == width, "h");
+  TORCH_CHECK(!shared || (bf16(*shared) && shared->numel() == rows * width), "shared expert's rows");
+  TORCH_CHECK(!gate_w || (shared && bf16(*gate_w) && gate_w->numel() == width), "shared expert's gate");
+  return {d.data_ptr(), shared ? shared->data_ptr() : nullptr, h.data_ptr(), gate_w ? gate_w->data_ptr() : nullptr,
+          place.data_ptr<int>(), wts.data_ptr<float>(), (long)h.stride(0), (int)top};
+}
+
+void add_rms_norm_sorted(Tensor x, Tensor d, Tensor place, Tensor wts, OptT shared, Tensor h, OptT gate_w, OptT wb, OptT add_vec,
+                         OptT next_w, OptT out, OptT cast, double eps) {
+  check_f32(x, "residual");
+  TORCH_CHECK(x.dim() == 2 && (bool)next_w == (bool)out, "residual; next_w and out go together");
+  const int64_t rows = x.size(0), width = x.size(1);
+  const Sorted e = check_sorted(d, place, wts, shared, h, gate_w, rows, width);
+  for (const OptT* t : {&out, &cast})
+    TORCH_CHECK(!*t || ((*t)->is_cuda() && (*t)->scalar_type() == at::kBFloat16 && (*t)->is_contiguous() && (*t)->sizes() == x.sizes()),
+                "out / cast");
+  chk(mx_add_rms_norm_sorted(x.data_ptr<float>(), e.d, e.place, e.wts, e.shared, e.h, e.h_stride, e.gate_w, e.top,
+                             row_weight(wb, width), row_weight(add_vec, width), row_weight(next_w, width),
+                             out ? out->data_ptr() : nullptr, cast ? cast->data_ptr() : nullptr, (int)rows, (int)width, (float)eps,
+                             stream()), "add_rms_norm_sorted");
+}
+
+void layer_norm_sorted(Tensor x, Tensor d, Tensor place, Tensor wts, OptT shared, Tensor h, OptT gate_w, Tensor w, Tensor b,
+                       Tensor cast, OptT next_w, OptT next_b, double eps) {
+  check_f32(x, "residual");
+  TORCH_CHECK(x.dim() == 2 && (bool)next_w == (bool)next_b, "residual; next norm: weight and bias");
+  const int64_t rows = x.size(0), width = x.size(1);
+  const Sorted e = check_sorted(d, place, wts, shared, h, gate_w, rows, width);
+  TORCH_CHECK(cast.is_cuda() && cast.scalar_type() == at::kBFloat16 && cast.is_contiguous() && cast.sizes() == x.sizes(), "cast");
+  chk(mx_layer_norm_sorted(x.data_ptr<float>(), e.d, e.place, e.wts, e.shared, e.h, e.h_stride, e.gate_w, e.top,
+                           row_weight(w, width), row_weight(b, width), cast.data_ptr(), row_weight(next_w, width),
+                           row_weight(next_b, width), (int)rows, (int)width, (float)eps, stream()), "layer_norm_sorted");
+}
+
 void layer_norm_experts(Tensor x, Tensor d, OptT wts, OptT shared, OptT gate, Tensor w, Tensor b, Tensor cast, OptT next_w,
                         OptT next_b, double eps) {
   check_f32(x, "residual");
@@ -1365,9 +1421,10 @@ void tile_gemm(Tensor y, Tensor x, Tensor w, OptT bias, int64_t act, double limi
                    (float)limit, (int)form, stream()), "tile_gemm");
 }
 
-void experts_many(Tensor out, Tensor h, Tensor idx, Tensor wts, Tensor wgu, Tensor wdown, double limit, int64_t act,
-                  OptT shared, OptT gate_w) {
-  check_f32(out, "out");
+// out: the sums, or, without it, only d [pairs, width] bf16 and place [rows, top], which a norm step sums (SortedRows)
+void experts_many(OptT out, Tensor d, Tensor sorted, Tensor h, Tensor idx, Tensor wts, Tensor wgu, Tensor wdown, double limit,
+                  int64_t act, OptT shared, OptT gate_w) {
+  if (out) check_f32(*out, "out");
   check_i32(idx, "idx");
   check_f32(wts, "wts");
   TORCH_CHECK(act >= 1 && act <= 5, "experts_many: activation");
@@ -1377,21 +1434,24 @@ void experts_many(Tensor out, Tensor h, Tensor idx, Tensor wts, Tensor wgu, Tens
               wgu.size(0) == wdown.size(0) && wgu.size(2) == width && wdown.size(1) == width &&
               wgu.size(1) == mult * wdown.size(2) && width % 8 == 0 && wdown.size(2) % 8 == 0,
               "experts_many: rows and expert weights");
-  TORCH_CHECK(idx.dim() == 2 && idx.size(0) == t && top >= 1 && wts.numel() == t * top && out.numel() == t * width,
+  TORCH_CHECK(idx.dim() == 2 && idx.size(0) == t && top >= 1 && wts.numel() == t * top && (!out || out->numel() == t * width),
               "experts_many: shapes");
   TORCH_CHECK(!shared || (bf16(*shared) && shared->numel() == t * width), "experts_many: shared expert's rows");
   TORCH_CHECK(!gate_w || (shared && bf16(*gate_w) && gate_w->numel() == width), "experts_many: shared expert's gate");
   const int64_t pairs = t * top, ff = wdown.size(2);
   const int experts = (int)wgu.size(0);
-  Tensor sorted = at::empty({2 * pairs + experts}, idx.options());
-  int *row = sorted.data_ptr<int>(), *place = row + pairs, *offs = place + pairs;
-  Tensor y = at::empty({pairs, ff}, h.options()), d = at::empty({pairs, width}, h.options());
+  check_i32(sorted, "sorted");
+  TORCH_CHECK(sorted.numel() == 2 * pairs + experts && bf16(d) && d.dim() == 2 && d.size(0) == pairs && d.size(1) == width,
+              "experts_many: results");
+  int *place = sorted.data_ptr<int>(), *row = place + pairs, *offs = row + pairs;
+  Tensor y = at::empty({pairs, ff}, h.options());
   chk(mx_pair_sort(offs, row, place, idx.data_ptr<int>(), t, (int)top, experts, stream()), "pair_sort");
   chk(mx_grouped_gemm(y.data_ptr(), h.data_ptr(), t, row, wgu.data_ptr(), offs, experts, pairs, (int)ff, (int)width,
                       (int)act, (float)limit, -1, stream()), "grouped_gemm");
   chk(mx_grouped_gemm(d.data_ptr(), y.data_ptr(), pairs, nullptr, wdown.data_ptr(), offs, experts, pairs, (int)width, (int)ff,
                       0, 0.f, -1, stream()), "grouped_gemm");
-  chk(mx_experts_merge(out.data_ptr<float>(), d.data_ptr(), place, wts.data_ptr<float>(),
+  if (!out) return;
+  chk(mx_experts_merge(out->data_ptr<float>(), d.data_ptr(), place, wts.data_ptr<float>(),
                        shared ? shared->data_ptr() : nullptr, h.data_ptr(), h.stride(0),
                        gate_w ? gate_w->data_ptr() : nullptr, t, (int)top, (int)width, stream()), "experts_merge");
 }
@@ -2000,6 +2060,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("expert_rows_fit", [](int64_t width) { return (bool)mx_expert_rows_fit((int)width); });
   m.def("add_rms_norm_experts", &add_rms_norm_experts);
   m.def("layer_norm_experts", &layer_norm_experts);
+  m.def("add_rms_norm_sorted", &add_rms_norm_sorted);
+  m.def("layer_norm_sorted", &layer_norm_sorted);
   m.def("add_norm_shift_experts", &add_norm_shift_experts);
   m.def("norm_route_fits", &norm_route_fits);
   m.def("norm_route", &norm_route);

@@ -266,7 +266,7 @@ struct RowsOf {
     __device__ __forceinline__ void ask(const RowsOf& y, long row, int width, const float* other) {
       r.ask(y.p != nullptr ? y.p + row * y.stride : (const T*)other, width);
     }
-    __device__ __forceinline__ void pin() {}
+    __device__ __forceinline__ void pin(const RowsOf&, int, float*) {}
     __device__ __forceinline__ void get(const RowsOf&, float (&v)[C][4], long, int width) { r.get(v, width); }
   };
 };
@@ -285,7 +285,7 @@ struct ExpertRows {
       if constexpr (kAskAhead<C>) load(y, row, width);
     }
     // behind all that is asked for: the compiler moves scalar loads to their use, one wait behind the other
-    __device__ __forceinline__ void pin() {
+    __device__ __forceinline__ void pin(const ExpertRows&, int, float*) {
       if constexpr (kAskAhead<C>) {
 #pragma unroll
         for (int k = 0; k < A; ++k) asm volatile("" : "+s"(w[k]));
@@ -325,6 +325,94 @@ struct ExpertRows {
           for (int k = A; k < y.top; ++k)
             add(*reinterpret_cast<const float4*>(y.d + (row * y.top + k) * width + i), y.wts != nullptr ? y.wts[row * y.top + k] : 1.f);
         if (in && y.shared != nullptr) add(shared[c], g);
+      }
+    }
+  };
+};
+// The same of many rows, from the grouped products (grouped_gemm.hip): sum_k w[row, k] d[place[row, k]] + shared[row] * (sigmoid(h[row] .
+// gate_w) or 1) of bf16 rows, which saves the launch that writes the sums as fp32 rows and the norm's read of those: 2000 rows of
+// 2048, 4 experts, layer norm 19.2 us (12.2 + 12.9 in two launches), 4096 rows with a gated shared expert, RMS norms 31.7 (23.2 +
+// 18.5), 300 rows 5.8 (5.0 + 4.6).
+struct SortedRows {
+  static constexpr bool kOneRow = false;
+  const bf16_t *d, *shared, *h, *gate_w;      // [pairs, width], [rows, width] or null, [rows, width], [width] or null
+  const int* place;                           // [rows, top]
+  const float* wts;                           // [rows, top]
+  long h_stride;
+  int top;
+  __device__ __forceinline__ bool any() const { return true; }
+  // (its rows are whole fours at 8 bytes whatever the others are)
+  template <bool VEC, int NT, int C>
+  struct Asked {
+    static constexpr int A = C <= 2 ? 4 : 1;  // of the `top` rows so many at once
+    uint2 d[A][C], shared[C], h[C], gw[C];
+    float w[A], gate;
+    __device__ __forceinline__ void ask(const SortedRows& y, long row, int width, const float*) {
+      if constexpr (kAskAhead<C>) load(y, row, width);
+    }
+    __device__ __forceinline__ void load(const SortedRows& y, long row, int width) {
+      const bf16_t* p[A];
+#pragma unroll
+      for (int k = 0; k < A; ++k) {
+        const long at = row * y.top + min(k, y.top - 1);
+        p[k] = y.d + (long)y.place[at] * width;
+        w[k] = y.wts[at];
+      }
+      const bf16_t* sp = y.shared != nullptr ? y.shared + row * width : p[0];
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        const int i = min((c * NT + (int)threadIdx.x) * 4, width - 4);
+        h[c] = *reinterpret_cast<const uint2*>(y.h + row * y.h_stride + i);
+        gw[c] = *reinterpret_cast<const uint2*>((y.gate_w != nullptr ? y.gate_w : p[0]) + i);
+#pragma unroll
+        for (int k = 0; k < A; ++k) d[k][c] = *reinterpret_cast<const uint2*>(p[k] + i);
+        shared[c] = *reinterpret_cast<const uint2*>(sp + i);
+      }
+    }
+    // behind all that is asked for: the shared expert's gate, a sum over the block
+    __device__ __forceinline__ void pin(const SortedRows& y, int width, float* red) {
+      gate = 1.f;
+      if (y.gate_w == nullptr) return;
+      float dot = 0.f;
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        const int i = (c * NT + (int)threadIdx.x) * 4;
+        uint2 hv = h[c], gv = gw[c];
+        if constexpr (!kAskAhead<C>) {
+          hv = *reinterpret_cast<const uint2*>(y.h + (long)blockIdx.x * y.h_stride + min(i, width - 4));
+          gv = *reinterpret_cast<const uint2*>(y.gate_w + min(i, width - 4));
+        }
+        float a[4], b[4];
+        ft::unpack2(hv.x, a[0], a[1]);
+        ft::unpack2(hv.y, a[2], a[3]);
+        ft::unpack2(gv.x, b[0], b[1]);
+        ft::unpack2(gv.y, b[2], b[3]);
+        if (i < width) dot += (a[0] * b[0] + a[1] * b[1]) + (a[2] * b[2] + a[3] * b[3]);
+      }
+      gate = sigmoidf_(block_sum<NT>(dot, red));
+    }
+    __device__ __forceinline__ void get(const SortedRows& y, float (&v)[C][4], long row, int width) {
+      if constexpr (!kAskAhead<C>) load(y, row, width);
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        const int i = (c * NT + (int)threadIdx.x) * 4;
+        const bool in = i < width;
+        v[c][0] = v[c][1] = v[c][2] = v[c][3] = 0.f;
+        auto add = [&](const uint2& u, float f) {
+          float x[4];
+          ft::unpack2(u.x, x[0], x[1]);
+          ft::unpack2(u.y, x[2], x[3]);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[c][e] += f * x[e];
+        };
+#pragma unroll
+        for (int k = 0; k < A; ++k)
+          if (in && k < y.top) add(d[k][c], w[k]);
+        if (in)
+#pragma unroll 4
+          for (int k = A; k < y.top; ++k)
+            add(*reinterpret_cast<const uint2*>(y.d + (long)y.place[row * y.top + k] * width + i), y.wts[row * y.top + k]);
+        if (in && y.shared != nullptr) add(shared[c], gate);
       }
     }
   };
@@ -456,7 +544,7 @@ layer_norm_row_kernel(float* __restrict__ x, Y y, const float* __restrict__ w,
   ba.ask(b, width);
   nwa.ask(next ? next_w : w, width);
   nba.ask(next ? next_b : b, width);
-  ya.pin();
+  ya.pin(y, width, red);
   auto norm = [&] {                          // u <- its layer norm, times wv plus bv
     float sum = 0.f;
 #pragma unroll
@@ -673,7 +761,7 @@ add_rms_norm_kernel(float* __restrict__ x, Y y, const float* __restrict__ wb,
   wa.ask(wb != nullptr ? wb : xr, width);
   aa.ask(add_vec != nullptr ? add_vec : xr, width);
   na.ask(out != nullptr ? next_w : xr, width);
-  ya.pin();
+  ya.pin(y, width, red);
   xa.get(v, width);
   if (y.any()) {
     ya.get(y, t, row, width);
@@ -750,7 +838,7 @@ add_norm_shift_kernel(float* x_out, const float* x_in, Y y, const float* __restr
   pr.ask(rel > 0 ? x_in + (row - 1) * width : old ? state + (long)sl * width : x_in + row * width, width);
   float xa[C][4], xp[C][4], t[C][4];
   if (rel > 0 && y.any()) ypr.ask(y, row - 1, width, x_in);
-  yr.pin();
+  yr.pin(y, width, nullptr);
   xr.get(xa, width);
   pr.get(xp, width);
   if (y.any()) {
@@ -1221,6 +1309,40 @@ extern "C" int mx_layer_norm_experts(float* x, const float* d, const float* wts,
   const ExpertRows y{d, wts, shared, gate, top};
   row_chunks(width, vec, [&](auto c, auto v4) {
     hipLaunchKernelGGL((layer_norm_row_kernel<ExpertRows, bf16_t, decltype(v4)::value, kRowThreads, decltype(c)::value>), dim3(rows),
+                       dim3(kRowThreads), 0, s, x, y, w, b, (bf16_t*)nullptr, (bf16_t*)cast, next_w, next_b, width, eps);
+  });
+  return (int)hipGetLastError();
+}
+
+// the two norm steps with the grouped products' rows as y (see SortedRows); bf16 results
+static int sorted_ok(const SortedRows& y, int width) {
+  return mx_expert_rows_fit(width) && y.top >= 1 && y.h_stride % 4 == 0 &&
+         ((uintptr_t)y.d | (uintptr_t)y.shared | (uintptr_t)y.h | (uintptr_t)y.gate_w) % 8 == 0;
+}
+
+extern "C" int mx_add_rms_norm_sorted(float* x, const void* d, const int* place, const float* wts, const void* shared, const void* h,
+                                      long h_stride, const void* gate_w, int top, const float* wb, const float* add_vec,
+                                      const float* next_w, void* out, void* cast, int rows, int width, float eps, hipStream_t s) {
+  if (rows <= 0) return 0;
+  const SortedRows y{(const bf16_t*)d, (const bf16_t*)shared, (const bf16_t*)h, (const bf16_t*)gate_w, place, wts, h_stride, top};
+  if (!sorted_ok(y, width)) return -1;
+  const int vec = ((uintptr_t)x | (uintptr_t)wb | (uintptr_t)add_vec | (uintptr_t)next_w | (uintptr_t)out | (uintptr_t)cast) % 16 == 0;
+  row_chunks(width, vec, [&](auto c, auto v4) {
+    hipLaunchKernelGGL((add_rms_norm_kernel<SortedRows, bf16_t, decltype(v4)::value, kRowThreads, decltype(c)::value>), dim3(rows),
+                       dim3(kRowThreads), 0, s, x, y, wb, add_vec, next_w, (bf16_t*)out, (bf16_t*)cast, width, eps);
+  });
+  return (int)hipGetLastError();
+}
+
+extern "C" int mx_layer_norm_sorted(float* x, const void* d, const int* place, const float* wts, const void* shared, const void* h,
+                                    long h_stride, const void* gate_w, int top, const float* w, const float* b, void* cast,
+                                    const float* next_w, const float* next_b, int rows, int width, float eps, hipStream_t s) {
+  if (rows <= 0) return 0;
+  const SortedRows y{(const bf16_t*)d, (const bf16_t*)shared, (const bf16_t*)h, (const bf16_t*)gate_w, place, wts, h_stride, top};
+  if (!sorted_ok(y, width)) return -1;
+  const int vec = ((uintptr_t)x | (uintptr_t)w | (uintptr_t)b | (uintptr_t)next_w | (uintptr_t)next_b | (uintptr_t)cast) % 16 == 0;
+  row_chunks(width, vec, [&](auto c, auto v4) {
+    hipLaunchKernelGGL((layer_norm_row_kernel<SortedRows, bf16_t, decltype(v4)::value, kRowThreads, decltype(c)::value>), dim3(rows),
                        dim3(kRowThreads), 0, s, x, y, w, b, (bf16_t*)nullptr, (bf16_t*)cast, next_w, next_b, width, eps);
   });
   return (int)hipGetLastError();

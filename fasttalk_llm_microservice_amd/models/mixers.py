@@ -889,7 +889,7 @@ class MoEFF:
 
     def __call__(self, h, ctx=None, routed=None, parts: bool = False):
         """``routed``: the choice (idx, wts), if :meth:`norm_route` made it; ``parts``: the result may be
-        :class:`..ops.mixers.ExpertParts`."""
+        :class:`..ops.mixers.ExpertParts` or :class:`..ops.mixers.SortedParts`."""
         t, width = h.shape
         if t <= self.PAIR_ROWS and M.experts_few_ok(h, self.wgu, self.wdown, self.shared) and \
                 M.experts_few_pays(t * self.top, self.e, self.wdown[0].numel(), self.shared is not None):
@@ -905,7 +905,7 @@ class MoEFF:
                 if self.shared_gate:
                     w1, gate_w = w1[:-1], w1[-1]
                 shared = M.linear(M.linear_act(h, w1, self.act, self.shared_limit), wdown)
-            return M.experts_many(h, idx, wts, self.wgu, self.wdown, self.act, self.limit, shared, gate_w)
+            return M.experts_many(h, idx, wts, self.wgu, self.wdown, self.act, self.limit, shared, gate_w, parts)
         if self.shared is not None and not self.shared_gate:
             # an ungated shared expert's output is what the chosen experts' are added to
             out = M.linear(self._act(M.linear(h, self.shared[0]), self.shared_limit), self.shared[1]).float()

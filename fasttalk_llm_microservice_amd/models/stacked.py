@@ -304,7 +304,7 @@ class StackedModel:
             h = M.add_layer_norm_rows(x, y, w, b, eps, dt)
         else:
             h, _ = M.add_rms_norm_rows(x, y, wb, eps, next_w=w, out_dtype=dt)
-        return ff(h, ctx)
+        return ff(h, ctx, None, parts) if isinstance(ff, MoEFF) else ff(h, ctx)
 
     def _embed(self, input_ids, ctx, caches: StackedCache, norm: Optional[torch.Tensor]):
         """(fp32 residual rows: embedding table, plus the pair table's rows if there is one; their RMS norm times ``norm``, if given)."""

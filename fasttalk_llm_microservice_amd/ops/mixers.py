@@ -369,15 +369,27 @@ class ExpertParts(NamedTuple):
     gate: Optional[torch.Tensor]      # fp32 [rows]
 
 
+class SortedParts(NamedTuple):
+    """The same of many rows (:func:`experts_many`): row t is sum_k wts[t, k] * d[place[t, k]] + shared[t] (times sigmoid(h[t] .
+    gate_w), if there is one), for :func:`add_rms_norm_rows` and :func:`add_layer_norm_rows`."""
+    d: torch.Tensor                   # bf16 [rows * top, width], sorted by expert
+    place: torch.Tensor               # int32, its first rows * top entries
+    wts: torch.Tensor                 # fp32 [rows, top]
+    shared: Optional[torch.Tensor]    # bf16 [rows, width]
+    h: torch.Tensor                   # bf16 [rows, width]
+    gate_w: Optional[torch.Tensor]    # bf16 [width]
+
+
 def add_layer_norm_rows(residual: torch.Tensor, y: Optional[torch.Tensor], w: torch.Tensor, b: torch.Tensor,
                         eps: float, out_dtype, next_norm: Optional[tuple] = None) -> torch.Tensor:
     """residual (fp32, in place) += layer_norm(y) * w + b, or, without y, residual <-
     layer_norm(residual) * w + b.  Returns the new residual in ``out_dtype`` (the residual
     itself when that is fp32): what the next sublayer of a post-norm stack reads; with ``next_norm`` (weight, bias) its layer
-    norm by these instead.  y may be :class:`ExpertParts`."""
-    if isinstance(y, ExpertParts):
+    norm by these instead.  y may be :class:`ExpertParts` or :class:`SortedParts`."""
+    if isinstance(y, (ExpertParts, SortedParts)):
         cast = torch.empty(residual.shape, dtype=out_dtype, device=residual.device)
-        native_mixers().layer_norm_experts(residual, *y, w, b, cast, *(next_norm or (None, None)), eps)
+        f = native_mixers().layer_norm_sorted if isinstance(y, SortedParts) else native_mixers().layer_norm_experts
+        f(residual, *y, w, b, cast, *(next_norm or (None, None)), eps)
         return cast
     if residual.is_cuda:
         cast = None if out_dtype == torch.float32 and next_norm is None else \
@@ -411,11 +423,13 @@ def add_rms_norm_rows(residual: torch.Tensor, y: torch.Tensor, wb: Optional[torc
                       add_vec: Optional[torch.Tensor] = None, next_w: Optional[torch.Tensor] = None,
                       out_dtype=None, want_cast: bool = False):
     """residual (fp32, in place) += rms_norm(y) * wb (y as it is without ``wb``) (+ add_vec); returns
-    (rms_norm(residual) * next_w or None, residual cast to out_dtype or None).  y may be :class:`ExpertParts`."""
-    if isinstance(y, ExpertParts):
+    (rms_norm(residual) * next_w or None, residual cast to out_dtype or None).  y may be :class:`ExpertParts` or
+    :class:`SortedParts`."""
+    if isinstance(y, (ExpertParts, SortedParts)):
         out = torch.empty(residual.shape, dtype=out_dtype, device=residual.device) if next_w is not None else None
         cast = torch.empty(residual.shape, dtype=out_dtype, device=residual.device) if want_cast else None
-        native_mixers().add_rms_norm_experts(residual, *y, wb, add_vec, next_w, out, cast, eps)
+        f = native_mixers().add_rms_norm_sorted if isinstance(y, SortedParts) else native_mixers().add_rms_norm_experts
+        f(residual, *y, wb, add_vec, next_w, out, cast, eps)
         return out, cast
     out_dtype = out_dtype or y.dtype
     if residual.is_cuda:
@@ -1714,13 +1728,18 @@ def experts_many_ok(h, wgu, wdown) -> bool:
                                   and x.data_ptr() % 16 == 0 for x in (h, wgu, wdown)))
 
 
-def experts_many(h, idx, wts, wgu, wdown, act: str, limit: float = 0.0, shared=None, gate_w=None) -> torch.Tensor:
+def experts_many(h, idx, wts, wgu, wdown, act: str, limit: float = 0.0, shared=None, gate_w=None, parts: bool = False):
     """fp32 sum_k wts[:, k] * expert_{idx[:, k]}(h) (+ ``shared``, bf16 rows, times sigmoid(h . gate_w) if
     there is a ``gate_w``), for many rows: (row, choice) pairs sorted by expert, every expert's pairs one
-    group of two grouped products.  No host round trip."""
-    out = torch.empty(h.shape, dtype=torch.float32, device=h.device)
-    native_mixers().experts_many(out, h, idx, wts, wgu, wdown, float(limit), FEW_ACTS[act], shared, gate_w)
-    return out
+    group of two grouped products.  No host round trip.  With ``parts``, where a norm step takes
+    rows of this width so, :class:`SortedParts` instead of the sum."""
+    pairs, width = h.shape[0] * idx.shape[1], h.shape[1]
+    d = torch.empty(pairs, width, dtype=h.dtype, device=h.device)
+    place = torch.empty(2 * pairs + wgu.shape[0], dtype=torch.int32, device=h.device)     # (and what the sort needs beside it)
+    parts = parts and native_mixers().expert_rows_fit(width)
+    out = None if parts else torch.empty(h.shape, dtype=torch.float32, device=h.device)
+    native_mixers().experts_many(out, d, place, h, idx, wts, wgu, wdown, float(limit), FEW_ACTS[act], shared, gate_w)
+    return SortedParts(d, place, wts, shared, h, gate_w) if parts else out
 
 
 def clamp_swiglu(gu, limit: float):
