@@ -108,7 +108,7 @@ class LatentAttention:
         self.table = M.rope_table(max_pos, rot_dims, rot_base, device=device)
 
     # segments of this many rows or more run as matrix products (ops.mixers
-    # latent_attention_products), shorter ones and decode rows in the per-row kernel
+    # latent_attention_products), shorter ones, decode rows and steps of few rows (latent_rows_pay) in the per-row kernel
     PRODUCT_ROWS = 32
 
     def cache_width(self) -> int:
@@ -134,7 +134,8 @@ class LatentAttention:
         qa, qr = M.latent_q_absorb(q, self.wuk, self.table, self.rot_dims, ctx.positions, self.heads, self.dn,
                                    self.dr, self.interleaved, self.wuk_tiles)         # [heads, T, rank]
         seg = ctx.seg
-        if seg.host is not None and seg.max_rows >= self.PRODUCT_ROWS:
+        if seg.host is not None and seg.max_rows >= self.PRODUCT_ROWS and \
+                not M.latent_rows_pay(qa, cache, seg, self.rank, self.dtype, self.PRODUCT_ROWS):
             # prefill chunks in tiles; short segments and decode rows (if any) keep the per-row
             # kernel (every row belongs to a segment, short or long)
             ol = torch.empty_like(qa)

@@ -988,6 +988,21 @@ def _latent_prefill_pays(seg: Segments, heads: int, min_rows: int) -> bool:
     return 20 + 0.06 * keys * ((blocks + 255) // 256) <= products
 
 
+def latent_rows_pay(qa, cache, seg: Segments, rank: int, dtype, min_rows: int) -> bool:
+    """Whether a prompt's step stays with the rows' kernel (:func:`latent_attention`, csrc/mixers/latent_decode.hip) although it has
+    segments of ``min_rows`` rows or more.  That kernel takes about 11 us, 0.065 a row and 0.2 a thousand pairs of row and key, the
+    tiles' kernel 28 and 0.05 a key of the longest segment (from some 600 on the products are the faster ones).  us, 16 heads, rows and
+    tiles: 32 rows 17 29, 128 18 35, 300 40 43, 400 52 48, 600 81 59, four of 40 19 31, of 100 36 34, of 200 68 42, 64 behind
+    600 keys 31 60, behind 2000 49 62.  A step with shorter segments as well saves their launch beside it."""
+    if qa.shape[0] > 16 or not latent_prefill_ok(qa, cache, rank, dtype):
+        return False
+    start, pos0, kv_len = seg.host
+    rows = [b - a for a, b in zip(start[:-1], start[1:])]
+    pairs = sum(n * (p + 1 + kv) / 2 for n, p, kv in zip(rows, pos0, kv_len))
+    keys = max((kv for n, kv in zip(rows, kv_len) if n >= min_rows), default=0)
+    return 11 + 0.065 * sum(rows) + 2e-4 * pairs <= 28 + 0.05 * min(keys, 600)
+
+
 def latent_attention_products(out, qa, qr, cache, seg: Segments, scale: float, rank: int,
                               min_rows: int, dtype, sink: Optional[torch.Tensor] = None):
     """Segments of ``min_rows`` rows or more, in one kernel (csrc/mixers/latent_prefill.hip: bf16, ranks of 512 + 64, dense
