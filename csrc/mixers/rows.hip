@@ -186,6 +186,7 @@ __global__ void tanh_cap_kernel(float* __restrict__ x, long n, float cap) {
 // all rows that it will need and only then looks at the first: `ask` loads, `get` waits and widens.  VEC (16-byte fp32 or
 // 8-byte bf16 pieces, width of whole fours): no load stands behind a branch, since the compiler has every load wait that
 // may write the registers of another side of a branch; columns past the width read the row's last four and count as zeros.
+// (With a branch, one load behind the other: a decode step's add and norm 4.7 us, 4.4 now, with a token shift 6.4 and 4.8.)
 // Rows of more than 8192 have no registers for that: they load where they are got.
 template <int C>
 constexpr bool kAskAhead = C <= 4;
