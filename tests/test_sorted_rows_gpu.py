@@ -50,3 +50,35 @@ def test_norm_steps(width, top, shared):
         xd = c(x)
         got = M.add_layer_norm_rows(xd, parts, c(w1), c(w2), EPS, bf, nxt and tuple(map(c, nxt)))
         close(xd, x1), close(got, x1 if nxt is None else layer(x1, *nxt))
+
+
+@pytest.mark.parametrize("top", [1, 2, 5, 9])
+@pytest.mark.parametrize("width", [1032, 2056, 4104, 8200])
+def test_unsorted_parts(width, top):
+    """Mixtures' results in fp32 and a product's parts (rows.hip ExpertRows, AnyRows): fewer and more than are read at once."""
+    g = torch.Generator().manual_seed(width + top)
+    rows, bf = 5, torch.bfloat16
+    d, d2, sh = rnd(rows * top, width, g=g), rnd(rows * top, width, g=g), rnd(rows, width, g=g)
+    gate, wts = rnd(rows, g=g), torch.rand(rows, top, generator=g)
+    x, w1, w2 = (rnd(*s, g=g) for s in ((rows, width), (width,), (width,)))
+    c = lambda t: t.to(DEV)                            # noqa: E731
+    sums = lambda t: t.double().view(rows, top, width).sum(1)      # noqa: E731
+    y = (d.double().view(rows, top, width) * wts.double()[:, :, None]).sum(1) + sh.double() * torch.sigmoid(gate.double())[:, None]
+
+    def close(got, want):
+        """As above; sums of up to nine terms of order one."""
+        tol = 4e-5 if got.dtype == torch.float32 else 2.0 ** -8
+        torch.testing.assert_close(got.cpu().double(), want, rtol=tol, atol=4e-5)
+
+    for parts, rows_y in ((M.ExpertParts(c(d), c(wts), c(sh), c(gate)), y), (M.ExpertParts(c(d), None, None, None), sums(d))):
+        xd = c(x)
+        out, _ = M.add_rms_norm_rows(xd, parts, c(w1), EPS, None, c(w2), bf)
+        x1 = x.double() + rms(rows_y, w1)
+        close(xd, x1), close(out, rms(x1, w2))
+    if top > 1:
+        a, b = M.ExpertParts(c(d), None, None, None), M.ExpertParts(c(d2), None, None, None)
+        xd = c(x)
+        out = M.add_scaled_rms_norm_rows(xd, a, b, 0.5, c(w2), EPS, bf)
+        x1 = x.double() + 0.5 * (sums(d) + sums(d2))
+        close(xd, x1), close(out, rms(x1, w2))
+        close(M.dual_rms_mean(a, b, c(w1), c(w2), EPS, 0.5, rows), 0.5 * (rms(sums(d), w1) + rms(sums(d2), w2)))
